@@ -168,7 +168,7 @@ YAN_API int yan_per_block_cast_to_fp8(const void* w, int w_is_fp32, void* q, flo
 /* Macro tile the library uses for a problem: op 0 = dense 16-bit, 1 = FP8 block-scaled, 2 = FP8 grouped contiguous
  * (m = total rows, and `k` carries the number of groups instead of the depth), 3 = fp32. Writes BLOCK_M / BLOCK_N.
  * op 4 (m, `k` as for op 2): 256 x 256 when the contiguous entry point runs the kernel that holds 256 x 256 and 128 x 256
- * tiles and decides on the device, from m_indices, which tile rows run as which (groups of 256 to 2047 rows on average),
+ * tiles and places them along the groups on the device, from m_indices (groups of 128 rows or more on average),
  * 0 x 0 when it runs the tile op 2 names.
  * For ops 0 and 1 with few activation rows the answer is (16 * atoms, 16): the weight-streaming kernels.
  * Host-only (no device call). Stands where the reference leaves tile choice to the caller's keys

@@ -284,6 +284,11 @@ GROUPED_CONTIGUOUS_TEST_CASES = [
 # The same kernel built for small problems through explicit keys (the cost table gives those to smaller tiles): whole
 # 256-row tiles, two groups in every other tile row, and a padding block in the middle with one boundary off.
 GROUPED_ROWS_ON_DEVICE_CASES = [((512,) * 6, 768, 512, 0), ((384, 640) * 3, 768, 512, 1), ((512, 256, -128, 500, 512), 768, 384, 0)]
+# Contiguous tiles that follow the groups, where the cutting into tall and flat tiles can go wrong: a run of odd length across the
+# 64 blocks a wave looks at at once and one that starts right behind it, padding inside, in front of and behind groups, a group of
+# one block, one k-tile (no second one to fetch), an odd number of them, outputs that are no multiple of 8.
+GROUPED_FOLLOW_GROUPS_CASES = [((63 * 128, 3 * 128, 1, 2 * 128), 264, 128, 0), ((-128, 100, -256, 5 * 128, 385, -128, 128), 520, 384, 1),
+                               ((128,) * 5, 1028, 640, 0), ((64 * 128, 65 * 128), 12, 256, 2), ((128,), 256, 128, 0)]
 GROUPED_MASKED_TEST_CASES = [
     (3, 200, 320, 384, (200, 0, 77), 128), (4, 256, 4096, 1024, (1, 256, 130, 64), 64), (2, 64, 200, 128, (64, 3), 32),
     (4, 1024, 4096, 7168, (1024, 900, 512, 1), 1024),
@@ -440,7 +445,7 @@ def jit_kernels_in_use(num_cus: int = 256):
     for rows, n, k in (((896, 1152) * 4, 4096, 7168), ((1024,) * 8, 4096, 7168), ((512,) * 16, 4096, 7168), ((384, 640) * 8, 4096, 7168)):
         name, keys, arg_defs, _ = m_grouped_gemm.grouped_kernel_plan('GroupedContiguous', len(rows), sum(rows), n, k, num_cus)
         add(name, arg_defs, m_grouped_gemm.includes, m_grouped_gemm.rows_on_device_template if 'ROWS' in keys else m_grouped_gemm.template, keys)
-    for rows, n, k, _ in GROUPED_ROWS_ON_DEVICE_CASES:
+    for rows, n, k, _ in GROUPED_ROWS_ON_DEVICE_CASES + GROUPED_FOLLOW_GROUPS_CASES:
         name, keys, arg_defs, code_template = grouped_rows_on_device_plan(sum(1 for r in rows if r > 0), n, k)
         add(name, arg_defs, m_grouped_gemm.includes, code_template, keys)
     # the grouped layouts under the compute-unit cap: tiles chosen for NUM_SMS_CAP units

@@ -87,8 +87,9 @@ struct Fp8TileConfig {
 
 // The two LDS stages of the 256-row tiles (operand tiles of Fp8TileConfig::LDS_ROWS_A / LDS_ROWS_B rows each), declared
 // once in the kernel and handed to whichever of its bodies runs; unused by the ring tiles, which declare their own ring.
+// `b2`: a third weight stage, for the tiles that fetch their weights two k-tiles ahead (kDeepB below).
 struct Fp8TwoStages {
-    uint8_t *a0, *b0, *a1, *b1;
+    uint8_t *a0, *b0, *a1, *b1, *b2;
 };
 
 // The MFMA operand of a 16-row atom whose rows start at `atom_rows` in a staged tile: lane group g holds bytes
@@ -227,45 +228,41 @@ fp8_meet_partials(f32x4 (&acc)[TN][TM], float* __restrict__ partials, unsigned* 
     return meet_partials<SPLIT_K, NW, TN * TM>([&](int v) -> f32x4& { return acc[v / TM][v % TM]; }, partials, counters, tile_slot, split, wave, lane);
 }
 
-// Contiguous groups on 256-row tiles: which tile rows hold two groups (they go first in the launch order, ContiguousSlots in
-// scheduler.hpp) is in `grouped_layout`, on the device; every wave works it out for itself, 64 tile rows at a time with a
-// row per lane. Bit `lane` of the result: tile row 64 * chunk + lane has a group in either half, and not the same.
-__device__ __forceinline__ unsigned long long
-two_group_rows_of_chunk(const int* __restrict__ grouped_layout, int m, int tiles_m, int chunk, int lane) {
-    const int row = chunk * kWaveSize + lane, m0 = row * 256;
-    bool yes = false;
-    if (row < tiles_m && m0 + 128 < m) {
-        const int g0 = grouped_layout[m0], g1 = grouped_layout[m0 + 128];
-        yes = g0 >= 0 && g1 >= 0 && g0 != g1;
-    }
-    return __ballot(yes);
+// Contiguous groups on tiles that follow the groups (fp8_gemm_contiguous_rows_kernel). A group is a run of 128-row blocks with
+// one index; walked from its first block it is cut into tall tiles of two blocks and, where it has an odd number, a flat tile
+// of one. Bit `lane` of `tall` / `flat`: such a tile starts at block 64 * chunk + lane. Padding (negative indices) has neither.
+// Chunks are taken in ascending order: `odd` carries from one to the next whether the run across the border is an odd number
+// of blocks long so far (0 in front of the first).
+struct ContiguousTileStarts { unsigned long long tall, flat; };
+__device__ __forceinline__ ContiguousTileStarts
+contiguous_tile_starts(const int* __restrict__ grouped_layout, int blocks, int chunk, int lane, int& odd) {
+    const int b = chunk * kWaveSize + lane;
+    const bool real = b < blocks;
+    const int g = real ? grouped_layout[b * 128] : -1;
+    const int before = real && b > 0 ? grouped_layout[(b - 1) * 128] : -1, behind = b + 1 < blocks ? grouped_layout[(b + 1) * 128] : -1;
+    // how far into its run this block is: counted from the last start of a run at or in front of it
+    const unsigned long long starts = __ballot(b == 0 || g != before), at_or_before = starts & (~0ull >> (63 - lane));
+    const int into = at_or_before ? lane - (63 - __clzll((long long)at_or_before)) : lane + odd;
+    const bool opens = real && g >= 0 && (into & 1) == 0;
+    odd = (__builtin_amdgcn_readlane(into, kWaveSize - 1) + 1) & 1;
+    return {__ballot(opens && behind == g), __ballot(opens && behind != g)};
 }
 
+// The block at which the tall (flat) tile row number `rank` starts. Wave-uniform; `rank` is below the number there are.
 __device__ __forceinline__ int
-count_two_group_rows(const int* __restrict__ grouped_layout, int m, int tiles_m, int lane) {
-    int count = 0;
-    for (int c = 0; c < ceil_div(tiles_m, kWaveSize); ++c) count += __popcll(two_group_rows_of_chunk(grouped_layout, m, tiles_m, c, lane));
-    return count;
-}
-
-// The tile row at position `pos` of the order "two-group rows first, then the others, either kind ascending". Wave-uniform.
-__device__ __forceinline__ int
-contiguous_row_at(const int* __restrict__ grouped_layout, int m, int tiles_m, int count, int pos, int lane) {
-    const bool among_two = pos < count;
-    int rank = among_two ? pos : pos - count;
-    for (int c = 0; c < ceil_div(tiles_m, kWaveSize); ++c) {
-        const int rows_here = min(kWaveSize, tiles_m - c * kWaveSize);
-        const unsigned long long all = rows_here == 64 ? ~0ull : ((1ull << rows_here) - 1);
-        const unsigned long long two = two_group_rows_of_chunk(grouped_layout, m, tiles_m, c, lane), mask = among_two ? two : (~two & all);
+contiguous_block_at(const int* __restrict__ grouped_layout, int blocks, bool tall, int rank, int lane) {
+    int odd = 0;
+    for (int c = 0; c < ceil_div(blocks, kWaveSize); ++c) {
+        const ContiguousTileStarts starts = contiguous_tile_starts(grouped_layout, blocks, c, lane, odd);
+        const unsigned long long mask = tall ? starts.tall : starts.flat;
         const int here = __popcll(mask);
         if (rank < here) {
-            const bool mine = ((mask >> lane) & 1) && __popcll(mask & ((1ull << lane) - 1)) == rank;
-            const unsigned long long found = __ballot(mine);
-            return found ? c * kWaveSize + __ffsll((long long)found) - 1 : pos;
+            const unsigned long long found = __ballot(((mask >> lane) & 1) && __popcll(mask & ((1ull << lane) - 1)) == rank);
+            return c * kWaveSize + __ffsll((long long)found) - 1;
         }
         rank -= here;
     }
-    return pos;         // not reached: pos < tiles_m
+    return 0;           // not reached
 }
 
 // STAGES: 2 = two LDS stages with the next k-tile's scales in registers; 3.. = a ring of that many stages.
@@ -273,8 +270,8 @@ contiguous_row_at(const int* __restrict__ grouped_layout, int m, int tiles_m, in
 // EXTERNAL_RING: the ring of a tile with STAGES > 2 lives in `ring_lds` (LDS the caller declared, 1024-byte aligned, at least
 // STAGES * Fp8TileConfig::RING_STAGE_BYTES) instead of an array of this function's own: for kernels that hold two kinds of
 // tile and run one of them (fp8_gemm_contiguous_rows_kernel).
-// EXPLICIT_TILE: `bid` names the tile itself, row-major over the tile grid (m_idx * tiles_n + n_idx), for callers that order the
-// tiles themselves.
+// EXPLICIT_TILE: `bid` names the tile itself, as (its first row / 128) * tiles_n + n_idx, for callers that order the tiles
+// themselves; in the contiguous layout all rows of such a tile belong to the group of its first row.
 template <int SHAPE_N, int SHAPE_K, int BLOCK_M, int BLOCK_N, GemmType kGemmType, int STAGES, int SPLIT_K = 1, bool EXTERNAL_RING = false,
           bool EXPLICIT_TILE = false>
 __device__ __forceinline__ void
@@ -314,8 +311,8 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     if constexpr (kGemmType == GemmType::GroupedContiguous) sched.fit_bands_to_groups(sched.tiles_m / max(num_groups, 1));
     TileCoord tile;
     if constexpr (EXPLICIT_TILE) {
-        static_assert(kGemmType != GemmType::GroupedMasked);
-        tile = TileCoord{bid / sched.tiles_n, bid % sched.tiles_n, bid >= 0 && bid < sched.total};
+        static_assert(kGemmType != GemmType::GroupedMasked && BLOCK_M % 128 == 0);
+        tile = TileCoord{bid / sched.tiles_n, bid % sched.tiles_n, true};
     } else if constexpr (kGemmType == GemmType::GroupedMasked) {
         int group;
         tile = MaskedSlots(num_groups, m, N, BLOCK_M, BLOCK_N, expected_m).tile_of(bid, &group);
@@ -325,41 +322,21 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
         rhs        += size_t(group) * N * K;
         rhs_scales += size_t(group) * NUM_N_BLOCKS * NUM_K_BLOCKS;
         m = min(m, grouped_layout[group]);        // rows of this group that exist; tiles past them leave at once
-    } else if constexpr (kGemmType == GemmType::GroupedContiguous && BLOCK_M == 256) {
-        const int two_group_rows = count_two_group_rows(grouped_layout, m, sched.tiles_m, get_lane_id());
-        tile = ContiguousSlots(m, N, BLOCK_M, BLOCK_N, num_groups, two_group_rows).tile_of(bid);
-        if (tile.valid && two_group_rows) tile.m_idx = contiguous_row_at(grouped_layout, m, sched.tiles_m, two_group_rows, tile.m_idx, get_lane_id());
     } else {
         tile = sched.tile_of(bid);
     }
     if (!tile.valid) return;
-    const int m0 = tile.m_idx * BLOCK_M, n0 = tile.n_idx * BLOCK_N;
+    const int m0 = tile.m_idx * (EXPLICIT_TILE ? 128 : BLOCK_M), n0 = tile.n_idx * BLOCK_N;
     if (m0 >= m) return;
-    // Contiguous groups are padded to 128 rows. A tile of up to 128 rows lies in one group. A 256-row tile may
-    // hold two: it then makes two passes over K, one per 128-row half, each with its own group's weights and
-    // storing only its half (rare when groups are long, and long groups are when 256-row tiles pay off).
-    constexpr bool kTwoHalves = kGemmType == GemmType::GroupedContiguous && BLOCK_M == 256;
-    int num_passes = 1, pass_group[2] = {0, 0}, pass_lo[2] = {m0, m0}, pass_hi[2] = {m, m};
+    // Contiguous groups are padded to 128 rows: a tile of up to 128 rows lies in one group, and taller tiles are placed by
+    // their caller so that they do.
     if constexpr (kGemmType == GemmType::GroupedContiguous) {
-        static_assert(128 % BLOCK_M == 0 || BLOCK_M == 256, "tiles are 128-row blocks, parts of one, or two of them");
-        const int g0 = grouped_layout[m0];
-        const int g1 = (kTwoHalves && m0 + 128 < m) ? grouped_layout[m0 + 128] : g0;
-        if (g0 == g1) {
-            if (g0 < 0) return;
-            pass_group[0] = g0;
-        } else {
-            // constant indices only: an index computed at run time would put these arrays into scratch memory
-            const bool first = g0 >= 0, second = g1 >= 0;
-            if (!first && !second) return;
-            if (first) { pass_group[0] = g0; pass_hi[0] = m0 + 128; }
-            if (second && first)  { pass_group[1] = g1; pass_lo[1] = m0 + 128; }
-            if (second && !first) { pass_group[0] = g1; pass_lo[0] = m0 + 128; }
-            num_passes = int(first) + int(second);
-        }
+        static_assert(128 % BLOCK_M == 0 || EXPLICIT_TILE, "a tile is a 128-row block, a part of one, or one its caller placed");
+        const int group = grouped_layout[m0];
+        if (group < 0) return;
+        rhs        += size_t(group) * N * K;
+        rhs_scales += size_t(group) * NUM_N_BLOCKS * NUM_K_BLOCKS;
     }
-    const uint8_t* const rhs_all = rhs;
-    const float* const rhs_scales_all = rhs_scales;
-
     const int lane = get_lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
     const int wn = wave % Cfg::WAVES_N, wm = wave / Cfg::WAVES_N;
@@ -367,7 +344,7 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     const int m_slab = m0 + wm * Cfg::WTM, n_slab = n0 + wn * Cfg::WTN;
 
     const __amdgpu_buffer_rsrc_t rsrc_a = make_rsrc(lhs, uint32_t(m) * K);
-    __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(rhs, uint32_t(N) * K);
+    const __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(rhs, uint32_t(N) * K);
     // copies of k-tiles past the end of the range keep the count of instructions in flight and move nothing
     const __amdgpu_buffer_rsrc_t rsrc_none = make_rsrc(lhs, 0);
     TileStager<BLOCK_M, NW> stage_a;
@@ -421,24 +398,36 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     using StB = TileStager<BLOCK_N, NW>;
     constexpr int NUM_COPIES = StA::PASSES + StB::PASSES, SPREAD_ROWS = TN >= 2 ? TN / 2 : 1;
     float sa_cur[TM], sb_cur[NB];
-    // A pass over one 128-row half of a 256-row tile does not fetch the other half of the activation tile: the copy passes of
-    // those rows (the first or the second half of them) go through the empty descriptor and move zeros.
-    [[maybe_unused]] __amdgpu_buffer_rsrc_t rsrc_a_half[2] = {rsrc_a, rsrc_a};
-    static_assert(!kTwoHalves || StA::PASSES % 2 == 0);
+    // Tall tiles of the contiguous layout hold a third stage of weights (160 KB of LDS with it) and fetch them two k-tiles
+    // ahead. Groups of a few hundred rows stream their weights from HBM, every weight panel for one or two tiles, and one
+    // k-tile of prefetch does not cover that: 16 groups of 256 rows x 4096 x 7168, 470 MB of weights in one round of tiles,
+    // 143 -> 135 us; 48 blocks of 128 rows over 16 groups 219 -> 201 us, and 197 with the copies handed out in the order of
+    // their deadlines, activations (due at the next k-tile) two per row of atoms, then weights one per row. One group of
+    // 8192 rows, whose weights come from the caches, runs level (195 us).
+    constexpr bool kDeepB = kGemmType == GemmType::GroupedContiguous && EXPLICIT_TILE && STAGES == 2;
+    static_assert(!kDeepB || (StA::PASSES + 1) / 2 + StB::PASSES <= TN);
+    auto row_of_copy = [](int d) { return !kDeepB ? d * SPREAD_ROWS / NUM_COPIES : (d < StA::PASSES ? d / 2 : (StA::PASSES + 1) / 2 + d - StA::PASSES); };
     auto k_step = [&](int kb, const uint8_t* a_cur, const uint8_t* b_cur, uint8_t* a_nxt, uint8_t* b_nxt) {
 #pragma unroll
         for (int j = 0; j < TM; ++j) sa_cur[j] = sa_next[j];
 #pragma unroll
         for (int b = 0; b < NB; ++b) sb_cur[b] = sb_next[b];
-        wait_for_copies();
-        __syncthreads();
+        if constexpr (kDeepB) {         // all but the youngest copies, the weights of k-tile kb + 1
+            __builtin_amdgcn_s_waitcnt(waitcnt_imm(StB::PASSES, kNoWaitLgkm));
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        } else {
+            wait_for_copies();
+            __syncthreads();
+        }
         load_scales(min(kb + 1, NUM_K_BLOCKS - 1));
         compute_tile(a_cur, b_cur, sa_cur, sb_cur, [&](int row) {
 #pragma unroll
             for (int d = 0; d < NUM_COPIES; ++d) {
-                if (d * SPREAD_ROWS / NUM_COPIES != row) continue;
-                if (d < StA::PASSES) stage_a.issue_pass(kTwoHalves ? rsrc_a_half[d * 2 / StA::PASSES] : rsrc_a, a_nxt, (kb + 1) * kRowBytes, wave, d);
-                else stage_b.issue_pass(rsrc_b, b_nxt, (kb + 1) * kRowBytes, wave, d - StA::PASSES);
+                if (row_of_copy(d) != row) continue;
+                if (d < StA::PASSES) stage_a.issue_pass(rsrc_a, a_nxt, (kb + 1) * kRowBytes, wave, d);
+                else stage_b.issue_pass(rsrc_b, b_nxt, (kb + (kDeepB ? 2 : 1)) * kRowBytes, wave, d - StA::PASSES);
             }
         });
     };
@@ -447,23 +436,6 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     constexpr bool kStagedEpilogue = Cfg::WTN >= 32;
     [[maybe_unused]] uint8_t* epi_a = nullptr;
     [[maybe_unused]] uint8_t* epi_b = nullptr;
-    // The second pass is a copy of the code, not a trip round a loop: as a loop with a run-time count even a single pass ran
-    // 10 % slower (the compiler keeps less of the main loop's state where it was).
-    constexpr int kMaxPasses = kTwoHalves ? 2 : 1;
-#pragma unroll
-    for (int pass = 0; pass < kMaxPasses; ++pass) {
-    if (kTwoHalves && pass >= num_passes) break;
-    if constexpr (kGemmType == GemmType::GroupedContiguous) {
-        rhs        = rhs_all + size_t(pass_group[pass]) * N * K;
-        rhs_scales = rhs_scales_all + size_t(pass_group[pass]) * NUM_N_BLOCKS * NUM_K_BLOCKS;
-        rsrc_b     = make_rsrc(rhs, uint32_t(N) * K);
-        if (pass) __syncthreads();        // every wave has read the last k-tile of the previous pass
-        if constexpr (kTwoHalves) {
-            const bool half_pass = num_passes == 2;
-            rsrc_a_half[0] = half_pass && pass_lo[pass] != m0 ? rsrc_none : rsrc_a;
-            rsrc_a_half[1] = half_pass && pass_hi[pass] == m0 + 128 ? rsrc_none : rsrc_a;
-        }
-    }
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
@@ -476,38 +448,28 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     stage_a.issue(rsrc_a, lds_a0, 0, wave);
     stage_b.issue(rsrc_b, lds_b0, 0, wave);
     load_scales(0);
-    // A pass over one 128-row half of a 256-row tile: the waves whose slabs lie in the other half have nothing to multiply.
-    // They run a loop of their own with the same barriers and their share of the copies, which leaves the matrix cores half
-    // a tile per k-tile (a SIMD holds one wave of either half).
-    bool other_half = false;
-    if constexpr (kTwoHalves) {
-        static_assert(128 % Cfg::WTM == 0, "a wave's slab lies in one half of the tile");
-        other_half = num_passes == 2 && (m_slab < pass_lo[pass] || m_slab >= pass_hi[pass]);
-    }
-    if (kTwoHalves && other_half) {
-        auto copy_step = [&](int kb, uint8_t* a_nxt, uint8_t* b_nxt) {
-            wait_for_copies();
-            __syncthreads();
-#pragma unroll
-            for (int d = 0; d < NUM_COPIES; ++d) {
-                if (d < StA::PASSES) stage_a.issue_pass(rsrc_a_half[d * 2 / StA::PASSES], a_nxt, (kb + 1) * kRowBytes, wave, d);
-                else stage_b.issue_pass(rsrc_b, b_nxt, (kb + 1) * kRowBytes, wave, d - StA::PASSES);
-            }
-        };
-        for (int kb = 0; kb + 1 < NUM_K_BLOCKS; kb += 2) {
-            copy_step(kb, lds_a1, lds_b1);
-            copy_step(kb + 1, lds_a0, lds_b0);
+    if constexpr (kDeepB) {
+        stage_b.issue(rsrc_b, lds_b1, kRowBytes, wave);
+        uint8_t *a_cur = lds_a0, *a_nxt = lds_a1, *b_cur = lds_b0, *b_one = lds_b1, *b_two = two_stages.b2;
+#pragma unroll 1
+        for (int kb = 0; kb < NUM_K_BLOCKS; ++kb) {
+            k_step(kb, a_cur, b_cur, a_nxt, b_two);
+            uint8_t* t = a_cur;
+            a_cur = a_nxt; a_nxt = t;
+            t = b_cur;
+            b_cur = b_one; b_one = b_two; b_two = t;
         }
-        if (NUM_K_BLOCKS % 2 == 1) copy_step(NUM_K_BLOCKS - 1, lds_a1, lds_b1);
+        epi_a = a_nxt;          // the stages of the last k-tile
+        epi_b = b_two;
     } else {
         for (int kb = 0; kb + 1 < NUM_K_BLOCKS; kb += 2) {
             k_step(kb, lds_a0, lds_b0, lds_a1, lds_b1);
             k_step(kb + 1, lds_a1, lds_b1, lds_a0, lds_b0);
         }
         if (NUM_K_BLOCKS % 2 == 1) k_step(NUM_K_BLOCKS - 1, lds_a0, lds_b0, lds_a1, lds_b1);
+        epi_a = (NUM_K_BLOCKS % 2 == 1) ? lds_a0 : lds_a1;
+        epi_b = (NUM_K_BLOCKS % 2 == 1) ? lds_b0 : lds_b1;
     }
-    epi_a = (NUM_K_BLOCKS % 2 == 1) ? lds_a0 : lds_a1;
-    epi_b = (NUM_K_BLOCKS % 2 == 1) ? lds_b0 : lds_b1;
     } else {
     // Ring of STAGES stages, STAGES - 1 k-tiles in flight: what a small tile needs when the problem is bound by
     // streaming its operands and one k-tile of prefetch cannot cover the memory latency. Every wave issues the same
@@ -682,14 +644,13 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
         if constexpr (SPLIT_K > 1)
             if (!fp8_meet_partials<SPLIT_K, NW, TN, TM>(acc, partials, counters, tile_slot, split, wave, lane_late)) return;
         uint8_t* region = (wave < NW / 2 ? epi_a : epi_b) + (wave % (NW / 2)) * REGION;
-        fp8_store_slab<Cfg, kStagedEpilogue>(acc, region, rsrc_out, m_slab, n_slab, m0, n0, pass_lo[pass], pass_hi[pass], N, stream_out, lane_late);
+        fp8_store_slab<Cfg, kStagedEpilogue>(acc, region, rsrc_out, m_slab, n_slab, m0, n0, m0, m, N, stream_out, lane_late);
     } else {
         if (LW > NW && wave >= NW) return;              // waves that only copy
         if constexpr (SPLIT_K > 1)
             if (!fp8_meet_partials<SPLIT_K, NW, TN, TM>(acc, partials, counters, tile_slot, split, wave, lane)) return;
-        fp8_store_slab<Cfg, false>(acc, nullptr, rsrc_out, m_slab, n_slab, m0, n0, pass_lo[pass], pass_hi[pass], N, stream_out, lane);
+        fp8_store_slab<Cfg, false>(acc, nullptr, rsrc_out, m_slab, n_slab, m0, n0, m0, m, N, stream_out, lane);
     }
-    }   // pass
 }
 
 // Whether a problem runs the persistent walk below: the plain GEMM on two LDS stages with an even number of k-tiles
@@ -879,14 +840,14 @@ fp8_gemm_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_s
                 const uint8_t* __restrict__ rhs, const float* __restrict__ rhs_scales,
                 __bf16* __restrict__ out, int m, int n_rt, int k_rt, int sa_stride_m, int sa_stride_k,
                 const int* __restrict__ grouped_layout, int sa_stride_g, int num_slots, int num_groups, int expected_m) {
-    Fp8TwoStages two_stages = {nullptr, nullptr, nullptr, nullptr};
+    Fp8TwoStages two_stages = {};
     if constexpr (STAGES == 2) {
         using Cfg = Fp8TileConfig<BLOCK_M, BLOCK_N>;
         __shared__ __attribute__((aligned(1024))) uint8_t lds_a0[Cfg::LDS_ROWS_A * kRowBytes];
         __shared__ __attribute__((aligned(1024))) uint8_t lds_b0[Cfg::LDS_ROWS_B * kRowBytes];
         __shared__ __attribute__((aligned(1024))) uint8_t lds_a1[Cfg::LDS_ROWS_A * kRowBytes];
         __shared__ __attribute__((aligned(1024))) uint8_t lds_b1[Cfg::LDS_ROWS_B * kRowBytes];
-        two_stages = {lds_a0, lds_b0, lds_a1, lds_b1};
+        two_stages = {lds_a0, lds_b0, lds_a1, lds_b1, nullptr};
     }
     if constexpr (fp8_walks<STAGES, kGemmType>(SHAPE_K)) {
         if (SHAPE_K != 0 || fp8_walks<STAGES, kGemmType>(k_rt)) {
@@ -911,21 +872,17 @@ fp8_gemm_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_s
     }
 }
 
-// Contiguous groups on 256-row tiles, with what a tile row that holds two groups costs decided on the device. Which rows
-// those are is in the caller's layout; the host cannot look. A 256-row tile whose halves belong to two groups makes two
-// passes over K and takes about 1.7 tile times (fp8_gemm_tile's two-pass path); as two 128 x BLOCK_N tiles on the ring its
-// halves take 1.2 to 1.3 together and can go to two workgroups, but a launch that ends on half tiles ends raggedly.
-// This kernel holds both tiles over one pool of LDS; every workgroup counts the tile rows that hold two groups (two
-// loads per lane and a ballot: `two` of `rows`) and all number the slots alike, one of three ways (measured with
-// 4096 x 7168 weights; all three give the same bits):
-//   * two * 20 < rows (long groups, or every boundary on a multiple of 256 rows): 256-row tiles throughout, the two-pass
-//     tiles first (ContiguousSlots). 16 groups of 512 rows: 225 us against 264 on 128 x 256 tiles; groups of 1920 to 2176 rows
-//     with one such row in 32: 223 against 238 for the next way;
-//   * up to a quarter of the rows: the whole 256-row tiles of the other rows first, in band order dealt to the XCDs in
-//     patches, then the half tiles of the two-group rows, the shorter jobs, which fill the end of the launch. 8 groups of
-//     896 and 1152 rows: 230 us against 251 with two-pass tiles; 16 of 384 and 640: 271 against 284 on 128-row tiles;
-//   * more than a quarter (groups of less than two tile rows: a 256-row tile has no neighbour to share its weight panel
-//     with): 128 x BLOCK_N tiles throughout. 16 groups of 384 rows: 205 us against 216 for the second way.
+// Contiguous groups on tiles that follow the groups, whatever rows they start at: two blocks of 128 rows at a time as tall
+// 256 x BLOCK_N tiles, and the block that is left of a group with an odd number of them as a flat 128 x BLOCK_N tile. Where the
+// groups lie is in the caller's layout, on the device, where the host cannot look: every wave reads the index of every
+// block (64 blocks at a time, a block per lane) and all number the slots alike: the tall tiles first, dealt to the XCDs in
+// patches, then the flat ones, the shorter jobs, which fill the end of the launch.
+// It is bound by streaming the groups' weights from HBM and, for longer groups, by the matrix cores. On a fixed grid of
+// 256-row tiles a tile that holds two groups needs two passes over K, and so many did with groups of a few blocks that
+// 128-row tiles ran throughout: 48 blocks over 16 groups x 4096 x 7168 219 -> 216 us by following the groups, 197 with the third
+// weight stage the tall tiles have room for (kDeepB); 10240 rows in 4 groups 290 -> 276 us, 8320 in 64 x 7168 x 2048 185 -> 172.
+// Mixing flat and tall tiles in the order of the groups (every weight panel then read at one time) measured the same, and
+// running tall rows flat where the tall tiles end in a round that is mostly empty gains 2-4 % there and loses 1 % elsewhere.
 // It is launched with eight slots more than the 128-row tiling has, which covers every case; workgroups beyond the last
 // slot leave at once.
 template <int SHAPE_N, int SHAPE_K, int BLOCK_N>
@@ -937,59 +894,41 @@ fp8_gemm_contiguous_rows_kernel(const uint8_t* __restrict__ lhs, const float* __
     using Tall = Fp8TileConfig<256, BLOCK_N>;
     using Flat = Fp8TileConfig<128, BLOCK_N>;
     constexpr int FLAT_STAGES = Flat::MAX_RING_STAGES;
-    constexpr int TALL_BYTES = 2 * (Tall::LDS_ROWS_A + Tall::LDS_ROWS_B) * kRowBytes, FLAT_BYTES = FLAT_STAGES * Flat::RING_STAGE_BYTES;
+    constexpr int TALL_BYTES = (2 * Tall::LDS_ROWS_A + 3 * Tall::LDS_ROWS_B) * kRowBytes, FLAT_BYTES = FLAT_STAGES * Flat::RING_STAGE_BYTES;
     static_assert(FLAT_STAGES >= 3 && fp8_launch_waves(256, BLOCK_N, 2) == 8 && fp8_launch_waves(128, BLOCK_N, FLAT_STAGES) == 8);
     __shared__ __attribute__((aligned(1024))) uint8_t pool[TALL_BYTES > FLAT_BYTES ? TALL_BYTES : FLAT_BYTES];
     uint8_t* const a0 = pool;
     uint8_t* const b0 = a0 + Tall::LDS_ROWS_A * kRowBytes;
     uint8_t* const a1 = b0 + Tall::LDS_ROWS_B * kRowBytes;
     uint8_t* const b1 = a1 + Tall::LDS_ROWS_A * kRowBytes;
+    uint8_t* const b2 = b1 + Tall::LDS_ROWS_B * kRowBytes;
     const int N = SHAPE_N ? SHAPE_N : n_rt;
     const int lane = get_lane_id();
-    const int tall_rows = ceil_div(m, 256), tiles_n = ceil_div(N, BLOCK_N);
-    const int two_group_rows = count_two_group_rows(grouped_layout, m, tall_rows, lane);
-    // tile (row, column) of the 256-row / 128-row grid
-    auto tall_tile = [&](int row, int n_idx) {
-        fp8_gemm_tile<SHAPE_N, SHAPE_K, 256, BLOCK_N, GemmType::GroupedContiguous, 2, 1, false, true>(
-            lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt, sa_stride_m, sa_stride_k, grouped_layout, 0, row * tiles_n + n_idx, num_groups, 0,
-            Fp8TwoStages{a0, b0, a1, b1});
-    };
-    auto flat_tile = [&](int row, int n_idx) {
-        fp8_gemm_tile<SHAPE_N, SHAPE_K, 128, BLOCK_N, GemmType::GroupedContiguous, FLAT_STAGES, 1, true, true>(
-            lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt, sa_stride_m, sa_stride_k, grouped_layout, 0, row * tiles_n + n_idx, num_groups, 0,
-            Fp8TwoStages{nullptr, nullptr, nullptr, nullptr}, nullptr, nullptr, pool);
-    };
-    const int mode = two_group_rows * 20 < tall_rows ? 0 : (two_group_rows * 4 <= tall_rows ? 1 : 2);
-    // the rows that hold one group (or one group and padding), as a grid of their own (mode 1)
-    XcdTileScheduler<> whole((tall_rows - two_group_rows) * 256, N, 256, BLOCK_N);
-    whole.fit_bands_to_groups((tall_rows - two_group_rows) / max(num_groups, 1));
-    XcdTileScheduler<> flat(m, N, 128, BLOCK_N);
-    flat.fit_bands_to_groups(flat.tiles_m / max(num_groups, 1));
-    const ContiguousSlots two_pass_first(m, N, 256, BLOCK_N, num_groups, two_group_rows);
-    const int whole_slots = whole.grid_size();
-    const int slots = mode == 0 ? int(ContiguousSlots::num_slots(m, N, 256, BLOCK_N))
-                                : (mode == 1 ? whole_slots + 2 * two_group_rows * tiles_n : flat.grid_size());
+    const int blocks = m / 128, tiles_n = ceil_div(N, BLOCK_N);
+    int tall_rows = 0, flat_rows = 0, odd = 0;
+    for (int c = 0; c < ceil_div(blocks, kWaveSize); ++c) {
+        const ContiguousTileStarts starts = contiguous_tile_starts(grouped_layout, blocks, c, lane, odd);
+        tall_rows += __popcll(starts.tall);
+        flat_rows += __popcll(starts.flat);
+    }
+    XcdTileScheduler<> tall(tall_rows * 256, N, 256, BLOCK_N), flat(flat_rows * 128, N, 128, BLOCK_N);
+    tall.fit_bands_to_groups(tall_rows / max(num_groups, 1));
+    flat.fit_bands_to_groups(1);
+    const int tall_slots = tall.grid_size(), slots = tall_slots + flat.grid_size();
     // Either tile's code appears once (the compiler gives each copy of it its own registers, and four copies spill).
     auto run_slot = [&](int slot) {
-        TileCoord t{0, 0, false};       // of the 256-row grid, or of the 128-row grid when `half_tile`
-        bool half_tile = false;
-        if (mode == 0) {
-            t = two_pass_first.tile_of(slot);
-            if (t.valid && two_group_rows) t.m_idx = contiguous_row_at(grouped_layout, m, tall_rows, two_group_rows, t.m_idx, lane);
-        } else if (mode == 2) {
-            t = flat.tile_of(slot);
-            half_tile = true;
-        } else if (slot < whole_slots) {
-            t = whole.dealt_band_tile_of(slot);
-            if (t.valid) t.m_idx = contiguous_row_at(grouped_layout, m, tall_rows, two_group_rows, two_group_rows + t.m_idx, lane);
-        } else {
-            const int h = slot - whole_slots, within = h % (2 * tiles_n);
-            t = TileCoord{2 * contiguous_row_at(grouped_layout, m, tall_rows, two_group_rows, h / (2 * tiles_n), lane) + (within & 1), within / 2, true};
-            half_tile = true;
-        }
+        const bool is_tall = slot < tall_slots;
+        const TileCoord t = is_tall ? tall.dealt_band_tile_of(slot) : flat.dealt_band_tile_of(slot - tall_slots);
         if (!t.valid) return;
-        if (half_tile) flat_tile(t.m_idx, t.n_idx);
-        else tall_tile(t.m_idx, t.n_idx);
+        const int tile = contiguous_block_at(grouped_layout, blocks, is_tall, t.m_idx, lane) * tiles_n + t.n_idx;
+        if (is_tall)
+            fp8_gemm_tile<SHAPE_N, SHAPE_K, 256, BLOCK_N, GemmType::GroupedContiguous, 2, 1, false, true>(
+                lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt, sa_stride_m, sa_stride_k, grouped_layout, 0, tile, num_groups, 0,
+                Fp8TwoStages{a0, b0, a1, b1, b2});
+        else
+            fp8_gemm_tile<SHAPE_N, SHAPE_K, 128, BLOCK_N, GemmType::GroupedContiguous, FLAT_STAGES, 1, true, true>(
+                lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt, sa_stride_m, sa_stride_k, grouped_layout, 0, tile, num_groups, 0,
+                Fp8TwoStages{}, nullptr, nullptr, pool);
     };
     const int grid = gridDim.x;
     // a workgroup per slot (no cap): the tile without a loop around it
@@ -1012,7 +951,7 @@ fp8_gemm_split_k_kernel(const uint8_t* __restrict__ lhs, const float* __restrict
                         float* __restrict__ partials, unsigned* __restrict__ counters) {
     fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, GemmType::Normal, STAGES, SPLIT_K>(
         lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt, sa_stride_m, sa_stride_k, nullptr, 0, int(blockIdx.x), 1, 0,
-        Fp8TwoStages{nullptr, nullptr, nullptr, nullptr}, partials, counters);
+        Fp8TwoStages{}, partials, counters);
 }
 
 // Host side of the kernel, shaped after the class the reference's JIT template instantiates
@@ -1048,6 +987,10 @@ public:
                                   const int* grouped_layout, int num_groups, int m, int n, int k, hipStream_t stream,
                                   int num_sms = 0, int expected_m = 0) {
         static_assert(kGemmType != GemmType::Normal);
+        if constexpr (kGemmType == GemmType::GroupedContiguous && BLOCK_M == 256)
+            return run_grouped_rows_on_device(out, lhs, lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k, rhs, rhs_scales, grouped_layout,
+                                              num_groups, m, n, k, stream, num_sms);
+        else {
         if (m == 0 || n == 0 || num_groups == 0) return hipSuccess;
         if (m < 0 || n < 0 || k <= 0 || num_groups < 0 || (n % 4) != 0 || (k % 128) != 0) return hipErrorInvalidValue;
         if ((SHAPE_N && n != int(SHAPE_N)) || (SHAPE_K && k != int(SHAPE_K))) return hipErrorInvalidValue;
@@ -1062,7 +1005,7 @@ public:
         const XcdTileScheduler<> sched(m, n, BLOCK_M, BLOCK_N);
         const uint64_t slots = kGemmType == GemmType::GroupedMasked
                                    ? uint64_t(MaskedSlots(num_groups, m, n, BLOCK_M, BLOCK_N, expected_m).num_slots())
-                                   : (BLOCK_M == 256 ? uint64_t(ContiguousSlots::num_slots(m, n, BLOCK_M, BLOCK_N)) : uint64_t(sched.grid_size()));
+                                   : uint64_t(sched.grid_size());
         if (slots >= kOutOfRange) return hipErrorInvalidValue;
         const int grid = capped_grid(int(slots), num_sms, device_cu_count());
         hipLaunchKernelGGL((fp8_gemm_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, int(kNumStages)>), dim3(grid),
@@ -1071,15 +1014,16 @@ public:
                            lhs_scales_stride_m, lhs_scales_stride_k, grouped_layout, lhs_scales_stride_g, int(slots), num_groups,
                            expected_m);
         return hipGetLastError();
+        }
     }
 
-    // The contiguous layout with the tile height chosen on the device, tile row by tile row (fp8_gemm_contiguous_rows_kernel):
-    // 256 x BLOCK_N tiles where a tile row holds one group, 128 x BLOCK_N where it holds two. Arguments as run_grouped.
+    // The contiguous layout on tiles that follow the groups (fp8_gemm_contiguous_rows_kernel): 256 x BLOCK_N tiles, and a
+    // 128 x BLOCK_N tile for the last block of a group with an odd number of them. Arguments as run_grouped.
     static hipError_t run_grouped_rows_on_device(__hip_bfloat16* out, const void* lhs, const float* lhs_scales, int lhs_scales_stride_m,
                                                  int lhs_scales_stride_k, const void* rhs, const float* rhs_scales,
                                                  const int* grouped_layout, int num_groups, int m, int n, int k, hipStream_t stream,
                                                  int num_sms = 0) {
-        static_assert(kGemmType == GemmType::GroupedContiguous && BLOCK_M == 256 && kNumStages == 2);
+        static_assert(kGemmType == GemmType::GroupedContiguous && BLOCK_M == 256 && BLOCK_N >= 160 && kNumStages == 2);
         if (m == 0 || n == 0 || num_groups == 0) return hipSuccess;
         if (m < 0 || n < 0 || k <= 0 || num_groups < 0 || (n % 4) != 0 || (k % 128) != 0 || (m % 128) != 0) return hipErrorInvalidValue;
         if ((SHAPE_N && n != int(SHAPE_N)) || (SHAPE_K && k != int(SHAPE_K))) return hipErrorInvalidValue;
@@ -1087,7 +1031,7 @@ public:
         if (!out || !lhs || !lhs_scales || !rhs || !rhs_scales || !grouped_layout) return hipErrorInvalidValue;
         const uint64_t m_pad = uint64_t(ceil_div<uint32_t>(m, BLOCK_M)) * BLOCK_M, n_pad = uint64_t(ceil_div<uint32_t>(n, BLOCK_N)) * BLOCK_N;
         if (m_pad * k >= kOutOfRange || n_pad * k >= kOutOfRange || uint64_t(BLOCK_M) * n * 2 >= kOutOfRange) return hipErrorInvalidValue;
-        // whole tiles (rounded up to the 8 XCDs) plus two half tiles for every other tile: at most the tiles of the 128-row tiling + 8
+        // tall and flat tiles, each rounded up to the 8 XCDs: at most the tiles of the 128-row tiling + 8
         const long long slots = (long long)XcdTileScheduler<>(m, n, 128, BLOCK_N).grid_size() + kNumXCD;
         if (slots >= kOutOfRange) return hipErrorInvalidValue;
         const int grid = capped_grid(int(slots), num_sms, device_cu_count());

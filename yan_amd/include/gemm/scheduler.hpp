@@ -189,9 +189,10 @@ struct MaskedSlots {
     }
 };
 
-// Slot numbering of the contiguous layout on 256-row tiles. A tile row whose two 128-row halves belong to two groups makes
+// A slot numbering of the contiguous layout on a fixed grid of 256-row tiles. (The kernels of this directory place their tall
+// tiles along the groups instead, fp8_gemm_contiguous_rows_kernel, and have no tile of two groups.) A tile row whose two 128-row halves belong to two groups makes
 // two passes over K and takes about half as long again as the others; started last, one of them ends alone after everyone
-// else. `two_group_rows` of the `tiles_m` rows are of that kind (the kernel counts them in the caller's layout; the host
+// else. `two_group_rows` of the `tiles_m` rows are of that kind (a kernel counts them in the caller's layout; the host
 // does not know them and launches `num_slots()` workgroups whatever their number). Their tiles come first in every XCD's
 // share of the slots and are dealt to the XCDs one by one, so that every XCD gets as many (an XCD runs its own slots, and
 // a patch of 32 slow tiles would fall to one of them); the other rows follow in band order dealt out in patches of 32.

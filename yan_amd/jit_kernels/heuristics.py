@@ -94,29 +94,25 @@ def get_fp8_num_stages(block_m: int, block_n: int) -> int:
 
 def get_best_grouped_fp8_config(m: int, n: int, k: int, num_cus: int, groups: int = 1, m_alignment: int = 0,
                                 groups_in_m: int = 1) -> Tuple[int, int]:
-    """Tile of a grouped FP8 GEMM, among the tiles 64, 128 or 256 columns wide. Contiguous layout: `m` is the total row count, `m_alignment` the padding of every
-    group and `groups_in_m` the number of groups sharing the rows: a tile of up to `m_alignment` rows must divide it;
-    the 256-row tile, which handles a group boundary in its middle with a second pass over K, is offered when groups
-    average at least 1024 rows. Masked layout: `m` is the expected row count of one group and `groups` multiplies
-    the tile count."""
+    """Tile of a grouped FP8 GEMM, among the tiles 64, 128 or 256 columns wide. Contiguous layout: `m` is the total row count and
+    `m_alignment` the padding of every group, which the tile's rows must divide (taller tiles belong to the kernel that places
+    them on the device, `get_contiguous_rows_on_device`). Masked layout: `m` is the expected row count of one group and `groups`
+    multiplies the tile count. `groups_in_m` (the groups sharing the rows of the contiguous layout) does not matter here."""
     def allowed(bm):
-        if m_alignment == 0 or m_alignment % bm == 0:
-            return True
-        return bm == 2 * m_alignment and m >= 1024 * groups_in_m
+        return m_alignment == 0 or m_alignment % bm == 0
     table = {t: c for t, c in _FP8_TILES.items() if t[1] in (64, 128, 256) and allowed(t[0])}
     return rank_tiles(max(m, 1), n, num_cus, table, groups)[0][1]
 
 
 def get_contiguous_rows_on_device(m: int, n: int, k: int, num_cus: int, groups_in_m: int) -> bool:
-    """Whether a contiguous grouped GEMM runs the kernel that decides on the device what its 256-row tiles do about group
-    boundaries (`fp8_gemm_contiguous_rows_kernel`): groups of 256 to 2047 rows on average for which the cost table, with
-    256-row tiles allowed, takes 256 x 256 tiles. Which tile rows hold two groups stands in `m_indices`: with none (every
-    boundary on a multiple of 256 rows) 256-row tiles are 13-17 % faster than 128 x 256 ones (16 groups of 512 rows x 4096 x
-    7168: 225 against 264 us), with a few the kernel runs those rows as 128-row tiles at the end of the launch (8 groups
-    of 896 and 1152 rows: 230 against 250 us with two-pass tiles), with many it runs 128-row tiles throughout. Longer groups keep
-    the fixed 256-row tiles (within 2 % either way, and the fixed kernel is the faster when no row holds two groups). Same
-    rule as `rows_on_device` in yan_amd/csrc/yan_gemm_capi.hip."""
-    if groups_in_m <= 0 or not 256 * groups_in_m <= m < 2048 * groups_in_m:
+    """Whether a contiguous grouped GEMM runs the kernel whose tiles follow the groups (`fp8_gemm_contiguous_rows_kernel`: 256 x
+    256 tiles and, for the odd block of a group, 128 x 256): groups that average a block of 128 rows or more, for which the
+    cost table, with 256-row tiles allowed, takes 256 x 256. Against 128 x 256 tiles and 256-row tiles on a fixed grid, which ran
+    two passes over K where a tile held two groups: 16 groups of 128 to 768 rows x 4096 x 7168 220 -> 197 us, 4 of about 2500 290 ->
+    276, 7 of about 2300 x 2112 x 5120 210 -> 197, 64 of about 130 x 7168 x 2048 185 -> 172; level (0.5 %) for 4 of 8192 and
+    2 % behind at one shape tried (32 of about 190 x 4096 x 4096). Same rule as `rows_on_device` in
+    yan_amd/csrc/yan_gemm_capi.hip."""
+    if groups_in_m <= 0 or m < 128 * groups_in_m:
         return False
     table = {t: c for t, c in _FP8_TILES.items() if t[1] in (64, 128, 256) and t[0] in (64, 128, 256)}
     return rank_tiles(m, n, num_cus, table)[0][1] == (256, 256)

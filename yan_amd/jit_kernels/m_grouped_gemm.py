@@ -37,7 +37,7 @@ __return_code = static_cast<int>(GemmType::run_grouped(out, lhs, lhs_scales, lhs
                                                        kNumGroups, m, N, K, stream, num_sms, expected_m));
 """
 
-# Contiguous groups of a few hundred rows: the kernel that holds 256 x 256 and 128 x 256 tiles and picks on the device
+# The contiguous layout on tiles that follow the groups: the kernel that holds 256 x 256 and 128 x 256 tiles and places them on the device
 # (Gemm::run_grouped_rows_on_device in gemm/fp8_gemm.hpp); same keys and arguments.
 rows_on_device_template = template.replace(
     """GemmType::run_grouped(out, lhs, lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k,
