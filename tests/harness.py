@@ -215,6 +215,10 @@ REFERENCE_FLOAT_TEST_SHAPES = [(m, n, k) for m in (128, 4096)
 # 64x64 with K split over the waves; 128x64, 128x128, 128x256, 256x256)
 FLOAT_TEST_SHAPES = [(128, 64, 16), (128, 64, 1), (128, 192, 17), (256, 320, 100), (384, 1024, 260), (128, 24576, 40),
                      (512, 4096, 40), (256, 32768, 24), (4096, 32768, 8)]
+# fp32 problems that split K: (m, n, k) -> (BLOCK_M, BLOCK_N, parts), every tile of the plans
+FLOAT_SPLIT_K_SHAPES = {(128, 64, 2050): (32, 32, 7), (256, 320, 3001): (32, 32, 3), (384, 320, 3001): (32, 64, 4), (128, 576, 4099): (32, 64, 7),
+                        (1024, 320, 2050): (64, 64, 3), (640, 320, 7168): (64, 64, 5), (640, 1088, 4099): (128, 64, 3),
+                        (128, 2112, 9001): (128, 64, 7)}
 FP8_TEST_SHAPES = [
     (4096, 7168, 7168), (64, 4096, 7168), (16384, 16384, 16384),
     (64, 256, 384), (512, 1024, 1024), (1, 128, 128), (63, 192, 256), (129, 320, 128), (300, 96, 640),
@@ -430,6 +434,10 @@ def jit_kernels_in_use(num_cus: int = 256):
         name, keys, space, arg_defs, code_template = gemm.fp8_tuning_plan(m, n, k, num_cus, True)
         for extra in space:
             add(name, arg_defs, gemm.includes, code_template, {**keys, **extra})
+    for m, n, k in list(FLOAT_SPLIT_K_SHAPES) + REFERENCE_FLOAT_TEST_SHAPES + FLOAT_TEST_SHAPES:
+        plan = simple_gemm.float_split_k_plan(m, n, k, num_cus)
+        if plan is not None:
+            add(plan[0], plan[2], simple_gemm.includes, simple_gemm.split_k_template, plan[1])
     for kind in ('per_token', 'per_block'):
         for dtype in (torch.bfloat16, torch.float32):
             name, keys, arg_defs, code_template = fp8_cast.cast_kernel_plan(kind, dtype)

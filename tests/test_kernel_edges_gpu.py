@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import oracle
+import yan_amd as yan
 import harness as testing
 from yan_amd import jit
 
@@ -46,3 +47,30 @@ def test_contiguous_tiles_follow_the_groups(rows, n, k, pad_blocks):
     assert torch.equal(results[0], results[1])
     assert torch.equal(results[0][~real], out[~real])                   # padding blocks keep what they held
     assert _fp8_close(results[0][real].float(), ref[real])
+
+
+@pytest.mark.parametrize('m,n,k', testing.FLOAT_SPLIT_K_SHAPES)
+def test_float_split_k_matches_the_oracle_and_repeats(m, n, k):
+    """gemm_cute_split_k through the entry: k that is no multiple of a k-tile or of the parts, last parts shorter than the
+    others, tiles past n; alpha and beta, NaN in c with beta = 0; the same bits twice, counters back at zero."""
+    from yan_amd.jit_kernels import simple_gemm, split_k
+    _announce('fp32 split-K', m, n, k)
+    name, keys, _ = simple_gemm.float_split_k_plan(m, n, k, 256)
+    assert (keys['BLOCK_M'], keys['BLOCK_N'], keys['SPLIT_K']) == testing.FLOAT_SPLIT_K_SHAPES[(m, n, k)]
+    a, b, c = testing.make_float_case(m, n, k, seed=13, device='cuda')
+    start = torch.randn(m, n, generator=torch.Generator().manual_seed(14))
+    ad, bd = a.double(), b.double()
+    # every product and every sum of the at most k + 8 in a row rounds once, relative to the sum of magnitudes
+    bound = (k + 8) * 2.0 ** -24 * (ad.abs() @ bd.abs().t() + start.abs().double().cuda()) * 2
+    for alpha, beta in ((1.0, 0.0), (-0.5, 2.0)):
+        results = []
+        for _ in range(2):
+            c.copy_(start if beta else torch.full_like(c, float('nan')))
+            yan.gemm_float_nt(a, b, c, alpha=alpha, beta=beta)
+            results.append(c.clone())
+        want = alpha * (ad @ bd.t()) + (beta * start.double().cuda() if beta else 0.0)
+        assert torch.equal(results[0], results[1])
+        assert bool(((results[0].double() - want).abs() <= bound).all())
+        assert ((results[0].double() - want).norm() / want.norm()).item() < 5e-6
+    workspace, _ = split_k.split_k_workspace(c.device, torch.cuda.current_stream().cuda_stream)
+    assert int(workspace[:split_k.SPLIT_K_COUNTER_BYTES].view(torch.int32).abs().sum()) == 0

@@ -15,8 +15,12 @@
 //     accumulators are VN consecutive n of one m, one 16-byte access in C;
 //   * tiles below 128 rows (64 x 64, 32 x 64, 32 x 32) are for problems with too few outputs to give every CU a
 //     large tile: there the four waves split K instead of the tile (each takes a quarter of every 64-deep k-tile
-//     over the whole tile) and their partial sums are added through LDS in a fixed order at the end, so results do
-//     not depend on timing;
+//     over the whole tile) and their partial sums meet in LDS at the end, where every wave adds up and stores a quarter of the
+//     tile, in a fixed order, so results do not depend on timing (against one wave doing it all, on 64 x 64 tiles:
+//     4096 x 1024 x 512 49 -> 42 us, 4096 x 7168 x 512 337 -> 290);
+//   * problems with a long K and a number of tiles that shares badly over the CUs split K over SPLIT_K workgroups per tile
+//     (gemm_cute_split_k), which meet in a workspace as those of the other GEMMs do; the matrix cores bound these problems at
+//     the 82-92 % of their rate the chip sustains, and what the split buys is an even share (128 x 2112 x 7168 57 -> 40 us);
 //   * rows past m / n are not written, k rows past the end read as zero: any m, n, k with m, n, ldA, ldB, ldC
 //     multiples of 4 and 16-byte aligned bases.
 // beta == 0 does not read C (the BLAS convention).
@@ -53,7 +57,7 @@ struct FloatTileConfig {
     // deeper ring).
     static constexpr int RING_BUDGET = (BLOCK_M == 32 || (BLOCK_M == 128 && BLOCK_N <= 128)) ? 72 * 1024 : 128 * 1024;
     static constexpr int MAX_STAGES = RING_BUDGET / STAGE_BYTES < 3 ? 3 : (RING_BUDGET / STAGE_BYTES < 8 ? RING_BUDGET / STAGE_BYTES : 8);
-    static_assert(K_SPLIT == 1 || 3 * VM * VN * 16 * 256 <= 3 * STAGE_BYTES, "partial sums of three waves fit the ring");
+    static_assert(K_SPLIT == 1 || 4 * VM * VN * 16 * 256 <= 3 * STAGE_BYTES, "partial sums of the four waves fit the ring");
 };
 
 template <int N> struct FloatVec;
@@ -66,12 +70,15 @@ __device__ __forceinline__ float vec_at(const typename FloatVec<N>::type& v, int
     if constexpr (N == 1) return v; else return v[i];
 }
 
-// The kernel keeps the reference kernel's name (simple_gemm.cuh:22) so that profiler filters written for it
-// (tests/test_simple.py:35 looks for 'gemm_cute') keep finding it.
-template <int BLOCK_M, int BLOCK_N, int STAGES>
-__global__ void __launch_bounds__(4 * kWaveSize)
-gemm_cute(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C,
-          int m, int n, int k, int ldA, int ldB, int ldC, float alpha, float beta) {
+// One workgroup's share of the problem: an output tile, or with SPLIT_K > 1 the k-tiles of one of its SPLIT_K parts.
+// Launch slot s is part s / tile slots of tile slot s % tile slots: the parts of a tile run on one XCD (the tile slots are a
+// multiple of 8) and the parts that are dispatched first are the first ones of every tile. The parts meet in `partials`
+// (meet_partials in tile_io.hpp): the last to arrive adds them up in the order of their K ranges.
+template <int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K>
+__device__ __forceinline__ void
+float_gemm_body(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C,
+                int m, int n, int k, int ldA, int ldB, int ldC, float alpha, float beta,
+                [[maybe_unused]] float* __restrict__ partials, [[maybe_unused]] unsigned* __restrict__ counters) {
     using Cfg = FloatTileConfig<BLOCK_M, BLOCK_N>;
     constexpr int VM = Cfg::VM, VN = Cfg::VN, BLOCK_K = Cfg::BLOCK_K, OPS = Cfg::OPS;
     static_assert(STAGES >= 3 && STAGES <= Cfg::MAX_STAGES && (STAGES - 2) * OPS <= 63);
@@ -79,17 +86,23 @@ gemm_cute(const float* __restrict__ A, const float* __restrict__ B, float* __res
     using VecN = typename FloatVec<VN>::type;
 
     const XcdTileScheduler<> sched(m, n, BLOCK_M, BLOCK_N);
-    const TileCoord tile = sched.tile_of(blockIdx.x);
+    const int tile_slots = SPLIT_K > 1 ? sched.grid_size() : 0;
+    const int split = SPLIT_K > 1 ? int(blockIdx.x) / tile_slots : 0, tile_slot = int(blockIdx.x) - split * tile_slots;
+    const TileCoord tile = sched.tile_of(tile_slot);
     if (!tile.valid) return;
+    // the k-tiles of this workgroup; k rows from k_end on read as zero
+    const int all_k_tiles = ceil_div(k, BLOCK_K), per = ceil_div(all_k_tiles, SPLIT_K);
+    const int kt_lo = min(split * per, all_k_tiles), kt_hi = min(kt_lo + per, all_k_tiles);
+    const int k_end = SPLIT_K > 1 ? min(k, kt_hi * BLOCK_K) : k;
     const int m0 = tile.m_idx * BLOCK_M, n0 = tile.n_idx * BLOCK_N;
 
     const int lane = get_lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
     const int wm = Cfg::K_SPLIT == 4 ? 0 : wave / Cfg::WAVES_N, wn = Cfg::K_SPLIT == 4 ? 0 : wave % Cfg::WAVES_N;
 
-    // Descriptors end with the last element of the last k-row, so every k-row past k reads as zero.
-    const __amdgpu_buffer_rsrc_t rsrc_a = make_rsrc(A, k > 0 ? (uint32_t(k - 1) * uint32_t(ldA) + uint32_t(m)) * 4u : 0u);
-    const __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(B, k > 0 ? (uint32_t(k - 1) * uint32_t(ldB) + uint32_t(n)) * 4u : 0u);
+    // Descriptors end with the last element of the last k-row, so every k-row past it reads as zero.
+    const __amdgpu_buffer_rsrc_t rsrc_a = make_rsrc(A, k_end > 0 ? (uint32_t(k_end - 1) * uint32_t(ldA) + uint32_t(m)) * 4u : 0u);
+    const __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(B, k_end > 0 ? (uint32_t(k_end - 1) * uint32_t(ldB) + uint32_t(n)) * 4u : 0u);
     // One copy instruction moves 1 KB of a stage: 1024 / (4 * BLOCK) consecutive k-rows of BLOCK floats each.
     constexpr int A_LANES = BLOCK_M / 4, B_LANES = BLOCK_N / 4;                 // lanes per k-row
     constexpr int A_ROWS = kWaveSize / A_LANES, B_ROWS = kWaveSize / B_LANES;   // k-rows per instruction
@@ -125,17 +138,16 @@ gemm_cute(const float* __restrict__ A, const float* __restrict__ B, float* __res
     const int frag_b = Cfg::A_BYTES + ((2 * first_kp + h) * BLOCK_N + wn * Cfg::WTN + VN * i) * 4;
 
     __shared__ __attribute__((aligned(1024))) uint8_t ring[STAGES * Cfg::STAGE_BYTES];
-    const int num_k_tiles = ceil_div(k, BLOCK_K);
 #pragma unroll
     for (int t = 0; t < STAGES - 1; ++t)
 #pragma unroll
-        for (int d = 0; d < OPS; ++d) copy_op(d, t, ring + t * Cfg::STAGE_BYTES);
+        for (int d = 0; d < OPS; ++d) copy_op(d, kt_lo + t, ring + t * Cfg::STAGE_BYTES);
 
     // Every wave issues OPS copies per k-tile in the same order, so "k-tile kt has landed" is "at most
     // (STAGES - 2) * OPS of my copies are outstanding"; the copies of k-tile kt + STAGES - 1 go to the stage consumed
     // in iteration kt - 1, which every wave has left once it is past the barrier.
     int st = 0;
-    for (int kt = 0; kt < num_k_tiles; ++kt) {
+    for (int kt = kt_lo; kt < kt_hi; ++kt) {
         __builtin_amdgcn_s_waitcnt(waitcnt_imm((STAGES - 2) * OPS, kNoWaitLgkm));
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
@@ -163,57 +175,97 @@ gemm_cute(const float* __restrict__ A, const float* __restrict__ B, float* __res
         st = st + 1 == STAGES ? 0 : st + 1;
     }
 
+    // What a wave takes through the rest: QUADS vectors of four accumulator registers per MFMA (t, u), the registers
+    // 4 * (first_quad + q) .. + 3. With K split over the waves their partial sums meet in LDS (register-major, lane-minor: no
+    // bank conflicts) and every wave adds up one quarter of the registers, in the order of the waves.
+    constexpr int QUADS = Cfg::K_SPLIT == 4 ? 1 : 4;
+    const int first_quad = Cfg::K_SPLIT == 4 ? wave : 0;
+    f32x4 sums[VM * VN * QUADS];
+    auto sum_of = [&](int t, int u, int q) -> f32x4& { return sums[(t * VN + u) * QUADS + q]; };
     if constexpr (Cfg::K_SPLIT == 4) {
-        // Partial sums of waves 1..3 go through LDS (register-major, lane-minor: no bank conflicts) and wave 0 adds
-        // them in the order 1, 2, 3. The ring is free once nobody reads it and no copy is still on its way into it.
-        constexpr int REGS = VM * VN * 16;
+        // the ring is free once nobody reads it and no copy is still on its way into it
         wait_for_copies();
         __syncthreads();
-        float* partial = reinterpret_cast<float*>(ring);
-        if (wave != 0) {
+        f32x4* partial = reinterpret_cast<f32x4*>(ring);         // [wave][quad][t, u][lane]
+        constexpr int QUAD_VECS = VM * VN * kWaveSize, WAVE_VECS = 4 * QUAD_VECS;
 #pragma unroll
-            for (int t = 0; t < VM; ++t)
+        for (int t = 0; t < VM; ++t)
 #pragma unroll
-                for (int u = 0; u < VN; ++u)
+            for (int u = 0; u < VN; ++u)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        partial[((wave - 1) * REGS + (t * VN + u) * 16 + r) * kWaveSize + lane] = acc[t][u][r];
-        }
+                for (int q = 0; q < 4; ++q)
+                    partial[wave * WAVE_VECS + q * QUAD_VECS + (t * VN + u) * kWaveSize + lane] =
+                        f32x4{acc[t][u][4 * q], acc[t][u][4 * q + 1], acc[t][u][4 * q + 2], acc[t][u][4 * q + 3]};
         __syncthreads();
-        if (wave != 0) return;
 #pragma unroll
-        for (int w = 0; w < 3; ++w)
+        for (int t = 0; t < VM; ++t)
 #pragma unroll
-            for (int t = 0; t < VM; ++t)
+            for (int u = 0; u < VN; ++u) {
+                const f32x4* mine = partial + wave * QUAD_VECS + (t * VN + u) * kWaveSize + lane;
+                sum_of(t, u, 0) = ((mine[0] + mine[WAVE_VECS]) + mine[2 * WAVE_VECS]) + mine[3 * WAVE_VECS];
+            }
+    } else {
 #pragma unroll
-                for (int u = 0; u < VN; ++u)
+        for (int t = 0; t < VM; ++t)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        acc[t][u][r] += partial[(w * REGS + (t * VN + u) * 16 + r) * kWaveSize + lane];
+            for (int u = 0; u < VN; ++u)
+#pragma unroll
+                for (int q = 0; q < QUADS; ++q)
+                    sum_of(t, u, q) = f32x4{acc[t][u][4 * q], acc[t][u][4 * q + 1], acc[t][u][4 * q + 2], acc[t][u][4 * q + 3]};
     }
+    if constexpr (SPLIT_K > 1)
+        if (!meet_partials<SPLIT_K, Cfg::NUM_WAVES, VM * VN * QUADS>([&](int v) -> f32x4& { return sums[v]; }, partials, counters,
+                                                                     tile_slot, split, wave, lane)) return;
 
     // Epilogue: register r of an atom is MFMA row 8 * (r / 4) + 4 * h + r % 4 of MFMA column i; MFMA (t, u) holds
     // slab row VM * mfma_row + t and slab column VN * mfma_col + u.
     const int n_lane = n0 + wn * Cfg::WTN + VN * i;
     if (n_lane >= n) return;                                   // n % 4 == 0 and VN | 4: a lane's VN columns exist together
+    auto row_of = [&](int q, int r, int t) { return m0 + wm * Cfg::WTM + VM * (8 * (first_quad + q) + 4 * h + r) + t; };
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int mfma_row = 8 * (r / 4) + 4 * h + r % 4;
+    for (int q = 0; q < QUADS; ++q) {
+        // what C holds, 4 * VM rows at a time (rows past m read the last one again): a load behind every row's branch waits for
+        // memory once per row (beta = 1: 1024^3 28.6 -> 19.8 us, 4096 x 7168 x 512 257 -> 231, beta = 0 19.4 and 221)
+        VecN held[4][VM];
+        if (beta != 0.f) {
 #pragma unroll
-        for (int t = 0; t < VM; ++t) {
-            const int mm = m0 + wm * Cfg::WTM + VM * mfma_row + t;
-            if (mm >= m) continue;
-            VecN* dst = reinterpret_cast<VecN*>(C + size_t(mm) * ldC + n_lane);
-            VecN v;
-            if constexpr (VN == 1) v = alpha * acc[t][0][r];
-            else {
+            for (int r = 0; r < 4; ++r)
 #pragma unroll
-                for (int u = 0; u < VN; ++u) v[u] = alpha * acc[t][u][r];
-            }
-            if (beta != 0.f) v += beta * *dst;
-            *dst = v;
+                for (int t = 0; t < VM; ++t) held[r][t] = *reinterpret_cast<const VecN*>(C + size_t(min(row_of(q, r, t), m - 1)) * ldC + n_lane);
         }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int t = 0; t < VM; ++t) {
+                const int mm = row_of(q, r, t);
+                if (mm >= m) continue;
+                VecN v;
+                if constexpr (VN == 1) v = alpha * sum_of(t, 0, q)[r];
+                else {
+#pragma unroll
+                    for (int u = 0; u < VN; ++u) v[u] = alpha * sum_of(t, u, q)[r];
+                }
+                if (beta != 0.f) v += beta * held[r][t];
+                *reinterpret_cast<VecN*>(C + size_t(mm) * ldC + n_lane) = v;
+            }
     }
+}
+
+// The kernel keeps the reference kernel's name (simple_gemm.cuh:22) so that profiler filters written for it
+// (tests/test_simple.py:35 looks for 'gemm_cute') keep finding it.
+template <int BLOCK_M, int BLOCK_N, int STAGES>
+__global__ void __launch_bounds__(4 * kWaveSize)
+gemm_cute(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C,
+          int m, int n, int k, int ldA, int ldB, int ldC, float alpha, float beta) {
+    float_gemm_body<BLOCK_M, BLOCK_N, STAGES, 1>(A, B, C, m, n, k, ldA, ldB, ldC, alpha, beta, nullptr, nullptr);
+}
+
+template <int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K>
+__global__ void __launch_bounds__(4 * kWaveSize, (STAGES * FloatTileConfig<BLOCK_M, BLOCK_N>::STAGE_BYTES <= 80 * 1024 ? 2 : 1))
+gemm_cute_split_k(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C,
+                  int m, int n, int k, int ldA, int ldB, int ldC, float alpha, float beta,
+                  float* __restrict__ partials, unsigned* __restrict__ counters) {
+    float_gemm_body<BLOCK_M, BLOCK_N, STAGES, SPLIT_K>(A, B, C, m, n, k, ldA, ldB, ldC, alpha, beta, partials, counters);
 }
 
 // Arguments the fp32 launcher checks before touching the GPU.
@@ -238,6 +290,27 @@ inline hipError_t launch_float_nt(int m, int n, int k, float alpha, const float*
     const XcdTileScheduler<> sched(m, n, BLOCK_M, BLOCK_N);
     hipLaunchKernelGGL((gemm_cute<BLOCK_M, BLOCK_N, STAGES>), dim3(sched.grid_size()), dim3(4 * kWaveSize), 0, stream,
                        A, B, C, m, n, k, ldA, ldB, ldC, alpha, beta);
+    return hipGetLastError();
+}
+
+// K split SPLIT_K ways over as many workgroups per tile: problems whose tiles leave compute units idle, or fill a last round
+// badly, and whose K is long. `workspace` as for the other split-K launchers (kSplitKCounterBytes of counters that are zero
+// before and after every launch, then the partial sums; launches that share it must not overlap).
+template <int BLOCK_M, int BLOCK_N, int SPLIT_K, int STAGES = FloatTileConfig<BLOCK_M, BLOCK_N>::MAX_STAGES>
+inline hipError_t launch_float_nt_split_k(int m, int n, int k, float alpha, const float* A, int ldA, const float* B, int ldB,
+                                          float beta, float* C, int ldC, hipStream_t stream, void* workspace, size_t workspace_bytes) {
+    static_assert(SPLIT_K > 1);
+    using Cfg = FloatTileConfig<BLOCK_M, BLOCK_N>;
+    if (m == 0 || n == 0) return hipSuccess;
+    if (hipError_t e = check_float_args(m, n, k, A, ldA, B, ldB, C, ldC, BLOCK_M, BLOCK_N); e != hipSuccess) return e;
+    if (!workspace) return hipErrorInvalidValue;
+    const XcdTileScheduler<> sched(m, n, BLOCK_M, BLOCK_N);
+    const uint64_t slots = uint64_t(sched.grid_size());
+    if (slots * Cfg::NUM_WAVES * 4 > kSplitKCounterBytes) return hipErrorInvalidValue;
+    if (kSplitKCounterBytes + slots * SPLIT_K * BLOCK_M * BLOCK_N * 4 > workspace_bytes) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((gemm_cute_split_k<BLOCK_M, BLOCK_N, STAGES, SPLIT_K>), dim3(uint32_t(slots * SPLIT_K)), dim3(4 * kWaveSize), 0, stream,
+                       A, B, C, m, n, k, ldA, ldB, ldC, alpha, beta,
+                       reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kSplitKCounterBytes), static_cast<unsigned*>(workspace));
     return hipGetLastError();
 }
 

@@ -280,3 +280,37 @@ def get_best_float_config(m: int, n: int, num_cus: int) -> Tuple[int, int]:
         if best_cost is None or cost < best_cost:
             best, best_cost = (bm, bn), cost
     return best
+
+
+# Split-K of the fp32 GEMM: microseconds a compute unit spends on 1024 k-rows of a tile under sustained load (measured with one
+# and with two workgroups per unit, operands cycling: 82-92 % of the matrix rate). Plans use the first four.
+_FLOAT_US_PER_1024_K = {(32, 32): 4.7, (32, 64): 8.7, (64, 64): 16.7, (128, 64): 33.1, (128, 128): 64.0, (128, 256): 122.0, (256, 256): 235.0}
+_FLOAT_BLOCK_K = {(32, 32): 64, (32, 64): 64, (64, 64): 64, (128, 64): 32}
+FLOAT_SPLIT_K_FACTORS = (2, 3, 4, 5, 6, 7, 8)
+
+
+def get_split_k_float_config(m: int, n: int, k: int, num_cus: int) -> Optional[Tuple[int, int, int]]:
+    """(BLOCK_M, BLOCK_N, SPLIT_K) when the fp32 GEMM should split K over SPLIT_K workgroups per tile, else None. The matrix cores
+    bound this GEMM, so what splitting buys is an even share of the work: 128 x 2112 has 132 tiles of 32 x 64 for 256 compute
+    units, and 462 parts of 64 x 64 tiles in seven are two almost full rounds. Modelled time of a plan: rounds x the tile's time
+    for its k-rows + 6 us (launch, first copies, the meeting) + 12.5 ns per KB of partial sums the last part reads; taken when it
+    is below 0.88 of the unsplit pick's. Measured (unsplit -> plan, operands cycling): 128 x 2112 x 7168 57 -> 40 us,
+    256 x 2112 x 7168 86 -> 67, 128 x 256 x 8192 35 -> 11. On 19 shapes swept with four tiles and every factor the plan is within 3 %
+    of the fastest measured; shapes whose best plan gains less than 5 % (128 x 4096 x 7168 64 -> 62) stay unsplit."""
+    if m <= 0 or n <= 0 or k <= 0:
+        return None
+    tile = get_best_float_config(m, n, num_cus)
+    base = ceil_div(ceil_div(m, tile[0]) * ceil_div(n, tile[1]), num_cus) * _FLOAT_US_PER_1024_K[tile] * k / 1024 + 3.5
+    best, best_plan = 0.88 * base, None
+    for (bm, bn), block_k in _FLOAT_BLOCK_K.items():
+        tiles, k_tiles = ceil_div(m, bm) * ceil_div(n, bn), ceil_div(k, block_k)
+        slots = ceil_div(tiles, 8) * 8
+        for split in FLOAT_SPLIT_K_FACTORS:
+            # 16 MB of partial sums, four counters per tile slot in 16 KB, at least 256 k-rows per part
+            part = ceil_div(k_tiles, split) * block_k
+            if slots * split * bm * bn * 4 > 1 << 24 or slots > 1024 or part < 256:
+                continue
+            t = ceil_div(tiles * split, num_cus) * _FLOAT_US_PER_1024_K[(bm, bn)] * part / 1024 + 6 + split * bm * bn * 4 / 1024 * 0.0125
+            if t < best:
+                best, best_plan = t, (bm, bn, split)
+    return best_plan

@@ -11,7 +11,8 @@ import functools
 
 import torch
 
-from .heuristics import get_best_float_config
+from .heuristics import get_best_float_config, get_split_k_float_config
+from .split_k import SPLIT_K_WORKSPACE_BYTES, split_k_launch_failed, split_k_workspace
 from .tuner import FrozenKeys, jit_tuner
 from .utils import current_raw_stream, get_num_sms
 
@@ -30,6 +31,22 @@ __return_code = static_cast<int>(gemm_nt<BLOCK_M, BLOCK_N>(m, n, k,
         stream));
 """
 
+# K split over SPLIT_K workgroups per tile; the parts meet in `workspace` (launch_float_nt_split_k in gemm/simple_gemm.hpp).
+split_k_template = """
+// Templated args from Python JIT call
+constexpr auto BLOCK_M = {BLOCK_M};
+constexpr auto BLOCK_N = {BLOCK_N};
+constexpr auto kSplitK = {SPLIT_K};
+
+__return_code = static_cast<int>(yan::launch_float_nt_split_k<BLOCK_M, BLOCK_N, kSplitK>(m, n, k,
+        alpha,
+        static_cast<float const*>(A), ldA,
+        static_cast<float const*>(B), ldB,
+        beta,
+        static_cast<float*>(C), ldC,
+        stream, workspace, workspace_bytes));
+"""
+
 arg_defs = (('m', int), ('n', int), ('k', int),
             ('alpha', float),
             ('A', torch.float), ('ldA', int),
@@ -37,6 +54,7 @@ arg_defs = (('m', int), ('n', int), ('k', int),
             ('beta', float),
             ('C', torch.float), ('ldC', int),
             ('stream', torch.cuda.Stream))
+split_k_arg_defs = arg_defs + (('workspace', torch.uint8), ('workspace_bytes', int))
 
 
 @functools.lru_cache(maxsize=None)
@@ -44,6 +62,17 @@ def float_kernel_plan(m: int, n: int, num_cus: int):
     """(name, keys, arg_defs) of the JIT kernel a call with these sizes uses; needs no GPU."""
     block_m, block_n = get_best_float_config(m, n, num_cus)
     return 'gemm_float_nt', FrozenKeys({'BLOCK_M': block_m, 'BLOCK_N': block_n}), arg_defs
+
+
+@functools.lru_cache(maxsize=None)
+def float_split_k_plan(m: int, n: int, k: int, num_cus: int):
+    """(name, keys, arg_defs) of the split-K kernel a call with these sizes uses, or None when K is not split
+    (`get_split_k_float_config`); needs no GPU."""
+    plan = get_split_k_float_config(m, n, k, num_cus)
+    if plan is None:
+        return None
+    block_m, block_n, split_k = plan
+    return 'gemm_float_nt_split_k', FrozenKeys({'BLOCK_M': block_m, 'BLOCK_N': block_n, 'SPLIT_K': split_k}), split_k_arg_defs
 
 
 def _leading_dim(x: torch.Tensor) -> int:
@@ -74,9 +103,19 @@ def gemm_float_nt(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor,
     stream = current_raw_stream()
     args = (m, n, k, float(alpha), a, ldA, b, ldB, float(beta), c, ldC, stream)
     name, keys, defs = float_kernel_plan(m, n, get_num_sms())
+    code_template, workspace_token = template, None
+    split = float_split_k_plan(m, n, k, get_num_sms())
+    if split is not None:
+        workspace, workspace_token = split_k_workspace(c.device, stream)
+        if workspace is not None:
+            name, keys, defs = split
+            code_template = split_k_template
+            args += (workspace, SPLIT_K_WORKSPACE_BYTES)
     runtime = jit_tuner.compile_and_tune(name=name, keys=keys, space=(), includes=includes,
-                                         arg_defs=defs, template=template, args=args)
+                                         arg_defs=defs, template=code_template, args=args)
     rc = runtime(*args)
+    if rc != 0 and workspace_token is not None:
+        split_k_launch_failed(workspace_token)
     assert rc == 0, f'{name} failed with HIP error {rc}'
 
 
