@@ -12,9 +12,8 @@
 //     busy, and the barrier between two k-tiles sits two steps before the end of the first, so that every wave still
 //     holds work when it has passed it; one workgroup per compute unit walks the tiles (dense_gemm_body_8w);
 //   * the smaller tiles (256 x 128 down to 64 x 64, widths of 64, 128, 192 and 256), which run problems bound by operand
-//     streaming: a ring of three to eight LDS stages, 4 waves, one per SIMD, each with a (BLOCK_N/WAVES_N) x
-//     (BLOCK_M/WAVES_M) slab of 32x32x16 MFMAs, up to 128 x 128 (256 accumulator registers, which the compiler keeps in
-//     AGPRs) (dense_gemm_body);
+//     streaming: a ring of three to eight LDS stages, 4 waves that compute, one per SIMD, each with a (BLOCK_N/WAVES_N) x
+//     (BLOCK_M/WAVES_M) slab of 32x32x16 MFMAs, up to 128 x 64, and 4 that only copy (dense_gemm_body);
 //   * problems with long K and fewer ring tiles than compute units split K over SPLIT_K workgroups per tile, which meet in a
 //     caller-provided workspace (dense_gemm_split_k, dense_meet_partials; 64 x 4096 x 7168: 64 workgroups of 64 x 64 become 256);
 //   * B rows feed the MFMA row operand and A rows the column operand, so a lane's four consecutive accumulator
@@ -76,12 +75,23 @@ dense_meet_partials(Acc (&acc)[TN][TM], float* __restrict__ partials, unsigned* 
                                                    tile_slot, split, wave, lane);
 }
 
+// Waves of a ring tile's workgroup: DenseTileConfig::NUM_WAVES compute, and four more take half of the copies off them. The
+// tiles are bound by their copies (2048 x 2112 x 7168 on 128 x 192: 86 us whole, 80 with the copies alone, 52 with the MFMAs
+// alone), and those by the bytes a compute unit can have on their way, whoever asks for them, so what this gains is the time the
+// computing waves stood in the queue: 37 shapes and tiles -7 to +2 %, 256 x 128 -4 to -11 % (2048 x 2112 x 7168 105.6 -> 94.3 us),
+// 128 x 192 81.4 -> 79.0, 64 x 192 at 1024 x 2112 x 7168 66.3 -> 62.2. With the four extra waves doing all the copies: between the two.
+// 128 x 128 tiles in four parts are 4 to 8 % slower with the extra waves (14 k-tiles per part at K = 7168) and stay without.
+__host__ __device__ constexpr int dense_launch_waves(int block_m, int block_n, int split_k = 1) {
+    return block_m * block_n >= 128 * 128 && split_k >= 4 ? 4 : 8;
+}
+
 template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K = 1>
 __device__ __forceinline__ void
 dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, Elem* __restrict__ C,
                 int m, int n, int k, int bid, float* __restrict__ partials = nullptr, unsigned* __restrict__ counters = nullptr) {
     using Cfg = DenseTileConfig<BLOCK_M, BLOCK_N>;
-    constexpr int NW = Cfg::NUM_WAVES, TN = Cfg::WTN / 32, TM = Cfg::WTM / 32;
+    // NW waves compute, all LW copy
+    constexpr int NW = Cfg::NUM_WAVES, LW = dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K), TN = Cfg::WTN / 32, TM = Cfg::WTM / 32;
     static_assert(STAGES >= 3 && STAGES <= Cfg::MAX_STAGES, "a ring of three or more stages that fits the LDS");
     // SPLIT_K > 1: launch slot `bid` is part `bid % SPLIT_K` of tile slot `bid / SPLIT_K`
     [[maybe_unused]] int split = 0;
@@ -99,8 +109,8 @@ dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
     const uint32_t ld_bytes = uint32_t(k) * 2;
     const __amdgpu_buffer_rsrc_t rsrc_a = make_rsrc(A, uint32_t(m) * ld_bytes);
     const __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(B, uint32_t(n) * ld_bytes);
-    TileStager<BLOCK_M, NW> stage_a;
-    TileStager<BLOCK_N, NW> stage_b;
+    TileStager<BLOCK_M, LW> stage_a;
+    TileStager<BLOCK_N, LW> stage_b;
     stage_a.init(m0, ld_bytes, wave, lane);
     stage_b.init(n0, ld_bytes, wave, lane);
 
@@ -117,8 +127,8 @@ dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
         kt_hi = min(kt_lo + per, num_k_tiles);
     }
     const __amdgpu_buffer_rsrc_t rsrc_none = make_rsrc(A, 0);
-    using StA = TileStager<BLOCK_M, NW>;
-    using StB = TileStager<BLOCK_N, NW>;
+    using StA = TileStager<BLOCK_M, LW>;
+    using StB = TileStager<BLOCK_N, LW>;
     constexpr int NUM_COPIES = StA::PASSES + StB::PASSES;
     static_assert(StA::PADDED_ROWS == BLOCK_M && StB::PADDED_ROWS == BLOCK_N, "tiles are whole copy passes");
     // Copy number `d` (A passes first, then B passes) of k-tile `kt` into the given stage.
@@ -191,7 +201,7 @@ dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
     // Ring: every wave issues NUM_COPIES copies per k-tile, in the same order, so "k-tile kt has landed" is "at
     // most (STAGES - 2) * NUM_COPIES of my copies are outstanding". The copies of k-tile kt + STAGES - 1 go to
     // the stage that was consumed in iteration kt - 1, which every wave has left once it is past the barrier.
-    static_assert((BLOCK_M / 8) % NW == 0 && (BLOCK_N / 8) % NW == 0 && (STAGES - 2) * NUM_COPIES <= 63);
+    static_assert((BLOCK_M / 8) % LW == 0 && (BLOCK_N / 8) % LW == 0 && (STAGES - 2) * NUM_COPIES <= 63);
     constexpr int STAGE_BYTES = Cfg::STAGE_BYTES;
     __shared__ __attribute__((aligned(1024))) uint8_t ring[STAGES * STAGE_BYTES];
 #pragma unroll
@@ -199,6 +209,20 @@ dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
 #pragma unroll
         for (int d = 0; d < NUM_COPIES; ++d) copy_pass(d, kt_lo + t, ring + t * STAGE_BYTES, ring + t * STAGE_BYTES + BLOCK_M * kRowBytes);
     int st = 0;
+    if (LW > NW && wave >= NW) {            // waves that only copy
+        for (int kt = kt_lo; kt < kt_hi; ++kt) {
+            __builtin_amdgcn_s_waitcnt(waitcnt_imm((STAGES - 2) * NUM_COPIES, kNoWaitLgkm));
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            uint8_t* nxt = ring + (st == 0 ? STAGES - 1 : st - 1) * STAGE_BYTES;
+#pragma unroll
+            for (int d = 0; d < NUM_COPIES; ++d) copy_pass(d, kt + STAGES - 1, nxt, nxt + BLOCK_M * kRowBytes);
+            st = st + 1 == STAGES ? 0 : st + 1;
+        }
+        if (SPLIT_K > 1 || (n % 8) == 0) __builtin_amdgcn_s_barrier();      // the one in front of the epilogue
+        return;
+    }
     for (int kt = kt_lo; kt < kt_hi; ++kt) {
         __builtin_amdgcn_s_waitcnt(waitcnt_imm((STAGES - 2) * NUM_COPIES, kNoWaitLgkm));
         asm volatile("" ::: "memory");
@@ -861,14 +885,14 @@ dense_gemm_walk(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
 }
 
 template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES>
-__global__ void __launch_bounds__(4 * kWaveSize)
+__global__ void __launch_bounds__((dense_launch_waves(BLOCK_M, BLOCK_N) * kWaveSize))
 dense_gemm_mfma(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, Elem* __restrict__ C, int m, int n, int k, int num_slots) {
     dense_gemm_walk<Atom, Elem, BLOCK_M, BLOCK_N, STAGES>(A, B, C, m, n, k, num_slots);
 }
 
 // The ring tiles with K split SPLIT_K ways: launch slot s is part s % SPLIT_K of tile slot s / SPLIT_K.
 template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K>
-__global__ void __launch_bounds__(4 * kWaveSize)
+__global__ void __launch_bounds__((dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize))
 dense_gemm_split_k(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, Elem* __restrict__ C, int m, int n, int k,
                    float* __restrict__ partials, unsigned* __restrict__ counters) {
     dense_gemm_body<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, SPLIT_K>(A, B, C, m, n, k, int(blockIdx.x), partials, counters);
@@ -877,13 +901,13 @@ dense_gemm_split_k(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
 // The fp16 flavour under the name of the reference's kernel (yan/include/gemm/cute_gemm.cuh:20), so that profiler
 // filters written for it (tests/test_cute.py:35 looks for 'fp16_gemm_cute') keep finding it.
 template <int BLOCK_M, int BLOCK_N, int STAGES>
-__global__ void __launch_bounds__(4 * kWaveSize)
+__global__ void __launch_bounds__((dense_launch_waves(BLOCK_M, BLOCK_N) * kWaveSize))
 fp16_gemm_cute(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, _Float16* __restrict__ C, int m, int n, int k, int num_slots) {
     dense_gemm_walk<MfmaF16_32x32x16, _Float16, BLOCK_M, BLOCK_N, STAGES>(A, B, C, m, n, k, num_slots);
 }
 
 template <int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K>
-__global__ void __launch_bounds__(4 * kWaveSize)
+__global__ void __launch_bounds__((dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize))
 fp16_gemm_cute_split_k(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, _Float16* __restrict__ C, int m, int n, int k,
                        float* __restrict__ partials, unsigned* __restrict__ counters) {
     dense_gemm_body<MfmaF16_32x32x16, _Float16, BLOCK_M, BLOCK_N, STAGES, SPLIT_K>(A, B, C, m, n, k, int(blockIdx.x), partials, counters);
@@ -952,15 +976,14 @@ inline hipError_t launch_dense(int m, int n, int k, const void* a, const void* b
                                dim3(8 * kWaveSize), 0, stream, static_cast<const uint8_t*>(a), static_cast<const uint8_t*>(b),
                                static_cast<Elem*>(c), m, n, k);
     } else {
-        using Cfg = DenseTileConfig<BLOCK_M, BLOCK_N>;
         const int grid = capped_grid(slots, num_sms, device_cu_count());
         if constexpr (__is_same(Elem, _Float16))
             hipLaunchKernelGGL((fp16_gemm_cute<BLOCK_M, BLOCK_N, STAGES>), dim3(grid),
-                               dim3(Cfg::NUM_WAVES * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
+                               dim3(dense_launch_waves(BLOCK_M, BLOCK_N) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
                                static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, slots);
         else
             hipLaunchKernelGGL((dense_gemm_mfma<Atom, Elem, BLOCK_M, BLOCK_N, STAGES>), dim3(grid),
-                               dim3(Cfg::NUM_WAVES * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
+                               dim3(dense_launch_waves(BLOCK_M, BLOCK_N) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
                                static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, slots);
     }
     return hipGetLastError();
@@ -985,11 +1008,11 @@ inline hipError_t launch_dense_split_k(int m, int n, int k, const void* a, const
     float* partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kSplitKCounterBytes);
     if constexpr (__is_same(Elem, _Float16))
         hipLaunchKernelGGL((fp16_gemm_cute_split_k<BLOCK_M, BLOCK_N, STAGES, SPLIT_K>), dim3(int(slots) * SPLIT_K),
-                           dim3(Cfg::NUM_WAVES * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
+                           dim3(dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
                            static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, partials, counters);
     else
         hipLaunchKernelGGL((dense_gemm_split_k<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, SPLIT_K>), dim3(int(slots) * SPLIT_K),
-                           dim3(Cfg::NUM_WAVES * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
+                           dim3(dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
                            static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, partials, counters);
     return hipGetLastError();
 }
