@@ -172,3 +172,32 @@ def test_gemm_kernels_compile_for_gfx950(cache_dir):
     name, keys, defs, _, tmpl = gemm.fp8_kernel_plan(1, 128, 128, 256)
     rt = jit.build(name, defs, jit.generate(gemm.includes, defs, jit.cpp_format(tmpl, keys)))
     assert runtime.Runtime.is_path_valid(rt.path)
+
+
+def test_runtime_call_takes_subclasses_the_checked_way(cache_dir):
+    # plain tensors, ints and floats go through the call written for the kernel's arguments, everything else through the loop
+    args = (('n', int), ('x', float), ('data', torch.int), ('stream', torch.cuda.Stream))
+    body = '\n__return_code = n + static_cast<int>(x * 10) + (data != nullptr ? 1000 : 0) + (stream != nullptr ? 10000 : 0);\n'
+    rt = jit.build('host_only', args, jit.generate((), args, body))
+    data = torch.zeros(4, dtype=torch.int)
+
+    class Count(int):
+        pass
+
+    assert rt(5, 0.5, data, 8) == rt(Count(5), 0.5, torch.nn.Parameter(data, requires_grad=False), 8) == 5 + 5 + 1000 + 10000
+    assert rt(True, 0.5, data, 0) == 1 + 5 + 1000
+    with pytest.raises(AssertionError, match='dtype'):
+        rt(5, 0.5, torch.nn.Parameter(torch.zeros(4)), 8)
+    with pytest.raises(AssertionError, match='Expected a stream'):
+        rt(5, 0.5, data, 'stream')
+    with pytest.raises(AssertionError, match='built-in type'):
+        rt(5, 1, data, 8)
+
+
+def test_environment_switches_are_read_on_every_call(monkeypatch):
+    from yan_amd.jit_kernels.utils import env_switch
+    monkeypatch.delenv('YAN_SPLIT_K', raising=False)
+    assert env_switch(b'YAN_SPLIT_K', True) and not env_switch(b'YAN_SPLIT_K', False)
+    for text, on in (('0', False), ('', False), ('1', True), ('no', True)):
+        monkeypatch.setenv('YAN_SPLIT_K', text)
+        assert env_switch(b'YAN_SPLIT_K', True) is env_switch(b'YAN_SPLIT_K', False) is on

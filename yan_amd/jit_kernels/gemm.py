@@ -15,9 +15,10 @@ from typing import Tuple
 
 import torch
 
+from .fp8_cast import per_token_cast_to_fp8
 from .heuristics import (get_best_fp8_config, get_fp8_num_stages, get_fp8_tile_space, get_skinny_fp8_config,
                          get_split_k_fp8_config, tuning_enabled)
-from .split_k import SPLIT_K_COUNTER_BYTES, SPLIT_K_WORKSPACE_BYTES, split_k_launch_failed, split_k_workspace
+from .split_k import SPLIT_K_COUNTER_BYTES, SPLIT_K_WORKSPACE_BYTES, split_k_enabled, split_k_launch_failed, split_k_workspace
 from .tuner import FrozenKeys, jit_tuner
 from .utils import current_raw_stream, get_num_sms, ceil_div, get_col_major_tensor, scales_for_kernel
 
@@ -246,8 +247,6 @@ def gemm_bf16_fp8_bf16_nt(x: torch.Tensor, rhs: Tuple[torch.Tensor, torch.Tensor
     9.6 us of vector arithmetic per workgroup against 2.5 us for the quantiser kernel spread over the chip (21.5 us in one
     kernel against 3 + 9.7 us in two; same bits). Problems whose codes do not fit the scratch area (or with
     `YAN_SPLIT_K=0`, which means no memory kept by the entries) run the two entries one after the other."""
-    from .fp8_cast import per_token_cast_to_fp8
-    from .split_k import split_k_enabled
     rhs_q, rhs_scales = rhs
     m, k = x.shape
     n, k_ = rhs_q.shape
@@ -265,10 +264,10 @@ def gemm_bf16_fp8_bf16_nt(x: torch.Tensor, rhs: Tuple[torch.Tensor, torch.Tensor
     name, keys, defs, code_template, smem_size = plan
     stream = current_raw_stream()
     workspace, workspace_token = split_k_workspace(out.device, stream)
-    values = {'x': x, 'buffer': workspace, 'scratch_bytes': CAST_SCRATCH_BYTES, 'rhs': rhs_q, 'rhs_scales': rhs_scales,
-              'out': out, 'm': m, 'stream': stream, 'num_sms': num_sms, 'smem_size': smem_size, 'workspace': workspace,
-              'workspace_bytes': SPLIT_K_WORKSPACE_BYTES}
-    args = tuple(values[d[0]] for d in defs)
+    # in the order of _cast_arg_defs_head and arg_defs without lhs and lhs_scales, then what the split-K kernels take in addition
+    args = (x, workspace, CAST_SCRATCH_BYTES, rhs_q, rhs_scales, out, m, stream, num_sms, smem_size)
+    if 'SPLIT_K' in keys:
+        args += (workspace, SPLIT_K_WORKSPACE_BYTES)
     runtime = jit_tuner.compile_and_tune(name=name, keys=keys, space=(), includes=cast_includes, arg_defs=defs, template=code_template, args=args)
     rc = runtime(*args)
     if rc != 0:

@@ -9,7 +9,7 @@ flop as the tile gets larger (fewer operand bytes fetched per flop).
 """
 from typing import List, Optional, Tuple
 
-from .utils import ceil_div
+from .utils import ceil_div, env_switch
 
 # (BLOCK_M, BLOCK_N): relative time per unit of tile area. Bigger tiles reuse operands better.
 # Dense tiles: 256 rows x {256, 224, 192, 160} columns run the persistent 4-wave kernel with a ring of five LDS units (the
@@ -47,8 +47,7 @@ def tuning_enabled() -> bool:
     three best tiles to the tuner as its `space` and the fastest on the device wins, as the reference's tuner does with
     its candidate list (`yan/jit_kernels/cute_gemm.py:42-53`, `tuner.py:42-69`). Off by default: the first call of a
     shape then costs up to three compilations and sixty timed launches."""
-    import os
-    return os.getenv('YAN_TUNE_TILES', '0') not in ('', '0')
+    return env_switch(b'YAN_TUNE_TILES', False)
 
 
 def get_dense_tile_space(m: int, n: int, k: int, num_cus: int, count: int = 3) -> List[Tuple[int, int]]:

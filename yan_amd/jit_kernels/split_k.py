@@ -14,10 +14,11 @@ must not overlap on the device. The reference's template leaves `split` to the c
 * `YAN_SPLIT_K=0` switches split-K off: the entry points then allocate nothing and keep no state between calls.
 """
 import ctypes
-import os
 from typing import Callable, Dict, Hashable, Optional
 
 import torch
+
+from .utils import env_switch
 
 # kSplitKCounterBytes and kSplitKWorkspaceBytes of gemm/scheduler.hpp: arrival counters, then the partial sums of the
 # largest plan the heuristics make.
@@ -30,7 +31,7 @@ MAX_EAGER_WORKSPACES = 8
 
 
 def split_k_enabled() -> bool:
-    return os.getenv('YAN_SPLIT_K', '1') not in ('', '0')
+    return env_switch(b'YAN_SPLIT_K', True)
 
 
 class WorkspaceBook:
@@ -124,7 +125,7 @@ def split_k_workspace(device: torch.device, stream: int):
     """(workspace, token) for a split-K launch on `stream` (the bare handle of the current stream), or (None, None) when
     split-K is switched off. Hand `token` to `split_k_launch_failed` if the launch reports an error."""
     global _last
-    if os.environ.get('YAN_SPLIT_K', '1') in ('', '0'):
+    if not env_switch(b'YAN_SPLIT_K', True):
         return None, None
     capture = capture_id(stream) if _is_capturing() else None
     index = device.index
