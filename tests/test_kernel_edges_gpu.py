@@ -74,3 +74,44 @@ def test_float_split_k_matches_the_oracle_and_repeats(m, n, k):
         assert ((results[0].double() - want).norm() / want.norm()).item() < 5e-6
     workspace, _ = split_k.split_k_workspace(c.device, torch.cuda.current_stream().cuda_stream)
     assert int(workspace[:split_k.SPLIT_K_COUNTER_BYTES].view(torch.int32).abs().sum()) == 0
+
+
+def _odd_floats(shape, dtype, seed):
+    """Every kind of bit pattern: subnormals, huge values, zeros of both signs, and infinities and NaN here and there."""
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(shape, generator=g) * torch.exp2(torch.randint(-130, 100, shape, generator=g).float())
+    special = torch.tensor([float('inf'), float('-inf'), float('nan'), 0.0, -0.0])
+    return torch.where(torch.rand(shape, generator=g) < 0.002, special[torch.randint(0, 5, shape, generator=g)], x).to(dtype)
+
+
+def _groups_quantised(x, amax):
+    """Codes and scales from each group's maximum, both quotients tensor by tensor (correctly rounded)."""
+    factor = torch.full_like(amax, 448.0) / amax
+    return x.float() * factor, amax / torch.full_like(amax, 448.0)
+
+
+# below, at and past a workgroup's 32 rows; the last three on either side of where sources (32 MB) and codes (32 MB) are streamed
+CAST_SHAPES = [(1, 128), (15, 384), (33, 128), (31, 4224), (65, 1152), (2341, 7168), (4682, 7168), (4097, 8192)]
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize('m,k', CAST_SHAPES)
+def test_quantisers_on_odd_sizes_and_odd_values(m, k, dtype):
+    """Both orders a workgroup takes its groups in and all three ways through the caches, against torch. A group with a NaN is
+    scaled by the maximum of the others and a group with an infinity gets the scale infinity (codes there are NaN and 0)."""
+    _announce('quantisers', m, k, dtype)
+    x = _odd_floats((m, k), dtype, seed=m + k).cuda()
+    tame = torch.where(torch.isnan(x.float()), torch.zeros((), device='cuda'), x.float().abs())
+    amax = tame.view(m, k // 128, 128).amax(-1).clamp(min=1e-4)
+    want, scales = _groups_quantised(x.view(m, k // 128, 128), amax.unsqueeze(-1))
+    finite = (want.abs() <= 448.0).view(m, k)
+    codes = want.view(m, k).to(torch.float8_e4m3fn).view(torch.uint8)
+    for q, sc in (yan.per_token_cast_to_fp8(x), yan.per_token_cast_to_fp8(x, col_major_scales=True)):
+        assert torch.equal(sc, scales.squeeze(-1))
+        assert torch.equal(q.view(torch.uint8)[finite], codes[finite])
+    block_amax = torch.nn.functional.pad(amax, (0, 0, 0, -m % 128)).view(-1, 128, k // 128).amax(1)
+    want, _ = _groups_quantised(x, block_amax.repeat_interleave(128, 0)[:m].repeat_interleave(128, 1))
+    q, sc = yan.per_block_cast_to_fp8(x)
+    assert torch.equal(sc, block_amax / torch.full_like(block_amax, 448.0))
+    finite = want.abs() <= 448.0
+    assert torch.equal(q.view(torch.uint8)[finite], want.to(torch.float8_e4m3fn).view(torch.uint8)[finite])
