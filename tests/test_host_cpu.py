@@ -535,3 +535,27 @@ def test_the_bf16_activation_entry_chains_the_quantiser_in_front_of_whatever_the
         assert '{' + 'SCRATCH_OFFSET' + '}' not in code and smem_size > 0
     # without split-K (YAN_SPLIT_K=0 leaves the entries without memory of their own) the entry makes two calls; the plan for it is not asked
     assert gemm.fp8_cast_chain_plan(64, 4096, 7168, 256, False)[1].get('SPLIT_K') is None
+
+
+def test_contiguous_kernel_waits_for_its_copies_between_two_tiles_of_a_walk(tmp_path):
+    """Workgroups that walk several slots of `fp8_gemm_contiguous_rows_kernel` go from tall to flat tiles, whose LDS stages are laid out
+    differently: every wave's copies have to land before the barrier between two slots. Checked on the generated code (the
+    main loops wait for a count of their own): each barrier is found with the wait in front of it, and exactly one of
+    them, the one that is followed by the jump back to the walk, waits for all copies."""
+    import re
+    import subprocess
+    import harness as testing
+    from yan_amd.jit import cpp_format, generate
+    from yan_amd.jit.compiler import get_hipcc_compiler, get_jit_include_dir, get_offload_arch
+    from yan_amd.jit_kernels import m_grouped_gemm
+    _, keys, arg_defs, template = testing.grouped_rows_on_device_plan(4, 4096, 7168)
+    src, asm = tmp_path / 'kernel.cu', tmp_path / 'kernel.s'
+    src.write_text(generate(m_grouped_gemm.includes, arg_defs, cpp_format(template, keys)))
+    subprocess.check_call([get_hipcc_compiler()[0], '-x', 'hip', '--cuda-device-only', '-S', '-std=c++20', '-O3',
+                           f'--offload-arch={get_offload_arch()}', '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops',
+                           f'-I{get_jit_include_dir()}', str(src), '-o', str(asm)])
+    lines = [line.split(';')[0].strip() for line in asm.read_text().split('\n')]
+    lines = [line for line in lines if line and not line.startswith('.') or line.endswith(':')]
+    waits = [re.search(r'vmcnt\((\d+)\)', ' '.join(ln for ln in lines[i - 2:i] if ln.startswith('s_waitcnt')))
+             for i, line in enumerate(lines) if line == 's_barrier']
+    assert len(waits) >= 6 and sum(w is not None and int(w.group(1)) == 0 for w in waits) == 1

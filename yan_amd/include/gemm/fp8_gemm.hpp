@@ -938,7 +938,14 @@ fp8_gemm_contiguous_rows_kernel(const uint8_t* __restrict__ lhs, const float* __
     }
     for (int slot = blockIdx.x; slot < slots; slot += grid) {
         run_slot(slot);
-        if (slot + grid < slots) __syncthreads();
+        if (slot + grid < slots) {
+            // A tile ends with copies of k-tiles past its last one still on their way into the pool. Between two tiles of a kind
+            // that is harmless (the wave that started such a copy starts the next one to the same place, and they land in
+            // order), but a stage of the flat tile is 49 KB, so its rows fall to other waves than the tall tile's and a late
+            // copy of one wave could land on what another has just fetched. No wave goes on before its own have landed.
+            wait_for_copies();
+            __syncthreads();
+        }
     }
 }
 
