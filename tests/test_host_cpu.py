@@ -559,3 +559,24 @@ def test_contiguous_kernel_waits_for_its_copies_between_two_tiles_of_a_walk(tmp_
     waits = [re.search(r'vmcnt\((\d+)\)', ' '.join(ln for ln in lines[i - 2:i] if ln.startswith('s_waitcnt')))
              for i, line in enumerate(lines) if line == 's_barrier']
     assert len(waits) >= 6 and sum(w is not None and int(w.group(1)) == 0 for w in waits) == 1
+
+
+def test_streams_forked_inside_a_capture_get_a_workspace_each(monkeypatch):
+    """Two streams that record into one capture are branches of the graph that may run side by side: their split-K launches must
+    not meet in one workspace. Launches on one of them share theirs, and another capture gets others."""
+    from yan_amd.jit_kernels import split_k
+    made = []
+    monkeypatch.setattr(split_k, '_book', split_k.WorkspaceBook(make=lambda: made.append(object()) or made[-1], clear=lambda w: None))
+    monkeypatch.setattr(split_k, '_last', (None, None))
+    monkeypatch.setattr(split_k, '_is_capturing', lambda: True)
+    capture = [7]
+    monkeypatch.setattr(split_k, 'capture_id', lambda stream: capture[0])
+    monkeypatch.delenv('YAN_SPLIT_K', raising=False)
+    device = torch.device('cuda', 0)
+    main, token = split_k.split_k_workspace(device, 111)
+    side, _ = split_k.split_k_workspace(device, 222)
+    assert side is not main and split_k.split_k_workspace(device, 111)[0] is main and split_k.split_k_workspace(device, 222)[0] is side
+    split_k.split_k_launch_failed(token)
+    assert split_k.split_k_workspace(device, 111)[0] is main
+    capture[0] = 8
+    assert split_k.split_k_workspace(device, 111)[0] not in (main, side) and len(made) == 3

@@ -7,7 +7,8 @@ must not overlap on the device. The reference's template leaves `split` to the c
 
 * eager launches share one workspace per (device, stream): launches on one stream run one after the other. At most
   `MAX_EAGER_WORKSPACES` are kept; the oldest goes back to torch's allocator, which hands it out again in stream order;
-* launches recorded into a graph get a workspace of their own per capture, made and zeroed inside the capture (the fill is
+* launches recorded into a graph get a workspace of their own per capture and per stream that takes part in it (streams forked
+  inside a capture become branches of the graph that run side by side), made and zeroed inside the capture (the fill is
   a node of the graph: every replay starts from zero counters, whatever happened before), never shared with another
   capture or with eager launches, and kept for the life of the process: a graph may be replayed on any stream, at any time;
 * a workspace whose last launch reported an error has its counters cleared before it is used again;
@@ -44,9 +45,9 @@ class WorkspaceBook:
         self.captures: Dict[Hashable, object] = {}
         self.suspect = set()
 
-    def get(self, device: int, stream: int, capture: Optional[int] = None):
-        """The workspace of a launch on `stream` of `device`; `capture` is the id of the capture the stream is recording
-        into, None for an eager launch."""
+    def get(self, device: int, stream: int, capture: Optional[Hashable] = None):
+        """The workspace of a launch on `stream` of `device`; `capture` names the part of a capture the launch is recorded
+        into, launches of which run one after the other in every replay; None for an eager launch."""
         if capture is not None:
             key = (device, capture)
             workspace = self.captures.get(key)
@@ -66,7 +67,7 @@ class WorkspaceBook:
         self.suspect.discard(key)
         return workspace
 
-    def launch_failed(self, device: int, stream: int, capture: Optional[int] = None) -> None:
+    def launch_failed(self, device: int, stream: int, capture: Optional[Hashable] = None) -> None:
         """A launch on this workspace reported an error: its counters may not be zero. (A capture's workspace is zeroed
         by the graph itself at every replay.)"""
         if capture is None:
@@ -128,6 +129,8 @@ def split_k_workspace(device: torch.device, stream: int):
     if not env_switch(b'YAN_SPLIT_K', True):
         return None, None
     capture = capture_id(stream) if _is_capturing() else None
+    if capture is not None:
+        capture = (capture, stream)
     index = device.index
     if index is None:
         index = torch.cuda.current_device()
