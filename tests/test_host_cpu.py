@@ -580,3 +580,28 @@ def test_streams_forked_inside_a_capture_get_a_workspace_each(monkeypatch):
     assert split_k.split_k_workspace(device, 111)[0] is main
     capture[0] = 8
     assert split_k.split_k_workspace(device, 111)[0] not in (main, side) and len(made) == 3
+
+
+def test_a_thread_on_another_stream_cannot_slip_in_its_workspace(monkeypatch):
+    """The latest eager workspace is remembered for the next call; a call that finds its own stream remembered must return that
+    stream's workspace also when a thread on another stream is served between the look and the return."""
+    from yan_amd.jit_kernels import split_k
+    monkeypatch.setattr(split_k, '_book', split_k.WorkspaceBook(make=object, clear=lambda w: None))
+    monkeypatch.setattr(split_k, '_last', (None, None))
+    monkeypatch.setattr(split_k, '_is_capturing', lambda: False)
+    monkeypatch.delenv('YAN_SPLIT_K', raising=False)
+    device = torch.device('cuda', 0)
+    mine, _ = split_k.split_k_workspace(device, 111)
+    others = []
+
+    class Stream(int):          # compared while the other thread gets its turn
+        __hash__ = int.__hash__
+
+        def __eq__(self, other):
+            if not others:
+                others.append(None)
+                others[0] = split_k.split_k_workspace(device, 222)[0]
+            return int(self) == int(other)
+
+    assert split_k.split_k_workspace(device, Stream(111))[0] is mine
+    assert others[0] is not None and others[0] is not mine

@@ -15,6 +15,7 @@ must not overlap on the device. The reference's template leaves `split` to the c
 * `YAN_SPLIT_K=0` switches split-K off: the entry points then allocate nothing and keep no state between calls.
 """
 import ctypes
+import threading
 from typing import Callable, Dict, Hashable, Optional
 
 import torch
@@ -85,6 +86,7 @@ def _clear_workspace(workspace: torch.Tensor) -> None:
 
 
 _book = WorkspaceBook(_make_workspace, _clear_workspace)
+_book_lock = threading.Lock()
 _hip = None
 
 
@@ -135,9 +137,11 @@ def split_k_workspace(device: torch.device, stream: int):
     if index is None:
         index = torch.cuda.current_device()
     token = (index, stream, capture)
-    if token == _last[0]:
-        return _last[1], token
-    workspace = _book.get(index, stream, capture)
+    last = _last            # one look: another thread may put its own stream's workspace there at any time
+    if token == last[0]:
+        return last[1], token
+    with _book_lock:
+        workspace = _book.get(index, stream, capture)
     if capture is None:
         _last = (token, workspace)
     return workspace, token
@@ -146,4 +150,5 @@ def split_k_workspace(device: torch.device, stream: int):
 def split_k_launch_failed(token) -> None:
     global _last
     _last = (None, None)
-    _book.launch_failed(*token)
+    with _book_lock:
+        _book.launch_failed(*token)
