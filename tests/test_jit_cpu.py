@@ -201,3 +201,12 @@ def test_environment_switches_are_read_on_every_call(monkeypatch):
     for text, on in (('0', False), ('', False), ('1', True), ('no', True)):
         monkeypatch.setenv('YAN_SPLIT_K', text)
         assert env_switch(b'YAN_SPLIT_K', True) is env_switch(b'YAN_SPLIT_K', False) is on
+
+
+def test_environment_switches_follow_a_replaced_environ(monkeypatch):
+    from yan_amd.jit_kernels.utils import env_switch
+    monkeypatch.setenv('YAN_SPLIT_K', '1')
+    monkeypatch.setattr(os, 'environ', {'YAN_SPLIT_K': '0'})
+    assert not env_switch(b'YAN_SPLIT_K', True)
+    os.environ.pop('YAN_SPLIT_K')
+    assert env_switch(b'YAN_SPLIT_K', True) and not env_switch(b'YAN_SPLIT_K', False)
