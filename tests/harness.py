@@ -293,6 +293,10 @@ GROUPED_ROWS_ON_DEVICE_CASES = [((512,) * 6, 768, 512, 0), ((384, 640) * 3, 768,
 # one block, one k-tile (no second one to fetch), an odd number of them, outputs that are no multiple of 8.
 GROUPED_FOLLOW_GROUPS_CASES = [((63 * 128, 3 * 128, 1, 2 * 128), 264, 128, 0), ((-128, 100, -256, 5 * 128, 385, -128, 128), 520, 384, 1),
                                ((128,) * 5, 1028, 640, 0), ((64 * 128, 65 * 128), 12, 256, 2), ((128,), 256, 128, 0)]
+# (BLOCK_N, NUM_STAGES) that go with BLOCK_M = 256 in the keys of a contiguous call: the widths of the cost table, the other ones the
+# tiles support, with and without a ring and a 128-row tile beside them
+GROUPED_256_ROW_KEYS = [(256, 2), (224, 2), (192, 2), (160, 2), (128, 3), (128, 2), (96, 2), (32, 2)]
+GROUPED_256_ROW_KEYS_CASE = ((-128, 100, -256, 5 * 128, 385, -128, 3 * 128), 520, 384, 0)
 GROUPED_MASKED_TEST_CASES = [
     (3, 200, 320, 384, (200, 0, 77), 128), (4, 256, 4096, 1024, (1, 256, 130, 64), 64), (2, 64, 200, 128, (64, 3), 32),
     (4, 1024, 4096, 7168, (1024, 900, 512, 1), 1024),
@@ -352,6 +356,14 @@ def grouped_rows_on_device_plan(num_groups: int, n: int, k: int):
     keys = {'N': n, 'K': k, 'BLOCK_M': 256, 'BLOCK_N': 256, 'NUM_GROUPS': num_groups, 'NUM_STAGES': 2, 'NUM_TMA_MULTICAST': 1,
             'GEMM_TYPE': 'GroupedContiguous', 'ROWS': 'picked on the device'}
     return 'm_grouped_gemm_fp8_fp8_bf16_nt_rows_on_device', keys, m_grouped_gemm.arg_defs, m_grouped_gemm.rows_on_device_template
+
+
+def grouped_256_row_plan(block_n: int, stages: int, num_groups: int, n: int, k: int):
+    """(name, keys, arg_defs, template) of a contiguous grouped call whose keys name a tile of 256 x `block_n` outright."""
+    from yan_amd.jit_kernels import m_grouped_gemm
+    keys = {'N': n, 'K': k, 'BLOCK_M': 256, 'BLOCK_N': block_n, 'NUM_GROUPS': num_groups, 'NUM_STAGES': stages, 'NUM_TMA_MULTICAST': 1,
+            'GEMM_TYPE': 'GroupedContiguous'}
+    return 'm_grouped_gemm_fp8_fp8_bf16_nt', keys, m_grouped_gemm.arg_defs, m_grouped_gemm.template
 
 
 def jit_kernels_in_use(num_cus: int = 256):
@@ -455,6 +467,10 @@ def jit_kernels_in_use(num_cus: int = 256):
         add(name, arg_defs, m_grouped_gemm.includes, m_grouped_gemm.rows_on_device_template if 'ROWS' in keys else m_grouped_gemm.template, keys)
     for rows, n, k, _ in GROUPED_ROWS_ON_DEVICE_CASES + GROUPED_FOLLOW_GROUPS_CASES:
         name, keys, arg_defs, code_template = grouped_rows_on_device_plan(sum(1 for r in rows if r > 0), n, k)
+        add(name, arg_defs, m_grouped_gemm.includes, code_template, keys)
+    rows, n, k, _ = GROUPED_256_ROW_KEYS_CASE
+    for block_n, stages in GROUPED_256_ROW_KEYS:
+        name, keys, arg_defs, code_template = grouped_256_row_plan(block_n, stages, sum(1 for r in rows if r > 0), n, k)
         add(name, arg_defs, m_grouped_gemm.includes, code_template, keys)
     # the grouped layouts under the compute-unit cap: tiles chosen for NUM_SMS_CAP units
     rows, n, k, pad_blocks = GROUPED_TWO_GROUP_ROWS_FIRST_CASE

@@ -605,3 +605,17 @@ def test_a_thread_on_another_stream_cannot_slip_in_its_workspace(monkeypatch):
 
     assert split_k.split_k_workspace(device, Stream(111))[0] is mine
     assert others[0] is not None and others[0] is not mine
+
+
+def test_contiguous_keys_may_name_any_tile_of_256_rows(tmp_path):
+    """`Gemm<..., 256, BLOCK_N, ..., kNumStages, ..., GroupedContiguous>::run_grouped` takes every width and depth the tiles support,
+    not only those a plan names: the static checks of host and device code pass for all of them."""
+    import subprocess
+    import harness as testing
+    from yan_amd.jit.compiler import get_hipcc_compiler, get_jit_include_dir, get_offload_arch
+    src = tmp_path / 'keys.hip'
+    calls = '\n'.join(f'    yan::Gemm<520, 384, 256, {n}, 128, 4, {stages}, 1, yan::GemmType::GroupedContiguous>::run_grouped('
+                      'out, q, s, 1, 1, 0, q, s, g, 4, 256, 520, 384, nullptr, 0, 0);' for n, stages in testing.GROUPED_256_ROW_KEYS)
+    src.write_text('#include "gemm/fp8_gemm.hpp"\nvoid keys(__hip_bfloat16* out, const void* q, const float* s, const int* g) {\n' + calls + '\n}\n')
+    subprocess.check_call([get_hipcc_compiler()[0], '--cuda-device-only', '-fsyntax-only', '-std=c++20', f'--offload-arch={get_offload_arch()}',
+                           f'-I{get_jit_include_dir()}', str(src)])

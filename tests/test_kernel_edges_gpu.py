@@ -49,6 +49,32 @@ def test_contiguous_tiles_follow_the_groups(rows, n, k, pad_blocks):
     assert _fp8_close(results[0][real].float(), ref[real])
 
 
+@pytest.mark.parametrize('block_n,stages', testing.GROUPED_256_ROW_KEYS)
+def test_contiguous_keys_that_name_a_tile_of_256_rows(block_n, stages):
+    """Every width and depth such keys may hold, against the oracle, capped and not, with a row count that ends inside a block (the
+    class takes one, the entries ask for whole blocks)."""
+    from yan_amd.jit_kernels import m_grouped_gemm
+    _announce('contiguous keys', block_n, stages)
+    rows, n, k, pad_blocks = testing.GROUPED_256_ROW_KEYS_CASE
+    (a8, sa), (b8, sb), out, idx = testing.make_grouped_contiguous_case(rows, n, k, seed=12, padding_blocks=pad_blocks)
+    name, keys, arg_defs, code_template = testing.grouped_256_row_plan(block_n, stages, b8.size(0), n, k)
+    kernel = jit.build(name, arg_defs, jit.generate(m_grouped_gemm.includes, arg_defs, jit.cpp_format(code_template, keys)))
+    ref = torch.from_numpy(oracle.m_grouped_gemm_contiguous_ref(_codes(a8), sa.numpy(), _codes(b8), sb.numpy(), idx.numpy(),
+                                                                out_init=out.float().numpy()))
+    a8d, sad, b8d, sbd, idxd = a8.cuda(), sa.cuda(), b8.cuda(), sb.cuda(), idx.cuda()
+    for m in (a8.size(0), a8.size(0) - 60):
+        results = []
+        for cap in (256, 8):
+            got = out.cuda()
+            assert kernel(a8d, sad, b8d, sbd, got, idxd, m, torch.cuda.current_stream(), cap, 0, sad.stride(0), sad.stride(1), 0, 0) == 0
+            torch.cuda.synchronize()
+            results.append(got.cpu())
+        written = (idx >= 0) & (torch.arange(a8.size(0)) < m)
+        assert torch.equal(results[0], results[1])
+        assert torch.equal(results[0][~written], out[~written])
+        assert _fp8_close(results[0][written].float(), ref[written])
+
+
 @pytest.mark.parametrize('m,n,k', testing.FLOAT_SPLIT_K_SHAPES)
 def test_float_split_k_matches_the_oracle_and_repeats(m, n, k):
     """gemm_cute_split_k through the entry: k that is no multiple of a k-tile or of the parts, last parts shorter than the

@@ -82,6 +82,10 @@ struct Fp8TileConfig {
     // flight (a stage is only 9 to 13 KB there). Measured with every unit pulling: about 60 GB/s per unit whatever the
     // tile, so the tile to prefer is the one that moves the fewest bytes per output, 32 x 32 for a 64-row problem.
     static constexpr int  RING_DEPTH_CAP = BLOCK_N <= 32 ? 12 : 8;
+    // Room for a third stage of weights next to two of activations, and rows of atoms enough to hand its copies out one per row
+    // (kDeepB in fp8_gemm_tile).
+    static constexpr bool DEEP_B_CAPABLE = LDS_BYTES + LDS_ROWS_B * kRowBytes <= 160 * 1024 &&
+                                           (TileStager<BLOCK_M, NUM_WAVES>::PASSES + 1) / 2 + TileStager<BLOCK_N, NUM_WAVES>::PASSES <= WTN / 16;
     static constexpr int  MAX_RING_STAGES = RING_CAPABLE ? (160 * 1024 / RING_STAGE_BYTES < RING_DEPTH_CAP ? 160 * 1024 / RING_STAGE_BYTES : RING_DEPTH_CAP) : 2;
 };
 
@@ -404,8 +408,7 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     // 143 -> 135 us; 48 blocks of 128 rows over 16 groups 219 -> 201 us, and 197 with the copies handed out in the order of
     // their deadlines, activations (due at the next k-tile) two per row of atoms, then weights one per row. One group of
     // 8192 rows, whose weights come from the caches, runs level (195 us).
-    constexpr bool kDeepB = kGemmType == GemmType::GroupedContiguous && EXPLICIT_TILE && STAGES == 2;
-    static_assert(!kDeepB || (StA::PASSES + 1) / 2 + StB::PASSES <= TN);
+    constexpr bool kDeepB = kGemmType == GemmType::GroupedContiguous && EXPLICIT_TILE && STAGES == 2 && Cfg::DEEP_B_CAPABLE;
     auto row_of_copy = [](int d) { return !kDeepB ? d * SPREAD_ROWS / NUM_COPIES : (d < StA::PASSES ? d / 2 : (StA::PASSES + 1) / 2 + d - StA::PASSES); };
     auto k_step = [&](int kb, const uint8_t* a_cur, const uint8_t* b_cur, uint8_t* a_nxt, uint8_t* b_nxt) {
 #pragma unroll
@@ -883,10 +886,13 @@ fp8_gemm_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_s
 // weight stage the tall tiles have room for (kDeepB); 10240 rows in 4 groups 290 -> 276 us, 8320 in 64 x 7168 x 2048 185 -> 172.
 // Mixing flat and tall tiles in the order of the groups (every weight panel then read at one time) measured the same, and
 // running tall rows flat where the tall tiles end in a round that is mostly empty gains 2-4 % there and loses 1 % elsewhere.
+// STAGES belongs to the tall tile: 2, or a ring as everywhere else (256 x 128). The flat tile runs the deepest ring it has. Where
+// it has none, or runs on another number of waves (256 x 160 and the other widths no plan takes), the odd block is a tall
+// tile whose rows end with the block.
 // It is launched with eight slots more than the 128-row tiling has, which covers every case; workgroups beyond the last
 // slot leave at once.
-template <int SHAPE_N, int SHAPE_K, int BLOCK_N>
-__global__ void __launch_bounds__(8 * kWaveSize)
+template <int SHAPE_N, int SHAPE_K, int BLOCK_N, int STAGES>
+__global__ void __launch_bounds__((fp8_launch_waves(256, BLOCK_N, STAGES) * kWaveSize))
 fp8_gemm_contiguous_rows_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_scales,
                                 const uint8_t* __restrict__ rhs, const float* __restrict__ rhs_scales,
                                 __bf16* __restrict__ out, int m, int n_rt, int k_rt, int sa_stride_m, int sa_stride_k,
@@ -894,17 +900,19 @@ fp8_gemm_contiguous_rows_kernel(const uint8_t* __restrict__ lhs, const float* __
     using Tall = Fp8TileConfig<256, BLOCK_N>;
     using Flat = Fp8TileConfig<128, BLOCK_N>;
     constexpr int FLAT_STAGES = Flat::MAX_RING_STAGES;
-    constexpr int TALL_BYTES = (2 * Tall::LDS_ROWS_A + 3 * Tall::LDS_ROWS_B) * kRowBytes, FLAT_BYTES = FLAT_STAGES * Flat::RING_STAGE_BYTES;
-    static_assert(FLAT_STAGES >= 3 && fp8_launch_waves(256, BLOCK_N, 2) == 8 && fp8_launch_waves(128, BLOCK_N, FLAT_STAGES) == 8);
+    constexpr bool HAS_FLAT = FLAT_STAGES >= 3 && fp8_launch_waves(128, BLOCK_N, FLAT_STAGES) == fp8_launch_waves(256, BLOCK_N, STAGES);
+    constexpr bool TALL_RING = STAGES > 2;
+    constexpr int TALL_BYTES = TALL_RING ? STAGES * Tall::RING_STAGE_BYTES : Tall::LDS_BYTES + (Tall::DEEP_B_CAPABLE ? Tall::LDS_ROWS_B * kRowBytes : 0);
+    constexpr int FLAT_BYTES = HAS_FLAT ? FLAT_STAGES * Flat::RING_STAGE_BYTES : 0;
     __shared__ __attribute__((aligned(1024))) uint8_t pool[TALL_BYTES > FLAT_BYTES ? TALL_BYTES : FLAT_BYTES];
     uint8_t* const a0 = pool;
     uint8_t* const b0 = a0 + Tall::LDS_ROWS_A * kRowBytes;
     uint8_t* const a1 = b0 + Tall::LDS_ROWS_B * kRowBytes;
     uint8_t* const b1 = a1 + Tall::LDS_ROWS_A * kRowBytes;
-    uint8_t* const b2 = b1 + Tall::LDS_ROWS_B * kRowBytes;
+    uint8_t* const b2 = Tall::DEEP_B_CAPABLE ? b1 + Tall::LDS_ROWS_B * kRowBytes : nullptr;
     const int N = SHAPE_N ? SHAPE_N : n_rt;
     const int lane = get_lane_id();
-    const int blocks = m / 128, tiles_n = ceil_div(N, BLOCK_N);
+    const int blocks = ceil_div(m, 128), tiles_n = ceil_div(N, BLOCK_N);
     int tall_rows = 0, flat_rows = 0, odd = 0;
     for (int c = 0; c < ceil_div(blocks, kWaveSize); ++c) {
         const ContiguousTileStarts starts = contiguous_tile_starts(grouped_layout, blocks, c, lane, odd);
@@ -920,15 +928,17 @@ fp8_gemm_contiguous_rows_kernel(const uint8_t* __restrict__ lhs, const float* __
         const bool is_tall = slot < tall_slots;
         const TileCoord t = is_tall ? tall.dealt_band_tile_of(slot) : flat.dealt_band_tile_of(slot - tall_slots);
         if (!t.valid) return;
-        const int tile = contiguous_block_at(grouped_layout, blocks, is_tall, t.m_idx, lane) * tiles_n + t.n_idx;
-        if (is_tall)
-            fp8_gemm_tile<SHAPE_N, SHAPE_K, 256, BLOCK_N, GemmType::GroupedContiguous, 2, 1, false, true>(
-                lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt, sa_stride_m, sa_stride_k, grouped_layout, 0, tile, num_groups, 0,
-                Fp8TwoStages{a0, b0, a1, b1, b2});
-        else
+        const int block = contiguous_block_at(grouped_layout, blocks, is_tall, t.m_idx, lane), tile = block * tiles_n + t.n_idx;
+        if (is_tall || !HAS_FLAT) {
+            const int rows_end = HAS_FLAT || is_tall ? m : min(m, (block + 1) * 128);
+            fp8_gemm_tile<SHAPE_N, SHAPE_K, 256, BLOCK_N, GemmType::GroupedContiguous, STAGES, 1, TALL_RING, true>(
+                lhs, lhs_scales, rhs, rhs_scales, out, rows_end, n_rt, k_rt, sa_stride_m, sa_stride_k, grouped_layout, 0, tile, num_groups, 0,
+                Fp8TwoStages{a0, b0, a1, b1, b2}, nullptr, nullptr, pool);
+        } else if constexpr (HAS_FLAT) {
             fp8_gemm_tile<SHAPE_N, SHAPE_K, 128, BLOCK_N, GemmType::GroupedContiguous, FLAT_STAGES, 1, true, true>(
                 lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt, sa_stride_m, sa_stride_k, grouped_layout, 0, tile, num_groups, 0,
                 Fp8TwoStages{}, nullptr, nullptr, pool);
+        }
     };
     const int grid = gridDim.x;
     // a workgroup per slot (no cap): the tile without a loop around it
@@ -941,7 +951,7 @@ fp8_gemm_contiguous_rows_kernel(const uint8_t* __restrict__ lhs, const float* __
         if (slot + grid < slots) {
             // A tile ends with copies of k-tiles past its last one still on their way into the pool. Between two tiles of a kind
             // that is harmless (the wave that started such a copy starts the next one to the same place, and they land in
-            // order), but a stage of the flat tile is 49 KB, so its rows fall to other waves than the tall tile's and a late
+            // order), but the stages of the flat tile are smaller, so its rows fall to other waves than the tall tile's and a late
             // copy of one wave could land on what another has just fetched. No wave goes on before its own have landed.
             wait_for_copies();
             __syncthreads();
@@ -1030,20 +1040,21 @@ public:
                                                  int lhs_scales_stride_k, const void* rhs, const float* rhs_scales,
                                                  const int* grouped_layout, int num_groups, int m, int n, int k, hipStream_t stream,
                                                  int num_sms = 0) {
-        static_assert(kGemmType == GemmType::GroupedContiguous && BLOCK_M == 256 && BLOCK_N >= 160 && kNumStages == 2);
+        static_assert(kGemmType == GemmType::GroupedContiguous && BLOCK_M == 256);
         if (m == 0 || n == 0 || num_groups == 0) return hipSuccess;
-        if (m < 0 || n < 0 || k <= 0 || num_groups < 0 || (n % 4) != 0 || (k % 128) != 0 || (m % 128) != 0) return hipErrorInvalidValue;
+        if (m < 0 || n < 0 || k <= 0 || num_groups < 0 || (n % 4) != 0 || (k % 128) != 0) return hipErrorInvalidValue;
         if ((SHAPE_N && n != int(SHAPE_N)) || (SHAPE_K && k != int(SHAPE_K))) return hipErrorInvalidValue;
         if (kNumGroups > 1 && num_groups != int(kNumGroups)) return hipErrorInvalidValue;
         if (!out || !lhs || !lhs_scales || !rhs || !rhs_scales || !grouped_layout) return hipErrorInvalidValue;
         const uint64_t m_pad = uint64_t(ceil_div<uint32_t>(m, BLOCK_M)) * BLOCK_M, n_pad = uint64_t(ceil_div<uint32_t>(n, BLOCK_N)) * BLOCK_N;
         if (m_pad * k >= kOutOfRange || n_pad * k >= kOutOfRange || uint64_t(BLOCK_M) * n * 2 >= kOutOfRange) return hipErrorInvalidValue;
+        if (m_pad * num_groups >= kOutOfRange) return hipErrorInvalidValue;
         // tall and flat tiles, each rounded up to the 8 XCDs: at most the tiles of the 128-row tiling + 8
         const long long slots = (long long)XcdTileScheduler<>(m, n, 128, BLOCK_N).grid_size() + kNumXCD;
         if (slots >= kOutOfRange) return hipErrorInvalidValue;
         const int grid = capped_grid(int(slots), num_sms, device_cu_count());
-        hipLaunchKernelGGL((fp8_gemm_contiguous_rows_kernel<SHAPE_N, SHAPE_K, BLOCK_N>), dim3(grid), dim3(8 * kWaveSize), 0, stream,
-                           static_cast<const uint8_t*>(lhs), lhs_scales, static_cast<const uint8_t*>(rhs), rhs_scales,
+        hipLaunchKernelGGL((fp8_gemm_contiguous_rows_kernel<SHAPE_N, SHAPE_K, BLOCK_N, int(kNumStages)>), dim3(grid),
+                           dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream, static_cast<const uint8_t*>(lhs), lhs_scales, static_cast<const uint8_t*>(rhs), rhs_scales,
                            reinterpret_cast<__bf16*>(out), m, n, k, lhs_scales_stride_m, lhs_scales_stride_k, grouped_layout, num_groups);
         return hipGetLastError();
     }
