@@ -168,8 +168,9 @@ YAN_API int yan_per_block_cast_to_fp8(const void* w, int w_is_fp32, void* q, flo
 /* Macro tile the library uses for a problem: op 0 = dense 16-bit, 1 = FP8 block-scaled, 2 = FP8 grouped contiguous
  * (m = total rows, and `k` carries the number of groups instead of the depth), 3 = fp32. Writes BLOCK_M / BLOCK_N.
  * op 4 (m, `k` as for op 2): 256 x 256 when the contiguous entry point runs the kernel that holds 256 x 256 and 128 x 256
- * tiles and places them along the groups on the device, from m_indices (groups of 128 rows or more on average),
- * 0 x 0 when it runs the tile op 2 names.
+ * tiles and places them along the groups on the device, from m_indices (groups of 128 rows or more on average), at a depth of 1024;
+ * 0 x 0 when it runs the tile op 2 names. For groups of 128 to 255 rows the answer depends on the depth.
+ * op 5: the same for the depth `k`, with the number of groups in *block_m when it is called.
  * For ops 0 and 1 with few activation rows the answer is (16 * atoms, 16): the weight-streaming kernels.
  * Host-only (no device call). Stands where the reference leaves tile choice to the caller's keys
  * (yan/jit_kernels/cute_gemm.py:41, yan/jit_kernels/gemm.py:13-16). Returns 0, or 1 for an unknown op. */

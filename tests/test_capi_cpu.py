@@ -117,3 +117,17 @@ def test_compute_entry_points_validate_before_touching_a_device(lib):
     assert grouped_m(null, null, 1, 1, 1, null, null, null, null, 2, 64, 0, 128, 128, null, 256) != 0      # expected_m
     assert grouped_m(null, null, 1, 1, 1, null, null, null, null, 2, 64, 64, 126, 128, null, 256) != 0     # n % 4
     assert grouped_m(null, null, 1, 1, 1, null, null, null, null, 2, 64, 64, 128, 128, null, 256) != 0     # null operands
+
+
+def test_contiguous_tiles_follow_the_groups_by_the_same_rule(lib):
+    taken = 0
+    for m in range(1024, 16385, 640):
+        for n in (1088, 1344, 2112, 2304, 4160, 7168):
+            for k in (1024, 1280, 2048, 7168):
+                for groups in (1, 5, 24, 46, 64, 100):
+                    for cus in (256, 80):
+                        want = heuristics.get_contiguous_rows_on_device(m, n, k, cus, groups)
+                        assert capi.contiguous_follows_groups(m, n, k, groups, cus) == want, (m, n, k, groups, cus)
+                        taken += want
+    assert taken > 1000
+    assert not capi.contiguous_follows_groups(0, 128, 128, 1, 256) and not capi.contiguous_follows_groups(128, 128, 0, 1, 256)

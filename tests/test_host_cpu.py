@@ -619,3 +619,30 @@ def test_contiguous_keys_may_name_any_tile_of_256_rows(tmp_path):
     src.write_text('#include "gemm/fp8_gemm.hpp"\nvoid keys(__hip_bfloat16* out, const void* q, const float* s, const int* g) {\n' + calls + '\n}\n')
     subprocess.check_call([get_hipcc_compiler()[0], '--cuda-device-only', '-fsyntax-only', '-std=c++20', f'--offload-arch={get_offload_arch()}',
                            f'-I{get_jit_include_dir()}', str(src)])
+
+
+# (groups, rows, n, k): microseconds of the 128-row tile the cost table takes and of the kernel whose tiles follow the groups (MI355X,
+# router-like layouts)
+SHORT_GROUPS = {(49, 9856, 1344, 1280): (36.6, 41.8), (43, 7040, 2112, 1152): (35.4, 39.4), (46, 8320, 1344, 1024): (29.7, 31.7),
+                (29, 3712, 4352, 2560): (69.7, 74.4), (33, 4608, 3392, 1792): (50.5, 52.6), (40, 9344, 2304, 1280): (47.5, 52.0),
+                (41, 8448, 1600, 1664): (41.2, 47.3), (21, 2688, 5824, 1536): (46.6, 47.6),
+                (64, 8320, 7168, 2048): (188.9, 173.0), (32, 6144, 4096, 4096): (148.4, 135.4), (24, 3968, 2880, 2048): (48.7, 42.7),
+                (23, 2944, 4032, 1664): (43.1, 39.4), (50, 9728, 1152, 1408): (36.4, 33.4), (10, 1280, 7168, 2048): (44.5, 33.5),
+                (29, 6784, 4160, 1152): (98.7, 59.1), (13, 1920, 4992, 2560): (56.9, 43.3), (59, 11392, 6144, 2176): (222.5, 206.1)}
+
+
+def test_short_contiguous_groups_get_the_kernel_that_measured_faster():
+    for (groups, m, n, k), (fixed, follows) in SHORT_GROUPS.items():
+        assert heuristics.get_contiguous_rows_on_device(m, n, k, 256, groups) == (follows < fixed), (groups, m, n, k)
+
+
+def test_time_of_tall_and_flat_tiles_is_that_of_a_list_schedule():
+    import heapq
+    flat_time = heuristics._FP8_TILES[(128, 256)] / 2
+    for cus in (1, 8, 80, 256):
+        for tall in (0, 1, cus - 1, cus, cus + 3, 3 * cus + cus // 2):
+            for flat in (0, 1, cus // 2, cus, 2 * cus + 5, 7 * cus):
+                free = [0.0] * cus
+                for time in [1.0] * tall + [flat_time] * flat:
+                    heapq.heapreplace(free, free[0] + time)
+                assert heuristics._tall_then_flat(tall, flat, cus) == pytest.approx(max(free)), (tall, flat, cus)

@@ -113,6 +113,13 @@ def select_split_k(m: int, n: int, k: int, num_cus: int, op: int = 1):
     return (bm.value, bn.value, split.value) if split.value > 1 else None
 
 
+def contiguous_follows_groups(m: int, n: int, k: int, num_groups: int, num_cus: int) -> bool:
+    """Whether the library's contiguous grouped GEMM places its tiles along the groups, on the device."""
+    bm, bn = ctypes.c_int(num_groups), ctypes.c_int(0)
+    assert load().yan_gemm_select_tile(5, m, n, k, num_cus, ctypes.byref(bm), ctypes.byref(bn)) == 0
+    return bm.value == 256
+
+
 def m_grouped_gemm_fp8_fp8_bf16_nt_contiguous(lhs, rhs, out: torch.Tensor, m_indices: torch.Tensor, num_sms: int = 0) -> int:
     (a8, sa), (b8, sb) = lhs, rhs
     (m, k), (groups, n, _) = a8.shape, b8.shape

@@ -40,7 +40,7 @@ void pick(const TileCost (&tiles)[COUNT], int m, int n, int num_cus, int* bm, in
 
 // Tile of a grouped FP8 GEMM (get_best_grouped_fp8_config in heuristics.py): tiles 64, 128 or 256 wide; with a non-zero
 // `m_alignment` BLOCK_M divides it; the tile count is multiplied by `groups`.
-void pick_grouped(int m, int n, int num_cus, int groups, int m_alignment, int* bm, int* bn) {
+double pick_grouped(int m, int n, int num_cus, int groups, int m_alignment, int* bm, int* bn) {
     double best = -1;
     if (m < 1) m = 1;
     for (const TileCost& t : kFp8Tiles) {
@@ -51,11 +51,28 @@ void pick_grouped(int m, int n, int num_cus, int groups, int m_alignment, int* b
         const double cost = double(rounds) * t.bm * t.bn * t.per_area;
         if (best < 0 || cost < best || (cost == best && (t.bm < *bm || (t.bm == *bm && t.bn < *bn)))) { best = cost; *bm = t.bm; *bn = t.bn; }
     }
+    return best;
+}
+
+// When the last of `tall` tiles of 256 x 256 and, behind them, `flat` ones of 128 x 256 ends, in times of a tall tile
+// (_tall_then_flat in heuristics.py).
+double tall_then_flat(long long tall, long long flat, int num_cus) {
+    const double flat_time = 1.34 / 2;
+    const long long full = tall / num_cus, over = tall % num_cus;
+    double end = double(full + (over ? 1 : 0)), early = double(full) + flat_time, late = double(full + 1) + flat_time;
+    while (flat > 0) {
+        double& next = over == 0 || early <= late ? early : late;
+        flat -= &next == &early ? num_cus - over : over;
+        if (next > end) end = next;
+        next += flat_time;
+    }
+    return end;
 }
 
 // Whether a contiguous grouped GEMM runs the kernel whose tiles follow the groups (get_contiguous_rows_on_device in
-// heuristics.py): groups of 128 rows or more on average that get 256 x 256 tiles when every tile height is allowed.
-bool rows_on_device(int m, int n, int num_cus, int groups_in_m) {
+// heuristics.py): groups of 128 rows or more on average that get 256 x 256 tiles when every tile height is allowed, those
+// below 256 rows where the tiles that run, tall and flat, are still the cheaper ones.
+bool rows_on_device(int m, int n, int k, int num_cus, int groups_in_m) {
     if (groups_in_m <= 0 || (long long)m < 128ll * groups_in_m) return false;
     // the same table with every tile height allowed
     double best = -1;
@@ -67,7 +84,14 @@ bool rows_on_device(int m, int n, int num_cus, int groups_in_m) {
         const double cost = double(rounds) * t.bm * t.bn * t.per_area;
         if (best < 0 || cost < best || (cost == best && (t.bm < tm || (t.bm == tm && t.bn < tn)))) { best = cost; tm = t.bm; tn = t.bn; }
     }
-    return tm == 256 && tn == 256;
+    if (tm != 256 || tn != 256) return false;
+    if ((long long)m >= 256ll * groups_in_m) return true;
+    const int blocks = (m + 127) / 128, tall_rows = (blocks - (groups_in_m + 1) / 2) / 2;
+    const long long tiles_n = (n + 255) / 256;
+    const double time = tall_then_flat(tall_rows * tiles_n, (blocks - 2 * tall_rows) * tiles_n, num_cus) * 65536 * (1 + 280.0 / k);
+    int bm = 0, bn = 0;
+    const double cost = pick_grouped(m, n, num_cus, 1, 128, &bm, &bn);
+    return time < cost * (bm == 128 && bn == 128 ? 1.43 : 1.0);
 }
 
 // Activation atoms of the weight-streaming kernel, or 0 for the tiled kernel (get_skinny_fp8_config in heuristics.py).
@@ -324,7 +348,7 @@ int yan_m_grouped_gemm_fp8_fp8_bf16_nt_contiguous(const void* lhs, const float* 
     const long long last = (long long)(m - 1) * lhs_scales_stride_m + (long long)(k / 128 - 1) * lhs_scales_stride_k;
     if (lhs_scales_stride_m < 0 || lhs_scales_stride_k < 0 || last >= (1ll << 28)) return int(hipErrorInvalidValue);
     const int cus = (num_sms > 0 && num_sms < device_cus()) ? num_sms : device_cus();
-    if (rows_on_device(m, n, cus, num_groups))
+    if (rows_on_device(m, n, k, cus, num_groups))
         return int(yan::Gemm<0, 0, 256, 256, 128, 1, 2, 1, yan::GemmType::GroupedContiguous>::run_grouped_rows_on_device(
             static_cast<__hip_bfloat16*>(out), lhs, lhs_scales, int(lhs_scales_stride_m), int(lhs_scales_stride_k), rhs, rhs_scales, m_indices,
             num_groups, m, n, k, static_cast<hipStream_t>(stream), num_sms));
@@ -390,7 +414,8 @@ int yan_gemm_select_tile(int op, int m, int n, int k, int num_cus, int* block_m,
     }
     else if (op == 2) pick_grouped(m, n, num_cus, 1, 128, block_m, block_n);
     else if (op == 3) { const yan::FloatTile t = yan::pick_float_tile(m, n, num_cus); *block_m = t.block_m; *block_n = t.block_n; }
-    else if (op == 4) { const bool device = rows_on_device(m, n, num_cus, k); *block_m = device ? 256 : 0; *block_n = device ? 256 : 0; }
+    else if (op == 4) { const bool device = rows_on_device(m, n, 1024, num_cus, k); *block_m = device ? 256 : 0; *block_n = device ? 256 : 0; }
+    else if (op == 5) { const bool device = k > 0 && rows_on_device(m, n, k, num_cus, *block_m); *block_m = device ? 256 : 0; *block_n = device ? 256 : 0; }
     else return 1;
     return 0;
 }

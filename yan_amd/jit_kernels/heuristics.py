@@ -103,18 +103,51 @@ def get_best_grouped_fp8_config(m: int, n: int, k: int, num_cus: int, groups: in
     return rank_tiles(max(m, 1), n, num_cus, table, groups)[0][1]
 
 
+def _tall_then_flat(tall: int, flat: int, num_cus: int) -> float:
+    """When the last of `tall` tiles of 256 x 256 and, behind them, `flat` ones of 128 x 256 ends, in times of a tall tile, with every
+    compute unit taking the next tile when it is done with one."""
+    flat_time = _FP8_TILES[(128, 256)] / 2
+    full, over = divmod(tall, num_cus)          # `over` units run one tall tile more than the others
+    end = full + (1 if over else 0)
+    early, late = full + flat_time, full + 1 + flat_time        # when the next flat tile ends on a unit of either kind
+    while flat > 0:
+        if over == 0 or early <= late:
+            flat -= num_cus - over
+            end = max(end, early)
+            early += flat_time
+        else:
+            flat -= over
+            end = max(end, late)
+            late += flat_time
+    return end
+
+
 def get_contiguous_rows_on_device(m: int, n: int, k: int, num_cus: int, groups_in_m: int) -> bool:
     """Whether a contiguous grouped GEMM runs the kernel whose tiles follow the groups (`fp8_gemm_contiguous_rows_kernel`: 256 x
     256 tiles and, for the odd block of a group, 128 x 256): groups that average a block of 128 rows or more, for which the
     cost table, with 256-row tiles allowed, takes 256 x 256. Against 128 x 256 tiles and 256-row tiles on a fixed grid, which ran
     two passes over K where a tile held two groups: 16 groups of 128 to 768 rows x 4096 x 7168 220 -> 197 us, 4 of about 2500 290 ->
-    276, 7 of about 2300 x 2112 x 5120 210 -> 197, 64 of about 130 x 7168 x 2048 185 -> 172; level (0.5 %) for 4 of 8192 and
-    2 % behind at one shape tried (32 of about 190 x 4096 x 4096). Same rule as `rows_on_device` in
-    yan_amd/csrc/yan_gemm_capi.hip."""
+    276, 7 of about 2300 x 2112 x 5120 210 -> 197; level (0.5 %) for 4 of 8192.
+    Groups that average less than 256 rows have no tile row of 256 rows to every 256: the table counts too few tiles there.
+    They are priced by what runs if every second group has an odd number of blocks, tall tiles first, and by 280 k-rows more
+    for finding the tiles and filling three stages; 128 x 128 tiles cost 1.43 times what the table says next to that (the
+    table comes from plain problems, where their panels are shared). Measured, 128-row tile that the table takes -> this
+    kernel, over 55 shapes with groups of 128 to 255 rows: 64 of about 130 x 7168 x 2048 189 -> 173, 32 of about 190 x 4096 x 4096 148 -> 135,
+    24 of about 165 x 2880 x 2048 49 -> 43 (taken); 49 of about 200 x 1344 x 1280 36.6 -> 41.8, 43 of about 165 x 2112 x 1152 35.4 -> 39.4,
+    46 of about 180 x 1344 x 1024 29.7 -> 31.7, 40 of about 235 x 2304 x 1280 47.5 -> 52.0 (not taken). On 44 further shapes of
+    that class this rule's pick takes 0.57 to 1.006 times the time of the 128-row tile. Same rule as `rows_on_device` in yan_amd/csrc/yan_gemm_capi.hip."""
     if groups_in_m <= 0 or m < 128 * groups_in_m:
         return False
     table = {t: c for t, c in _FP8_TILES.items() if t[1] in (64, 128, 256) and t[0] in (64, 128, 256)}
-    return rank_tiles(m, n, num_cus, table)[0][1] == (256, 256)
+    if rank_tiles(m, n, num_cus, table)[0][1] != (256, 256):
+        return False
+    if m >= 256 * groups_in_m:
+        return True
+    blocks, tiles_n = ceil_div(m, 128), ceil_div(n, 256)
+    tall_rows = (blocks - (groups_in_m + 1) // 2) // 2
+    time = _tall_then_flat(tall_rows * tiles_n, (blocks - 2 * tall_rows) * tiles_n, num_cus) * 65536 * (1 + 280 / max(k, 1))
+    cost, tile = rank_tiles(m, n, num_cus, {t: c for t, c in table.items() if t[0] <= 128})[0]
+    return time < cost * (1.43 if tile == (128, 128) else 1.0)
 
 
 def get_skinny_fp8_config(m: int, n: int, k: int, num_cus: int) -> int:
