@@ -274,6 +274,7 @@ GROUPED_TWO_PASS_CASE = ((8192, -128, 8064, 8192, 8192), 4096, 1024, 1)
 # Sixteen groups of nine blocks: every other boundary falls in the middle of a 256-row tile, and the 73 tile rows are more
 # than the 64 a wave looks at at once when it works out which rows hold two groups (those go first in the launch order).
 GROUPED_TWO_GROUP_ROWS_FIRST_CASE = ((1152,) * 16, 512, 512, 1)
+GROUPED_256_BY_128_CASE = ((2432, 2500, 3072, 2816), 1284, 256, 1)
 GROUPED_CONTIGUOUS_TEST_CASES = [
     GROUPED_TWO_PASS_CASE, GROUPED_TWO_GROUP_ROWS_FIRST_CASE,
     ((100, 128, 1, 300), 320, 384, 1), ((128, 128), 4096, 1024, 0), ((129,), 200, 128, 2),
@@ -284,6 +285,8 @@ GROUPED_CONTIGUOUS_TEST_CASES = [
     # groups of a few hundred rows run the kernel that picks its tile height on the device: every boundary on a multiple of 256 rows
     # (it takes 256 x 256 tiles), every other one in the middle of such a tile (128 x 256 tiles)
     ((512,) * 16, 4096, 1024, 0), ((384, 640) * 8, 4096, 1024, 1),
+    # long groups and more than a round of 256 x 128 tiles, which follow the groups (one of an odd number of blocks, one of padded rows)
+    GROUPED_256_BY_128_CASE,
 ]
 # The same kernel built for small problems through explicit keys (the cost table gives those to smaller tiles): whole
 # 256-row tiles, two groups in every other tile row, and a padding block in the middle with one boundary off.

@@ -646,3 +646,10 @@ def test_time_of_tall_and_flat_tiles_is_that_of_a_list_schedule():
                 for time in [1.0] * tall + [flat_time] * flat:
                     heapq.heapreplace(free, free[0] + time)
                 assert heuristics._tall_then_flat(tall, flat, cus) == pytest.approx(max(free)), (tall, flat, cus)
+
+
+def test_long_contiguous_groups_get_256_by_128_tiles_where_these_are_more_than_a_round():
+    for groups, m, n, k, tile in ((4, 11008, 1284, 256, (256, 128)), (10, 11136, 1408, 1280, (256, 128)), (10, 15104, 2112, 5760, (256, 128)), (6, 11264, 1408, 5504, (256, 128)),
+                                  (4, 5504, 2944, 6528, (256, 128)), (6, 6784, 1152, 6912, (128, 128)), (4, 4352, 1856, 6912, (128, 128)),
+                                  (11, 11136, 1408, 1280, (128, 128))):
+        assert heuristics.get_best_grouped_fp8_config(m, n, k, 256, 1, 128, groups) == tile

@@ -39,14 +39,16 @@ void pick(const TileCost (&tiles)[COUNT], int m, int n, int num_cus, int* bm, in
 }
 
 // Tile of a grouped FP8 GEMM (get_best_grouped_fp8_config in heuristics.py): tiles 64, 128 or 256 wide; with a non-zero
-// `m_alignment` BLOCK_M divides it; the tile count is multiplied by `groups`.
-double pick_grouped(int m, int n, int num_cus, int groups, int m_alignment, int* bm, int* bn) {
+// `m_alignment` BLOCK_M divides it, or the tile is 256 x 128, more than a round of them, and the `groups_in_m` groups (0: not
+// asked) average 1024 rows or more; the tile count is multiplied by `groups`.
+double pick_grouped(int m, int n, int num_cus, int groups, int m_alignment, int groups_in_m, int* bm, int* bn) {
     double best = -1;
     if (m < 1) m = 1;
     for (const TileCost& t : kFp8Tiles) {
-        const bool fits = m_alignment == 0 || m_alignment % t.bm == 0;
-        if ((t.bn != 64 && t.bn != 128 && t.bn != 256) || !fits) continue;
         const long long count  = (long long)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * groups;
+        const bool fits = m_alignment == 0 || m_alignment % t.bm == 0 ||
+                          (t.bm == 2 * m_alignment && t.bn == 128 && groups_in_m > 0 && m >= 1024ll * groups_in_m && count > num_cus);
+        if ((t.bn != 64 && t.bn != 128 && t.bn != 256) || !fits) continue;
         const long long rounds = (count + num_cus - 1) / num_cus;
         const double cost = double(rounds) * t.bm * t.bn * t.per_area;
         if (best < 0 || cost < best || (cost == best && (t.bm < *bm || (t.bm == *bm && t.bn < *bn)))) { best = cost; *bm = t.bm; *bn = t.bn; }
@@ -90,7 +92,7 @@ bool rows_on_device(int m, int n, int k, int num_cus, int groups_in_m) {
     const long long tiles_n = (n + 255) / 256;
     const double time = tall_then_flat(tall_rows * tiles_n, (blocks - 2 * tall_rows) * tiles_n, num_cus) * 65536 * (1 + 280.0 / k);
     int bm = 0, bn = 0;
-    const double cost = pick_grouped(m, n, num_cus, 1, 128, &bm, &bn);
+    const double cost = pick_grouped(m, n, num_cus, 1, 128, 0, &bm, &bn);
     return time < cost * (bm == 128 && bn == 128 ? 1.43 : 1.0);
 }
 
@@ -353,13 +355,13 @@ int yan_m_grouped_gemm_fp8_fp8_bf16_nt_contiguous(const void* lhs, const float* 
             static_cast<__hip_bfloat16*>(out), lhs, lhs_scales, int(lhs_scales_stride_m), int(lhs_scales_stride_k), rhs, rhs_scales, m_indices,
             num_groups, m, n, k, static_cast<hipStream_t>(stream), num_sms));
     int bm = 0, bn = 0;
-    pick_grouped(m, n, cus, 1, 128, &bm, &bn);
+    pick_grouped(m, n, cus, 1, 128, num_groups, &bm, &bn);
 #define YAN_GROUPED_CASE(BM, BN)                                                                                     \
     if (bm == BM && bn == BN)                                                                                        \
         return int(yan::Gemm<0, 0, BM, BN, 128, 1, yan::Fp8TileConfig<BM, BN>::MAX_RING_STAGES, 1, yan::GemmType::GroupedContiguous>::run_grouped(             \
             static_cast<__hip_bfloat16*>(out), lhs, lhs_scales, int(lhs_scales_stride_m), int(lhs_scales_stride_k), 0, rhs, \
             rhs_scales, m_indices, num_groups, m, n, k, static_cast<hipStream_t>(stream), num_sms));
-    YAN_GROUPED_CASE(128, 256) YAN_GROUPED_CASE(128, 128)
+    YAN_GROUPED_CASE(256, 128) YAN_GROUPED_CASE(128, 256) YAN_GROUPED_CASE(128, 128)
     YAN_GROUPED_CASE(64, 128) YAN_GROUPED_CASE(64, 64)
 #undef YAN_GROUPED_CASE
     return int(hipErrorInvalidValue);
@@ -376,7 +378,7 @@ int yan_m_grouped_gemm_fp8_fp8_bf16_nt_masked(const void* lhs, const float* lhs_
         lhs_scales_stride_g >= (1ll << 31)) return int(hipErrorInvalidValue);
     const int cus = (num_sms > 0 && num_sms < device_cus()) ? num_sms : device_cus();
     int bm = 0, bn = 0;
-    pick_grouped(expected_m < m_max ? expected_m : m_max, n, cus, num_groups, 0, &bm, &bn);
+    pick_grouped(expected_m < m_max ? expected_m : m_max, n, cus, num_groups, 0, 0, &bm, &bn);
 #define YAN_GROUPED_CASE(BM, BN)                                                                                     \
     if (bm == BM && bn == BN)                                                                                        \
         return int(yan::Gemm<0, 0, BM, BN, 128, 1, yan::Fp8TileConfig<BM, BN>::MAX_RING_STAGES, 1, yan::GemmType::GroupedMasked>::run_grouped(                 \
@@ -412,7 +414,7 @@ int yan_gemm_select_tile(int op, int m, int n, int k, int num_cus, int* block_m,
         if (const int atoms = skinny_atoms(m, n, num_cus)) { *block_m = 16 * atoms; *block_n = 16; }
         else pick(kFp8Tiles, m, n, num_cus, block_m, block_n);
     }
-    else if (op == 2) pick_grouped(m, n, num_cus, 1, 128, block_m, block_n);
+    else if (op == 2) pick_grouped(m, n, num_cus, 1, 128, k, block_m, block_n);
     else if (op == 3) { const yan::FloatTile t = yan::pick_float_tile(m, n, num_cus); *block_m = t.block_m; *block_n = t.block_n; }
     else if (op == 4) { const bool device = rows_on_device(m, n, 1024, num_cus, k); *block_m = device ? 256 : 0; *block_n = device ? 256 : 0; }
     else if (op == 5) { const bool device = k > 0 && rows_on_device(m, n, k, num_cus, *block_m); *block_m = device ? 256 : 0; *block_n = device ? 256 : 0; }
@@ -428,6 +430,6 @@ int yan_gemm_select_split_k(int op, int m, int n, int k, int num_cus, int* block
     return 0;
 }
 
-const char* yan_gemm_version(void) { return "yan-gemm gfx950 11 dense + 22 split-K dense + 2 weight-streaming dense + 7 fp32 + 10 fp8 tile variants + 15 split-K fp8 variants + 1 weight-streaming fp8 variant + 11 grouped fp8 variants + 4 quantiser kernels"; }
+const char* yan_gemm_version(void) { return "yan-gemm gfx950 11 dense + 22 split-K dense + 2 weight-streaming dense + 7 fp32 + 10 fp8 tile variants + 15 split-K fp8 variants + 1 weight-streaming fp8 variant + 12 grouped fp8 variants + 4 quantiser kernels"; }
 
 } // extern "C"

@@ -94,12 +94,17 @@ def get_fp8_num_stages(block_m: int, block_n: int) -> int:
 def get_best_grouped_fp8_config(m: int, n: int, k: int, num_cus: int, groups: int = 1, m_alignment: int = 0,
                                 groups_in_m: int = 1) -> Tuple[int, int]:
     """Tile of a grouped FP8 GEMM, among the tiles 64, 128 or 256 columns wide. Contiguous layout: `m` is the total row count and
-    `m_alignment` the padding of every group, which the tile's rows must divide (taller tiles belong to the kernel that places
-    them on the device, `get_contiguous_rows_on_device`). Masked layout: `m` is the expected row count of one group and `groups`
-    multiplies the tile count. `groups_in_m` (the groups sharing the rows of the contiguous layout) does not matter here."""
-    def allowed(bm):
-        return m_alignment == 0 or m_alignment % bm == 0
-    table = {t: c for t, c in _FP8_TILES.items() if t[1] in (64, 128, 256) and allowed(t[0])}
+    `m_alignment` the padding of every group, which the tile's rows must divide. 256 x 128, whose tiles follow the `groups_in_m`
+    groups as the 256 x 256 ones of `get_contiguous_rows_on_device` do, is offered when they average 1024 rows or more and the
+    tiles are more than one round: 10 groups, 11136 x 1408 x 1280 61 us on 128 x 128 tiles, 43 on these; 10 groups, 15104 x 2112 x
+    5760 255 and 227; 23 such shapes 0.71 to 1.04 times the time on 128 x 128. In one round it loses (6 groups, 6784 x 1152 x
+    6912: 77 us on 128 x 128, 88 on these). Masked layout: `m` is the expected row count of one group and `groups` multiplies
+    the tile count."""
+    def allowed(bm, bn):
+        if m_alignment == 0 or m_alignment % bm == 0:
+            return True
+        return (bm, bn) == (2 * m_alignment, 128) and m >= 1024 * groups_in_m and ceil_div(m, bm) * ceil_div(n, bn) > num_cus
+    table = {t: c for t, c in _FP8_TILES.items() if t[1] in (64, 128, 256) and allowed(*t)}
     return rank_tiles(max(m, 1), n, num_cus, table, groups)[0][1]
 
 
