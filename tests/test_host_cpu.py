@@ -653,3 +653,19 @@ def test_long_contiguous_groups_get_256_by_128_tiles_where_these_are_more_than_a
                                   (4, 5504, 2944, 6528, (256, 128)), (6, 6784, 1152, 6912, (128, 128)), (4, 4352, 1856, 6912, (128, 128)),
                                   (11, 11136, 1408, 1280, (128, 128))):
         assert heuristics.get_best_grouped_fp8_config(m, n, k, 256, 1, 128, groups) == tile
+
+
+@pytest.mark.parametrize('m,n,k', [(330, 3648, 256), (300, 4004, 256)])
+def test_fp8_kernels_of_two_k_tiles_compile(tmp_path, m, n, k):
+    """64 x 128 tiles with K = 256: every LDS address of the unrolled loop is known at compile time."""
+    import subprocess
+    from yan_amd.jit import cpp_format, generate
+    from yan_amd.jit.compiler import get_hipcc_compiler, get_jit_include_dir, get_offload_arch
+    from yan_amd.jit_kernels import gemm
+    _, keys, arg_defs, _, template = gemm.fp8_kernel_plan(m, n, k, 256, True)
+    assert (keys['BLOCK_M'], keys['BLOCK_N']) == (64, 128)
+    src = tmp_path / 'kernel.cu'
+    src.write_text(generate(gemm.includes, arg_defs, cpp_format(template, keys)))
+    subprocess.check_call([get_hipcc_compiler()[0], '-x', 'hip', '--cuda-device-only', '-S', '-std=c++20', '-O3', f'--offload-arch={get_offload_arch()}',
+                           '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops', f'-I{get_jit_include_dir()}', str(src),
+                           '-o', str(tmp_path / 'kernel.s')])

@@ -28,7 +28,9 @@ constexpr int kChunk     = 16;    // bytes moved per lane per memory instruction
 constexpr int kNumXCD    = 8;     // MI355X: 8 accelerator dies, 32 CUs and one 4 MB L2 each
 
 #define YAN_GLOBAL_PTR(p) ((const __attribute__((address_space(1))) void*)(p))
-#define YAN_LDS_PTR(p)    ((__attribute__((address_space(3))) void*)(p))
+// By way of the offset (the low half of a flat address): a cast of the pointer itself asks whether it is null, a compare that
+// costs instructions, and one that the compiler cannot encode where the address is known at compile time (FP8, 64 x 128 tile, K = 256).
+#define YAN_LDS_PTR(p)    ((__attribute__((address_space(3))) void*)(uint32_t)(uintptr_t)(p))
 
 // s_waitcnt immediates on gfx9: vmcnt = bits [3:0] | [15:14], expcnt [6:4], lgkmcnt [11:8].
 __host__ __device__ constexpr int waitcnt_imm(int vmcnt, int lgkmcnt) {
