@@ -669,3 +669,19 @@ def test_fp8_kernels_of_two_k_tiles_compile(tmp_path, m, n, k):
     subprocess.check_call([get_hipcc_compiler()[0], '-x', 'hip', '--cuda-device-only', '-S', '-std=c++20', '-O3', f'--offload-arch={get_offload_arch()}',
                            '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops', f'-I{get_jit_include_dir()}', str(src),
                            '-o', str(tmp_path / 'kernel.s')])
+
+
+@pytest.mark.parametrize('tile,k', [((128, 128), 1152), ((128, 256), 768), ((256, 128), 512)])
+def test_fp8_ring_tiles_do_not_spill_where_k_is_short(tmp_path, tile, k):
+    import re
+    import subprocess
+    import harness as testing
+    from yan_amd.jit import cpp_format, generate
+    from yan_amd.jit.compiler import get_hipcc_compiler, get_jit_include_dir, get_offload_arch
+    from yan_amd.jit_kernels import gemm
+    _, keys, arg_defs, template = testing.fp8_explicit_tile_plan(*tile, 4096, k)
+    src, asm = tmp_path / 'kernel.cu', tmp_path / 'kernel.s'
+    src.write_text(generate(gemm.includes, arg_defs, cpp_format(template, keys)))
+    subprocess.check_call([get_hipcc_compiler()[0], '-x', 'hip', '--cuda-device-only', '-S', '-std=c++20', '-O3', f'--offload-arch={get_offload_arch()}',
+                           '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops', f'-I{get_jit_include_dir()}', str(src), '-o', str(asm)])
+    assert set(re.findall(r'vgpr_spill_count: *(\d+)', asm.read_text())) == {'0'}

@@ -596,7 +596,7 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
         for (int d = 0; d < OPS; ++d) issue_op(d, kb_lo + t, ring + t * STAGE_BYTES);
     load_weight_scales(min(kb_lo, NUM_K_BLOCKS - 1));
     int st = 0;
-    for (int kb = kb_lo; kb < kb_hi; ++kb) {
+    auto ring_step = [&](int kb) {
 #pragma unroll
         for (int b = 0; b < NB; ++b) sb_cur[b] = sb_next[b];
         __builtin_amdgcn_s_waitcnt(waitcnt_imm((STAGES - 2) * OPS, kNoWaitLgkm));
@@ -616,6 +616,21 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
                 if (d * SPREAD_ROWS / OPS == row) issue_op(d, kb + STAGES - 1, nxt);
         });
         st = st + 1 == STAGES ? 0 : st + 1;
+    };
+    // Unrolled in full where K is compiled in and short: worth 3 to 10 % (422 x 9088 x 1280 on 64 x 128 tiles 15.5 -> 14.0 us), but
+    // left to itself the compiler goes on where it has no registers for it any more, tiles of 16 atoms a wave from 4 k-tiles
+    // on, of 8 from 9, and spills among the copies, whose waits then are waits for the scratch memory too
+    // (1301 x 5824 x 768 on 128 x 256: 37 us, 12.4 as a loop; 376 x 8320 x 1280 on 128 x 128: 13.5 and 10.4; 370 x 9216 x 1152 12.0
+    // or 14.4 by where the spills fall). Those stay loops. Longer ones, and run-time K, are as the compiler has them.
+    constexpr int ATOMS = TN * TM, K_TILES = SPLIT_K > 1 ? 0 : SHAPE_K / 128, UNROLLED = ATOMS > 8 ? 3 : (ATOMS > 4 ? 8 : (ATOMS > 2 ? 12 : 16));
+    if constexpr (K_TILES > 0 && K_TILES <= UNROLLED) {
+#pragma unroll
+        for (int kb = kb_lo; kb < kb_hi; ++kb) ring_step(kb);
+    } else if constexpr (K_TILES > 0 && ATOMS >= 8) {
+#pragma unroll 1
+        for (int kb = kb_lo; kb < kb_hi; ++kb) ring_step(kb);
+    } else {
+        for (int kb = kb_lo; kb < kb_hi; ++kb) ring_step(kb);
     }
     epi_a = ring + (st == 0 ? STAGES - 1 : st - 1) * STAGE_BYTES;
     epi_b = epi_a + A_BYTES;
