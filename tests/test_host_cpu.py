@@ -623,12 +623,12 @@ def test_contiguous_keys_may_name_any_tile_of_256_rows(tmp_path):
 
 # (groups, rows, n, k): microseconds of the 128-row tile the cost table takes and of the kernel whose tiles follow the groups (MI355X,
 # router-like layouts)
-SHORT_GROUPS = {(49, 9856, 1344, 1280): (36.6, 41.8), (43, 7040, 2112, 1152): (35.4, 39.4), (46, 8320, 1344, 1024): (29.7, 31.7),
-                (29, 3712, 4352, 2560): (69.7, 74.4), (33, 4608, 3392, 1792): (50.5, 52.6), (40, 9344, 2304, 1280): (47.5, 52.0),
-                (41, 8448, 1600, 1664): (41.2, 47.3), (21, 2688, 5824, 1536): (46.6, 47.6),
-                (64, 8320, 7168, 2048): (188.9, 173.0), (32, 6144, 4096, 4096): (148.4, 135.4), (24, 3968, 2880, 2048): (48.7, 42.7),
-                (23, 2944, 4032, 1664): (43.1, 39.4), (50, 9728, 1152, 1408): (36.4, 33.4), (10, 1280, 7168, 2048): (44.5, 33.5),
-                (29, 6784, 4160, 1152): (98.7, 59.1), (13, 1920, 4992, 2560): (56.9, 43.3), (59, 11392, 6144, 2176): (222.5, 206.1)}
+SHORT_GROUPS = {(49, 9856, 1344, 1280): (34.1, 40.1), (43, 7040, 2112, 1152): (32.7, 38.8), (46, 8320, 1344, 1024): (28.0, 31.9),
+                (29, 3712, 4352, 2560): (67.8, 73.6), (33, 4608, 3392, 1792): (48.2, 51.8), (41, 8448, 1600, 1664): (40.3, 46.4),
+                (21, 2688, 5824, 1536): (45.5, 46.9),
+                (64, 8320, 7168, 2048): (190.5, 174.8), (32, 6144, 4096, 4096): (142.3, 130.0), (24, 3968, 2880, 2048): (46.2, 41.2),
+                (23, 2944, 4032, 1664): (41.5, 38.9), (50, 9728, 1152, 1408): (36.0, 32.6), (10, 1280, 7168, 2048): (44.0, 33.9),
+                (29, 6784, 4160, 1152): (66.7, 57.7), (13, 1920, 4992, 2560): (55.9, 42.0), (59, 11392, 6144, 2176): (223.7, 203.2)}
 
 
 def test_short_contiguous_groups_get_the_kernel_that_measured_faster():

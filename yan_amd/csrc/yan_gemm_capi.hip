@@ -90,10 +90,11 @@ bool rows_on_device(int m, int n, int k, int num_cus, int groups_in_m) {
     if ((long long)m >= 256ll * groups_in_m) return true;
     const int blocks = (m + 127) / 128, tall_rows = (blocks - (groups_in_m + 1) / 2) / 2;
     const long long tiles_n = (n + 255) / 256;
-    const double time = tall_then_flat(tall_rows * tiles_n, (blocks - 2 * tall_rows) * tiles_n, num_cus) * 65536 * (1 + 280.0 / k);
+    const double time = tall_then_flat(tall_rows * tiles_n, (blocks - 2 * tall_rows) * tiles_n, num_cus);
     int bm = 0, bn = 0;
     const double cost = pick_grouped(m, n, num_cus, 1, 128, 0, &bm, &bn);
-    return time < cost * (bm == 128 && bn == 128 ? 1.43 : 1.0);
+    if (bm == 128 && bn == 128) return time * (1 + 180.0 / k) * 65536 < cost * 1.36;
+    return (time + 750.0 / k) * 65536 < cost;
 }
 
 // Activation atoms of the weight-streaming kernel, or 0 for the tiled kernel (get_skinny_fp8_config in heuristics.py).

@@ -134,13 +134,14 @@ def get_contiguous_rows_on_device(m: int, n: int, k: int, num_cus: int, groups_i
     two passes over K where a tile held two groups: 16 groups of 128 to 768 rows x 4096 x 7168 220 -> 197 us, 4 of about 2500 290 ->
     276, 7 of about 2300 x 2112 x 5120 210 -> 197; level (0.5 %) for 4 of 8192.
     Groups that average less than 256 rows have no tile row of 256 rows to every 256: the table counts too few tiles there.
-    They are priced by what runs if every second group has an odd number of blocks, tall tiles first, and by 280 k-rows more
-    for finding the tiles and filling three stages; 128 x 128 tiles cost 1.43 times what the table says next to that (the
-    table comes from plain problems, where their panels are shared). Measured, 128-row tile that the table takes -> this
-    kernel, over 55 shapes with groups of 128 to 255 rows: 64 of about 130 x 7168 x 2048 189 -> 173, 32 of about 190 x 4096 x 4096 148 -> 135,
-    24 of about 165 x 2880 x 2048 49 -> 43 (taken); 49 of about 200 x 1344 x 1280 36.6 -> 41.8, 43 of about 165 x 2112 x 1152 35.4 -> 39.4,
-    46 of about 180 x 1344 x 1024 29.7 -> 31.7, 40 of about 235 x 2304 x 1280 47.5 -> 52.0 (not taken). On 44 further shapes of
-    that class this rule's pick takes 0.57 to 1.006 times the time of the 128-row tile. Same rule as `rows_on_device` in yan_amd/csrc/yan_gemm_capi.hip."""
+    They are priced by what runs if every second group has an odd number of blocks, tall tiles first. Next to 128 x 256 tiles a
+    launch takes 750 k-rows of a tall tile more, for finding the tiles and filling three stages; next to 128 x 128 tiles, whose
+    rounds each have a start of their own, 180 per round, and those cost 1.36 times what the table says (it comes from plain
+    problems, where their panels are shared). Measured, 128-row tile that the table takes -> this kernel: 64 of about 130 x 7168 x
+    2048 190 -> 175, 32 of about 190 x 4096 x 4096 142 -> 130, 24 of about 165 x 2880 x 2048 46 -> 41 (taken); 49 of about 200 x 1344 x
+    1280 34.1 -> 40.1, 43 of about 165 x 2112 x 1152 32.7 -> 38.8, 46 of about 180 x 1344 x 1024 28.0 -> 31.9, 41 of about 205 x 1600 x
+    1664 40.3 -> 46.4 (not taken). Over the 78 shapes the rule was made on its pick takes 0.90 of the time of the 128-row tile (1.04
+    at worst), over 44 others 0.74 to 1.02. Same rule as `rows_on_device` in yan_amd/csrc/yan_gemm_capi.hip."""
     if groups_in_m <= 0 or m < 128 * groups_in_m:
         return False
     table = {t: c for t, c in _FP8_TILES.items() if t[1] in (64, 128, 256) and t[0] in (64, 128, 256)}
@@ -150,9 +151,11 @@ def get_contiguous_rows_on_device(m: int, n: int, k: int, num_cus: int, groups_i
         return True
     blocks, tiles_n = ceil_div(m, 128), ceil_div(n, 256)
     tall_rows = (blocks - (groups_in_m + 1) // 2) // 2
-    time = _tall_then_flat(tall_rows * tiles_n, (blocks - 2 * tall_rows) * tiles_n, num_cus) * 65536 * (1 + 280 / max(k, 1))
+    time = _tall_then_flat(tall_rows * tiles_n, (blocks - 2 * tall_rows) * tiles_n, num_cus)
     cost, tile = rank_tiles(m, n, num_cus, {t: c for t, c in table.items() if t[0] <= 128})[0]
-    return time < cost * (1.43 if tile == (128, 128) else 1.0)
+    if tile == (128, 128):
+        return time * (1 + 180 / max(k, 1)) * 65536 < cost * 1.36
+    return (time + 750 / max(k, 1)) * 65536 < cost
 
 
 def get_skinny_fp8_config(m: int, n: int, k: int, num_cus: int) -> int:
