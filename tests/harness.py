@@ -216,9 +216,9 @@ REFERENCE_FLOAT_TEST_SHAPES = [(m, n, k) for m in (128, 4096)
 FLOAT_TEST_SHAPES = [(128, 64, 16), (128, 64, 1), (128, 192, 17), (256, 320, 100), (384, 1024, 260), (128, 24576, 40),
                      (512, 4096, 40), (256, 32768, 24), (4096, 32768, 8)]
 # fp32 problems that split K: (m, n, k) -> (BLOCK_M, BLOCK_N, parts), every tile of the plans
-FLOAT_SPLIT_K_SHAPES = {(128, 64, 2050): (32, 32, 7), (256, 320, 3001): (32, 32, 3), (384, 320, 3001): (32, 64, 4), (128, 576, 4099): (32, 64, 7),
-                        (1024, 320, 2050): (64, 64, 3), (640, 320, 7168): (64, 64, 5), (640, 1088, 4099): (128, 64, 3),
-                        (128, 2112, 9001): (128, 64, 7)}
+FLOAT_SPLIT_K_SHAPES = {(128, 64, 2050): (32, 32, 7), (256, 320, 3001): (32, 32, 3), (384, 320, 3001): (32, 64, 4), (128, 576, 4099): (32, 64, 6),
+                        (1024, 320, 2050): (64, 64, 3), (256, 704, 4110): (64, 64, 5), (256, 2112, 2111): (128, 64, 3),
+                        (128, 2112, 9001): (64, 64, 7), (640, 832, 1997): (128, 64, 7)}
 FP8_TEST_SHAPES = [
     (4096, 7168, 7168), (64, 4096, 7168), (16384, 16384, 16384),
     (64, 256, 384), (512, 1024, 1024), (1, 128, 128), (63, 192, 256), (129, 320, 128), (300, 96, 640),

@@ -332,16 +332,18 @@ FLOAT_SPLIT_K_FACTORS = (2, 3, 4, 5, 6, 7, 8)
 def get_split_k_float_config(m: int, n: int, k: int, num_cus: int) -> Optional[Tuple[int, int, int]]:
     """(BLOCK_M, BLOCK_N, SPLIT_K) when the fp32 GEMM should split K over SPLIT_K workgroups per tile, else None. The matrix cores
     bound this GEMM, so what splitting buys is an even share of the work: 128 x 2112 has 132 tiles of 32 x 64 for 256 compute
-    units, and 462 parts of 64 x 64 tiles in seven are two almost full rounds. Modelled time of a plan: rounds x the tile's time
-    for its k-rows + 6 us (launch, first copies, the meeting) + 12.5 ns per KB of partial sums the last part reads; taken when it
-    is below 0.88 of the unsplit pick's. Measured (unsplit -> plan, operands cycling): 128 x 2112 x 7168 57 -> 40 us,
-    256 x 2112 x 7168 86 -> 67, 128 x 256 x 8192 35 -> 11. On 19 shapes swept with four tiles and every factor the plan is within 3 %
-    of the fastest measured; shapes whose best plan gains less than 5 % (128 x 4096 x 7168 64 -> 62) stay unsplit."""
+    units, and 462 parts of 64 x 64 tiles in seven are two almost full rounds. The parts of a tile run on one XCD, so a round is a
+    part on each of the 32 units of the XCD that has most tiles: 50 tiles of 64 x 64 are 7 on seven XCDs and 1 on the last,
+    35 parts in five, two rounds (640 x 320 x 7168: 49 us that way, 38 unsplit). Modelled time of a plan: rounds x (the tile's
+    time for its k-rows + 1 us) + 5 us (launch, first copies, the meeting) + 12.5 ns per KB of partial sums the last part reads;
+    taken when it is below 0.92 of the unsplit pick's and 1.2 us, the longer way through the entry, below it. Measured (unsplit ->
+    plan, operands cycling): 128 x 2112 x 7168 58 -> 45 us, 256 x 2112 x 7168 93 -> 75, 128 x 256 x 8192 36 -> 12; 264 shapes that
+    split 0.32 to 0.99 times the unsplit time, 0.78 on average."""
     if m <= 0 or n <= 0 or k <= 0:
         return None
     tile = get_best_float_config(m, n, num_cus)
     base = ceil_div(ceil_div(m, tile[0]) * ceil_div(n, tile[1]), num_cus) * _FLOAT_US_PER_1024_K[tile] * k / 1024 + 3.5
-    best, best_plan = 0.88 * base, None
+    best, best_plan = min(0.92 * base, base - 1.2), None
     for (bm, bn), block_k in _FLOAT_BLOCK_K.items():
         tiles, k_tiles = ceil_div(m, bm) * ceil_div(n, bn), ceil_div(k, block_k)
         slots = ceil_div(tiles, 8) * 8
@@ -350,7 +352,8 @@ def get_split_k_float_config(m: int, n: int, k: int, num_cus: int) -> Optional[T
             part = ceil_div(k_tiles, split) * block_k
             if slots * split * bm * bn * 4 > 1 << 24 or slots > 1024 or part < 256:
                 continue
-            t = ceil_div(tiles * split, num_cus) * _FLOAT_US_PER_1024_K[(bm, bn)] * part / 1024 + 6 + split * bm * bn * 4 / 1024 * 0.0125
+            rounds = ceil_div(slots // 8 * split, max(num_cus // 8, 1))
+            t = rounds * (_FLOAT_US_PER_1024_K[(bm, bn)] * part / 1024 + 1) + 5 + split * bm * bn * 4 / 1024 * 0.0125
             if t < best:
                 best, best_plan = t, (bm, bn, split)
     return best_plan
