@@ -709,3 +709,22 @@ def test_fp32_split_k_counts_the_rounds_of_the_fullest_xcd():
                     rounds = ceil_div(ceil_div(ceil_div(m, tile[0]) * ceil_div(n, tile[1]), 8) * split, 32)
                     whole = heuristics.get_best_float_config(m, n, 256)
                     assert rounds * us[tile] / split < ceil_div(ceil_div(m, whole[0]) * ceil_div(n, whole[1]), 256) * us[whole]
+
+
+@pytest.mark.parametrize('kind,streams_codes', [('per_token', False), ('per_block', True)])
+def test_codes_of_activations_are_stored_for_the_gemm_behind(tmp_path, kind, streams_codes):
+    """The GEMM that follows a per-token cast reads its codes from the caches: no store of them carries the non-temporal hint.
+    Weights are quantised ahead of time, those of a large matrix go past the caches."""
+    import re
+    import subprocess
+    from yan_amd.jit import cpp_format, generate
+    from yan_amd.jit.compiler import get_hipcc_compiler, get_jit_include_dir, get_offload_arch
+    from yan_amd.jit_kernels import fp8_cast
+    _, keys, arg_defs, template = fp8_cast.cast_kernel_plan(kind, torch.bfloat16)
+    src, asm = tmp_path / 'kernel.cu', tmp_path / 'kernel.s'
+    src.write_text(generate(fp8_cast.includes, arg_defs, cpp_format(template, keys)))
+    subprocess.check_call([get_hipcc_compiler()[0], '-x', 'hip', '--cuda-device-only', '-S', '-std=c++20', '-O3', f'--offload-arch={get_offload_arch()}',
+                           '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops', f'-I{get_jit_include_dir()}', str(src), '-o', str(asm)])
+    text = asm.read_text()
+    assert re.search(r'global_load\S* .* nt\b', text)
+    assert bool(re.search(r'global_store\S* .* nt\b', text)) == streams_codes

@@ -27,14 +27,18 @@ namespace yan {
 constexpr float kFp8Max = 448.0f;
 
 // How a launch treats the caches. Sources and codes that outgrow the L2s together (8 x 4 MB) only push each other out
-// of them: past that size each of the two is moved with the non-temporal hint. Below it the plain forms are as fast or
-// faster (64 x 7168: 2.5 us plain, 2.7 with either hint) and leave the codes in L2 for the GEMM that follows. Measured
-// cold, bf16, token-contiguous scales, kPlain / kStreamSource / kStreamBoth: 4096 x 7168 (59 MB read, 29 written)
-// 17.5 / 16.0 / 16.3 us, 16384 x 7168 64.0 / 61.7 / 59.3; per block 16384 x 7168 66.1 / 62.3 / 59.6.
+// of them: past that size sources are moved with the non-temporal hint, and so are the codes of weights, which nobody reads
+// for a while. Those of activations are read at once, by the GEMM behind, which finds them in the memory-side cache only if
+// they were stored plainly: per-token cast and GEMM together, codes streamed / plain, 6144 x 7168 (x 2112 outputs) 117.5 / 114.9 us,
+// 16384 x 7168 (x 2112) 293 / 276, 12288 x 4096 (x 512) 62.4 / 59.3. Small launches take the plain forms, which are as fast or
+// faster (64 x 7168: 2.5 us plain, 2.7 with either hint). Measured cold and alone, bf16, token-contiguous scales, kPlain /
+// kStreamSource / kStreamBoth: 4096 x 7168 (59 MB read, 29 written) 17.5 / 16.0 / 16.3 us, 16384 x 7168 64.0 / 61.7 / 59.3; per
+// block 16384 x 7168 66.1 / 62.3 / 59.6.
 enum CastStream { kPlain, kStreamSource, kStreamBoth };
 constexpr long long kCastL2Bytes = 32ll << 20;
-inline CastStream cast_stream(long long elements, int bytes_per_element) {
-    return elements > kCastL2Bytes ? kStreamBoth : (elements * bytes_per_element > kCastL2Bytes ? kStreamSource : kPlain);
+inline CastStream cast_stream(long long elements, int bytes_per_element, bool codes_read_next) {
+    if (elements > kCastL2Bytes && !codes_read_next) return kStreamBoth;
+    return elements * bytes_per_element > kCastL2Bytes ? kStreamSource : kPlain;
 }
 
 // Eight elements of a group as loaded, and as fp32: lane `part` of the group's sixteen has 8 part .. 8 part + 7 of bf16 and, so
@@ -214,11 +218,9 @@ inline hipError_t launch_per_token_cast(const T* x, void* q, float* scales, long
                            uint32_t(m), uint32_t(k_blocks), stride_m, stride_k);
         return hipGetLastError();
     };
-    switch (cast_stream(groups * 128, sizeof(T))) {
-        case kPlain: return by_rows ? launch(per_token_cast_kernel<T, UNROLL, true, kPlain>) : launch(per_token_cast_kernel<T, UNROLL, false, kPlain>);
-        case kStreamSource: return by_rows ? launch(per_token_cast_kernel<T, UNROLL, true, kStreamSource>) : launch(per_token_cast_kernel<T, UNROLL, false, kStreamSource>);
-        default: return by_rows ? launch(per_token_cast_kernel<T, UNROLL, true, kStreamBoth>) : launch(per_token_cast_kernel<T, UNROLL, false, kStreamBoth>);
-    }
+    if (cast_stream(groups * 128, sizeof(T), true) == kPlain)
+        return by_rows ? launch(per_token_cast_kernel<T, UNROLL, true, kPlain>) : launch(per_token_cast_kernel<T, UNROLL, false, kPlain>);
+    return by_rows ? launch(per_token_cast_kernel<T, UNROLL, true, kStreamSource>) : launch(per_token_cast_kernel<T, UNROLL, false, kStreamSource>);
 }
 
 // w [n, k] -> q [n, k] e4m3, scales fp32 [ceil(n/128), k/128] row-major.
@@ -233,7 +235,7 @@ inline hipError_t launch_per_block_cast(const T* w, void* q, float* scales, int 
         hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(blocks)), dim3(256), 0, stream, w, static_cast<uint8_t*>(q), scales, n, k);
         return hipGetLastError();
     };
-    switch (cast_stream(static_cast<long long>(n) * k, sizeof(T))) {
+    switch (cast_stream(static_cast<long long>(n) * k, sizeof(T), false)) {
         case kPlain: return launch(per_block_cast_kernel<T, kPlain>);
         case kStreamSource: return launch(per_block_cast_kernel<T, kStreamSource>);
         default: return launch(per_block_cast_kernel<T, kStreamBoth>);
