@@ -320,6 +320,19 @@ NUM_SMS_CAP = 64
 CAPPED_SHAPES = [(2048, 4096, 1024), (512, 4096, 2048), (300, 2112, 640)]
 
 
+# Dense ring tiles walked under a cap where their copying waves end a k-tile early and meet no staged epilogue: rows of the output
+# that are 8 but not 16 bytes apart, a k tail, fewer k-tiles than stages. Tiles, (m, n), depths, cap.
+DENSE_RAGGED_CAP_CASE = ([(128, 128), (128, 192), (64, 64), (256, 128)], (390, 516), (72, 200), 8)
+
+
+def dense_tile_plan(tile, dtype: torch.dtype, cap: int):
+    """(name, keys, arg_defs, includes, template) of the dense GEMM on a tile given outright."""
+    from yan_amd.jit_kernels import bf16_gemm, heuristics
+    keys = {'BLOCK_M': tile[0], 'BLOCK_N': tile[1], 'NUM_STAGES': heuristics.get_dense_num_stages(*tile), 'NUM_SMS': cap}
+    return ('gemm_bf16_tn' if dtype == torch.bfloat16 else 'gemm_fp16_tn', keys, bf16_gemm._arg_defs(dtype), bf16_gemm.includes,
+            bf16_gemm.template)
+
+
 # A problem of 6 x 3 tiles of 256 x 256 (18: not a multiple of the 8 XCDs, so some XCDs' ranges end in an empty slot) run by
 # 3 and 5 workgroups: walks that cross the XCDs' ranges. (m, n, k), caps.
 ODD_CAP_CASE = ((1300, 768, 512), (3, 5))
@@ -446,6 +459,11 @@ def jit_kernels_in_use(num_cus: int = 256):
     for cap in (0,) + ODD_CAP_CASE[1]:
         for name, keys, arg_defs, includes, code_template in odd_cap_plans(cap):
             add(name, arg_defs, includes, code_template, keys)
+    for tile in DENSE_RAGGED_CAP_CASE[0]:
+        for dtype in (torch.bfloat16, torch.half):
+            for cap in (0, DENSE_RAGGED_CAP_CASE[3]):
+                name, keys, arg_defs, includes, code_template = dense_tile_plan(tile, dtype, cap)
+                add(name, arg_defs, includes, code_template, keys)
     for m, n, k in TUNED_SHAPES:
         name, keys, space, arg_defs = bf16_gemm.dense_tuning_plan(m, n, k, torch.bfloat16, num_cus)
         for extra in space:

@@ -8,8 +8,8 @@
 //     exactly once and, for grids that are multiples of 8, never leaves the XCD residue b % 8;
 //   * the masked layout's slot numbering (MaskedSlots) visits every (group, tile) once, likely tile rows first, and bands
 //     fitted to the height of a group lose no tile and keep a patch inside one group;
-//   * the contiguous layout's slot numbering on 256-row tiles (ContiguousSlots) visits every tile once within the launched
-//     slots for any number of two-group rows, and deals those rows' tiles evenly to the XCDs, first in each;
+//   * the contiguous layout cut along its groups (ContiguousBlock) covers every block of a group exactly once, no tile reaches
+//     from one group into another, and the slots of the tall and flat tiles fit the launched ones and visit every tile once;
 //   * the same holds in region order (operand rows long enough that the problem outgrows the memory-side cache), whose
 //     choice of region is pinned for a few measured shapes.
 #include "gemm/scheduler.hpp"
@@ -119,35 +119,61 @@ int main() {
                     for (int v : seen) CHECK(v == 1);
                     ++cases;
                 }
-    // the contiguous layout's slot numbering on 256-row tiles (ContiguousSlots): every (row position, column) once within the
-    // slots the host launches, whatever number of two-group rows the device finds; those rows' tiles come first in every
-    // XCD's slots and no XCD gets two more of them than another
-    for (int tm : {1, 2, 7, 8, 32, 33, 73, 128})
-        for (int tn : {1, 2, 16, 28, 33})
-            for (int groups : {1, 4, 16})
-                for (int two : {0, 1, 2, 7, 8, 31, 64, 127}) {
-                    if (two > tm) continue;
-                    const int bm = 256, bn = 256, m = (tm - 1) * bm + 129, n = (tn - 1) * bn + 1;
-                    const yan::ContiguousSlots slots(m, n, bm, bn, groups, two);
-                    const long long num_slots = yan::ContiguousSlots::num_slots(m, n, bm, bn);
-                    CHECK(num_slots % yan::kNumXCD == 0 && num_slots <= (long long)tm * tn + 2 * yan::kNumXCD);
-                    std::vector<int> seen(size_t(tm) * tn, 0);
-                    int first_of_xcd[yan::kNumXCD] = {0};
-                    bool other_seen[yan::kNumXCD] = {false};
-                    for (int s = 0; s < num_slots; ++s) {
-                        const yan::TileCoord t = slots.tile_of(s);
-                        if (!t.valid) continue;
-                        CHECK(t.m_idx >= 0 && t.m_idx < tm && t.n_idx >= 0 && t.n_idx < tn);
-                        ++seen[size_t(t.m_idx) * tn + t.n_idx];
-                        if (two == 0) continue;
-                        const int x = s % yan::kNumXCD;
-                        if (t.m_idx < two) { CHECK(!other_seen[x]); ++first_of_xcd[x]; }
-                        else other_seen[x] = true;
-                    }
-                    for (int v : seen) CHECK(v == 1);
-                    for (int x = 0; x < yan::kNumXCD; ++x) CHECK(first_of_xcd[x] - first_of_xcd[yan::kNumXCD - 1] <= 1 && first_of_xcd[x] >= first_of_xcd[yan::kNumXCD - 1]);
-                    ++cases;
+    // the contiguous layout on tiles that follow the groups: layouts of up to 200 blocks in runs of 1 to 70, padding among them,
+    // cut 64 blocks at a time as a wave does it
+    unsigned rng = 1;
+    auto random = [&](int below) { rng = rng * 1664525u + 1013904223u; return int((rng >> 8) % unsigned(below)); };
+    for (int trial = 0; trial < 400; ++trial) {
+        const int bm = 256, bn = trial % 2 ? 256 : 128, tn = 1 + random(20), n = (tn - 1) * bn + 4 + random(bn - 4);
+        std::vector<int> group_of;
+        const int blocks = 1 + random(200), longest = trial % 3 == 0 ? 70 : (trial % 3 == 1 ? 4 : 1);
+        for (int g = 0; int(group_of.size()) < blocks;) {
+            const int run = 1 + random(longest), group = random(5) == 0 ? -1 - random(2) : g++;
+            for (int r = 0; r < run && int(group_of.size()) < blocks; ++r) group_of.push_back(group);
+        }
+        const int m = blocks * 128 - (trial % 5 == 0 ? random(127) : 0);
+        std::vector<int> layout(size_t(blocks) * 128);
+        for (int b = 0; b < blocks; ++b) for (int r = 0; r < 128; ++r) layout[b * 128 + r] = group_of[b];
+        std::vector<int> covered(blocks, 0);
+        int tall_rows = 0, flat_rows = 0, odd = 0;
+        for (int chunk = 0; chunk * 64 < blocks; ++chunk) {
+            unsigned long long starts = 0;
+            for (int lane = 0; lane < 64; ++lane)
+                if (yan::ContiguousBlock(layout.data(), blocks, chunk * 64 + lane).starts_run) starts |= 1ull << lane;
+            for (int lane = 0; lane < 64; ++lane) {
+                const int b = chunk * 64 + lane, into = yan::ContiguousBlock::into_run(starts, lane, odd);
+                const yan::ContiguousBlock block(layout.data(), blocks, b);
+                CHECK(!(block.starts_tall(into) && block.starts_flat(into)));
+                if (block.starts_tall(into)) {
+                    CHECK(b + 1 < blocks && group_of[b] >= 0 && group_of[b + 1] == group_of[b]);
+                    ++covered[b], ++covered[b + 1], ++tall_rows;
                 }
+                if (block.starts_flat(into)) {
+                    CHECK(b < blocks && group_of[b] >= 0);
+                    ++covered[b], ++flat_rows;
+                }
+            }
+            odd = (yan::ContiguousBlock::into_run(starts, 63, odd) + 1) & 1;
+        }
+        for (int b = 0; b < blocks; ++b) CHECK(covered[b] == (group_of[b] >= 0 ? 1 : 0));
+        const long long launched = (long long)yan::XcdTileScheduler<>(m, n, 128, bn).grid_size() + yan::kNumXCD;
+        yan::XcdTileScheduler<> tall(tall_rows * 256, n, 256, bn), flat(flat_rows * 128, n, 128, bn);
+        tall.fit_bands_to_groups(tall_rows / 3);
+        flat.fit_bands_to_groups(1);
+        CHECK((long long)tall.grid_size() + flat.grid_size() <= launched);
+        for (const auto* tiles : {&tall, &flat}) {
+            const int rows = tiles == &tall ? tall_rows : flat_rows;
+            std::vector<int> seen(size_t(rows) * tn, 0);
+            for (int slot = 0; slot < tiles->grid_size(); ++slot) {
+                const yan::TileCoord t = tiles->dealt_band_tile_of(slot);
+                if (!t.valid) continue;
+                CHECK(t.m_idx >= 0 && t.m_idx < rows && t.n_idx >= 0 && t.n_idx < tn);
+                ++seen[size_t(t.m_idx) * tn + t.n_idx];
+            }
+            for (int v : seen) CHECK(v == 1);
+        }
+        ++cases;
+    }
     // what the traffic model picks for shapes that were measured (bf16, 256 x 256 tiles)
     {
         const int m = 0, n = 0, bm = 256, bn = 256;

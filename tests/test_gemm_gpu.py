@@ -763,8 +763,7 @@ def test_num_sms_caps_the_workgroups_without_changing_a_bit(m, n, k):
 
 def test_grouped_layouts_under_a_compute_unit_cap_give_the_same_bits():
     """Both grouped layouts with `set_num_sms(64)`: 64 workgroups walk the slots, several tiles each (for the contiguous
-    layout on 256-row tiles the slots of `ContiguousSlots`, two-group rows first), and write the bits of the uncapped
-    launch."""
+    layout on tiles that follow the groups the tall ones, then the flat ones), and write the bits of the uncapped launch."""
     from yan_amd.jit_kernels.m_grouped_gemm import grouped_kernel_plan
     cap, full = testing.NUM_SMS_CAP, yan.get_num_sms()
     rows, n, k, pad_blocks = testing.GROUPED_TWO_GROUP_ROWS_FIRST_CASE
@@ -1085,8 +1084,8 @@ def test_grouped_contiguous_parity(rows, n, k, pad_blocks):
 
 @pytest.mark.parametrize('rows,n,k,pad_blocks', testing.GROUPED_ROWS_ON_DEVICE_CASES)
 def test_grouped_contiguous_kernel_that_picks_its_tile_height_on_the_device(rows, n, k, pad_blocks):
-    """fp8_gemm_contiguous_rows_kernel on problems small enough for the oracle in full: with every group boundary on a
-    multiple of 256 rows it runs 256 x 256 tiles, otherwise 128 x 256 ones; either way the oracle's result, the bits of the
+    """fp8_gemm_contiguous_rows_kernel on problems small enough for the oracle in full: groups of an even number of blocks
+    run 256 x 256 tiles throughout, the others end on one of 128 x 256; either way the oracle's result, the bits of the
     entry (which gives problems this small to other tiles: all tiles form the same sums), padding blocks untouched, and
     the same again under a compute-unit cap, where workgroups walk several tiles."""
     _announce('grouped rows on device', rows, n, k)
@@ -1095,7 +1094,7 @@ def test_grouped_contiguous_kernel_that_picks_its_tile_height_on_the_device(rows
     blocks = idx.view(-1, 128)[:, 0]
     halves = blocks[:len(blocks) // 2 * 2].view(-1, 2)
     two_group_rows = int(((halves[:, 0] != halves[:, 1]) & (halves >= 0).all(1)).sum())
-    assert (two_group_rows == 0) == (rows == (512,) * 6)              # the first case is the one that runs 256-row tiles
+    assert (two_group_rows == 0) == (rows == (512,) * 6)              # the first case is the one whose boundaries all lie on multiples of 256 rows
     name, keys, arg_defs, code_template = testing.grouped_rows_on_device_plan(groups, n, k)
     from yan_amd.jit_kernels import m_grouped_gemm
     kernel = jit.build(name, arg_defs, jit.generate(m_grouped_gemm.includes, arg_defs, jit.cpp_format(code_template, keys)))

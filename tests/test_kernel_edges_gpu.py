@@ -94,6 +94,28 @@ def test_fp8_ring_tiles_where_the_k_loop_is_unrolled_and_where_not(tile, k):
     assert _fp8_close(results[0].float(), ref)
 
 
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.half])
+@pytest.mark.parametrize('tile', testing.DENSE_RAGGED_CAP_CASE[0])
+def test_dense_ring_tiles_walked_with_ragged_rows_and_few_k_tiles(tile, dtype):
+    _, (m, n), depths, cap = testing.DENSE_RAGGED_CAP_CASE
+    for k in depths:
+        _announce('dense ragged under a cap', tile, dtype, k)
+        a, b, c = testing.make_bf16_case(m, n, k, seed=16, dtype=dtype, device='cuda')
+        results = []
+        for num_sms in (0, cap):
+            name, keys, arg_defs, includes, code_template = testing.dense_tile_plan(tile, dtype, num_sms)
+            kernel = jit.build(name, arg_defs, jit.generate(includes, arg_defs, jit.cpp_format(code_template, keys)))
+            c.fill_(float('nan'))
+            assert kernel(m, n, k, a, b, c, torch.cuda.current_stream()) == 0
+            torch.cuda.synchronize()
+            results.append(c.clone())
+        ref = a.double().cpu() @ b.double().cpu().t()
+        # one rounding of the result to its type, and of each of at most k + 8 sums in a row relative to the sum of magnitudes
+        bound = ref.abs() * 2.0 ** (-8 if dtype == torch.bfloat16 else -11) + (k + 8) * 2.0 ** -24 * (a.double().abs().cpu() @ b.double().abs().cpu().t())
+        assert torch.equal(results[0], results[1])
+        assert bool(((results[0].double().cpu() - ref).abs() <= bound).all())
+
+
 @pytest.mark.parametrize('m,n,k', testing.FLOAT_SPLIT_K_SHAPES)
 def test_float_split_k_matches_the_oracle_and_repeats(m, n, k):
     """gemm_cute_split_k through the entry: k that is no multiple of a k-tile or of the parts, last parts shorter than the

@@ -173,13 +173,13 @@ fp8_compute_k_tile(f32x4 (&acc)[TN][TM], const uint8_t* pa, const uint8_t* pb, c
 // of 16 * (2 WTN + 16) bytes that nobody else touches) the slab instead turns round through it, 16 rows at a time, and
 // is stored 16 bytes per lane in runs of 2 * WTN consecutive bytes per row; rows are 2 * WTN + 16 bytes apart in LDS,
 // which spreads the 8-byte writes of 16 rows over the banks. STAGED = false: the direct stores, `region` unused.
-// Rows outside [row_lo, row_hi) and columns from n on are not stored. `rsrc_out` addresses the output tile that starts
+// Rows from row_end on and columns from n on are not stored. `rsrc_out` addresses the output tile that starts
 // at (m0, n0); `lane` should be an opaque copy of the lane number made after the main loop, which has no registers to
 // spare for addresses computed ahead of time.
 template <typename Cfg, bool STAGED, int TN, int TM>
 __device__ __forceinline__ void
 fp8_store_slab(const f32x4 (&acc)[TN][TM], uint8_t* region, __amdgpu_buffer_rsrc_t rsrc_out, int m_slab, int n_slab, int m0, int n0,
-               int row_lo, int row_hi, int n, bool stream_out, int lane) {
+               int row_end, int n, bool stream_out, int lane) {
     const int col = lane % 16, g = lane / 16;
     if constexpr (STAGED) {
         {
@@ -198,7 +198,7 @@ fp8_store_slab(const f32x4 (&acc)[TN][TM], uint8_t* region, __amdgpu_buffer_rsrc
                     const int row = ROWS_PER_STORE * q + r_in, mm = m_slab + 16 * j + row;
                     const i32x4 v = *reinterpret_cast<const i32x4*>(region + row * PITCH + c * 16);
                     // a slab width that does not divide 64 lanes leaves the last lanes, and rows past 16, without work
-                    const bool live = mm >= row_lo && mm < row_hi && nn < n && r_in < ROWS_PER_STORE && row < 16;
+                    const bool live = mm < row_end && nn < n && r_in < ROWS_PER_STORE && row < 16;
                     if (live) buffer_store_16(v, rsrc_out, uint32_t((mm - m0) * n + nn - n0) * 2u, stream_out);
                 }
                 __builtin_amdgcn_sched_barrier(0);      // one 16-row pass at a time: the registers are full of sums
@@ -208,7 +208,7 @@ fp8_store_slab(const f32x4 (&acc)[TN][TM], uint8_t* region, __amdgpu_buffer_rsrc
 #pragma unroll
         for (int j = 0; j < TM; ++j) {
             const int mm = m_slab + j * 16 + col;
-            if (mm < row_lo || mm >= row_hi) continue;
+            if (mm >= row_end) continue;
 #pragma unroll
             for (int i = 0; i < TN; ++i) {
                 const int nn = n_slab + i * 16 + 4 * g;
@@ -232,24 +232,17 @@ fp8_meet_partials(f32x4 (&acc)[TN][TM], float* __restrict__ partials, unsigned* 
     return meet_partials<SPLIT_K, NW, TN * TM>([&](int v) -> f32x4& { return acc[v / TM][v % TM]; }, partials, counters, tile_slot, split, wave, lane);
 }
 
-// Contiguous groups on tiles that follow the groups (fp8_gemm_contiguous_rows_kernel). A group is a run of 128-row blocks with
-// one index; walked from its first block it is cut into tall tiles of two blocks and, where it has an odd number, a flat tile
-// of one. Bit `lane` of `tall` / `flat`: such a tile starts at block 64 * chunk + lane. Padding (negative indices) has neither.
-// Chunks are taken in ascending order: `odd` carries from one to the next whether the run across the border is an odd number
-// of blocks long so far (0 in front of the first).
+// Contiguous groups on tiles that follow the groups (fp8_gemm_contiguous_rows_kernel): bit `lane` of `tall` / `flat` is set where
+// such a tile starts at block 64 * chunk + lane (ContiguousBlock in scheduler.hpp). Chunks are taken in ascending order: `odd`
+// carries from one to the next whether the run across the border is an odd number of blocks long so far (0 in front of the
+// first).
 struct ContiguousTileStarts { unsigned long long tall, flat; };
 __device__ __forceinline__ ContiguousTileStarts
 contiguous_tile_starts(const int* __restrict__ grouped_layout, int blocks, int chunk, int lane, int& odd) {
-    const int b = chunk * kWaveSize + lane;
-    const bool real = b < blocks;
-    const int g = real ? grouped_layout[b * 128] : -1;
-    const int before = real && b > 0 ? grouped_layout[(b - 1) * 128] : -1, behind = b + 1 < blocks ? grouped_layout[(b + 1) * 128] : -1;
-    // how far into its run this block is: counted from the last start of a run at or in front of it
-    const unsigned long long starts = __ballot(b == 0 || g != before), at_or_before = starts & (~0ull >> (63 - lane));
-    const int into = at_or_before ? lane - (63 - __clzll((long long)at_or_before)) : lane + odd;
-    const bool opens = real && g >= 0 && (into & 1) == 0;
+    const ContiguousBlock block(grouped_layout, blocks, chunk * kWaveSize + lane);
+    const int into = ContiguousBlock::into_run(__ballot(block.starts_run), lane, odd);
     odd = (__builtin_amdgcn_readlane(into, kWaveSize - 1) + 1) & 1;
-    return {__ballot(opens && behind == g), __ballot(opens && behind != g)};
+    return {__ballot(block.starts_tall(into)), __ballot(block.starts_flat(into))};
 }
 
 // The block at which the tall (flat) tile row number `rank` starts. Wave-uniform; `rank` is below the number there are.
@@ -662,12 +655,12 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
         if constexpr (SPLIT_K > 1)
             if (!fp8_meet_partials<SPLIT_K, NW, TN, TM>(acc, partials, counters, tile_slot, split, wave, lane_late)) return;
         uint8_t* region = (wave < NW / 2 ? epi_a : epi_b) + (wave % (NW / 2)) * REGION;
-        fp8_store_slab<Cfg, kStagedEpilogue>(acc, region, rsrc_out, m_slab, n_slab, m0, n0, m0, m, N, stream_out, lane_late);
+        fp8_store_slab<Cfg, kStagedEpilogue>(acc, region, rsrc_out, m_slab, n_slab, m0, n0, m, N, stream_out, lane_late);
     } else {
         if (LW > NW && wave >= NW) return;              // waves that only copy
         if constexpr (SPLIT_K > 1)
             if (!fp8_meet_partials<SPLIT_K, NW, TN, TM>(acc, partials, counters, tile_slot, split, wave, lane)) return;
-        fp8_store_slab<Cfg, false>(acc, nullptr, rsrc_out, m_slab, n_slab, m0, n0, m0, m, N, stream_out, lane);
+        fp8_store_slab<Cfg, false>(acc, nullptr, rsrc_out, m_slab, n_slab, m0, n0, m, N, stream_out, lane);
     }
 }
 
@@ -832,10 +825,10 @@ fp8_gemm_walk(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
             uint8_t* region = (wave < NW / 2 ? lds_a1 : lds_b1) + (wave % (NW / 2)) * REGION;
             if ((N % 8) == 0)
                 fp8_store_slab<Cfg, true>(acc, region, rsrc_out, cur.m0 + wm * Cfg::WTM, cur.n0 + wn * Cfg::WTN, cur.m0, cur.n0,
-                                          0, m, N, stream_out, lane_late);
+                                          m, N, stream_out, lane_late);
             else
                 fp8_store_slab<Cfg, false>(acc, region, rsrc_out, cur.m0 + wm * Cfg::WTM, cur.n0 + wn * Cfg::WTN, cur.m0, cur.n0,
-                                           0, m, N, stream_out, lane_late);
+                                           m, N, stream_out, lane_late);
         }
         if (!nxt.valid) break;
         cur = nxt;

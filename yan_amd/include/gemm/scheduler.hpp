@@ -189,46 +189,31 @@ struct MaskedSlots {
     }
 };
 
-// A slot numbering of the contiguous layout on a fixed grid of 256-row tiles. (The kernels of this directory place their tall
-// tiles along the groups instead, fp8_gemm_contiguous_rows_kernel, and have no tile of two groups.) A tile row whose two 128-row halves belong to two groups makes
-// two passes over K and takes about half as long again as the others; started last, one of them ends alone after everyone
-// else. `two_group_rows` of the `tiles_m` rows are of that kind (a kernel counts them in the caller's layout; the host
-// does not know them and launches `num_slots()` workgroups whatever their number). Their tiles come first in every XCD's
-// share of the slots and are dealt to the XCDs one by one, so that every XCD gets as many (an XCD runs its own slots, and
-// a patch of 32 slow tiles would fall to one of them); the other rows follow in band order dealt out in patches of 32.
-// `tile_of` names rows by position: positions below `two_group_rows` are the two-group rows, the others follow, either
-// kind in ascending order. With no such row the order is the plain one (a contiguous range of the band order per XCD).
-struct ContiguousSlots {
-    XcdTileScheduler<> all, rest;
-    int two_group_rows, first_tiles;
+// The contiguous layout on tiles that follow the groups (fp8_gemm_contiguous_rows_kernel). A group is a run of 128-row blocks with
+// one index; walked from its first block it is cut into tall tiles of two blocks and, where it has an odd number, a flat tile
+// of one. Padding (negative indices) has neither. A wave looks at 64 blocks at a time, one per lane: this is what a lane
+// knows of its block, and what follows from the ballot of `starts_run` and from the blocks in front of the 64.
+struct ContiguousBlock {
+    int group, behind;          // of this block and the next one; -1 past the end
+    bool starts_run;
 
-    __host__ __device__ ContiguousSlots(int m, int n, int block_m, int block_n, int num_groups, int two_group_rows_)
-        : all(m, n, block_m, block_n), rest(0, 0, block_m, block_n), two_group_rows(two_group_rows_) {
-        all.fit_bands_to_groups(all.tiles_m / (num_groups > 0 ? num_groups : 1));
-        rest = XcdTileScheduler<>((all.tiles_m - two_group_rows) * block_m, n, block_m, block_n);
-        rest.band_height = all.band_height;
-        first_tiles = two_group_rows * all.tiles_n;
+    __host__ __device__ ContiguousBlock(const int* grouped_layout, int blocks, int b) {
+        const bool real = b < blocks;
+        group = real ? grouped_layout[b * 128] : -1;
+        const int before = real && b > 0 ? grouped_layout[(b - 1) * 128] : -1;
+        behind = b + 1 < blocks ? grouped_layout[(b + 1) * 128] : -1;
+        starts_run = b == 0 || group != before;
     }
 
-    // one slot per XCD more than the tiles need: the two kinds of rows are rounded up to whole slots per XCD separately
-    __host__ __device__ static long long num_slots(int m, int n, int block_m, int block_n) {
-        return (long long)XcdTileScheduler<>(m, n, block_m, block_n).grid_size() + kNumXCD;
+    // How far into its run the block of lane `lane` is, counted from the last start of a run at or in front of it; `odd`: whether
+    // the run that reaches the 64 blocks from in front is an odd number of blocks long there.
+    __host__ __device__ static int into_run(unsigned long long starts, int lane, int odd) {
+        const unsigned long long at_or_before = starts & (~0ull >> (63 - lane));
+        return at_or_before ? lane - (63 - __builtin_clzll(at_or_before)) : lane + odd;
     }
 
-    __host__ __device__ TileCoord tile_of(int slot) const {
-        if (two_group_rows == 0) return slot < all.grid_size() ? all.tile_of(slot) : TileCoord{0, 0, false};
-        const int x = slot % kNumXCD, q = slot / kNumXCD;
-        const int mine = first_tiles > x ? (first_tiles - x + kNumXCD - 1) / kNumXCD : 0;      // two-group tiles of this XCD
-        if (q < mine) {
-            const int t = q * kNumXCD + x;
-            return {t / all.tiles_n, t % all.tiles_n, true};
-        }
-        const int s = (q - mine) * kNumXCD + x;
-        if (s >= rest.grid_size()) return {0, 0, false};
-        TileCoord t = rest.dealt_band_tile_of(s);
-        t.m_idx += two_group_rows;
-        return t;
-    }
+    __host__ __device__ bool starts_tall(int into) const { return group >= 0 && (into & 1) == 0 && behind == group; }
+    __host__ __device__ bool starts_flat(int into) const { return group >= 0 && (into & 1) == 0 && behind != group; }
 };
 
 // Workgroups to launch for `slots` units of work (tiles, or groups x tiles) under the caller's compute-unit cap, the

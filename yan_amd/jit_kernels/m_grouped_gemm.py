@@ -66,7 +66,7 @@ def grouped_kernel_plan(gemm_type: str, num_groups: int, m: int, n: int, k: int,
             # both tile heights in one kernel, named by the taller one
             keys = FrozenKeys({'N': n, 'K': k, 'BLOCK_M': 256, 'BLOCK_N': 256, 'NUM_GROUPS': num_groups, 'NUM_STAGES': 2,
                                'NUM_TMA_MULTICAST': 1, 'GEMM_TYPE': gemm_type, 'ROWS': 'picked on the device'})
-            return name + '_rows_on_device', keys, arg_defs, 2 * (256 + 256) * 128
+            return name + '_rows_on_device', keys, arg_defs, (2 * 256 + 3 * 256) * 128      # two stages of rows, three of weights
     else:
         block_m, block_n = get_best_grouped_fp8_config(m, n, k, num_cus, num_groups)
         name = 'm_grouped_gemm_fp8_fp8_bf16_nt'
