@@ -136,8 +136,8 @@ YAN_API int yan_gemm_split_k_reset(void* workspace, void* stream);
  * contiguous: lhs [m,k] holds the rows of all groups one after the other, every group padded to a multiple of 128 rows
  *   (get_m_alignment_for_contiguous_layout, yan/jit_kernels/utils.py:46-55), so m % 128 == 0; m_indices[i] (device,
  *   int32 [m]) is the group of row i, constant over each aligned block of 128 rows; a negative value marks a block of
- *   padding rows, whose rows of `out` are not written. Groups of a few hundred rows that are padded to multiples of 256 rows
- *   run up to 17 % faster than others (no 256-row tile then holds two groups; see yan_gemm_select_tile op 4). */
+ *   padding rows, whose rows of `out` are not written. Tiles of 256 rows follow the groups wherever these start, so padding a
+ *   group to more than 128 rows buys nothing (see yan_gemm_select_tile op 4). */
 YAN_API int yan_m_grouped_gemm_fp8_fp8_bf16_nt_contiguous(const void* lhs, const float* lhs_scales, long long lhs_scales_stride_m,
                                                   long long lhs_scales_stride_k, const void* rhs, const float* rhs_scales,
                                                   void* out, const int* m_indices, int num_groups, int m, int n, int k,

@@ -37,7 +37,8 @@ namespace yan {
 template <int BLOCK_M, int BLOCK_N>
 struct DenseTileConfig {
     static constexpr int NUM_WAVES = 4;
-    // A slab of at most 128 x 128 outputs: 256 accumulator registers per lane, out of the 512 a lone wave may hold.
+    // A slab of at most 128 x 128 outputs, 256 accumulator registers per lane: what a wave alone on its SIMD has room for. The ring
+    // tiles share it with a wave that copies, 256 registers each, and stay at 128 x 64 and below.
     static constexpr int WAVES_N   = pick_waves_n(BLOCK_M, BLOCK_N, NUM_WAVES, 32, 128 * 128);
     static_assert(WAVES_N > 0, "no wave layout fits this tile");
     static constexpr int WAVES_M   = NUM_WAVES / WAVES_N;
@@ -80,7 +81,8 @@ dense_meet_partials(Acc (&acc)[TN][TM], float* __restrict__ partials, unsigned* 
 // alone), and those by the bytes a compute unit can have on their way, whoever asks for them, so what this gains is the time the
 // computing waves stood in the queue: 37 shapes and tiles -7 to +2 %, 256 x 128 -4 to -11 % (2048 x 2112 x 7168 105.6 -> 94.3 us),
 // 128 x 192 81.4 -> 79.0, 64 x 192 at 1024 x 2112 x 7168 66.3 -> 62.2. With the four extra waves doing all the copies: between the two.
-// 128 x 128 tiles in four parts are 4 to 8 % slower with the extra waves (14 k-tiles per part at K = 7168) and stay without.
+// 128 x 128 tiles in four parts or more stay without: 24 shapes of 68 to 583 rows with K = 5120 to 16384 (20 to 64 k-tiles a part)
+// are 0 to 8 % faster that way (95 x 7104 x 5312 29.4 -> 27.1 us), one 2.6 % slower.
 __host__ __device__ constexpr int dense_launch_waves(int block_m, int block_n, int split_k = 1) {
     return block_m * block_n >= 128 * 128 && split_k >= 4 ? 4 : 8;
 }

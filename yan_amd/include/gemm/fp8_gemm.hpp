@@ -220,7 +220,7 @@ fp8_store_slab(const f32x4 (&acc)[TN][TM], uint8_t* region, __amdgpu_buffer_rsrc
 
 // Normal:            lhs [m, K], rhs [N, K], out [m, N]; grouped_layout unused.
 // GroupedContiguous: lhs [m, K] is the concatenation of the groups' rows, every group padded to a multiple of 128
-//                    rows (BLOCK_M divides 128); grouped_layout[i] is the group of row i, negative for padding rows,
+//                    rows (BLOCK_M divides 128, or the tiles are placed along the groups); grouped_layout[i] is the group of row i, negative for padding rows,
 //                    whose tiles are skipped; rhs [G, N, K], rhs_scales [G, ceil(N/128), K/128].
 // GroupedMasked:     lhs [G, m, K], out [G, m, N], rhs as above; only the first grouped_layout[g] rows of group g
 //                    are computed; lhs_scales of group g start at g * sa_stride_g floats. Slots are numbered by

@@ -224,17 +224,18 @@ float_gemm_body(const float* __restrict__ A, const float* __restrict__ B, float*
     const int n_lane = n0 + wn * Cfg::WTN + VN * i;
     if (n_lane >= n) return;                                   // n % 4 == 0 and VN | 4: a lane's VN columns exist together
     auto row_of = [&](int q, int r, int t) { return m0 + wm * Cfg::WTM + VM * (8 * (first_quad + q) + 4 * h + r) + t; };
-    // beta chooses between two copies of this: asked in it, the compiler keeps both ways open from row to row, with the address
-    // of every row worked out twice (beta = 0: 2176 x 768 x 454 20.0 us before there was a load ahead of the stores, 20.7 with
-    // both in one copy, 20.0 with two; 1408 x 1152 x 487 21.4, 21.9 and 21.1).
-    auto store = [&](auto onto_c) {
-        constexpr bool ONTO_C = decltype(onto_c)::value;
+    // Where a wave stores all of its sums, beta chooses between two copies of this: asked in it, the compiler keeps both ways open
+    // from row to row, with the address of every row worked out twice (beta = 0: 2176 x 768 x 454 20.0 us before there was a
+    // load ahead of the stores, 20.7 with both in one copy, 20.0 with two; 1408 x 1152 x 487 21.4, 21.9 and 21.1). A quarter of
+    // them (K_SPLIT) is quicker through one.
+    auto store = [&](auto onto_c) {         // 0: C = ..., 1: C = ... + beta C, 2: as beta says
+        const bool reads_c = onto_c == 2 ? beta != 0.f : onto_c == 1;
 #pragma unroll
         for (int q = 0; q < QUADS; ++q) {
             // what C holds, 4 * VM rows at a time (rows past m read the last one again): a load behind every row's branch waits for
             // memory once per row (beta = 1: 1024^3 28.6 -> 19.8 us, 4096 x 7168 x 512 257 -> 231, beta = 0 19.4 and 221)
-            [[maybe_unused]] VecN held[4][VM];
-            if constexpr (ONTO_C) {
+            VecN held[4][VM];
+            if (reads_c) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -252,13 +253,14 @@ float_gemm_body(const float* __restrict__ A, const float* __restrict__ B, float*
 #pragma unroll
                         for (int u = 0; u < VN; ++u) v[u] = alpha * sum_of(t, u, q)[r];
                     }
-                    if constexpr (ONTO_C) v += beta * held[r][t];
+                    if (reads_c) v += beta * held[r][t];
                     *reinterpret_cast<VecN*>(C + size_t(mm) * ldC + n_lane) = v;
                 }
         }
     };
-    if (beta != 0.f) store(std::true_type{});
-    else store(std::false_type{});
+    if constexpr (Cfg::K_SPLIT == 4) store(std::integral_constant<int, 2>{});
+    else if (beta != 0.f) store(std::integral_constant<int, 1>{});
+    else store(std::integral_constant<int, 0>{});
 }
 
 // The kernel keeps the reference kernel's name (simple_gemm.cuh:22) so that profiler filters written for it
