@@ -18,8 +18,10 @@ from .utils import ceil_div, env_switch
 # (8192 x 32 BLOCK_N x 8192), relative to 256 x 256 (1.02-1.04, 1.035-1.06, 1.07-1.10 over three boxes). The ring tiles measure
 # 1.30-1.32 (256 x 128, 128 x 256) and 1.49 (128 x 128) there, but no problem of four rounds ever takes them: where they
 # compete, in launches of one or two rounds, a tile pays its first loads and its epilogue in full, and 1.40 / 1.42 is what
-# makes the table's pick the fastest tile or within 1.2 % of it on all 67 shapes swept with every tile forced in turn (with
-# 1.30, 128 x 256 took eight one-round shapes from 256 x 160, which is 4 to 17 % faster there).
+# made the table's pick the fastest tile or within 1.2 % of it on all 67 shapes swept with every tile forced in turn (with
+# 1.30, 128 x 256 took eight one-round shapes from 256 x 160, which is 4 to 17 % faster there). That was before the ring tiles
+# had waves that only copy: over 70 shapes since then the pick is within 2 % of the fastest on 57, and 64 x 192 is 5 to 17 %
+# behind 128 x 128 on seven (670 x 4416 x 3264 29.5 against 25.2 us).
 # 128 x 192 and 64 x 192 (ring kernel, wave slabs 96 columns wide) are for problems that leave most compute units idle with
 # 256-wide tiles and need two rounds with 128-wide ones (2048 x 2112 x 7168: 144 tiles of 128 x 256 run 85 us, 176 of 128 x 192 68 us).
 _DENSE_TILES = {(256, 256): 1.00, (256, 224): 1.03, (256, 192): 1.05, (256, 160): 1.085, (256, 128): 1.42, (128, 256): 1.40,
@@ -96,9 +98,9 @@ def get_best_grouped_fp8_config(m: int, n: int, k: int, num_cus: int, groups: in
     """Tile of a grouped FP8 GEMM, among the tiles 64, 128 or 256 columns wide. Contiguous layout: `m` is the total row count and
     `m_alignment` the padding of every group, which the tile's rows must divide. 256 x 128, whose tiles follow the `groups_in_m`
     groups as the 256 x 256 ones of `get_contiguous_rows_on_device` do, is offered when they average 1024 rows or more and the
-    tiles are more than one round: 10 groups, 11136 x 1408 x 1280 61 us on 128 x 128 tiles, 43 on these; 10 groups, 15104 x 2112 x
-    5760 255 and 227; 23 such shapes 0.71 to 1.04 times the time on 128 x 128. In one round it loses (6 groups, 6784 x 1152 x
-    6912: 77 us on 128 x 128, 88 on these). Masked layout: `m` is the expected row count of one group and `groups` multiplies
+    tiles are more than one round: 10 groups, 15104 x 2112 x 5760 244 us on 128 x 128 tiles, 220 on these; 3 groups, 8832 x 3648 x
+    5632 231 and 203; 23 such shapes 0.88 to 1.03 times the time on 128 x 128, one 1.11. In one round it loses (4 groups,
+    4352 x 1856 x 6912: 73 us on 128 x 128, 86 on these). Masked layout: `m` is the expected row count of one group and `groups` multiplies
     the tile count."""
     def allowed(bm, bn):
         if m_alignment == 0 or m_alignment % bm == 0:
