@@ -519,10 +519,10 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
         const bool data = sl * LW + LW - 1 < GROUPS_AB || (sl * LW < GROUPS_AB && o < GROUPS_AB);
         const bool in_a = sl * LW + LW - 1 < GA || (sl * LW < GA && o < GA);
         if (data) {
-            if (in_a) __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_a : rsrc_none, YAN_LDS_PTR(stage + o * 8 * kRowBytes), kChunk, slot_voff[sl], kb * kRowBytes, 0, 0);
-            else __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_b : rsrc_none, YAN_LDS_PTR(stage + o * 8 * kRowBytes), kChunk, slot_voff[sl], kb * kRowBytes, 0, 0);
+            if (in_a) __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_a : rsrc_none, YAN_LDS_CAST(stage + o * 8 * kRowBytes), kChunk, slot_voff[sl], kb * kRowBytes, 0, 0);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_b : rsrc_none, YAN_LDS_CAST(stage + o * 8 * kRowBytes), kChunk, slot_voff[sl], kb * kRowBytes, 0, 0);
         } else {
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_sa : rsrc_none, YAN_LDS_PTR(stage + TILE_BYTES), 4, scale_voff, kb * sa_stride_k * 4, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_sa : rsrc_none, YAN_LDS_CAST(stage + TILE_BYTES), 4, scale_voff, kb * sa_stride_k * 4, 0, 0);
         }
     };
 #pragma unroll
