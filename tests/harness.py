@@ -300,9 +300,11 @@ GROUPED_FOLLOW_GROUPS_CASES = [((63 * 128, 3 * 128, 1, 2 * 128), 264, 128, 0), (
 # tiles support, with and without a ring and a 128-row tile beside them
 GROUPED_256_ROW_KEYS = [(256, 2), (224, 2), (192, 2), (160, 2), (128, 3), (128, 2), (96, 2), (32, 2)]
 GROUPED_256_ROW_KEYS_CASE = ((-128, 100, -256, 5 * 128, 385, -128, 3 * 128), 520, 384, 0)
-# Ring tiles of the FP8 kernel with K on either side of where their k-loop stops being unrolled, and as short as it gets
+# Tiles of the FP8 kernel with K on either side of where the form of their k-loop changes, and as short as it gets
 FP8_SHORT_K_TILES = [((64, 64), (128, 2048, 2176)), ((64, 128), (256, 1536, 1664)), ((128, 128), (128, 1024, 1152)),
-                     ((128, 256), (128, 384, 512, 768)), ((256, 128), (256, 384, 512, 768))]
+                     ((128, 256), (128, 384, 512, 768)), ((256, 128), (256, 384, 512, 768)),
+                     # two stages, odd numbers of k-tiles: one copy of the k-step up to 31 of them, three from there
+                     ((256, 256), (128, 384, 3968, 4224))]
 FP8_SHORT_K_SIZES = (390, 516)
 GROUPED_MASKED_TEST_CASES = [
     (3, 200, 320, 384, (200, 0, 77), 128), (4, 256, 4096, 1024, (1, 256, 130, 64), 64), (2, 64, 200, 128, (64, 3), 32),

@@ -671,8 +671,8 @@ def test_fp8_kernels_of_two_k_tiles_compile(tmp_path, m, n, k):
                            '-o', str(tmp_path / 'kernel.s')])
 
 
-@pytest.mark.parametrize('tile,k', [((128, 128), 1152), ((128, 256), 768), ((256, 128), 512)])
-def test_fp8_ring_tiles_do_not_spill_where_k_is_short(tmp_path, tile, k):
+@pytest.mark.parametrize('tile,k', [((128, 128), 1152), ((128, 256), 768), ((256, 128), 512), ((256, 256), 384), ((256, 256), 1664)])
+def test_fp8_tiles_do_not_spill_where_k_is_short(tmp_path, tile, k):
     import re
     import subprocess
     import harness as testing

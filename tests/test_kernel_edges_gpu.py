@@ -76,7 +76,7 @@ def test_contiguous_keys_that_name_a_tile_of_256_rows(block_n, stages):
 
 
 @pytest.mark.parametrize('tile,k', [(tile, k) for tile, depths in testing.FP8_SHORT_K_TILES for k in depths])
-def test_fp8_ring_tiles_where_the_k_loop_is_unrolled_and_where_not(tile, k):
+def test_fp8_tiles_on_either_side_of_a_change_of_their_k_loop(tile, k):
     m, n = testing.FP8_SHORT_K_SIZES
     _announce('fp8 short k', tile, k)
     from yan_amd.jit_kernels import gemm

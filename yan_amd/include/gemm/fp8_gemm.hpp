@@ -457,6 +457,22 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
         }
         epi_a = a_nxt;          // the stages of the last k-tile
         epi_b = b_two;
+    } else if constexpr (SHAPE_K != 0 && (SHAPE_K / 128) % 2 == 1 && SHAPE_K / 128 <= 31 && TN * TM >= 32) {
+        // One copy of the k-step with the stages changing places. An odd number of k-tiles has a third copy behind the loop's two,
+        // and 256 x 256 tiles, whose registers are full, spill 32 of them around it, at three k-tiles 239: 5658 x 8256 x 2688 133
+        // us that way, 128 this way, 3529 x 7616 x 896 38.7 and 35.2. Changing places costs in every step, and from some 35 k-tiles on
+        // more than the spills do (3186 x 4032 x 8320 112 and 116). Narrower tiles do not spill.
+        uint8_t *a_cur = lds_a0, *a_nxt = lds_a1, *b_cur = lds_b0, *b_nxt = lds_b1;
+#pragma unroll 1
+        for (int kb = 0; kb < NUM_K_BLOCKS; ++kb) {
+            k_step(kb, a_cur, b_cur, a_nxt, b_nxt);
+            uint8_t* t = a_cur;
+            a_cur = a_nxt; a_nxt = t;
+            t = b_cur;
+            b_cur = b_nxt; b_nxt = t;
+        }
+        epi_a = lds_a0;         // the stages of the last k-tile
+        epi_b = lds_b0;
     } else {
         for (int kb = 0; kb + 1 < NUM_K_BLOCKS; kb += 2) {
             k_step(kb, lds_a0, lds_b0, lds_a1, lds_b1);
