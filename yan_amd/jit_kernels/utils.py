@@ -21,13 +21,13 @@ def _device_cu_count() -> int:
 # What os.environ keeps on POSIX, bytes to bytes: a look there costs a tenth of os.environ.get, which goes through three Python
 # functions and two encodings (0.7 us, two or three times a call). A program may put another mapping in the place of
 # os.environ (tests do); then it is asked the ordinary way.
-_environ = os.environ
 _environ_bytes = getattr(os.environ, '_data', None)
+_environ = None if _environ_bytes is None else os.environ
 
 
 def env_switch(name: bytes, default: bool) -> bool:
     """Whether the environment variable `name` is on as of now: unset means `default`, empty and '0' mean off."""
-    if os.environ is _environ and _environ_bytes is not None:
+    if os.environ is _environ:
         value = _environ_bytes.get(name)
         return default if value is None else value not in (b'', b'0')
     value = os.environ.get(name.decode())
