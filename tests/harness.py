@@ -303,9 +303,13 @@ GROUPED_256_ROW_KEYS_CASE = ((-128, 100, -256, 5 * 128, 385, -128, 3 * 128), 520
 # Tiles of the FP8 kernel with K on either side of where the form of their k-loop changes, and as short as it gets
 FP8_SHORT_K_TILES = [((64, 64), (128, 2048, 2176)), ((64, 128), (256, 1536, 1664)), ((128, 128), (128, 1024, 1152)),
                      ((128, 256), (128, 384, 512, 768)), ((256, 128), (256, 384, 512, 768)),
-                     # two stages, odd numbers of k-tiles: one copy of the k-step up to 31 of them, three from there
+                     # two stages: no walk, a walk whose first k-tile is the last but two, long ones
                      ((256, 256), (128, 384, 3968, 4224))]
 FP8_SHORT_K_SIZES = (390, 516)
+# Tiles on two stages (three of the weights) that are walked, several to a workgroup: the seam between two tiles where every k-tile
+# fetches for the next one (two of them) and where one does not; tiles whose copies are handed out one and several to a row
+FP8_WALK_CASES = [((256, 256), (256, 384)), ((256, 224), (256, )), ((256, 160), (256, 384)), ((128, 256), (256, 384)), ((64, 64), (384, ))]
+FP8_WALK_SIZES = (1300, 772)
 GROUPED_MASKED_TEST_CASES = [
     (3, 200, 320, 384, (200, 0, 77), 128), (4, 256, 4096, 1024, (1, 256, 130, 64), 64), (2, 64, 200, 128, (64, 3), 32),
     (4, 1024, 4096, 7168, (1024, 900, 512, 1), 1024),
@@ -362,11 +366,12 @@ FP8_EXPLICIT_TILE_CASES = [(256, 224, (600, 1344, 640)), (256, 224, (300, 1000, 
                            (64, 160, (1000, 2100, 384)), (64, 160, (200, 1156, 1024))]
 
 
-def fp8_explicit_tile_plan(block_m: int, block_n: int, n: int, k: int):
-    """(name, keys, arg_defs, template) of the FP8 JIT kernel with this tile and token-contiguous scales."""
+def fp8_explicit_tile_plan(block_m: int, block_n: int, n: int, k: int, stages: int = 0):
+    """(name, keys, arg_defs, template) of the FP8 JIT kernel with this tile and token-contiguous scales; `stages` 0: as many as
+    the entry would take."""
     from yan_amd.jit_kernels import gemm
     from yan_amd.jit_kernels.heuristics import get_fp8_num_stages
-    keys = {'N': n, 'K': k, 'BLOCK_M': block_m, 'BLOCK_N': block_n, 'NUM_STAGES': get_fp8_num_stages(block_m, block_n),
+    keys = {'N': n, 'K': k, 'BLOCK_M': block_m, 'BLOCK_N': block_n, 'NUM_STAGES': stages or get_fp8_num_stages(block_m, block_n),
             'NUM_TMA_MULTICAST': 1}
     return 'gemm_fp8_fp8_bf16_nt', keys, gemm.arg_defs, gemm.template
 
@@ -476,6 +481,10 @@ def jit_kernels_in_use(num_cus: int = 256):
     for tile, depths in FP8_SHORT_K_TILES:
         for k in depths:
             name, keys, arg_defs, code_template = fp8_explicit_tile_plan(*tile, FP8_SHORT_K_SIZES[1], k)
+            add(name, arg_defs, gemm.includes, code_template, keys)
+    for tile, depths in FP8_WALK_CASES:
+        for k in depths:
+            name, keys, arg_defs, code_template = fp8_explicit_tile_plan(*tile, FP8_WALK_SIZES[1], k, 2)
             add(name, arg_defs, gemm.includes, code_template, keys)
     for m, n, k in list(FLOAT_SPLIT_K_SHAPES) + REFERENCE_FLOAT_TEST_SHAPES + FLOAT_TEST_SHAPES:
         plan = simple_gemm.float_split_k_plan(m, n, k, num_cus)

@@ -8,7 +8,7 @@
 //     the tiles from 256 x 128 up and for the tiles from 64 x 64 up whose sides are multiples of 64 (get_num_waves in
 //     mfma_utils.hpp), so one wave's scale arithmetic and LDS traffic hide under the other's MFMAs and eight waves issue
 //     the copies; 4 waves otherwise;
-//   * HBM -> LDS with buffer_load ... lds (tile_io.hpp) into two LDS stages for the 256-row tiles (160 to 256 columns) and
+//   * HBM -> LDS with buffer_load ... lds (tile_io.hpp) into two LDS stages, three of the weights, for the 256-row tiles (160 to 256 columns) and
 //     into a ring of 3 to 12 stages for the smaller tiles, which run problems bound by operand streaming; the tiles of the
 //     decode shapes (32 x 32, 64 x 32) consume their ring four k-tiles per barrier, with four more waves that only copy;
 //   * 16x16x128 e4m3 MFMAs: one instruction covers a whole scale block, starts from a zero accumulator and
@@ -17,8 +17,7 @@
 //     meets one activation row per atom: one sA per lane per atom per K block, and sB is wave-uniform;
 //   * the running sums stay in architectural VGPRs (the VALU cannot address AGPRs): 128 per wave;
 //   * the output leaves through LDS: each wave turns its slab round through the stage that was consumed last and stores
-//     16 bytes per lane in row runs of 2 * WTN bytes (non-temporal when the output is larger than the L2s together,
-//     except in the persistent walk, whose stores are plain);
+//     16 bytes per lane in row runs of 2 * WTN bytes (non-temporal when the output is larger than the L2s together);
 //   * the plain GEMM on the 256-row tiles is a persistent walk: one workgroup per compute unit takes tile after tile and
 //     overlaps the seams (fp8_gemm_walk); every other case runs a workgroup per tile, or a plain loop under a cap;
 //   * problems with long K and fewer tiles than compute units split K over SPLIT_K workgroups per tile on the ring tiles
@@ -82,10 +81,15 @@ struct Fp8TileConfig {
     // flight (a stage is only 9 to 13 KB there). Measured with every unit pulling: about 60 GB/s per unit whatever the
     // tile, so the tile to prefer is the one that moves the fewest bytes per output, 32 x 32 for a 64-row problem.
     static constexpr int  RING_DEPTH_CAP = BLOCK_N <= 32 ? 12 : 8;
-    // Room for a third stage of weights next to two of activations, and rows of atoms enough to hand its copies out one per row
-    // (kDeepB in fp8_gemm_tile).
-    static constexpr bool DEEP_B_CAPABLE = LDS_BYTES + LDS_ROWS_B * kRowBytes <= 160 * 1024 &&
-                                           (TileStager<BLOCK_M, NUM_WAVES>::PASSES + 1) / 2 + TileStager<BLOCK_N, NUM_WAVES>::PASSES <= WTN / 16;
+    // Room for a third stage of weights next to two of activations: every tile of 256 rows has it. A wave hands its copies out
+    // while it multiplies, activations (due at the next k-tile) two per row of atoms, then weights (due a k-tile later) one per
+    // row; tiles with few rows of atoms spread them evenly.
+    static constexpr bool DEEP_B_CAPABLE = LDS_BYTES + LDS_ROWS_B * kRowBytes <= 160 * 1024;
+    static constexpr int  COPIES_A = TileStager<BLOCK_M, NUM_WAVES>::PASSES, COPIES_B = TileStager<BLOCK_N, NUM_WAVES>::PASSES;
+    __device__ static constexpr int row_of_deep_copy(int d) {
+        if ((COPIES_A + 1) / 2 + COPIES_B > WTN / 16) return d * (WTN / 16) / (COPIES_A + COPIES_B);
+        return d < COPIES_A ? d / 2 : (COPIES_A + 1) / 2 + d - COPIES_A;
+    }
     static constexpr int  MAX_RING_STAGES = RING_CAPABLE ? (160 * 1024 / RING_STAGE_BYTES < RING_DEPTH_CAP ? 160 * 1024 / RING_STAGE_BYTES : RING_DEPTH_CAP) : 2;
 };
 
@@ -395,25 +399,20 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     using StB = TileStager<BLOCK_N, NW>;
     constexpr int NUM_COPIES = StA::PASSES + StB::PASSES, SPREAD_ROWS = TN >= 2 ? TN / 2 : 1;
     float sa_cur[TM], sb_cur[NB];
-    // Tall tiles of the contiguous layout hold a third stage of weights (160 KB of LDS with it) and fetch them two k-tiles
-    // ahead. Groups of a few hundred rows stream their weights from HBM, every weight panel for one or two tiles, and one
-    // k-tile of prefetch does not cover that: 16 groups of 256 rows x 4096 x 7168, 470 MB of weights in one round of tiles,
-    // 143 -> 135 us; 48 blocks of 128 rows over 16 groups 219 -> 201 us, and 197 with the copies handed out in the order of
-    // their deadlines, activations (due at the next k-tile) two per row of atoms, then weights one per row. One group of
-    // 8192 rows, whose weights come from the caches, runs level (195 us).
-    constexpr bool kDeepB = kGemmType == GemmType::GroupedContiguous && EXPLICIT_TILE && STAGES == 2 && Cfg::DEEP_B_CAPABLE;
-    auto row_of_copy = [](int d) { return !kDeepB ? d * SPREAD_ROWS / NUM_COPIES : (d < StA::PASSES ? d / 2 : (StA::PASSES + 1) / 2 + d - StA::PASSES); };
+    // Where the LDS has room for it (all tiles of 256 rows) a third stage of weights lets them be fetched two k-tiles ahead, and the
+    // copies are handed out in the order of their deadlines (row_of_deep_copy): one k-tile does not cover operands that come
+    // from HBM. 16 groups of 256 rows x 4096 x 7168, 470 MB of weights in one round of tiles, 143 -> 135 us; 48 blocks of 128
+    // rows over 16 groups 219 -> 201 us, and 197 with the order; one group of 8192 rows, whose weights come from the caches,
+    // level (195 us).
+    constexpr bool kDeepB = STAGES == 2 && Cfg::DEEP_B_CAPABLE;
+    auto row_of_copy = [](int d) { return kDeepB ? Cfg::row_of_deep_copy(d) : d * SPREAD_ROWS / NUM_COPIES; };
     auto k_step = [&](int kb, const uint8_t* a_cur, const uint8_t* b_cur, uint8_t* a_nxt, uint8_t* b_nxt) {
 #pragma unroll
         for (int j = 0; j < TM; ++j) sa_cur[j] = sa_next[j];
 #pragma unroll
         for (int b = 0; b < NB; ++b) sb_cur[b] = sb_next[b];
-        if constexpr (kDeepB) {         // all but the youngest copies, the weights of k-tile kb + 1
-            __builtin_amdgcn_s_waitcnt(waitcnt_imm(StB::PASSES, kNoWaitLgkm));
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-        } else {
+        if constexpr (kDeepB) meet_all_but<StB::PASSES>();      // all but the youngest copies, the weights of k-tile kb + 1
+        else {
             wait_for_copies();
             __syncthreads();
         }
@@ -457,22 +456,6 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
         }
         epi_a = a_nxt;          // the stages of the last k-tile
         epi_b = b_two;
-    } else if constexpr (SHAPE_K != 0 && (SHAPE_K / 128) % 2 == 1 && SHAPE_K / 128 <= 31 && TN * TM >= 32) {
-        // One copy of the k-step with the stages changing places. An odd number of k-tiles has a third copy behind the loop's two,
-        // and 256 x 256 tiles, whose registers are full, spill 32 of them around it, at three k-tiles 239: 5658 x 8256 x 2688 133
-        // us that way, 128 this way, 3529 x 7616 x 896 38.7 and 35.2. Changing places costs in every step, and from some 35 k-tiles on
-        // more than the spills do (3186 x 4032 x 8320 112 and 116). Narrower tiles do not spill.
-        uint8_t *a_cur = lds_a0, *a_nxt = lds_a1, *b_cur = lds_b0, *b_nxt = lds_b1;
-#pragma unroll 1
-        for (int kb = 0; kb < NUM_K_BLOCKS; ++kb) {
-            k_step(kb, a_cur, b_cur, a_nxt, b_nxt);
-            uint8_t* t = a_cur;
-            a_cur = a_nxt; a_nxt = t;
-            t = b_cur;
-            b_cur = b_nxt; b_nxt = t;
-        }
-        epi_a = lds_a0;         // the stages of the last k-tile
-        epi_b = lds_b0;
     } else {
         for (int kb = 0; kb + 1 < NUM_K_BLOCKS; kb += 2) {
             k_step(kb, lds_a0, lds_b0, lds_a1, lds_b1);
@@ -680,20 +663,28 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     }
 }
 
-// Whether a problem runs the persistent walk below: the plain GEMM on two LDS stages with an even number of k-tiles
-// (every tile then starts in stage 0).
-template <int STAGES, GemmType kGemmType>
+// Whether a problem runs the persistent walk below: the plain GEMM on two LDS stages (three of the weights) with two k-tiles or more.
+template <int BLOCK_M, int BLOCK_N, int STAGES, GemmType kGemmType>
 __host__ __device__ constexpr bool fp8_walks(int k) {
-    return STAGES == 2 && kGemmType == GemmType::Normal && (k / 128) % 2 == 0;
+    return STAGES == 2 && kGemmType == GemmType::Normal && Fp8TileConfig<BLOCK_M, BLOCK_N>::DEEP_B_CAPABLE && k >= 256;
 }
 
 // The plain GEMM on two LDS stages as a persistent walk: workgroup b takes slots b, b + gridDim.x, ... (the launcher
 // starts one workgroup per CU, or as many as the caller's cap allows) and overlaps the seams between them. The copies of
-// the next tile's first k-tile and its first scales start during the last k-tile of the current one, every wave waits
-// for them in front of the epilogue, and the output stores drain while the next tile's first k-tile is being
-// multiplied. With a workgroup per tile every tile pays for its first loads, its store drain and a workgroup launch:
-// 4096 x 7168 x 7168 runs 1.5 % faster this way, 4096 x 24576 x 1536 5 %, 4096 x 32768 x 512 15 %. Same bits: the sum
-// over K is formed in the same order.
+// the next tile's first k-tile and its first scales start during the last k-tile of the current one (weights one k-tile
+// earlier), every wave waits for them in front of the epilogue, and the output stores drain while the next tile's first
+// k-tile is being multiplied. With a workgroup per tile every tile pays for its first loads, its store drain and a
+// workgroup launch: 4096 x 7168 x 7168 runs 1.5 % faster this way, 4096 x 24576 x 1536 5 %, 4096 x 32768 x 512 15 %. Same
+// bits: the sum over K is formed in the same order.
+// Bound by the matrix cores and, under load, by energy (a tile's time at the clock the power allows). What a first pass over
+// new operands adds is waiting for HBM, which one k-tile of prefetch does not cover: weights are fetched two k-tiles ahead into
+// a third stage, and activations handed out first (row_of_deep_copy). The k-tiles that fetch for their own tile are a loop of
+// their own, without the selects of the last two (2 % of a k-tile), and outputs larger than the L2s together are stored with the
+// non-temporal hint (2-7 %; with the same operands call after call plain stores were 1 % faster). Inputs changing from call to
+// call, two stages and plain stores before -> now: 4096 x 7168 x 7168 189 -> 178 us, 8192 x 7168 x 7168 371 -> 350, 8192 x 2112 x
+// 7168 on 256 x 160 tiles 159 -> 140, 4096 x 24576 x 1536 159 -> 143, 3529 x 7616 x 1024 39.8 -> 33.3, one round of tiles
+// (4096 x 4096 x 7168) 101.8 -> 100.8; twelve shapes 0.92 on average, an odd number of k-tiles (3529 x 7616 x 896, a workgroup per tile
+// before) 31.7 -> 30.6.
 // What a wave needs to know of a tile is wave-uniform: the per-lane parts of every address (the lane's row within a copy
 // pass, its row within the slab) do not depend on the tile, and the tile's first row rides in the scalar offset.
 template <int SHAPE_N, int SHAPE_K, int BLOCK_M, int BLOCK_N>
@@ -705,11 +696,11 @@ fp8_gemm_walk(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     constexpr int NW = Cfg::NUM_WAVES, TN = Cfg::WTN / 16, TM = Cfg::WTM / 16, NB = Cfg::SCALE_B_PER_SLAB;
     // SHAPE_N / SHAPE_K == 0 selects the run-time sizes (ahead-of-time library); the JIT bakes them in.
     const int N = SHAPE_N ? SHAPE_N : n_rt, K = SHAPE_K ? SHAPE_K : k_rt;
-    const int NUM_K_BLOCKS = K / 128, NUM_N_BLOCKS = ceil_div(N, 128);          // NUM_K_BLOCKS is even: the caller checked
+    const int NUM_K_BLOCKS = K / 128, NUM_N_BLOCKS = ceil_div(N, 128);          // two k-tiles or more: the caller checked
     static_assert(Cfg::WTN >= 32);
     using StA = TileStager<BLOCK_M, NW>;
     using StB = TileStager<BLOCK_N, NW>;
-    constexpr int NUM_COPIES = StA::PASSES + StB::PASSES, SPREAD_ROWS = TN >= 2 ? TN / 2 : 1;
+    constexpr int NUM_COPIES = StA::PASSES + StB::PASSES;
 
     const XcdTileScheduler<> sched(m, N, BLOCK_M, BLOCK_N, (long long)K);
     const int lane = get_lane_id();
@@ -721,12 +712,8 @@ fp8_gemm_walk(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     const __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(rhs, uint32_t(N) * K);
     const uint32_t sa_bytes = (uint32_t(m - 1) * sa_stride_m + uint32_t(NUM_K_BLOCKS - 1) * sa_stride_k + 1) * 4;
     const __amdgpu_buffer_rsrc_t rsrc_sa = make_rsrc(lhs_scales, sa_bytes);
-    // Output stores are plain here at every size: they drain while the next tile's first k-tile is multiplied, and
-    // since loads and stores of a wave complete in order, stores that the L2 takes in at once free the loads behind
-    // them sooner than non-temporal ones (4096 x 24576 x 1536: 145 -> 138 us; 8192 x 7168 x 7168: 339 -> 336 us).
-    // The one-tile-per-slot kernel above is the other way round (4 groups of 4096 x 4096 x 7168: 439 us non-temporal,
-    // 506 us plain).
-    constexpr bool stream_out = false;
+    // as in fp8_gemm_tile: an output larger than the L2s together must not push the operand panels out of them
+    const bool stream_out = size_t(m) * N * 2 > (size_t(32) << 20);
 
     struct TileIo {
         int m0, n0;
@@ -754,43 +741,43 @@ fp8_gemm_walk(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
 
     f32x4 acc[TN][TM];
     float sa_next[TM], sb_next[NB], sa_cur[TM], sb_cur[NB];
-    auto load_scales = [&](const TileIo& t, int kb) {
+    auto load_scales = [&](int m0, int base_blk, int kb) {
 #pragma unroll
         for (int j = 0; j < TM; ++j)
-            sa_next[j] = buffer_load_f32(rsrc_sa, sa_voff, (kb * sa_stride_k + (t.m0 + j * 16) * sa_stride_m) * 4);
+            sa_next[j] = buffer_load_f32(rsrc_sa, sa_voff, (kb * sa_stride_k + (m0 + j * 16) * sa_stride_m) * 4);
 #pragma unroll
-        for (int b = 0; b < NB; ++b) sb_next[b] = rhs_scales[min(t.base_blk + b, NUM_N_BLOCKS - 1) * NUM_K_BLOCKS + kb];
+        for (int b = 0; b < NB; ++b) sb_next[b] = rhs_scales[min(base_blk + b, NUM_N_BLOCKS - 1) * NUM_K_BLOCKS + kb];
     };
 
-    uint8_t* const lds_a0 = two_stages.a0;
-    uint8_t* const lds_b0 = two_stages.b0;
-    uint8_t* const lds_a1 = two_stages.a1;
-    uint8_t* const lds_b1 = two_stages.b1;
+    uint8_t *a_cur = two_stages.a0, *a_nxt = two_stages.a1;                                    // stages of this k-tile and the next,
+    uint8_t *b_cur = two_stages.b0, *b_nxt = two_stages.b1, *b_third = two_stages.b2;          // and the one after that
 
-    // One k-tile of tile `t`, staged in (a_cur, b_cur) and known to have landed when `landed`; meanwhile the copies of
-    // k-tile `kb_src` of tile `src` go into (a_nxt, b_nxt) and its scales into registers (`src` is `t` itself, or the
-    // next tile during the last k-tile).
-    auto k_step = [&](const TileIo& t, const uint8_t* a_cur, const uint8_t* b_cur, uint8_t* a_nxt, uint8_t* b_nxt,
-                      const TileIo& src, int kb_src, bool landed) {
-        const int a_byte0 = src.m0 * K + kb_src * kRowBytes, b_byte0 = src.n0 * K + kb_src * kRowBytes;
+    // k-tile `kb` of tile `t`, which has landed when LANDED. Meanwhile the activations and scales of the k-tile behind it and
+    // the weights of the one behind that are fetched, from tile `nxt` past the last of `t` (INSIDE: both belong to `t`).
+    auto k_step = [&]<bool LANDED, bool INSIDE>(const TileIo& t, const TileIo& nxt, int kb) {
+        const bool own_a = INSIDE || kb + 1 < NUM_K_BLOCKS, own_b = INSIDE || kb + 2 < NUM_K_BLOCKS;
+        const int kb_a = own_a ? kb + 1 : 0, kb_b = own_b ? kb + 2 : kb + 2 - NUM_K_BLOCKS;
+        const int m0_a = own_a ? t.m0 : nxt.m0;
+        const int a_byte0 = m0_a * K + kb_a * kRowBytes, b_byte0 = (own_b ? t.n0 : nxt.n0) * K + kb_b * kRowBytes;
 #pragma unroll
         for (int j = 0; j < TM; ++j) sa_cur[j] = sa_next[j];
 #pragma unroll
         for (int b = 0; b < NB; ++b) sb_cur[b] = sb_next[b];
-        if (!landed) {
-            wait_for_copies();
-            __syncthreads();
-        }
-        load_scales(src, kb_src);
+        if constexpr (!LANDED) meet_all_but<StB::PASSES>();
+        load_scales(m0_a, own_a ? t.base_blk : nxt.base_blk, kb_a);
         fp8_compute_k_tile<Cfg>(acc, a_cur + wm * Cfg::WTM * kRowBytes, b_cur + wn * Cfg::WTN * kRowBytes, sa_cur, sb_cur,
                                 t.rows_in_first_block, off0, off1, [&](int row) {
 #pragma unroll
             for (int d = 0; d < NUM_COPIES; ++d) {
-                if (d * SPREAD_ROWS / NUM_COPIES != row) continue;
+                if (Cfg::row_of_deep_copy(d) != row) continue;
                 if (d < StA::PASSES) stage_a.issue_pass(rsrc_a, a_nxt, a_byte0, wave, d);
-                else stage_b.issue_pass(rsrc_b, b_nxt, b_byte0, wave, d - StA::PASSES);
+                else stage_b.issue_pass(rsrc_b, b_third, b_byte0, wave, d - StA::PASSES);
             }
         });
+        uint8_t* p = a_cur;
+        a_cur = a_nxt; a_nxt = p;
+        p = b_cur;
+        b_cur = b_nxt; b_nxt = b_third; b_third = p;
     };
 
     // The next slot of this workgroup's walk that holds a tile. Under a cap that is not a multiple of the 8 XCDs a walk
@@ -802,11 +789,11 @@ fp8_gemm_walk(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     int slot = seek(blockIdx.x);
     TileIo cur = open_tile(slot);
     if (!cur.valid) return;
-    stage_a.issue(rsrc_a, lds_a0, cur.m0 * K, wave);
-    stage_b.issue(rsrc_b, lds_b0, cur.n0 * K, wave);
-    load_scales(cur, 0);
-    wait_for_copies();
-    __syncthreads();
+    stage_a.issue(rsrc_a, a_cur, cur.m0 * K, wave);
+    stage_b.issue(rsrc_b, b_cur, cur.n0 * K, wave);
+    load_scales(cur.m0, cur.base_blk, 0);
+    stage_b.issue(rsrc_b, b_nxt, cur.n0 * K + kRowBytes, wave);
+    meet_all_but<StB::PASSES>();
     while (true) {
         slot = seek(slot + gridDim.x);
         const TileIo nxt = open_tile(slot);
@@ -815,13 +802,12 @@ fp8_gemm_walk(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
 #pragma unroll
             for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         // k-tile 0 has landed for every wave: the barrier in front of the loop, or the one in front of the last epilogue
-        k_step(cur, lds_a0, lds_b0, lds_a1, lds_b1, cur, 1, true);
-        for (int kb = 1; kb + 2 < NUM_K_BLOCKS; kb += 2) {
-            k_step(cur, lds_a1, lds_b1, lds_a0, lds_b0, cur, kb + 1, false);
-            k_step(cur, lds_a0, lds_b0, lds_a1, lds_b1, cur, kb + 2, false);
-        }
-        // the last k-tile, in stage 1; stage 0 takes the first k-tile of the next tile
-        k_step(cur, lds_a1, lds_b1, lds_a0, lds_b0, nxt, 0, false);
+        k_step.template operator()<true, false>(cur, nxt, 0);
+        int kb = 1;
+#pragma unroll 1
+        for (; kb + 2 < NUM_K_BLOCKS; ++kb) k_step.template operator()<false, true>(cur, nxt, kb);
+#pragma unroll 1
+        for (; kb < NUM_K_BLOCKS; ++kb) k_step.template operator()<false, false>(cur, nxt, kb);
         // the sums are complete here: without this the compiler moves the last folds down into the epilogue, next to their
         // first use, and parks the partial sums they wait for in scratch memory
 #pragma unroll
@@ -829,16 +815,17 @@ fp8_gemm_walk(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
 #pragma unroll
             for (int j = 0; j < TM; ++j) asm volatile("" : "+v"(acc[i][j]));
 
-        // every wave has read the last k-tile and the next tile's first k-tile has landed; then the epilogue through stage 1
-        wait_for_copies();
-        __syncthreads();
+        // every wave has read the last k-tile, and the next tile's first k-tile has landed; then the epilogue through the stages of
+        // the last k-tile, which no copy is on its way into
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm(kNoWaitVm, 0));
+        meet_all_but<StB::PASSES>();
         {
             constexpr int REGION = 16 * (Cfg::WTN * 2 + 16);
             static_assert((NW / 2) * REGION <= Cfg::LDS_ROWS_A * kRowBytes && (NW / 2) * REGION <= Cfg::LDS_ROWS_B * kRowBytes);
             const __amdgpu_buffer_rsrc_t rsrc_out = make_out_rsrc(out + size_t(cur.m0) * N + cur.n0);
             int lane_late = lane;
             asm volatile("" : "+v"(lane_late));
-            uint8_t* region = (wave < NW / 2 ? lds_a1 : lds_b1) + (wave % (NW / 2)) * REGION;
+            uint8_t* region = (wave < NW / 2 ? a_nxt : b_third) + (wave % (NW / 2)) * REGION;
             if ((N % 8) == 0)
                 fp8_store_slab<Cfg, true>(acc, region, rsrc_out, cur.m0 + wm * Cfg::WTM, cur.n0 + wn * Cfg::WTN, cur.m0, cur.n0,
                                           m, N, stream_out, lane_late);
@@ -846,9 +833,12 @@ fp8_gemm_walk(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
                 fp8_store_slab<Cfg, false>(acc, region, rsrc_out, cur.m0 + wm * Cfg::WTM, cur.n0 + wn * Cfg::WTN, cur.m0, cur.n0,
                                            m, N, stream_out, lane_late);
         }
-        if (!nxt.valid) break;
+        if (!nxt.valid) {
+            wait_for_copies();          // of weights nobody will read: none lands in LDS that is no longer this workgroup's
+            break;
+        }
         cur = nxt;
-        // the next tile's second k-tile is copied into the stage the epilogue went through: every wave has to be out of it
+        // the next tile's second k-tile is copied into the stages the epilogue went through: every wave has to be out of them
         __builtin_amdgcn_s_waitcnt(waitcnt_imm(kNoWaitVm, 0));
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
@@ -874,10 +864,13 @@ fp8_gemm_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_s
         __shared__ __attribute__((aligned(1024))) uint8_t lds_b0[Cfg::LDS_ROWS_B * kRowBytes];
         __shared__ __attribute__((aligned(1024))) uint8_t lds_a1[Cfg::LDS_ROWS_A * kRowBytes];
         __shared__ __attribute__((aligned(1024))) uint8_t lds_b1[Cfg::LDS_ROWS_B * kRowBytes];
-        two_stages = {lds_a0, lds_b0, lds_a1, lds_b1, nullptr};
+        if constexpr (Cfg::DEEP_B_CAPABLE) {
+            __shared__ __attribute__((aligned(1024))) uint8_t lds_b2[Cfg::LDS_ROWS_B * kRowBytes];
+            two_stages = {lds_a0, lds_b0, lds_a1, lds_b1, lds_b2};
+        } else two_stages = {lds_a0, lds_b0, lds_a1, lds_b1, nullptr};
     }
-    if constexpr (fp8_walks<STAGES, kGemmType>(SHAPE_K)) {
-        if (SHAPE_K != 0 || fp8_walks<STAGES, kGemmType>(k_rt)) {
+    if constexpr (fp8_walks<BLOCK_M, BLOCK_N, STAGES, kGemmType>(SHAPE_K ? SHAPE_K : 256)) {
+        if (SHAPE_K != 0 || fp8_walks<BLOCK_M, BLOCK_N, STAGES, kGemmType>(k_rt)) {
             fp8_gemm_walk<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N>(lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt, sa_stride_m, sa_stride_k,
                                                               num_slots, two_stages);
             return;
@@ -1136,7 +1129,7 @@ public:
         const XcdTileScheduler<> sched(m, n, BLOCK_M, BLOCK_N);
         const int slots = sched.grid_size();
         int grid = capped_grid(slots, num_sms, device_cu_count());
-        if (fp8_walks<int(kNumStages), GemmType::Normal>(k)) {
+        if (fp8_walks<BLOCK_M, BLOCK_N, int(kNumStages), GemmType::Normal>(k)) {
             // persistent: one workgroup per CU (a multiple of the 8 XCDs, so a workgroup's tiles stay on one XCD), or as
             // many as the caller's cap allows
             const int cus = device_cu_count() / kNumXCD * kNumXCD;

@@ -38,6 +38,15 @@ __device__ __forceinline__ void wait_for_copies() {
     __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, kNoWaitLgkm));
 }
 
+// All waves of a workgroup meet once each has at most its YOUNGEST latest vector-memory operations outstanding.
+template <int YOUNGEST>
+__device__ __forceinline__ void meet_all_but() {
+    __builtin_amdgcn_s_waitcnt(waitcnt_imm(YOUNGEST, kNoWaitLgkm));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // One fp32 through a descriptor: per-lane byte offset + wave-uniform byte offset; out of range reads 0.0f.
 __device__ __forceinline__ float buffer_load_f32(__amdgpu_buffer_rsrc_t rsrc, uint32_t voffset, uint32_t soffset) {
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, voffset, soffset, 0));
