@@ -331,6 +331,29 @@ CAPPED_SHAPES = [(2048, 4096, 1024), (512, 4096, 2048), (300, 2112, 640)]
 DENSE_RAGGED_CAP_CASE = ([(128, 128), (128, 192), (64, 64), (256, 128)], (390, 516), (72, 200), 8)
 
 
+# Weights of 32 MB and more are fetched with the non-temporal hint where few tile rows read them: (tile, parts of K), rows, (n, k)
+# of a problem that has them so and whose halves along n do not.
+STREAM_FP8_CASES = [((32, 32), 1), ((64, 128), 1), ((64, 64), 4)]
+STREAM_DENSE_CASES = [((64, 64), 1), ((128, 128), 1), ((64, 64), 4)]
+STREAM_FP8_SIZES, STREAM_DENSE_SIZES = (61, 8192, 4096), (125, 8192, 2048)
+STREAM_GROUPED_SIZES = (8, 64, 2048, 2048)          # groups, rows of each, n, k
+
+
+def stream_plans(kind: str, tile, split_k: int, n: int):
+    """(name, keys, arg_defs, includes, template) of the plain FP8 or dense kernel with this tile and factor for `n` columns."""
+    from yan_amd.jit_kernels import bf16_gemm, gemm, heuristics
+    if kind == 'fp8':
+        name, keys, arg_defs, template = fp8_explicit_tile_plan(*tile, n, STREAM_FP8_SIZES[2])
+        if split_k > 1:
+            name, keys, arg_defs, template = name + '_split_k', {**keys, 'SPLIT_K': split_k}, gemm.split_k_arg_defs, gemm.split_k_template
+        return name, keys, arg_defs, gemm.includes, template
+    name, keys, arg_defs, includes, template = dense_tile_plan(tile, torch.bfloat16, 0)
+    if split_k > 1:
+        keys = {'BLOCK_M': tile[0], 'BLOCK_N': tile[1], 'NUM_STAGES': heuristics.get_dense_num_stages(*tile), 'SPLIT_K': split_k}
+        return name + '_split_k', keys, bf16_gemm._split_k_arg_defs(torch.bfloat16), includes, bf16_gemm.split_k_template
+    return name, keys, arg_defs, includes, template
+
+
 def dense_tile_plan(tile, dtype: torch.dtype, cap: int):
     """(name, keys, arg_defs, includes, template) of the dense GEMM on a tile given outright."""
     from yan_amd.jit_kernels import bf16_gemm, heuristics
@@ -482,6 +505,18 @@ def jit_kernels_in_use(num_cus: int = 256):
         for k in depths:
             name, keys, arg_defs, code_template = fp8_explicit_tile_plan(*tile, FP8_SHORT_K_SIZES[1], k)
             add(name, arg_defs, gemm.includes, code_template, keys)
+    for tile, split_k in STREAM_FP8_CASES:
+        for n in (STREAM_FP8_SIZES[1], STREAM_FP8_SIZES[1] // 2):
+            name, keys, arg_defs, includes, code_template = stream_plans('fp8', tile, split_k, n)
+            add(name, arg_defs, includes, code_template, keys)
+    for tile, split_k in STREAM_DENSE_CASES:
+        name, keys, arg_defs, includes, code_template = stream_plans('dense', tile, split_k, 0)
+        add(name, arg_defs, includes, code_template, keys)
+    for kind in ('GroupedMasked', 'GroupedContiguous'):
+        for n in (STREAM_GROUPED_SIZES[2], STREAM_GROUPED_SIZES[2] // 2):
+            m = STREAM_GROUPED_SIZES[1] if kind == 'GroupedMasked' else 128 * STREAM_GROUPED_SIZES[0]
+            name, keys, arg_defs, _ = m_grouped_gemm.grouped_kernel_plan(kind, STREAM_GROUPED_SIZES[0], m, n, STREAM_GROUPED_SIZES[3], num_cus)
+            add(name, arg_defs, m_grouped_gemm.includes, m_grouped_gemm.template, keys)
     for tile, depths in FP8_WALK_CASES:
         for k in depths:
             name, keys, arg_defs, code_template = fp8_explicit_tile_plan(*tile, FP8_WALK_SIZES[1], k, 2)

@@ -201,3 +201,54 @@ def test_quantisers_on_odd_sizes_and_odd_values(m, k, dtype):
     assert torch.equal(sc, block_amax / torch.full_like(block_amax, 448.0))
     finite = want.abs() <= 448.0
     assert torch.equal(q.view(torch.uint8)[finite], want.to(torch.float8_e4m3fn).view(torch.uint8)[finite])
+
+
+def _streamed_weights_case(kind, tile, split_k):
+    """The kernel on all columns (weights streamed) and on either half of them (not)."""
+    dense = kind == 'dense'
+    m, n, k = testing.STREAM_DENSE_SIZES if dense else testing.STREAM_FP8_SIZES
+    outs = []
+    if dense:
+        a, b, c = testing.make_bf16_case(m, n, k, seed=17, device='cuda')
+    else:
+        (a, sa), (b, sb), c = testing.make_fp8_case(m, n, k, seed=17, device='cuda', gen_device='cuda')
+        sa = yan.get_col_major_tensor(sa)
+    workspace = torch.zeros(16384 + 256 * 128 * 128 * 4, dtype=torch.uint8, device='cuda')
+    stream = torch.cuda.current_stream()
+    for lo, hi in ((0, n), (0, n // 2), (n // 2, n)):
+        name, keys, arg_defs, includes, code_template = testing.stream_plans(kind, tile, split_k, hi - lo)
+        kernel = jit.build(name, arg_defs, jit.generate(includes, arg_defs, jit.cpp_format(code_template, keys)))
+        out = torch.full((m, hi - lo), float('nan'), dtype=torch.bfloat16, device='cuda')
+        args = (m, hi - lo, k, a, b[lo:hi], out, stream) if dense else (a, sa, b[lo:hi], sb[lo // 128:hi // 128], out, m, stream, 0, 0)
+        assert kernel(*args, *((workspace, workspace.numel()) if split_k > 1 else ())) == 0
+        torch.cuda.synchronize()
+        outs.append(out)
+    return outs
+
+
+@pytest.mark.parametrize('kind,tile,split_k', [('fp8', *c) for c in testing.STREAM_FP8_CASES] + [('dense', *c) for c in testing.STREAM_DENSE_CASES])
+def test_streamed_weights_give_the_same_bits(kind, tile, split_k):
+    _announce('streamed weights', kind, tile, split_k)
+    whole, left, right = _streamed_weights_case(kind, tile, split_k)
+    assert torch.equal(whole, torch.cat([left, right], dim=1))
+
+
+@pytest.mark.parametrize('masked', [False, True])
+def test_streamed_weights_of_groups_give_the_same_bits(masked):
+    groups, rows, n, k = testing.STREAM_GROUPED_SIZES
+    _announce('streamed weights of groups', masked)
+    if masked:
+        (a, sa), (b, sb), out, layout = testing.make_grouped_masked_case(groups, rows, n, k, (5, 64, 0, 1, 33, 64, 2, 17), seed=18, device='cuda')
+    else:
+        (a, sa), (b, sb), out, layout = testing.make_grouped_contiguous_case((128, 7, 100, 1, 128, 64, 2, 90), n, k, seed=18, device='cuda')
+
+    def run(lo, hi):
+        part = torch.full_like(out[..., lo:hi], -7.0, memory_format=torch.contiguous_format)
+        rhs = b[:, lo:hi].contiguous(), sb[:, lo // 128:hi // 128].contiguous()
+        if masked:
+            yan.m_grouped_gemm_fp8_fp8_bf16_nt_masked((a, sa), rhs, part, layout, rows)
+        else:
+            yan.m_grouped_gemm_fp8_fp8_bf16_nt_contiguous((a, sa), rhs, part, layout)
+        torch.cuda.synchronize()
+        return part
+    assert torch.equal(run(0, n), torch.cat([run(0, n // 2), run(n // 2, n)], dim=-1))

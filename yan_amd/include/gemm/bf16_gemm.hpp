@@ -26,6 +26,8 @@
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 
+#include <type_traits>
+
 #include "utils.hpp"
 #include "mfma_utils.hpp"
 #include "scheduler.hpp"
@@ -87,7 +89,8 @@ __host__ __device__ constexpr int dense_launch_waves(int block_m, int block_n, i
     return block_m * block_n >= 128 * 128 && split_k >= 4 ? 4 : 8;
 }
 
-template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K = 1>
+// STREAM: the copies of B carry the non-temporal hint (streams_weights in scheduler.hpp).
+template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K = 1, bool STREAM = false>
 __device__ __forceinline__ void
 dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, Elem* __restrict__ C,
                 int m, int n, int k, int bid, float* __restrict__ partials = nullptr, unsigned* __restrict__ counters = nullptr) {
@@ -112,7 +115,7 @@ dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
     const __amdgpu_buffer_rsrc_t rsrc_a = make_rsrc(A, uint32_t(m) * ld_bytes);
     const __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(B, uint32_t(n) * ld_bytes);
     TileStager<BLOCK_M, LW> stage_a;
-    TileStager<BLOCK_N, LW> stage_b;
+    TileStager<BLOCK_N, LW, STREAM> stage_b;
     stage_a.init(m0, ld_bytes, wave, lane);
     stage_b.init(n0, ld_bytes, wave, lane);
 
@@ -872,47 +875,47 @@ dense_gemm_mfma_8w(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
 // Workgroup b runs tiles b, b + gridDim.x, ...: exactly one when the launcher starts a workgroup per tile, several under
 // a compute-unit cap. Between two tiles every wave must have left the epilogue of the first, which reads an LDS stage
 // the second one's first copies go into.
-template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES>
+template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES, bool STREAM>
 __device__ __forceinline__ void
 dense_gemm_walk(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, Elem* __restrict__ C, int m, int n, int k, int num_slots) {
     // a workgroup per tile (no cap): the tile without a loop around it (up to 2 % faster than one trip round the loop below)
     if (int(gridDim.x) >= num_slots) {
-        dense_gemm_body<Atom, Elem, BLOCK_M, BLOCK_N, STAGES>(A, B, C, m, n, k, int(blockIdx.x));
+        dense_gemm_body<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, 1, STREAM>(A, B, C, m, n, k, int(blockIdx.x));
         return;
     }
     for (int slot = blockIdx.x; slot < num_slots; slot += gridDim.x) {
-        dense_gemm_body<Atom, Elem, BLOCK_M, BLOCK_N, STAGES>(A, B, C, m, n, k, slot);
+        dense_gemm_body<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, 1, STREAM>(A, B, C, m, n, k, slot);
         if (slot + int(gridDim.x) < num_slots) __syncthreads();
     }
 }
 
-template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES>
+template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES, bool STREAM = false>
 __global__ void __launch_bounds__((dense_launch_waves(BLOCK_M, BLOCK_N) * kWaveSize))
 dense_gemm_mfma(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, Elem* __restrict__ C, int m, int n, int k, int num_slots) {
-    dense_gemm_walk<Atom, Elem, BLOCK_M, BLOCK_N, STAGES>(A, B, C, m, n, k, num_slots);
+    dense_gemm_walk<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, STREAM>(A, B, C, m, n, k, num_slots);
 }
 
 // The ring tiles with K split SPLIT_K ways: launch slot s is part s % SPLIT_K of tile slot s / SPLIT_K.
-template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K>
+template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K, bool STREAM = false>
 __global__ void __launch_bounds__((dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize))
 dense_gemm_split_k(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, Elem* __restrict__ C, int m, int n, int k,
                    float* __restrict__ partials, unsigned* __restrict__ counters) {
-    dense_gemm_body<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, SPLIT_K>(A, B, C, m, n, k, int(blockIdx.x), partials, counters);
+    dense_gemm_body<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, SPLIT_K, STREAM>(A, B, C, m, n, k, int(blockIdx.x), partials, counters);
 }
 
 // The fp16 flavour under the name of the reference's kernel (yan/include/gemm/cute_gemm.cuh:20), so that profiler
 // filters written for it (tests/test_cute.py:35 looks for 'fp16_gemm_cute') keep finding it.
-template <int BLOCK_M, int BLOCK_N, int STAGES>
+template <int BLOCK_M, int BLOCK_N, int STAGES, bool STREAM = false>
 __global__ void __launch_bounds__((dense_launch_waves(BLOCK_M, BLOCK_N) * kWaveSize))
 fp16_gemm_cute(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, _Float16* __restrict__ C, int m, int n, int k, int num_slots) {
-    dense_gemm_walk<MfmaF16_32x32x16, _Float16, BLOCK_M, BLOCK_N, STAGES>(A, B, C, m, n, k, num_slots);
+    dense_gemm_walk<MfmaF16_32x32x16, _Float16, BLOCK_M, BLOCK_N, STAGES, STREAM>(A, B, C, m, n, k, num_slots);
 }
 
-template <int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K>
+template <int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K, bool STREAM = false>
 __global__ void __launch_bounds__((dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize))
 fp16_gemm_cute_split_k(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, _Float16* __restrict__ C, int m, int n, int k,
                        float* __restrict__ partials, unsigned* __restrict__ counters) {
-    dense_gemm_body<MfmaF16_32x32x16, _Float16, BLOCK_M, BLOCK_N, STAGES, SPLIT_K>(A, B, C, m, n, k, int(blockIdx.x), partials, counters);
+    dense_gemm_body<MfmaF16_32x32x16, _Float16, BLOCK_M, BLOCK_N, STAGES, SPLIT_K, STREAM>(A, B, C, m, n, k, int(blockIdx.x), partials, counters);
 }
 
 template <int BLOCK_N>
@@ -979,14 +982,19 @@ inline hipError_t launch_dense(int m, int n, int k, const void* a, const void* b
                                static_cast<Elem*>(c), m, n, k);
     } else {
         const int grid = capped_grid(slots, num_sms, device_cu_count());
-        if constexpr (__is_same(Elem, _Float16))
-            hipLaunchKernelGGL((fp16_gemm_cute<BLOCK_M, BLOCK_N, STAGES>), dim3(grid),
-                               dim3(dense_launch_waves(BLOCK_M, BLOCK_N) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
-                               static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, slots);
-        else
-            hipLaunchKernelGGL((dense_gemm_mfma<Atom, Elem, BLOCK_M, BLOCK_N, STAGES>), dim3(grid),
-                               dim3(dense_launch_waves(BLOCK_M, BLOCK_N) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
-                               static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, slots);
+        auto launch = [&](auto stream_weights) {
+            constexpr bool STREAM = decltype(stream_weights)::value;
+            if constexpr (__is_same(Elem, _Float16))
+                hipLaunchKernelGGL((fp16_gemm_cute<BLOCK_M, BLOCK_N, STAGES, STREAM>), dim3(grid),
+                                   dim3(dense_launch_waves(BLOCK_M, BLOCK_N) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
+                                   static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, slots);
+            else
+                hipLaunchKernelGGL((dense_gemm_mfma<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, STREAM>), dim3(grid),
+                                   dim3(dense_launch_waves(BLOCK_M, BLOCK_N) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
+                                   static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, slots);
+        };
+        if (streams_weights(sched.tiles_m, uint64_t(n) * k * 2)) launch(std::true_type{});
+        else launch(std::false_type{});
     }
     return hipGetLastError();
 }
@@ -1008,14 +1016,19 @@ inline hipError_t launch_dense_split_k(int m, int n, int k, const void* a, const
     if (workspace_bytes < kSplitKCounterBytes + slots * SPLIT_K * BLOCK_M * BLOCK_N * 4) return hipErrorInvalidValue;
     unsigned* counters = static_cast<unsigned*>(workspace);
     float* partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kSplitKCounterBytes);
-    if constexpr (__is_same(Elem, _Float16))
-        hipLaunchKernelGGL((fp16_gemm_cute_split_k<BLOCK_M, BLOCK_N, STAGES, SPLIT_K>), dim3(int(slots) * SPLIT_K),
-                           dim3(dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
-                           static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, partials, counters);
-    else
-        hipLaunchKernelGGL((dense_gemm_split_k<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, SPLIT_K>), dim3(int(slots) * SPLIT_K),
-                           dim3(dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
-                           static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, partials, counters);
+    auto launch = [&](auto stream_weights) {
+        constexpr bool STREAM = decltype(stream_weights)::value;
+        if constexpr (__is_same(Elem, _Float16))
+            hipLaunchKernelGGL((fp16_gemm_cute_split_k<BLOCK_M, BLOCK_N, STAGES, SPLIT_K, STREAM>), dim3(int(slots) * SPLIT_K),
+                               dim3(dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
+                               static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, partials, counters);
+        else
+            hipLaunchKernelGGL((dense_gemm_split_k<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, SPLIT_K, STREAM>), dim3(int(slots) * SPLIT_K),
+                               dim3(dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
+                               static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, partials, counters);
+    };
+    if (streams_weights(sched.tiles_m, uint64_t(n) * k * 2)) launch(std::true_type{});
+    else launch(std::false_type{});
     return hipGetLastError();
 }
 

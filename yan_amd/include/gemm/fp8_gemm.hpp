@@ -35,6 +35,8 @@
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp8.h>
 
+#include <type_traits>
+
 #include "utils.hpp"
 #include "mfma_utils.hpp"
 #include "scheduler.hpp"
@@ -273,8 +275,9 @@ contiguous_block_at(const int* __restrict__ grouped_layout, int blocks, bool tal
 // tile and run one of them (fp8_gemm_contiguous_rows_kernel).
 // EXPLICIT_TILE: `bid` names the tile itself, as (its first row / 128) * tiles_n + n_idx, for callers that order the tiles
 // themselves; in the contiguous layout all rows of such a tile belong to the group of its first row.
+// STREAM: a ring tile's copies of the weights carry the non-temporal hint (streams_weights in scheduler.hpp).
 template <int SHAPE_N, int SHAPE_K, int BLOCK_M, int BLOCK_N, GemmType kGemmType, int STAGES, int SPLIT_K = 1, bool EXTERNAL_RING = false,
-          bool EXPLICIT_TILE = false>
+          bool EXPLICIT_TILE = false, bool STREAM = false>
 __device__ __forceinline__ void
 fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_scales,
               const uint8_t* __restrict__ rhs, const float* __restrict__ rhs_scales,
@@ -349,7 +352,7 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     // copies of k-tiles past the end of the range keep the count of instructions in flight and move nothing
     const __amdgpu_buffer_rsrc_t rsrc_none = make_rsrc(lhs, 0);
     TileStager<BLOCK_M, NW> stage_a;
-    TileStager<BLOCK_N, NW> stage_b;
+    TileStager<BLOCK_N, NW, STREAM> stage_b;
     stage_a.init(m0, K, wave, lane);
     stage_b.init(n0, K, wave, lane);
 
@@ -519,7 +522,7 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
         const bool in_a = sl * LW + LW - 1 < GA || (sl * LW < GA && o < GA);
         if (data) {
             if (in_a) __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_a : rsrc_none, YAN_LDS_CAST(stage + o * 8 * kRowBytes), kChunk, slot_voff[sl], kb * kRowBytes, 0, 0);
-            else __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_b : rsrc_none, YAN_LDS_CAST(stage + o * 8 * kRowBytes), kChunk, slot_voff[sl], kb * kRowBytes, 0, 0);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_b : rsrc_none, YAN_LDS_CAST(stage + o * 8 * kRowBytes), kChunk, slot_voff[sl], kb * kRowBytes, 0, STREAM ? kNonTemporal : 0);
         } else {
             __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_sa : rsrc_none, YAN_LDS_CAST(stage + TILE_BYTES), 4, scale_voff, kb * sa_stride_k * 4, 0, 0);
         }
@@ -851,7 +854,7 @@ fp8_gemm_walk(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
 // units (the reference's persistent kernel under `num_sms`,
 // yan/include/gemm/fp8_gemm.cuh:40, scheduler.cuh:39-58). Between two tiles every wave must have left the epilogue of
 // the first (which reads the LDS stage the second one's first copies go into).
-template <int SHAPE_N, int SHAPE_K, int BLOCK_M, int BLOCK_N, GemmType kGemmType = GemmType::Normal, int STAGES = 2>
+template <int SHAPE_N, int SHAPE_K, int BLOCK_M, int BLOCK_N, GemmType kGemmType = GemmType::Normal, int STAGES = 2, bool STREAM = false>
 __global__ void __launch_bounds__((fp8_launch_waves(BLOCK_M, BLOCK_N, STAGES) * kWaveSize))
 fp8_gemm_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_scales,
                 const uint8_t* __restrict__ rhs, const float* __restrict__ rhs_scales,
@@ -879,13 +882,13 @@ fp8_gemm_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_s
     // A workgroup per slot (no cap): the tile without a loop around it. Inside the loop below the same code runs 2 to 14 %
     // slower on the ring tiles even for a single trip (64 x 7168 x 2048 on 64 x 32 tiles: 6.0 against 5.2 us).
     if (int(gridDim.x) >= num_slots) {
-        fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, STAGES>(lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt,
+        fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, STAGES, 1, false, false, STREAM>(lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt,
                                                                              sa_stride_m, sa_stride_k, grouped_layout, sa_stride_g,
                                                                              int(blockIdx.x), num_groups, expected_m, two_stages);
         return;
     }
     for (int slot = blockIdx.x; slot < num_slots; slot += gridDim.x) {
-        fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, STAGES>(lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt,
+        fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, STAGES, 1, false, false, STREAM>(lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt,
                                                                              sa_stride_m, sa_stride_k, grouped_layout, sa_stride_g,
                                                                              slot, num_groups, expected_m, two_stages);
         if (slot + int(gridDim.x) < num_slots) __syncthreads();
@@ -977,13 +980,13 @@ fp8_gemm_contiguous_rows_kernel(const uint8_t* __restrict__ lhs, const float* __
 }
 
 // The same tiles with K split SPLIT_K ways: launch slot s is part s % SPLIT_K of tile slot s / SPLIT_K.
-template <int SHAPE_N, int SHAPE_K, int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K>
+template <int SHAPE_N, int SHAPE_K, int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K, bool STREAM = false>
 __global__ void __launch_bounds__((fp8_launch_waves(BLOCK_M, BLOCK_N, STAGES) * kWaveSize))
 fp8_gemm_split_k_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_scales,
                         const uint8_t* __restrict__ rhs, const float* __restrict__ rhs_scales,
                         __bf16* __restrict__ out, int m, int n_rt, int k_rt, int sa_stride_m, int sa_stride_k,
                         float* __restrict__ partials, unsigned* __restrict__ counters) {
-    fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, GemmType::Normal, STAGES, SPLIT_K>(
+    fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, GemmType::Normal, STAGES, SPLIT_K, false, false, STREAM>(
         lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt, sa_stride_m, sa_stride_k, nullptr, 0, int(blockIdx.x), 1, 0,
         Fp8TwoStages{}, partials, counters);
 }
@@ -1042,12 +1045,18 @@ public:
                                    : uint64_t(sched.grid_size());
         if (slots >= kOutOfRange) return hipErrorInvalidValue;
         const int grid = capped_grid(int(slots), num_sms, device_cu_count());
-        hipLaunchKernelGGL((fp8_gemm_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, int(kNumStages)>), dim3(grid),
-                           dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream, static_cast<const uint8_t*>(lhs), lhs_scales,
-                           static_cast<const uint8_t*>(rhs), rhs_scales, reinterpret_cast<__bf16*>(out), m, n, k,
-                           lhs_scales_stride_m, lhs_scales_stride_k, grouped_layout, lhs_scales_stride_g, int(slots), num_groups,
-                           expected_m);
-        return hipGetLastError();
+        // rows of tiles that read a group's weights: those a masked group is expected to have; contiguous groups of a block each
+        // on average (two to a group, and a group's tile rows are on different XCDs: 8 groups, 2048 rows 45.6 -> 50 us)
+        const int tile_rows = kGemmType == GemmType::GroupedMasked ? ceil_div(expected_m > 0 && expected_m < m ? expected_m : m, int(BLOCK_M))
+                                                                   : (m <= 128 * (long long)num_groups ? 1 : 1 << 30);
+        return pick_stream(tile_rows, uint64_t(num_groups) * n * k, [&](auto stream_weights) {
+            hipLaunchKernelGGL((fp8_gemm_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, int(kNumStages), decltype(stream_weights)::value>),
+                               dim3(grid), dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream,
+                               static_cast<const uint8_t*>(lhs), lhs_scales, static_cast<const uint8_t*>(rhs), rhs_scales,
+                               reinterpret_cast<__bf16*>(out), m, n, k, lhs_scales_stride_m, lhs_scales_stride_k, grouped_layout,
+                               lhs_scales_stride_g, int(slots), num_groups, expected_m);
+            return hipGetLastError();
+        });
         }
     }
 
@@ -1104,11 +1113,13 @@ public:
         const long long grid = (long long)sched.grid_size() * SPLIT_K;
         unsigned* counters = static_cast<unsigned*>(workspace);
         float* partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kSplitKCounterBytes);
-        hipLaunchKernelGGL((fp8_gemm_split_k_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, int(kNumStages), SPLIT_K>), dim3(int(grid)),
-                           dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream, static_cast<const uint8_t*>(lhs), lhs_scales,
-                           static_cast<const uint8_t*>(rhs), rhs_scales, reinterpret_cast<__bf16*>(out), m, n, k,
-                           lhs_scales_stride_m, lhs_scales_stride_k, partials, counters);
-        return hipGetLastError();
+        return pick_stream(sched.tiles_m, uint64_t(n) * k, [&](auto stream_weights) {
+            hipLaunchKernelGGL((fp8_gemm_split_k_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, int(kNumStages), SPLIT_K, decltype(stream_weights)::value>),
+                               dim3(int(grid)), dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream,
+                               static_cast<const uint8_t*>(lhs), lhs_scales, static_cast<const uint8_t*>(rhs), rhs_scales,
+                               reinterpret_cast<__bf16*>(out), m, n, k, lhs_scales_stride_m, lhs_scales_stride_k, partials, counters);
+            return hipGetLastError();
+        });
     }
 
     // Same with explicit n and k, which must equal SHAPE_N / SHAPE_K unless those are 0 (sizes known at run time).
@@ -1135,11 +1146,25 @@ public:
             const int cus = device_cu_count() / kNumXCD * kNumXCD;
             grid = capped_grid(slots < cus ? slots : cus, num_sms, device_cu_count());
         }
-        hipLaunchKernelGGL((fp8_gemm_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, GemmType::Normal, int(kNumStages)>), dim3(grid),
-                           dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream, static_cast<const uint8_t*>(lhs), lhs_scales,
-                           static_cast<const uint8_t*>(rhs), rhs_scales, reinterpret_cast<__bf16*>(out), m, n, k,
-                           lhs_scales_stride_m, lhs_scales_stride_k, static_cast<const int*>(nullptr), 0, slots, 1, 0);
-        return hipGetLastError();
+        return pick_stream(sched.tiles_m, uint64_t(n) * k, [&](auto stream_weights) {
+            hipLaunchKernelGGL((fp8_gemm_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, GemmType::Normal, int(kNumStages), decltype(stream_weights)::value>),
+                               dim3(grid), dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream,
+                               static_cast<const uint8_t*>(lhs), lhs_scales, static_cast<const uint8_t*>(rhs), rhs_scales,
+                               reinterpret_cast<__bf16*>(out), m, n, k, lhs_scales_stride_m, lhs_scales_stride_k,
+                               static_cast<const int*>(nullptr), 0, slots, 1, 0);
+            return hipGetLastError();
+        });
+    }
+
+private:
+    // Calls `launch` with std::true_type where the weights are streamed (ring tiles only), else std::false_type. Sizes that are known
+    // when the kernel is compiled and never stream leave out the kernel that does.
+    template <typename Launch>
+    static hipError_t pick_stream(int tile_rows, uint64_t weight_bytes, Launch&& launch) {
+        constexpr uint64_t KNOWN = uint64_t(SHAPE_N) * SHAPE_K * kNumGroups;
+        if constexpr (kNumStages > 2 && (KNOWN == 0 || (kGemmType != GemmType::Normal && kNumGroups == 1) || streams_weights(1, KNOWN)))
+            if (streams_weights(tile_rows, weight_bytes)) return launch(std::true_type{});
+        return launch(std::false_type{});
     }
 };
 

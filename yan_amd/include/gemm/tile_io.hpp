@@ -73,7 +73,9 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_out_rsrc(const void* orig
 // Per-thread state for staging a ROWS x 128-byte tile with NUM_WAVES waves: one VGPR. Everything that varies
 // per pass or per k-tile is wave-uniform and rides in the instruction's scalar offset, which the hardware adds
 // before its bounds check; a row past the end of the matrix lands at or beyond num_records and reads as zero.
-template <int ROWS, int NUM_WAVES>
+// STREAM: the copies carry the non-temporal hint (streams_weights in scheduler.hpp).
+constexpr int kNonTemporal = 2;         // cache-policy bit of gfx950 buffer instructions
+template <int ROWS, int NUM_WAVES, bool STREAM = false>
 struct TileStager {
     static_assert(ROWS % 16 == 0 && NUM_WAVES % 2 == 0);
     static constexpr int GROUPS = ROWS / 8;                       // 8-row groups, one instruction each
@@ -116,7 +118,7 @@ struct TileStager {
         const int q = j * NUM_WAVES + wave;
         const uint32_t past_tile = (GROUPS % NUM_WAVES == 0 || q < GROUPS) ? 0u : kOutOfRange;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, YAN_LDS_PTR(lds_tile + q * 8 * kRowBytes), kChunk, lane_voff | past_tile,
-                                                 k_byte0 + j * pass_pitch, 0, 0);
+                                                 k_byte0 + j * pass_pitch, 0, STREAM ? kNonTemporal : 0);
     }
 
     __device__ __forceinline__ void issue_from(__amdgpu_buffer_rsrc_t rsrc, uint8_t* lds_tile, int k_byte0, int wave,
@@ -126,7 +128,7 @@ struct TileStager {
             const int q = j * NUM_WAVES + wave;
             const uint32_t past_tile = (GROUPS % NUM_WAVES == 0 || q < GROUPS) ? 0u : kOutOfRange;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, YAN_LDS_PTR(lds_tile + q * 8 * kRowBytes), kChunk,
-                                                     lane_voff | past_tile, k_byte0 + j * pass_pitch, 0, 0);
+                                                     lane_voff | past_tile, k_byte0 + j * pass_pitch, 0, STREAM ? kNonTemporal : 0);
         }
     }
 };
