@@ -295,7 +295,10 @@ GROUPED_ROWS_ON_DEVICE_CASES = [((512,) * 6, 768, 512, 0), ((384, 640) * 3, 768,
 # 64 blocks a wave looks at at once and one that starts right behind it, padding inside, in front of and behind groups, a group of
 # one block, one k-tile (no second one to fetch), an odd number of them, outputs that are no multiple of 8.
 GROUPED_FOLLOW_GROUPS_CASES = [((63 * 128, 3 * 128, 1, 2 * 128), 264, 128, 0), ((-128, 100, -256, 5 * 128, 385, -128, 128), 520, 384, 1),
-                               ((128,) * 5, 1028, 640, 0), ((64 * 128, 65 * 128), 12, 256, 2), ((128,), 256, 128, 0)]
+                               ((128,) * 5, 1028, 640, 0), ((64 * 128, 65 * 128), 12, 256, 2), ((128,), 256, 128, 0),
+                               # tall rows that run as two flat ones each on eight compute units: two of ten, one of nine behind two flat
+                               # ones, one of five with two tiles each, the last of which ends inside a block
+                               ((20 * 128,), 12, 256, 0), ((11 * 128, 9 * 128), 12, 384, 1), ((10 * 128 - 50,), 260, 128, 0)]
 # (BLOCK_N, NUM_STAGES) that go with BLOCK_M = 256 in the keys of a contiguous call: the widths of the cost table, the other ones the
 # tiles support, with and without a ring and a 128-row tile beside them
 GROUPED_256_ROW_KEYS = [(256, 2), (224, 2), (192, 2), (160, 2), (128, 3), (128, 2), (96, 2), (32, 2)]

@@ -26,7 +26,7 @@
     } while (0)
 
 int main() {
-    int cases = 0, region_cases = 0;
+    int cases = 0, region_cases = 0, halved_cases = 0;
     const int blocks[][2] = {{256, 256}, {128, 256}, {64, 16}, {256, 224}};
     for (const auto& blk : blocks) {
         const int bm = blk[0], bn = blk[1];
@@ -124,7 +124,7 @@ int main() {
     unsigned rng = 1;
     auto random = [&](int below) { rng = rng * 1664525u + 1013904223u; return int((rng >> 8) % unsigned(below)); };
     for (int trial = 0; trial < 400; ++trial) {
-        const int bm = 256, bn = trial % 2 ? 256 : 128, tn = 1 + random(20), n = (tn - 1) * bn + 4 + random(bn - 4);
+        const int bm = 256, bn = (trial / 4) % 2 ? 256 : 128, tn = 1 + random(20), n = (tn - 1) * bn + 4 + random(bn - 4);
         std::vector<int> group_of;
         const int blocks = 1 + random(200), longest = trial % 3 == 0 ? 70 : (trial % 3 == 1 ? 4 : 1);
         for (int g = 0; int(group_of.size()) < blocks;) {
@@ -157,6 +157,16 @@ int main() {
         }
         for (int b = 0; b < blocks; ++b) CHECK(covered[b] == (group_of[b] >= 0 ? 1 : 0));
         const long long launched = (long long)yan::XcdTileScheduler<>(m, n, 128, bn).grid_size() + yan::kNumXCD;
+        const int cus[] = {1 << 30, 8, 40, 256};          // 2^30: no tall row ever runs flat
+        const int halved = yan::tall_rows_run_flat(tall_rows, flat_rows, tn, cus[trial % 4]);
+        CHECK(halved >= 0 && halved <= tall_rows && (trial % 4 != 0 || halved == 0));
+        if (halved) {        // whole rounds of tall tiles and less than a row, then all the rest at one time
+            const int rest = (tall_rows - halved) * tn % cus[trial % 4];
+            CHECK(rest < tn && rest + (flat_rows + 2 * halved) * tn <= cus[trial % 4]);
+            ++halved_cases;
+        }
+        tall_rows -= halved;
+        flat_rows += 2 * halved;
         yan::XcdTileScheduler<> tall(tall_rows * 256, n, 256, bn), flat(flat_rows * 128, n, 128, bn);
         tall.fit_bands_to_groups(tall_rows / 3);
         flat.fit_bands_to_groups(1);
@@ -183,7 +193,7 @@ int main() {
         CHECK(b.region_rows == 16 && c.region_rows == 32);
         CHECK(d.region_rows == 0);                           // 2 x 128 MiB of operands fit
         CHECK(e.region_rows == 32 && e.rows_outer);          // the FP8 16384^3 shape
-        CHECK(region_cases > 100);
+        CHECK(region_cases > 100 && halved_cases > 10);
     }
     std::printf("ok %d\n", cases);
     return 0;

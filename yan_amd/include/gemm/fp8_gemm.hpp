@@ -904,8 +904,10 @@ fp8_gemm_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_s
 // 256-row tiles a tile that holds two groups needs two passes over K, and so many did with groups of a few blocks that
 // 128-row tiles ran throughout: 48 blocks over 16 groups x 4096 x 7168 219 -> 216 us by following the groups, 197 with the third
 // weight stage the tall tiles have room for (kDeepB); 10240 rows in 4 groups 290 -> 276 us, 8320 in 64 x 7168 x 2048 185 -> 172.
-// Mixing flat and tall tiles in the order of the groups (every weight panel then read at one time) measured the same, and
-// running tall rows flat where the tall tiles end in a round that is mostly empty gains 2-4 % there and loses 1 % elsewhere.
+// Mixing flat and tall tiles in the order of the groups (every weight panel then read at one time) measured the same.
+// Where the tall tiles end in a round with room for it, the tall rows of that round run as two flat ones each (tall_rows_run_flat in
+// scheduler.hpp): a workgroup alone on its compute unit takes 85-89 us for a tall tile of K = 7168 and 61-73 for a flat one. 48 blocks
+// over 16 groups 195 -> 186, over 8 groups 183 -> 175, 10240 rows in 6 groups x 4096 x 5120 214 -> 206; no change elsewhere.
 // STAGES belongs to the tall tile: 2, or a ring as everywhere else (256 x 128). The flat tile runs the deepest ring it has. Where
 // it has none, or runs on another number of waves (256 x 160 and the other widths no plan takes), the odd block is a tall
 // tile whose rows end with the block.
@@ -916,7 +918,7 @@ __global__ void __launch_bounds__((fp8_launch_waves(256, BLOCK_N, STAGES) * kWav
 fp8_gemm_contiguous_rows_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_scales,
                                 const uint8_t* __restrict__ rhs, const float* __restrict__ rhs_scales,
                                 __bf16* __restrict__ out, int m, int n_rt, int k_rt, int sa_stride_m, int sa_stride_k,
-                                const int* __restrict__ grouped_layout, int num_groups) {
+                                const int* __restrict__ grouped_layout, int num_groups, int compute_units) {
     using Tall = Fp8TileConfig<256, BLOCK_N>;
     using Flat = Fp8TileConfig<128, BLOCK_N>;
     constexpr int FLAT_STAGES = Flat::MAX_RING_STAGES;
@@ -939,6 +941,10 @@ fp8_gemm_contiguous_rows_kernel(const uint8_t* __restrict__ lhs, const float* __
         tall_rows += __popcll(starts.tall);
         flat_rows += __popcll(starts.flat);
     }
+    // the last tall rows run as two flat ones each, numbered behind those that are flat by themselves
+    const int odd_rows = flat_rows, halved = HAS_FLAT ? tall_rows_run_flat(tall_rows, flat_rows, tiles_n, compute_units) : 0;
+    tall_rows -= halved;
+    flat_rows += 2 * halved;
     XcdTileScheduler<> tall(tall_rows * 256, N, 256, BLOCK_N), flat(flat_rows * 128, N, 128, BLOCK_N);
     tall.fit_bands_to_groups(tall_rows / max(num_groups, 1));
     flat.fit_bands_to_groups(1);
@@ -948,7 +954,10 @@ fp8_gemm_contiguous_rows_kernel(const uint8_t* __restrict__ lhs, const float* __
         const bool is_tall = slot < tall_slots;
         const TileCoord t = is_tall ? tall.dealt_band_tile_of(slot) : flat.dealt_band_tile_of(slot - tall_slots);
         if (!t.valid) return;
-        const int block = contiguous_block_at(grouped_layout, blocks, is_tall, t.m_idx, lane), tile = block * tiles_n + t.n_idx;
+        const int half = is_tall ? -1 : t.m_idx - odd_rows;          // 0 and up: a half of a tall row
+        const int block = contiguous_block_at(grouped_layout, blocks, is_tall || half >= 0, half >= 0 ? tall_rows + half / 2 : t.m_idx, lane) +
+                          (half >= 0 ? half % 2 : 0);
+        const int tile = block * tiles_n + t.n_idx;
         if (is_tall || !HAS_FLAT) {
             const int rows_end = HAS_FLAT || is_tall ? m : min(m, (block + 1) * 128);
             fp8_gemm_tile<SHAPE_N, SHAPE_K, 256, BLOCK_N, GemmType::GroupedContiguous, STAGES, 1, TALL_RING, true>(
@@ -1078,10 +1087,11 @@ public:
         // tall and flat tiles, each rounded up to the 8 XCDs: at most the tiles of the 128-row tiling + 8
         const long long slots = (long long)XcdTileScheduler<>(m, n, 128, BLOCK_N).grid_size() + kNumXCD;
         if (slots >= kOutOfRange) return hipErrorInvalidValue;
-        const int grid = capped_grid(int(slots), num_sms, device_cu_count());
+        const int cus = device_cu_count(), grid = capped_grid(int(slots), num_sms, cus);
         hipLaunchKernelGGL((fp8_gemm_contiguous_rows_kernel<SHAPE_N, SHAPE_K, BLOCK_N, int(kNumStages)>), dim3(grid),
                            dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream, static_cast<const uint8_t*>(lhs), lhs_scales, static_cast<const uint8_t*>(rhs), rhs_scales,
-                           reinterpret_cast<__bf16*>(out), m, n, k, lhs_scales_stride_m, lhs_scales_stride_k, grouped_layout, num_groups);
+                           reinterpret_cast<__bf16*>(out), m, n, k, lhs_scales_stride_m, lhs_scales_stride_k, grouped_layout, num_groups,
+                           grid < cus ? grid : cus);
         return hipGetLastError();
     }
 
