@@ -357,6 +357,21 @@ def stream_plans(kind: str, tile, split_k: int, n: int):
     return name, keys, arg_defs, includes, template
 
 
+# Activation scales in every strided layout a call takes, on tiles that copy row-major ones four k-tiles at a time: (tile, parts of
+# K), rows, columns, depths with four k-tiles and more, and one whose rows of scales are no whole 16-byte pieces
+SCALE_LAYOUT_TILES = [((128, 256), 1), ((128, 128), 1), ((64, 128), 1), ((64, 64), 4), ((256, 128), 1), ((32, 32), 1)]
+SCALE_LAYOUT_SIZES = (333, 388, (512, 3584, 1664))
+
+
+def strided_tile_plan(tile, split_k: int, n: int, k: int):
+    """(name, keys, arg_defs, template) of the FP8 JIT kernel with this tile and factor for activation scales of any strides."""
+    from yan_amd.jit_kernels import gemm
+    name, keys, _, _ = fp8_explicit_tile_plan(*tile, n, k)
+    if split_k > 1:
+        return name + '_split_k_strided', {**keys, 'SPLIT_K': split_k}, gemm.split_k_strided_arg_defs, gemm.split_k_strided_template
+    return name + '_strided', keys, gemm.strided_arg_defs, gemm.strided_template
+
+
 def dense_tile_plan(tile, dtype: torch.dtype, cap: int):
     """(name, keys, arg_defs, includes, template) of the dense GEMM on a tile given outright."""
     from yan_amd.jit_kernels import bf16_gemm, heuristics
@@ -507,6 +522,10 @@ def jit_kernels_in_use(num_cus: int = 256):
     for tile, depths in FP8_SHORT_K_TILES:
         for k in depths:
             name, keys, arg_defs, code_template = fp8_explicit_tile_plan(*tile, FP8_SHORT_K_SIZES[1], k)
+            add(name, arg_defs, gemm.includes, code_template, keys)
+    for tile, split_k in SCALE_LAYOUT_TILES:
+        for k in SCALE_LAYOUT_SIZES[2]:
+            name, keys, arg_defs, code_template = strided_tile_plan(tile, split_k, SCALE_LAYOUT_SIZES[1], k)
             add(name, arg_defs, gemm.includes, code_template, keys)
     for tile, split_k in STREAM_FP8_CASES:
         for n in (STREAM_FP8_SIZES[1], STREAM_FP8_SIZES[1] // 2):

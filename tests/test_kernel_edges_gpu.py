@@ -252,3 +252,64 @@ def test_streamed_weights_of_groups_give_the_same_bits(masked):
         torch.cuda.synchronize()
         return part
     assert torch.equal(run(0, n), torch.cat([run(0, n // 2), run(n // 2, n)], dim=-1))
+
+
+def _scale_layouts(scales):
+    """The values of `scales` [..., rows, k/128] in the layouts a caller may hand over."""
+    *lead, rows, blocks = scales.shape
+
+    def row_pitch(extra, offset):
+        buf = torch.full((*lead, rows, blocks + extra), float('nan'), device=scales.device).flatten()
+        buf = torch.cat([torch.full((offset, ), float('nan'), device=scales.device), buf])[offset:].view(*lead, rows, blocks + extra)
+        return buf[..., :blocks].copy_(scales)
+    return {'row-major': scales.contiguous(), 'four apart': row_pitch(4, 0), 'one apart': row_pitch(1, 0), 'base off by one': row_pitch(0, 1),
+            'base off by four': row_pitch(0, 4), 'every other': torch.stack([scales, scales], dim=-1).flatten(-2)[..., ::2]}
+
+
+@pytest.mark.parametrize('tile,split_k,k', [(*t, k) for t in testing.SCALE_LAYOUT_TILES for k in testing.SCALE_LAYOUT_SIZES[2]])
+def test_activation_scales_of_any_layout_give_the_same_bits(tile, split_k, k):
+    from yan_amd.jit_kernels import gemm
+    m, n, _ = testing.SCALE_LAYOUT_SIZES
+    _announce('scale layouts', tile, split_k, k)
+    (a8, sa), (b8, sb), out = testing.make_fp8_case(m, n, k, seed=19, device='cuda')
+    name, keys, arg_defs, code_template = testing.strided_tile_plan(tile, split_k, n, k)
+    kernel = jit.build(name, arg_defs, jit.generate(gemm.includes, arg_defs, jit.cpp_format(code_template, keys)))
+    workspace = torch.zeros(16384 + 256 * 128 * 128 * 4, dtype=torch.uint8, device='cuda')
+
+    def run(scales, cap=0):
+        got = torch.full_like(out, float('nan'))
+        split = (workspace, workspace.numel()) if split_k > 1 else ()
+        assert kernel(a8, scales, b8, sb, got, m, torch.cuda.current_stream(), cap, 0, *split, *scales.stride()) == 0
+        torch.cuda.synchronize()
+        return got
+    expected = run(yan.get_col_major_tensor(sa))
+    ref = torch.from_numpy(oracle.gemm_fp8_block_scaled_ref(_codes(a8), sa.cpu().numpy(), _codes(b8), sb.cpu().numpy()))
+    assert _fp8_close(expected.cpu().float(), ref)
+    for layout, scales in _scale_layouts(sa).items():
+        assert torch.equal(scales, sa), layout
+        assert torch.equal(run(scales), expected), layout
+    assert torch.equal(run(sa, 8), expected)
+    same = sa[:1].expand(m, -1)
+    assert torch.equal(run(same), run(yan.get_col_major_tensor(same.contiguous())))
+
+
+@pytest.mark.parametrize('masked', [False, True])
+def test_activation_scales_of_groups_of_any_layout_give_the_same_bits(masked):
+    groups, rows, n, k = testing.STREAM_GROUPED_SIZES
+    _announce('scale layouts of groups', masked)
+    if masked:
+        (a, sa), rhs, out, layout = testing.make_grouped_masked_case(groups, rows, n, k, (5, 64, 0, 1, 33, 64, 2, 17), seed=20, device='cuda')
+    else:
+        (a, sa), rhs, out, layout = testing.make_grouped_contiguous_case((128, 7, 100, 1, 128, 64, 2, 90), n, k, seed=20, device='cuda')
+
+    def run(scales):
+        got = torch.full_like(out, -7.0)
+        if masked:
+            yan.m_grouped_gemm_fp8_fp8_bf16_nt_masked((a, scales), rhs, got, layout, rows)
+        else:
+            yan.m_grouped_gemm_fp8_fp8_bf16_nt_contiguous((a, scales), rhs, got, layout)
+        torch.cuda.synchronize()
+        return got
+    expected = run(yan.get_col_major_tensor(sa))
+    for name, scales in _scale_layouts(sa).items():
+        assert torch.equal(run(scales), expected), name

@@ -78,6 +78,11 @@ struct Fp8TileConfig {
     static constexpr int  RING_SCALE_BYTES = ceil_div(BLOCK_M * 4, 1024) * 1024;
     static constexpr int  RING_STAGE_BYTES = (LDS_ROWS_A + LDS_ROWS_B) * kRowBytes + RING_SCALE_BYTES;
     static constexpr bool RING_CAPABLE = BLOCK_M % 32 == 0 && (BLOCK_M / 8) % NUM_WAVES == 0 && BLOCK_N % 16 == 0;
+    // Behind the stages: room for activation scales that come four k-tiles at a time (fp8_quad_scales), 16 bytes a row; a slot is taken again when every k-tile of its four has been consumed, with STAGES - 1 k-tiles in flight. Then
+    // 1 KB that takes what copies of nothing write.
+    static constexpr int  SCALE_PARTS = ceil_div(BLOCK_M, 64);
+    __host__ __device__ static constexpr int quad_slots(int stages) { return (stages + 6) / 4; }
+    __host__ __device__ static constexpr int ring_bytes(int stages, bool quad) { return stages * RING_STAGE_BYTES + ((quad ? quad_slots(stages) * SCALE_PARTS : 0) + 1) * 1024; }
     // At most 8 stages, 12 for the narrow tiles of the decode shapes (16 or 32 weight rows per workgroup): those have next
     // to nothing to compute per k-tile and run at the rate their compute unit takes bytes in, which needs many k-tiles in
     // flight (a stage is only 9 to 13 KB there). Measured with every unit pulling: about 60 GB/s per unit whatever the
@@ -271,13 +276,14 @@ contiguous_block_at(const int* __restrict__ grouped_layout, int blocks, bool tal
 // STAGES: 2 = two LDS stages with the next k-tile's scales in registers; 3.. = a ring of that many stages.
 // One output tile (one slot of the launch: `bid` is what blockIdx.x would be with a workgroup per slot).
 // EXTERNAL_RING: the ring of a tile with STAGES > 2 lives in `ring_lds` (LDS the caller declared, 1024-byte aligned, at least
-// STAGES * Fp8TileConfig::RING_STAGE_BYTES) instead of an array of this function's own: for kernels that hold two kinds of
+// Fp8TileConfig::ring_bytes(STAGES, QUAD)) instead of an array of this function's own: for kernels that hold two kinds of
 // tile and run one of them (fp8_gemm_contiguous_rows_kernel).
 // EXPLICIT_TILE: `bid` names the tile itself, as (its first row / 128) * tiles_n + n_idx, for callers that order the tiles
 // themselves; in the contiguous layout all rows of such a tile belong to the group of its first row.
 // STREAM: a ring tile's copies of the weights carry the non-temporal hint (streams_weights in scheduler.hpp).
+// QUAD: a ring tile copies its activation scales four k-tiles at a time (fp8_quad_scales).
 template <int SHAPE_N, int SHAPE_K, int BLOCK_M, int BLOCK_N, GemmType kGemmType, int STAGES, int SPLIT_K = 1, bool EXTERNAL_RING = false,
-          bool EXPLICIT_TILE = false, bool STREAM = false>
+          bool EXPLICIT_TILE = false, bool STREAM = false, bool QUAD = false>
 __device__ __forceinline__ void
 fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_scales,
               const uint8_t* __restrict__ rhs, const float* __restrict__ rhs_scales,
@@ -472,38 +478,33 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     // Ring of STAGES stages, STAGES - 1 k-tiles in flight: what a small tile needs when the problem is bound by
     // streaming its operands and one k-tile of prefetch cannot cover the memory latency. Every wave issues the same
     // number of copies for every k-tile (OPS), in the same order, so "k-tile kb has landed" is "at most
-    // (STAGES - 2) * OPS of my copies are outstanding". The activation scales of a k-tile travel through the stage as well (a register load between the
-    // copies would make the in-order counter wait for every older copy): every wave copies one 64-row part of them
-    // with one full-width instruction; waves that share a part write the same bytes twice.
+    // (STAGES - 2) * OPS of my copies are outstanding". The activation scales of a k-tile travel through LDS as well (a register
+    // load between the copies would make the in-order counter wait for every older copy): the first waves copy a 64-row part of
+    // them each, and the others nothing, with the same number of instructions. Row-major scales are a cache line a row and k-tile,
+    // four k-tiles of them with QUAD. Every wave copying a part, as before, 512 x 7168 x 7168 took 65.7 us with row-major scales and
+    // 38 with token-contiguous ones; one wave a part 47, four k-tiles at a time 40
+    // (1500 x 4096 x 4096 43.2 -> 35.8, 640 x 9216 x 4096 47.3 -> 36.1; K no multiple of 512: 900 x 4096 x 7040 53.7 -> 43.3). The scales go first
+    // in a k-tile, before its MFMAs: among them they cost 512 x 7168 x 7168 with token-contiguous scales 39.1 us, 36.8 now.
     constexpr int STAGE_BYTES = Cfg::RING_STAGE_BYTES, A_BYTES = Cfg::LDS_ROWS_A * kRowBytes, TILE_BYTES = A_BYTES + Cfg::LDS_ROWS_B * kRowBytes;
-    constexpr int OPS = StA::PASSES + StB::PASSES + 1, SCALE_PARTS = BLOCK_M >= 64 ? BLOCK_M / 64 : 1;
-    static_assert(Cfg::RING_CAPABLE && (fp8_ring_group(BLOCK_M, BLOCK_N, STAGES) > 1 || (STAGES - 2) * OPS <= 63) && STAGES * STAGE_BYTES <= 160 * 1024);
+    constexpr int G = fp8_ring_group(BLOCK_M, BLOCK_N, STAGES);
+    constexpr int OPS = NUM_COPIES + 1, SCALE_PARTS = Cfg::SCALE_PARTS;
+    constexpr int RING_BYTES = G > 1 ? STAGES * STAGE_BYTES : Cfg::ring_bytes(STAGES, QUAD);
+    static_assert(Cfg::RING_CAPABLE && (G > 1 || (STAGES - 2) * OPS <= 63) && SCALE_PARTS <= NW && RING_BYTES <= 160 * 1024);
     uint8_t* ring = ring_lds;
     if constexpr (!EXTERNAL_RING) {
-        __shared__ __attribute__((aligned(1024))) uint8_t own_ring[STAGES * STAGE_BYTES];
+        __shared__ __attribute__((aligned(1024))) uint8_t own_ring[RING_BYTES];
         ring = own_ring;
     }
     const uint32_t scale_voff = uint32_t(m0 + lane) * sa_stride_m * 4;
-    auto issue_op = [&](int d, int kb, uint8_t* stage) {
-        const bool live = kb < kb_hi;
-        if (d < StA::PASSES) stage_a.issue_pass(live ? rsrc_a : rsrc_none, stage, kb * kRowBytes, wave, d);
-        else if (d < StA::PASSES + StB::PASSES) stage_b.issue_pass(live ? rsrc_b : rsrc_none, stage + A_BYTES, kb * kRowBytes, wave, d - StA::PASSES);
-        else {
-            const int part = wave % SCALE_PARTS;                    // rows m0 + 64 * part + lane
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_sa : rsrc_none, YAN_LDS_PTR(stage + TILE_BYTES + part * 256), 4,
-                                                     scale_voff, (kb * sa_stride_k + part * 64 * sa_stride_m) * 4, 0, 0);
-        }
-    };
     // Tiles of one or two atoms per wave (the decode shapes: 16 or 32 weight rows per workgroup) have almost nothing to
     // compute per k-tile, and a loop that meets at a barrier for every k-tile is bound by that chain of waits: barrier,
     // fragment reads, one MFMA, its fold, 56 times over. They consume the ring G k-tiles at a time instead: one
     // barrier, the fragments of G k-tiles, G independent MFMAs, G folds; the copies of the G k-tiles that go where the
     // previous group was start right after the barrier, so STAGES - 2G to STAGES - G k-tiles are in flight.
-    constexpr int G = fp8_ring_group(BLOCK_M, BLOCK_N, STAGES);
     if constexpr (G > 1) {
     // Eight waves share the copies of a k-tile: operation o = slot * 8 + wave is the o-th 8-row group of the stage
-    // (activation rows first, then weight rows: the two tiles lie back to back) or, past the last group, the copy of
-    // the activation scales (which several waves may repeat: same bytes).
+    // (activation rows first, then weight rows: the two tiles lie back to back) or, behind the last group, the copy of
+    // the activation scales; further operations copy nothing, behind those.
     constexpr int GA = BLOCK_M / 8, GROUPS_AB = (BLOCK_M + BLOCK_N) / 8, SLOTS = ceil_div(GROUPS_AB + 1, LW);
     static_assert(LW == 8 && NW == 4 && A_BYTES == GA * 8 * kRowBytes && TILE_BYTES == GROUPS_AB * 8 * kRowBytes && SCALE_PARTS == 1);
     static_assert(Cfg::UNIFORM_SCALE_B && NB == 1 && (STAGES - 2 * G) * SLOTS <= 63);
@@ -524,7 +525,7 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
             if (in_a) __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_a : rsrc_none, YAN_LDS_CAST(stage + o * 8 * kRowBytes), kChunk, slot_voff[sl], kb * kRowBytes, 0, 0);
             else __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_b : rsrc_none, YAN_LDS_CAST(stage + o * 8 * kRowBytes), kChunk, slot_voff[sl], kb * kRowBytes, 0, STREAM ? kNonTemporal : 0);
         } else {
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_sa : rsrc_none, YAN_LDS_CAST(stage + TILE_BYTES), 4, scale_voff, kb * sa_stride_k * 4, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(live && o == GROUPS_AB ? rsrc_sa : rsrc_none, YAN_LDS_CAST(stage + TILE_BYTES + (o == GROUPS_AB ? 0 : 256)), 4, scale_voff, kb * sa_stride_k * 4, 0, 0);
         }
     };
 #pragma unroll
@@ -585,10 +586,32 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     epi_a = ring + (base == 0 ? STAGES - G : base - G) * STAGE_BYTES;
     epi_b = epi_a + A_BYTES;
     } else {
+    auto issue_copy = [&](int d, int kb, uint8_t* stage) {
+        const bool live = kb < kb_hi;
+        if (d < StA::PASSES) stage_a.issue_pass(live ? rsrc_a : rsrc_none, stage, kb * kRowBytes, wave, d);
+        else stage_b.issue_pass(live ? rsrc_b : rsrc_none, stage + A_BYTES, kb * kRowBytes, wave, d - StA::PASSES);
+    };
+    // QUAD: four k-tiles of a row at a time into a slot behind the stages
+    uint8_t* const quads = ring + STAGES * STAGE_BYTES;
+    uint8_t* const nowhere = quads + (QUAD ? Cfg::quad_slots(STAGES) * SCALE_PARTS * 1024 : 0);
+    auto quad_of = [&](int kb) { return quads + (kb / 4 % Cfg::quad_slots(STAGES)) * (SCALE_PARTS * 1024); };
+    auto issue_scales = [&](int kb, uint8_t* stage) {
+        const bool mine = kb < kb_hi && wave < SCALE_PARTS;         // rows m0 + 64 * wave + lane
+        if constexpr (QUAD) {
+            const bool now = mine && (kb % 4 == 0 || kb == kb_lo);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(now ? rsrc_sa : rsrc_none, YAN_LDS_PTR(now ? quad_of(kb) + wave * 1024 : nowhere), 16,
+                                                     scale_voff, (kb / 4 * 4 + wave * 64 * sa_stride_m) * 4, 0, 0);
+        } else {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(mine ? rsrc_sa : rsrc_none, YAN_LDS_PTR(mine ? stage + TILE_BYTES + wave * 256 : nowhere), 4,
+                                                     scale_voff, (kb * sa_stride_k + wave * 64 * sa_stride_m) * 4, 0, 0);
+        }
+    };
 #pragma unroll
-    for (int t = 0; t < STAGES - 1; ++t)
+    for (int t = 0; t < STAGES - 1; ++t) {
+        issue_scales(kb_lo + t, ring + t * STAGE_BYTES);
 #pragma unroll
-        for (int d = 0; d < OPS; ++d) issue_op(d, kb_lo + t, ring + t * STAGE_BYTES);
+        for (int d = 0; d < NUM_COPIES; ++d) issue_copy(d, kb_lo + t, ring + t * STAGE_BYTES);
+    }
     load_weight_scales(min(kb_lo, NUM_K_BLOCKS - 1));
     int st = 0;
     auto ring_step = [&](int kb) {
@@ -602,13 +625,15 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
         const uint8_t* cur = ring + st * STAGE_BYTES;
         const int st_nxt = st + STAGES - 1 >= STAGES ? st - 1 : st + STAGES - 1;
         uint8_t* nxt = ring + st_nxt * STAGE_BYTES;
-        const float* my_scales = reinterpret_cast<const float*>(cur + TILE_BYTES) + wm * Cfg::WTM + col;
+        issue_scales(kb + STAGES - 1, nxt);
+        const uint8_t* scales = QUAD ? quad_of(kb) + kb % 4 * 4 : cur + TILE_BYTES;
+        constexpr int scale_pitch = QUAD ? 16 : 4;
 #pragma unroll
-        for (int j = 0; j < TM; ++j) sa_cur[j] = my_scales[j * 16];
+        for (int j = 0; j < TM; ++j) sa_cur[j] = *reinterpret_cast<const float*>(scales + (wm * Cfg::WTM + col + j * 16) * scale_pitch);
         compute_tile(cur, cur + A_BYTES, sa_cur, sb_cur, [&](int row) {
 #pragma unroll
-            for (int d = 0; d < OPS; ++d)
-                if (d * SPREAD_ROWS / OPS == row) issue_op(d, kb + STAGES - 1, nxt);
+            for (int d = 0; d < NUM_COPIES; ++d)
+                if (d * SPREAD_ROWS / NUM_COPIES == row) issue_copy(d, kb + STAGES - 1, nxt);
         });
         st = st + 1 == STAGES ? 0 : st + 1;
     };
@@ -664,6 +689,12 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
             if (!fp8_meet_partials<SPLIT_K, NW, TN, TM>(acc, partials, counters, tile_slot, split, wave, lane)) return;
         fp8_store_slab<Cfg, false>(acc, nullptr, rsrc_out, m_slab, n_slab, m0, n0, m, N, stream_out, lane);
     }
+}
+
+// Whether the activation scales are copied four k-tiles at a time: rows of whole 16-byte pieces, as row-major scales are where K is a
+// multiple of 512. A kernel of its own: the choice inside the k-loop cost the token-contiguous layout 2 to 5 %.
+inline bool fp8_quad_scales(const float* scales, int stride_m, int stride_k, int stride_g, int k) {
+    return stride_k == 1 && stride_m % 4 == 0 && stride_g % 4 == 0 && k % 512 == 0 && reinterpret_cast<uintptr_t>(scales) % 16 == 0;
 }
 
 // Whether a problem runs the persistent walk below: the plain GEMM on two LDS stages (three of the weights) with two k-tiles or more.
@@ -854,7 +885,8 @@ fp8_gemm_walk(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
 // units (the reference's persistent kernel under `num_sms`,
 // yan/include/gemm/fp8_gemm.cuh:40, scheduler.cuh:39-58). Between two tiles every wave must have left the epilogue of
 // the first (which reads the LDS stage the second one's first copies go into).
-template <int SHAPE_N, int SHAPE_K, int BLOCK_M, int BLOCK_N, GemmType kGemmType = GemmType::Normal, int STAGES = 2, bool STREAM = false>
+template <int SHAPE_N, int SHAPE_K, int BLOCK_M, int BLOCK_N, GemmType kGemmType = GemmType::Normal, int STAGES = 2, bool STREAM = false,
+          bool QUAD = false>
 __global__ void __launch_bounds__((fp8_launch_waves(BLOCK_M, BLOCK_N, STAGES) * kWaveSize))
 fp8_gemm_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_scales,
                 const uint8_t* __restrict__ rhs, const float* __restrict__ rhs_scales,
@@ -882,13 +914,13 @@ fp8_gemm_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_s
     // A workgroup per slot (no cap): the tile without a loop around it. Inside the loop below the same code runs 2 to 14 %
     // slower on the ring tiles even for a single trip (64 x 7168 x 2048 on 64 x 32 tiles: 6.0 against 5.2 us).
     if (int(gridDim.x) >= num_slots) {
-        fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, STAGES, 1, false, false, STREAM>(lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt,
+        fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, STAGES, 1, false, false, STREAM, QUAD>(lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt,
                                                                              sa_stride_m, sa_stride_k, grouped_layout, sa_stride_g,
                                                                              int(blockIdx.x), num_groups, expected_m, two_stages);
         return;
     }
     for (int slot = blockIdx.x; slot < num_slots; slot += gridDim.x) {
-        fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, STAGES, 1, false, false, STREAM>(lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt,
+        fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, STAGES, 1, false, false, STREAM, QUAD>(lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt,
                                                                              sa_stride_m, sa_stride_k, grouped_layout, sa_stride_g,
                                                                              slot, num_groups, expected_m, two_stages);
         if (slot + int(gridDim.x) < num_slots) __syncthreads();
@@ -924,8 +956,8 @@ fp8_gemm_contiguous_rows_kernel(const uint8_t* __restrict__ lhs, const float* __
     constexpr int FLAT_STAGES = Flat::MAX_RING_STAGES;
     constexpr bool HAS_FLAT = FLAT_STAGES >= 3 && fp8_launch_waves(128, BLOCK_N, FLAT_STAGES) == fp8_launch_waves(256, BLOCK_N, STAGES);
     constexpr bool TALL_RING = STAGES > 2;
-    constexpr int TALL_BYTES = TALL_RING ? STAGES * Tall::RING_STAGE_BYTES : Tall::LDS_BYTES + (Tall::DEEP_B_CAPABLE ? Tall::LDS_ROWS_B * kRowBytes : 0);
-    constexpr int FLAT_BYTES = HAS_FLAT ? FLAT_STAGES * Flat::RING_STAGE_BYTES : 0;
+    constexpr int TALL_BYTES = TALL_RING ? Tall::ring_bytes(STAGES, false) : Tall::LDS_BYTES + (Tall::DEEP_B_CAPABLE ? Tall::LDS_ROWS_B * kRowBytes : 0);
+    constexpr int FLAT_BYTES = HAS_FLAT ? Flat::ring_bytes(FLAT_STAGES, false) : 0;
     __shared__ __attribute__((aligned(1024))) uint8_t pool[TALL_BYTES > FLAT_BYTES ? TALL_BYTES : FLAT_BYTES];
     uint8_t* const a0 = pool;
     uint8_t* const b0 = a0 + Tall::LDS_ROWS_A * kRowBytes;
@@ -989,13 +1021,13 @@ fp8_gemm_contiguous_rows_kernel(const uint8_t* __restrict__ lhs, const float* __
 }
 
 // The same tiles with K split SPLIT_K ways: launch slot s is part s % SPLIT_K of tile slot s / SPLIT_K.
-template <int SHAPE_N, int SHAPE_K, int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K, bool STREAM = false>
+template <int SHAPE_N, int SHAPE_K, int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K, bool STREAM = false, bool QUAD = false>
 __global__ void __launch_bounds__((fp8_launch_waves(BLOCK_M, BLOCK_N, STAGES) * kWaveSize))
 fp8_gemm_split_k_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_scales,
                         const uint8_t* __restrict__ rhs, const float* __restrict__ rhs_scales,
                         __bf16* __restrict__ out, int m, int n_rt, int k_rt, int sa_stride_m, int sa_stride_k,
                         float* __restrict__ partials, unsigned* __restrict__ counters) {
-    fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, GemmType::Normal, STAGES, SPLIT_K, false, false, STREAM>(
+    fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, GemmType::Normal, STAGES, SPLIT_K, false, false, STREAM, QUAD>(
         lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt, sa_stride_m, sa_stride_k, nullptr, 0, int(blockIdx.x), 1, 0,
         Fp8TwoStages{}, partials, counters);
 }
@@ -1016,12 +1048,15 @@ class Gemm {
 public:
     // lhs [m, K] e4m3 row-major; lhs_scales fp32, element (i, kb) at i * stride_m + kb * stride_k;
     // rhs [N, K] e4m3 row-major; rhs_scales fp32 [ceil(N/128), K/128] row-major; out [m, N] bf16 row-major.
+    // The last argument: std::true_type where the scales have stride_m 1 whenever this is called, which leaves kernels for other
+    // layouts out.
+    template <typename TokenContiguous = std::false_type>
     static hipError_t run(__hip_bfloat16* out, const void* lhs, const float* lhs_scales, int lhs_scales_stride_m,
                           int lhs_scales_stride_k, const void* rhs, const float* rhs_scales, int m,
-                          hipStream_t stream, int num_sms, uint32_t smem_size) {
+                          hipStream_t stream, int num_sms, uint32_t smem_size, TokenContiguous token_contiguous = {}) {
         static_assert(kGemmType == GemmType::Normal, "grouped layouts go through run_grouped");
         return run_sized(out, lhs, lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k, rhs, rhs_scales, m,
-                         int(SHAPE_N), int(SHAPE_K), stream, num_sms, smem_size);
+                         int(SHAPE_N), int(SHAPE_K), stream, num_sms, smem_size, token_contiguous);
     }
 
     // Grouped layouts (see the kernel's comment). `m` is the total number of rows (contiguous) or the rows
@@ -1058,8 +1093,11 @@ public:
         // on average (two to a group, and a group's tile rows are on different XCDs: 8 groups, 2048 rows 45.6 -> 50 us)
         const int tile_rows = kGemmType == GemmType::GroupedMasked ? ceil_div(expected_m > 0 && expected_m < m ? expected_m : m, int(BLOCK_M))
                                                                    : (m <= 128 * (long long)num_groups ? 1 : 1 << 30);
-        return pick_stream(tile_rows, uint64_t(num_groups) * n * k, [&](auto stream_weights) {
-            hipLaunchKernelGGL((fp8_gemm_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, int(kNumStages), decltype(stream_weights)::value>),
+        const bool quad = fp8_quad_scales(lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k,
+                                          kGemmType == GemmType::GroupedMasked ? lhs_scales_stride_g : 0, k);
+        return pick_kernel<false>(tile_rows, uint64_t(num_groups) * n * k, quad, [&](auto stream_weights, auto quad_scales) {
+            hipLaunchKernelGGL((fp8_gemm_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, int(kNumStages), decltype(stream_weights)::value,
+                                                decltype(quad_scales)::value>),
                                dim3(grid), dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream,
                                static_cast<const uint8_t*>(lhs), lhs_scales, static_cast<const uint8_t*>(rhs), rhs_scales,
                                reinterpret_cast<__bf16*>(out), m, n, k, lhs_scales_stride_m, lhs_scales_stride_k, grouped_layout,
@@ -1104,10 +1142,11 @@ public:
         const XcdTileScheduler<> sched(m, n, BLOCK_M, BLOCK_N);
         return kSplitKCounterBytes + size_t(sched.grid_size()) * SPLIT_K * BLOCK_M * BLOCK_N * 4;
     }
-    template <int SPLIT_K>
+    // The last argument is that of run.
+    template <int SPLIT_K, typename TokenContiguous = std::false_type>
     static hipError_t run_split_k(__hip_bfloat16* out, const void* lhs, const float* lhs_scales, int lhs_scales_stride_m,
                                   int lhs_scales_stride_k, const void* rhs, const float* rhs_scales, int m, int n, int k,
-                                  hipStream_t stream, void* workspace, size_t workspace_bytes) {
+                                  hipStream_t stream, void* workspace, size_t workspace_bytes, TokenContiguous = {}) {
         static_assert(kGemmType == GemmType::Normal && SPLIT_K > 1);
         if (m == 0 || n == 0) return hipSuccess;
         if (m < 0 || n < 0 || k <= 0 || (n % 4) != 0 || (k % 128) != 0) return hipErrorInvalidValue;
@@ -1123,8 +1162,10 @@ public:
         const long long grid = (long long)sched.grid_size() * SPLIT_K;
         unsigned* counters = static_cast<unsigned*>(workspace);
         float* partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kSplitKCounterBytes);
-        return pick_stream(sched.tiles_m, uint64_t(n) * k, [&](auto stream_weights) {
-            hipLaunchKernelGGL((fp8_gemm_split_k_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, int(kNumStages), SPLIT_K, decltype(stream_weights)::value>),
+        const bool quad = fp8_quad_scales(lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k, 0, k);
+        return pick_kernel<TokenContiguous::value>(sched.tiles_m, uint64_t(n) * k, quad, [&](auto stream_weights, auto quad_scales) {
+            hipLaunchKernelGGL((fp8_gemm_split_k_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, int(kNumStages), SPLIT_K, decltype(stream_weights)::value,
+                                                        decltype(quad_scales)::value>),
                                dim3(int(grid)), dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream,
                                static_cast<const uint8_t*>(lhs), lhs_scales, static_cast<const uint8_t*>(rhs), rhs_scales,
                                reinterpret_cast<__bf16*>(out), m, n, k, lhs_scales_stride_m, lhs_scales_stride_k, partials, counters);
@@ -1133,9 +1174,10 @@ public:
     }
 
     // Same with explicit n and k, which must equal SHAPE_N / SHAPE_K unless those are 0 (sizes known at run time).
+    template <typename TokenContiguous = std::false_type>
     static hipError_t run_sized(__hip_bfloat16* out, const void* lhs, const float* lhs_scales, int lhs_scales_stride_m,
                                 int lhs_scales_stride_k, const void* rhs, const float* rhs_scales, int m, int n, int k,
-                                hipStream_t stream, int num_sms, uint32_t smem_size) {
+                                hipStream_t stream, int num_sms, uint32_t smem_size, TokenContiguous = {}) {
         (void)smem_size;
         if (m == 0 || n == 0) return hipSuccess;
         if (m < 0 || n < 0 || k <= 0 || (n % 4) != 0 || (k % 128) != 0) return hipErrorInvalidValue;
@@ -1156,8 +1198,10 @@ public:
             const int cus = device_cu_count() / kNumXCD * kNumXCD;
             grid = capped_grid(slots < cus ? slots : cus, num_sms, device_cu_count());
         }
-        return pick_stream(sched.tiles_m, uint64_t(n) * k, [&](auto stream_weights) {
-            hipLaunchKernelGGL((fp8_gemm_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, GemmType::Normal, int(kNumStages), decltype(stream_weights)::value>),
+        const bool quad = fp8_quad_scales(lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k, 0, k);
+        return pick_kernel<TokenContiguous::value>(sched.tiles_m, uint64_t(n) * k, quad, [&](auto stream_weights, auto quad_scales) {
+            hipLaunchKernelGGL((fp8_gemm_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, GemmType::Normal, int(kNumStages), decltype(stream_weights)::value,
+                                                decltype(quad_scales)::value>),
                                dim3(grid), dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream,
                                static_cast<const uint8_t*>(lhs), lhs_scales, static_cast<const uint8_t*>(rhs), rhs_scales,
                                reinterpret_cast<__bf16*>(out), m, n, k, lhs_scales_stride_m, lhs_scales_stride_k,
@@ -1167,14 +1211,24 @@ public:
     }
 
 private:
-    // Calls `launch` with std::true_type where the weights are streamed (ring tiles only), else std::false_type. Sizes that are known
-    // when the kernel is compiled and never stream leave out the kernel that does.
-    template <typename Launch>
-    static hipError_t pick_stream(int tile_rows, uint64_t weight_bytes, Launch&& launch) {
+    // Calls `launch` with two of std::true_type / std::false_type: whether the weights are streamed, and whether the scales are copied four
+    // k-tiles at a time (ring tiles that consume a k-tile per barrier). What the sizes or the caller's scale layout rule out when the
+    // kernel is compiled is left out.
+    template <bool TOKEN_CONTIGUOUS, typename Launch>
+    static hipError_t pick_kernel(int tile_rows, uint64_t weight_bytes, bool quad, Launch&& launch) {
         constexpr uint64_t KNOWN = uint64_t(SHAPE_N) * SHAPE_K * kNumGroups;
-        if constexpr (kNumStages > 2 && (KNOWN == 0 || (kGemmType != GemmType::Normal && kNumGroups == 1) || streams_weights(1, KNOWN)))
-            if (streams_weights(tile_rows, weight_bytes)) return launch(std::true_type{});
-        return launch(std::false_type{});
+        constexpr bool RING = kNumStages > 2;
+        constexpr bool MAY_STREAM = RING && (KNOWN == 0 || (kGemmType != GemmType::Normal && kNumGroups == 1) || streams_weights(1, KNOWN));
+        constexpr bool MAY_QUAD = RING && !TOKEN_CONTIGUOUS && SHAPE_K % 512 == 0 && fp8_ring_group(BLOCK_M, BLOCK_N, int(kNumStages)) == 1 &&
+                                  Fp8TileConfig<BLOCK_M, BLOCK_N>::ring_bytes(int(kNumStages), true) <= 160 * 1024;
+        auto with_scales = [&](auto stream_weights) {
+            if constexpr (MAY_QUAD)
+                if (quad) return launch(stream_weights, std::true_type{});
+            return launch(stream_weights, std::false_type{});
+        };
+        if constexpr (MAY_STREAM)
+            if (streams_weights(tile_rows, weight_bytes)) return with_scales(std::true_type{});
+        return with_scales(std::false_type{});
     }
 };
 

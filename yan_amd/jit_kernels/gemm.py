@@ -20,7 +20,7 @@ from .heuristics import (get_best_fp8_config, get_fp8_num_stages, get_fp8_tile_s
                          get_split_k_fp8_config, tuning_enabled)
 from .split_k import SPLIT_K_COUNTER_BYTES, SPLIT_K_WORKSPACE_BYTES, split_k_enabled, split_k_launch_failed, split_k_workspace
 from .tuner import FrozenKeys, jit_tuner
-from .utils import current_raw_stream, get_num_sms, ceil_div, get_col_major_tensor, scales_for_kernel
+from .utils import current_raw_stream, get_num_sms, ceil_div, get_col_major_tensor, scales_for_kernel, SCALE_RELAYOUT_MIN_FLOP
 
 # C++ code templates
 includes = ('"gemm/fp8_gemm.hpp"', '"gemm/fp8_gemm_skinny.hpp"')
@@ -39,6 +39,10 @@ constexpr auto kNumTMAMulticast = {NUM_TMA_MULTICAST};
 _token_contiguous_scales = """
 // Token-contiguous activation scales
 const int lhs_scales_stride_m = 1, lhs_scales_stride_k = m;
+constexpr std::true_type kTokenContiguous;
+"""
+_strided_scales = """
+constexpr std::false_type kTokenContiguous;
 """
 _tiled_launch = """
 // Make a templated GEMM
@@ -46,7 +50,7 @@ using GemmType = Gemm<N, K, BLOCK_M, BLOCK_N, 128, 1, kNumStages, kNumTMAMultica
 
 // Launch kernel
 __return_code = static_cast<int>(GemmType::run(out, lhs, lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k,
-                                               rhs, rhs_scales, m, stream, num_sms, smem_size));
+                                               rhs, rhs_scales, m, stream, num_sms, smem_size, kTokenContiguous));
 """
 # A handful of activation rows: BLOCK_M / 16 activation atoms and 16 weight rows per workgroup, the K blocks of a
 # workgroup shared out over NUM_WAVES waves; no LDS staging, NUM_STAGES is the per-wave load depth's name only.
@@ -64,7 +68,7 @@ using GemmType = Gemm<N, K, BLOCK_M, BLOCK_N, 128, 1, kNumStages, kNumTMAMultica
 
 // Launch kernel
 __return_code = static_cast<int>(GemmType::run_split_k<{SPLIT_K}>(out, lhs, lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k,
-                                                                  rhs, rhs_scales, m, N, K, stream, workspace, workspace_bytes));
+                                                                  rhs, rhs_scales, m, N, K, stream, workspace, workspace_bytes, kTokenContiguous));
 """
 
 # bf16 activations: the quantiser and the GEMM enqueued by one `launch` (gemm_bf16_fp8_bf16_nt below). The codes and their
@@ -92,13 +96,13 @@ arg_defs = (('lhs', torch.float8_e4m3fn), ('lhs_scales', torch.float),
             ('stream', torch.cuda.Stream), ('num_sms', int), ('smem_size', int))
 # Any other strided layout of the activation scales (row-major included) runs without a transposing copy: the same
 # kernels with the two strides, in elements, as two more run-time arguments.
-strided_template = _keys_block + _tiled_launch
+strided_template = _keys_block + _strided_scales + _tiled_launch
 strided_arg_defs = arg_defs + (('lhs_scales_stride_m', int), ('lhs_scales_stride_k', int))
 skinny_template = _keys_block + _token_contiguous_scales + _skinny_launch
 skinny_strided_template = _keys_block + _skinny_launch
 # Split-K kernels take their workspace as two more arguments (in front of the strides, when those are passed).
 split_k_template = _keys_block + _token_contiguous_scales + _split_k_launch
-split_k_strided_template = _keys_block + _split_k_launch
+split_k_strided_template = _keys_block + _strided_scales + _split_k_launch
 split_k_arg_defs = arg_defs + (('workspace', torch.uint8), ('workspace_bytes', int))
 split_k_strided_arg_defs = split_k_arg_defs + (('lhs_scales_stride_m', int), ('lhs_scales_stride_k', int))
 
@@ -180,7 +184,9 @@ def gemm_fp8_fp8_bf16_nt(lhs: Tuple[torch.Tensor, torch.Tensor],
         return
 
     num_sms = get_num_sms()
-    lhs_scales = scales_for_kernel(lhs_scales, 2.0 * m * n * k)
+    flop = 2.0 * m * n * k
+    if flop >= SCALE_RELAYOUT_MIN_FLOP:
+        lhs_scales = scales_for_kernel(lhs_scales, flop, fp8_kernel_plan(m, n, k, num_sms)[1])
     stride_m, stride_k = lhs_scales.stride()
     token_contiguous = (m == 1 or stride_m == 1) and (lhs_scales.size(1) == 1 or stride_k == m)
     name, keys, defs, smem_size, code_template = fp8_kernel_plan(m, n, k, num_sms, token_contiguous)

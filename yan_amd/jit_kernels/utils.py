@@ -88,20 +88,27 @@ def get_col_major_tensor(x: torch.Tensor) -> torch.Tensor:
 
 
 # From this much arithmetic on (about 40 us of kernel time) a GEMM whose activation scales are not token-contiguous gets a
-# token-contiguous copy of them first: the kernels read a scale per lane and k-tile, which in the row-major layout is a
-# cache line per lane (4096 x 4096 x 7168: 110 us against 96 us; 1024 x 4096 x 7168: 46.9 against 41.8), and the copy costs
-# about 3 us on the device. Below it the copy costs as much as it saves (512 x 7168 x 4096: 25.8 against 24.0 us).
+# token-contiguous copy of them first: the kernels read a scale per row and k-tile, which in the row-major layout is a
+# cache line per row (4096 x 4096 x 7168: 110 us against 96 us), and the copy costs about 3 us on the device. Below it the copy
+# costs as much as it saves. Ring tiles that copy row-major scales four k-tiles at a time (`fp8_quad_scales` in
+# gemm/fp8_gemm.hpp) need none: 1023 x 7168 x 4096 40.3 us with the copy, 38.9 without, 1024 x 4096 x 7168 42.4 and 42.0.
 SCALE_RELAYOUT_MIN_FLOP = 6e10
 
 
-def scales_for_kernel(scales: torch.Tensor, flop: float) -> torch.Tensor:
+def scales_for_kernel(scales: torch.Tensor, flop: float, keys=None) -> torch.Tensor:
     """The activation scales `[m, k/128]` (or `[groups, m, k/128]`) as the FP8 kernels should be given them: as they are
-    when they are token-contiguous already or the problem is small, else a token-contiguous copy (same values, so the
-    same result bits; allocated from torch's caching allocator on the current stream)."""
+    when they are token-contiguous already, the problem is small, or the kernel of `keys` takes them in this layout at no cost, else a
+    token-contiguous copy (same values, so the same result bits; allocated from torch's caching allocator on the current
+    stream)."""
     if flop < SCALE_RELAYOUT_MIN_FLOP or scales.size(-1) == 1 or scales.size(-2) == 1:
         return scales
     if scales.stride(-2) == 1 and scales.stride(-1) == scales.size(-2):
         return scales
+    # ring tiles, except where the contiguous layout's tiles follow the groups (256 rows there)
+    if keys is not None and keys['NUM_STAGES'] > 2 and (keys['BLOCK_M'] < 256 or keys.get('GEMM_TYPE') != 'GroupedContiguous'):
+        if (scales.stride(-1) == 1 and scales.size(-1) % 4 == 0 and scales.stride(-2) % 4 == 0 and scales.data_ptr() % 16 == 0
+                and (scales.dim() == 2 or scales.stride(0) % 4 == 0)):
+            return scales
     return get_col_major_tensor(scales)
 
 
