@@ -1095,7 +1095,7 @@ public:
                                                                    : (m <= 128 * (long long)num_groups ? 1 : 1 << 30);
         const bool quad = fp8_quad_scales(lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k,
                                           kGemmType == GemmType::GroupedMasked ? lhs_scales_stride_g : 0, k);
-        return pick_kernel<false>(tile_rows, uint64_t(num_groups) * n * k, quad, [&](auto stream_weights, auto quad_scales) {
+        return pick_kernel<false>(tile_rows, uint64_t(num_groups) * n * k, k, quad, [&](auto stream_weights, auto quad_scales) {
             hipLaunchKernelGGL((fp8_gemm_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, int(kNumStages), decltype(stream_weights)::value,
                                                 decltype(quad_scales)::value>),
                                dim3(grid), dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream,
@@ -1163,7 +1163,7 @@ public:
         unsigned* counters = static_cast<unsigned*>(workspace);
         float* partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kSplitKCounterBytes);
         const bool quad = fp8_quad_scales(lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k, 0, k);
-        return pick_kernel<TokenContiguous::value>(sched.tiles_m, uint64_t(n) * k, quad, [&](auto stream_weights, auto quad_scales) {
+        return pick_kernel<TokenContiguous::value>(sched.tiles_m, uint64_t(n) * k, k / SPLIT_K, quad, [&](auto stream_weights, auto quad_scales) {
             hipLaunchKernelGGL((fp8_gemm_split_k_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, int(kNumStages), SPLIT_K, decltype(stream_weights)::value,
                                                         decltype(quad_scales)::value>),
                                dim3(int(grid)), dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream,
@@ -1199,7 +1199,7 @@ public:
             grid = capped_grid(slots < cus ? slots : cus, num_sms, device_cu_count());
         }
         const bool quad = fp8_quad_scales(lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k, 0, k);
-        return pick_kernel<TokenContiguous::value>(sched.tiles_m, uint64_t(n) * k, quad, [&](auto stream_weights, auto quad_scales) {
+        return pick_kernel<TokenContiguous::value>(sched.tiles_m, uint64_t(n) * k, k, quad, [&](auto stream_weights, auto quad_scales) {
             hipLaunchKernelGGL((fp8_gemm_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, GemmType::Normal, int(kNumStages), decltype(stream_weights)::value,
                                                 decltype(quad_scales)::value>),
                                dim3(grid), dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream,
@@ -1215,10 +1215,10 @@ private:
     // k-tiles at a time (ring tiles that consume a k-tile per barrier). What the sizes or the caller's scale layout rule out when the
     // kernel is compiled is left out.
     template <bool TOKEN_CONTIGUOUS, typename Launch>
-    static hipError_t pick_kernel(int tile_rows, uint64_t weight_bytes, bool quad, Launch&& launch) {
+    static hipError_t pick_kernel(int tile_rows, uint64_t weight_bytes, int row_bytes, bool quad, Launch&& launch) {
         constexpr uint64_t KNOWN = uint64_t(SHAPE_N) * SHAPE_K * kNumGroups;
         constexpr bool RING = kNumStages > 2;
-        constexpr bool MAY_STREAM = RING && (KNOWN == 0 || (kGemmType != GemmType::Normal && kNumGroups == 1) || streams_weights(1, KNOWN));
+        constexpr bool MAY_STREAM = RING && (KNOWN == 0 || (kGemmType != GemmType::Normal && kNumGroups == 1) || streams_weights(1, KNOWN, 0));
         constexpr bool MAY_QUAD = RING && !TOKEN_CONTIGUOUS && SHAPE_K % 512 == 0 && fp8_ring_group(BLOCK_M, BLOCK_N, int(kNumStages)) == 1 &&
                                   Fp8TileConfig<BLOCK_M, BLOCK_N>::ring_bytes(int(kNumStages), true) <= 160 * 1024;
         auto with_scales = [&](auto stream_weights) {
@@ -1227,7 +1227,7 @@ private:
             return launch(stream_weights, std::false_type{});
         };
         if constexpr (MAY_STREAM)
-            if (streams_weights(tile_rows, weight_bytes)) return with_scales(std::true_type{});
+            if (streams_weights(tile_rows, weight_bytes, row_bytes)) return with_scales(std::true_type{});
         return with_scales(std::false_type{});
     }
 };
