@@ -154,14 +154,14 @@ DENSE_TEST_SHAPES = [
     (256, 5120, 5120), (4096, 2048, 7168), (4096, 7168, 2048), (256, 24576, 1536),
     (128, 4096, 7168), (512, 4096, 2048), (1024, 7168, 1024),
     (3000, 5000, 1000),          # the 256 x 256 tile (8-wave kernel: K is not whole k-tiles) with ragged m, n and a k tail
-    (2900, 5004, 520),           # same with n % 8 == 4 (narrow stores) and an odd number of k-tiles
+    (2900, 5004, 520),           # same with n % 8 == 4 (rows that end inside a 16-byte store) and an odd number of k-tiles
     (2900, 5000, 64),            # same with a single k-tile
     (3000, 5000, 960),           # the 256 x 256 tile on the 4-wave kernel (whole k-tiles, an odd number of them), ragged m and n
     (2900, 5000, 256),           # same with four k-tiles, the fewest it takes
     # the narrower tiles of 256 rows: 256 x 160, 256 x 224, 256 x 192, each once whole (4-wave kernel) and once ragged in m, n
     # and k (8-wave kernel)
     (4096, 5120, 512), (4000, 5000, 520), (2048, 7168, 256), (2047, 7100, 264), (4096, 6144, 256), (4090, 6100, 72),
-    # and ragged in m and n on the 4-wave kernel (whole k-tiles, n a multiple of 8)
+    # and ragged in m and n on the 4-wave kernel (whole k-tiles)
     (4000, 5000, 576), (2047, 7096, 832), (4090, 6104, 320),
     # the 192-wide tiles of the ring kernel (wave slabs of 96 columns), whole and ragged
     (2048, 2112, 264), (2000, 2100, 136), (1024, 2112, 264), (1000, 2100, 72),
@@ -332,6 +332,11 @@ CAPPED_SHAPES = [(2048, 4096, 1024), (512, 4096, 2048), (300, 2112, 640)]
 # Dense ring tiles walked under a cap where their copying waves end a k-tile early and meet no staged epilogue: rows of the output
 # that are 8 but not 16 bytes apart, a k tail, fewer k-tiles than stages. Tiles, (m, n), depths, cap.
 DENSE_RAGGED_CAP_CASE = ([(128, 128), (128, 192), (64, 64), (256, 128)], (390, 516), (72, 200), 8)
+
+
+# Outputs whose rows are no multiple of 16 bytes, on every width of the 256-row kernels and two ring tiles: tiles, rows, columns, depths
+# (whole k-tiles: the 4-wave kernel, else the 8-wave one)
+RAGGED_ROWS_CASE = ([(256, 256), (256, 224), (256, 192), (256, 160), (128, 192), (64, 64)], 259, (4, 12, 132, 236, 772), (320, 264))
 
 
 # Weights of 32 MB and more are fetched with the non-temporal hint where few tile rows read them: (tile, parts of K), rows, (n, k)
@@ -523,6 +528,10 @@ def jit_kernels_in_use(num_cus: int = 256):
         for k in depths:
             name, keys, arg_defs, code_template = fp8_explicit_tile_plan(*tile, FP8_SHORT_K_SIZES[1], k)
             add(name, arg_defs, gemm.includes, code_template, keys)
+    for tile in RAGGED_ROWS_CASE[0]:
+        for dtype in (torch.bfloat16, torch.half):
+            name, keys, arg_defs, includes, code_template = dense_tile_plan(tile, dtype, 0)
+            add(name, arg_defs, includes, code_template, keys)
     for tile, split_k in SCALE_LAYOUT_TILES:
         for k in SCALE_LAYOUT_SIZES[2]:
             name, keys, arg_defs, code_template = strided_tile_plan(tile, split_k, SCALE_LAYOUT_SIZES[1], k)

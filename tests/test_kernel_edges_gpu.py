@@ -313,3 +313,24 @@ def test_activation_scales_of_groups_of_any_layout_give_the_same_bits(masked):
     expected = run(yan.get_col_major_tensor(sa))
     for name, scales in _scale_layouts(sa).items():
         assert torch.equal(run(scales), expected), name
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.half])
+@pytest.mark.parametrize('tile', testing.RAGGED_ROWS_CASE[0])
+def test_output_rows_that_end_inside_a_16_byte_store(tile, dtype):
+    """The bits of the same problem with four columns more, whose rows are whole 16-byte pieces, and nothing past the output."""
+    _, m, columns, depths = testing.RAGGED_ROWS_CASE
+    name, keys, arg_defs, includes, code_template = testing.dense_tile_plan(tile, dtype, 0)
+    kernel = jit.build(name, arg_defs, jit.generate(includes, arg_defs, jit.cpp_format(code_template, keys)))
+    stream = torch.cuda.current_stream()
+    for k in depths:
+        a, b, _ = testing.make_bf16_case(m, max(columns) + 4, k, seed=21, dtype=dtype, device='cuda')
+        for n in columns:
+            _announce('ragged rows', tile, dtype, n, k)
+            whole = torch.full((m, n + 4), float('nan'), dtype=dtype, device='cuda')
+            assert kernel(m, n + 4, k, a, b, whole, stream) == 0
+            room = torch.full((m * n + 64, ), -7.0, dtype=dtype, device='cuda')
+            assert kernel(m, n, k, a, b, room, stream) == 0
+            torch.cuda.synchronize()
+            assert torch.equal(room[:m * n].view(m, n), whole[:, :n])
+            assert (room[m * n:] == -7.0).all()

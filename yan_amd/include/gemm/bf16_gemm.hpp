@@ -225,7 +225,7 @@ dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
             for (int d = 0; d < NUM_COPIES; ++d) copy_pass(d, kt + STAGES - 1, nxt, nxt + BLOCK_M * kRowBytes);
             st = st + 1 == STAGES ? 0 : st + 1;
         }
-        if (SPLIT_K > 1 || (n % 8) == 0) __builtin_amdgcn_s_barrier();      // the one in front of the epilogue
+        __builtin_amdgcn_s_barrier();      // the one in front of the epilogue
         return;
     }
     for (int kt = kt_lo; kt < kt_hi; ++kt) {
@@ -263,52 +263,32 @@ dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
     // lanes idle); store instructions per 32 rows
     constexpr int LANES_PER_ROW = Cfg::WTN / 8, ROWS_PER_STORE = kWaveSize / LANES_PER_ROW, STORES = ceil_div(32, ROWS_PER_STORE);
     static_assert(NW * REGION <= STAGE_BYTES && STORES >= 1 && sizeof(Elem) == 2);
-    if ((n % 8) == 0) {
-        // every wave has read the last k-tile (a bare barrier: nothing here depends on the copies still under way)
-        if constexpr (SPLIT_K == 1) {
-            __builtin_amdgcn_s_waitcnt(waitcnt_imm(kNoWaitVm, 0));
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-        }
-        uint8_t* region = ring + (st == 0 ? STAGES - 1 : st - 1) * STAGE_BYTES + wave * REGION;
-        const int ml = lane % 32, r_in = lane / LANES_PER_ROW, c = lane % LANES_PER_ROW;
-        const int n_in_tile = wn * Cfg::WTN + 8 * c;
-#pragma unroll
-        for (int j = 0; j < TM; ++j) {
-#pragma unroll
-            for (int i = 0; i < TN; ++i)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-                    *reinterpret_cast<decltype(pack4(v, Elem{}))*>(region + ml * PITCH + (32 * i + 8 * q + 4 * g) * 2) = pack4(v, Elem{});
-                }
-#pragma unroll
-            for (int s = 0; s < STORES; ++s) {
-                const int row = ROWS_PER_STORE * s + r_in, m_in_tile = wm * Cfg::WTM + 32 * j + row;
-                const i32x4 v = *reinterpret_cast<const i32x4*>(region + row * PITCH + c * 16);
-                if (r_in < ROWS_PER_STORE && row < 32 && m0 + m_in_tile < m && n0 + n_in_tile < n)
-                    buffer_store_16(v, rsrc_c, uint32_t(m_in_tile * n + n_in_tile) * 2u, stream_out);
-            }
-        }
-        return;
+    // every wave has read the last k-tile (a bare barrier: nothing here depends on the copies still under way)
+    if constexpr (SPLIT_K == 1) {
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm(kNoWaitVm, 0));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
     }
-    const int m_lane = m0 + wm * Cfg::WTM + lane % 32;
-    const int n_lane = n0 + wn * Cfg::WTN + 4 * g;
+    uint8_t* region = ring + (st == 0 ? STAGES - 1 : st - 1) * STAGE_BYTES + wave * REGION;
+    const int ml = lane % 32, r_in = lane / LANES_PER_ROW, c = lane % LANES_PER_ROW;
+    const int n_in_tile = wn * Cfg::WTN + 8 * c;
 #pragma unroll
     for (int j = 0; j < TM; ++j) {
-        const int mm = m_lane + j * 32;
-        if (mm >= m) continue;
 #pragma unroll
         for (int i = 0; i < TN; ++i)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const int nn = n_lane + i * 32 + q * 8;
-                if (nn < n) {
-                    const f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-                    buffer_store_8(pack4(v, Elem{}), rsrc_c, uint32_t((mm - m0) * n + nn - n0) * 2u, stream_out);
-                }
+                const f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+                *reinterpret_cast<decltype(pack4(v, Elem{}))*>(region + ml * PITCH + (32 * i + 8 * q + 4 * g) * 2) = pack4(v, Elem{});
             }
+#pragma unroll
+        for (int s = 0; s < STORES; ++s) {
+            const int row = ROWS_PER_STORE * s + r_in, m_in_tile = wm * Cfg::WTM + 32 * j + row;
+            const i32x4 v = *reinterpret_cast<const i32x4*>(region + row * PITCH + c * 16);
+            if (r_in < ROWS_PER_STORE && row < 32 && m0 + m_in_tile < m && n0 + n_in_tile < n)
+                buffer_store_columns(v, rsrc_c, uint32_t(m_in_tile * n + n_in_tile) * 2u, n0 + n_in_tile, n, stream_out);
+        }
     }
 }
 
@@ -515,7 +495,7 @@ dense_gemm_body_8w(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
         // receiving the next tile meanwhile.
         const int m_slab = cur.m0 + wm * WTM, n_slab = cur.n0 + wn * WTN;
         static_assert(sizeof(Elem) == 2);
-        if ((n % 8) == 0) {
+        {
             constexpr int PITCH = 2 * WTN + 16;
             // lanes per row segment; rows one store instruction covers (lanes beyond the last whole row sit idle when the
             // segment length does not divide the wave); store instructions per 16 rows
@@ -537,20 +517,8 @@ dense_gemm_body_8w(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
                     if (r_in < ROWS_PER_STORE && row < 16) {
                         const i32x4 v = *reinterpret_cast<const i32x4*>(region + row * PITCH + c * 16);
                         if (mm < m && nn < n)
-                            buffer_store_16(v, rsrc_c, uint32_t((wm * WTM + 16 * j + row) * n + wn * WTN + 8 * c) * 2u, stream_out);
+                            buffer_store_columns(v, rsrc_c, uint32_t((wm * WTM + 16 * j + row) * n + wn * WTN + 8 * c) * 2u, nn, n, stream_out);
                     }
-                }
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < TM; ++j) {
-                const int mm = m_slab + j * 16 + col;
-                if (mm >= m) continue;
-                Elem* row = C + size_t(mm) * n;
-#pragma unroll
-                for (int i = 0; i < TN; ++i) {
-                    const int nn = n_slab + i * 16 + 4 * g;
-                    if (nn < n) *reinterpret_cast<decltype(pack4(acc[i][j], Elem{}))*>(row + nn) = pack4(acc[i][j], Elem{});
                 }
             }
         }
@@ -580,8 +548,7 @@ dense_gemm_body_8w(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
 //     the place along K ride in the scalar offset, which the hardware adds before its bounds check.
 // Persistent like the 8-wave kernel, same walk, same K rotation per XCD, same order of summation, same bits: from the last but
 // one k-tile of a tile on the copies fetch the next tile; the epilogue turns the slab round through the fifth unit and its
-// stores drain under the next tile. For k % 64 == 0, k >= 128, n % 8 == 0; the launcher sends everything else to the
-// 8-wave kernel.
+// stores drain under the next tile. For k % 64 == 0, k >= 128; the launcher sends everything else to the 8-wave kernel.
 template <typename Elem, int BLOCK_N>
 __device__ __forceinline__ void
 dense_gemm_body_4w(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, Elem* __restrict__ C, int m, int n, int k) {
@@ -804,8 +771,10 @@ dense_gemm_body_4w(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
             uint32_t off[PIECES_PER_GROUP];
 #pragma unroll
             for (int h = 0; h < PIECES_PER_GROUP; ++h)
-                off[h] = r_in < ROWS_PER_STORE && n0 + wn * WTN + PIECE_COLS * h + 8 * c < n
+                off[h] = r_in < ROWS_PER_STORE && n0 + wn * WTN + PIECE_COLS * h + 8 * c + 8 <= n
                              ? uint32_t((wm * WTM + r_in) * n + wn * WTN + PIECE_COLS * h + 8 * c) * 2u : kOutOfRange;
+            // where rows end inside a lane's 16 bytes (n % 8 == 4), the lane that has the end stores 8
+            const bool row_ends_here = n % 8 != 0 && n - n0 < BLOCK_N;
             const uint32_t row_bytes = uint32_t(n) * 2u;
             i32x4 back[2][STORES];
             auto into_lds = [&](int u) __attribute__((always_inline)) {
@@ -835,6 +804,13 @@ dense_gemm_body_4w(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
                     // the last store of a piece may reach past its 16 rows
                     const uint32_t lane_off = (16 % ROWS_PER_STORE == 0 || ROWS_PER_STORE * s + r_in < 16) ? off[h] : kOutOfRange;
                     __builtin_amdgcn_raw_buffer_store_b128(back[u & 1][s], rsrc_c, lane_off, (16 * j + ROWS_PER_STORE * s) * row_bytes, decltype(policy_c)::value);
+                    if (row_ends_here) {
+                        typedef int i32x2 __attribute__((ext_vector_type(2)));
+                        const bool mine = r_in < ROWS_PER_STORE && n0 + wn * WTN + PIECE_COLS * h + 8 * c + 4 == n && ROWS_PER_STORE * s + r_in < 16;
+                        const uint32_t end_off = mine ? uint32_t((wm * WTM + r_in) * n + wn * WTN + PIECE_COLS * h + 8 * c) * 2u : kOutOfRange;
+                        __builtin_amdgcn_raw_buffer_store_b64(i32x2{back[u & 1][s][0], back[u & 1][s][1]}, rsrc_c, end_off,
+                                                              (16 * j + ROWS_PER_STORE * s) * row_bytes, decltype(policy_c)::value);
+                    }
                 }
             };
 #pragma unroll
@@ -957,14 +933,14 @@ inline hipError_t launch_dense(int m, int n, int k, const void* a, const void* b
         const int cus = device_cu_count() / kNumXCD * kNumXCD;
         const int grid = capped_grid(slots < cus ? slots : cus, num_sms, device_cu_count());
         // The tiles of 256 rows and 160 to 256 columns have two kernels that give the same bits: 4 waves with slabs of 128 rows
-        // where its conditions hold (whole k-tiles, output rows of whole 16-byte segments) and K is long enough for it to pay
+        // where its conditions hold (whole k-tiles) and K is long enough for it to pay
         // (256 x 256: level at k = 256, 5 to 14 % faster from k = 1024 on; the narrower tiles gain 8 to 20 %), 8 waves with
         // slabs of 64 rows otherwise.
         // (its copies address the operands 3 KB above their descriptors' start: that much less than 2 GiB per operand)
         const uint64_t m_pad = uint64_t(ceil_div(m, BLOCK_M)) * BLOCK_M, n_pad = uint64_t(ceil_div(n, BLOCK_N)) * BLOCK_N;
         const bool in_reach = (m_pad > n_pad ? m_pad : n_pad) * k * 2 + 4096 < kOutOfRange;
         if constexpr (WAVES == 0 && BLOCK_N >= 160)
-        if (k % 64 == 0 && k >= 256 && n % 8 == 0 && in_reach) {
+        if (k % 64 == 0 && k >= 256 && in_reach) {
             if constexpr (__is_same(Elem, _Float16))
                 hipLaunchKernelGGL((fp16_gemm_cute_4w<BLOCK_N>), dim3(grid), dim3(4 * kWaveSize), 0, stream,
                                    static_cast<const uint8_t*>(a), static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k);

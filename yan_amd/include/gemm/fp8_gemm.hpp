@@ -210,7 +210,7 @@ fp8_store_slab(const f32x4 (&acc)[TN][TM], uint8_t* region, __amdgpu_buffer_rsrc
                     const i32x4 v = *reinterpret_cast<const i32x4*>(region + row * PITCH + c * 16);
                     // a slab width that does not divide 64 lanes leaves the last lanes, and rows past 16, without work
                     const bool live = mm < row_end && nn < n && r_in < ROWS_PER_STORE && row < 16;
-                    if (live) buffer_store_16(v, rsrc_out, uint32_t((mm - m0) * n + nn - n0) * 2u, stream_out);
+                    if (live) buffer_store_columns(v, rsrc_out, uint32_t((mm - m0) * n + nn - n0) * 2u, nn, n, stream_out);
                 }
                 __builtin_amdgcn_sched_barrier(0);      // one 16-row pass at a time: the registers are full of sums
             }
@@ -658,16 +658,14 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     }
 
     // Epilogue (fp8_store_slab): slabs of 32 columns or more turn round through the LDS stage that was consumed last (the
-    // only one no copy is on its way into) when the rows of the output are 16-byte aligned.
+    // only one no copy is on its way into).
     // An output larger than the L2s together (8 x 4 MB) is stored with the non-temporal hint: kept in L2 it pushes out
     // the operand panels the other workgroups of the XCD are about to read.
-    bool staged = false;
-    if constexpr (kStagedEpilogue) staged = (N % 8) == 0;
     const bool stream_out = size_t(m) * N * 2 * (kGemmType == GemmType::GroupedMasked ? num_groups : 1) > (size_t(32) << 20);
     const __amdgpu_buffer_rsrc_t rsrc_out = make_out_rsrc(out + size_t(m0) * N + n0);
-    if (staged) {
+    if constexpr (kStagedEpilogue) {
         constexpr int REGION = 16 * (Cfg::WTN * 2 + 16);
-        static_assert(!kStagedEpilogue || ((NW / 2) * REGION <= Cfg::LDS_ROWS_A * kRowBytes && (NW / 2) * REGION <= Cfg::LDS_ROWS_B * kRowBytes));
+        static_assert((NW / 2) * REGION <= Cfg::LDS_ROWS_A * kRowBytes && (NW / 2) * REGION <= Cfg::LDS_ROWS_B * kRowBytes);
         // every wave has read the last k-tile (a bare barrier: __syncthreads() would also wait for the copies still
         // on their way into the other stages, which nobody will read)
         __builtin_amdgcn_s_waitcnt(waitcnt_imm(kNoWaitVm, 0));
@@ -682,7 +680,7 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
         if constexpr (SPLIT_K > 1)
             if (!fp8_meet_partials<SPLIT_K, NW, TN, TM>(acc, partials, counters, tile_slot, split, wave, lane_late)) return;
         uint8_t* region = (wave < NW / 2 ? epi_a : epi_b) + (wave % (NW / 2)) * REGION;
-        fp8_store_slab<Cfg, kStagedEpilogue>(acc, region, rsrc_out, m_slab, n_slab, m0, n0, m, N, stream_out, lane_late);
+        fp8_store_slab<Cfg, true>(acc, region, rsrc_out, m_slab, n_slab, m0, n0, m, N, stream_out, lane_late);
     } else {
         if (LW > NW && wave >= NW) return;              // waves that only copy
         if constexpr (SPLIT_K > 1)
@@ -860,12 +858,8 @@ fp8_gemm_walk(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
             int lane_late = lane;
             asm volatile("" : "+v"(lane_late));
             uint8_t* region = (wave < NW / 2 ? a_nxt : b_third) + (wave % (NW / 2)) * REGION;
-            if ((N % 8) == 0)
-                fp8_store_slab<Cfg, true>(acc, region, rsrc_out, cur.m0 + wm * Cfg::WTM, cur.n0 + wn * Cfg::WTN, cur.m0, cur.n0,
-                                          m, N, stream_out, lane_late);
-            else
-                fp8_store_slab<Cfg, false>(acc, region, rsrc_out, cur.m0 + wm * Cfg::WTM, cur.n0 + wn * Cfg::WTN, cur.m0, cur.n0,
-                                           m, N, stream_out, lane_late);
+            fp8_store_slab<Cfg, true>(acc, region, rsrc_out, cur.m0 + wm * Cfg::WTM, cur.n0 + wn * Cfg::WTN, cur.m0, cur.n0, m, N,
+                                      stream_out, lane_late);
         }
         if (!nxt.valid) {
             wait_for_copies();          // of weights nobody will read: none lands in LDS that is no longer this workgroup's

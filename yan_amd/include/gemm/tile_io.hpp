@@ -66,6 +66,14 @@ __device__ __forceinline__ void buffer_store_8(T8 v, __amdgpu_buffer_rsrc_t rsrc
     if (streaming) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(i32x2, v), rsrc, voffset, 0, 2);
     else __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(i32x2, v), rsrc, voffset, 0, 0);
 }
+// Eight 16-bit columns `nn` .. of a row of `n` (n % 4 == 0, nn % 8 == 0, nn < n): 16 bytes, or the first 8 where the row ends inside
+// them. Rows of n % 8 == 4 are 8 bytes off 16-byte alignment every other time, which a 16-byte buffer store takes (it asks for
+// 4): such outputs left in pieces of 8 bytes straight from the accumulators before, 16 or 32 rows an instruction.
+__device__ __forceinline__ void buffer_store_columns(i32x4 v, __amdgpu_buffer_rsrc_t rsrc, uint32_t voffset, int nn, int n, bool streaming) {
+    typedef int i32x2 __attribute__((ext_vector_type(2)));
+    if (n % 8 == 0 || nn + 8 <= n) buffer_store_16(v, rsrc, voffset, streaming);
+    else buffer_store_8(i32x2{v[0], v[1]}, rsrc, voffset, streaming);
+}
 // Descriptor over an output tile whose first element is `origin`: offsets are relative to it, bounds are the caller's
 // business (rows and columns past the matrix are skipped by predicate).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_out_rsrc(const void* origin) { return make_rsrc(origin, 0xffffffffu); }
