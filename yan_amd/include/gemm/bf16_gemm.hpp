@@ -1003,7 +1003,7 @@ inline hipError_t launch_dense_split_k(int m, int n, int k, const void* a, const
                                dim3(dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
                                static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, partials, counters);
     };
-    if (streams_weights(sched.tiles_m, uint64_t(n) * k * 2, k * 2 / SPLIT_K)) launch(std::true_type{});
+    if (streams_weights(sched.tiles_m, uint64_t(n) * k * 2, k * 2)) launch(std::true_type{});
     else launch(std::false_type{});
     return hipGetLastError();
 }

@@ -44,6 +44,20 @@
 
 namespace yan {
 
+// How the waves of a ring tile copy a k-tile's activation scales, 64 rows an instruction. Token-contiguous ones are two cache lines
+// each, and every wave copies a part, several the same one: telling the waves apart costs 1 to 3 %. Any other layout is a line a
+// row, more requests than the operands if several waves ask for it: the first waves copy a part each, the others nothing. Rows
+// of whole 16-byte pieces, as row-major scales are where K is a multiple of 512, are copied four k-tiles at a time. Row-major,
+// every wave -> one wave -> four k-tiles: 512 x 7168 x 7168 62.8 -> 47.2 -> 39.8 us (37 token-contiguous); 640 x 9216 x 4096 47.3 -> 36.1 and
+// 1500 x 4096 x 4096 43.2 -> 35.8 with four, 900 x 4096 x 7040 53.7 -> 43.3 with one. Kernels of their own: the choice inside the
+// k-loop cost the token-contiguous layout 2 to 5 %.
+enum class Fp8ScaleCopies { EveryWave, OneWave, FourKTiles };
+inline Fp8ScaleCopies fp8_scale_copies(const float* scales, int stride_m, int stride_k, int stride_g, int k) {
+    if (stride_m == 1) return Fp8ScaleCopies::EveryWave;
+    const bool pieces = stride_k == 1 && stride_m % 4 == 0 && stride_g % 4 == 0 && k % 512 == 0 && reinterpret_cast<uintptr_t>(scales) % 16 == 0;
+    return pieces ? Fp8ScaleCopies::FourKTiles : Fp8ScaleCopies::OneWave;
+}
+
 // K-tiles a tile's ring is consumed by per barrier (1: one at a time) and the waves its workgroup is launched with.
 // Tiles of one or two atoms per wave (the decode shapes) with a ring of 12 stages take four k-tiles per barrier, and
 // four more waves that only copy: a wave gets one copy instruction through per ~50 ns, and three per k-tile on each
@@ -78,7 +92,7 @@ struct Fp8TileConfig {
     static constexpr int  RING_SCALE_BYTES = ceil_div(BLOCK_M * 4, 1024) * 1024;
     static constexpr int  RING_STAGE_BYTES = (LDS_ROWS_A + LDS_ROWS_B) * kRowBytes + RING_SCALE_BYTES;
     static constexpr bool RING_CAPABLE = BLOCK_M % 32 == 0 && (BLOCK_M / 8) % NUM_WAVES == 0 && BLOCK_N % 16 == 0;
-    // Behind the stages: room for activation scales that come four k-tiles at a time (fp8_quad_scales), 16 bytes a row; a slot is taken again when every k-tile of its four has been consumed, with STAGES - 1 k-tiles in flight. Then
+    // Behind the stages: room for activation scales that come four k-tiles at a time (Fp8ScaleCopies), 16 bytes a row; a slot is taken again when every k-tile of its four has been consumed, with STAGES - 1 k-tiles in flight. Then
     // 1 KB that takes what copies of nothing write.
     static constexpr int  SCALE_PARTS = ceil_div(BLOCK_M, 64);
     __host__ __device__ static constexpr int quad_slots(int stages) { return (stages + 6) / 4; }
@@ -281,9 +295,9 @@ contiguous_block_at(const int* __restrict__ grouped_layout, int blocks, bool tal
 // EXPLICIT_TILE: `bid` names the tile itself, as (its first row / 128) * tiles_n + n_idx, for callers that order the tiles
 // themselves; in the contiguous layout all rows of such a tile belong to the group of its first row.
 // STREAM: a ring tile's copies of the weights carry the non-temporal hint (streams_weights in scheduler.hpp).
-// QUAD: a ring tile copies its activation scales four k-tiles at a time (fp8_quad_scales).
+// SCALES: how a ring tile copies its activation scales (Fp8ScaleCopies).
 template <int SHAPE_N, int SHAPE_K, int BLOCK_M, int BLOCK_N, GemmType kGemmType, int STAGES, int SPLIT_K = 1, bool EXTERNAL_RING = false,
-          bool EXPLICIT_TILE = false, bool STREAM = false, bool QUAD = false>
+          bool EXPLICIT_TILE = false, bool STREAM = false, Fp8ScaleCopies SCALES = Fp8ScaleCopies::EveryWave>
 __device__ __forceinline__ void
 fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_scales,
               const uint8_t* __restrict__ rhs, const float* __restrict__ rhs_scales,
@@ -479,12 +493,9 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     // streaming its operands and one k-tile of prefetch cannot cover the memory latency. Every wave issues the same
     // number of copies for every k-tile (OPS), in the same order, so "k-tile kb has landed" is "at most
     // (STAGES - 2) * OPS of my copies are outstanding". The activation scales of a k-tile travel through LDS as well (a register
-    // load between the copies would make the in-order counter wait for every older copy): the first waves copy a 64-row part of
-    // them each, and the others nothing, with the same number of instructions. Row-major scales are a cache line a row and k-tile,
-    // four k-tiles of them with QUAD. Every wave copying a part, as before, 512 x 7168 x 7168 took 65.7 us with row-major scales and
-    // 38 with token-contiguous ones; one wave a part 47, four k-tiles at a time 40
-    // (1500 x 4096 x 4096 43.2 -> 35.8, 640 x 9216 x 4096 47.3 -> 36.1; K no multiple of 512: 900 x 4096 x 7040 53.7 -> 43.3). The scales go first
-    // in a k-tile, before its MFMAs: among them they cost 512 x 7168 x 7168 with token-contiguous scales 39.1 us, 36.8 now.
+    // load between the copies would make the in-order counter wait for every older copy), with one instruction of every wave:
+    // Fp8ScaleCopies says who copies what. The scales go first in a k-tile, before its MFMAs (among them: 1-3 % slower).
+    constexpr bool QUAD = SCALES == Fp8ScaleCopies::FourKTiles, EVERY_WAVE = SCALES == Fp8ScaleCopies::EveryWave;
     constexpr int STAGE_BYTES = Cfg::RING_STAGE_BYTES, A_BYTES = Cfg::LDS_ROWS_A * kRowBytes, TILE_BYTES = A_BYTES + Cfg::LDS_ROWS_B * kRowBytes;
     constexpr int G = fp8_ring_group(BLOCK_M, BLOCK_N, STAGES);
     constexpr int OPS = NUM_COPIES + 1, SCALE_PARTS = Cfg::SCALE_PARTS;
@@ -504,7 +515,7 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     if constexpr (G > 1) {
     // Eight waves share the copies of a k-tile: operation o = slot * 8 + wave is the o-th 8-row group of the stage
     // (activation rows first, then weight rows: the two tiles lie back to back) or, behind the last group, the copy of
-    // the activation scales; further operations copy nothing, behind those.
+    // the activation scales, which several waves may repeat (same bytes) or only the first makes.
     constexpr int GA = BLOCK_M / 8, GROUPS_AB = (BLOCK_M + BLOCK_N) / 8, SLOTS = ceil_div(GROUPS_AB + 1, LW);
     static_assert(LW == 8 && NW == 4 && A_BYTES == GA * 8 * kRowBytes && TILE_BYTES == GROUPS_AB * 8 * kRowBytes && SCALE_PARTS == 1);
     static_assert(Cfg::UNIFORM_SCALE_B && NB == 1 && (STAGES - 2 * G) * SLOTS <= 63);
@@ -525,7 +536,8 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
             if (in_a) __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_a : rsrc_none, YAN_LDS_CAST(stage + o * 8 * kRowBytes), kChunk, slot_voff[sl], kb * kRowBytes, 0, 0);
             else __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_b : rsrc_none, YAN_LDS_CAST(stage + o * 8 * kRowBytes), kChunk, slot_voff[sl], kb * kRowBytes, 0, STREAM ? kNonTemporal : 0);
         } else {
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(live && o == GROUPS_AB ? rsrc_sa : rsrc_none, YAN_LDS_CAST(stage + TILE_BYTES + (o == GROUPS_AB ? 0 : 256)), 4, scale_voff, kb * sa_stride_k * 4, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(live && (EVERY_WAVE || o == GROUPS_AB) ? rsrc_sa : rsrc_none,
+                                                     YAN_LDS_CAST(stage + TILE_BYTES + (EVERY_WAVE || o == GROUPS_AB ? 0 : 256)), 4, scale_voff, kb * sa_stride_k * 4, 0, 0);
         }
     };
 #pragma unroll
@@ -591,19 +603,20 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
         if (d < StA::PASSES) stage_a.issue_pass(live ? rsrc_a : rsrc_none, stage, kb * kRowBytes, wave, d);
         else stage_b.issue_pass(live ? rsrc_b : rsrc_none, stage + A_BYTES, kb * kRowBytes, wave, d - StA::PASSES);
     };
-    // QUAD: four k-tiles of a row at a time into a slot behind the stages
+    // four k-tiles of a row at a time go into a slot behind the stages
     uint8_t* const quads = ring + STAGES * STAGE_BYTES;
     uint8_t* const nowhere = quads + (QUAD ? Cfg::quad_slots(STAGES) * SCALE_PARTS * 1024 : 0);
     auto quad_of = [&](int kb) { return quads + (kb / 4 % Cfg::quad_slots(STAGES)) * (SCALE_PARTS * 1024); };
     auto issue_scales = [&](int kb, uint8_t* stage) {
-        const bool mine = kb < kb_hi && wave < SCALE_PARTS;         // rows m0 + 64 * wave + lane
+        const int part = EVERY_WAVE ? wave % SCALE_PARTS : wave;        // rows m0 + 64 * part + lane
+        const bool mine = kb < kb_hi && (EVERY_WAVE || wave < SCALE_PARTS);
         if constexpr (QUAD) {
             const bool now = mine && (kb % 4 == 0 || kb == kb_lo);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(now ? rsrc_sa : rsrc_none, YAN_LDS_PTR(now ? quad_of(kb) + wave * 1024 : nowhere), 16,
-                                                     scale_voff, (kb / 4 * 4 + wave * 64 * sa_stride_m) * 4, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(now ? rsrc_sa : rsrc_none, YAN_LDS_PTR(now ? quad_of(kb) + part * 1024 : nowhere), 16,
+                                                     scale_voff, (kb / 4 * 4 + part * 64 * sa_stride_m) * 4, 0, 0);
         } else {
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(mine ? rsrc_sa : rsrc_none, YAN_LDS_PTR(mine ? stage + TILE_BYTES + wave * 256 : nowhere), 4,
-                                                     scale_voff, (kb * sa_stride_k + wave * 64 * sa_stride_m) * 4, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(mine ? rsrc_sa : rsrc_none, YAN_LDS_PTR(EVERY_WAVE || mine ? stage + TILE_BYTES + part * 256 : nowhere), 4,
+                                                     scale_voff, (kb * sa_stride_k + part * 64 * sa_stride_m) * 4, 0, 0);
         }
     };
 #pragma unroll
@@ -687,12 +700,6 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
             if (!fp8_meet_partials<SPLIT_K, NW, TN, TM>(acc, partials, counters, tile_slot, split, wave, lane)) return;
         fp8_store_slab<Cfg, false>(acc, nullptr, rsrc_out, m_slab, n_slab, m0, n0, m, N, stream_out, lane);
     }
-}
-
-// Whether the activation scales are copied four k-tiles at a time: rows of whole 16-byte pieces, as row-major scales are where K is a
-// multiple of 512. A kernel of its own: the choice inside the k-loop cost the token-contiguous layout 2 to 5 %.
-inline bool fp8_quad_scales(const float* scales, int stride_m, int stride_k, int stride_g, int k) {
-    return stride_k == 1 && stride_m % 4 == 0 && stride_g % 4 == 0 && k % 512 == 0 && reinterpret_cast<uintptr_t>(scales) % 16 == 0;
 }
 
 // Whether a problem runs the persistent walk below: the plain GEMM on two LDS stages (three of the weights) with two k-tiles or more.
@@ -880,7 +887,7 @@ fp8_gemm_walk(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
 // yan/include/gemm/fp8_gemm.cuh:40, scheduler.cuh:39-58). Between two tiles every wave must have left the epilogue of
 // the first (which reads the LDS stage the second one's first copies go into).
 template <int SHAPE_N, int SHAPE_K, int BLOCK_M, int BLOCK_N, GemmType kGemmType = GemmType::Normal, int STAGES = 2, bool STREAM = false,
-          bool QUAD = false>
+          Fp8ScaleCopies SCALES = Fp8ScaleCopies::EveryWave>
 __global__ void __launch_bounds__((fp8_launch_waves(BLOCK_M, BLOCK_N, STAGES) * kWaveSize))
 fp8_gemm_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_scales,
                 const uint8_t* __restrict__ rhs, const float* __restrict__ rhs_scales,
@@ -908,13 +915,13 @@ fp8_gemm_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_s
     // A workgroup per slot (no cap): the tile without a loop around it. Inside the loop below the same code runs 2 to 14 %
     // slower on the ring tiles even for a single trip (64 x 7168 x 2048 on 64 x 32 tiles: 6.0 against 5.2 us).
     if (int(gridDim.x) >= num_slots) {
-        fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, STAGES, 1, false, false, STREAM, QUAD>(lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt,
+        fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, STAGES, 1, false, false, STREAM, SCALES>(lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt,
                                                                              sa_stride_m, sa_stride_k, grouped_layout, sa_stride_g,
                                                                              int(blockIdx.x), num_groups, expected_m, two_stages);
         return;
     }
     for (int slot = blockIdx.x; slot < num_slots; slot += gridDim.x) {
-        fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, STAGES, 1, false, false, STREAM, QUAD>(lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt,
+        fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, STAGES, 1, false, false, STREAM, SCALES>(lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt,
                                                                              sa_stride_m, sa_stride_k, grouped_layout, sa_stride_g,
                                                                              slot, num_groups, expected_m, two_stages);
         if (slot + int(gridDim.x) < num_slots) __syncthreads();
@@ -1015,13 +1022,14 @@ fp8_gemm_contiguous_rows_kernel(const uint8_t* __restrict__ lhs, const float* __
 }
 
 // The same tiles with K split SPLIT_K ways: launch slot s is part s % SPLIT_K of tile slot s / SPLIT_K.
-template <int SHAPE_N, int SHAPE_K, int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K, bool STREAM = false, bool QUAD = false>
+template <int SHAPE_N, int SHAPE_K, int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K, bool STREAM = false,
+          Fp8ScaleCopies SCALES = Fp8ScaleCopies::EveryWave>
 __global__ void __launch_bounds__((fp8_launch_waves(BLOCK_M, BLOCK_N, STAGES) * kWaveSize))
 fp8_gemm_split_k_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_scales,
                         const uint8_t* __restrict__ rhs, const float* __restrict__ rhs_scales,
                         __bf16* __restrict__ out, int m, int n_rt, int k_rt, int sa_stride_m, int sa_stride_k,
                         float* __restrict__ partials, unsigned* __restrict__ counters) {
-    fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, GemmType::Normal, STAGES, SPLIT_K, false, false, STREAM, QUAD>(
+    fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, GemmType::Normal, STAGES, SPLIT_K, false, false, STREAM, SCALES>(
         lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt, sa_stride_m, sa_stride_k, nullptr, 0, int(blockIdx.x), 1, 0,
         Fp8TwoStages{}, partials, counters);
 }
@@ -1087,11 +1095,11 @@ public:
         // on average (two to a group, and a group's tile rows are on different XCDs: 8 groups, 2048 rows 45.6 -> 50 us)
         const int tile_rows = kGemmType == GemmType::GroupedMasked ? ceil_div(expected_m > 0 && expected_m < m ? expected_m : m, int(BLOCK_M))
                                                                    : (m <= 128 * (long long)num_groups ? 1 : 1 << 30);
-        const bool quad = fp8_quad_scales(lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k,
-                                          kGemmType == GemmType::GroupedMasked ? lhs_scales_stride_g : 0, k);
-        return pick_kernel<false>(tile_rows, uint64_t(num_groups) * n * k, k, quad, [&](auto stream_weights, auto quad_scales) {
+        const Fp8ScaleCopies copies = fp8_scale_copies(lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k,
+                                                       kGemmType == GemmType::GroupedMasked ? lhs_scales_stride_g : 0, k);
+        return pick_kernel<false>(tile_rows, uint64_t(num_groups) * n * k, k, copies, [&](auto stream_weights, auto scale_copies) {
             hipLaunchKernelGGL((fp8_gemm_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, int(kNumStages), decltype(stream_weights)::value,
-                                                decltype(quad_scales)::value>),
+                                                decltype(scale_copies)::value>),
                                dim3(grid), dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream,
                                static_cast<const uint8_t*>(lhs), lhs_scales, static_cast<const uint8_t*>(rhs), rhs_scales,
                                reinterpret_cast<__bf16*>(out), m, n, k, lhs_scales_stride_m, lhs_scales_stride_k, grouped_layout,
@@ -1156,10 +1164,10 @@ public:
         const long long grid = (long long)sched.grid_size() * SPLIT_K;
         unsigned* counters = static_cast<unsigned*>(workspace);
         float* partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kSplitKCounterBytes);
-        const bool quad = fp8_quad_scales(lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k, 0, k);
-        return pick_kernel<TokenContiguous::value>(sched.tiles_m, uint64_t(n) * k, k / SPLIT_K, quad, [&](auto stream_weights, auto quad_scales) {
+        const Fp8ScaleCopies copies = fp8_scale_copies(lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k, 0, k);
+        return pick_kernel<TokenContiguous::value>(sched.tiles_m, uint64_t(n) * k, k, copies, [&](auto stream_weights, auto scale_copies) {
             hipLaunchKernelGGL((fp8_gemm_split_k_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, int(kNumStages), SPLIT_K, decltype(stream_weights)::value,
-                                                        decltype(quad_scales)::value>),
+                                                        decltype(scale_copies)::value>),
                                dim3(int(grid)), dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream,
                                static_cast<const uint8_t*>(lhs), lhs_scales, static_cast<const uint8_t*>(rhs), rhs_scales,
                                reinterpret_cast<__bf16*>(out), m, n, k, lhs_scales_stride_m, lhs_scales_stride_k, partials, counters);
@@ -1192,10 +1200,10 @@ public:
             const int cus = device_cu_count() / kNumXCD * kNumXCD;
             grid = capped_grid(slots < cus ? slots : cus, num_sms, device_cu_count());
         }
-        const bool quad = fp8_quad_scales(lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k, 0, k);
-        return pick_kernel<TokenContiguous::value>(sched.tiles_m, uint64_t(n) * k, k, quad, [&](auto stream_weights, auto quad_scales) {
+        const Fp8ScaleCopies copies = fp8_scale_copies(lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k, 0, k);
+        return pick_kernel<TokenContiguous::value>(sched.tiles_m, uint64_t(n) * k, k, copies, [&](auto stream_weights, auto scale_copies) {
             hipLaunchKernelGGL((fp8_gemm_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, GemmType::Normal, int(kNumStages), decltype(stream_weights)::value,
-                                                decltype(quad_scales)::value>),
+                                                decltype(scale_copies)::value>),
                                dim3(grid), dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream,
                                static_cast<const uint8_t*>(lhs), lhs_scales, static_cast<const uint8_t*>(rhs), rhs_scales,
                                reinterpret_cast<__bf16*>(out), m, n, k, lhs_scales_stride_m, lhs_scales_stride_k,
@@ -1205,11 +1213,11 @@ public:
     }
 
 private:
-    // Calls `launch` with two of std::true_type / std::false_type: whether the weights are streamed, and whether the scales are copied four
-    // k-tiles at a time (ring tiles that consume a k-tile per barrier). What the sizes or the caller's scale layout rule out when the
-    // kernel is compiled is left out.
+    // Calls `launch` with what a kernel is compiled for: whether the weights are streamed (std::true_type or std::false_type), and how the
+    // scales are copied (a std::integral_constant). What the sizes or the caller's scale layout rule out when the kernel is
+    // compiled is left out. Tiles that are no ring of one k-tile per barrier have no copies four k-tiles at a time.
     template <bool TOKEN_CONTIGUOUS, typename Launch>
-    static hipError_t pick_kernel(int tile_rows, uint64_t weight_bytes, int row_bytes, bool quad, Launch&& launch) {
+    static hipError_t pick_kernel(int tile_rows, uint64_t weight_bytes, int row_bytes, Fp8ScaleCopies copies, Launch&& launch) {
         constexpr uint64_t KNOWN = uint64_t(SHAPE_N) * SHAPE_K * kNumGroups;
         constexpr bool RING = kNumStages > 2;
         constexpr bool MAY_STREAM = RING && (KNOWN == 0 || (kGemmType != GemmType::Normal && kNumGroups == 1) || streams_weights(1, KNOWN, 0));
@@ -1217,8 +1225,10 @@ private:
                                   Fp8TileConfig<BLOCK_M, BLOCK_N>::ring_bytes(int(kNumStages), true) <= 160 * 1024;
         auto with_scales = [&](auto stream_weights) {
             if constexpr (MAY_QUAD)
-                if (quad) return launch(stream_weights, std::true_type{});
-            return launch(stream_weights, std::false_type{});
+                if (copies == Fp8ScaleCopies::FourKTiles) return launch(stream_weights, std::integral_constant<Fp8ScaleCopies, Fp8ScaleCopies::FourKTiles>{});
+            if constexpr (RING && !TOKEN_CONTIGUOUS)
+                if (copies != Fp8ScaleCopies::EveryWave) return launch(stream_weights, std::integral_constant<Fp8ScaleCopies, Fp8ScaleCopies::OneWave>{});
+            return launch(stream_weights, std::integral_constant<Fp8ScaleCopies, Fp8ScaleCopies::EveryWave>{});
         };
         if constexpr (MAY_STREAM)
             if (streams_weights(tile_rows, weight_bytes, row_bytes)) return with_scales(std::true_type{});

@@ -90,7 +90,7 @@ def get_col_major_tensor(x: torch.Tensor) -> torch.Tensor:
 # From this much arithmetic on (about 40 us of kernel time) a GEMM whose activation scales are not token-contiguous gets a
 # token-contiguous copy of them first: the kernels read a scale per row and k-tile, which in the row-major layout is a
 # cache line per row (4096 x 4096 x 7168: 110 us against 96 us), and the copy costs about 3 us on the device. Below it the copy
-# costs as much as it saves. Ring tiles that copy row-major scales four k-tiles at a time (`fp8_quad_scales` in
+# costs as much as it saves. Ring tiles that copy row-major scales four k-tiles at a time (`Fp8ScaleCopies` in
 # gemm/fp8_gemm.hpp) need none: 1023 x 7168 x 4096 40.3 us with the copy, 38.9 without, 1024 x 4096 x 7168 42.4 and 42.0.
 SCALE_RELAYOUT_MIN_FLOP = 6e10
 
