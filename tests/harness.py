@@ -339,12 +339,12 @@ DENSE_RAGGED_CAP_CASE = ([(128, 128), (128, 192), (64, 64), (256, 128)], (390, 5
 RAGGED_ROWS_CASE = ([(256, 256), (256, 224), (256, 192), (256, 160), (128, 192), (64, 64)], 259, (4, 12, 132, 236, 772), (320, 264))
 
 
-# Weights of 32 MB and more are fetched with the non-temporal hint where few tile rows read them: (tile, parts of K), rows, (n, k)
+# Weights of 96 MB and more are fetched with the non-temporal hint where few tile rows read them: (tile, parts of K), rows, (n, k)
 # of a problem that has them so and whose halves along n do not.
 STREAM_FP8_CASES = [((32, 32), 1), ((64, 128), 1), ((64, 64), 4)]
 STREAM_DENSE_CASES = [((64, 64), 1), ((128, 128), 1), ((64, 64), 4)]
-STREAM_FP8_SIZES, STREAM_DENSE_SIZES = (61, 8192, 4096), (125, 8192, 2048)
-STREAM_GROUPED_SIZES = (8, 64, 2048, 2048)          # groups, rows of each, n, k
+STREAM_FP8_SIZES, STREAM_DENSE_SIZES = (61, 24832, 4096), (125, 25088, 2048)
+STREAM_GROUPED_SIZES = (8, 64, 6400, 2048)          # groups, rows of each, n, k
 
 
 def stream_plans(kind: str, tile, split_k: int, n: int):

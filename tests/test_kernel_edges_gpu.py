@@ -209,11 +209,11 @@ def _streamed_weights_case(kind, tile, split_k):
     m, n, k = testing.STREAM_DENSE_SIZES if dense else testing.STREAM_FP8_SIZES
     outs = []
     if dense:
-        a, b, c = testing.make_bf16_case(m, n, k, seed=17, device='cuda')
+        a, b, c = testing.make_bf16_case(m, n, k, seed=17, device='cuda', gen_device='cuda')
     else:
         (a, sa), (b, sb), c = testing.make_fp8_case(m, n, k, seed=17, device='cuda', gen_device='cuda')
         sa = yan.get_col_major_tensor(sa)
-    workspace = torch.zeros(16384 + 256 * 128 * 128 * 4, dtype=torch.uint8, device='cuda')
+    workspace = torch.zeros(16384 + (64 << 20), dtype=torch.uint8, device='cuda')
     stream = torch.cuda.current_stream()
     for lo, hi in ((0, n), (0, n // 2), (n // 2, n)):
         name, keys, arg_defs, includes, code_template = testing.stream_plans(kind, tile, split_k, hi - lo)
@@ -238,9 +238,9 @@ def test_streamed_weights_of_groups_give_the_same_bits(masked):
     groups, rows, n, k = testing.STREAM_GROUPED_SIZES
     _announce('streamed weights of groups', masked)
     if masked:
-        (a, sa), (b, sb), out, layout = testing.make_grouped_masked_case(groups, rows, n, k, (5, 64, 0, 1, 33, 64, 2, 17), seed=18, device='cuda')
+        (a, sa), (b, sb), out, layout = testing.make_grouped_masked_case(groups, rows, n, k, (5, 64, 0, 1, 33, 64, 2, 17), seed=18, device='cuda', gen_device='cuda')
     else:
-        (a, sa), (b, sb), out, layout = testing.make_grouped_contiguous_case((128, 7, 100, 1, 128, 64, 2, 90), n, k, seed=18, device='cuda')
+        (a, sa), (b, sb), out, layout = testing.make_grouped_contiguous_case((128, 7, 100, 1, 128, 64, 2, 90), n, k, seed=18, device='cuda', gen_device='cuda')
 
     def run(lo, hi):
         part = torch.full_like(out[..., lo:hi], -7.0, memory_format=torch.contiguous_format)
@@ -298,9 +298,9 @@ def test_activation_scales_of_groups_of_any_layout_give_the_same_bits(masked):
     groups, rows, n, k = testing.STREAM_GROUPED_SIZES
     _announce('scale layouts of groups', masked)
     if masked:
-        (a, sa), rhs, out, layout = testing.make_grouped_masked_case(groups, rows, n, k, (5, 64, 0, 1, 33, 64, 2, 17), seed=20, device='cuda')
+        (a, sa), rhs, out, layout = testing.make_grouped_masked_case(groups, rows, n, k, (5, 64, 0, 1, 33, 64, 2, 17), seed=20, device='cuda', gen_device='cuda')
     else:
-        (a, sa), rhs, out, layout = testing.make_grouped_contiguous_case((128, 7, 100, 1, 128, 64, 2, 90), n, k, seed=20, device='cuda')
+        (a, sa), rhs, out, layout = testing.make_grouped_contiguous_case((128, 7, 100, 1, 128, 64, 2, 90), n, k, seed=20, device='cuda', gen_device='cuda')
 
     def run(scales):
         got = torch.full_like(out, -7.0)

@@ -237,19 +237,19 @@ __host__ __device__ inline int capped_grid(int slots, int num_sms, int device_cu
     return num_sms >= kNumXCD ? num_sms / kNumXCD * kNumXCD : num_sms;
 }
 
-// Whether a ring tile's copies of the weights carry the non-temporal hint: more weights than the L2s hold together, so that none is
-// still in a cache at the next call of a model whose other weights came by in between, and each panel read once, by one tile row,
-// or by a few that stay together because a row of K (`row_bytes`) is short. Such weights gain nothing from the
-// memory-side cache, and left out of it they stream at 6.6 TB/s instead of 5.9: masked 32 groups x 8 rows x 4096 x 7168 158 -> 141 us,
-// 8 x 30 rows 44 -> 40, contiguous 64 x 64 rows x 2048 x 4096 60.6 -> 57.7; FP8 16 x 16384 x 4096 19.6 -> 16.7, 64 x 16384 x 7168 26.8 ->
-// 24.0, 128 x 16384 x 2048 12.6 -> 11.4; 16-bit 32 x 8192 x 8192 31.1 -> 27.7, 128 x 16384 x 2048 21.3 -> 19.4, 37 x 4096 x 7168 15.1 -> 14.8;
-// 0.85 to 1.01 over 40 shapes. Tile rows drift apart along a long K, most of all where the last is ragged and runs ahead, and a
-// panel that one has let go comes from HBM again for the next: 300 x 8192 x 5120 in FP8 28.3 -> 33.1, 16-bit 300 x 5000 x 7168 in two
-// parts 36.0 -> 44.9, where 256 rows, in step, gain 1 to 5 %; parts of a longer K do too (200 x 4096 x 10240 in four 24.4 -> 25.7); five tile rows and more are on two XCDs (900 x 3072 x 7168 on 64 x 192
-// 62 -> 76.5). Smaller weights may still be in the cache (0.91 to 1.11 by what else the program does: 256 x 4096 x 7168 in FP8 19.6 ->
-// 21.4, 32 x 4096 x 7168 10.2 -> 9.5).
+// Whether a ring tile's copies of the weights carry the non-temporal hint: so many weights that the 256 MB memory-side cache cannot
+// hold them until their next use even in a program that goes round three such matrices, and each panel read once, by one tile
+// row, or by a few that stay together because a row of K (`row_bytes`) is short. Such weights gain nothing from that cache, and left
+// out of it they stream at 6.6 TB/s instead of 5.9: masked 32 groups x 8 rows x 4096 x 7168 158 -> 141 us, 8 x 30 rows 44 -> 40, contiguous
+// 64 x 64 rows x 2048 x 4096 60.6 -> 57.7, FP8 64 x 16384 x 7168 26.8 -> 24.0, 16-bit 16 x 16384 x 4096 22.6 -> 19.6.
+// Smaller ones may still be in the cache. From 32 MB on they gain as much where they are not (16-bit 32 x 8192 x 8192 31.1 -> 27.7, 37 x
+// 4096 x 7168 15.1 -> 14.8) but lose more where they are (going round three: 16-bit 128 x 12288 x 2048 12.0 -> 17.6, FP8 16 x 16384 x
+// 4096 13.4 -> 16.0, contiguous 32 x 64 rows x 2048 x 2048 14.7 -> 16.9). Tile rows drift apart along a long K, most of all where the last
+// is ragged and runs ahead, and a panel that one has let go comes from HBM again for the next: FP8 300 x 8192 x 5120 28.3 -> 33.1,
+// 16-bit 300 x 5000 x 7168 36.0 -> 44.9, where 256 rows, in step, gain 1 to 5 %; five tile rows and more are on two XCDs (900 x 3072 x
+// 7168 on 64 x 192 62 -> 76.5).
 __host__ __device__ constexpr bool streams_weights(int tile_rows, uint64_t weight_bytes, int row_bytes) {
-    return (tile_rows <= 1 || (tile_rows <= 4 && row_bytes <= 4096)) && weight_bytes >= (uint64_t(32) << 20);
+    return (tile_rows <= 1 || (tile_rows <= 4 && row_bytes <= 4096)) && weight_bytes >= (uint64_t(96) << 20);
 }
 
 // Split-K workspaces (fp8_gemm.hpp, bf16_gemm.hpp): the arrival counters take the first kSplitKCounterBytes whatever the
