@@ -334,6 +334,11 @@ CAPPED_SHAPES = [(2048, 4096, 1024), (512, 4096, 2048), (300, 2112, 640)]
 DENSE_RAGGED_CAP_CASE = ([(128, 128), (128, 192), (64, 64), (256, 128)], (390, 516), (72, 200), 8)
 
 
+# Rows a multiple of 16 KB apart, whose tiles start at different places along K: (tile, parts of K), rows, columns, depth
+ROTATED_CASES = [((64, 64), 1), ((64, 64), 4), ((128, 128), 2), ((64, 128), 3)]
+ROTATED_SIZES = (77, 1412, 8192)
+
+
 # Outputs whose rows are no multiple of 16 bytes, on every width of the 256-row kernels and two ring tiles: tiles, rows, columns, depths
 # (whole k-tiles: the 4-wave kernel, else the 8-wave one)
 RAGGED_ROWS_CASE = ([(256, 256), (256, 224), (256, 192), (256, 160), (128, 192), (64, 64)], 259, (4, 12, 132, 236, 772), (320, 264))
@@ -528,6 +533,9 @@ def jit_kernels_in_use(num_cus: int = 256):
         for k in depths:
             name, keys, arg_defs, code_template = fp8_explicit_tile_plan(*tile, FP8_SHORT_K_SIZES[1], k)
             add(name, arg_defs, gemm.includes, code_template, keys)
+    for tile, split_k in ROTATED_CASES:
+        name, keys, arg_defs, includes, code_template = stream_plans('dense', tile, split_k, 0)
+        add(name, arg_defs, includes, code_template, keys)
     for tile in RAGGED_ROWS_CASE[0]:
         for dtype in (torch.bfloat16, torch.half):
             name, keys, arg_defs, includes, code_template = dense_tile_plan(tile, dtype, 0)

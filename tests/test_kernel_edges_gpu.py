@@ -334,3 +334,24 @@ def test_output_rows_that_end_inside_a_16_byte_store(tile, dtype):
             torch.cuda.synchronize()
             assert torch.equal(room[:m * n].view(m, n), whole[:, :n])
             assert (room[m * n:] == -7.0).all()
+
+
+@pytest.mark.parametrize('tile,split_k', testing.ROTATED_CASES)
+def test_dense_tiles_that_start_at_different_places_along_k(tile, split_k):
+    m, n, k = testing.ROTATED_SIZES
+    _announce('rotated', tile, split_k)
+    a, b, c = testing.make_bf16_case(m, n, k, seed=22, device='cuda')
+    name, keys, arg_defs, includes, code_template = testing.stream_plans('dense', tile, split_k, 0)
+    kernel = jit.build(name, arg_defs, jit.generate(includes, arg_defs, jit.cpp_format(code_template, keys)))
+    workspace = torch.zeros(16384 + 256 * 128 * 128 * 4, dtype=torch.uint8, device='cuda')
+    results = []
+    for _ in range(2):
+        c.fill_(float('nan'))
+        assert kernel(m, n, k, a, b, c, torch.cuda.current_stream(), *((workspace, workspace.numel()) if split_k > 1 else ())) == 0
+        torch.cuda.synchronize()
+        results.append(c.cpu())
+    assert torch.equal(results[0], results[1])
+    # bf16 rounding, and fp32 sums of k products: k * 2^-24 of the sum of their magnitudes at the most
+    a64, b64 = a.double(), b.double()
+    bound = (a64 @ b64.t()).abs() * 2.0 ** -8 + (a64.abs() @ b64.abs().t()) * (k * 2.0 ** -24)
+    assert ((c.double() - a64 @ b64.t()).abs() <= bound).all()
