@@ -89,8 +89,11 @@ __host__ __device__ constexpr int dense_launch_waves(int block_m, int block_n, i
     return block_m * block_n >= 128 * 128 && split_k >= 4 ? 4 : 8;
 }
 
-// STREAM: the copies of B carry the non-temporal hint (streams_weights in scheduler.hpp).
-template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K = 1, bool STREAM = false>
+// COPIES: how a ring tile's copies go about K and B, chosen by the launcher (with_dense_copies): bits kStreamedWeights, the copies of B
+// carry the non-temporal hint (streams_weights in scheduler.hpp), and kSpreadStarts. Compiled in, since looking at a start in
+// every k-tile cost the depths that have none 1 to 4 % (90 x 5004 x 2048 9.4 -> 9.8 us, 37 x 4096 x 7168 15.1 -> 15.3).
+constexpr int kStreamedWeights = 1, kSpreadStarts = 2;
+template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K = 1, int COPIES = 0>
 __device__ __forceinline__ void
 dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, Elem* __restrict__ C,
                 int m, int n, int k, int bid, float* __restrict__ partials = nullptr, unsigned* __restrict__ counters = nullptr) {
@@ -115,7 +118,7 @@ dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
     const __amdgpu_buffer_rsrc_t rsrc_a = make_rsrc(A, uint32_t(m) * ld_bytes);
     const __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(B, uint32_t(n) * ld_bytes);
     TileStager<BLOCK_M, LW> stage_a;
-    TileStager<BLOCK_N, LW, STREAM> stage_b;
+    TileStager<BLOCK_N, LW, (COPIES & kStreamedWeights) != 0> stage_b;
     stage_a.init(m0, ld_bytes, wave, lane);
     stage_b.init(n0, ld_bytes, wave, lane);
 
@@ -137,16 +140,20 @@ dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
     constexpr int NUM_COPIES = StA::PASSES + StB::PASSES;
     static_assert(StA::PADDED_ROWS == BLOCK_M && StB::PADDED_ROWS == BLOCK_N, "tiles are whole copy passes");
     // Workgroups march along K in step. Where rows are a multiple of 16 KB apart, one k-tile of all rows lies in a few of the memory
-    // channels, which all of them then ask at a time: there column c of the tiles starts 5 c k-tiles into its range and comes
-    // round to them at the end. 37 x 4096 x 8192 20.2 -> 16.8 us, 37 x 16384 x 8192 50.2 -> 41.2, 37 x 4096 x 16384 30.9 -> 25.6, 128 x
-    // 8192 x 8192 38.5 -> 34.7. At other depths it changes nothing (K = 7168) or loses 1 % (4096), as with many tile rows, which share
-    // panels that some have passed then (1024 x 4096 x 8192 75.5 -> 76.3).
-    const int range = kt_hi - kt_lo, first = ld_bytes % 16384 == 0 && sched.tiles_m <= 4 && range > 0 ? tile.n_idx * 5 % range : 0;
+    // channels, which all of them then ask at a time: there (kSpreadStarts) the columns of the tiles start at places spread over
+    // their range, multiples of the golden ratio, and come round to the k-tiles in front at the end. 37 x 4096 x 8192 20.2 -> 16.8 us,
+    // 37 x 16384 x 8192 56.7 -> 41.6, 37 x 4096 x 16384 35.6 -> 26.6, 128 x 8192 x 8192 42.0 -> 37.9. At other depths it changes nothing
+    // (K = 7168) or loses 1 % (4096), as with many tile rows, which share panels that some have passed then (1024 x 4096 x 8192
+    // 75.5 -> 76.3).
+    constexpr bool SPREAD = (COPIES & kSpreadStarts) != 0;
+    const int range = kt_hi - kt_lo, first = SPREAD && range > 0 ? int(__umulhi(uint32_t(tile.n_idx) * 0x9e3779b9u, uint32_t(range))) : 0;
     // Copy number `d` (A passes first, then B passes) of the `kt`-th k-tile into the given stage.
     auto copy_pass = [&](int d, int kt, uint8_t* la, uint8_t* lb) {
         const bool live = kt < kt_hi;
-        kt += first;
-        if (kt >= kt_hi) kt -= range;
+        if constexpr (SPREAD) {
+            kt += first;
+            if (kt >= kt_hi) kt -= range;
+        }
         const bool tail = kt == tail_tile;
         if (d < StA::PASSES) stage_a.issue_pass_from(live ? rsrc_a : rsrc_none, la, kt * kRowBytes, wave, d, tail ? tail_a : stage_a.voff);
         else stage_b.issue_pass_from(live ? rsrc_b : rsrc_none, lb, kt * kRowBytes, wave, d - StA::PASSES, tail ? tail_b : stage_b.voff);
@@ -859,47 +866,47 @@ dense_gemm_mfma_8w(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
 // Workgroup b runs tiles b, b + gridDim.x, ...: exactly one when the launcher starts a workgroup per tile, several under
 // a compute-unit cap. Between two tiles every wave must have left the epilogue of the first, which reads an LDS stage
 // the second one's first copies go into.
-template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES, bool STREAM>
+template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES, int COPIES>
 __device__ __forceinline__ void
 dense_gemm_walk(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, Elem* __restrict__ C, int m, int n, int k, int num_slots) {
     // a workgroup per tile (no cap): the tile without a loop around it (up to 2 % faster than one trip round the loop below)
     if (int(gridDim.x) >= num_slots) {
-        dense_gemm_body<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, 1, STREAM>(A, B, C, m, n, k, int(blockIdx.x));
+        dense_gemm_body<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, 1, COPIES>(A, B, C, m, n, k, int(blockIdx.x));
         return;
     }
     for (int slot = blockIdx.x; slot < num_slots; slot += gridDim.x) {
-        dense_gemm_body<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, 1, STREAM>(A, B, C, m, n, k, slot);
+        dense_gemm_body<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, 1, COPIES>(A, B, C, m, n, k, slot);
         if (slot + int(gridDim.x) < num_slots) __syncthreads();
     }
 }
 
-template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES, bool STREAM = false>
+template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES, int COPIES = 0>
 __global__ void __launch_bounds__((dense_launch_waves(BLOCK_M, BLOCK_N) * kWaveSize))
 dense_gemm_mfma(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, Elem* __restrict__ C, int m, int n, int k, int num_slots) {
-    dense_gemm_walk<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, STREAM>(A, B, C, m, n, k, num_slots);
+    dense_gemm_walk<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, COPIES>(A, B, C, m, n, k, num_slots);
 }
 
 // The ring tiles with K split SPLIT_K ways: launch slot s is part s % SPLIT_K of tile slot s / SPLIT_K.
-template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K, bool STREAM = false>
+template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K, int COPIES = 0>
 __global__ void __launch_bounds__((dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize))
 dense_gemm_split_k(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, Elem* __restrict__ C, int m, int n, int k,
                    float* __restrict__ partials, unsigned* __restrict__ counters) {
-    dense_gemm_body<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, SPLIT_K, STREAM>(A, B, C, m, n, k, int(blockIdx.x), partials, counters);
+    dense_gemm_body<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, SPLIT_K, COPIES>(A, B, C, m, n, k, int(blockIdx.x), partials, counters);
 }
 
 // The fp16 flavour under the name of the reference's kernel (yan/include/gemm/cute_gemm.cuh:20), so that profiler
 // filters written for it (tests/test_cute.py:35 looks for 'fp16_gemm_cute') keep finding it.
-template <int BLOCK_M, int BLOCK_N, int STAGES, bool STREAM = false>
+template <int BLOCK_M, int BLOCK_N, int STAGES, int COPIES = 0>
 __global__ void __launch_bounds__((dense_launch_waves(BLOCK_M, BLOCK_N) * kWaveSize))
 fp16_gemm_cute(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, _Float16* __restrict__ C, int m, int n, int k, int num_slots) {
-    dense_gemm_walk<MfmaF16_32x32x16, _Float16, BLOCK_M, BLOCK_N, STAGES, STREAM>(A, B, C, m, n, k, num_slots);
+    dense_gemm_walk<MfmaF16_32x32x16, _Float16, BLOCK_M, BLOCK_N, STAGES, COPIES>(A, B, C, m, n, k, num_slots);
 }
 
-template <int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K, bool STREAM = false>
+template <int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K, int COPIES = 0>
 __global__ void __launch_bounds__((dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize))
 fp16_gemm_cute_split_k(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, _Float16* __restrict__ C, int m, int n, int k,
                        float* __restrict__ partials, unsigned* __restrict__ counters) {
-    dense_gemm_body<MfmaF16_32x32x16, _Float16, BLOCK_M, BLOCK_N, STAGES, SPLIT_K, STREAM>(A, B, C, m, n, k, int(blockIdx.x), partials, counters);
+    dense_gemm_body<MfmaF16_32x32x16, _Float16, BLOCK_M, BLOCK_N, STAGES, SPLIT_K, COPIES>(A, B, C, m, n, k, int(blockIdx.x), partials, counters);
 }
 
 template <int BLOCK_N>
@@ -925,6 +932,17 @@ inline hipError_t check_dense_args(int m, int n, int k, const void* a, const voi
     // output stores address a tile with 32-bit byte offsets from its first element: block_m rows of n elements
     if (uint64_t(block_m) * n * 2 >= kOutOfRange) return hipErrorInvalidValue;
     return hipSuccess;
+}
+
+// Calls `launch` with the copies (COPIES, a std::integral_constant) of a ring tile's launch. Why the starts are spread for rows a
+// multiple of 16 KB apart, and up to four tile rows: dense_gemm_body.
+template <typename Launch>
+inline void with_dense_copies(int tiles_m, int n, int k, Launch&& launch) {
+    const bool streamed = streams_weights(tiles_m, uint64_t(n) * k * 2, k * 2), spread = k % 8192 == 0 && tiles_m <= 4;
+    if (streamed && spread) launch(std::integral_constant<int, kStreamedWeights | kSpreadStarts>{});
+    else if (streamed) launch(std::integral_constant<int, kStreamedWeights>{});
+    else if (spread) launch(std::integral_constant<int, kSpreadStarts>{});
+    else launch(std::integral_constant<int, 0>{});
 }
 
 // `num_sms`: the caller's compute-unit cap (0 = none), see capped_grid in scheduler.hpp.
@@ -966,19 +984,18 @@ inline hipError_t launch_dense(int m, int n, int k, const void* a, const void* b
                                static_cast<Elem*>(c), m, n, k);
     } else {
         const int grid = capped_grid(slots, num_sms, device_cu_count());
-        auto launch = [&](auto stream_weights) {
-            constexpr bool STREAM = decltype(stream_weights)::value;
+        auto launch = [&](auto copies) {
+            constexpr int COPIES = decltype(copies)::value;
             if constexpr (__is_same(Elem, _Float16))
-                hipLaunchKernelGGL((fp16_gemm_cute<BLOCK_M, BLOCK_N, STAGES, STREAM>), dim3(grid),
+                hipLaunchKernelGGL((fp16_gemm_cute<BLOCK_M, BLOCK_N, STAGES, COPIES>), dim3(grid),
                                    dim3(dense_launch_waves(BLOCK_M, BLOCK_N) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
                                    static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, slots);
             else
-                hipLaunchKernelGGL((dense_gemm_mfma<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, STREAM>), dim3(grid),
+                hipLaunchKernelGGL((dense_gemm_mfma<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, COPIES>), dim3(grid),
                                    dim3(dense_launch_waves(BLOCK_M, BLOCK_N) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
                                    static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, slots);
         };
-        if (streams_weights(sched.tiles_m, uint64_t(n) * k * 2, k * 2)) launch(std::true_type{});
-        else launch(std::false_type{});
+        with_dense_copies(sched.tiles_m, n, k, launch);
     }
     return hipGetLastError();
 }
@@ -1000,19 +1017,18 @@ inline hipError_t launch_dense_split_k(int m, int n, int k, const void* a, const
     if (workspace_bytes < kSplitKCounterBytes + slots * SPLIT_K * BLOCK_M * BLOCK_N * 4) return hipErrorInvalidValue;
     unsigned* counters = static_cast<unsigned*>(workspace);
     float* partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kSplitKCounterBytes);
-    auto launch = [&](auto stream_weights) {
-        constexpr bool STREAM = decltype(stream_weights)::value;
+    auto launch = [&](auto copies) {
+        constexpr int COPIES = decltype(copies)::value;
         if constexpr (__is_same(Elem, _Float16))
-            hipLaunchKernelGGL((fp16_gemm_cute_split_k<BLOCK_M, BLOCK_N, STAGES, SPLIT_K, STREAM>), dim3(int(slots) * SPLIT_K),
+            hipLaunchKernelGGL((fp16_gemm_cute_split_k<BLOCK_M, BLOCK_N, STAGES, SPLIT_K, COPIES>), dim3(int(slots) * SPLIT_K),
                                dim3(dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
                                static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, partials, counters);
         else
-            hipLaunchKernelGGL((dense_gemm_split_k<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, SPLIT_K, STREAM>), dim3(int(slots) * SPLIT_K),
+            hipLaunchKernelGGL((dense_gemm_split_k<Atom, Elem, BLOCK_M, BLOCK_N, STAGES, SPLIT_K, COPIES>), dim3(int(slots) * SPLIT_K),
                                dim3(dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
                                static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, partials, counters);
     };
-    if (streams_weights(sched.tiles_m, uint64_t(n) * k * 2, k * 2)) launch(std::true_type{});
-    else launch(std::false_type{});
+    with_dense_copies(sched.tiles_m, n, k, launch);
     return hipGetLastError();
 }
 
