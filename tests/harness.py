@@ -313,6 +313,10 @@ FP8_SHORT_K_SIZES = (390, 516)
 # fetches for the next one (two of them) and where one does not; tiles whose copies are handed out one and several to a row
 FP8_WALK_CASES = [((256, 256), (256, 384)), ((256, 224), (256, )), ((256, 160), (256, 384)), ((128, 256), (256, 384)), ((64, 64), (384, ))]
 FP8_WALK_SIZES = (1300, 772)
+# Tiles on two stages whose slabs are 16 columns wide: a workgroup per tile whatever K, stored straight from the accumulators
+FP8_NARROW_TWO_STAGE_CASES = [((16, 64), (128, 384, 512)), ((48, 64), (384, )), ((80, 64), (256, )), ((32, 32), (384, 512)),
+                              ((160, 32), (384, )), ((256, 16), (256, 384)), ((96, 32), (640, ))]
+FP8_NARROW_TWO_STAGE_SIZES = (333, 172)
 GROUPED_MASKED_TEST_CASES = [
     (3, 200, 320, 384, (200, 0, 77), 128), (4, 256, 4096, 1024, (1, 256, 130, 64), 64), (2, 64, 200, 128, (64, 3), 32),
     (4, 1024, 4096, 7168, (1024, 900, 512, 1), 1024),
@@ -559,6 +563,10 @@ def jit_kernels_in_use(num_cus: int = 256):
     for tile, depths in FP8_WALK_CASES:
         for k in depths:
             name, keys, arg_defs, code_template = fp8_explicit_tile_plan(*tile, FP8_WALK_SIZES[1], k, 2)
+            add(name, arg_defs, gemm.includes, code_template, keys)
+    for tile, depths in FP8_NARROW_TWO_STAGE_CASES:
+        for k in depths:
+            name, keys, arg_defs, code_template = fp8_explicit_tile_plan(*tile, FP8_NARROW_TWO_STAGE_SIZES[1], k, 2)
             add(name, arg_defs, gemm.includes, code_template, keys)
     for m, n, k in list(FLOAT_SPLIT_K_SHAPES) + REFERENCE_FLOAT_TEST_SHAPES + FLOAT_TEST_SHAPES:
         plan = simple_gemm.float_split_k_plan(m, n, k, num_cus)

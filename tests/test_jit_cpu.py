@@ -174,6 +174,16 @@ def test_gemm_kernels_compile_for_gfx950(cache_dir):
     assert runtime.Runtime.is_path_valid(rt.path)
 
 
+@pytest.mark.parametrize('tile,k', [((16, 64), 384), ((32, 32), 512)])
+def test_fp8_tiles_with_narrow_slabs_compile_on_two_stages(cache_dir, tile, k):
+    import harness as testing
+    from yan_amd.jit_kernels import gemm
+    assert (tile, k) in [(t, d) for t, depths in testing.FP8_NARROW_TWO_STAGE_CASES for d in depths]
+    name, keys, defs, tmpl = testing.fp8_explicit_tile_plan(*tile, testing.FP8_NARROW_TWO_STAGE_SIZES[1], k, 2)
+    rt = jit.build(name, defs, jit.generate(gemm.includes, defs, jit.cpp_format(tmpl, keys)))
+    assert runtime.Runtime.is_path_valid(rt.path)
+
+
 def test_runtime_call_takes_subclasses_the_checked_way(cache_dir):
     # plain tensors, ints and floats go through the call written for the kernel's arguments, everything else through the loop
     args = (('n', int), ('x', float), ('data', torch.int), ('stream', torch.cuda.Stream))

@@ -94,6 +94,25 @@ def test_fp8_walk_over_several_tiles_of_few_k_tiles(tile, k):
     assert _fp8_close(results[0].float(), ref)
 
 
+@pytest.mark.parametrize('tile,k', [(tile, k) for tile, depths in testing.FP8_NARROW_TWO_STAGE_CASES for k in depths])
+def test_fp8_two_stage_tiles_with_slabs_of_16_columns(tile, k):
+    from yan_amd.jit_kernels import gemm
+    m, n = testing.FP8_NARROW_TWO_STAGE_SIZES
+    _announce('fp8 narrow', tile, k)
+    (a8, sa), (b8, sb), out = testing.make_fp8_case(m, n, k, seed=23, device='cuda')
+    name, keys, arg_defs, code_template = testing.fp8_explicit_tile_plan(*tile, n, k, 2)
+    kernel = jit.build(name, arg_defs, jit.generate(gemm.includes, arg_defs, jit.cpp_format(code_template, keys)))
+    ref = torch.from_numpy(oracle.gemm_fp8_block_scaled_ref(_codes(a8), sa.cpu().numpy(), _codes(b8), sb.cpu().numpy()))
+    sa_t, results = yan.get_col_major_tensor(sa), []
+    for cap in (0, 8):
+        out.fill_(float('nan'))
+        assert kernel(a8, sa_t, b8, sb, out, m, torch.cuda.current_stream(), cap, 0) == 0
+        torch.cuda.synchronize()
+        results.append(out.cpu())
+    assert torch.equal(results[0], results[1])
+    assert _fp8_close(results[0].float(), ref)
+
+
 @pytest.mark.parametrize('tile,k', [(tile, k) for tile, depths in testing.FP8_SHORT_K_TILES for k in depths])
 def test_fp8_tiles_on_either_side_of_a_change_of_their_k_loop(tile, k):
     m, n = testing.FP8_SHORT_K_SIZES

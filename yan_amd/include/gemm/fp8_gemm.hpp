@@ -702,10 +702,12 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     }
 }
 
-// Whether a problem runs the persistent walk below: the plain GEMM on two LDS stages (three of the weights) with two k-tiles or more.
+// Whether a problem runs the persistent walk below: the plain GEMM on two LDS stages (three of the weights) with two k-tiles or
+// more, on tiles whose slabs are wide enough for the staged epilogue the walk ends a tile with.
 template <int BLOCK_M, int BLOCK_N, int STAGES, GemmType kGemmType>
 __host__ __device__ constexpr bool fp8_walks(int k) {
-    return STAGES == 2 && kGemmType == GemmType::Normal && Fp8TileConfig<BLOCK_M, BLOCK_N>::DEEP_B_CAPABLE && k >= 256;
+    using Cfg = Fp8TileConfig<BLOCK_M, BLOCK_N>;
+    return STAGES == 2 && kGemmType == GemmType::Normal && Cfg::DEEP_B_CAPABLE && Cfg::WTN >= 32 && k >= 256;
 }
 
 // The plain GEMM on two LDS stages as a persistent walk: workgroup b takes slots b, b + gridDim.x, ... (the launcher
