@@ -311,7 +311,7 @@ FP8_SHORT_K_TILES = [((64, 64), (128, 2048, 2176)), ((64, 128), (256, 1536, 1664
 FP8_SHORT_K_SIZES = (390, 516)
 # Tiles on two stages (three of the weights) that are walked, several to a workgroup: the seam between two tiles where every k-tile
 # fetches for the next one (two of them) and where one does not; tiles whose copies are handed out one and several to a row
-FP8_WALK_CASES = [((256, 256), (256, 384)), ((256, 224), (256, )), ((256, 160), (256, 384)), ((128, 256), (256, 384)), ((64, 64), (384, ))]
+FP8_WALK_CASES = [((256, 256), (256, 384, 512)), ((256, 224), (256, )), ((256, 160), (256, 384)), ((128, 256), (256, 384)), ((64, 64), (384, ))]
 FP8_WALK_SIZES = (1300, 772)
 # Tiles on two stages whose slabs are 16 columns wide: a workgroup per tile whatever K, stored straight from the accumulators
 FP8_NARROW_TWO_STAGE_CASES = [((16, 64), (128, 384, 512)), ((48, 64), (384, )), ((80, 64), (256, )), ((32, 32), (384, 512)),

@@ -184,6 +184,29 @@ def test_fp8_tiles_with_narrow_slabs_compile_on_two_stages(cache_dir, tile, k):
     assert runtime.Runtime.is_path_valid(rt.path)
 
 
+def _scratch_bytes(cache_dir, includes, defs, tmpl, keys):
+    """Scratch memory a lane of each kernel of this source asks for, as the compiler reports it."""
+    src = cache_dir / f'scratch_{abs(hash(str(sorted(keys.items()))))}.hip'
+    src.write_text(jit.generate(includes, defs, jit.cpp_format(tmpl, keys)))
+    flags = [f for f in compiler.get_compile_flags() if f != '-shared']
+    done = subprocess.run([compiler.get_hipcc_compiler()[0], '-x', 'hip', str(src), '-c', '--offload-device-only', '-o', str(src) + '.o', *flags,
+                           f'-I{compiler.get_jit_include_dir()}', '-Rpass-analysis=kernel-resource-usage'],
+                          stdout=subprocess.PIPE, stderr=subprocess.STDOUT, universal_newlines=True)
+    assert done.returncode == 0, done.stdout[-2000:]
+    return [int(line.split(':')[-1].split()[0]) for line in done.stdout.splitlines() if 'ScratchSize' in line]
+
+
+def test_fp8_walks_of_few_k_tiles_fit_their_registers(cache_dir):
+    """Their loops have no trip, one or a few, which the compiler may take out and then run out of registers."""
+    from concurrent.futures import ThreadPoolExecutor
+    import harness as testing
+    from yan_amd.jit_kernels import gemm
+    plans = [testing.fp8_explicit_tile_plan(256, 256, 7168, k, 2) for k in (256, 384, 512, 640)]
+    with ThreadPoolExecutor(4) as pool:
+        scratch = list(pool.map(lambda p: _scratch_bytes(cache_dir, gemm.includes, p[2], p[3], p[1]), plans))
+    assert all(len(s) == 1 for s in scratch) and sum(scratch, []) == [0] * len(plans)
+
+
 def test_runtime_call_takes_subclasses_the_checked_way(cache_dir):
     # plain tensors, ints and floats go through the call written for the kernel's arguments, everything else through the loop
     args = (('n', int), ('x', float), ('data', torch.int), ('stream', torch.cuda.Stream))

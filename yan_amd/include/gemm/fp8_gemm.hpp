@@ -845,6 +845,9 @@ fp8_gemm_walk(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
         // k-tile 0 has landed for every wave: the barrier in front of the loop, or the one in front of the last epilogue
         k_step.template operator()<true, false>(cur, nxt, 0);
         int kb = 1;
+        // a loop of one trip is compiled without the loop, and the k-steps of 256 x 256 tiles in one piece spill 47 registers
+        // (4096 x 7168 x 512 33 us, 22 as a loop)
+        if constexpr (SHAPE_K == 512) asm volatile("" : "+s"(kb));
         // two at a time where K is long (1-1.5 %: 4096 x 4096 x 7168 101.0 -> 99.5 us; compiled in and short, the compiler unrolls
         // the rest of it as well and spills)
         if constexpr (SHAPE_K >= 2048) {
