@@ -195,6 +195,15 @@ int main() {
         CHECK(e.region_rows == 32 && e.rows_outer);          // the FP8 16384^3 shape
         CHECK(region_cases > 100 && halved_cases > 10);
     }
+    {
+        // Outputs the walk stores with the non-temporal hint: from past 64 MB, behind a long K from past 32 MB.
+        const int m = 0, n = 0, bm = 256, bn = 256;
+        const uint64_t mb = uint64_t(1) << 20;
+        CHECK(!yan::fp8_walk_streams_output(2ull * 8192 * 2560, 1024) && !yan::fp8_walk_streams_output(2ull * 4096 * 7168, 512));
+        CHECK(yan::fp8_walk_streams_output(2ull * 8192 * 7168, 512) && yan::fp8_walk_streams_output(2ull * 4096 * 7168, 7168));
+        CHECK(!yan::fp8_walk_streams_output(64 * mb, 2944) && yan::fp8_walk_streams_output(64 * mb + 8, 2944));
+        CHECK(!yan::fp8_walk_streams_output(32 * mb, 3072) && yan::fp8_walk_streams_output(32 * mb + 8, 3072));
+    }
     std::printf("ok %d\n", cases);
     return 0;
 }

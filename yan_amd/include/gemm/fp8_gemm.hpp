@@ -17,7 +17,8 @@
 //     meets one activation row per atom: one sA per lane per atom per K block, and sB is wave-uniform;
 //   * the running sums stay in architectural VGPRs (the VALU cannot address AGPRs): 128 per wave;
 //   * the output leaves through LDS: each wave turns its slab round through the stage that was consumed last and stores
-//     16 bytes per lane in row runs of 2 * WTN bytes (non-temporal when the output is larger than the L2s together);
+//     16 bytes per lane in row runs of 2 * WTN bytes (non-temporal when the output is larger than the L2s together; in the
+//     walk from 64 MB on, or 32 MB behind a long K);
 //   * the plain GEMM on the 256-row tiles is a persistent walk: one workgroup per compute unit takes tile after tile and
 //     overlaps the seams (fp8_gemm_walk); every other case runs a workgroup per tile, or a plain loop under a cap;
 //   * problems with long K and fewer tiles than compute units split K over SPLIT_K workgroups per tile on the ring tiles
@@ -720,8 +721,8 @@ __host__ __device__ constexpr bool fp8_walks(int k) {
 // Bound by the matrix cores and, under load, by energy (a tile's time at the clock the power allows). What a first pass over
 // new operands adds is waiting for HBM, which one k-tile of prefetch does not cover: weights are fetched two k-tiles ahead into
 // a third stage, and activations handed out first (row_of_deep_copy). The k-tiles that fetch for their own tile are a loop of
-// their own, without the selects of the last two (2 % of a k-tile), and outputs larger than the L2s together are stored with the
-// non-temporal hint (2-7 %; with the same operands call after call plain stores were 1 % faster). Inputs changing from call to
+// their own, without the selects of the last two (2 % of a k-tile), and large outputs are stored with the non-temporal hint
+// (fp8_walk_streams_output in scheduler.hpp; with the same operands call after call plain stores were 1 % faster). Inputs changing from call to
 // call, two stages and plain stores before -> now: 4096 x 7168 x 7168 189 -> 178 us, 8192 x 7168 x 7168 371 -> 350, 8192 x 2112 x
 // 7168 on 256 x 160 tiles 159 -> 140, 4096 x 24576 x 1536 159 -> 143, 3529 x 7616 x 1024 39.8 -> 33.3, one round of tiles
 // (4096 x 4096 x 7168) 101.8 -> 100.8; twelve shapes 0.92 on average, an odd number of k-tiles (3529 x 7616 x 896, a workgroup per tile
@@ -753,8 +754,7 @@ fp8_gemm_walk(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
     const __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(rhs, uint32_t(N) * K);
     const uint32_t sa_bytes = (uint32_t(m - 1) * sa_stride_m + uint32_t(NUM_K_BLOCKS - 1) * sa_stride_k + 1) * 4;
     const __amdgpu_buffer_rsrc_t rsrc_sa = make_rsrc(lhs_scales, sa_bytes);
-    // as in fp8_gemm_tile: an output larger than the L2s together must not push the operand panels out of them
-    const bool stream_out = size_t(m) * N * 2 > (size_t(32) << 20);
+    const bool stream_out = fp8_walk_streams_output(uint64_t(m) * N * 2, K);
 
     struct TileIo {
         int m0, n0;

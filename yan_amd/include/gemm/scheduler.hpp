@@ -237,6 +237,15 @@ __host__ __device__ inline int capped_grid(int slots, int num_sms, int device_cu
     return num_sms >= kNumXCD ? num_sms / kNumXCD * kNumXCD : num_sms;
 }
 
+// Whether the persistent FP8 walk stores its output (`bytes`) with the non-temporal hint: outputs that would push the operands out of
+// the 256 MB memory-side cache, from 64 MB on whatever K, from 32 MB on where the k-loop is long (operands many times the output).
+// Plain -> hint, inputs changing: 8192 x 7168 x 768 57.4 -> 54.7 us, 4096 x 16384 x 3072 184.7 -> 175.2, 2048 x 12288 x 4096
+// 100.8 -> 96.4, 4096 x 7168 x 7168 183.5 -> 177.3. Outputs of 32 to 64 MB behind a short K are quick to write and stay in that
+// cache: 8192 x 2560 x 1024 27.1 -> 29.9, 4096 x 4608 x 768 21.8 -> 23.5, 2048 x 12288 x 2048 53.2 -> 54.7.
+__host__ __device__ constexpr bool fp8_walk_streams_output(uint64_t bytes, int k) {
+    return bytes > (uint64_t(k >= 3072 ? 32 : 64) << 20);
+}
+
 // Whether a ring tile's copies of the weights carry the non-temporal hint: so many weights that the 256 MB memory-side cache cannot
 // hold them until their next use even in a program that goes round three such matrices, and each panel read once, by one tile
 // row, or by a few that stay together because a row of K (`row_bytes`) is short. Such weights gain nothing from that cache, and left
