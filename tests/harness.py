@@ -313,6 +313,8 @@ FP8_SHORT_K_SIZES = (390, 516)
 # fetches for the next one (two of them) and where one does not; tiles whose copies are handed out one and several to a row
 FP8_WALK_CASES = [((256, 256), (256, 384, 512)), ((256, 224), (256, )), ((256, 160), (256, 384)), ((128, 256), (256, 384)), ((64, 64), (384, ))]
 FP8_WALK_SIZES = (1300, 772)
+# Few k-tiles, an odd number: an output of more than 64 MB is walked, its halves along n run a workgroup per tile
+FP8_ODD_K_TILE, FP8_ODD_K_SIZES = (256, 256), (5000, 6912, (384, 640))
 # Tiles on two stages whose slabs are 16 columns wide: a workgroup per tile whatever K, stored straight from the accumulators
 FP8_NARROW_TWO_STAGE_CASES = [((16, 64), (128, 384, 512)), ((48, 64), (384, )), ((80, 64), (256, )), ((32, 32), (384, 512)),
                               ((160, 32), (384, )), ((256, 16), (256, 384)), ((96, 32), (640, ))]
@@ -563,6 +565,10 @@ def jit_kernels_in_use(num_cus: int = 256):
     for tile, depths in FP8_WALK_CASES:
         for k in depths:
             name, keys, arg_defs, code_template = fp8_explicit_tile_plan(*tile, FP8_WALK_SIZES[1], k, 2)
+            add(name, arg_defs, gemm.includes, code_template, keys)
+    for k in FP8_ODD_K_SIZES[2]:
+        for n in (FP8_ODD_K_SIZES[1], FP8_ODD_K_SIZES[1] // 2):
+            name, keys, arg_defs, code_template = fp8_explicit_tile_plan(*FP8_ODD_K_TILE, n, k, 2)
             add(name, arg_defs, gemm.includes, code_template, keys)
     for tile, depths in FP8_NARROW_TWO_STAGE_CASES:
         for k in depths:

@@ -199,6 +199,9 @@ int main() {
         // Outputs the walk stores with the non-temporal hint: from past 64 MB, behind a long K from past 32 MB.
         const int m = 0, n = 0, bm = 256, bn = 256;
         const uint64_t mb = uint64_t(1) << 20;
+        // Problems that walk: not the odd numbers of up to 17 k-tiles, unless the output is large.
+        CHECK(!yan::fp8_walk_pays(384, 64 * mb) && !yan::fp8_walk_pays(640, 2ull * 7902 * 2624) && !yan::fp8_walk_pays(2176, 0));
+        CHECK(yan::fp8_walk_pays(384, 64 * mb + 8) && yan::fp8_walk_pays(2432, 0) && yan::fp8_walk_pays(256, 0) && yan::fp8_walk_pays(2048, 0));
         CHECK(!yan::fp8_walk_streams_output(2ull * 8192 * 2560, 1024) && !yan::fp8_walk_streams_output(2ull * 4096 * 7168, 512));
         CHECK(yan::fp8_walk_streams_output(2ull * 8192 * 7168, 512) && yan::fp8_walk_streams_output(2ull * 4096 * 7168, 7168));
         CHECK(!yan::fp8_walk_streams_output(64 * mb, 2944) && yan::fp8_walk_streams_output(64 * mb + 8, 2944));

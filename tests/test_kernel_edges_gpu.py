@@ -94,6 +94,37 @@ def test_fp8_walk_over_several_tiles_of_few_k_tiles(tile, k):
     assert _fp8_close(results[0].float(), ref)
 
 
+@pytest.mark.parametrize('k', testing.FP8_ODD_K_SIZES[2])
+def test_fp8_few_k_tiles_an_odd_number_of_them_give_the_same_bits_walked_or_not(k):
+    from yan_amd import capi
+    from yan_amd.jit_kernels import gemm
+    m, n, _ = testing.FP8_ODD_K_SIZES
+    _announce('fp8 odd k-tiles', k)
+    assert m * n * 2 > 64 << 20 >= m * n
+    (a8, sa), (b8, sb), _ = testing.make_fp8_case(m, n, k, seed=24, device='cuda', gen_device='cuda')
+    sa = yan.get_col_major_tensor(sa)
+    outs = []
+    for lo, hi in ((0, n), (0, n // 2), (n // 2, n)):
+        name, keys, arg_defs, code_template = testing.fp8_explicit_tile_plan(*testing.FP8_ODD_K_TILE, hi - lo, k, 2)
+        kernel = jit.build(name, arg_defs, jit.generate(gemm.includes, arg_defs, jit.cpp_format(code_template, keys)))
+        outs.append(torch.full((m, hi - lo), float('nan'), dtype=torch.bfloat16, device='cuda'))
+        assert kernel(a8, sa, b8[lo:hi], sb[lo // 128:hi // 128], outs[-1], m, torch.cuda.current_stream(), 0, 0) == 0
+        torch.cuda.synchronize()
+    assert torch.equal(outs[0], torch.cat(outs[1:], dim=1))
+    # the library, whose kernel finds out when it runs
+    via_lib = torch.full_like(outs[0], float('nan'))
+    assert capi.gemm_fp8_fp8_bf16_nt((a8, sa), (b8, sb), via_lib) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(via_lib, outs[0])
+    half = torch.full_like(outs[1], float('nan'))
+    assert capi.gemm_fp8_fp8_bf16_nt((a8, sa), (b8[:n // 2], sb[:n // 2 // 128]), half) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(half, outs[1])
+    rows = slice(0, m, 127)
+    ref = testing.dequant_lhs(a8[rows], sa[rows].contiguous()) @ testing.dequant_rhs(b8, sb).t()
+    assert _fp8_close(outs[0][rows].float(), ref)
+
+
 @pytest.mark.parametrize('tile,k', [(tile, k) for tile, depths in testing.FP8_NARROW_TWO_STAGE_CASES for k in depths])
 def test_fp8_two_stage_tiles_with_slabs_of_16_columns(tile, k):
     from yan_amd.jit_kernels import gemm

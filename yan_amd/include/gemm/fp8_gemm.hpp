@@ -707,11 +707,12 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
 }
 
 // Whether a problem runs the persistent walk below: the plain GEMM on two LDS stages (three of the weights) with two k-tiles or
-// more, on tiles whose slabs are wide enough for the staged epilogue the walk ends a tile with.
+// more, on tiles whose slabs are wide enough for the staged epilogue the walk ends a tile with, where it pays
+// (fp8_walk_pays in scheduler.hpp; `output_bytes` decides only where K does not).
 template <int BLOCK_M, int BLOCK_N, int STAGES, GemmType kGemmType>
-__host__ __device__ constexpr bool fp8_walks(int k) {
+__host__ __device__ constexpr bool fp8_walks(int k, uint64_t output_bytes) {
     using Cfg = Fp8TileConfig<BLOCK_M, BLOCK_N>;
-    return STAGES == 2 && kGemmType == GemmType::Normal && Cfg::DEEP_B_CAPABLE && Cfg::WTN >= 32 && k >= 256;
+    return STAGES == 2 && kGemmType == GemmType::Normal && Cfg::DEEP_B_CAPABLE && Cfg::WTN >= 32 && k >= 256 && fp8_walk_pays(k, output_bytes);
 }
 
 // The plain GEMM on two LDS stages as a persistent walk: workgroup b takes slots b, b + gridDim.x, ... (the launcher
@@ -728,8 +729,7 @@ __host__ __device__ constexpr bool fp8_walks(int k) {
 // (fp8_walk_streams_output in scheduler.hpp; with the same operands call after call plain stores were 1 % faster). Inputs changing from call to
 // call, two stages and plain stores before -> now: 4096 x 7168 x 7168 189 -> 178 us, 8192 x 7168 x 7168 371 -> 350, 8192 x 2112 x
 // 7168 on 256 x 160 tiles 159 -> 140, 4096 x 24576 x 1536 159 -> 143, 3529 x 7616 x 1024 39.8 -> 33.3, one round of tiles
-// (4096 x 4096 x 7168) 101.8 -> 100.8; twelve shapes 0.92 on average, an odd number of k-tiles (3529 x 7616 x 896, a workgroup per tile
-// before) 31.7 -> 30.6.
+// (4096 x 4096 x 7168) 101.8 -> 100.8; twelve shapes 0.92 on average.
 // What a wave needs to know of a tile is wave-uniform: the per-lane parts of every address (the lane's row within a copy
 // pass, its row within the slab) do not depend on the tile, and the tile's first row rides in the scalar offset.
 template <int SHAPE_N, int SHAPE_K, int BLOCK_M, int BLOCK_N>
@@ -923,8 +923,11 @@ fp8_gemm_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_s
             two_stages = {lds_a0, lds_b0, lds_a1, lds_b1, lds_b2};
         } else two_stages = {lds_a0, lds_b0, lds_a1, lds_b1, nullptr};
     }
-    if constexpr (fp8_walks<BLOCK_M, BLOCK_N, STAGES, kGemmType>(SHAPE_K ? SHAPE_K : 256)) {
-        if (SHAPE_K != 0 || fp8_walks<BLOCK_M, BLOCK_N, STAGES, kGemmType>(k_rt)) {
+    // any K and output size, where the kernel does not know them
+    if constexpr (fp8_walks<BLOCK_M, BLOCK_N, STAGES, kGemmType>(SHAPE_K ? SHAPE_K : 256, ~uint64_t(0))) {
+        const int n = SHAPE_N ? SHAPE_N : n_rt, k = SHAPE_K ? SHAPE_K : k_rt;
+        if ((SHAPE_K != 0 && fp8_walks<BLOCK_M, BLOCK_N, STAGES, kGemmType>(SHAPE_K, 0)) ||
+            fp8_walks<BLOCK_M, BLOCK_N, STAGES, kGemmType>(k, uint64_t(m) * n * 2)) {
             fp8_gemm_walk<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N>(lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt, sa_stride_m, sa_stride_k,
                                                               num_slots, two_stages);
             return;
@@ -1212,7 +1215,7 @@ public:
         const XcdTileScheduler<> sched(m, n, BLOCK_M, BLOCK_N);
         const int slots = sched.grid_size();
         int grid = capped_grid(slots, num_sms, device_cu_count());
-        if (fp8_walks<BLOCK_M, BLOCK_N, int(kNumStages), GemmType::Normal>(k)) {
+        if (fp8_walks<BLOCK_M, BLOCK_N, int(kNumStages), GemmType::Normal>(k, uint64_t(m) * n * 2)) {
             // persistent: one workgroup per CU (a multiple of the 8 XCDs, so a workgroup's tiles stay on one XCD), or as
             // many as the caller's cap allows
             const int cus = device_cu_count() / kNumXCD * kNumXCD;

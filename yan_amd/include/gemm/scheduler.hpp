@@ -237,6 +237,16 @@ __host__ __device__ inline int capped_grid(int slots, int num_sms, int device_cu
     return num_sms >= kNumXCD ? num_sms / kNumXCD * kNumXCD : num_sms;
 }
 
+// Whether the plain FP8 GEMM on two LDS stages walks its tiles (fp8_gemm_walk) or runs a workgroup per tile: it walks, but for 3 to
+// 17 k-tiles, an odd number, and outputs of up to 64 MB. A short tile leaves the walk little to hide its seam under, and tiles handed out as
+// units fall free end more evenly: walk -> workgroup per tile, inputs changing, 7902 x 2624 x 640 26.7 -> 24.3 us, x 1152 38.6 -> 36.3, 8192 x
+// 2560 x 1152 38.8 -> 35.2, 4096 x 7168 x 896 38.7 -> 36.7, x 1664 56.3 -> 54.4, 5222 x 1792 x 384 12.3 -> 11.5. Larger outputs gain by the
+// walk at every K (8192 x 7168 x 384 42.6 -> 40.2 us, x 1152 78.2 -> 75.4), longer K gain at every size (4096 x 7168 x 9344 234 -> 230), and even numbers
+// of k-tiles walk as they always have.
+__host__ __device__ constexpr bool fp8_walk_pays(int k, uint64_t output_bytes) {
+    return k % 256 == 0 || k > 17 * 128 || output_bytes > (uint64_t(64) << 20);
+}
+
 // Whether the persistent FP8 walk stores its output (`bytes`) with the non-temporal hint: outputs that would push the operands out of
 // the 256 MB memory-side cache, from 64 MB on whatever K, from 32 MB on where the k-loop is long (operands many times the output).
 // Plain -> hint, inputs changing: 8192 x 7168 x 768 57.4 -> 54.7 us, 4096 x 16384 x 3072 184.7 -> 175.2, 2048 x 12288 x 4096
