@@ -342,7 +342,7 @@ DENSE_RAGGED_CAP_CASE = ([(128, 128), (128, 192), (64, 64), (256, 128)], (390, 5
 
 # Rows a multiple of 16 KB apart, whose tiles start at different places along K: (tile, parts of K), rows, columns, depth
 ROTATED_CASES = [((64, 64), 1), ((64, 64), 4), ((128, 128), 2), ((64, 128), 3)]
-ROTATED_SIZES = (77, 1412, 8192)
+ROTATED_SIZES = [(77, 1412, 8192), (77, 3140, 8192)]         # weights too small for it, and large enough
 
 
 # Outputs whose rows are no multiple of 16 bytes, on every width of the 256-row kernels and two ring tiles: tiles, rows, columns, depths

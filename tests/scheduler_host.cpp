@@ -199,6 +199,11 @@ int main() {
         // Outputs the walk stores with the non-temporal hint: from past 64 MB, behind a long K from past 32 MB.
         const int m = 0, n = 0, bm = 256, bn = 256;
         const uint64_t mb = uint64_t(1) << 20;
+        // Launches whose tiles start at different places along K: (tile rows, m, n, k, parts)
+        auto spreads = [](int rows, int m, int n, int k, int parts) { return yan::spreads_starts(rows, m, uint64_t(n) * k * 2, k, parts); };
+        CHECK(spreads(1, 37, 4096, 8192, 4) && spreads(2, 128, 16384, 8192, 1) && spreads(2, 256, 8192, 16384, 2) && spreads(1, 37, 3072, 8192, 4));
+        CHECK(!spreads(1, 64, 1024, 16384, 8) && !spreads(4, 200, 4096, 8192, 4) && !spreads(1, 37, 4096, 7168, 4));
+        CHECK(!spreads(2, 256, 16384, 16384, 1) && !spreads(2, 256, 16384, 8192, 1) && !spreads(4, 400, 8192, 16384, 1) && !spreads(1, 128, 45056, 16384, 1));
         // Problems that walk: not the odd numbers of up to 17 k-tiles, unless the output is large.
         CHECK(!yan::fp8_walk_pays(384, 64 * mb) && !yan::fp8_walk_pays(640, 2ull * 7902 * 2624) && !yan::fp8_walk_pays(2176, 0));
         CHECK(yan::fp8_walk_pays(384, 64 * mb + 8) && yan::fp8_walk_pays(2432, 0) && yan::fp8_walk_pays(256, 0) && yan::fp8_walk_pays(2048, 0));

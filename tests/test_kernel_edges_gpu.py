@@ -386,10 +386,10 @@ def test_output_rows_that_end_inside_a_16_byte_store(tile, dtype):
             assert (room[m * n:] == -7.0).all()
 
 
+@pytest.mark.parametrize('m,n,k', testing.ROTATED_SIZES)
 @pytest.mark.parametrize('tile,split_k', testing.ROTATED_CASES)
-def test_dense_tiles_that_start_at_different_places_along_k(tile, split_k):
-    m, n, k = testing.ROTATED_SIZES
-    _announce('rotated', tile, split_k)
+def test_dense_tiles_that_start_at_different_places_along_k(tile, split_k, m, n, k):
+    _announce('rotated', tile, split_k, m, n, k)
     a, b, c = testing.make_bf16_case(m, n, k, seed=22, device='cuda')
     name, keys, arg_defs, includes, code_template = testing.stream_plans('dense', tile, split_k, 0)
     kernel = jit.build(name, arg_defs, jit.generate(includes, arg_defs, jit.cpp_format(code_template, keys)))

@@ -141,10 +141,8 @@ dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
     static_assert(StA::PADDED_ROWS == BLOCK_M && StB::PADDED_ROWS == BLOCK_N, "tiles are whole copy passes");
     // Workgroups march along K in step. Where rows are a multiple of 16 KB apart, one k-tile of all rows lies in a few of the memory
     // channels, which all of them then ask at a time: there (kSpreadStarts) the columns of the tiles start at places spread over
-    // their range, multiples of the golden ratio, and come round to the k-tiles in front at the end. 37 x 4096 x 8192 20.2 -> 16.8 us,
-    // 37 x 16384 x 8192 56.7 -> 41.6, 37 x 4096 x 16384 35.6 -> 26.6, 128 x 8192 x 8192 42.0 -> 37.9. At other depths it changes nothing
-    // (K = 7168) or loses 1 % (4096), as with many tile rows, which share panels that some have passed then (1024 x 4096 x 8192
-    // 75.5 -> 76.3).
+    // their range, multiples of the golden ratio, and come round to the k-tiles in front at the end. At other depths it changes
+    // nothing (K = 7168) or loses 1 % (4096). Which launches gain by it, and the times: spreads_starts in scheduler.hpp.
     constexpr bool SPREAD = (COPIES & kSpreadStarts) != 0;
     const int range = kt_hi - kt_lo, first = SPREAD && range > 0 ? int(__umulhi(uint32_t(tile.n_idx) * 0x9e3779b9u, uint32_t(range))) : 0;
     // Copy number `d` (A passes first, then B passes) of the `kt`-th k-tile into the given stage.
@@ -934,11 +932,11 @@ inline hipError_t check_dense_args(int m, int n, int k, const void* a, const voi
     return hipSuccess;
 }
 
-// Calls `launch` with the copies (COPIES, a std::integral_constant) of a ring tile's launch. Why the starts are spread for rows a
-// multiple of 16 KB apart, and up to four tile rows: dense_gemm_body.
-template <typename Launch>
-inline void with_dense_copies(int tiles_m, int n, int k, Launch&& launch) {
-    const bool streamed = streams_weights(tiles_m, uint64_t(n) * k * 2, k * 2), spread = k % 8192 == 0 && tiles_m <= 4;
+// Calls `launch` with the copies (COPIES, a std::integral_constant) of a ring tile's launch.
+template <int SPLIT_K, typename Launch>
+inline void with_dense_copies(int tiles_m, int m, int n, int k, Launch&& launch) {
+    const uint64_t weight_bytes = uint64_t(n) * k * 2;
+    const bool streamed = streams_weights(tiles_m, weight_bytes, k * 2), spread = spreads_starts(tiles_m, m, weight_bytes, k, SPLIT_K);
     if (streamed && spread) launch(std::integral_constant<int, kStreamedWeights | kSpreadStarts>{});
     else if (streamed) launch(std::integral_constant<int, kStreamedWeights>{});
     else if (spread) launch(std::integral_constant<int, kSpreadStarts>{});
@@ -995,7 +993,7 @@ inline hipError_t launch_dense(int m, int n, int k, const void* a, const void* b
                                    dim3(dense_launch_waves(BLOCK_M, BLOCK_N) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
                                    static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, slots);
         };
-        with_dense_copies(sched.tiles_m, n, k, launch);
+        with_dense_copies<1>(sched.tiles_m, m, n, k, launch);
     }
     return hipGetLastError();
 }
@@ -1028,7 +1026,7 @@ inline hipError_t launch_dense_split_k(int m, int n, int k, const void* a, const
                                dim3(dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
                                static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, partials, counters);
     };
-    with_dense_copies(sched.tiles_m, n, k, launch);
+    with_dense_copies<SPLIT_K>(sched.tiles_m, m, n, k, launch);
     return hipGetLastError();
 }
 

@@ -271,6 +271,21 @@ __host__ __device__ constexpr bool streams_weights(int tile_rows, uint64_t weigh
     return (tile_rows <= 1 || (tile_rows <= 4 && row_bytes <= 4096)) && weight_bytes >= (uint64_t(96) << 20);
 }
 
+// Whether the tiles of a 16-bit ring launch start at different places along K (kSpreadStarts in bf16_gemm.hpp): rows a multiple
+// of 16 KB apart, few tile rows, and
+//   * weights of 48 MB and more. Smaller ones are often still in the 256 MB memory-side cache, whose channels do not mind, and
+//     lose: going round three, 64 x 1024 x 16384 14.6 -> 15.3 us, 128 x 2048 x 8192 13.7 -> 14.3;
+//   * activations that stay in an XCD's 4 MB of L2 while its tiles are all over the part's range of K (in step they stay whatever
+//     their size): 400 x 8192 x 16384 141 -> 181 us, 256 x 16384 x 16384 176 -> 218, 128 x 45056 x 16384 269 -> 275 unsplit, but
+//     256 x 8192 x 16384 in two parts 101 -> 96;
+//   * at most two tile rows: with four nothing gains (200 x 1024 x 8192 14.5 -> 15.2 us, 400 x 4096 x 16384 77.8 -> 79.2).
+// Where it spreads: 37 x 4096 x 8192 22.2 -> 18.4 us, 64 x 8192 x 16384 58.4 -> 50.8, 128 x 8192 x 16384 72.2 -> 59.0, 200 x 4096 x
+// 16384 56.7 -> 51.7, 128 x 3072 x 8192 24.7 -> 24.1.
+__host__ __device__ constexpr bool spreads_starts(int tile_rows, int m, uint64_t weight_bytes, int k, int split_k) {
+    const uint64_t activations = uint64_t(m) * k * 2 / split_k, l2 = uint64_t(4) << 20;
+    return k % 8192 == 0 && tile_rows <= 2 && weight_bytes >= (uint64_t(48) << 20) && (split_k > 1 ? activations <= l2 : activations < l2);
+}
+
 // Split-K workspaces (fp8_gemm.hpp, bf16_gemm.hpp): the arrival counters take the first kSplitKCounterBytes whatever the
 // problem, so that launches of different shapes and kernels can share a workspace; the largest plan of the tile heuristics
 // (256 workgroups of 128 x 128 partial sums) fits kSplitKWorkspaceBytes.
