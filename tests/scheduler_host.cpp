@@ -204,6 +204,9 @@ int main() {
         CHECK(spreads(1, 37, 4096, 8192, 4) && spreads(2, 128, 16384, 8192, 1) && spreads(2, 256, 8192, 16384, 2) && spreads(1, 37, 3072, 8192, 4));
         CHECK(!spreads(1, 64, 1024, 16384, 8) && !spreads(4, 200, 4096, 8192, 4) && !spreads(1, 37, 4096, 7168, 4));
         CHECK(!spreads(2, 256, 16384, 16384, 1) && !spreads(2, 256, 16384, 8192, 1) && !spreads(4, 400, 8192, 16384, 1) && !spreads(1, 128, 45056, 16384, 1));
+        // Row-major scales four k-tiles at a time: not where many 64 x 64 tile rows loop over few of them.
+        CHECK(!yan::fp8_scale_pieces_pay(5, 64, 64, 2560) && !yan::fp8_scale_pieces_pay(4, 64, 64, 4096) && yan::fp8_scale_pieces_pay(3, 64, 64, 2560));
+        CHECK(yan::fp8_scale_pieces_pay(5, 64, 64, 2048) && yan::fp8_scale_pieces_pay(5, 64, 64, 4608) && yan::fp8_scale_pieces_pay(5, 64, 128, 2560));
         // Problems that walk: not the odd numbers of up to 17 k-tiles, unless the output is large.
         CHECK(!yan::fp8_walk_pays(384, 64 * mb) && !yan::fp8_walk_pays(640, 2ull * 7902 * 2624) && !yan::fp8_walk_pays(2176, 0));
         CHECK(yan::fp8_walk_pays(384, 64 * mb + 8) && yan::fp8_walk_pays(2432, 0) && yan::fp8_walk_pays(256, 0) && yan::fp8_walk_pays(2048, 0));

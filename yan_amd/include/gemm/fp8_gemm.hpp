@@ -50,12 +50,12 @@ namespace yan {
 // row, more requests than the operands if several waves ask for it: the first waves copy a part each, the others nothing. Rows
 // of whole 16-byte pieces, as row-major scales are where K is a multiple of 512, are copied four k-tiles at a time. Row-major,
 // every wave -> one wave -> four k-tiles: 512 x 7168 x 7168 62.8 -> 47.2 -> 39.8 us (37 token-contiguous); 640 x 9216 x 4096 47.3 -> 36.1 and
-// 1500 x 4096 x 4096 43.2 -> 35.8 with four, 900 x 4096 x 7040 53.7 -> 43.3 with one. Kernels of their own: the choice inside the
+// 1500 x 4096 x 4096 43.2 -> 35.8 with four, 900 x 4096 x 7040 53.7 -> 43.3 with one; fp8_scale_pieces_pay says where one is enough. Kernels of their own: the choice inside the
 // k-loop cost the token-contiguous layout 2 to 5 %.
 enum class Fp8ScaleCopies { EveryWave, OneWave, FourKTiles };
-inline Fp8ScaleCopies fp8_scale_copies(const float* scales, int stride_m, int stride_k, int stride_g, int k) {
+inline Fp8ScaleCopies fp8_scale_copies(const float* scales, int stride_m, int stride_k, int stride_g, int k, bool pieces_pay = true) {
     if (stride_m == 1) return Fp8ScaleCopies::EveryWave;
-    const bool pieces = stride_k == 1 && stride_m % 4 == 0 && stride_g % 4 == 0 && k % 512 == 0 && reinterpret_cast<uintptr_t>(scales) % 16 == 0;
+    const bool pieces = pieces_pay && stride_k == 1 && stride_m % 4 == 0 && stride_g % 4 == 0 && k % 512 == 0 && reinterpret_cast<uintptr_t>(scales) % 16 == 0;
     return pieces ? Fp8ScaleCopies::FourKTiles : Fp8ScaleCopies::OneWave;
 }
 
@@ -1225,7 +1225,8 @@ public:
             const int cus = device_cu_count() / kNumXCD * kNumXCD;
             grid = capped_grid(slots < cus ? slots : cus, num_sms, device_cu_count());
         }
-        const Fp8ScaleCopies copies = fp8_scale_copies(lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k, 0, k);
+        const Fp8ScaleCopies copies = fp8_scale_copies(lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k, 0, k,
+                                                       fp8_scale_pieces_pay(sched.tiles_m, BLOCK_M, BLOCK_N, k));
         return pick_kernel<TokenContiguous::value>(sched.tiles_m, uint64_t(n) * k, k, copies, [&](auto stream_weights, auto scale_copies) {
             hipLaunchKernelGGL((fp8_gemm_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, GemmType::Normal, int(kNumStages), decltype(stream_weights)::value,
                                                 decltype(scale_copies)::value>),

@@ -271,6 +271,15 @@ __host__ __device__ constexpr bool streams_weights(int tile_rows, uint64_t weigh
     return (tile_rows <= 1 || (tile_rows <= 4 && row_bytes <= 4096)) && weight_bytes >= (uint64_t(96) << 20);
 }
 
+// Whether four k-tiles of row-major scales a copy (Fp8ScaleCopies) are worth it in an unsplit plain FP8 GEMM of `tile_rows` rows of BLOCK_M x BLOCK_N tiles.
+// On 64 x 64 tiles in a loop (K beyond 2048) they are not while a row's scales are at most one cache line (K = 4096), which stays in
+// the caches from copy to copy where four tile rows and more read it: four a copy -> one, 300 x 2112 x 2560 11.0 -> 10.2 us, 395 x 1728 x
+// 3072 12.7 -> 11.8, 500 x 1088 x 4096 15.3 -> 13.4, 256 x 4096 x 4096 17.0 -> 16.4. They are elsewhere: 64 x 64 with K = 1024 (256 x
+// 3072 5.5 against 5.65), one tile row (62 x 16384 x 7168 30.0 against 33.4), 128 x 128 (1000 x 2112 x 4096 24.5 against 27.2).
+__host__ __device__ constexpr bool fp8_scale_pieces_pay(int tile_rows, int block_m, int block_n, int k) {
+    return block_m * block_n > 64 * 64 || tile_rows < 4 || k <= 2048 || k > 4096;
+}
+
 // Whether the tiles of a 16-bit ring launch start at different places along K (kSpreadStarts in bf16_gemm.hpp): rows a multiple
 // of 16 KB apart, few tile rows, and
 //   * weights of 48 MB and more. Smaller ones are often still in the 256 MB memory-side cache, whose channels do not mind, and
