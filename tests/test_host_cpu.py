@@ -68,6 +68,16 @@ def test_activation_scales_are_relaid_only_where_it_pays():
     assert scales_for_kernel(relaid, 1e15) is relaid
 
 
+def test_row_major_scales_stay_as_they_are_for_ring_tiles_up_to_k_8192():
+    from yan_amd.jit_kernels.utils import scales_for_kernel
+    ring = {'NUM_STAGES': 3, 'BLOCK_M': 128}
+    for k_tiles, kept in ((32, True), (64, True), (68, False), (128, False), (30, False)):
+        rows = torch.arange(128 * k_tiles, dtype=torch.float32).reshape(128, k_tiles)
+        assert (scales_for_kernel(rows, 1e12, ring) is rows) == kept
+        assert scales_for_kernel(rows, 1e12, {'NUM_STAGES': 2, 'BLOCK_M': 256}).stride() == (1, 128)
+        assert torch.equal(scales_for_kernel(rows, 1e12, ring), rows)
+
+
 def test_split_k_plans():
     """K is split when the unsplit tiles leave the chip short of work and K is long; every plan fits one round of
     workgroups and the workspace, leaves each part 14 k-tiles or more (24 of two), and the shapes of the GPU suite get the plans the

@@ -91,8 +91,11 @@ def get_col_major_tensor(x: torch.Tensor) -> torch.Tensor:
 # token-contiguous copy of them first: the kernels read a scale per row and k-tile, which in the row-major layout is a
 # cache line per row (4096 x 4096 x 7168: 110 us against 96 us), and the copy costs about 3 us on the device. Below it the copy
 # costs as much as it saves. Ring tiles that copy row-major scales four k-tiles at a time (`Fp8ScaleCopies` in
-# gemm/fp8_gemm.hpp) need none: 1023 x 7168 x 4096 40.3 us with the copy, 38.9 without, 1024 x 4096 x 7168 42.4 and 42.0.
+# gemm/fp8_gemm.hpp) need none up to K = 8192: 2048 x 4096 x 4096 45.4 us with the copy, 44.1 without, 900 x 4096 x 8192 50.6
+# and 48.7, 32 contiguous groups, 4096 x 4096 x 2048 64.8 and 61.9; beyond, the rows are too long for the caches: 1500 x 4096 x 16384
+# 124.3 and 129.3, 200 x 9216 x 16384 77.6 and 80.0, 512 x 7168 x 9216 54.0 and 55.1.
 SCALE_RELAYOUT_MIN_FLOP = 6e10
+ROW_MAJOR_SCALES_MAX_K_TILES = 64
 
 
 def scales_for_kernel(scales: torch.Tensor, flop: float, keys=None) -> torch.Tensor:
@@ -106,8 +109,8 @@ def scales_for_kernel(scales: torch.Tensor, flop: float, keys=None) -> torch.Ten
         return scales
     # ring tiles, except where the contiguous layout's tiles follow the groups (256 rows there)
     if keys is not None and keys['NUM_STAGES'] > 2 and (keys['BLOCK_M'] < 256 or keys.get('GEMM_TYPE') != 'GroupedContiguous'):
-        if (scales.stride(-1) == 1 and scales.size(-1) % 4 == 0 and scales.stride(-2) % 4 == 0 and scales.data_ptr() % 16 == 0
-                and (scales.dim() == 2 or scales.stride(0) % 4 == 0)):
+        if (scales.size(-1) <= ROW_MAJOR_SCALES_MAX_K_TILES and scales.stride(-1) == 1 and scales.size(-1) % 4 == 0 and scales.stride(-2) % 4 == 0
+                and scales.data_ptr() % 16 == 0 and (scales.dim() == 2 or scales.stride(0) % 4 == 0)):
             return scales
     return get_col_major_tensor(scales)
 
