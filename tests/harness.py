@@ -298,7 +298,11 @@ GROUPED_FOLLOW_GROUPS_CASES = [((63 * 128, 3 * 128, 1, 2 * 128), 264, 128, 0), (
                                ((128,) * 5, 1028, 640, 0), ((64 * 128, 65 * 128), 12, 256, 2), ((128,), 256, 128, 0),
                                # tall rows that run as two flat ones each on eight compute units: two of ten, one of nine behind two flat
                                # ones, one of five with two tiles each, the last of which ends inside a block
-                               ((20 * 128,), 12, 256, 0), ((11 * 128, 9 * 128), 12, 384, 1), ((10 * 128 - 50,), 260, 128, 0)]
+                               ((20 * 128,), 12, 256, 0), ((11 * 128, 9 * 128), 12, 384, 1), ((10 * 128 - 50,), 260, 128, 0),
+                               # (with K long enough for it)
+                               ((20 * 128,), 12, 2048, 0), ((11 * 128, 9 * 128), 12, 2176, 1), ((10 * 128 - 50,), 260, 2048, 0)]
+# More than a round of tall tiles on the whole chip, the rows of the last one flat: 66 rows of four tiles, two rows behind 256 tiles
+GROUPED_LAST_ROUND_FLAT_CASE = ((40 * 256, 26 * 256), 1024, 2048)
 # (BLOCK_N, NUM_STAGES) that go with BLOCK_M = 256 in the keys of a contiguous call: the widths of the cost table, the other ones the
 # tiles support, with and without a ring and a 128-row tile beside them
 GROUPED_256_ROW_KEYS = [(256, 2), (224, 2), (192, 2), (160, 2), (128, 3), (128, 2), (96, 2), (32, 2)]
@@ -593,7 +597,7 @@ def jit_kernels_in_use(num_cus: int = 256):
     for rows, n, k in (((896, 1152) * 4, 4096, 7168), ((1024,) * 8, 4096, 7168), ((512,) * 16, 4096, 7168), ((384, 640) * 8, 4096, 7168)):
         name, keys, arg_defs, _ = m_grouped_gemm.grouped_kernel_plan('GroupedContiguous', len(rows), sum(rows), n, k, num_cus)
         add(name, arg_defs, m_grouped_gemm.includes, m_grouped_gemm.rows_on_device_template if 'ROWS' in keys else m_grouped_gemm.template, keys)
-    for rows, n, k, _ in GROUPED_ROWS_ON_DEVICE_CASES + GROUPED_FOLLOW_GROUPS_CASES:
+    for rows, n, k, _ in GROUPED_ROWS_ON_DEVICE_CASES + GROUPED_FOLLOW_GROUPS_CASES + [(*GROUPED_LAST_ROUND_FLAT_CASE, 0)]:
         name, keys, arg_defs, code_template = grouped_rows_on_device_plan(sum(1 for r in rows if r > 0), n, k)
         add(name, arg_defs, m_grouped_gemm.includes, code_template, keys)
     rows, n, k, _ = GROUPED_256_ROW_KEYS_CASE

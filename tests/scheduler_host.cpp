@@ -123,8 +123,8 @@ int main() {
     // cut 64 blocks at a time as a wave does it
     unsigned rng = 1;
     auto random = [&](int below) { rng = rng * 1664525u + 1013904223u; return int((rng >> 8) % unsigned(below)); };
-    for (int trial = 0; trial < 400; ++trial) {
-        const int bm = 256, bn = (trial / 4) % 2 ? 256 : 128, tn = 1 + random(20), n = (tn - 1) * bn + 4 + random(bn - 4);
+    for (int trial = 0; trial < 2000; ++trial) {
+        const int bm = 256, bn = (trial / 4) % 2 ? 256 : 128, tn = (trial / 8) % 2 ? 1 << random(4) : 1 + random(20), n = (tn - 1) * bn + 4 + random(bn - 4);
         std::vector<int> group_of;
         const int blocks = 1 + random(200), longest = trial % 3 == 0 ? 70 : (trial % 3 == 1 ? 4 : 1);
         for (int g = 0; int(group_of.size()) < blocks;) {
@@ -158,11 +158,11 @@ int main() {
         for (int b = 0; b < blocks; ++b) CHECK(covered[b] == (group_of[b] >= 0 ? 1 : 0));
         const long long launched = (long long)yan::XcdTileScheduler<>(m, n, 128, bn).grid_size() + yan::kNumXCD;
         const int cus[] = {1 << 30, 8, 40, 256};          // 2^30: no tall row ever runs flat
-        const int halved = yan::tall_rows_run_flat(tall_rows, flat_rows, tn, cus[trial % 4]);
+        const int halved = yan::tall_rows_run_flat(tall_rows, flat_rows, tn, cus[trial % 4], 2048);
         CHECK(halved >= 0 && halved <= tall_rows && (trial % 4 != 0 || halved == 0));
-        if (halved) {        // whole rounds of tall tiles and less than a row, then all the rest at one time
-            const int rest = (tall_rows - halved) * tn % cus[trial % 4];
-            CHECK(rest < tn && rest + (flat_rows + 2 * halved) * tn <= cus[trial % 4]);
+        CHECK(yan::tall_rows_run_flat(tall_rows, flat_rows, tn, cus[trial % 4], 1920) == 0);
+        if (halved) {        // whole rounds of tall tiles, then all the rest at one time
+            CHECK((tall_rows - halved) * tn % cus[trial % 4] == 0 && (flat_rows + 2 * halved) * tn <= cus[trial % 4]);
             ++halved_cases;
         }
         tall_rows -= halved;
@@ -194,6 +194,8 @@ int main() {
         CHECK(d.region_rows == 0);                           // 2 x 128 MiB of operands fit
         CHECK(e.region_rows == 32 && e.rows_outer);          // the FP8 16384^3 shape
         CHECK(region_cases > 100 && halved_cases > 10);
+        CHECK(yan::tall_rows_run_flat(32, 0, 20, 256, 7168) == 0);          // 120 of 128 tiles would be flat, 8 stay tall
+        CHECK(yan::tall_rows_run_flat(24, 0, 16, 256, 7168) == 8 && yan::tall_rows_run_flat(38, 4, 16, 256, 7168) == 6);
     }
     {
         // Outputs the walk stores with the non-temporal hint: from past 64 MB, behind a long K from past 32 MB.

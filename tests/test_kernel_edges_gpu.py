@@ -49,6 +49,25 @@ def test_contiguous_tiles_follow_the_groups(rows, n, k, pad_blocks):
     assert _fp8_close(results[0][real].float(), ref[real])
 
 
+def test_contiguous_tall_rows_of_the_last_round_run_flat():
+    """On the whole chip, where only the row count decides: the bits of the same rows in one round (no row runs flat there)."""
+    from yan_amd.jit_kernels import m_grouped_gemm
+    rows, n, k = testing.GROUPED_LAST_ROUND_FLAT_CASE
+    _announce('last round flat', rows, n, k)
+    (a8, sa), (b8, sb), out, idx = testing.make_grouped_contiguous_case(rows, n, k, seed=25, device='cuda', gen_device='cuda')
+    assert sum(rows) // 256 * (n // 256) == 264 and torch.cuda.get_device_properties(0).multi_processor_count == 256
+    name, keys, arg_defs, code_template = testing.grouped_rows_on_device_plan(b8.size(0), n, k)
+    kernel = jit.build(name, arg_defs, jit.generate(m_grouped_gemm.includes, arg_defs, jit.cpp_format(code_template, keys)))
+
+    def run(lo, hi):
+        got, scales = out[lo:hi].clone(), yan.get_col_major_tensor(sa[lo:hi])
+        assert kernel(a8[lo:hi], scales, b8, sb, got, idx[lo:hi], hi - lo, torch.cuda.current_stream(), 256, 0, scales.stride(0), scales.stride(1), 0, 0) == 0
+        torch.cuda.synchronize()
+        return got
+    m = sum(rows)
+    assert torch.equal(run(0, m), torch.cat([run(0, m // 2), run(m // 2, m)]))
+
+
 @pytest.mark.parametrize('block_n,stages', testing.GROUPED_256_ROW_KEYS)
 def test_contiguous_keys_that_name_a_tile_of_256_rows(block_n, stages):
     """Every width and depth such keys may hold, against the oracle, capped and not, with a row count that ends inside a block (the

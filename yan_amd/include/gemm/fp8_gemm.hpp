@@ -963,9 +963,9 @@ fp8_gemm_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_s
 // 128-row tiles ran throughout: 48 blocks over 16 groups x 4096 x 7168 219 -> 216 us by following the groups, 197 with the third
 // weight stage the tall tiles have room for (kDeepB); 10240 rows in 4 groups 290 -> 276 us, 8320 in 64 x 7168 x 2048 185 -> 172.
 // Mixing flat and tall tiles in the order of the groups (every weight panel then read at one time) measured the same.
-// Where the tall tiles end in a round with room for it, the tall rows of that round run as two flat ones each (tall_rows_run_flat in
-// scheduler.hpp): a workgroup alone on its compute unit takes 85-89 us for a tall tile of K = 7168 and 61-73 for a flat one. 48 blocks
-// over 16 groups 195 -> 186, over 8 groups 183 -> 175, 10240 rows in 6 groups x 4096 x 5120 214 -> 206; no change elsewhere.
+// Where the tall tiles end in a round of whole rows with room for it, the rows of that round run as two flat ones each
+// (tall_rows_run_flat in scheduler.hpp): a workgroup alone on its compute unit takes 85-89 us for a tall tile of K = 7168 and 61-73
+// for a flat one. 48 blocks over 16 uneven groups 195 -> 186, over 8 groups 180 -> 171.
 // STAGES belongs to the tall tile: 2, or a ring as everywhere else (256 x 128). The flat tile runs the deepest ring it has. Where
 // it has none, or runs on another number of waves (256 x 160 and the other widths no plan takes), the odd block is a tall
 // tile whose rows end with the block.
@@ -1000,7 +1000,7 @@ fp8_gemm_contiguous_rows_kernel(const uint8_t* __restrict__ lhs, const float* __
         flat_rows += __popcll(starts.flat);
     }
     // the last tall rows run as two flat ones each, numbered behind those that are flat by themselves
-    const int odd_rows = flat_rows, halved = HAS_FLAT ? tall_rows_run_flat(tall_rows, flat_rows, tiles_n, compute_units) : 0;
+    const int odd_rows = flat_rows, halved = HAS_FLAT ? tall_rows_run_flat(tall_rows, flat_rows, tiles_n, compute_units, SHAPE_K ? SHAPE_K : k_rt) : 0;
     tall_rows -= halved;
     flat_rows += 2 * halved;
     XcdTileScheduler<> tall(tall_rows * 256, N, 256, BLOCK_N), flat(flat_rows * 128, N, 128, BLOCK_N);

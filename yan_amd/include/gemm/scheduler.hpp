@@ -216,14 +216,17 @@ struct ContiguousBlock {
     __host__ __device__ bool starts_flat(int into) const { return group >= 0 && (into & 1) == 0 && behind != group; }
 };
 
-// How many of a contiguous layout's tall tile rows run as two flat ones each: the whole rows of the tall tiles' last, partial round,
-// where all flat tiles and what is left of that round then run at one time on the units it leaves. A flat tile takes 0.7 to
-// 0.8 of a tall one's time, so two flat rounds would take longer than the tall one.
-__host__ __device__ inline int tall_rows_run_flat(int tall_rows, int flat_rows, int tiles_n, int compute_units) {
+// How many of a contiguous layout's tall tile rows run as two flat ones each: those of the tall tiles' last, partial round, where it
+// is made of whole rows and all flat tiles then run at one time. A flat tile takes 0.7 to 0.8 of a tall one's time, so two flat
+// rounds would take longer than the tall one, and so does a round in which some tall tiles are left: 8192 rows in 4 groups x
+// 5120 x 7168, 128 tiles of 20 a row, 268 -> 279 us with six rows of them flat. With few k-tiles the flat tile's start weighs
+// more. Whole rows, tall -> flat, 10240 rows in 6 groups x 4096: K = 512 39.7 -> 41.9 us, 1024 58.9 -> 60.2, 1536 79.3 -> 79.7, 2688 118.0 ->
+// 117.5, 5120 213.5 -> 206.8; 6144 in 8 groups x 4096: K = 512 25.7 -> 26.9, 1536 52.3 -> 51.9, 2688 77.4 -> 75.4, 7168 180.1 -> 175.0.
+__host__ __device__ inline int tall_rows_run_flat(int tall_rows, int flat_rows, int tiles_n, int compute_units, int k) {
     const long long tall = (long long)tall_rows * tiles_n, flat = (long long)flat_rows * tiles_n;
-    if (tall <= compute_units) return 0;
-    const int over = int(tall % compute_units), rows = over / tiles_n;
-    return flat + over + (long long)rows * tiles_n <= compute_units ? rows : 0;
+    const int over = int(tall % compute_units);
+    if (k < 2048 || tall <= compute_units || over % tiles_n != 0) return 0;
+    return flat + 2 * (long long)over <= compute_units ? over / tiles_n : 0;
 }
 
 // Workgroups to launch for `slots` units of work (tiles, or groups x tiles) under the caller's compute-unit cap, the
