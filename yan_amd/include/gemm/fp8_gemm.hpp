@@ -1122,7 +1122,8 @@ public:
                                                                    : (m <= 128 * (long long)num_groups ? 1 : 1 << 30);
         const Fp8ScaleCopies copies = fp8_scale_copies(lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k,
                                                        kGemmType == GemmType::GroupedMasked ? lhs_scales_stride_g : 0, k);
-        return pick_kernel<false>(tile_rows, uint64_t(num_groups) * n * k, k, copies, [&](auto stream_weights, auto scale_copies) {
+        const uint64_t weight_bytes = kGemmType == GemmType::GroupedMasked ? uint64_t(num_groups) * n * k : contiguous_weight_bytes(num_groups, m, n, k);
+        return pick_kernel<false>(tile_rows, weight_bytes, k, copies, [&](auto stream_weights, auto scale_copies) {
             hipLaunchKernelGGL((fp8_gemm_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, int(kNumStages), decltype(stream_weights)::value,
                                                 decltype(scale_copies)::value>),
                                dim3(grid), dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream,

@@ -274,6 +274,13 @@ __host__ __device__ constexpr bool streams_weights(int tile_rows, uint64_t weigh
     return (tile_rows <= 1 || (tile_rows <= 4 && row_bytes <= 4096)) && weight_bytes >= (uint64_t(96) << 20);
 }
 
+// Weights that a contiguous grouped launch reads at the most: of as many groups as it has blocks of 128 rows. (With 59 groups and ten
+// blocks, 10 x 5184 x 1792, weights that the caches held were streamed for the sake of the 49 not read: 23.4 -> 26.2 us.)
+__host__ __device__ constexpr uint64_t contiguous_weight_bytes(int num_groups, int m, int n, int k) {
+    const int blocks = ceil_div(m, 128);
+    return uint64_t(num_groups < blocks ? num_groups : blocks) * n * k;
+}
+
 // Whether four k-tiles of row-major scales a copy (Fp8ScaleCopies) are worth it in an unsplit plain FP8 GEMM of `tile_rows` rows of BLOCK_M x BLOCK_N tiles.
 // On 64 x 64 tiles in a loop (K beyond 2048) they are not while a row's scales are at most one cache line (K = 4096), which stays in
 // the caches from copy to copy where four tile rows and more read it: four a copy -> one, 300 x 2112 x 2560 11.0 -> 10.2 us, 395 x 1728 x
