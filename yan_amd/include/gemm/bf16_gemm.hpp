@@ -932,15 +932,20 @@ inline hipError_t check_dense_args(int m, int n, int k, const void* a, const voi
     return hipSuccess;
 }
 
-// Calls `launch` with the copies (COPIES, a std::integral_constant) of a ring tile's launch.
-template <int SPLIT_K, typename Launch>
+// Calls `launch` with the copies (COPIES, a std::integral_constant) of a ring tile's launch. A kernel is compiled for each that a plan
+// can ask for: none for 256-row rings, and no streamed weights in six and eight parts, which have 96 MB of weights from
+// K = 24576 on only.
+template <int BLOCK_M, int SPLIT_K, typename Launch>
 inline void with_dense_copies(int tiles_m, int m, int n, int k, Launch&& launch) {
     const uint64_t weight_bytes = uint64_t(n) * k * 2;
     const bool streamed = streams_weights(tiles_m, weight_bytes, k * 2), spread = spreads_starts(tiles_m, m, weight_bytes, k, SPLIT_K);
-    if (streamed && spread) launch(std::integral_constant<int, kStreamedWeights | kSpreadStarts>{});
-    else if (streamed) launch(std::integral_constant<int, kStreamedWeights>{});
-    else if (spread) launch(std::integral_constant<int, kSpreadStarts>{});
-    else launch(std::integral_constant<int, 0>{});
+    if constexpr (BLOCK_M < 256 && SPLIT_K <= 4) {
+        if (streamed && spread) return launch(std::integral_constant<int, kStreamedWeights | kSpreadStarts>{});
+        if (streamed) return launch(std::integral_constant<int, kStreamedWeights>{});
+    }
+    if constexpr (BLOCK_M < 256)
+        if (spread) return launch(std::integral_constant<int, kSpreadStarts>{});
+    launch(std::integral_constant<int, 0>{});
 }
 
 // `num_sms`: the caller's compute-unit cap (0 = none), see capped_grid in scheduler.hpp.
@@ -993,7 +998,7 @@ inline hipError_t launch_dense(int m, int n, int k, const void* a, const void* b
                                    dim3(dense_launch_waves(BLOCK_M, BLOCK_N) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
                                    static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, slots);
         };
-        with_dense_copies<1>(sched.tiles_m, m, n, k, launch);
+        with_dense_copies<BLOCK_M, 1>(sched.tiles_m, m, n, k, launch);
     }
     return hipGetLastError();
 }
@@ -1026,7 +1031,7 @@ inline hipError_t launch_dense_split_k(int m, int n, int k, const void* a, const
                                dim3(dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
                                static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, partials, counters);
     };
-    with_dense_copies<SPLIT_K>(sched.tiles_m, m, n, k, launch);
+    with_dense_copies<BLOCK_M, SPLIT_K>(sched.tiles_m, m, n, k, launch);
     return hipGetLastError();
 }
 

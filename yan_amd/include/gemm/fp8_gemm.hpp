@@ -1191,7 +1191,7 @@ public:
         unsigned* counters = static_cast<unsigned*>(workspace);
         float* partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kSplitKCounterBytes);
         const Fp8ScaleCopies copies = fp8_scale_copies(lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k, 0, k);
-        return pick_kernel<TokenContiguous::value>(sched.tiles_m, uint64_t(n) * k, k, copies, [&](auto stream_weights, auto scale_copies) {
+        return pick_kernel<TokenContiguous::value, SPLIT_K>(sched.tiles_m, uint64_t(n) * k, k, copies, [&](auto stream_weights, auto scale_copies) {
             hipLaunchKernelGGL((fp8_gemm_split_k_kernel<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, int(kNumStages), SPLIT_K, decltype(stream_weights)::value,
                                                         decltype(scale_copies)::value>),
                                dim3(int(grid)), dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream,
@@ -1242,24 +1242,39 @@ public:
 private:
     // Calls `launch` with what a kernel is compiled for: whether the weights are streamed (std::true_type or std::false_type), and how the
     // scales are copied (a std::integral_constant). What the sizes or the caller's scale layout rule out when the kernel is
-    // compiled is left out. Tiles that are no ring of one k-tile per barrier have no copies four k-tiles at a time.
-    template <bool TOKEN_CONTIGUOUS, typename Launch>
+    // compiled is left out. Tiles that are no ring of one k-tile per barrier have no copies four k-tiles at a time. In the plain
+    // GEMM, streamed weights are left out for 64 x 32 and 256 x 128 tiles and for split tiles up to 64 x 64, which gain nothing by
+    // them or have 96 MB of weights from K = 24576 on only, and for scales in other layouts that do not come four k-tiles at a time
+    // (64 x 24832 x 7040 47.1 us against 48.2 without).
+    template <bool TOKEN_CONTIGUOUS, int SPLIT_K = 1, typename Launch>
     static hipError_t pick_kernel(int tile_rows, uint64_t weight_bytes, int row_bytes, Fp8ScaleCopies copies, Launch&& launch) {
+        using EveryWave  = std::integral_constant<Fp8ScaleCopies, Fp8ScaleCopies::EveryWave>;
+        using OneWave    = std::integral_constant<Fp8ScaleCopies, Fp8ScaleCopies::OneWave>;
+        using FourKTiles = std::integral_constant<Fp8ScaleCopies, Fp8ScaleCopies::FourKTiles>;
         constexpr uint64_t KNOWN = uint64_t(SHAPE_N) * SHAPE_K * kNumGroups;
-        constexpr bool RING = kNumStages > 2;
-        constexpr bool MAY_STREAM = RING && (KNOWN == 0 || (kGemmType != GemmType::Normal && kNumGroups == 1) || streams_weights(1, KNOWN, 0));
+        constexpr bool RING = kNumStages > 2, GROUPED = kGemmType != GemmType::Normal;
+        constexpr bool WORTH_STREAMING = GROUPED || (SPLIT_K > 1 ? BLOCK_M * BLOCK_N > 64 * 64 : BLOCK_M < 256 && !(BLOCK_M == 64 && BLOCK_N == 32));
+        constexpr bool MAY_STREAM = RING && WORTH_STREAMING && (KNOWN == 0 || (GROUPED && kNumGroups == 1) || streams_weights(1, KNOWN, 0));
         constexpr bool MAY_QUAD = RING && !TOKEN_CONTIGUOUS && SHAPE_K % 512 == 0 && fp8_ring_group(BLOCK_M, BLOCK_N, int(kNumStages)) == 1 &&
                                   Fp8TileConfig<BLOCK_M, BLOCK_N>::ring_bytes(int(kNumStages), true) <= 160 * 1024;
-        auto with_scales = [&](auto stream_weights) {
-            if constexpr (MAY_QUAD)
-                if (copies == Fp8ScaleCopies::FourKTiles) return launch(stream_weights, std::integral_constant<Fp8ScaleCopies, Fp8ScaleCopies::FourKTiles>{});
-            if constexpr (RING && !TOKEN_CONTIGUOUS)
-                if (copies != Fp8ScaleCopies::EveryWave) return launch(stream_weights, std::integral_constant<Fp8ScaleCopies, Fp8ScaleCopies::OneWave>{});
-            return launch(stream_weights, std::integral_constant<Fp8ScaleCopies, Fp8ScaleCopies::EveryWave>{});
-        };
+        const bool streamed = MAY_STREAM && streams_weights(tile_rows, weight_bytes, row_bytes);
+        if constexpr (MAY_QUAD) {
+            if (copies == Fp8ScaleCopies::FourKTiles) {
+                if constexpr (MAY_STREAM)
+                    if (streamed) return launch(std::true_type{}, FourKTiles{});
+                return launch(std::false_type{}, FourKTiles{});
+            }
+        }
+        if constexpr (RING && !TOKEN_CONTIGUOUS) {
+            if (copies != Fp8ScaleCopies::EveryWave) {
+                if constexpr (MAY_STREAM && GROUPED)
+                    if (streamed) return launch(std::true_type{}, OneWave{});
+                return launch(std::false_type{}, OneWave{});
+            }
+        }
         if constexpr (MAY_STREAM)
-            if (streams_weights(tile_rows, weight_bytes, row_bytes)) return with_scales(std::true_type{});
-        return with_scales(std::false_type{});
+            if (streamed) return launch(std::true_type{}, EveryWave{});
+        return launch(std::false_type{}, EveryWave{});
     }
 };
 
