@@ -316,6 +316,11 @@ FP8_SHORT_K_SIZES = (390, 516)
 # Tiles on two stages (three of the weights) that are walked, several to a workgroup: the seam between two tiles where every k-tile
 # fetches for the next one (two of them) and where one does not; tiles whose copies are handed out one and several to a row
 FP8_WALK_CASES = [((256, 256), (256, 384, 512)), ((256, 224), (256, )), ((256, 160), (256, 384)), ((128, 256), (256, 384)), ((64, 64), (384, ))]
+# and those that run a workgroup per tile, or several one after the other under a cap: a single k-tile, an odd number of few, and
+# a tile that has no room for the third stage of weights
+FP8_TWO_STAGE_LOOP_CASES = [((256, 256), (128, 640)), ((256, 160), (128, 896)), ((192, 320), (128, 384, 512))]
+# The masked layout on 256 x 256 tiles: groups without a row, with one, with a tile and a part, full ones; even and odd numbers of k-tiles
+MASKED_256_ROW_CASE = (520, 516, (520, 0, 300, 1, 256, 0, 257, 520), (128, 384, 512))
 FP8_WALK_SIZES = (1300, 772)
 # Few k-tiles, an odd number: an output of more than 64 MB is walked, its halves along n run a workgroup per tile
 FP8_ODD_K_TILE, FP8_ODD_K_SIZES = (256, 256), (5000, 6912, (384, 640))
@@ -356,9 +361,13 @@ RAGGED_ROWS_CASE = ([(256, 256), (256, 224), (256, 192), (256, 160), (128, 192),
 
 # Weights of 96 MB and more are fetched with the non-temporal hint where few tile rows read them: (tile, parts of K), rows, (n, k)
 # of a problem that has them so and whose halves along n do not.
-STREAM_FP8_CASES = [((32, 32), 1), ((64, 128), 1), ((64, 64), 4)]
+STREAM_FP8_CASES = [((32, 32), 1), ((64, 128), 1), ((64, 64), 4), ((64, 128), 2), ((128, 128), 2)]
 STREAM_DENSE_CASES = [((64, 64), 1), ((128, 128), 1), ((64, 64), 4)]
 STREAM_FP8_SIZES, STREAM_DENSE_SIZES = (61, 24832, 4096), (125, 25088, 2048)
+# Through the library: FP8 weights of 96 MB and more on a tile per workgroup and split; 16-bit ones that are spread (and K split), spread
+# and streamed (split and not), streamed
+CAPI_STREAMED_FP8_SIZES = [(64, 24832, 4096), (61, 13568, 8192), (113, 13568, 8192)]
+CAPI_STREAMED_DENSE_SIZES = [(37, 4096, 8192), (61, 8192, 8192), (33, 16448, 8192), (61, 14080, 4096)]
 STREAM_GROUPED_SIZES = (8, 64, 6400, 2048)          # groups, rows of each, n, k
 
 
@@ -454,6 +463,14 @@ def grouped_256_row_plan(block_n: int, stages: int, num_groups: int, n: int, k: 
     return 'm_grouped_gemm_fp8_fp8_bf16_nt', keys, m_grouped_gemm.arg_defs, m_grouped_gemm.template
 
 
+def masked_256_row_plan(num_groups: int, n: int, k: int):
+    """(name, keys, arg_defs, template) of a masked grouped call whose keys name a tile of 256 x 256 outright."""
+    from yan_amd.jit_kernels import m_grouped_gemm
+    keys = {'N': n, 'K': k, 'BLOCK_M': 256, 'BLOCK_N': 256, 'NUM_GROUPS': num_groups, 'NUM_STAGES': 2, 'NUM_TMA_MULTICAST': 1,
+            'GEMM_TYPE': 'GroupedMasked'}
+    return 'm_grouped_gemm_fp8_fp8_bf16_nt', keys, m_grouped_gemm.arg_defs, m_grouped_gemm.template
+
+
 def jit_kernels_in_use(num_cus: int = 256):
     """(name, arg_defs, code) of every distinct JIT kernel the shapes above, and the quantisers select."""
     from yan_amd.jit import cpp_format, generate
@@ -465,7 +482,7 @@ def jit_kernels_in_use(num_cus: int = 256):
         kernels.setdefault((name, code), (name, arg_defs, code))
 
     # the last four: shapes only the benchmark's --also legs run
-    for m, n, k in DENSE_TEST_SHAPES + REFERENCE_DENSE_TEST_SHAPES + DENSE_SPLIT_K_SHAPES + [(256, 512, 512), (4096, 5120, 5120), (2048, 7168, 7168), (4096, 7168, 16384), (8192, 8192, 9216)]:
+    for m, n, k in DENSE_TEST_SHAPES + REFERENCE_DENSE_TEST_SHAPES + DENSE_SPLIT_K_SHAPES + CAPI_STREAMED_DENSE_SIZES + [(256, 512, 512), (4096, 5120, 5120), (2048, 7168, 7168), (4096, 7168, 16384), (8192, 8192, 9216)]:
         for dtype in (torch.bfloat16, torch.half):
             if m and n:
                 name, keys, arg_defs = bf16_gemm.dense_kernel_plan(m, n, k, dtype, num_cus)
@@ -570,6 +587,19 @@ def jit_kernels_in_use(num_cus: int = 256):
         for k in depths:
             name, keys, arg_defs, code_template = fp8_explicit_tile_plan(*tile, FP8_WALK_SIZES[1], k, 2)
             add(name, arg_defs, gemm.includes, code_template, keys)
+    for m, n, k in CAPI_STREAMED_FP8_SIZES:
+        for token_contiguous in (True, False):
+            split = gemm.fp8_split_k_plan(m, n, k, num_cus, token_contiguous)
+            if split is not None:
+                name, keys, arg_defs, code_template = split
+                add(name, arg_defs, gemm.includes, code_template, keys)
+    for tile, depths in FP8_TWO_STAGE_LOOP_CASES:
+        for k in depths:
+            name, keys, arg_defs, code_template = fp8_explicit_tile_plan(*tile, FP8_WALK_SIZES[1], k, 2)
+            add(name, arg_defs, gemm.includes, code_template, keys)
+    for k in MASKED_256_ROW_CASE[3]:
+        name, keys, arg_defs, code_template = masked_256_row_plan(len(MASKED_256_ROW_CASE[2]), MASKED_256_ROW_CASE[1], k)
+        add(name, arg_defs, m_grouped_gemm.includes, code_template, keys)
     for k in FP8_ODD_K_SIZES[2]:
         for n in (FP8_ODD_K_SIZES[1], FP8_ODD_K_SIZES[1] // 2):
             name, keys, arg_defs, code_template = fp8_explicit_tile_plan(*FP8_ODD_K_TILE, n, k, 2)

@@ -94,10 +94,11 @@ def test_contiguous_keys_that_name_a_tile_of_256_rows(block_n, stages):
         assert _fp8_close(results[0][written].float(), ref[written])
 
 
-@pytest.mark.parametrize('tile,k', [(tile, k) for tile, depths in testing.FP8_WALK_CASES for k in depths])
+@pytest.mark.parametrize('tile,k', [(tile, k) for tile, depths in testing.FP8_WALK_CASES + testing.FP8_TWO_STAGE_LOOP_CASES for k in depths])
 def test_fp8_walk_over_several_tiles_of_few_k_tiles(tile, k):
     m, n = testing.FP8_WALK_SIZES
     _announce('fp8 walk', tile, k)
+    assert -(-m // tile[0]) * -(-n // tile[1]) > 2 * 8              # several tiles to a workgroup under the cap
     from yan_amd.jit_kernels import gemm
     (a8, sa), (b8, sb), out = testing.make_fp8_case(m, n, k, seed=16, device='cuda')
     name, keys, arg_defs, code_template = testing.fp8_explicit_tile_plan(*tile, n, k, 2)
@@ -111,6 +112,79 @@ def test_fp8_walk_over_several_tiles_of_few_k_tiles(tile, k):
         results.append(out.cpu())
     assert torch.equal(results[0], results[1])
     assert _fp8_close(results[0].float(), ref)
+
+
+@pytest.mark.parametrize('k', testing.MASKED_256_ROW_CASE[3])
+def test_masked_layout_on_256_row_tiles_one_after_the_other(k):
+    from yan_amd.jit_kernels import m_grouped_gemm
+    m, n, masked, _ = testing.MASKED_256_ROW_CASE
+    _announce('masked 256 rows', k)
+    (a8, sa), (b8, sb), out, mm = testing.make_grouped_masked_case(len(masked), m, n, k, masked, seed=26)
+    name, keys, arg_defs, code_template = testing.masked_256_row_plan(len(masked), n, k)
+    kernel = jit.build(name, arg_defs, jit.generate(m_grouped_gemm.includes, arg_defs, jit.cpp_format(code_template, keys)))
+    ref = torch.from_numpy(oracle.m_grouped_gemm_masked_ref(_codes(a8), sa.numpy(), _codes(b8), sb.numpy(), mm.numpy(), out_init=out.float().numpy()))
+    a8d, sad, b8d, sbd, mmd = a8.cuda(), sa.cuda(), b8.cuda(), sb.cuda(), mm.cuda()
+    assert len(masked) * -(-m // 256) * -(-n // 256) > 2 * 8
+    for expected_m in (m, 256):
+        results = []
+        for cap in (0, 8):
+            got = out.cuda()
+            assert kernel(a8d, sad, b8d, sbd, got, mmd, m, torch.cuda.current_stream(), cap, 0, sad.stride(1), sad.stride(2), sad.stride(0), expected_m) == 0
+            torch.cuda.synchronize()
+            results.append(got.cpu())
+        assert torch.equal(results[0], results[1])
+        for g, r in enumerate(masked):
+            assert torch.equal(results[0][g, r:], out[g, r:]) and (r == 0 or _fp8_close(results[0][g, :r].float(), ref[g, :r]))
+
+
+@pytest.mark.parametrize('col_major', [False, True])
+@pytest.mark.parametrize('m,n,k', testing.CAPI_STREAMED_FP8_SIZES)
+def test_library_streams_fp8_weights_to_the_same_bits(m, n, k, col_major):
+    """All columns (weights streamed) against either half of them (not), with K split where the plan splits it and without."""
+    from yan_amd import capi
+    _announce('library, streamed fp8 weights', m, n, k, col_major)
+    (a8, sa), (b8, sb), out = testing.make_fp8_case(m, n, k, seed=27, device='cuda', gen_device='cuda')
+    if col_major:
+        sa = yan.get_col_major_tensor(sa)
+    ref = testing.dequant_lhs(a8, sa.contiguous()) @ testing.dequant_rhs(b8, sb).t()
+    halves = []
+    for lo, hi in ((0, n // 2), (n // 2, n)):
+        halves.append(torch.full((m, hi - lo), float('nan'), dtype=torch.bfloat16, device='cuda'))
+        assert capi.gemm_fp8_fp8_bf16_nt((a8, sa), (b8[lo:hi], sb[lo // 128:hi // 128]), halves[-1]) == 0
+    out.fill_(float('nan'))
+    assert capi.gemm_fp8_fp8_bf16_nt((a8, sa), (b8, sb), out) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(out, torch.cat(halves, dim=1)) and _fp8_close(out.float(), ref)
+    out.fill_(float('nan'))
+    assert capi.gemm_fp8_fp8_bf16_nt_split_k((a8, sa), (b8, sb), out, capi.split_k_workspace()) == 0
+    torch.cuda.synchronize()
+    assert _fp8_close(out.float(), ref)
+    if capi.select_split_k(m, n, k, 256):           # the plan the entry compiles
+        jit_out = torch.full_like(out, float('nan'))
+        yan.gemm_fp8_fp8_bf16_nt((a8, sa), (b8, sb), jit_out)
+        torch.cuda.synchronize()
+        assert torch.equal(out, jit_out)
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.half])
+@pytest.mark.parametrize('m,n,k', testing.CAPI_STREAMED_DENSE_SIZES)
+def test_library_spreads_and_streams_16_bit_weights_as_the_entry_does(m, n, k, dtype):
+    from yan_amd import capi
+    _announce('library, spread and streamed weights', m, n, k, dtype)
+    a, b, c = testing.make_bf16_case(m, n, k, seed=28, dtype=dtype, device='cuda', gen_device='cuda')
+    (yan.gemm_bf16_tn if dtype == torch.bfloat16 else yan.gemm_fp16_tn)(a, b, c)
+    torch.cuda.synchronize()
+    a64, b64 = a.double(), b.double()
+    ref, magnitude = a64 @ b64.t(), a64.abs() @ b64.abs().t()
+    # rounding to 8 or 11 bits, and fp32 sums of k products: k * 2^-24 of the sum of their magnitudes at the most
+    bound = ref.abs() * (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) + magnitude * (k * 2.0 ** -24)
+    assert ((c.double() - ref).abs() <= bound).all()
+    unsplit, split = torch.full_like(c, float('nan')), torch.full_like(c, float('nan'))
+    assert (capi.gemm_bf16_tn if dtype == torch.bfloat16 else capi.gemm_fp16_tn)(a, b, unsplit) == 0
+    assert capi.gemm_bf16_tn_split_k(a, b, split, capi.split_k_workspace()) == 0
+    torch.cuda.synchronize()
+    assert ((unsplit.double() - ref).abs() <= bound).all()
+    assert torch.equal(split, c)                     # the same plan and kernel source
 
 
 @pytest.mark.parametrize('k', testing.FP8_ODD_K_SIZES[2])
