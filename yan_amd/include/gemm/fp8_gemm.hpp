@@ -50,12 +50,13 @@ namespace yan {
 // row, more requests than the operands if several waves ask for it: the first waves copy a part each, the others nothing. Rows
 // of whole 16-byte pieces, as row-major scales are where K is a multiple of 512, are copied four k-tiles at a time. Row-major,
 // every wave -> one wave -> four k-tiles: 512 x 7168 x 7168 62.8 -> 47.2 -> 39.8 us (37 token-contiguous); 640 x 9216 x 4096 47.3 -> 36.1 and
-// 1500 x 4096 x 4096 43.2 -> 35.8 with four, 900 x 4096 x 7040 53.7 -> 43.3 with one; fp8_scale_pieces_pay says where one is enough. Kernels of their own: the choice inside the
-// k-loop cost the token-contiguous layout 2 to 5 %.
+// 1500 x 4096 x 4096 43.2 -> 35.8 with four, 900 x 4096 x 7040 53.7 -> 43.3 with one; fp8_scale_pieces_pay says where one
+// is enough. Kernels of their own: the choice inside the k-loop cost the token-contiguous layout 2 to 5 %.
 enum class Fp8ScaleCopies { EveryWave, OneWave, FourKTiles };
 inline Fp8ScaleCopies fp8_scale_copies(const float* scales, int stride_m, int stride_k, int stride_g, int k, bool pieces_pay = true) {
     if (stride_m == 1) return Fp8ScaleCopies::EveryWave;
-    const bool pieces = pieces_pay && stride_k == 1 && stride_m % 4 == 0 && stride_g % 4 == 0 && k % 512 == 0 && reinterpret_cast<uintptr_t>(scales) % 16 == 0;
+    const bool pieces = pieces_pay && stride_k == 1 && stride_m % 4 == 0 && stride_g % 4 == 0 && k % 512 == 0 &&
+                        reinterpret_cast<uintptr_t>(scales) % 16 == 0;
     return pieces ? Fp8ScaleCopies::FourKTiles : Fp8ScaleCopies::OneWave;
 }
 
@@ -93,11 +94,14 @@ struct Fp8TileConfig {
     static constexpr int  RING_SCALE_BYTES = ceil_div(BLOCK_M * 4, 1024) * 1024;
     static constexpr int  RING_STAGE_BYTES = (LDS_ROWS_A + LDS_ROWS_B) * kRowBytes + RING_SCALE_BYTES;
     static constexpr bool RING_CAPABLE = BLOCK_M % 32 == 0 && (BLOCK_M / 8) % NUM_WAVES == 0 && BLOCK_N % 16 == 0;
-    // Behind the stages: room for activation scales that come four k-tiles at a time (Fp8ScaleCopies), 16 bytes a row; a slot is taken again when every k-tile of its four has been consumed, with STAGES - 1 k-tiles in flight. Then
-    // 1 KB that takes what copies of nothing write.
+    // Behind the stages: room for activation scales that come four k-tiles at a time (Fp8ScaleCopies), 16 bytes a row; a slot is
+    // taken again when every k-tile of its four has been consumed, with STAGES - 1 k-tiles in flight. Then 1 KB that takes what
+    // copies of nothing write.
     static constexpr int  SCALE_PARTS = ceil_div(BLOCK_M, 64);
     __host__ __device__ static constexpr int quad_slots(int stages) { return (stages + 6) / 4; }
-    __host__ __device__ static constexpr int ring_bytes(int stages, bool quad) { return stages * RING_STAGE_BYTES + ((quad ? quad_slots(stages) * SCALE_PARTS : 0) + 1) * 1024; }
+    __host__ __device__ static constexpr int ring_bytes(int stages, bool quad) {
+        return stages * RING_STAGE_BYTES + ((quad ? quad_slots(stages) * SCALE_PARTS : 0) + 1) * 1024;
+    }
     // At most 8 stages, 12 for the narrow tiles of the decode shapes (16 or 32 weight rows per workgroup): those have next
     // to nothing to compute per k-tile and run at the rate their compute unit takes bytes in, which needs many k-tiles in
     // flight (a stage is only 9 to 13 KB there). Measured with every unit pulling: about 60 GB/s per unit whatever the
@@ -537,11 +541,16 @@ fp8_gemm_tile(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
         const bool data = sl * LW + LW - 1 < GROUPS_AB || (sl * LW < GROUPS_AB && o < GROUPS_AB);
         const bool in_a = sl * LW + LW - 1 < GA || (sl * LW < GA && o < GA);
         if (data) {
-            if (in_a) __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_a : rsrc_none, YAN_LDS_CAST(stage + o * 8 * kRowBytes), kChunk, slot_voff[sl], kb * kRowBytes, 0, 0);
-            else __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_b : rsrc_none, YAN_LDS_CAST(stage + o * 8 * kRowBytes), kChunk, slot_voff[sl], kb * kRowBytes, 0, STREAM ? kNonTemporal : 0);
+            if (in_a)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_a : rsrc_none, YAN_LDS_CAST(stage + o * 8 * kRowBytes), kChunk, slot_voff[sl],
+                                                         kb * kRowBytes, 0, 0);
+            else
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(live ? rsrc_b : rsrc_none, YAN_LDS_CAST(stage + o * 8 * kRowBytes), kChunk, slot_voff[sl],
+                                                         kb * kRowBytes, 0, STREAM ? kNonTemporal : 0);
         } else {
             __builtin_amdgcn_raw_ptr_buffer_load_lds(live && (EVERY_WAVE || o == GROUPS_AB) ? rsrc_sa : rsrc_none,
-                                                     YAN_LDS_CAST(stage + TILE_BYTES + (EVERY_WAVE || o == GROUPS_AB ? 0 : 256)), 4, scale_voff, kb * sa_stride_k * 4, 0, 0);
+                                                     YAN_LDS_CAST(stage + TILE_BYTES + (EVERY_WAVE || o == GROUPS_AB ? 0 : 256)), 4, scale_voff,
+                                                     kb * sa_stride_k * 4, 0, 0);
         }
     };
 #pragma unroll
@@ -890,10 +899,9 @@ fp8_gemm_walk(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_sca
             fp8_store_slab<Cfg, true>(acc, region, rsrc_out, cur.m0 + wm * Cfg::WTM, cur.n0 + wn * Cfg::WTN, cur.m0, cur.n0, m, N,
                                       stream_out, lane_late);
         }
-        if (!nxt.valid) {
-            wait_for_copies();          // of weights nobody will read: none lands in LDS that is no longer this workgroup's
-            break;
-        }
+        // (copies of weights nobody will read are on their way here, as wherever a tile's loop ends: a wave's program does not
+        // end before its memory operations have, S_ENDPGM waits for them)
+        if (!nxt.valid) break;
         cur = nxt;
         // the next tile's second k-tile is copied into the stages the epilogue went through: every wave has to be out of them
         __builtin_amdgcn_s_waitcnt(waitcnt_imm(kNoWaitVm, 0));
@@ -940,15 +948,15 @@ fp8_gemm_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_s
     // A workgroup per slot (no cap): the tile without a loop around it. Inside the loop below the same code runs 2 to 14 %
     // slower on the ring tiles even for a single trip (64 x 7168 x 2048 on 64 x 32 tiles: 6.0 against 5.2 us).
     if (int(gridDim.x) >= num_slots) {
-        fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, STAGES, 1, false, false, STREAM, SCALES>(lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt,
-                                                                             sa_stride_m, sa_stride_k, grouped_layout, sa_stride_g,
-                                                                             int(blockIdx.x), num_groups, expected_m, two_stages);
+        fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, STAGES, 1, false, false, STREAM, SCALES>(
+            lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt, sa_stride_m, sa_stride_k, grouped_layout, sa_stride_g,
+            int(blockIdx.x), num_groups, expected_m, two_stages);
         return;
     }
     for (int slot = blockIdx.x; slot < num_slots; slot += gridDim.x) {
-        fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, STAGES, 1, false, false, STREAM, SCALES>(lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt,
-                                                                             sa_stride_m, sa_stride_k, grouped_layout, sa_stride_g,
-                                                                             slot, num_groups, expected_m, two_stages);
+        fp8_gemm_tile<SHAPE_N, SHAPE_K, BLOCK_M, BLOCK_N, kGemmType, STAGES, 1, false, false, STREAM, SCALES>(
+            lhs, lhs_scales, rhs, rhs_scales, out, m, n_rt, k_rt, sa_stride_m, sa_stride_k, grouped_layout, sa_stride_g,
+            slot, num_groups, expected_m, two_stages);
         if (slot + int(gridDim.x) < num_slots) __syncthreads();
     }
 }
@@ -1155,7 +1163,8 @@ public:
         if (slots >= kOutOfRange) return hipErrorInvalidValue;
         const int cus = device_cu_count(), grid = capped_grid(int(slots), num_sms, cus);
         hipLaunchKernelGGL((fp8_gemm_contiguous_rows_kernel<SHAPE_N, SHAPE_K, BLOCK_N, int(kNumStages)>), dim3(grid),
-                           dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream, static_cast<const uint8_t*>(lhs), lhs_scales, static_cast<const uint8_t*>(rhs), rhs_scales,
+                           dim3(fp8_launch_waves(BLOCK_M, BLOCK_N, int(kNumStages)) * kWaveSize), 0, stream,
+                           static_cast<const uint8_t*>(lhs), lhs_scales, static_cast<const uint8_t*>(rhs), rhs_scales,
                            reinterpret_cast<__bf16*>(out), m, n, k, lhs_scales_stride_m, lhs_scales_stride_k, grouped_layout, num_groups,
                            grid < cus ? grid : cus);
         return hipGetLastError();

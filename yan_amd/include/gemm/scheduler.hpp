@@ -241,11 +241,11 @@ __host__ __device__ inline int capped_grid(int slots, int num_sms, int device_cu
 }
 
 // Whether the plain FP8 GEMM on two LDS stages walks its tiles (fp8_gemm_walk) or runs a workgroup per tile: it walks, but for 3 to
-// 17 k-tiles, an odd number, and outputs of up to 64 MB. A short tile leaves the walk little to hide its seam under, and tiles handed out as
-// units fall free end more evenly: walk -> workgroup per tile, inputs changing, 7902 x 2624 x 640 26.7 -> 24.3 us, x 1152 38.6 -> 36.3, 8192 x
-// 2560 x 1152 38.8 -> 35.2, 4096 x 7168 x 896 38.7 -> 36.7, x 1664 56.3 -> 54.4, 5222 x 1792 x 384 12.3 -> 11.5. Larger outputs gain by the
-// walk at every K (8192 x 7168 x 384 42.6 -> 40.2 us, x 1152 78.2 -> 75.4), longer K gain at every size (4096 x 7168 x 9344 234 -> 230), and even numbers
-// of k-tiles walk as they always have.
+// 17 k-tiles, an odd number, and outputs of up to 64 MB. A short tile leaves the walk little to hide its seam under, and tiles handed
+// out as units fall free end more evenly: walk -> workgroup per tile, inputs changing, 7902 x 2624 x 640 26.8 -> 24.2 us, x 1152 38.3 ->
+// 35.7, 8192 x 2560 x 1152 38.9 -> 36.0 (x 384 20.1 -> 21.3), 4096 x 7168 x 896 39.4 -> 36.6, x 1664 55.5 -> 53.9, 5222 x 1792 x 384 12.5 ->
+// 11.7. Larger outputs gain by the walk at every K (8192 x 7168 x 384 42.6 -> 40.2 us, x 1152 78.2 -> 75.4), longer K gain at every
+// size (4096 x 7168 x 9344 234 -> 230), and even numbers of k-tiles walk as they always have.
 __host__ __device__ constexpr bool fp8_walk_pays(int k, uint64_t output_bytes) {
     return k % 256 == 0 || k > 17 * 128 || output_bytes > (uint64_t(64) << 20);
 }
@@ -281,7 +281,8 @@ __host__ __device__ constexpr uint64_t contiguous_weight_bytes(int num_groups, i
     return uint64_t(num_groups < blocks ? num_groups : blocks) * n * k;
 }
 
-// Whether four k-tiles of row-major scales a copy (Fp8ScaleCopies) are worth it in an unsplit plain FP8 GEMM of `tile_rows` rows of BLOCK_M x BLOCK_N tiles.
+// Whether four k-tiles of row-major scales a copy (Fp8ScaleCopies) are worth it in an unsplit plain FP8 GEMM of `tile_rows` rows of
+// BLOCK_M x BLOCK_N tiles.
 // On 64 x 64 tiles in a loop (K beyond 2048) they are not while a row's scales are at most one cache line (K = 4096), which stays in
 // the caches from copy to copy where four tile rows and more read it: four a copy -> one, 300 x 2112 x 2560 11.0 -> 10.2 us, 395 x 1728 x
 // 3072 12.7 -> 11.8, 500 x 1088 x 4096 15.3 -> 13.4, 256 x 4096 x 4096 17.0 -> 16.4. They are elsewhere: 64 x 64 with K = 1024 (256 x
