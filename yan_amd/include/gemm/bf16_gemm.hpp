@@ -139,8 +139,8 @@ dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
     using StB = TileStager<BLOCK_N, LW>;
     constexpr int NUM_COPIES = StA::PASSES + StB::PASSES;
     static_assert(StA::PADDED_ROWS == BLOCK_M && StB::PADDED_ROWS == BLOCK_N, "tiles are whole copy passes");
-    // Workgroups march along K in step. Where rows are a multiple of 16 KB apart, one k-tile of all rows lies in a few of the memory
-    // channels, which all of them then ask at a time: there (kSpreadStarts) the columns of the tiles start at places spread over
+    // Workgroups march along K in step. Where rows are a multiple of 16 KB apart, one k-tile of all rows should by its addresses lie in a
+    // few of the memory channels, which all of them then ask at a time: there (kSpreadStarts) the columns of the tiles start at places spread over
     // their range, multiples of the golden ratio, and come round to the k-tiles in front at the end. At other depths it changes
     // nothing (K = 7168) or loses 1 % (4096). Which launches gain by it, and the times: spreads_starts in scheduler.hpp.
     constexpr bool SPREAD = (COPIES & kSpreadStarts) != 0;
