@@ -209,6 +209,8 @@ int main() {
         // Row-major scales four k-tiles at a time: not where many 64 x 64 tile rows loop over few of them.
         CHECK(!yan::fp8_scale_pieces_pay(5, 64, 64, 2560) && !yan::fp8_scale_pieces_pay(4, 64, 64, 4096) && yan::fp8_scale_pieces_pay(3, 64, 64, 2560));
         CHECK(yan::fp8_scale_pieces_pay(5, 64, 64, 2048) && yan::fp8_scale_pieces_pay(5, 64, 64, 4608) && yan::fp8_scale_pieces_pay(5, 64, 128, 2560));
+        // Weights whose rows end inside a 128-byte line are not streamed.
+        CHECK(!yan::streams_weights(1, 12628ull * 4760 * 2, 4760 * 2) && yan::streams_weights(1, 12672ull * 4736 * 2, 4736 * 2));
         // A contiguous layout of few blocks reads few groups' weights.
         CHECK(yan::contiguous_weight_bytes(59, 1280, 5184, 1792) == 10ull * 5184 * 1792 && yan::contiguous_weight_bytes(4, 1280, 512, 256) == 4ull * 512 * 256);
         CHECK(!yan::streams_weights(1, yan::contiguous_weight_bytes(59, 1280, 5184, 1792), 1792));

@@ -269,9 +269,10 @@ __host__ __device__ constexpr bool fp8_walk_streams_output(uint64_t bytes, int k
 // 4096 13.4 -> 16.0, contiguous 32 x 64 rows x 2048 x 2048 14.7 -> 16.9). Tile rows drift apart along a long K, most of all where the last
 // is ragged and runs ahead, and a panel that one has let go comes from HBM again for the next: FP8 300 x 8192 x 5120 28.3 -> 33.1,
 // 16-bit 300 x 5000 x 7168 36.0 -> 44.9, where 256 rows, in step, gain 1 to 5 %; five tile rows and more are on two XCDs (900 x 3072 x
-// 7168 on 64 x 192 62 -> 76.5).
+// 7168 on 64 x 192 62 -> 76.5). Rows of no whole 128-byte lines are read plainly: a k-tile ends inside a line, and the rest of it, wanted
+// a k-tile later, is no longer there (fp16 26 x 12628 x 4760 35.7 -> 39.1).
 __host__ __device__ constexpr bool streams_weights(int tile_rows, uint64_t weight_bytes, int row_bytes) {
-    return (tile_rows <= 1 || (tile_rows <= 4 && row_bytes <= 4096)) && weight_bytes >= (uint64_t(96) << 20);
+    return (tile_rows <= 1 || (tile_rows <= 4 && row_bytes <= 4096)) && row_bytes % 128 == 0 && weight_bytes >= (uint64_t(96) << 20);
 }
 
 // Weights that a contiguous grouped launch reads at the most: of as many groups as it has blocks of 128 rows. (With 59 groups and ten
