@@ -238,7 +238,7 @@ def main():
         'steps': args.steps, 'warmup': args.warmup, 'ms_per_step': round(wall_ms, 5),
         'higher_is_better': True, 'scaling': 'weak', 'vs_baseline': None, 'dtype': 'fp8_e4m3 (fp32 accumulate, bf16 out)',
         'data': 'synthetic: N(0,1) sources, seed 42, quantised per-token 1x128 / per-block 128x128',
-        'config': {'workload': 'configs[2]: FP8 e4m3 block-scaled GEMM M=4096 N=7168 K=7168, bf16 out',
+        'config': {'workload': 'FP8 e4m3 block-scaled GEMM M=4096 N=7168 K=7168, bf16 out',
                    'tile': f"{keys['BLOCK_M']}x{keys['BLOCK_N']}x128", 'cache_state': 'warm (same operands every step)',
                    'settle_launches': settle['cfg3'],
                    'settle': 'untimed launches of the same kernel before the warm-up: the power controller takes ~100 launches '
@@ -263,7 +263,7 @@ def main():
 
     extra = {}
     if not args.no_extra:
-        # configs[1]: bf16 8192^3, next to torch.matmul (hipBLASLt) on the same operands
+        # bf16 8192^3, next to torch.matmul (hipBLASLt) on the same operands
         mm, nn, kk = harness.BASELINE_BF16['cfg2']
         a, b, c = harness.make_bf16_case(mm, nn, kk, seed=42, scale=kk ** -0.5, device='cuda', gen_device='cuda')
         ms, _ = _event_time_ms(lambda: yan.gemm_bf16_tn(a, b, c), 20, 5, settle['cfg2'])
@@ -285,7 +285,7 @@ def main():
         if load and load['shader_clock_mhz']:
             extra['bf16_8192_torch_hipblaslt']['under_load'] = load
         del a, b, c
-        # configs[3]: the M=64 decode shape, HBM-bound. The kernel is shorter than the host side of a call, so its
+        # the M=64 decode shape, HBM-bound. The kernel is shorter than the host side of a call, so its
         # device time comes from the profiler; cold = a 512 MB write before every call.
         mm, nn, kk = harness.BASELINE_FP8['cfg4']
         (x8, sx), (w8, sw), o = harness.make_fp8_case(mm, nn, kk, seed=42, device='cuda')
@@ -356,7 +356,7 @@ def main():
             'call_to_call_us_quantiser_then_gemm_two_calls': round(wall_two * 1e3, 2),
             'call_to_call_us_one_call': round(wall_one * 1e3, 2), 'quantiser_kernel_us': round(t_cast * 1e6, 2), 'same_bits': True}
         del x8, sx, w8, sw, o, xb
-        # configs[4]: FP8 16384^3, uniform[-4, 4] sources with 1 % of the entries x 50
+        # FP8 16384^3, uniform[-4, 4] sources with 1 % of the entries x 50
         mm, nn, kk = harness.BASELINE_FP8['cfg5']
         (x8, sx), (w8, sw), o = harness.make_fp8_case(mm, nn, kk, seed=42, dist='outlier', device='cuda', gen_device='cuda')
         sx = yan.get_col_major_tensor(sx)
