@@ -219,6 +219,21 @@ FLOAT_TEST_SHAPES = [(128, 64, 16), (128, 64, 1), (128, 192, 17), (256, 320, 100
 FLOAT_SPLIT_K_SHAPES = {(128, 64, 2050): (32, 32, 7), (256, 320, 3001): (32, 32, 3), (384, 320, 3001): (32, 64, 4), (128, 576, 4099): (32, 64, 6),
                         (1024, 320, 2050): (64, 64, 3), (256, 704, 4110): (64, 64, 5), (256, 2112, 2111): (128, 64, 3),
                         (128, 2112, 9001): (64, 64, 7), (640, 832, 1997): (128, 64, 7)}
+# fp32 on the bf16 matrix cores: (tile, parts, (m, n, k)) built through explicit keys. Ragged tiles on both sides, K around the 16 rows of an
+# MFMA and the k-tiles of 16, 32 and 64 rows, fewer k-tiles than stages, parts of unequal length and parts without any
+FLOAT_BF16X3_CASES = [((256, 256), 1, (300, 260, 1)), ((256, 256), 1, (256, 516, 95)), ((256, 256), 3, (260, 256, 145)),
+                      ((256, 128), 1, (260, 132, 33)), ((256, 128), 2, (512, 128, 97)), ((128, 256), 1, (132, 260, 31)), ((128, 256), 4, (128, 512, 130)),
+                      ((128, 128), 1, (132, 132, 17)), ((128, 128), 1, (256, 256, 128)), ((128, 128), 5, (128, 256, 650)),
+                      ((128, 64), 1, (4, 4, 16)), ((128, 64), 1, (132, 68, 64)), ((128, 64), 7, (128, 2112, 1000)), ((128, 64), 15, (256, 64, 200))]
+
+
+def float_bf16x3_explicit_plan(tile, parts):
+    """(name, keys, arg_defs) of the fp32 kernel on the bf16 matrix cores with this tile and split."""
+    from yan_amd.jit_kernels import simple_gemm
+    keys = {'BLOCK_M': tile[0], 'BLOCK_N': tile[1], 'SPLIT_K': parts, 'WORKSPACE': ', workspace, workspace_bytes' if parts > 1 else ''}
+    return 'gemm_float_nt_bf16x3' + ('_split_k' if parts > 1 else ''), keys, simple_gemm.split_k_arg_defs if parts > 1 else simple_gemm.arg_defs
+
+
 FP8_TEST_SHAPES = [
     (4096, 7168, 7168), (64, 4096, 7168), (16384, 16384, 16384),
     (64, 256, 384), (512, 1024, 1024), (1, 128, 128), (63, 192, 256), (129, 320, 128), (300, 96, 640),
@@ -612,6 +627,13 @@ def jit_kernels_in_use(num_cus: int = 256):
         plan = simple_gemm.float_split_k_plan(m, n, k, num_cus)
         if plan is not None:
             add(plan[0], plan[2], simple_gemm.includes, simple_gemm.split_k_template, plan[1])
+    for m, n, k in list(FLOAT_SPLIT_K_SHAPES) + REFERENCE_FLOAT_TEST_SHAPES + FLOAT_TEST_SHAPES + [(5120, 2048, 4096), (4096, 4096, 1024), (8192, 8192, 8192)]:
+        plan = simple_gemm.float_bf16x3_plan(m, n, k, num_cus)
+        if plan is not None:
+            add(plan[0], plan[2], simple_gemm.bf16x3_includes, simple_gemm.bf16x3_template, plan[1])
+    for tile, parts in sorted({(tile, parts) for tile, parts, _ in FLOAT_BF16X3_CASES}):
+        name, keys, arg_defs = float_bf16x3_explicit_plan(tile, parts)
+        add(name, arg_defs, simple_gemm.bf16x3_includes, simple_gemm.bf16x3_template, keys)
     for kind in ('per_token', 'per_block'):
         for dtype in (torch.bfloat16, torch.float32):
             name, keys, arg_defs, code_template = fp8_cast.cast_kernel_plan(kind, dtype)

@@ -721,6 +721,24 @@ def test_fp32_split_k_counts_the_rounds_of_the_fullest_xcd():
                     assert rounds * us[tile] / split < ceil_div(ceil_div(m, whole[0]) * ceil_div(n, whole[1]), 256) * us[whole]
 
 
+def test_fp32_plans_on_the_bf16_cores_fit_their_workspace():
+    from yan_amd.jit_kernels import simple_gemm, split_k
+    from yan_amd.jit_kernels.utils import ceil_div
+    assert heuristics.get_float_bf16x3_config(1024, 1024, 1023, 256) is None and heuristics.get_float_bf16x3_config(128, 2112, 7168, 256) == (128, 64, 7)
+    for m in (128, 384, 1024, 4096):
+        for n in range(64, 8193, 832):
+            for k in (1, 300, 2050, 8191):
+                plan = heuristics.get_float_bf16x3_config(m, n, k, 256)
+                whole = heuristics.get_float_bf16x3_config(m, n, k, 256, may_split=False)
+                assert (plan is None) == (whole is None) == (m * n * k < heuristics.FLOAT_BF16X3_MIN_MNK)
+                if plan is not None:
+                    tiles = ceil_div(m, plan[0]) * ceil_div(n, plan[1])
+                    assert whole[2] == 1
+                    assert plan[2] == 1 or (split_k.SPLIT_K_COUNTER_BYTES + tiles * plan[0] * plan[1] * plan[2] * 4 <= split_k.SPLIT_K_WORKSPACE_BYTES
+                                            and tiles * 8 * 4 <= split_k.SPLIT_K_COUNTER_BYTES)
+                    assert simple_gemm.float_bf16x3_plan(m, n, k, 256)[2] is (simple_gemm.split_k_arg_defs if plan[2] > 1 else simple_gemm.arg_defs)
+
+
 @pytest.mark.parametrize('kind,streams_codes', [('per_token', False), ('per_block', True)])
 def test_codes_of_activations_are_stored_for_the_gemm_behind(tmp_path, kind, streams_codes):
     """The GEMM that follows a per-token cast reads its codes from the caches: no store of them carries the non-temporal hint.

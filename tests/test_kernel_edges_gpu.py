@@ -305,6 +305,97 @@ def test_float_split_k_matches_the_oracle_and_repeats(m, n, k):
     assert int(workspace[:split_k.SPLIT_K_COUNTER_BYTES].view(torch.int32).abs().sum()) == 0
 
 
+def _run_float_bf16x3(tile, parts, a, b, c, alpha=1.0, beta=0.0):
+    from yan_amd.jit_kernels import simple_gemm, split_k
+    name, keys, arg_defs = testing.float_bf16x3_explicit_plan(tile, parts)
+    kernel = jit.build(name, arg_defs, jit.generate(simple_gemm.bf16x3_includes, arg_defs, jit.cpp_format(simple_gemm.bf16x3_template, keys)))
+    stream = torch.cuda.current_stream()
+    args = (a.size(0), b.size(0), a.size(1), alpha, a, a.size(0), b, b.size(0), beta, c, c.size(1), stream)
+    if parts > 1:
+        workspace, _ = split_k.split_k_workspace(c.device, stream.cuda_stream)
+        args += (workspace, split_k.SPLIT_K_WORKSPACE_BYTES)
+    assert kernel(*args) == 0
+
+
+@pytest.mark.parametrize('tile,parts,shape', testing.FLOAT_BF16X3_CASES)
+def test_float_on_the_bf16_cores_matches_the_product(tile, parts, shape):
+    m, n, k = shape
+    _announce('fp32 on bf16 cores', tile, parts, shape)
+    a, b, _ = testing.make_float_case(m, n, k, seed=17, device='cuda')
+    start = torch.randn(m + 1, n, generator=torch.Generator().manual_seed(18)).cuda()
+    ad, bd = a.double(), b.double()
+    # at most k + 16 roundings in a row, each relative to the sum of magnitudes
+    bound = (k + 16) * 2.0 ** -24 * (ad.abs() @ bd.abs().t() + start[:m].abs().double()) * 2
+    for alpha, beta in ((1.0, 0.0), (-0.5, 2.0)):
+        results = []
+        for _ in range(2):
+            c = start.clone() if beta else torch.full_like(start, float('nan'))
+            _run_float_bf16x3(tile, parts, a, b, c[:m], alpha, beta)
+            results.append(c)
+        want = alpha * (ad @ bd.t()) + (beta * start[:m].double() if beta else 0.0)
+        assert torch.equal(results[0][:m], results[1][:m])
+        assert bool(((results[0][:m].double() - want).abs() <= bound).all())
+        assert torch.equal(results[0][m], start[m]) if beta else bool(results[0][m].isnan().all())
+
+
+@pytest.mark.parametrize('tile,parts', [((256, 256), 1), ((128, 128), 5), ((128, 64), 7)])
+def test_floats_that_do_not_come_apart_take_the_fp32_cores(tile, parts):
+    """Numbers too small for three bf16, too large for the first of them, infinities, NaN and sums that leave the range give what the fp32
+    matrix cores give; each kind alone, so that none hides behind another's second run of the tile."""
+    m, n, k = 256, 256, 700
+    big = torch.finfo(torch.float32).max
+    for kind in ('tiny', 'subnormal', 'largest', 'infinity', 'nan', 'overflow'):
+        _announce('fp32 on bf16 cores', tile, parts, kind)
+        a, b, c = testing.make_float_case(m, n, k, seed=19, device='cuda')
+        if kind == 'tiny':
+            a[5] *= 2.0 ** -122
+            b[:, ::2] *= 2.0 ** 60
+        elif kind == 'subnormal':
+            a[5, 3], a[5, 4:] = 2.0 ** -140, 0.0
+            a[5, :3] = 0.0
+            b[:, 3] = 2.0 ** 100
+        elif kind == 'largest':
+            a[5, 7] = big
+            b[:, 7] = 2.0 ** -100
+        elif kind == 'infinity':
+            a[5, 7], b[9, 8] = float('inf'), float('-inf')
+        elif kind == 'nan':
+            a[5, 7] = float('nan')
+        else:
+            a[5, :200], b[9, :200] = 2.0 ** 65, 2.0 ** 63
+        _run_float_bf16x3(tile, parts, a, b, c)
+        ad, bd = a.double(), b.double()
+        want = ad @ bd.t()
+        beyond = want.isnan() | (want.abs() > big)
+        assert bool(beyond[5].any()) == (kind in ('infinity', 'nan', 'overflow'))
+        assert torch.equal(c.isnan(), want.isnan()) and torch.equal(c[beyond & ~want.isnan()].double(), want[beyond & ~want.isnan()].sign() * float('inf'))
+        bound = (k + 16) * 2.0 ** -24 * (ad.abs() @ bd.abs().t()) * 2
+        assert bool(((c.double() - want).abs() <= bound)[~beyond].all())
+
+
+@pytest.mark.parametrize('m,n,k', [(1024, 1024, 1024), (128, 2112, 7168), (640, 5120, 331)])
+def test_float_on_the_bf16_cores_is_no_further_from_the_product(m, n, k):
+    """Against 64 bits the error is no larger than on the fp32 matrix cores, with the same tile's parts of K or without."""
+    from yan_amd.jit_kernels import simple_gemm
+    _announce('fp32 error', m, n, k)
+    name, keys, arg_defs = simple_gemm.float_kernel_plan(m, n, 256)
+    fp32 = jit.build(name, arg_defs, jit.generate(simple_gemm.includes, arg_defs, jit.cpp_format(simple_gemm.template, keys)))
+    for kind in ('normal', 'positive', 'wide'):
+        a, b, c = testing.make_float_case(m, n, k, seed=23, device='cuda')
+        if kind == 'positive':
+            a, b = a.abs(), b.abs()
+        elif kind == 'wide':
+            a = a * torch.exp(3.0 * torch.randn(k, m, generator=torch.Generator().manual_seed(24)).cuda().t())
+        want = a.double() @ b.double().t()
+        assert fp32(m, n, k, 1.0, a, m, b, n, 0.0, c, n, torch.cuda.current_stream()) == 0
+        before = ((c.double() - want).norm() / want.norm()).item()
+        c.fill_(float('nan'))
+        _run_float_bf16x3((128, 64), 1, a, b, c)
+        after = ((c.double() - want).norm() / want.norm()).item()
+        print(f'{kind}: {before:.2e} -> {after:.2e}', flush=True)
+        assert after <= before
+
+
 def _odd_floats(shape, dtype, seed):
     """Every kind of bit pattern: subnormals, huge values, zeros of both signs, and infinities and NaN here and there."""
     g = torch.Generator().manual_seed(seed)

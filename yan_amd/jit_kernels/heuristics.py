@@ -359,3 +359,38 @@ def get_split_k_float_config(m: int, n: int, k: int, num_cus: int) -> Optional[T
             if t < best:
                 best, best_plan = t, (bm, bn, split)
     return best_plan
+
+
+# The fp32 GEMM on the bf16 matrix cores (gemm/simple_gemm_bf16x3.hpp): depth of a k-tile, microseconds per k-tile while few compute
+# units work, microseconds a tile costs besides (first copies, sums of its waves, epilogue). Fitted, with the rest of the model below, to
+# 190 shapes with every tile and split forced in turn, operands cycling: its pick takes 1.015 of the fastest's time on average, 1.13 at
+# worst above the limit.
+_FLOAT_BF16X3_TILES = {(256, 256): (16, 1.16, 9.8), (256, 128): (32, 1.15, 7.0), (128, 256): (32, 1.17, 6.8), (128, 128): (64, 1.18, 6.9),
+                       (128, 64): (64, 0.69, 4.9)}
+FLOAT_BF16X3_SPLIT_FACTORS = (1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 15)
+# m * n * k from which it is the faster one: above it 78 shapes took 0.50 to 1.00 of the fp32 matrix cores' time (0.72 on average), below
+# 5e8 it loses nearly everywhere (640 x 320 x 1153 9.3 against 13.9 us), in between it goes either way.
+FLOAT_BF16X3_MIN_MNK = 1 << 30
+
+
+def get_float_bf16x3_config(m: int, n: int, k: int, num_cus: int, may_split: bool = True) -> Optional[Tuple[int, int, int]]:
+    """(BLOCK_M, BLOCK_N, SPLIT_K) when the fp32 GEMM should run on the bf16 matrix cores, else None. Modelled time: rounds x (k-tiles of a
+    part x the tile's time per k-tile, twice that where every compute unit works (the power limit) + the tile's other costs) + 1.5 us, and
+    for a split 1.8 us + 13 ns per KB of partial sums the last part reads."""
+    if m * n * k < FLOAT_BF16X3_MIN_MNK:
+        return None
+    best, plan = None, None
+    for (bm, bn), (block_k, per_k_tile, per_tile) in _FLOAT_BF16X3_TILES.items():
+        tiles, k_tiles = ceil_div(m, bm) * ceil_div(n, bn), ceil_div(k, block_k)
+        for split in FLOAT_BF16X3_SPLIT_FACTORS if may_split else (1,):
+            # 16 MB of partial sums, eight counters per tile in 16 KB, two k-tiles per part
+            if split > 1 and (tiles * split * bm * bn * 4 > 1 << 24 or tiles > 512 or ceil_div(k_tiles, split) < 2):
+                continue
+            rounds = ceil_div(tiles * split, num_cus)
+            busy = tiles * split / (num_cus * rounds)
+            t = 1.5 + rounds * (ceil_div(k_tiles, split) * per_k_tile * (1 + busy) + per_tile)
+            if split > 1:
+                t += 1.8 + split * bm * bn * 4 / 1024 * 0.0133
+            if best is None or t < best:
+                best, plan = t, (bm, bn, split)
+    return plan
