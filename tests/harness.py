@@ -219,6 +219,12 @@ FLOAT_TEST_SHAPES = [(128, 64, 16), (128, 64, 1), (128, 192, 17), (256, 320, 100
 FLOAT_SPLIT_K_SHAPES = {(128, 64, 2050): (32, 32, 7), (256, 320, 3001): (32, 32, 3), (384, 320, 3001): (32, 64, 4), (128, 576, 4099): (32, 64, 6),
                         (1024, 320, 2050): (64, 64, 3), (256, 704, 4110): (64, 64, 5), (256, 2112, 2111): (128, 64, 3),
                         (128, 2112, 9001): (64, 64, 7), (640, 832, 1997): (128, 64, 7)}
+# 16-bit ring tiles whose rows do not start on cache lines: (tile, stages), and (m, n, k, elements the operands start behind a line): every
+# shift from row to row (8 and 56 elements a row, 24, 40), K that ends right behind a window and one chunk into it, operands shifted alike and not
+DENSE_LINE_WINDOW_TILES = [((128, 256), 3), ((128, 192), 4), ((128, 128), 5), ((64, 192), 5), ((64, 128), 6)]
+DENSE_LINE_WINDOW_SHAPES = [(131, 260, 264, 0, 0), (70, 132, 312, 8, 40), (257, 388, 328, 56, 0), (64, 68, 424, 24, 24), (130, 516, 1016, 48, 8)]
+
+
 # fp32 on the bf16 matrix cores: (tile, parts, (m, n, k)) built through explicit keys. Ragged tiles on both sides, K around the 16 rows of an
 # MFMA and the k-tiles of 16, 32 and 64 rows, fewer k-tiles than stages, parts of unequal length and parts without any
 FLOAT_BF16X3_CASES = [((256, 256), 1, (300, 260, 1)), ((256, 256), 1, (256, 516, 95)), ((256, 256), 3, (260, 256, 145)),
@@ -631,6 +637,10 @@ def jit_kernels_in_use(num_cus: int = 256):
         plan = simple_gemm.float_bf16x3_plan(m, n, k, num_cus)
         if plan is not None:
             add(plan[0], plan[2], simple_gemm.bf16x3_includes, simple_gemm.bf16x3_template, plan[1])
+    for tile, _ in DENSE_LINE_WINDOW_TILES + [((64, 64), 8)]:
+        for dtype in (torch.bfloat16, torch.half):
+            name, keys, arg_defs, includes, code_template = dense_tile_plan(tile, dtype, 0)
+            add(name, arg_defs, includes, code_template, keys)
     for tile, parts in sorted({(tile, parts) for tile, parts, _ in FLOAT_BF16X3_CASES}):
         name, keys, arg_defs = float_bf16x3_explicit_plan(tile, parts)
         add(name, arg_defs, simple_gemm.bf16x3_includes, simple_gemm.bf16x3_template, keys)

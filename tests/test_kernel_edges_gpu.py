@@ -305,6 +305,33 @@ def test_float_split_k_matches_the_oracle_and_repeats(m, n, k):
     assert int(workspace[:split_k.SPLIT_K_COUNTER_BYTES].view(torch.int32).abs().sum()) == 0
 
 
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.half])
+@pytest.mark.parametrize('tile,stages', testing.DENSE_LINE_WINDOW_TILES)
+def test_rows_off_cache_lines_give_the_bits_of_the_smallest_tile(tile, stages, dtype):
+    """Ring tiles that copy lines instead of rows' k-tiles (LineStager) against the 64 x 64 tile, which does not, and the product."""
+    def kernel(which):
+        name, keys, arg_defs, includes, code_template = testing.dense_tile_plan(which, dtype, 0)
+        assert which != tile or keys['NUM_STAGES'] == stages
+        return jit.build(name, arg_defs, jit.generate(includes, arg_defs, jit.cpp_format(code_template, keys)))
+    lines, plain = kernel(tile), kernel((64, 64))
+    for m, n, k, off_a, off_b in testing.DENSE_LINE_WINDOW_SHAPES:
+        _announce('rows off lines', tile, dtype, m, n, k, off_a, off_b)
+        g = torch.Generator().manual_seed(29)
+        a_buf, b_buf = (torch.randn(rows * k + off + 64, generator=g).to(dtype).cuda() for rows, off in ((m, off_a), (n, off_b)))
+        # what surrounds the operands must not get into a sum
+        a_buf[:off_a], a_buf[off_a + m * k:], b_buf[:off_b], b_buf[off_b + n * k:] = (float('nan'),) * 4
+        a, b = a_buf[off_a:off_a + m * k].view(m, k), b_buf[off_b:off_b + n * k].view(n, k)
+        got, want = (torch.full((m + 2, n), 7.0, dtype=dtype, device='cuda') for _ in range(2))
+        stream = torch.cuda.current_stream()
+        assert lines(m, n, k, a, b, got[:m], stream) == 0 and plain(m, n, k, a, b, want[:m], stream) == 0
+        assert torch.equal(got, want) and bool((got[m:] == 7.0).all())
+        ad, bd = a.double(), b.double()
+        ref = ad @ bd.t()
+        # one rounding to the type, and at most k + 8 in a row of fp32 sums relative to the sum of magnitudes
+        bound = ref.abs() * 2.0 ** (-8 if dtype == torch.bfloat16 else -11) + (k + 8) * 2.0 ** -24 * (ad.abs() @ bd.abs().t())
+        assert bool(((got[:m].double() - ref).abs() <= bound).all())
+
+
 def _run_float_bf16x3(tile, parts, a, b, c, alpha=1.0, beta=0.0):
     from yan_amd.jit_kernels import simple_gemm, split_k
     name, keys, arg_defs = testing.float_bf16x3_explicit_plan(tile, parts)

@@ -90,9 +90,10 @@ __host__ __device__ constexpr int dense_launch_waves(int block_m, int block_n, i
 }
 
 // COPIES: how a ring tile's copies go about K and B, chosen by the launcher (with_dense_copies): bits kStreamedWeights, the copies of B
-// carry the non-temporal hint (streams_weights in scheduler.hpp), and kSpreadStarts. Compiled in, since looking at a start in
+// carry the non-temporal hint (streams_weights in scheduler.hpp), and kSpreadStarts, or kLineWindows alone (LineStager in tile_io.hpp).
+// Compiled in, since looking at a start in
 // every k-tile cost the depths that have none 1 to 4 % (90 x 5004 x 2048 9.4 -> 9.8 us, 37 x 4096 x 7168 15.1 -> 15.3).
-constexpr int kStreamedWeights = 1, kSpreadStarts = 2;
+constexpr int kStreamedWeights = 1, kSpreadStarts = 2, kLineWindows = 4;
 template <typename Atom, typename Elem, int BLOCK_M, int BLOCK_N, int STAGES, int SPLIT_K = 1, int COPIES = 0>
 __device__ __forceinline__ void
 dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, Elem* __restrict__ C,
@@ -115,18 +116,27 @@ dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
     const int wn = wave % Cfg::WAVES_N, wm = wave / Cfg::WAVES_N;
 
     const uint32_t ld_bytes = uint32_t(k) * 2;
-    const __amdgpu_buffer_rsrc_t rsrc_a = make_rsrc(A, uint32_t(m) * ld_bytes);
-    const __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(B, uint32_t(n) * ld_bytes);
-    TileStager<BLOCK_M, LW> stage_a;
-    TileStager<BLOCK_N, LW, (COPIES & kStreamedWeights) != 0> stage_b;
-    stage_a.init(m0, ld_bytes, wave, lane);
-    stage_b.init(n0, ld_bytes, wave, lane);
+    constexpr bool WINDOWS = (COPIES & kLineWindows) != 0;
+    using StA = std::conditional_t<WINDOWS, LineStager<BLOCK_M, LW>, TileStager<BLOCK_M, LW>>;
+    using StB = std::conditional_t<WINDOWS, LineStager<BLOCK_N, LW>, TileStager<BLOCK_N, LW, (COPIES & kStreamedWeights) != 0>>;
+    const __amdgpu_buffer_rsrc_t rsrc_a = StA::rsrc(A, uint32_t(m) * ld_bytes);
+    const __amdgpu_buffer_rsrc_t rsrc_b = StB::rsrc(B, uint32_t(n) * ld_bytes);
+    StA stage_a;
+    StB stage_b;
+    if constexpr (WINDOWS) {
+        stage_a.init(A, m0, k, wave, lane);
+        stage_b.init(B, n0, k, wave, lane);
+    } else {
+        stage_a.init(m0, ld_bytes, wave, lane);
+        stage_b.init(n0, ld_bytes, wave, lane);
+    }
 
     // k-tiles: `num_k_tiles` in all, the last one possibly partial (only `tail_bytes` of each row exist).
     const int k_bytes = k * 2;
     const int num_k_tiles = ceil_div(k_bytes, kRowBytes);
     const int tail_tile = (k_bytes % kRowBytes) ? num_k_tiles - 1 : -1;
-    const uint32_t tail_a = stage_a.tail_voff(k_bytes % kRowBytes), tail_b = stage_b.tail_voff(k_bytes % kRowBytes);
+    [[maybe_unused]] uint32_t tail_a = 0, tail_b = 0;
+    if constexpr (!WINDOWS) tail_a = stage_a.tail_voff(k_bytes % kRowBytes), tail_b = stage_b.tail_voff(k_bytes % kRowBytes);
     // this part's k-tiles; copies past them keep the count of instructions in flight and move nothing
     int kt_lo = 0, kt_hi = num_k_tiles;
     if constexpr (SPLIT_K > 1) {
@@ -135,8 +145,6 @@ dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
         kt_hi = min(kt_lo + per, num_k_tiles);
     }
     const __amdgpu_buffer_rsrc_t rsrc_none = make_rsrc(A, 0);
-    using StA = TileStager<BLOCK_M, LW>;
-    using StB = TileStager<BLOCK_N, LW>;
     constexpr int NUM_COPIES = StA::PASSES + StB::PASSES;
     static_assert(StA::PADDED_ROWS == BLOCK_M && StB::PADDED_ROWS == BLOCK_N, "tiles are whole copy passes");
     // Workgroups march along K in step. Where rows are a multiple of 16 KB apart, one k-tile of all rows should by its addresses lie in a
@@ -145,23 +153,31 @@ dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
     // nothing (K = 7168) or loses 1 % (4096). Which launches gain by it, and the times: spreads_starts in scheduler.hpp.
     constexpr bool SPREAD = (COPIES & kSpreadStarts) != 0;
     const int range = kt_hi - kt_lo, first = SPREAD && range > 0 ? int(__umulhi(uint32_t(tile.n_idx) * 0x9e3779b9u, uint32_t(range))) : 0;
+    [[maybe_unused]] const int last_window = kt_lo < kt_hi ? kt_hi : -1;
     // Copy number `d` (A passes first, then B passes) of the `kt`-th k-tile into the given stage.
+    // WINDOWS: of the `kt`-th window of every row, of which the k-tiles need one more than there are of them.
     auto copy_pass = [&](int d, int kt, uint8_t* la, uint8_t* lb) {
-        const bool live = kt < kt_hi;
-        if constexpr (SPREAD) {
-            kt += first;
-            if (kt >= kt_hi) kt -= range;
+        if constexpr (WINDOWS) {
+            const bool live = kt <= last_window;
+            if (d < StA::PASSES) stage_a.issue_pass(live ? rsrc_a : rsrc_none, la, kt, num_k_tiles, wave, d);
+            else stage_b.issue_pass(live ? rsrc_b : rsrc_none, lb, kt, num_k_tiles, wave, d - StA::PASSES);
+        } else {
+            const bool live = kt < kt_hi;
+            if constexpr (SPREAD) {
+                kt += first;
+                if (kt >= kt_hi) kt -= range;
+            }
+            const bool tail = kt == tail_tile;
+            if (d < StA::PASSES) stage_a.issue_pass_from(live ? rsrc_a : rsrc_none, la, kt * kRowBytes, wave, d, tail ? tail_a : stage_a.voff);
+            else stage_b.issue_pass_from(live ? rsrc_b : rsrc_none, lb, kt * kRowBytes, wave, d - StA::PASSES, tail ? tail_b : stage_b.voff);
         }
-        const bool tail = kt == tail_tile;
-        if (d < StA::PASSES) stage_a.issue_pass_from(live ? rsrc_a : rsrc_none, la, kt * kRowBytes, wave, d, tail ? tail_a : stage_a.voff);
-        else stage_b.issue_pass_from(live ? rsrc_b : rsrc_none, lb, kt * kRowBytes, wave, d - StA::PASSES, tail ? tail_b : stage_b.voff);
     };
 
     // Lane-constant LDS offsets of the four 16-deep K steps inside a 64-deep tile.
     const int g = lane / 32;
-    int koff[4];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) koff[kk] = frag_offset<32>(lane, 2 * kk + g);
+    LaneChunks<WINDOWS> chunks_a, chunks_b;
+    chunks_a.init(A, ld_bytes, lane);
+    chunks_b.init(B, ld_bytes, lane);
 
     typename Atom::Acc acc[TN][TM];
 #pragma unroll
@@ -179,16 +195,20 @@ dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
         for (int d = 0; d < NUM_COPIES; ++d) c += (d * SPREAD_STEPS / NUM_COPIES == kk);
         return c;
     };
-    auto compute_tile = [&](const uint8_t* la, const uint8_t* lb, auto&& step_hook) {
+    // `ahead`: bytes from this k-tile's stage to the next one's.
+    auto compute_tile = [&](const uint8_t* la, const uint8_t* lb, [[maybe_unused]] int ahead, auto&& step_hook) {
         using Frag = typename Atom::Frag;
         const uint8_t* pa = la + wm * Cfg::WTM * kRowBytes;
         const uint8_t* pb = lb + wn * Cfg::WTN * kRowBytes;
         Frag nf[2][TN], mf[2][TM];
+        int off_a[4], off_b[4];
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) off_a[kk] = chunks_a.offset(kk, ahead), off_b[kk] = chunks_b.offset(kk, ahead);
         auto fetch = [&](int kk) {
 #pragma unroll
-            for (int i = 0; i < TN; ++i) nf[kk & 1][i] = *reinterpret_cast<const Frag*>(pb + i * 32 * kRowBytes + koff[kk]);
+            for (int i = 0; i < TN; ++i) nf[kk & 1][i] = *reinterpret_cast<const Frag*>(pb + i * 32 * kRowBytes + off_b[kk]);
 #pragma unroll
-            for (int j = 0; j < TM; ++j) mf[kk & 1][j] = *reinterpret_cast<const Frag*>(pa + j * 32 * kRowBytes + koff[kk]);
+            for (int j = 0; j < TM; ++j) mf[kk & 1][j] = *reinterpret_cast<const Frag*>(pa + j * 32 * kRowBytes + off_a[kk]);
         };
         fetch(0);
         __builtin_amdgcn_sched_barrier(0);
@@ -219,7 +239,9 @@ dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
     // Ring: every wave issues NUM_COPIES copies per k-tile, in the same order, so "k-tile kt has landed" is "at
     // most (STAGES - 2) * NUM_COPIES of my copies are outstanding". The copies of k-tile kt + STAGES - 1 go to
     // the stage that was consumed in iteration kt - 1, which every wave has left once it is past the barrier.
+    // A k-tile of WINDOWS needs the window behind its own as well: one less of them is on its way.
     static_assert((BLOCK_M / 8) % LW == 0 && (BLOCK_N / 8) % LW == 0 && (STAGES - 2) * NUM_COPIES <= 63);
+    constexpr int OUTSTANDING = (STAGES - (WINDOWS ? 3 : 2)) * NUM_COPIES;
     constexpr int STAGE_BYTES = Cfg::STAGE_BYTES;
     __shared__ __attribute__((aligned(1024))) uint8_t ring[STAGES * STAGE_BYTES];
 #pragma unroll
@@ -229,7 +251,7 @@ dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
     int st = 0;
     if (LW > NW && wave >= NW) {            // waves that only copy
         for (int kt = kt_lo; kt < kt_hi; ++kt) {
-            __builtin_amdgcn_s_waitcnt(waitcnt_imm((STAGES - 2) * NUM_COPIES, kNoWaitLgkm));
+            __builtin_amdgcn_s_waitcnt(waitcnt_imm(OUTSTANDING, kNoWaitLgkm));
             asm volatile("" ::: "memory");
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
@@ -242,13 +264,13 @@ dense_gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, El
         return;
     }
     for (int kt = kt_lo; kt < kt_hi; ++kt) {
-        __builtin_amdgcn_s_waitcnt(waitcnt_imm((STAGES - 2) * NUM_COPIES, kNoWaitLgkm));
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm(OUTSTANDING, kNoWaitLgkm));
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         const uint8_t* cur = ring + st * STAGE_BYTES;
         uint8_t* nxt = ring + (st == 0 ? STAGES - 1 : st - 1) * STAGE_BYTES;
-        compute_tile(cur, cur + BLOCK_M * kRowBytes, [&](int kk) {
+        compute_tile(cur, cur + BLOCK_M * kRowBytes, st + 1 == STAGES ? (1 - STAGES) * STAGE_BYTES : STAGE_BYTES, [&](int kk) {
 #pragma unroll
             for (int d = 0; d < NUM_COPIES; ++d)
                 if (d * SPREAD_STEPS / NUM_COPIES == kk) copy_pass(d, kt + STAGES - 1, nxt, nxt + BLOCK_M * kRowBytes);
@@ -932,11 +954,23 @@ inline hipError_t check_dense_args(int m, int n, int k, const void* a, const voi
     return hipSuccess;
 }
 
+// Whether a ring launch copies windows that are whole lines (kLineWindows): rows that do not start on 128-byte lines. Where they start on
+// halves of lines it gains 0 to 10 % and loses as much (512 x 4096 x 4128 on 64 x 128 30.5 -> 27.5 us, 200 x 5000 x 2976 on 128 x 128 22.3 ->
+// 24.9), elsewhere it takes 0.79 to 1.0 of the time (1111 x 5004 x 2056 on 128 x 192 35.5 -> 32.0, on 64 x 192 45.6 -> 37.7, 512 x 4096 x 4104
+// on 64 x 128 31.1 -> 26.7, 2000^2 x 2008 on 128 x 128 24.7 -> 22.3); the 64 x 64 tile, whose k-tiles are too short for where its chunks lie
+// to be worked out beside them, takes up to 1.04 and keeps its copies, as do the 256-row rings.
+inline bool copies_whole_lines(int k, const void* a, const void* b) {
+    return k >= 256 && ((uintptr_t(k) * 2) | reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) % 64 != 0;
+}
+
+
 // Calls `launch` with the copies (COPIES, a std::integral_constant) of a ring tile's launch. A kernel is compiled for each that a plan
 // can ask for: none for 256-row rings, and no streamed weights in six and eight parts, which have 96 MB of weights from
 // K = 24576 on only.
-template <int BLOCK_M, int SPLIT_K, typename Launch>
-inline void with_dense_copies(int tiles_m, int m, int n, int k, Launch&& launch) {
+template <int BLOCK_M, int BLOCK_N, int SPLIT_K, typename Launch>
+inline void with_dense_copies(int tiles_m, int m, int n, int k, const void* a, const void* b, Launch&& launch) {
+    if constexpr (BLOCK_M < 256 && BLOCK_M * BLOCK_N > 64 * 64 && SPLIT_K <= 4)
+        if (copies_whole_lines(k, a, b)) return launch(std::integral_constant<int, kLineWindows>{});
     const uint64_t weight_bytes = uint64_t(n) * k * 2;
     const bool streamed = streams_weights(tiles_m, weight_bytes, k * 2), spread = spreads_starts(tiles_m, m, weight_bytes, k, SPLIT_K);
     if constexpr (BLOCK_M < 256 && SPLIT_K <= 4) {
@@ -998,7 +1032,7 @@ inline hipError_t launch_dense(int m, int n, int k, const void* a, const void* b
                                    dim3(dense_launch_waves(BLOCK_M, BLOCK_N) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
                                    static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, slots);
         };
-        with_dense_copies<BLOCK_M, 1>(sched.tiles_m, m, n, k, launch);
+        with_dense_copies<BLOCK_M, BLOCK_N, 1>(sched.tiles_m, m, n, k, a, b, launch);
     }
     return hipGetLastError();
 }
@@ -1031,7 +1065,7 @@ inline hipError_t launch_dense_split_k(int m, int n, int k, const void* a, const
                                dim3(dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
                                static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, partials, counters);
     };
-    with_dense_copies<BLOCK_M, SPLIT_K>(sched.tiles_m, m, n, k, launch);
+    with_dense_copies<BLOCK_M, BLOCK_N, SPLIT_K>(sched.tiles_m, m, n, k, a, b, launch);
     return hipGetLastError();
 }
 

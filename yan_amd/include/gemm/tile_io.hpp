@@ -97,6 +97,8 @@ struct TileStager {
     uint32_t pass_pitch;  // bytes between the rows of consecutive passes (uniform)
     int      logical;     // logical chunk index this lane fetches
 
+    __device__ __forceinline__ static __amdgpu_buffer_rsrc_t rsrc(const uint8_t* base, uint32_t bytes) { return make_rsrc(base, bytes); }
+
     // The tile starts at matrix row `tile_row0`; rows have a pitch of `ld_bytes`.
     __device__ __forceinline__ void init(int tile_row0, uint32_t ld_bytes, int wave, int lane) {
         const int sub = lane >> 3, slot = lane & 7;
@@ -139,6 +141,59 @@ struct TileStager {
                                                      lane_voff | past_tile, k_byte0 + j * pass_pitch, 0, STREAM ? kNonTemporal : 0);
         }
     }
+};
+
+// Rows that do not start on 128-byte lines (16-bit operands of a K that is no multiple of 64): a k-tile's 128 bytes of such a row lie in
+// two lines, and a tile of them asks for twice as many as it holds (fp16 1111 x 5004 x 2056 34.8 us, 29.0 at K = 2112). LineStager copies a
+// row in windows that are its lines: window w of a row holds the chunks 8 w - s .. 8 w - s + 7, s the 16-byte chunks its start is behind
+// its line's, which differs from row to row and is the same for rows 8 apart. The k-tile t of a row is then in its windows t and t + 1, and
+// LaneChunks says where. Nothing outside of a row is read.
+template <int ROWS, int NUM_WAVES>
+struct LineStager {
+    static_assert(ROWS % (8 * NUM_WAVES) == 0);
+    static constexpr int PASSES = ROWS / 8 / NUM_WAVES, PADDED_ROWS = ROWS;
+    uint32_t voff;          // byte offset of this lane's chunk for pass 0 in window 0, from one line in front of the operand (rsrc)
+    uint32_t pass_pitch;
+    uint32_t outside;       // bits 0, 1, 2: the chunk is no part of the row in the first window, the last but one, the last
+
+    // The descriptor starts a line early, so that no offset is below zero; what is in front of the operand is not read (`outside`).
+    __device__ __forceinline__ static __amdgpu_buffer_rsrc_t rsrc(const uint8_t* base, uint32_t bytes) { return make_rsrc(base - kRowBytes, bytes + kRowBytes); }
+
+    // ceil(k / 64) k-tiles, at least two, and one more window
+    __device__ __forceinline__ void init(const void* base, int tile_row0, int k, int wave, int lane) {
+        const int sub = lane >> 3, slot = lane & 7;
+        const uint32_t ld_bytes = uint32_t(k) * 2, row = uint32_t(tile_row0 + wave * 8 + sub);
+        const int s = int((reinterpret_cast<uintptr_t>(base) / kChunk + row * (ld_bytes / kChunk)) % 8);
+        // a slot holds chunks of one place in the k-tile, the one it holds in TileStager, so that the fragment reads keep their banks
+        const int chunk = ((slot ^ sub ^ (wave & 1)) + s) & 7;
+        const int row_chunks = k / 8, left = row_chunks + s - 8 * (ceil_div(row_chunks, 8) - 1);     // chunks of the row from the last window but one on
+        voff = row * ld_bytes + uint32_t(kRowBytes + (chunk - s) * kChunk);
+        pass_pitch = uint32_t(NUM_WAVES * 8) * ld_bytes;
+        outside = (chunk < s ? 1u : 0u) | (chunk >= left ? 2u : 0u) | (chunk + 8 >= left ? 4u : 0u);
+    }
+    __device__ __forceinline__ void issue_pass(__amdgpu_buffer_rsrc_t rsrc, uint8_t* lds_tile, int window, int k_tiles, int wave, int j) const {
+        // the bit of this window, if it is one of the three, becomes kOutOfRange
+        const uint32_t shift = window == 0 ? 31u : window == k_tiles - 1 ? 30u : window == k_tiles ? 29u : 0u;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, YAN_LDS_PTR(lds_tile + (j * NUM_WAVES + wave) * 8 * kRowBytes), kChunk,
+                                                 voff | ((outside << shift) & kOutOfRange), window * kRowBytes + j * pass_pitch, 0, 0);
+    }
+};
+
+// Where a lane's chunks of a k-tile lie that 32-row atoms read in four steps (2 kk + lane / 32): bytes from its atom's first row, `ahead`
+// bytes further if they are in the next window's stage. Atoms start at multiples of 8 rows.
+template <bool WINDOWS>
+struct LaneChunks {
+    int  at[4];
+    bool next[4];
+    __device__ __forceinline__ void init(const void* base, uint32_t ld_bytes, int lane) {
+        const int i = lane % 32, s = WINDOWS ? int((reinterpret_cast<uintptr_t>(base) / kChunk + uint32_t(i) * (ld_bytes / kChunk)) % 8) : 0;
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+            at[kk] = i * kRowBytes + (((2 * kk + lane / 32) ^ swizzle_of_row(i)) * kChunk);
+            next[kk] = 2 * kk + lane / 32 + s >= 8;
+        }
+    }
+    __device__ __forceinline__ int offset(int kk, int ahead) const { return WINDOWS && next[kk] ? at[kk] + ahead : at[kk]; }
 };
 
 // Where the SPLIT_K parts of a split-K tile meet (fp8_gemm.hpp, bf16_gemm.hpp). Wave w of every part leaves its VECS
