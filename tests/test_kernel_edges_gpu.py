@@ -616,3 +616,83 @@ def test_dense_tiles_that_start_at_different_places_along_k(tile, split_k, m, n,
     a64, b64 = a.double(), b.double()
     bound = (a64 @ b64.t()).abs() * 2.0 ** -8 + (a64.abs() @ b64.abs().t()) * (k * 2.0 ** -24)
     assert ((c.double() - a64 @ b64.t()).abs() <= bound).all()
+
+
+def test_repeated_calls_are_made_natively_and_follow_what_changes(monkeypatch):
+    """A call an entry has served before is made by the native host module; other sizes, strides and types, the compute-unit cap, the
+    environment switches, another stream, a capture and wrong arguments still get what they ask for."""
+    from yan_amd.jit_kernels import host_calls
+    assert host_calls._host_calls is not None, 'yan_amd/csrc/build.py builds it'
+    host_calls._host_calls.forget()
+    m, n, k = 40, 2112, 7168                    # K is split: the call takes the stream's workspace
+    _announce('repeated calls', m, n, k)
+    cases = [testing.make_fp8_case(m, n, k, seed=s, device='cuda', col_major_scales=True) for s in (1, 2, 3)]
+    refs = [testing.dequant_lhs(*lhs) @ testing.dequant_rhs(*rhs).t() for lhs, rhs, _ in cases]
+
+    def right(out, ref):
+        return float(yan.calc_diff(out.float(), ref)) < 1e-5
+
+    def native(lhs, rhs, out):
+        out.fill_(float('nan'))
+        return host_calls.repeat_call(host_calls.FP8, *lhs, *rhs, out)
+
+    lhs, rhs, out = cases[0]
+    assert not native(lhs, rhs, out)
+    yan.gemm_fp8_fp8_bf16_nt(lhs, rhs, out)
+    for (lhs, rhs, out), ref in zip(cases, refs):       # other addresses, the same call
+        assert native(lhs, rhs, out) and right(out, ref)
+    lhs, rhs, out = cases[1]
+    row_major = lhs[1].contiguous()
+    assert row_major.stride() != lhs[1].stride() and not native((lhs[0], row_major), rhs, out)
+    yan.gemm_fp8_fp8_bf16_nt((lhs[0], row_major), rhs, out)
+    assert right(out, refs[1])
+    assert not native((lhs[0][:39], lhs[1][:39]), rhs, out[:39]) and not native((lhs[0].cpu(), lhs[1]), rhs, out)
+    with pytest.raises(AssertionError):
+        yan.gemm_fp8_fp8_bf16_nt(lhs, rhs, out[:39])
+    with pytest.raises(AssertionError):
+        yan.gemm_fp8_fp8_bf16_nt(lhs, rhs, out.half())
+    # what plans depend on
+    full = yan.get_num_sms()
+    try:
+        yan.set_num_sms(64)
+        assert not native(lhs, rhs, out)
+        yan.gemm_fp8_fp8_bf16_nt(lhs, rhs, out)
+        assert right(out, refs[1])
+    finally:
+        yan.set_num_sms(full)
+    for name, value in (('YAN_SPLIT_K', '0'), ('YAN_TUNE_TILES', '1')):
+        monkeypatch.setenv(name, value)
+        assert not native(lhs, rhs, out)
+        monkeypatch.delenv(name)
+    assert native(lhs, rhs, out) and right(out, refs[1])
+    # a stream of its own has a workspace of its own, and the first call on it goes round by Python; so does a capture
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        assert not native(lhs, rhs, out)
+        yan.gemm_fp8_fp8_bf16_nt(lhs, rhs, out)
+        assert native(lhs, rhs, out)
+    torch.cuda.synchronize()
+    assert right(out, refs[1])
+    yan.gemm_fp8_fp8_bf16_nt(lhs, rhs, out)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        assert not host_calls.repeat_call(host_calls.FP8, *lhs, *rhs, out)
+        yan.gemm_fp8_fp8_bf16_nt(lhs, rhs, out)
+    for i in range(3):
+        out.fill_(float('nan'))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert right(out, refs[1])
+        yan.gemm_fp8_fp8_bf16_nt(lhs, rhs, cases[2][2])
+    # one tensor in two places, then two; floats of the call
+    x, y, c = testing.make_float_case(128, 128, 64, seed=4, device='cuda')
+    for a, b in ((x, x), (x, y), (y, x)):
+        for alpha, beta in ((1.0, 0.0), (-0.5, 2.0)):
+            start = torch.ones_like(c)
+            c.copy_(start)
+            yan.gemm_float_nt(a, b, c, alpha, beta)
+            assert torch.allclose(c.double(), alpha * (a.double() @ b.double().t()) + beta * start.double(), atol=1e-3)
+            c.copy_(start)
+            assert host_calls.repeat_call(host_calls.FLOAT, alpha, a, b, beta, c)
+            assert torch.allclose(c.double(), alpha * (a.double() @ b.double().t()) + beta * start.double(), atol=1e-3)

@@ -1,6 +1,7 @@
 #!/usr/bin/env python3
 """Builds yan_amd/csrc/libyan_gemm.so, the ahead-of-time C-ABI library (declared in include/yan_gemm.h), with
-hipcc for gfx950. Cross-compiles: needs no GPU. `--force` rebuilds even when the library is newer than its sources."""
+hipcc for gfx950, and yan_amd/_host_calls.so, the host side of repeated calls, with the host compiler against torch's headers.
+Needs no GPU. `--force` rebuilds even when the libraries are newer than their sources."""
 import glob
 import os
 import subprocess
@@ -35,5 +36,27 @@ def build(force: bool = False) -> str:
     return OUT
 
 
+HOST_SRC = os.path.join(HERE, 'host_calls.cpp')
+HOST_OUT = os.path.join(ROOT, 'yan_amd', '_host_calls.so')
+
+
+def build_host_calls(force: bool = False) -> str:
+    if not force and os.path.exists(HOST_OUT) and os.path.getmtime(HOST_OUT) >= os.path.getmtime(HOST_SRC):
+        return HOST_OUT
+    import sysconfig
+    import torch
+    from torch.utils import cpp_extension
+    lib = os.path.join(os.path.dirname(torch.__file__), 'lib')
+    cmd = [os.getenv('CXX') or 'g++', HOST_SRC, '-o', HOST_OUT + '.tmp', '-std=c++17', '-O2', '-shared', '-fPIC',
+           f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}', *(f'-isystem{p}' for p in cpp_extension.include_paths()),
+           f'-I{sysconfig.get_paths()["include"]}', f'-L{lib}', '-ltorch_python', '-ltorch_cpu', '-lc10']
+    done = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, universal_newlines=True)
+    if done.returncode != 0:
+        raise RuntimeError(f'{cmd[0]} failed:\n{done.stdout[-4000:]}')
+    os.replace(HOST_OUT + '.tmp', HOST_OUT)
+    return HOST_OUT
+
+
 if __name__ == '__main__':
+    print(build_host_calls(force='--force' in sys.argv))
     print(build(force='--force' in sys.argv))

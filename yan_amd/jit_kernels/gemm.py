@@ -18,6 +18,7 @@ import torch
 from .fp8_cast import per_token_cast_to_fp8
 from .heuristics import (get_best_fp8_config, get_fp8_num_stages, get_fp8_tile_space, get_skinny_fp8_config,
                          get_split_k_fp8_config, tuning_enabled)
+from .host_calls import CAST_FP8, FP8, remember_call, repeat_call
 from .split_k import SPLIT_K_COUNTER_BYTES, SPLIT_K_WORKSPACE_BYTES, split_k_enabled, split_k_launch_failed, split_k_workspace
 from .tuner import FrozenKeys, jit_tuner
 from .utils import current_raw_stream, get_num_sms, ceil_div, get_col_major_tensor, scales_for_kernel, SCALE_RELAYOUT_MIN_FLOP
@@ -166,6 +167,8 @@ def gemm_fp8_fp8_bf16_nt(lhs: Tuple[torch.Tensor, torch.Tensor],
     """
     lhs, lhs_scales = lhs
     rhs, rhs_scales = rhs
+    if repeat_call(FP8, lhs, lhs_scales, rhs, rhs_scales, out):
+        return
     m, k = lhs.shape
     n, k_ = rhs.shape
     m_, n_ = out.shape
@@ -192,7 +195,7 @@ def gemm_fp8_fp8_bf16_nt(lhs: Tuple[torch.Tensor, torch.Tensor],
     name, keys, defs, smem_size, code_template = fp8_kernel_plan(m, n, k, num_sms, token_contiguous)
     stream = current_raw_stream()
     args = (lhs, lhs_scales, rhs, rhs_scales, out, m, stream, num_sms, smem_size)
-    space, workspace_token = (), None
+    space, workspace, workspace_token = (), None, None
     if tuning_enabled():
         tuning = fp8_tuning_plan(m, n, k, num_sms, token_contiguous)
         if tuning is not None:
@@ -212,6 +215,9 @@ def gemm_fp8_fp8_bf16_nt(lhs: Tuple[torch.Tensor, torch.Tensor],
     if rc != 0 and workspace_token is not None:
         split_k_launch_failed(workspace_token)
     assert rc == 0, f'{name} failed with HIP error {rc}'
+    # (what `scales_for_kernel` does with a large problem's other layouts is decided by the addresses of each call)
+    if flop < SCALE_RELAYOUT_MIN_FLOP or token_contiguous:
+        remember_call((FP8, lhs, lhs_scales, rhs, rhs_scales, out), runtime, args, workspace)
 
 
 # Scratch of the chained entry: behind the 16 MB of the split-K workspace, room for the codes and scales of up to
@@ -254,6 +260,8 @@ def gemm_bf16_fp8_bf16_nt(x: torch.Tensor, rhs: Tuple[torch.Tensor, torch.Tensor
     kernel against 3 + 9.7 us in two; same bits). Problems whose codes do not fit the scratch area (or with
     `YAN_SPLIT_K=0`, which means no memory kept by the entries) run the two entries one after the other."""
     rhs_q, rhs_scales = rhs
+    if repeat_call(CAST_FP8, x, rhs_q, rhs_scales, out):
+        return
     m, k = x.shape
     n, k_ = rhs_q.shape
     assert x.dtype == torch.bfloat16 and out.dtype == torch.bfloat16 and rhs_q.dtype == torch.float8_e4m3fn and rhs_scales.dtype == torch.float32
@@ -279,3 +287,4 @@ def gemm_bf16_fp8_bf16_nt(x: torch.Tensor, rhs: Tuple[torch.Tensor, torch.Tensor
     if rc != 0:
         split_k_launch_failed(workspace_token)
     assert rc == 0, f'{name} failed with HIP error {rc}'
+    remember_call((CAST_FP8, x, rhs_q, rhs_scales, out), runtime, args, workspace)

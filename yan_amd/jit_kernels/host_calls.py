@@ -1,0 +1,61 @@
+"""Repeated calls of the entry points, made in native code (`csrc/host_calls.cpp`).
+
+The reference's entries do their checks, their plan lookup and one ctypes call in Python on every call (`yan/jit_kernels/cute_gemm.py:39-64`,
+`yan/jit/runtime.py:34-68`). So does an entry here the first time it sees sizes, strides, types and devices; then it hands its launch over
+(`remember_call`), and a call that agrees in all of them is made natively (`repeat_call`), from the addresses of that call. A call that does
+not, or a process without the built module, takes the Python way, whose checks and errors are unchanged.
+
+Host time of a call, Python -> native: FP8 1 x 2112 x 7168 8.5 -> 3.5 us, of which 2.5 are the launch; 16-bit 6.4 -> 3.1, from bf16 activations
+14.1 -> 5.9. 256 x 832 x 455 in fp32 takes 4.7 us a call instead of 7.3, four 2 x 1984 x 4608 from bf16 activations 29 instead of 41.
+"""
+import ctypes
+import os
+
+import torch
+
+from ..jit.runtime import Runtime
+from . import split_k, utils
+from .heuristics import tuning_enabled
+
+try:
+    from .. import _host_calls
+except ImportError:
+    _host_calls = None
+
+# which entry a remembered call belongs to
+FP8, CAST_FP8, BF16, FP16, FLOAT, CONTIGUOUS, MASKED, PER_TOKEN, PER_BLOCK = range(1, 10)
+_TENSOR, _CONSTANT, _STREAM, _WORKSPACE = range(4)
+
+
+def _never(*_) -> bool:
+    return False
+
+
+repeat_call = _never
+if _host_calls is not None and utils._environ is not None:
+    try:
+        _host_calls.setup(utils.__dict__, split_k.__dict__, os.__dict__, utils._environ, utils._environ_bytes, torch._C._cuda_getDevice,
+                          torch._C._cuda_getCurrentRawStream, split_k._is_capturing)
+        repeat_call = _host_calls.call
+    except (AttributeError, TypeError):          # a torch without the raw accessors
+        pass
+
+
+def remember_call(call: tuple, runtime: Runtime, args: tuple, workspace=None) -> None:
+    """`call`: the entry and its arguments as `repeat_call` gets them, tensors and floats in the order of `args`, which `runtime` has just
+    been launched with. `workspace`: the split-K workspace among them, looked up anew by every call."""
+    if repeat_call is _never or type(runtime) is not Runtime or runtime._launch is None or not split_k.split_k_enabled() or tuning_enabled():
+        return
+    spec, tensors = [], 0
+    for arg, (_, kind) in zip(args, runtime.args):
+        if workspace is not None and arg is workspace:
+            spec.append((_WORKSPACE, 0))
+        elif isinstance(kind, torch.dtype):
+            spec.append((_TENSOR, tensors))
+            tensors += 1
+        elif kind is torch.cuda.Stream:
+            spec.append((_STREAM, 0))
+        elif kind is not float:
+            spec.append((_CONSTANT, int(arg)))
+    if tensors == sum(isinstance(a, torch.Tensor) for a in call):
+        _host_calls.remember(call, ctypes.cast(runtime._launch, ctypes.c_void_p).value, tuple(spec))

@@ -13,6 +13,7 @@ from typing import Tuple
 import torch
 
 from .gemm import includes
+from .host_calls import CONTIGUOUS, MASKED, remember_call, repeat_call
 from .heuristics import get_best_grouped_fp8_config, get_contiguous_rows_on_device, get_fp8_num_stages
 from .tuner import FrozenKeys, jit_tuner
 from .utils import ceil_div, current_raw_stream, get_m_alignment_for_contiguous_layout, get_num_sms, scales_for_kernel, SCALE_RELAYOUT_MIN_FLOP
@@ -76,7 +77,7 @@ def grouped_kernel_plan(gemm_type: str, num_groups: int, m: int, n: int, k: int,
     return name, keys, arg_defs, keys['NUM_STAGES'] * (block_m + block_n) * 128
 
 
-def _launch(gemm_type, num_groups, plan_m, m, n, k, lhs, lhs_scales, rhs, rhs_scales, out, layout, strides):
+def _launch(gemm_type, num_groups, plan_m, m, n, k, lhs, lhs_scales, rhs, rhs_scales, out, layout, strides, flop, call):
     # `strides`: the three strides of the activation scales, then expected_m (masked layout; 0 otherwise)
     num_sms = get_num_sms()
     name, keys, defs, smem_size = grouped_kernel_plan(gemm_type, num_groups, plan_m, n, k, num_sms)
@@ -85,6 +86,9 @@ def _launch(gemm_type, num_groups, plan_m, m, n, k, lhs, lhs_scales, rhs, rhs_sc
                                          template=rows_on_device_template if 'ROWS' in keys else template, args=args)
     rc = runtime(*args)
     assert rc == 0, f'{name} failed with HIP error {rc}'
+    # (what `scales_for_kernel` does with a large problem's other layouts is decided by the addresses of each call)
+    if flop < SCALE_RELAYOUT_MIN_FLOP or (lhs_scales.stride(-2) == 1 and lhs_scales.stride(-1) == lhs_scales.size(-2)):
+        remember_call((call[0], lhs, lhs_scales, rhs, rhs_scales, out, layout, *call[1:]), runtime, args)
 
 
 def m_grouped_gemm_fp8_fp8_bf16_nt_contiguous(lhs: Tuple[torch.Tensor, torch.Tensor],
@@ -102,6 +106,8 @@ def m_grouped_gemm_fp8_fp8_bf16_nt_contiguous(lhs: Tuple[torch.Tensor, torch.Ten
     """
     lhs, lhs_scales = lhs
     rhs, rhs_scales = rhs
+    if repeat_call(CONTIGUOUS, lhs, lhs_scales, rhs, rhs_scales, out, m_indices):
+        return
     m, k = lhs.shape
     num_groups, n, k_ = rhs.shape
     m_, n_ = out.shape
@@ -124,7 +130,7 @@ def m_grouped_gemm_fp8_fp8_bf16_nt_contiguous(lhs: Tuple[torch.Tensor, torch.Ten
     if flop >= SCALE_RELAYOUT_MIN_FLOP:
         lhs_scales = scales_for_kernel(lhs_scales, flop, grouped_kernel_plan('GroupedContiguous', num_groups, m, n, k, get_num_sms())[1])
     _launch('GroupedContiguous', num_groups, m, m, n, k, lhs, lhs_scales, rhs, rhs_scales, out, m_indices,
-            (lhs_scales.stride(0), lhs_scales.stride(1), 0, 0))
+            (lhs_scales.stride(0), lhs_scales.stride(1), 0, 0), flop, (CONTIGUOUS, ))
 
 
 def m_grouped_gemm_fp8_fp8_bf16_nt_masked(lhs: Tuple[torch.Tensor, torch.Tensor],
@@ -142,6 +148,8 @@ def m_grouped_gemm_fp8_fp8_bf16_nt_masked(lhs: Tuple[torch.Tensor, torch.Tensor]
     """
     lhs, lhs_scales = lhs
     rhs, rhs_scales = rhs
+    if repeat_call(MASKED, lhs, lhs_scales, rhs, rhs_scales, out, masked_m, expected_m):
+        return
     num_groups, m, k = lhs.shape
     num_groups_, n, k_ = rhs.shape
     num_groups__, m_, n_ = out.shape
@@ -164,4 +172,4 @@ def m_grouped_gemm_fp8_fp8_bf16_nt_masked(lhs: Tuple[torch.Tensor, torch.Tensor]
     if flop >= SCALE_RELAYOUT_MIN_FLOP:
         lhs_scales = scales_for_kernel(lhs_scales, flop, grouped_kernel_plan('GroupedMasked', num_groups, min(expected_m, m), n, k, get_num_sms())[1])
     _launch('GroupedMasked', num_groups, min(expected_m, m), m, n, k, lhs, lhs_scales, rhs, rhs_scales, out, masked_m,
-            (lhs_scales.stride(1), lhs_scales.stride(2), lhs_scales.stride(0), min(expected_m, m)))
+            (lhs_scales.stride(1), lhs_scales.stride(2), lhs_scales.stride(0), min(expected_m, m)), flop, (MASKED, expected_m))

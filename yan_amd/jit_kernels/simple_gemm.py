@@ -14,6 +14,7 @@ import functools
 import torch
 
 from .heuristics import get_best_float_config, get_float_bf16x3_config, get_split_k_float_config
+from .host_calls import FLOAT, remember_call, repeat_call
 from .split_k import SPLIT_K_WORKSPACE_BYTES, split_k_enabled, split_k_launch_failed, split_k_workspace
 from .tuner import FrozenKeys, jit_tuner
 from .utils import current_raw_stream, get_num_sms
@@ -116,6 +117,8 @@ def _leading_dim(x: torch.Tensor) -> int:
 
 def gemm_float_nt(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor,
                   alpha: float = 1.0, beta: float = 0.0) -> None:
+    if repeat_call(FLOAT, alpha, a, b, beta, c):
+        return
     m, k = a.shape
     n, k_ = b.shape
     m_, n_ = c.shape
@@ -133,7 +136,7 @@ def gemm_float_nt(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor,
     stream = current_raw_stream()
     args = (m, n, k, float(alpha), a, ldA, b, ldB, float(beta), c, ldC, stream)
     num_cus = get_num_sms()
-    kernel_includes, code_template, workspace_token = includes, template, None
+    kernel_includes, code_template, workspace, workspace_token = includes, template, None, None
     plan = float_bf16x3_plan(m, n, k, num_cus, split_k_enabled())
     if plan is not None:
         name, keys, defs = plan
@@ -156,6 +159,7 @@ def gemm_float_nt(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor,
     if rc != 0 and workspace_token is not None:
         split_k_launch_failed(workspace_token)
     assert rc == 0, f'{name} failed with HIP error {rc}'
+    remember_call((FLOAT, float(alpha), a, b, float(beta), c), runtime, args, workspace)
 
 
 def accuracy_test():
