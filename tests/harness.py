@@ -225,6 +225,12 @@ DENSE_LINE_WINDOW_TILES = [((128, 256), 3), ((128, 192), 4), ((128, 128), 5), ((
 DENSE_LINE_WINDOW_SHAPES = [(131, 260, 264, 0, 0), (70, 132, 312, 8, 40), (257, 388, 328, 56, 0), (64, 68, 424, 24, 24), (130, 516, 1016, 48, 8)]
 
 
+# The weight-streaming kernel through the entry points: every number of activation atoms on 8, 16 and 32 weight rows per workgroup,
+# m and n off the tiles, fewer K blocks than waves, one more than a whole round of the waves and of their slots.
+WEIGHT_STREAM_SHAPES = [(1, 196, 128), (8, 2044, 1152), (9, 2052, 4224), (16, 4100, 640), (17, 100, 4224), (32, 4096, 512), (33, 2052, 1152),
+                        (48, 4100, 512), (64, 196, 1024), (64, 4100, 1152)]
+
+
 # fp32 on the bf16 matrix cores: (tile, parts, (m, n, k)) built through explicit keys. Ragged tiles on both sides, K around the 16 rows of an
 # MFMA and the k-tiles of 16, 32 and 64 rows, fewer k-tiles than stages, parts of unequal length and parts without any
 FLOAT_BF16X3_CASES = [((256, 256), 1, (300, 260, 1)), ((256, 256), 1, (256, 516, 95)), ((256, 256), 3, (260, 256, 145)),
@@ -641,6 +647,13 @@ def jit_kernels_in_use(num_cus: int = 256):
         for dtype in (torch.bfloat16, torch.half):
             name, keys, arg_defs, includes, code_template = dense_tile_plan(tile, dtype, 0)
             add(name, arg_defs, includes, code_template, keys)
+    for m, n, k in WEIGHT_STREAM_SHAPES:
+        for token_contiguous in (True, False):
+            name, keys, arg_defs, _, code_template = gemm.fp8_kernel_plan(m, n, k, num_cus, token_contiguous)
+            add(name, arg_defs, gemm.includes, code_template, keys)
+        for dtype in (torch.bfloat16, torch.half):
+            name, keys, arg_defs = bf16_gemm.dense_kernel_plan(m, n, k, dtype, num_cus)
+            add(name, arg_defs, bf16_gemm.includes, bf16_gemm.template, keys)
     for tile, parts in sorted({(tile, parts) for tile, parts, _ in FLOAT_BF16X3_CASES}):
         name, keys, arg_defs = float_bf16x3_explicit_plan(tile, parts)
         add(name, arg_defs, simple_gemm.bf16x3_includes, simple_gemm.bf16x3_template, keys)

@@ -80,6 +80,24 @@ def test_version_and_tile_selection_match_python(lib):
     assert lib.yan_gemm_select_tile(0, 1, 1, 1, 0, ctypes.byref(bm), ctypes.byref(bn)) == 1
 
 
+def test_weight_stream_choice_matches_python(lib):
+    """Where the weight-streaming kernel goes before tiles and split-K plans: the same on both sides; up to 64 rows, one round of workgroups
+    of at most 32 weight rows, whole 128-byte K blocks, offsets of 32 bits."""
+    taken = 0
+    for m in (1, 8, 16, 17, 32, 40, 41, 48, 49, 64, 65):
+        for n in (12, 16, 100, 102, 1472, 2044, 2052, 4096, 4100, 8192, 8196):
+            for k in (64, 128, 576, 1536, 4608, 7168, 7176, 16384, 1 << 18):
+                for cus in (256, 80):
+                    dense, fp8 = (f(m, n, k, cus) for f in (heuristics.get_weight_stream_dense_config, heuristics.get_weight_stream_fp8_config))
+                    assert capi.select_tile(0, m, n, k, cus) == heuristics.get_dense_tile(m, n, k, cus), (m, n, k, cus)
+                    assert capi.select_tile(1, m, n, k, cus) == heuristics.get_fp8_tile(m, n, k, cus), (m, n, k, cus)
+                    for atoms, row_bytes in ((dense, 2 * k), (fp8, k)):
+                        taken += atoms > 0
+                        assert atoms in (0, yan.ceil_div(m, 16))
+                        assert not atoms or (m <= 64 and 16 <= n <= 32 * cus and n % 4 == 0 and row_bytes % 128 == 0 and (n + 32) * row_bytes < 1 << 31)
+    assert taken > 500
+
+
 def test_compute_entry_points_validate_before_touching_a_device(lib):
     null = ctypes.c_void_p(0)
     assert lib.yan_gemm_bf16_tn(0, 64, 64, null, null, null, null) == 0          # empty problem: no-op

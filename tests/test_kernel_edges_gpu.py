@@ -332,6 +332,38 @@ def test_rows_off_cache_lines_give_the_bits_of_the_smallest_tile(tile, stages, d
         assert bool(((got[:m].double() - ref).abs() <= bound).all())
 
 
+@pytest.mark.parametrize('m,n,k', testing.WEIGHT_STREAM_SHAPES)
+def test_weight_streaming_kernel_at_the_edges_of_its_tiles(m, n, k):
+    """FP8 with both layouts of the activation scales, bf16 and fp16, through the entry points, against the product in float64; the
+    rows behind the output stay untouched."""
+    from yan_amd.jit_kernels import heuristics
+    _announce('weight streaming', m, n, k)
+    cus, atoms = yan.get_num_sms(), yan.ceil_div(m, 16)
+    assert heuristics.get_weight_stream_fp8_config(m, n, k, cus) == heuristics.get_weight_stream_dense_config(m, n, k, cus) == atoms
+    g = torch.Generator().manual_seed(31)
+    x, w = (torch.randn(rows, k, generator=g) for rows in (m, n))
+
+    def check(run, a, b, dtype, sum_error):
+        out = torch.full((m + 2, n), 7.0, dtype=dtype, device='cuda')
+        run(out[:m])
+        assert bool((out[m:] == 7.0).all())
+        ref = a @ b.t()
+        # one rounding to the type, and an error per addition relative to the sum of magnitudes
+        bound = ref.abs() * 2.0 ** (-8 if dtype == torch.bfloat16 else -11) + (k + 8) * sum_error * (a.abs() @ b.abs().t())
+        assert bool(((out[:m].double().cpu() - ref).abs() <= bound).all())
+
+    for dtype, entry in ((torch.bfloat16, yan.gemm_bf16_tn), (torch.half, yan.gemm_fp16_tn)):
+        a, b = x.to(dtype), w.to(dtype)
+        check(lambda out: entry(a.cuda(), b.cuda(), out), a.double(), b.double(), dtype, 2.0 ** -24)
+    wq, ws = yan.per_block_cast_to_fp8(w.bfloat16().cuda())
+    b = wq.cpu().double() * ws.cpu().double().repeat_interleave(128, 0)[:n].repeat_interleave(128, 1)
+    for col_major in (True, False):
+        xq, xs = yan.per_token_cast_to_fp8(x.bfloat16().cuda(), col_major_scales=col_major)
+        # (the FP8 MFMA does not round its 128 products to nearest one by one: twice the error of a rounded sum)
+        check(lambda out: yan.gemm_fp8_fp8_bf16_nt((xq, xs), (wq, ws), out), xq.cpu().double() * xs.cpu().double().repeat_interleave(128, 1), b,
+              torch.bfloat16, 2.0 ** -23)
+
+
 def _run_float_bf16x3(tile, parts, a, b, c, alpha=1.0, beta=0.0):
     from yan_amd.jit_kernels import simple_gemm, split_k
     name, keys, arg_defs = testing.float_bf16x3_explicit_plan(tile, parts)

@@ -102,6 +102,33 @@ int skinny_atoms(int m, int n, int num_cus) {
     return (m > 0 && m <= 16 && n >= 16 && n <= 16 * num_cus) ? 1 : 0;
 }
 
+// Bytes a workgroup of the weight-streaming kernel pulls, or 0 (_weight_stream_pull in heuristics.py).
+long long weight_stream_pull(int m, int n, long long k_bytes, int num_cus) {
+    if (m <= 0 || m > 64 || n < 16 || n % 4 != 0 || k_bytes <= 0 || k_bytes % 128 != 0 || (n + 32ll) * k_bytes >= 1ll << 31) return 0;
+    for (const int rows : {8, 16, 32})
+        if ((n + rows - 1) / rows <= num_cus) return (rows + m) * k_bytes;
+    return 0;
+}
+
+// Activation atoms when the weight-streaming kernel goes before split-K plans and tiles, else 0 (get_weight_stream_fp8_config and
+// get_weight_stream_dense_config in heuristics.py).
+int weight_stream_fp8_atoms(int m, int n, int k, int num_cus) {
+    const long long pull = weight_stream_pull(m, n, k, num_cus);
+    const bool takes = pull <= 130000 || (m <= 48 && pull <= 300000) || (m <= 40 && (pull <= 400000 || n >= 16 * num_cus));
+    return pull && takes ? (m + 15) / 16 : 0;
+}
+int weight_stream_dense_atoms(int m, int n, int k, int num_cus) {
+    const long long pull = weight_stream_pull(m, n, 2ll * k, num_cus);
+    return pull && (m <= 16 || pull <= (n >= 16 * num_cus ? 580000 : 450000)) ? (m + 15) / 16 : 0;
+}
+
+// Whether a workspace holds what a split-K plan needs (launch_dense_split_k, Gemm::run_split_k): asked for also where the
+// weight-streaming kernel runs in the plan's place, so that what a call needs does not depend on it.
+bool split_k_fits(int m, int n, int bm, int bn, int split_k, size_t workspace_bytes) {
+    const size_t tiles = size_t((m + bm - 1) / bm) * ((n + bn - 1) / bn);
+    return workspace_bytes >= yan::kSplitKCounterBytes + (tiles + 7) / 8 * 8 * split_k * bm * bn * 4;
+}
+
 // Split-K plan of the plain FP8 GEMM (get_split_k_fp8_config in heuristics.py): false when K is not split.
 struct SplitKTile { int bm, bn; double us_per_k_tile, unsplit_us_per_k_tile; };
 constexpr SplitKTile kSplitKTiles[] = {{32, 32, 0.133, 0.117}, {64, 32, 0.192, 0.169}, {64, 64, 0.296, 0.275}, {64, 128, 0.395, 0.375},
@@ -196,9 +223,10 @@ int dense(int m, int n, int k, const void* a, const void* b, void* c, void* stre
     if (m < 0 || n < 0) return int(hipErrorInvalidValue);
     hipStream_t s = static_cast<hipStream_t>(stream);
     int bm = 0, bn = 0, split_k = 1;
-    // a split-K plan goes before the weight-streaming kernels (pick_dense_split_k makes none where the one-atom kernel is the
-    // faster: below 8 rows, and up to 16 rows on K beyond 8192)
-    if (workspace && pick_dense_split_k(m, n, k, device_cus(), &bm, &bn, &split_k)) {
+    const int stream_atoms = weight_stream_dense_atoms(m, n, k, device_cus());
+    const bool split = workspace && pick_dense_split_k(m, n, k, device_cus(), &bm, &bn, &split_k);
+    if (stream_atoms && split && !split_k_fits(m, n, bm, bn, split_k, workspace_bytes)) return int(hipErrorInvalidValue);
+    if (split && !stream_atoms) {
 #define YAN_DENSE_SPLIT_K_CASE(BM, BN, S) \
     if (bm == BM && bn == BN && split_k == S) return int(yan::launch_dense_split_k<Atom, Elem, BM, BN, S>(m, n, k, a, b, c, s, workspace, workspace_bytes));
 #define YAN_DENSE_SPLIT_K_TILE(BM, BN) YAN_DENSE_SPLIT_K_CASE(BM, BN, 2) YAN_DENSE_SPLIT_K_CASE(BM, BN, 3) YAN_DENSE_SPLIT_K_CASE(BM, BN, 4)
@@ -208,9 +236,10 @@ int dense(int m, int n, int k, const void* a, const void* b, void* c, void* stre
 #undef YAN_DENSE_SPLIT_K_CASE
         return int(hipErrorInvalidValue);
     }
-    if (const int atoms = dense_skinny_atoms(m, n, k, device_cus())) {
-        if (atoms == 1) return int(yan::launch_dense_skinny<SkinnyAtom, Elem, 1, 8>(m, n, k, a, b, c, s));
-        return int(yan::launch_dense_skinny<SkinnyAtom, Elem, 2, 8>(m, n, k, a, b, c, s));
+    if (const int atoms = stream_atoms ? stream_atoms : dense_skinny_atoms(m, n, k, device_cus())) {
+#define YAN_STREAM_CASE(TM) if (atoms == TM) return int(yan::launch_dense_skinny<SkinnyAtom, Elem, TM>(m, n, k, a, b, c, s));
+        YAN_STREAM_CASE(1) YAN_STREAM_CASE(2) YAN_STREAM_CASE(3) YAN_STREAM_CASE(4)
+#undef YAN_STREAM_CASE
     }
     pick(kDenseTiles, m, n, device_cus(), &bm, &bn);
 #define YAN_DENSE_CASE(BM, BN) if (bm == BM && bn == BN) return int(yan::launch_dense<Atom, Elem, BM, BN>(m, n, k, a, b, c, s));
@@ -252,8 +281,10 @@ int fp8_plain(const void* lhs, const float* lhs_scales, long long lhs_scales_str
     hipStream_t s = static_cast<hipStream_t>(stream);
     __hip_bfloat16* o = static_cast<__hip_bfloat16*>(out);
     int bm = 0, bn = 0, split_k = 1;
-    // a split-K plan goes before the weight-streaming kernel
-    if (workspace && pick_split_k(m, n, k, cus, &bm, &bn, &split_k)) {
+    const int stream_atoms = weight_stream_fp8_atoms(m, n, k, cus);
+    const bool split = workspace && pick_split_k(m, n, k, cus, &bm, &bn, &split_k);
+    if (stream_atoms && split && !split_k_fits(m, n, bm, bn, split_k, workspace_bytes)) return int(hipErrorInvalidValue);
+    if (split && !stream_atoms) {
 #define YAN_SPLIT_K_CASE(BM, BN, S)                                                                                  \
     if (bm == BM && bn == BN && split_k == S)                                                                        \
         return int(yan::Gemm<0, 0, BM, BN, 128, 1, yan::Fp8TileConfig<BM, BN>::MAX_RING_STAGES, 1, yan::GemmType::Normal>::run_split_k<S>( \
@@ -264,9 +295,14 @@ int fp8_plain(const void* lhs, const float* lhs_scales, long long lhs_scales_str
 #undef YAN_SPLIT_K_CASE
         return int(hipErrorInvalidValue);
     }
-    if (skinny_atoms(m, n, cus))
-        return int(yan::launch_fp8_skinny<0, 0, 1, 8>(o, lhs, lhs_scales, int(lhs_scales_stride_m), int(lhs_scales_stride_k), rhs,
-                                                      rhs_scales, m, n, k, s));
+    if (const int atoms = stream_atoms ? stream_atoms : skinny_atoms(m, n, cus)) {
+#define YAN_STREAM_CASE(TM)                                                                                          \
+    if (atoms == TM)                                                                                                 \
+        return int(yan::launch_fp8_skinny<0, 0, TM>(o, lhs, lhs_scales, int(lhs_scales_stride_m), int(lhs_scales_stride_k), rhs, \
+                                                    rhs_scales, m, n, k, s, num_sms));
+        YAN_STREAM_CASE(1) YAN_STREAM_CASE(2) YAN_STREAM_CASE(3) YAN_STREAM_CASE(4)
+#undef YAN_STREAM_CASE
+    }
     pick(kFp8Tiles, m, n, cus, &bm, &bn);
 #define YAN_FP8_CASE(BM, BN)                                                                                         \
     if (bm == BM && bn == BN)                                                                                        \
@@ -408,11 +444,13 @@ int yan_per_block_cast_to_fp8(const void* w, int w_is_fp32, void* q, float* scal
 int yan_gemm_select_tile(int op, int m, int n, int k, int num_cus, int* block_m, int* block_n) {
     if (!block_m || !block_n || num_cus <= 0) return 1;
     if (op == 0) {
-        if (const int atoms = dense_skinny_atoms(m, n, k, num_cus)) { *block_m = 16 * atoms; *block_n = 16; }
+        const int streamed = weight_stream_dense_atoms(m, n, k, num_cus);
+        if (const int atoms = streamed ? streamed : dense_skinny_atoms(m, n, k, num_cus)) { *block_m = 16 * atoms; *block_n = 16; }
         else pick(kDenseTiles, m, n, num_cus, block_m, block_n);
     }
     else if (op == 1) {
-        if (const int atoms = skinny_atoms(m, n, num_cus)) { *block_m = 16 * atoms; *block_n = 16; }
+        const int streamed = weight_stream_fp8_atoms(m, n, k, num_cus);
+        if (const int atoms = streamed ? streamed : skinny_atoms(m, n, num_cus)) { *block_m = 16 * atoms; *block_n = 16; }
         else pick(kFp8Tiles, m, n, num_cus, block_m, block_n);
     }
     else if (op == 2) pick_grouped(m, n, num_cus, 1, 128, k, block_m, block_n);
@@ -431,6 +469,6 @@ int yan_gemm_select_split_k(int op, int m, int n, int k, int num_cus, int* block
     return 0;
 }
 
-const char* yan_gemm_version(void) { return "yan-gemm gfx950 11 dense + 22 split-K dense + 2 weight-streaming dense + 7 fp32 + 10 fp8 tile variants + 15 split-K fp8 variants + 1 weight-streaming fp8 variant + 12 grouped fp8 variants + 4 quantiser kernels"; }
+const char* yan_gemm_version(void) { return "yan-gemm gfx950 11 dense + 22 split-K dense + 4 weight-streaming dense + 7 fp32 + 10 fp8 tile variants + 15 split-K fp8 variants + 4 weight-streaming fp8 variant + 12 grouped fp8 variants + 4 quantiser kernels"; }
 
 } // extern "C"

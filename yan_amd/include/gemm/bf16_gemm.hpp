@@ -1077,7 +1077,7 @@ template <int BLOCK_M, int BLOCK_N, int NUM_STAGES, int WAVES = 0>
 inline hipError_t gemm_tn(int m, int n, int k, const __hip_bfloat16* A, const __hip_bfloat16* B, __hip_bfloat16* C,
                           hipStream_t stream, int num_sms = 0) {
     // BLOCK_N == 16 names the weight-streaming kernel for up to BLOCK_M activation rows (bf16_gemm_skinny.hpp)
-    if constexpr (BLOCK_N == 16) return yan::launch_dense_skinny<yan::MfmaBF16_16x16x32, __bf16, BLOCK_M / 16, 8>(m, n, k, A, B, C, stream);
+    if constexpr (BLOCK_N == 16) return yan::launch_dense_skinny<yan::MfmaBF16_16x16x32, __bf16, BLOCK_M / 16>(m, n, k, A, B, C, stream, num_sms);
     else return yan::launch_dense<yan::MfmaBF16_32x32x16, __bf16, BLOCK_M, BLOCK_N, NUM_STAGES, WAVES>(m, n, k, A, B, C, stream, num_sms);
 }
 
@@ -1096,6 +1096,6 @@ inline hipError_t gemm_tn_split_k(int m, int n, int k, const __half* A, const __
 
 template <int BLOCK_M, int BLOCK_N, int NUM_STAGES, int WAVES = 0>
 inline hipError_t gemm_tn(int m, int n, int k, const __half* A, const __half* B, __half* C, hipStream_t stream, int num_sms = 0) {
-    if constexpr (BLOCK_N == 16) return yan::launch_dense_skinny<yan::MfmaF16_16x16x32, _Float16, BLOCK_M / 16, 8>(m, n, k, A, B, C, stream);
+    if constexpr (BLOCK_N == 16) return yan::launch_dense_skinny<yan::MfmaF16_16x16x32, _Float16, BLOCK_M / 16>(m, n, k, A, B, C, stream, num_sms);
     else return yan::launch_dense<yan::MfmaF16_32x32x16, _Float16, BLOCK_M, BLOCK_N, NUM_STAGES, WAVES>(m, n, k, A, B, C, stream, num_sms);
 }

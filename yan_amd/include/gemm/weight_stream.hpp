@@ -1,0 +1,199 @@
+// GEMM for few activation rows, bound by streaming the weights out of HBM once: one workgroup per 8, 16 or 32 weight rows, K shared
+// out over its 8 waves, no meeting of workgroups. FP8 with 128-block scales (fp8_gemm_skinny.hpp) and bf16 / fp16
+// (bf16_gemm_skinny.hpp) are launched from here; contracts as in fp8_gemm.hpp and bf16_gemm.hpp.
+//   * Wave w owns the 128-byte K blocks w, w + 8, w + 16, ... and copies the tile's weight rows and all activation rows of up to 4 of
+//     them ahead into LDS slots of its own (buffer_load .. lds): nothing is shared before the partial sums meet, so the main loop
+//     has no barrier, only the wave's own counts of copies in flight.
+//   * Whole 128-byte lines are what a compute unit copies fast. Read straight into fragments (16 rows at 16 or 64 bytes per lane
+//     group) operands that sit in L2 come in at 40 bytes/ns per compute unit, 8 rows x 128 bytes at a time at 125 - 190, into registers or
+//     into LDS alike. The kernel that loaded fragments, 1 row, FP8, call to call: 2112 x 7168 9.7 us, this one 5.3 (split K over 3
+//     workgroups per tile, their sums meeting in memory: 8.5); 1024 x 7168 9.3 / 4.5 (7.5); bf16 4096 x 2048 6.9 / 4.9,
+//     16 rows x 1984 x 4608 12.6 / 6.8 (split: 9.8).
+//   * What bounds it: weights at 6 - 7 TB/s where every compute unit has a tile, else the tile's rows + activation rows, pulled at
+//     about 62 bytes/ns per compute unit (half of them behind loads that go to HBM), + 3.3 us of launch, first loads and the sum.
+//   * Every workgroup reads all activations; each starts at another K block and wraps around, which spreads the requests over them.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "utils.hpp"
+#include "mfma_utils.hpp"
+#include "tile_io.hpp"
+
+namespace yan {
+
+// ROWS weight rows and A_ROWS activation rows per workgroup; a slot holds one K block of both and, with SCALES, a float per row.
+template <int ROWS, int A_ROWS, bool SCALES>
+struct WeightStreamShape {
+    static_assert((ROWS == 8 || ROWS % 16 == 0) && (A_ROWS == 8 || A_ROWS % 16 == 0) && A_ROWS <= kWaveSize);
+    static constexpr int NUM_WAVES = 8;
+    static constexpr int LOADS = ROWS / 8 + A_ROWS / 8 + (SCALES ? 1 : 0);
+    static constexpr int SLOT  = (ROWS + A_ROWS) * kRowBytes + (SCALES ? kWaveSize * 4 : 0);
+    static constexpr int FIT   = 152 * 1024 / (SLOT * NUM_WAVES);
+    static constexpr int DEPTH = FIT < 4 ? FIT : 4;         // 3 to 5 measure alike; 8 is slower on a row (more copies in front of the first sum)
+    static constexpr int ATOMS = ceil_div(A_ROWS, 16), B_ATOMS = ceil_div(ROWS, 16);
+    static_assert(DEPTH >= 1 && DEPTH * SLOT >= B_ATOMS * ATOMS * kWaveSize * 16 && (DEPTH - 1) * LOADS < kNoWaitVm);
+};
+
+// Wait for the oldest of a wave's blocks when `later` blocks of LOADS copies each were issued after it (at most MAX).
+template <int LOADS, int MAX>
+__device__ __forceinline__ void wait_for_block(int later) {
+    if constexpr (MAX > 0) {
+        if (later < MAX) return wait_for_block<LOADS, MAX - 1>(later);
+    }
+    __builtin_amdgcn_s_waitcnt(waitcnt_imm(MAX * LOADS, kNoWaitLgkm));
+    asm volatile("" ::: "memory");
+}
+
+// SCALES: FP8 operands with a scale per row and K block of the activations and per 128 weight rows and K block; else 16-bit ones.
+// SHAPE_N, SHAPE_K_BYTES: the sizes when known at compile time, or 0.
+template <typename Atom, typename Out, int SHAPE_N, int SHAPE_K_BYTES, int ROWS, int A_ROWS, bool SCALES>
+__global__ void __launch_bounds__(8 * kWaveSize)
+weight_stream_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_scales, const uint8_t* __restrict__ rhs,
+                     const float* __restrict__ rhs_scales, Out* __restrict__ out, int m, int n_rt, int k_bytes_rt, int sa_stride_m, int sa_stride_k) {
+    using Shape = WeightStreamShape<ROWS, A_ROWS, SCALES>;
+    constexpr int NUM_WAVES = Shape::NUM_WAVES, DEPTH = Shape::DEPTH, SLOT = Shape::SLOT, ATOMS = Shape::ATOMS, B_ATOMS = Shape::B_ATOMS;
+    constexpr int A_AT = ROWS * kRowBytes, SCALES_AT = (ROWS + A_ROWS) * kRowBytes;         // within a slot
+    const int n = SHAPE_N ? SHAPE_N : n_rt, k_bytes = SHAPE_K_BYTES ? SHAPE_K_BYTES : k_bytes_rt;
+    const int num_k_blocks = k_bytes / kRowBytes;
+
+    __shared__ __attribute__((aligned(1024))) uint8_t slots[NUM_WAVES * DEPTH * SLOT];
+
+    const int n0 = blockIdx.x * ROWS;
+    const int lane = get_lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+    const int g = lane / 16, col = lane % 16, sub = lane / 8;
+
+    const __amdgpu_buffer_rsrc_t rsrc_a = make_rsrc(lhs, uint32_t(m) * k_bytes);
+    const __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(rhs, uint32_t(n) * k_bytes);
+    __amdgpu_buffer_rsrc_t rsrc_sa = rsrc_a;
+    const float* sb_row = nullptr;
+    if constexpr (SCALES) {
+        rsrc_sa = make_rsrc(lhs_scales, (uint32_t(m - 1) * sa_stride_m + uint32_t(num_k_blocks - 1) * sa_stride_k + 1) * 4);
+        sb_row = rhs_scales + size_t(min(n0 / 128, ceil_div(n, 128) - 1)) * num_k_blocks;
+    }
+    // A copy moves 8 rows of a block, swizzled as tile_io.hpp has it; rows past the end of either matrix read as zero.
+    const uint32_t chunk = uint32_t((lane & 7) ^ sub) * kChunk;
+    const uint32_t voff_b = uint32_t(n0 + sub) * k_bytes, voff_a = uint32_t(sub) * k_bytes;
+    const uint32_t voff_sa = lane < m && lane < A_ROWS ? uint32_t(lane) * sa_stride_m * 4 : kOutOfRange;
+
+    const int rot = (blockIdx.x * 7) % num_k_blocks;
+    auto rotated = [&](int kb) { const int r = kb + rot; return r >= num_k_blocks ? r - num_k_blocks : r; };
+
+    uint8_t* const own = slots + wave * (DEPTH * SLOT);
+    auto issue = [&](int block, int slot) {
+        const int kb = rotated(block);
+        uint8_t* const to = own + slot * SLOT;
+#pragma unroll
+        for (int p = 0; p < ROWS / 8; ++p)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, YAN_LDS_PTR(to + p * 8 * kRowBytes), kChunk, voff_b + (chunk ^ (p & 1) * kChunk),
+                                                     kb * kRowBytes + p * 8 * k_bytes, 0, 0);
+#pragma unroll
+        for (int p = 0; p < A_ROWS / 8; ++p)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, YAN_LDS_PTR(to + A_AT + p * 8 * kRowBytes), kChunk, voff_a + (chunk ^ (p & 1) * kChunk),
+                                                     kb * kRowBytes + p * 8 * k_bytes, 0, 0);
+        if constexpr (SCALES) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_sa, YAN_LDS_PTR(to + SCALES_AT), 4, voff_sa, kb * sa_stride_k * 4, 0, 0);
+    };
+
+    // Lane (col, g) holds chunks 2g and 2g + 1 of row `col` of an atom. An atom of 8 rows is read twice, its second sums go nowhere.
+    auto offset = [&](int row, int c) { return row * kRowBytes + ((c ^ swizzle_of_row(row)) * kChunk); };
+    const int row_b = ROWS == 8 ? col & 7 : col, row_a = A_ROWS == 8 ? col & 7 : col;
+    const int b_lo = offset(row_b, 2 * g), b_hi = offset(row_b, 2 * g + 1), a_lo = A_AT + offset(row_a, 2 * g), a_hi = A_AT + offset(row_a, 2 * g + 1);
+
+    f32x4 acc[B_ATOMS][ATOMS];
+#pragma unroll
+    for (int i = 0; i < B_ATOMS; ++i)
+#pragma unroll
+        for (int j = 0; j < ATOMS; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+    for (int s = 0; s < DEPTH; ++s)
+        if (wave + s * NUM_WAVES < num_k_blocks) issue(wave + s * NUM_WAVES, s);
+    for (int first = wave; first < num_k_blocks; first += DEPTH * NUM_WAVES) {
+#pragma unroll
+        for (int s = 0; s < DEPTH; ++s) {
+            const int block = first + s * NUM_WAVES;
+            if (block >= num_k_blocks) break;
+            float sb = 0.f;
+            if constexpr (SCALES) sb = sb_row[rotated(block)];
+            wait_for_block<Shape::LOADS, DEPTH - 1>((num_k_blocks - 1 - block) / NUM_WAVES);
+            const uint8_t* const from = own + s * SLOT;
+            i32x4 b[B_ATOMS][2], a[ATOMS][2];
+            float scale[ATOMS];
+#pragma unroll
+            for (int i = 0; i < B_ATOMS; ++i) {
+                b[i][0] = *reinterpret_cast<const i32x4*>(from + b_lo + i * 16 * kRowBytes);
+                b[i][1] = *reinterpret_cast<const i32x4*>(from + b_hi + i * 16 * kRowBytes);
+            }
+#pragma unroll
+            for (int j = 0; j < ATOMS; ++j) {
+                a[j][0] = *reinterpret_cast<const i32x4*>(from + a_lo + j * 16 * kRowBytes);
+                a[j][1] = *reinterpret_cast<const i32x4*>(from + a_hi + j * 16 * kRowBytes);
+                if constexpr (SCALES) scale[j] = *reinterpret_cast<const float*>(from + SCALES_AT + (j * 16 + col) * 4);
+            }
+            // the slot is read: its next block may come
+            __builtin_amdgcn_s_waitcnt(waitcnt_imm(kNoWaitVm, 0));
+            asm volatile("" ::: "memory");
+            if (block + DEPTH * NUM_WAVES < num_k_blocks) issue(block + DEPTH * NUM_WAVES, s);
+#pragma unroll
+            for (int j = 0; j < ATOMS; ++j)
+#pragma unroll
+                for (int i = 0; i < B_ATOMS; ++i) {
+                    if constexpr (SCALES) {
+                        const i32x8 bf = {b[i][0][0], b[i][0][1], b[i][0][2], b[i][0][3], b[i][1][0], b[i][1][1], b[i][1][2], b[i][1][3]};
+                        const i32x8 af = {a[j][0][0], a[j][0][1], a[j][0][2], a[j][0][3], a[j][1][0], a[j][1][1], a[j][1][2], a[j][1][3]};
+                        const f32x4 p = Atom::mma(bf, af, f32x4{0.f, 0.f, 0.f, 0.f});
+                        const float ab = scale[j] * sb;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) acc[i][j][r] = __builtin_fmaf(p[r], ab, acc[i][j][r]);
+                    } else {
+                        using Frag = typename Atom::Frag;
+                        acc[i][j] = Atom::mma(__builtin_bit_cast(Frag, b[i][0]), __builtin_bit_cast(Frag, a[j][0]), acc[i][j]);
+                        acc[i][j] = Atom::mma(__builtin_bit_cast(Frag, b[i][1]), __builtin_bit_cast(Frag, a[j][1]), acc[i][j]);
+                    }
+                }
+        }
+    }
+
+    // The partial sums of the 8 waves meet in their slots (a wave has no copy in flight and no slot to read any more).
+#pragma unroll
+    for (int i = 0; i < B_ATOMS; ++i)
+#pragma unroll
+        for (int j = 0; j < ATOMS; ++j) *reinterpret_cast<f32x4*>(own + ((i * ATOMS + j) * kWaveSize + lane) * 16) = acc[i][j];
+    __syncthreads();
+    if (wave < B_ATOMS * ATOMS) {
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < NUM_WAVES; ++w) sum += *reinterpret_cast<const f32x4*>(slots + w * (DEPTH * SLOT) + (wave * kWaveSize + lane) * 16);
+        // the 4 registers are weight rows nn .. nn + 3 of activation row mm
+        const int nn = n0 + wave / ATOMS * 16 + 4 * g, mm = wave % ATOMS * 16 + col;
+        if (mm < m && 4 * g < ROWS && nn < n) *reinterpret_cast<decltype(pack4(sum, Out{}))*>(out + size_t(mm) * n + nn) = pack4(sum, Out{});
+    }
+}
+
+// Launch for m <= 16 * TM. Workgroups take as few weight rows as fit the chip (or the cap of `num_sms` workgroups) in one round:
+// less to pull for each of them. 8 rows: 1472 x 15104, one row, FP8, 6.9 us (16 rows: 8.2); 16 where 8 take two rounds:
+// 4096 x 7168 7.0 us (8: 7.4); 32 beyond: 7168 x 2048, 32 rows, bf16 8.0 us (16: 10.2). False when a 32-bit offset does not reach.
+template <typename Atom, typename Out, int SHAPE_N, int SHAPE_K_BYTES, int TM, bool SCALES>
+inline bool launch_weight_stream(const void* lhs, const float* lhs_scales, int sa_stride_m, int sa_stride_k, const void* rhs, const float* rhs_scales,
+                                 void* out, int m, int n, int k_bytes, int num_sms, hipStream_t stream) {
+    if (uint64_t(16 * TM) * k_bytes >= kOutOfRange || (uint64_t(n) + 32) * k_bytes >= kOutOfRange) return false;
+    const int cus = num_sms > 0 && num_sms < device_cu_count() ? num_sms : device_cu_count();
+    auto launch = [&]<int ROWS, int A_ROWS>() {
+        hipLaunchKernelGGL((weight_stream_kernel<Atom, Out, SHAPE_N, SHAPE_K_BYTES, ROWS, A_ROWS, SCALES>), dim3(ceil_div(n, ROWS)), dim3(8 * kWaveSize), 0,
+                           stream, static_cast<const uint8_t*>(lhs), lhs_scales, static_cast<const uint8_t*>(rhs), rhs_scales,
+                           static_cast<Out*>(out), m, n, k_bytes, sa_stride_m, sa_stride_k);
+    };
+    auto rows = [&]<int A_ROWS>() {
+        if (ceil_div(n, 8) <= cus) launch.template operator()<8, A_ROWS>();
+        else if (ceil_div(n, 16) <= cus) launch.template operator()<16, A_ROWS>();
+        else launch.template operator()<32, A_ROWS>();
+    };
+    if constexpr (TM == 1) {
+        if (m <= 8) rows.template operator()<8>();
+        else rows.template operator()<16>();
+    } else rows.template operator()<16 * TM>();
+    return true;
+}
+
+} // namespace yan

@@ -12,8 +12,8 @@ import functools
 
 import torch
 
-from .heuristics import (get_best_dense_config, get_dense_num_stages, get_dense_tile_space, get_skinny_dense_config,
-                         get_split_k_dense_config, tuning_enabled)
+from .heuristics import (get_best_dense_config, get_dense_num_stages, get_dense_tile, get_dense_tile_space, get_skinny_dense_config,
+                         get_split_k_dense_config, tuning_enabled, get_weight_stream_dense_config)
 from .host_calls import BF16, FP16, remember_call, repeat_call
 from .split_k import SPLIT_K_WORKSPACE_BYTES, split_k_launch_failed, split_k_workspace
 from .tuner import FrozenKeys, jit_tuner
@@ -52,7 +52,8 @@ def _split_k_arg_defs(dtype: torch.dtype):
 @functools.lru_cache(maxsize=None)
 def dense_split_k_plan(m: int, n: int, k: int, dtype: torch.dtype, num_cus: int):
     """(name, keys, arg_defs) of the split-K kernel a call with these sizes uses, or None when K is not split
-    (`get_split_k_dense_config`); needs no GPU."""
+    (`get_split_k_dense_config`); where `get_weight_stream_dense_config` takes a problem the entry goes by `dense_kernel_plan` instead.
+    Needs no GPU."""
     plan = get_split_k_dense_config(m, n, k, num_cus)
     if plan is None:
         return None
@@ -67,10 +68,10 @@ def dense_kernel_plan(m: int, n: int, k: int, dtype: torch.dtype, num_cus: int, 
     """(name, keys, arg_defs) of the JIT kernel a call with these sizes uses; needs no GPU. `num_cus` steers the tile
     choice, `num_sms_cap` (0 = none) is the number of workgroups the launch may start."""
     name = 'gemm_bf16_tn' if dtype == torch.bfloat16 else 'gemm_fp16_tn'
-    skinny_atoms = get_skinny_dense_config(m, n, k, num_cus)
+    skinny_atoms = get_weight_stream_dense_config(m, n, k, num_cus) or get_skinny_dense_config(m, n, k, num_cus)
     if skinny_atoms:
-        # the weight-streaming kernel for a handful of rows: BLOCK_N = 16 names it, its n / 16 workgroups are within any cap
-        return name, FrozenKeys({'BLOCK_M': 16 * skinny_atoms, 'BLOCK_N': 16, 'NUM_STAGES': 1, 'NUM_SMS': 0}), _arg_defs(dtype)
+        # the weight-streaming kernel for few rows: BLOCK_N = 16 names it, its launch takes the weight rows per workgroup that the cap asks for
+        return name, FrozenKeys({'BLOCK_M': 16 * skinny_atoms, 'BLOCK_N': 16, 'NUM_STAGES': 1, 'NUM_SMS': num_sms_cap}), _arg_defs(dtype)
     block_m, block_n = get_best_dense_config(m, n, k, num_cus)
     keys = FrozenKeys({'BLOCK_M': block_m, 'BLOCK_N': block_n, 'NUM_STAGES': get_dense_num_stages(block_m, block_n), 'NUM_SMS': num_sms_cap})
     return name, keys, _arg_defs(dtype)
@@ -103,11 +104,11 @@ def _gemm_16bit_tn(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, dtype: tor
     stream = current_raw_stream()
     args = (m, n, k, a, b, c, stream)
     code_template, workspace, workspace_token = template, None, None
-    if tuning_enabled() and not get_skinny_dense_config(m, n, k, get_num_sms()):
+    if tuning_enabled() and get_dense_tile(m, n, k, get_num_sms())[1] != 16:
         name, keys, space, arg_defs = dense_tuning_plan(m, n, k, dtype, get_num_sms(), get_num_sms_cap())
     else:
         (name, keys, arg_defs), space = dense_kernel_plan(m, n, k, dtype, get_num_sms(), get_num_sms_cap()), ()
-        split = dense_split_k_plan(m, n, k, dtype, get_num_sms())
+        split = None if get_weight_stream_dense_config(m, n, k, get_num_sms()) else dense_split_k_plan(m, n, k, dtype, get_num_sms())
         if split is not None:
             workspace, workspace_token = split_k_workspace(c.device, stream)
             if workspace is not None:

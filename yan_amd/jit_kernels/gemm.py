@@ -17,7 +17,7 @@ import torch
 
 from .fp8_cast import per_token_cast_to_fp8
 from .heuristics import (get_best_fp8_config, get_fp8_num_stages, get_fp8_tile_space, get_skinny_fp8_config,
-                         get_split_k_fp8_config, tuning_enabled)
+                         get_split_k_fp8_config, get_weight_stream_fp8_config, tuning_enabled)
 from .host_calls import CAST_FP8, FP8, remember_call, repeat_call
 from .split_k import SPLIT_K_COUNTER_BYTES, SPLIT_K_WORKSPACE_BYTES, split_k_enabled, split_k_launch_failed, split_k_workspace
 from .tuner import FrozenKeys, jit_tuner
@@ -53,13 +53,13 @@ using GemmType = Gemm<N, K, BLOCK_M, BLOCK_N, 128, 1, kNumStages, kNumTMAMultica
 __return_code = static_cast<int>(GemmType::run(out, lhs, lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k,
                                                rhs, rhs_scales, m, stream, num_sms, smem_size, kTokenContiguous));
 """
-# A handful of activation rows: BLOCK_M / 16 activation atoms and 16 weight rows per workgroup, the K blocks of a
-# workgroup shared out over NUM_WAVES waves; no LDS staging, NUM_STAGES is the per-wave load depth's name only.
+# Few activation rows: BLOCK_M / 16 activation atoms; BLOCK_N = 16 names the weight-streaming kernel, whose launch chooses the weight
+# rows of a workgroup by n, the m and the workgroups allowed (gemm/weight_stream.hpp).
 _skinny_launch = """static_assert(BLOCK_N == 16 && BLOCK_M % 16 == 0);
 
 // Launch kernel
-__return_code = static_cast<int>(launch_fp8_skinny<N, K, BLOCK_M / 16, {NUM_WAVES}>(
-    out, lhs, lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k, rhs, rhs_scales, m, N, K, stream));
+__return_code = static_cast<int>(launch_fp8_skinny<N, K, BLOCK_M / 16>(
+    out, lhs, lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k, rhs, rhs_scales, m, N, K, stream, num_sms));
 """
 
 # K split over SPLIT_K workgroups per tile; the parts meet in `workspace` (Gemm::run_split_k in gemm/fp8_gemm.hpp).
@@ -114,10 +114,9 @@ def fp8_kernel_plan(m: int, n: int, k: int, num_cus: int, token_contiguous_scale
     defs = arg_defs if token_contiguous_scales else strided_arg_defs
     # the tuner memoises per (name, keys): the two argument lists need two names
     name = 'gemm_fp8_fp8_bf16_nt' if token_contiguous_scales else 'gemm_fp8_fp8_bf16_nt_strided'
-    skinny_atoms = get_skinny_fp8_config(m, n, k, num_cus)
+    skinny_atoms = get_weight_stream_fp8_config(m, n, k, num_cus) or get_skinny_fp8_config(m, n, k, num_cus)
     if skinny_atoms:
-        keys = FrozenKeys({'N': n, 'K': k, 'BLOCK_M': 16 * skinny_atoms, 'BLOCK_N': 16, 'NUM_STAGES': 4, 'NUM_TMA_MULTICAST': 1,
-                'NUM_WAVES': 8})
+        keys = FrozenKeys({'N': n, 'K': k, 'BLOCK_M': 16 * skinny_atoms, 'BLOCK_N': 16, 'NUM_STAGES': 4, 'NUM_TMA_MULTICAST': 1})
         return (name, keys, defs, 8 * skinny_atoms * 64 * 16,
                 skinny_template if token_contiguous_scales else skinny_strided_template)
     block_m, block_n = get_best_fp8_config(m, n, k, num_cus)
@@ -130,7 +129,8 @@ def fp8_kernel_plan(m: int, n: int, k: int, num_cus: int, token_contiguous_scale
 @functools.lru_cache(maxsize=None)
 def fp8_split_k_plan(m: int, n: int, k: int, num_cus: int, token_contiguous_scales: bool = True):
     """(name, keys, arg_defs, template) of the split-K kernel a call with these sizes uses, or None when K is not split
-    (`get_split_k_fp8_config`); needs no GPU."""
+    (`get_split_k_fp8_config`); where `get_weight_stream_fp8_config` takes a problem the entry goes by `fp8_kernel_plan` instead. Needs
+    no GPU."""
     plan = get_split_k_fp8_config(m, n, k, num_cus)
     if plan is None:
         return None
@@ -146,7 +146,7 @@ def fp8_split_k_plan(m: int, n: int, k: int, num_cus: int, token_contiguous_scal
 def fp8_tuning_plan(m: int, n: int, k: int, num_cus: int, token_contiguous_scales: bool = True):
     """(name, keys, space, arg_defs, template) for empirical tile selection among the cost model's three best tiles of
     the tiled kernel (`m` joins the keys as the tuner's memo key), or None when the weight-streaming kernel runs."""
-    if get_skinny_fp8_config(m, n, k, num_cus):
+    if get_weight_stream_fp8_config(m, n, k, num_cus) or get_skinny_fp8_config(m, n, k, num_cus):
         return None
     space = tuple({'BLOCK_M': bm, 'BLOCK_N': bn, 'NUM_STAGES': get_fp8_num_stages(bm, bn)}
                   for bm, bn in get_fp8_tile_space(m, n, k, num_cus))
@@ -201,7 +201,7 @@ def gemm_fp8_fp8_bf16_nt(lhs: Tuple[torch.Tensor, torch.Tensor],
         if tuning is not None:
             name, keys, space, defs, code_template = tuning
     else:
-        split = fp8_split_k_plan(m, n, k, num_sms, token_contiguous)
+        split = None if get_weight_stream_fp8_config(m, n, k, num_sms) else fp8_split_k_plan(m, n, k, num_sms, token_contiguous)
         if split is not None:
             workspace, workspace_token = split_k_workspace(out.device, stream)
             if workspace is not None:
@@ -228,7 +228,7 @@ CAST_SCRATCH_BYTES = 4 << 20
 @functools.lru_cache(maxsize=None)
 def fp8_cast_chain_plan(m: int, n: int, k: int, num_cus: int, split_k_allowed: bool = True):
     """(name, keys, arg_defs, template, smem_size) of the kernel.so whose `launch` enqueues the per-token quantiser and then the
-    GEMM the FP8 entry would run for these sizes (split-K plan, weight-streaming kernel or tiles), or None when the codes
+    GEMM the FP8 entry would run for these sizes (split-K plan when allowed, weight-streaming kernel or tiles), or None when the codes
     and scales of `m` rows do not fit the scratch area; needs no GPU."""
     if m <= 0 or m * k + m * (k // 128) * 4 + 256 > CAST_SCRATCH_BYTES:
         return None
@@ -271,7 +271,9 @@ def gemm_bf16_fp8_bf16_nt(x: torch.Tensor, rhs: Tuple[torch.Tensor, torch.Tensor
     if m == 0:
         return
     num_sms = get_num_sms()
-    plan = fp8_cast_chain_plan(m, n, k, num_sms) if split_k_enabled() and not tuning_enabled() else None
+    plan = None
+    if split_k_enabled() and not tuning_enabled():
+        plan = fp8_cast_chain_plan(m, n, k, num_sms, split_k_allowed=not get_weight_stream_fp8_config(m, n, k, num_sms))
     if plan is None:
         gemm_fp8_fp8_bf16_nt(per_token_cast_to_fp8(x, col_major_scales=True), rhs, out)
         return

@@ -7,6 +7,7 @@ one workgroup per tile, one workgroup per CU at a time, so a launch costs
 `ceil(tiles / num_cus)` rounds of one tile time, and a tile's time grows with its MFMA work but shrinks per
 flop as the tile gets larger (fewer operand bytes fetched per flop).
 """
+import functools
 from typing import List, Optional, Tuple
 
 from .utils import ceil_div, env_switch
@@ -161,26 +162,18 @@ def get_contiguous_rows_on_device(m: int, n: int, k: int, num_cus: int, groups_i
 
 
 def get_skinny_fp8_config(m: int, n: int, k: int, num_cus: int) -> int:
-    """Number of 16-row activation atoms (1) when the weight-streaming kernel should run instead of the tiled one, else 0:
-    up to 16 activation rows, and few enough weight rows that its n/16 workgroups fit the chip in one round. Measured
-    on 256 CUs (kernel time warm / after a cache flush, weight-streaming vs tiled with its ring of LDS stages):
-    m = 1..16, n = 4096, k = 7168: 7.4-9.3 / 13.4 us vs 13.7-14.0 / 15.3 us; n = 2048: 6.9-9.1 / 9.4-10.4 vs 13.6 / 14.4;
-    n = 7168: 12.9-15.5 / 22 vs 15.5 / 21 (a tie, and two rounds of workgroups). From 17 rows up the tiled kernel wins or
-    ties everywhere (m = 64, n = 4096, k = 7168: 14.5 / 17.2 us)."""
+    """Number of 16-row activation atoms (1) when the weight-streaming kernel runs instead of the tiled one where K is not split,
+    else 0: up to 16 activation rows, and few enough weight rows that n / 16 workgroups fit the chip in one round. There it is
+    faster than the tiles whatever K is (16 rows x 1472 x 15104: 9.7 us). `get_weight_stream_fp8_config` says where it also goes
+    before a split-K plan and which problems beyond these it takes."""
     if 0 < m <= 16 and 16 <= n <= 16 * num_cus:
         return 1
     return 0
 
 
 def get_skinny_dense_config(m: int, n: int, k: int, num_cus: int) -> int:
-    """Number of 16-row activation atoms (1 or 2) when the weight-streaming dense kernel should run instead of the tiled
-    one, else 0: up to 32 activation rows, few enough weight rows that its n/16 workgroups fit the chip in one round, and
-    whole 128-byte K blocks. The smallest dense tile gives a workgroup 64 weight rows: n = 4096 puts 64 of 256 compute
-    units to work. Measured call to call with the weights cycling through more matrices than the caches hold (bf16,
-    n = 4096, k = 7168; weight-streaming vs 64 x 64 tiles): m = 1: 14.5 vs 25.9 us, m = 16: 18.3 vs 27.0, m = 17: 21.3 vs
-    27.1, m = 32: 25.4 vs 30.1, m = 48: 30.7 vs 33.3 (three atoms: not offered), m = 64: a tie; n = 2112 alike. Beyond one
-    round of workgroups the tiles win (n = 7168, k = 2048: 11.7 vs 10.2 us at m = 1; n = 16384, k = 4096: 34.0 vs 30.7),
-    and two atoms lose on short K (k = 1024: 7.2 vs 6.0 us)."""
+    """The same for the dense 16-bit GEMM: 1 or 2 atoms, whole 128-byte K blocks. `get_weight_stream_dense_config` says where the
+    kernel also goes before a split-K plan and which problems beyond these it takes."""
     if n < 16 or n > 16 * num_cus or n % 4 or k <= 0 or k % 64:
         return 0
     if 0 < m <= 16:
@@ -190,15 +183,59 @@ def get_skinny_dense_config(m: int, n: int, k: int, num_cus: int) -> int:
     return 0
 
 
+def _weight_stream_pull(m: int, n: int, k_bytes: int, num_cus: int) -> int:
+    """Bytes a workgroup of the weight-streaming kernel pulls: its 8, 16 or 32 weight rows, as few as give one round of workgroups
+    (`launch_weight_stream` in gemm/weight_stream.hpp), and all `m` activation rows; 0 when 32 rows take more than a round, or
+    beyond 32-bit offsets."""
+    if m <= 0 or m > 64 or n < 16 or n % 4 or k_bytes <= 0 or k_bytes % 128 or (n + 32) * k_bytes >= 1 << 31:
+        return 0
+    for rows in (8, 16, 32):
+        if ceil_div(n, rows) <= num_cus:
+            return (rows + m) * k_bytes
+    return 0
+
+
+@functools.lru_cache(maxsize=None)
+def get_weight_stream_fp8_config(m: int, n: int, k: int, num_cus: int) -> int:
+    """Number of 16-row activation atoms (1 to 4) when the weight-streaming kernel goes before split-K plans and tiles, else 0.
+
+    Its time is 3.3 us + what a workgroup pulls at about 62 bytes/ns, or the weights at 6 to 7 TB/s; a split-K plan
+    pays 2 us for the meeting of the parts, the tiles of a short K too few workgroups. Measured per call, weights cycling through
+    more matrices than the caches hold, 23 shapes of n = 256 .. 8192, k = 1024 .. 16384, ten m each (split-K plan or tiles -> this
+    kernel): 1 x 2112 x 7168 8.7 -> 5.4 us, 1 x 4096 x 7168 9.8 -> 7.6, 16 x 1984 x 4608 6.7 -> 4.5, 32 x 2944 x 5632 10.3 -> 7.8,
+    40 x 4096 x 16384 22.3 -> 19.8. Up to 40 rows it loses only where a workgroup pulls more than 400 KB and the chip is not full
+    (20 x 1472 x 15104 10.9 -> 11.3; 32: 11.1 -> 13.3); with 48 rows it is level from 300 KB on (4096 x 7168 11.1 -> 11.3), with
+    64 from 130 KB on (4096 x 2048 4.7 -> 4.8; 3072 x 1536 4.5 -> 4.2; 2112 x 7168 10.3 -> 12.2). Same rule as
+    `weight_stream_fp8_atoms` in yan_amd/csrc/yan_gemm_capi.hip."""
+    pull = _weight_stream_pull(m, n, k, num_cus)
+    if pull and (pull <= 130_000 or (m <= 48 and pull <= 300_000) or (m <= 40 and (pull <= 400_000 or n >= 16 * num_cus))):
+        return ceil_div(m, 16)
+    return 0
+
+
+@functools.lru_cache(maxsize=None)
+def get_weight_stream_dense_config(m: int, n: int, k: int, num_cus: int) -> int:
+    """The same for the dense 16-bit GEMM, whose smallest tile holds 64 weight rows: up to 16 rows always (1 x 1024 x 7168
+    12.7 -> 5.5 us, 16 x 1472 x 15104 31.1 -> 16.7, 16 x 2112 x 7168 11.5 -> 11.6, the closest), above that while a workgroup pulls at most 450 KB,
+    580 KB where its rows fill the chip (64 x 4096 x 2048 10.2 -> 8.2, 40 x 1984 x 4608 10.8 -> 10.3 at 442 KB,
+    48 x 1984 x 4608 11.1 -> 11.0 at 516 KB, 32 x 1024 x 7168 11.1 -> 11.7 at 573 KB; 24 x 4096 x 7168 15.9 -> 15.2 at 573 KB,
+    32 x 4096 x 7168 16.2 -> 16.4 at 688 KB, 64 x 6144 x 3072 14.2 -> 14.7 at 590 KB). Same rule as
+    `weight_stream_dense_atoms` in yan_amd/csrc/yan_gemm_capi.hip."""
+    pull = _weight_stream_pull(m, n, 2 * k, num_cus)
+    if pull and (m <= 16 or pull <= (580_000 if n >= 16 * num_cus else 450_000)):
+        return ceil_div(m, 16)
+    return 0
+
+
 def get_dense_tile(m: int, n: int, k: int, num_cus: int) -> Tuple[int, int]:
     """(BLOCK_M, BLOCK_N) of the dense kernel that runs: (16 * atoms, 16) for the weight-streaming kernel."""
-    atoms = get_skinny_dense_config(m, n, k, num_cus)
+    atoms = get_weight_stream_dense_config(m, n, k, num_cus) or get_skinny_dense_config(m, n, k, num_cus)
     return (16 * atoms, 16) if atoms else get_best_dense_config(m, n, k, num_cus)
 
 
 def get_fp8_tile(m: int, n: int, k: int, num_cus: int) -> Tuple[int, int]:
     """(BLOCK_M, BLOCK_N) of the FP8 kernel that runs: (16 * atoms, 16) for the weight-streaming kernel."""
-    atoms = get_skinny_fp8_config(m, n, k, num_cus)
+    atoms = get_weight_stream_fp8_config(m, n, k, num_cus) or get_skinny_fp8_config(m, n, k, num_cus)
     return (16 * atoms, 16) if atoms else get_best_fp8_config(m, n, k, num_cus)
 
 
@@ -225,9 +262,9 @@ def get_split_k_fp8_config(m: int, n: int, k: int, num_cus: int) -> Optional[Tup
     k = 1536..16384) swept with every tile and factor, weights cycling through more matrices than the caches hold, the
     plan taken is the fastest measured or within 1 % of it wherever one is taken (64 x 4096 x 7168: 64 x 64 tiles in four
     parts; 32 x 2112 x 7168: 32 x 32 in three); over 80 shapes with a plan (m = 17..1024, 13 (n, k)) it takes 0.47 to 1.04 of the
-    unsplit time, median 0.83; k up to about 5000 in two parts, k = 2048 and n = 16384 or more stay unsplit. A plan also goes before the weight-streaming kernel of up to 16 rows (32 x 32 tiles in two to four parts
-    against that kernel, m = 1..16: n = 4096, k = 7168: 9.7 - 9.8 against 10.7 - 12.2 us; n = 2048: 8.4 against 10.1 - 11.8; level
-    at k = 4096 and at k = 16384 below 8 rows), which runs where no plan exists or no workspace is at hand. Same rule as
+    unsplit time, median 0.83; k up to about 5000 in two parts, k = 2048 and n = 16384 or more stay unsplit.
+    The weight-streaming kernel goes before a plan where
+    `get_weight_stream_fp8_config` says so. Same rule as
     `pick_split_k` in yan_amd/csrc/yan_gemm_capi.hip (a CPU test keeps the two in step)."""
     if m <= 0 or n <= 0:
         return None
@@ -275,12 +312,9 @@ def get_split_k_dense_config(m: int, n: int, k: int, num_cus: int) -> Optional[T
     256 x 7168 x 16384 113.4 -> 90.9, 512 x 4096 x 7168 53.4 -> 43.9 (hipBLASLt on the first five and the 256-row shapes: 22.7, 24.7, 49.6, 140.4);
     over 54 shapes swept with every tile and factor the plan is the fastest measured or within 6 % of it (11 % in one case),
     and over 118 shapes with a plan (m = 33..1024, 14 (n, k)) it takes 0.35 to 0.92 of the unsplit time, median 0.65. Same rule as
-    `pick_dense_split_k` in yan_amd/csrc/yan_gemm_capi.hip (a CPU test keeps the two in step). A plan goes before the
-    two-atom weight-streaming kernel (17 to 32 rows; n = 4096, k = 7168: 21.1 - 25.2 us against 14.8 - 14.9 for 64 x 64 tiles
-    in four parts), which therefore runs only where no plan exists or no workspace is at hand (the C library's plain entry
-    points), and before the one-atom kernel from 8 rows on K up to 8192 (m = 8: 15.8 against 14.7 us, m = 16: 18.2 against 14.8;
-    n = 2048: 15.0 / 17.5 against 12.3 / 12.4); below 8 rows and on longer K that kernel stays (m = 1: 14.5 against 14.7;
-    k = 16384, m = 8: 28.9 against 31.0)."""
+    `pick_dense_split_k` in yan_amd/csrc/yan_gemm_capi.hip (a CPU test keeps the two in step).
+    The weight-streaming kernel goes before a plan where `get_weight_stream_dense_config` says so; below 8 rows, and up to 16
+    on a K beyond 8192, there is no plan where that kernel fits."""
     if m <= 0 or n <= 0 or k <= 0 or ((m < 8 or (m <= 16 and k > 8192)) and get_skinny_dense_config(m, n, k, num_cus)):
         return None         # a handful of rows, or up to 16 on a long K: the one-atom weight-streaming kernel is as fast or faster
     k_tiles = ceil_div(k, 64)
