@@ -82,10 +82,10 @@ def test_version_and_tile_selection_match_python(lib):
 
 def test_weight_stream_choice_matches_python(lib):
     """Where the weight-streaming kernel goes before tiles and split-K plans: the same on both sides; up to 64 rows, one round of workgroups
-    of at most 32 weight rows, whole 128-byte K blocks, offsets of 32 bits."""
+    of at most 64 weight rows, whole 128-byte K blocks, offsets of 32 bits."""
     taken = 0
     for m in (1, 8, 16, 17, 32, 40, 41, 48, 49, 64, 65):
-        for n in (12, 16, 100, 102, 1472, 2044, 2052, 4096, 4100, 8192, 8196):
+        for n in (12, 16, 100, 102, 1472, 2044, 2052, 4096, 4100, 8192, 8196, 16384, 16388):
             for k in (64, 128, 576, 1536, 4608, 7168, 7176, 16384, 1 << 18):
                 for cus in (256, 80):
                     dense, fp8 = (f(m, n, k, cus) for f in (heuristics.get_weight_stream_dense_config, heuristics.get_weight_stream_fp8_config))
@@ -94,7 +94,7 @@ def test_weight_stream_choice_matches_python(lib):
                     for atoms, row_bytes in ((dense, 2 * k), (fp8, k)):
                         taken += atoms > 0
                         assert atoms in (0, yan.ceil_div(m, 16))
-                        assert not atoms or (m <= 64 and 16 <= n <= 32 * cus and n % 4 == 0 and row_bytes % 128 == 0 and (n + 32) * row_bytes < 1 << 31)
+                        assert not atoms or (m <= 64 and 16 <= n <= 64 * cus and n % 4 == 0 and row_bytes % 128 == 0 and (n + 64) * row_bytes < 1 << 31)
     assert taken > 500
 
 

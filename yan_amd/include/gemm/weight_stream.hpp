@@ -1,4 +1,4 @@
-// GEMM for few activation rows, bound by streaming the weights out of HBM once: one workgroup per 8, 16 or 32 weight rows, K shared
+// GEMM for few activation rows, bound by streaming the weights out of HBM once: one workgroup per 8, 16, 32 or 64 weight rows, K shared
 // out over its 8 waves, no meeting of workgroups. FP8 with 128-block scales (fp8_gemm_skinny.hpp) and bf16 / fp16
 // (bf16_gemm_skinny.hpp) are launched from here; contracts as in fp8_gemm.hpp and bf16_gemm.hpp.
 //   * Wave w owns the 128-byte K blocks w, w + 8, w + 16, ... and copies the tile's weight rows and all activation rows of up to 4 of
@@ -32,7 +32,7 @@ struct WeightStreamShape {
     static constexpr int FIT   = 152 * 1024 / (SLOT * NUM_WAVES);
     static constexpr int DEPTH = FIT < 4 ? FIT : 4;         // 3 to 5 measure alike; 8 is slower on a row (more copies in front of the first sum)
     static constexpr int ATOMS = ceil_div(A_ROWS, 16), B_ATOMS = ceil_div(ROWS, 16);
-    static_assert(DEPTH >= 1 && DEPTH * SLOT >= B_ATOMS * ATOMS * kWaveSize * 16 && (DEPTH - 1) * LOADS < kNoWaitVm);
+    static_assert(DEPTH >= 1 && B_ATOMS * ATOMS <= NUM_WAVES && DEPTH * SLOT >= B_ATOMS * ATOMS * kWaveSize * 16 && (DEPTH - 1) * LOADS < kNoWaitVm);
 };
 
 // Wait for the oldest of a wave's blocks when `later` blocks of LOADS copies each were issued after it (at most MAX).
@@ -173,11 +173,12 @@ weight_stream_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ 
 
 // Launch for m <= 16 * TM. Workgroups take as few weight rows as fit the chip (or the cap of `num_sms` workgroups) in one round:
 // less to pull for each of them. 8 rows: 1472 x 15104, one row, FP8, 6.9 us (16 rows: 8.2); 16 where 8 take two rounds:
-// 4096 x 7168 7.0 us (8: 7.4); 32 beyond: 7168 x 2048, 32 rows, bf16 8.0 us (16: 10.2). False when a 32-bit offset does not reach.
+// 4096 x 7168 7.0 us (8: 7.4); 32 beyond: 7168 x 2048, 32 rows, bf16 8.0 us (16: 10.2); 64 (up to 32 activation rows: one sum per wave)
+// beyond that: 32 rows x 9216 x 4096, FP8, 11.5 us (32: 13.6; tiles: 15.2). False when a 32-bit offset does not reach.
 template <typename Atom, typename Out, int SHAPE_N, int SHAPE_K_BYTES, int TM, bool SCALES>
 inline bool launch_weight_stream(const void* lhs, const float* lhs_scales, int sa_stride_m, int sa_stride_k, const void* rhs, const float* rhs_scales,
                                  void* out, int m, int n, int k_bytes, int num_sms, hipStream_t stream) {
-    if (uint64_t(16 * TM) * k_bytes >= kOutOfRange || (uint64_t(n) + 32) * k_bytes >= kOutOfRange) return false;
+    if (uint64_t(16 * TM) * k_bytes >= kOutOfRange || (uint64_t(n) + 64) * k_bytes >= kOutOfRange) return false;
     const int cus = num_sms > 0 && num_sms < device_cu_count() ? num_sms : device_cu_count();
     auto launch = [&]<int ROWS, int A_ROWS>() {
         hipLaunchKernelGGL((weight_stream_kernel<Atom, Out, SHAPE_N, SHAPE_K_BYTES, ROWS, A_ROWS, SCALES>), dim3(ceil_div(n, ROWS)), dim3(8 * kWaveSize), 0,
@@ -187,7 +188,8 @@ inline bool launch_weight_stream(const void* lhs, const float* lhs_scales, int s
     auto rows = [&]<int A_ROWS>() {
         if (ceil_div(n, 8) <= cus) launch.template operator()<8, A_ROWS>();
         else if (ceil_div(n, 16) <= cus) launch.template operator()<16, A_ROWS>();
-        else launch.template operator()<32, A_ROWS>();
+        else if (TM > 2 || ceil_div(n, 32) <= cus) launch.template operator()<32, A_ROWS>();
+        else if constexpr (TM <= 2) launch.template operator()<64, A_ROWS>();
     };
     if constexpr (TM == 1) {
         if (m <= 8) rows.template operator()<8>();
