@@ -85,7 +85,7 @@ def test_weight_stream_choice_matches_python(lib):
     of at most 64 weight rows, whole 128-byte K blocks, offsets of 32 bits."""
     taken = 0
     for m in (1, 8, 16, 17, 32, 40, 41, 48, 49, 64, 65):
-        for n in (12, 16, 100, 102, 1472, 2044, 2052, 4096, 4100, 8192, 8196, 16384, 16388):
+        for n in (12, 16, 100, 102, 1472, 2044, 2052, 4096, 4100, 5120, 8192, 8196, 12288, 16384, 16388):
             for k in (64, 128, 576, 1536, 4608, 7168, 7176, 16384, 1 << 18):
                 for cus in (256, 80):
                     dense, fp8 = (f(m, n, k, cus) for f in (heuristics.get_weight_stream_dense_config, heuristics.get_weight_stream_fp8_config))

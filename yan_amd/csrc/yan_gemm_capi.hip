@@ -102,28 +102,36 @@ int skinny_atoms(int m, int n, int num_cus) {
     return (m > 0 && m <= 16 && n >= 16 && n <= 16 * num_cus) ? 1 : 0;
 }
 
-// Bytes a workgroup of the weight-streaming kernel pulls, or 0, its weight rows, and whether a round of 16 or 32 of them fills the chip
-// (_weight_stream_pull in heuristics.py).
-struct StreamPull { long long bytes; int rows; bool full; };
+// Bytes a workgroup of the weight-streaming kernel pulls, or 0, its weight rows, and the number of workgroups (_weight_stream_pull in
+// heuristics.py).
+struct StreamPull { long long bytes; int rows, groups; };
 StreamPull weight_stream_pull(int m, int n, long long k_bytes, int num_cus) {
     if (m <= 0 || m > 64 || n < 16 || n % 4 != 0 || k_bytes <= 0 || k_bytes % 128 != 0 || (n + 64ll) * k_bytes >= 1ll << 31) return {};
-    for (const int rows : {8, 16, 32, 64})
-        if (const int groups = (n + rows - 1) / rows; groups <= num_cus && (rows < 64 || m <= 32))
-            return {(rows + m) * k_bytes, rows, (rows == 16 || rows == 32) && groups * 8 >= num_cus * 7};
+    for (const int rows : {8, 16, 24, 32, 40, 48, 64})
+        if (const int groups = (n + rows - 1) / rows; groups <= num_cus && (rows <= 32 || m <= 32)) return {(rows + m) * k_bytes, rows, groups};
     return {};
 }
 
 // Activation atoms when the weight-streaming kernel goes before split-K plans and tiles, else 0 (get_weight_stream_fp8_config and
 // get_weight_stream_dense_config in heuristics.py).
 int weight_stream_fp8_atoms(int m, int n, int k, int num_cus) {
-    const auto [pull, rows, full] = weight_stream_pull(m, n, k, num_cus);
-    const bool takes = pull <= 130000 || (m <= 48 && pull <= 300000) || (m <= 40 && (pull <= 400000 || full)) || (m <= 32 && n >= 16 * num_cus);
+    const auto [pull, rows, groups] = weight_stream_pull(m, n, k, num_cus);
+    const bool full = rows >= 16 && groups * 8 >= num_cus * 7, wide = rows >= 24;
+    const bool takes = m <= 32   ? pull <= 400000 || full || n >= 16 * num_cus
+                       : m <= 40 ? pull <= 400000 || full || wide
+                       : m <= 48 ? pull <= (wide ? 400000 : 300000) || (rows == 32 && full)
+                                 : pull <= (rows == 24 ? 365000 : 130000);
     return pull && takes ? (m + 15) / 16 : 0;
 }
 int weight_stream_dense_atoms(int m, int n, int k, int num_cus) {
-    const auto [pull, rows, full] = weight_stream_pull(m, n, 2ll * k, num_cus);
-    const int limit = rows == 64 ? 600000 : full ? (rows == 32 ? 800000 : 580000) : m <= 16 ? 580000 : 450000;
-    return pull && (pull <= limit || (m <= 16 && (full || n <= 16 * num_cus))) ? (m + 15) / 16 : 0;
+    const auto [pull, rows, groups] = weight_stream_pull(m, n, 2ll * k, num_cus);
+    const bool full = groups * 8 >= num_cus * 7;
+    const long long share = 3000000ll * groups / num_cus - 1490000;
+    const long long limit = rows <= 16   ? (rows == 16 && full ? 580000 : 450000)
+                            : rows == 24 ? (m <= 16 ? 1400000 : share < 850000 ? share : 850000)
+                            : rows == 32 ? (full ? 780000 : 600000)
+                                         : (rows == 64 ? 600000 : 1400000);
+    return pull && (pull <= limit || (m <= 16 && (rows <= 16 || rows == 32))) ? (m + 15) / 16 : 0;
 }
 
 // Whether a workspace holds what a split-K plan needs (launch_dense_split_k, Gemm::run_split_k): asked for also where the

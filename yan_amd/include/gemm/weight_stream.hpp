@@ -1,4 +1,4 @@
-// GEMM for few activation rows, bound by streaming the weights out of HBM once: one workgroup per 8, 16, 32 or 64 weight rows, K shared
+// GEMM for few activation rows, bound by streaming the weights out of HBM once: one workgroup per 8 to 64 weight rows, K shared
 // out over its 8 waves, no meeting of workgroups. FP8 with 128-block scales (fp8_gemm_skinny.hpp) and bf16 / fp16
 // (bf16_gemm_skinny.hpp) are launched from here; contracts as in fp8_gemm.hpp and bf16_gemm.hpp.
 //   * Wave w owns the 128-byte K blocks w, w + 8, w + 16, ... and copies the tile's weight rows and all activation rows of up to 4 of
@@ -25,13 +25,14 @@ namespace yan {
 // ROWS weight rows and A_ROWS activation rows per workgroup; a slot holds one K block of both and, with SCALES, a float per row.
 template <int ROWS, int A_ROWS, bool SCALES>
 struct WeightStreamShape {
-    static_assert((ROWS == 8 || ROWS % 16 == 0) && (A_ROWS == 8 || A_ROWS % 16 == 0) && A_ROWS <= kWaveSize);
+    static_assert(ROWS % 8 == 0 && (A_ROWS == 8 || A_ROWS % 16 == 0) && A_ROWS <= kWaveSize);
     static constexpr int NUM_WAVES = 8;
     static constexpr int LOADS = ROWS / 8 + A_ROWS / 8 + (SCALES ? 1 : 0);
     static constexpr int SLOT  = (ROWS + A_ROWS) * kRowBytes + (SCALES ? kWaveSize * 4 : 0);
     static constexpr int FIT   = 152 * 1024 / (SLOT * NUM_WAVES);
     static constexpr int DEPTH = FIT < 4 ? FIT : 4;         // 3 to 5 measure alike; 8 is slower on a row (more copies in front of the first sum)
     static constexpr int ATOMS = ceil_div(A_ROWS, 16), B_ATOMS = ceil_div(ROWS, 16);
+    static constexpr bool TWO_SCALES = SCALES && 128 % ROWS != 0;       // a tile can lie in two blocks of 128 weight rows
     static_assert(DEPTH >= 1 && B_ATOMS * ATOMS <= NUM_WAVES && DEPTH * SLOT >= B_ATOMS * ATOMS * kWaveSize * 16 && (DEPTH - 1) * LOADS < kNoWaitVm);
 };
 
@@ -67,10 +68,14 @@ weight_stream_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ 
     const __amdgpu_buffer_rsrc_t rsrc_a = make_rsrc(lhs, uint32_t(m) * k_bytes);
     const __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(rhs, uint32_t(n) * k_bytes);
     __amdgpu_buffer_rsrc_t rsrc_sa = rsrc_a;
-    const float* sb_row = nullptr;
+    const float* sb_row = nullptr, *sb_next = nullptr;
+    bool in_next[B_ATOMS];          // this lane's four sums of an atom are in the second block of 128 rows (it starts at a multiple of 8)
     if constexpr (SCALES) {
         rsrc_sa = make_rsrc(lhs_scales, (uint32_t(m - 1) * sa_stride_m + uint32_t(num_k_blocks - 1) * sa_stride_k + 1) * 4);
-        sb_row = rhs_scales + size_t(min(n0 / 128, ceil_div(n, 128) - 1)) * num_k_blocks;
+        sb_row = rhs_scales + size_t(n0 / 128) * num_k_blocks;
+        sb_next = rhs_scales + size_t(min(n0 / 128 + 1, ceil_div(n, 128) - 1)) * num_k_blocks;
+#pragma unroll
+        for (int i = 0; i < B_ATOMS; ++i) in_next[i] = n0 % 128 + i * 16 + 4 * g >= 128;
     }
     // A copy moves 8 rows of a block, swizzled as tile_io.hpp has it; rows past the end of either matrix read as zero.
     const uint32_t chunk = uint32_t((lane & 7) ^ sub) * kChunk;
@@ -95,10 +100,11 @@ weight_stream_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ 
         if constexpr (SCALES) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_sa, YAN_LDS_PTR(to + SCALES_AT), 4, voff_sa, kb * sa_stride_k * 4, 0, 0);
     };
 
-    // Lane (col, g) holds chunks 2g and 2g + 1 of row `col` of an atom. An atom of 8 rows is read twice, its second sums go nowhere.
+    // Lane (col, g) holds chunks 2g and 2g + 1 of row `col` of an atom. Half an atom of 8 rows is read twice, its second sums go nowhere.
     auto offset = [&](int row, int c) { return row * kRowBytes + ((c ^ swizzle_of_row(row)) * kChunk); };
-    const int row_b = ROWS == 8 ? col & 7 : col, row_a = A_ROWS == 8 ? col & 7 : col;
-    const int b_lo = offset(row_b, 2 * g), b_hi = offset(row_b, 2 * g + 1), a_lo = A_AT + offset(row_a, 2 * g), a_hi = A_AT + offset(row_a, 2 * g + 1);
+    const int row_a = A_ROWS == 8 ? col & 7 : col;
+    const int b_lo = offset(col, 2 * g), b_hi = offset(col, 2 * g + 1), a_lo = A_AT + offset(row_a, 2 * g), a_hi = A_AT + offset(row_a, 2 * g + 1);
+    const int half_lo = offset(col & 7, 2 * g), half_hi = offset(col & 7, 2 * g + 1);
 
     f32x4 acc[B_ATOMS][ATOMS];
 #pragma unroll
@@ -114,16 +120,18 @@ weight_stream_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ 
         for (int s = 0; s < DEPTH; ++s) {
             const int block = first + s * NUM_WAVES;
             if (block >= num_k_blocks) break;
-            float sb = 0.f;
+            float sb = 0.f, sb2 = 0.f;
             if constexpr (SCALES) sb = sb_row[rotated(block)];
+            if constexpr (Shape::TWO_SCALES) sb2 = sb_next[rotated(block)];
             wait_for_block<Shape::LOADS, DEPTH - 1>((num_k_blocks - 1 - block) / NUM_WAVES);
             const uint8_t* const from = own + s * SLOT;
             i32x4 b[B_ATOMS][2], a[ATOMS][2];
             float scale[ATOMS];
 #pragma unroll
             for (int i = 0; i < B_ATOMS; ++i) {
-                b[i][0] = *reinterpret_cast<const i32x4*>(from + b_lo + i * 16 * kRowBytes);
-                b[i][1] = *reinterpret_cast<const i32x4*>(from + b_hi + i * 16 * kRowBytes);
+                const bool half = i * 16 + 8 == ROWS;
+                b[i][0] = *reinterpret_cast<const i32x4*>(from + (half ? half_lo : b_lo) + i * 16 * kRowBytes);
+                b[i][1] = *reinterpret_cast<const i32x4*>(from + (half ? half_hi : b_hi) + i * 16 * kRowBytes);
             }
 #pragma unroll
             for (int j = 0; j < ATOMS; ++j) {
@@ -143,7 +151,7 @@ weight_stream_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ 
                         const i32x8 bf = {b[i][0][0], b[i][0][1], b[i][0][2], b[i][0][3], b[i][1][0], b[i][1][1], b[i][1][2], b[i][1][3]};
                         const i32x8 af = {a[j][0][0], a[j][0][1], a[j][0][2], a[j][0][3], a[j][1][0], a[j][1][1], a[j][1][2], a[j][1][3]};
                         const f32x4 p = Atom::mma(bf, af, f32x4{0.f, 0.f, 0.f, 0.f});
-                        const float ab = scale[j] * sb;
+                        const float ab = scale[j] * (Shape::TWO_SCALES && in_next[i] ? sb2 : sb);
 #pragma unroll
                         for (int r = 0; r < 4; ++r) acc[i][j][r] = __builtin_fmaf(p[r], ab, acc[i][j][r]);
                     } else {
@@ -166,15 +174,16 @@ weight_stream_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ 
 #pragma unroll
         for (int w = 0; w < NUM_WAVES; ++w) sum += *reinterpret_cast<const f32x4*>(slots + w * (DEPTH * SLOT) + (wave * kWaveSize + lane) * 16);
         // the 4 registers are weight rows nn .. nn + 3 of activation row mm
-        const int nn = n0 + wave / ATOMS * 16 + 4 * g, mm = wave % ATOMS * 16 + col;
-        if (mm < m && 4 * g < ROWS && nn < n) *reinterpret_cast<decltype(pack4(sum, Out{}))*>(out + size_t(mm) * n + nn) = pack4(sum, Out{});
+        const int row = wave / ATOMS * 16 + 4 * g, nn = n0 + row, mm = wave % ATOMS * 16 + col;
+        if (mm < m && row < ROWS && nn < n) *reinterpret_cast<decltype(pack4(sum, Out{}))*>(out + size_t(mm) * n + nn) = pack4(sum, Out{});
     }
 }
 
-// Launch for m <= 16 * TM. Workgroups take as few weight rows as fit the chip (or the cap of `num_sms` workgroups) in one round:
-// less to pull for each of them. 8 rows: 1472 x 15104, one row, FP8, 6.9 us (16 rows: 8.2); 16 where 8 take two rounds:
-// 4096 x 7168 7.0 us (8: 7.4); 32 beyond: 7168 x 2048, 32 rows, bf16 8.0 us (16: 10.2); 64 (up to 32 activation rows: one sum per wave)
-// beyond that: 32 rows x 9216 x 4096, FP8, 11.5 us (32: 13.6; tiles: 15.2). False when a 32-bit offset does not reach.
+// Launch for m <= 16 * TM. Workgroups take as few weight rows as fit the chip (or the cap of `num_sms` workgroups) in one round: less to
+// pull for each of them, and more of them. 8 rows: 1472 x 15104, one row, FP8, 6.9 us (16 rows: 8.2); 16 where 8 take two rounds:
+// 4096 x 7168 7.0 us (8: 7.4); 24 for 8 x 4100 x 16384 14.0 (32: 15.6); 32 for 32 x 7168 x 2048 in bf16 8.0 us (16, two rounds: 10.2). Beyond that
+// up to 32 activation rows (one sum per wave): 40 for 32 x 8200 x 8192 15.3 (48: 16.3; 64: 19.8; tiles: 25.7), 48 for 32 x 12288 x 2048 7.3
+// (64: 7.9; tiles: 10.0), then 64: with 56 HBM-bound shapes lose (13000 x 16384 bf16 70.5 -> 74.2). False when a 32-bit offset does not reach.
 template <typename Atom, typename Out, int SHAPE_N, int SHAPE_K_BYTES, int TM, bool SCALES>
 inline bool launch_weight_stream(const void* lhs, const float* lhs_scales, int sa_stride_m, int sa_stride_k, const void* rhs, const float* rhs_scales,
                                  void* out, int m, int n, int k_bytes, int num_sms, hipStream_t stream) {
@@ -188,8 +197,13 @@ inline bool launch_weight_stream(const void* lhs, const float* lhs_scales, int s
     auto rows = [&]<int A_ROWS>() {
         if (ceil_div(n, 8) <= cus) launch.template operator()<8, A_ROWS>();
         else if (ceil_div(n, 16) <= cus) launch.template operator()<16, A_ROWS>();
+        else if (ceil_div(n, 24) <= cus) launch.template operator()<24, A_ROWS>();
         else if (TM > 2 || ceil_div(n, 32) <= cus) launch.template operator()<32, A_ROWS>();
-        else if constexpr (TM <= 2) launch.template operator()<64, A_ROWS>();
+        else if constexpr (TM <= 2) {
+            if (ceil_div(n, 40) <= cus) launch.template operator()<40, A_ROWS>();
+            else if (ceil_div(n, 48) <= cus) launch.template operator()<48, A_ROWS>();
+            else launch.template operator()<64, A_ROWS>();
+        }
     };
     if constexpr (TM == 1) {
         if (m <= 8) rows.template operator()<8>();

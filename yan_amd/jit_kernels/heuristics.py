@@ -183,17 +183,16 @@ def get_skinny_dense_config(m: int, n: int, k: int, num_cus: int) -> int:
     return 0
 
 
-def _weight_stream_pull(m: int, n: int, k_bytes: int, num_cus: int) -> Tuple[int, int, bool]:
-    """Bytes a workgroup of the weight-streaming kernel pulls: its 8, 16, 32 or (up to 32 activation rows) 64 weight rows, as few as
+def _weight_stream_pull(m: int, n: int, k_bytes: int, num_cus: int) -> Tuple[int, int, int]:
+    """Bytes a workgroup of the weight-streaming kernel pulls: its 8 to 32 or (up to 32 activation rows) 64 weight rows, as few as
     give one round of workgroups (`launch_weight_stream` in gemm/weight_stream.hpp), and all `m` activation rows; 0 when that takes
-    more than a round, or beyond 32-bit offsets. Also those weight rows, and whether a round of 16 or 32 fills seven eighths of
-    the chip or more."""
+    more than a round, or beyond 32-bit offsets. Also those weight rows, and the number of workgroups."""
     if m <= 0 or m > 64 or n < 16 or n % 4 or k_bytes <= 0 or k_bytes % 128 or (n + 64) * k_bytes >= 1 << 31:
-        return 0, 0, False
-    for rows in (8, 16, 32, 64):
-        if ceil_div(n, rows) <= num_cus and (rows < 64 or m <= 32):
-            return (rows + m) * k_bytes, rows, rows in (16, 32) and ceil_div(n, rows) * 8 >= num_cus * 7
-    return 0, 0, False
+        return 0, 0, 0
+    for rows in (8, 16, 24, 32, 40, 48, 64):
+        if ceil_div(n, rows) <= num_cus and (rows <= 32 or m <= 32):
+            return (rows + m) * k_bytes, rows, ceil_div(n, rows)
+    return 0, 0, 0
 
 
 @functools.lru_cache(maxsize=None)
@@ -202,35 +201,54 @@ def get_weight_stream_fp8_config(m: int, n: int, k: int, num_cus: int) -> int:
 
     Its time is 3.3 us + what a workgroup pulls at about 62 bytes/ns, or the weights at 6 to 7 TB/s; a split-K plan
     pays 2 us for the meeting of the parts, the tiles of a short K too few workgroups. Measured per call, weights cycling through
-    more matrices than the caches hold, 49 shapes of n = 128 .. 16384, k = 512 .. 16384, up to ten m each (split-K plan or tiles -> this
+    more matrices than the caches hold, 60 shapes of n = 128 .. 16384, k = 512 .. 16384, up to ten m each (split-K plan or tiles -> this
     kernel): 1 x 2112 x 7168 8.7 -> 5.4 us, 1 x 4096 x 7168 9.8 -> 7.6, 16 x 1984 x 4608 6.7 -> 4.5, 32 x 2944 x 5632 10.3 -> 7.8,
-    40 x 4096 x 16384 22.3 -> 19.8, 8 x 10240 x 7168 22.3 -> 16.8, 32 x 16384 x 16384 53.8 -> 47.5. Up to 40 rows it loses only where a workgroup pulls more than 400 KB and the chip is not full
-    (20 x 1472 x 15104 10.9 -> 11.3; 40 x 4100 x 16384, 129 workgroups, 21.1 -> 24.8, though with 32 rows it still wins, 23.9 ->
-    21.9); with 48 rows it is level from 300 KB on (4096 x 7168 11.1 -> 11.3), with
-    64 from 130 KB on (4096 x 2048 4.7 -> 4.8; 3072 x 1536 4.5 -> 4.2; 2112 x 7168 10.3 -> 12.2). Same rule as
-    `weight_stream_fp8_atoms` in yan_amd/csrc/yan_gemm_capi.hip."""
-    pull, _, full = _weight_stream_pull(m, n, k, num_cus)
-    if pull and (pull <= 130_000 or (m <= 48 and pull <= 300_000) or (m <= 40 and (pull <= 400_000 or full)) or (m <= 32 and n >= 16 * num_cus)):
-        return ceil_div(m, 16)
-    return 0
+    40 x 4096 x 16384 22.3 -> 19.8, 8 x 10240 x 7168 22.5 -> 15.0, 32 x 16384 x 16384 53.8 -> 47.5. It loses
+    up to 40 rows only where a workgroup of 8 or 16 weight rows pulls more than 400 KB and they do not fill the chip
+    (20 x 1472 x 15104 10.9 -> 11.3); with 48 rows it is level from 300 KB on (4096 x 7168 11.1 -> 11.3), 400 KB on more weight rows
+    (4100 x 7168 12.2 at 516 KB both ways, but 8192 x 4096 11.1 -> 10.1); with 64 from 130 KB on (4096 x 2048 4.7 -> 4.8;
+    3072 x 1536 4.5 -> 4.2; 2112 x 7168 10.3 -> 12.2; 7168 x 2048 7.1 both ways), on 24 weight rows 365 KB (4224 x 4096
+    10.5 -> 9.5; 5120 x 8192 14.2 -> 16.2 at 721 KB). Same rule as `weight_stream_fp8_atoms` in yan_amd/csrc/yan_gemm_capi.hip."""
+    pull, rows, groups = _weight_stream_pull(m, n, k, num_cus)
+    full, wide = rows >= 16 and groups * 8 >= num_cus * 7, rows >= 24
+    if not pull:
+        return 0
+    if m <= 32:
+        takes = pull <= 400_000 or full or n >= 16 * num_cus
+    elif m <= 40:
+        takes = pull <= 400_000 or full or wide
+    elif m <= 48:
+        takes = pull <= (400_000 if wide else 300_000) or (rows == 32 and full)
+    else:
+        takes = pull <= (365_000 if rows == 24 else 130_000)
+    return ceil_div(m, 16) if takes else 0
 
 
 @functools.lru_cache(maxsize=None)
 def get_weight_stream_dense_config(m: int, n: int, k: int, num_cus: int) -> int:
-    """The same for the dense 16-bit GEMM, whose smallest tile holds 64 weight rows. While a workgroup pulls at most 450 KB, or where
-    they fill the chip 580 KB on 16 weight rows and 800 KB on 32 (64 x 4096 x 2048 10.2 -> 8.2 us, 40 x 1984 x 4608 10.8 -> 10.3 at 442 KB,
-    48 x 1984 x 4608 11.1 -> 11.0 at 516 KB, 32 x 1024 x 7168 11.1 -> 11.7 at 573 KB, 24 x 4224 x 4096 11.5 -> 11.6 at 459 KB;
-    24 x 4096 x 7168 15.9 -> 15.2 at 573 KB, 32 x 4096 x 7168 16.2 -> 16.4 at 688 KB; 64 x 8192 x 4096 19.7 -> 18.8 at 786 KB,
-    32 x 8192 x 7168 24.0 -> 24.6 at 917 KB), 600 KB on 64 (8 x 9216 x 4096 20.0 -> 16.9, 32 x 11008 x 3072 17.5 -> 17.3, both 590 KB;
-    12 x 16384 x 4096 27.2 -> 28.1 at 623 KB). Up to 16 rows on any K (1 x 1024 x 7168
-    12.7 -> 5.5, 16 x 1472 x 15104 31.1 -> 16.7, 16 x 2112 x 7168 11.5 -> 11.6, the closest), except on 32 or 64 weight rows that leave
-    much of the chip idle (16 x 4100 x 16384 30.2 -> 33.3, 8 x 4100 x 7168 15.8 -> 15.4 at 573 KB). Same rule as
-    `weight_stream_dense_atoms` in yan_amd/csrc/yan_gemm_capi.hip."""
-    pull, rows, full = _weight_stream_pull(m, n, 2 * k, num_cus)
-    limit = 600_000 if rows == 64 else (800_000 if rows == 32 else 580_000) if full else 580_000 if m <= 16 else 450_000
-    if pull and (pull <= limit or (m <= 16 and (full or n <= 16 * num_cus))):
-        return ceil_div(m, 16)
-    return 0
+    """The same for the dense 16-bit GEMM, whose smallest tile holds 64 weight rows: while a workgroup pulls no more than a limit that
+    depends on its weight rows and on how much of the chip they fill. 8 and 16 weight rows: 450 KB (40 x 1984 x 4608 10.8 -> 10.3 us at
+    442 KB, 48 rows 11.1 -> 11.0 at 516 KB, 32 x 1024 x 7168 11.1 -> 11.7 at 573 KB), 580 KB where they fill the chip (24 x 4096 x 7168
+    15.9 -> 15.2 at 573 KB, 32 rows 16.2 -> 16.4 at 688 KB). 24: 510 KB for two thirds of the chip up to 850 KB (40 x 4224 x 4096 12.0 -> 12.1 at
+    524 KB, 24 x 4100 x 7168 16.7 -> 16.5 at 688 KB, 32 x 5120 x 8192 21.5 -> 19.5 at 918 KB, 40 rows 21.6 -> 21.4). 32: 600 KB, full
+    780 KB (64 x 8192 x 4096 19.7 -> 18.8 at 786 KB, 24 x 7168 x 7168 22.2 -> 22.1 at 860 KB, 32 x 8192 x 7168 24.0 -> 24.6 at 917 KB). 40, 48:
+    1.4 MB (32 x 10240 x 7168 33.3 -> 28.2, 32 x 12288 x 8192 36.5 -> 36.0, 1 x 8256 x 16384 49.2 -> 46.9; 24 rows there 48.4 both ways).
+    64: 600 KB (32 x 14336 x 2048 15.4 -> 13.0; 12 x 16384 x 4096 27.2 -> 28.1 at 623 KB). Up to 16 rows also beyond: 24 weight rows
+    1.4 MB (16 x 4100 x 16384 30.7 -> 28.3), 8, 16 and 32 on any K (1 x 1024 x 7168 12.7 -> 5.5, 16 x 1472 x 15104 31.1 -> 16.7,
+    16 x 2112 x 7168 11.5 -> 11.6, the closest). Same rule as `weight_stream_dense_atoms` in yan_amd/csrc/yan_gemm_capi.hip."""
+    pull, rows, groups = _weight_stream_pull(m, n, 2 * k, num_cus)
+    full = groups * 8 >= num_cus * 7
+    if not pull:
+        return 0
+    if rows <= 16:
+        limit = 580_000 if rows == 16 and full else 450_000
+    elif rows == 24:
+        limit = 1_400_000 if m <= 16 else min(850_000, 3_000_000 * groups // num_cus - 1_490_000)
+    elif rows == 32:
+        limit = 780_000 if full else 600_000
+    else:
+        limit = 600_000 if rows == 64 else 1_400_000
+    return ceil_div(m, 16) if pull <= limit or (m <= 16 and rows in (8, 16, 32)) else 0
 
 
 def get_dense_tile(m: int, n: int, k: int, num_cus: int) -> Tuple[int, int]:
