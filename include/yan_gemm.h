@@ -171,7 +171,8 @@ YAN_API int yan_per_block_cast_to_fp8(const void* w, int w_is_fp32, void* q, flo
  * tiles and places them along the groups on the device, from m_indices (groups of 128 rows or more on average), at a depth of 1024;
  * 0 x 0 when it runs the tile op 2 names. For groups of 128 to 255 rows the answer depends on the depth.
  * op 5: the same for the depth `k`, with the number of groups in *block_m when it is called.
- * For ops 0 and 1 with few activation rows the answer is (16 * atoms, 16): the weight-streaming kernels.
+ * For ops 0 and 1 with few activation rows the answer can be (16 * atoms, 16): the weight-streaming kernel. From 17 rows on it then runs
+ * in place of a split-K plan too; up to 16 rows a plan goes first where a workgroup would pull much (a long K).
  * Host-only (no device call). Stands where the reference leaves tile choice to the caller's keys
  * (yan/jit_kernels/cute_gemm.py:41, yan/jit_kernels/gemm.py:13-16). Returns 0, or 1 for an unknown op. */
 YAN_API int yan_gemm_select_tile(int op, int m, int n, int k, int num_cus, int* block_m, int* block_n);

@@ -225,13 +225,12 @@ DENSE_LINE_WINDOW_TILES = [((128, 256), 3), ((128, 192), 4), ((128, 128), 5), ((
 DENSE_LINE_WINDOW_SHAPES = [(131, 260, 264, 0, 0), (70, 132, 312, 8, 40), (257, 388, 328, 56, 0), (64, 68, 424, 24, 24), (130, 516, 1016, 48, 8)]
 
 
-# The weight-streaming kernel through the entry points: every number of activation atoms on 8, 16, 24, 32, 40, 48 and 64 weight rows per workgroup (24, 40 and
-# 48 lie across two blocks of 128 weight rows in places),
-# m and n off the tiles, fewer K blocks than waves, one more than a whole round of the waves and of their slots.
+# The weight-streaming kernel through the entry points: every number of activation atoms on 8, 16, 24, 32, 40, 48 and 64 weight rows per
+# workgroup (24, 40 and 48 lie across two blocks of 128 weight rows in places), m and n off the tiles, fewer K blocks than waves, one more
+# than a whole round of the waves and of their slots.
 WEIGHT_STREAM_SHAPES = [(1, 196, 128), (8, 2044, 1152), (9, 2052, 4224), (16, 4100, 640), (17, 100, 4224), (32, 4096, 512), (33, 2052, 1152),
-                        (48, 4100, 512), (64, 196, 1024), (64, 4100, 1152),
-                        (40, 6148, 640),
-                        (7, 8260, 1152), (25, 8196, 1152), (16, 10252, 640), (31, 12284, 256), (16, 12300, 640), (32, 16384, 256)]
+                        (48, 4100, 512), (64, 196, 1024), (64, 4100, 1152), (40, 6148, 640), (7, 8260, 1152), (25, 8196, 1152), (16, 10252, 640),
+                        (31, 12284, 256), (16, 12300, 640), (32, 16384, 256)]
 
 
 # fp32 on the bf16 matrix cores: (tile, parts, (m, n, k)) built through explicit keys. Ragged tiles on both sides, K around the 16 rows of an
