@@ -233,6 +233,12 @@ WEIGHT_STREAM_SHAPES = [(1, 196, 128), (8, 2044, 1152), (9, 2052, 4224), (16, 41
                         (31, 12284, 256), (16, 12300, 640), (32, 16384, 256)]
 
 
+# bf16 activations quantised by the weight-streaming kernel: 1, 2, 4 and 8 rows of it and fewer than those, waves without a K block, groups that
+# do not fill a step, the most steps.
+CAST_STREAM_SHAPES = [(1, 196, 128), (1, 516, 16384), (1, 2112, 7168), (2, 2052, 1152), (2, 4100, 16384), (3, 100, 640), (4, 5120, 8192), (5, 8260, 1152),
+                      (8, 16384, 2048), (7, 1984, 2048)]
+
+
 # fp32 on the bf16 matrix cores: (tile, parts, (m, n, k)) built through explicit keys. Ragged tiles on both sides, K around the 16 rows of an
 # MFMA and the k-tiles of 16, 32 and 64 rows, fewer k-tiles than stages, parts of unequal length and parts without any
 FLOAT_BF16X3_CASES = [((256, 256), 1, (300, 260, 1)), ((256, 256), 1, (256, 516, 95)), ((256, 256), 3, (260, 256, 145)),
@@ -649,6 +655,11 @@ def jit_kernels_in_use(num_cus: int = 256):
         for dtype in (torch.bfloat16, torch.half):
             name, keys, arg_defs, includes, code_template = dense_tile_plan(tile, dtype, 0)
             add(name, arg_defs, includes, code_template, keys)
+    for m, n, k in CAST_STREAM_SHAPES:
+        name, keys, arg_defs, code_template = gemm.fp8_cast_stream_plan(m, n, k, num_cus)
+        add(name, arg_defs, gemm.includes, code_template, keys)
+        name, keys, arg_defs, _, code_template = gemm.fp8_kernel_plan(m, n, k, num_cus)
+        add(name, arg_defs, gemm.includes, code_template, keys)
     for m, n, k in WEIGHT_STREAM_SHAPES:
         for token_contiguous in (True, False):
             name, keys, arg_defs, _, code_template = gemm.fp8_kernel_plan(m, n, k, num_cus, token_contiguous)

@@ -364,6 +364,28 @@ def test_weight_streaming_kernel_at_the_edges_of_its_tiles(m, n, k):
               torch.bfloat16, 2.0 ** -23)
 
 
+@pytest.mark.parametrize('m,n,k', testing.CAST_STREAM_SHAPES)
+def test_activations_quantised_by_the_weight_streaming_kernel(m, n, k):
+    """The bits of the quantiser and the FP8 entry one after the other, for ordinary rows, a row of zeros, an outlier, infinities and NaN; the
+    rows behind the output stay untouched."""
+    from yan_amd.jit_kernels import gemm as fp8_entry
+    _announce('cast and weight streaming', m, n, k)
+    assert fp8_entry.fp8_cast_stream_plan(m, n, k, yan.get_num_sms()) is not None
+    g = torch.Generator().manual_seed(37)
+    x = torch.randn(m, k, generator=g)
+    x[0, 3], x[m // 2, k // 2:k // 2 + 64], x[m - 1, -1] = 3e4, 0.0, -2e-5
+    w = yan.per_block_cast_to_fp8((torch.randn(n, k, generator=g) * k ** -0.5).bfloat16().cuda())
+    for odd in (None, float('inf'), float('nan')):
+        if odd is not None:
+            x[m - 1, 7] = odd
+        xd = x.bfloat16().cuda()
+        two, one = (torch.full((m + 2, n), 7.0, dtype=torch.bfloat16, device='cuda') for _ in range(2))
+        yan.gemm_fp8_fp8_bf16_nt(yan.per_token_cast_to_fp8(xd, col_major_scales=True), w, two[:m])
+        yan.gemm_bf16_fp8_bf16_nt(xd, w, one[:m])
+        assert bool((one[m:] == 7.0).all())
+        assert torch.equal(one.isnan(), two.isnan()) and torch.equal(one.nan_to_num(), two.nan_to_num())
+
+
 def _run_float_bf16x3(tile, parts, a, b, c, alpha=1.0, beta=0.0):
     from yan_amd.jit_kernels import simple_gemm, split_k
     name, keys, arg_defs = testing.float_bf16x3_explicit_plan(tile, parts)

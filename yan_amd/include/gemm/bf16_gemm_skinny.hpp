@@ -23,7 +23,7 @@ template <typename Atom, typename Elem, int TM>
 inline hipError_t launch_dense_skinny(int m, int n, int k, const void* a, const void* b, void* c, hipStream_t stream, int num_sms = 0) {
     if (m == 0 || n == 0) return hipSuccess;
     if (!dense_skinny_fits(m, n, k, TM) || !a || !b || !c) return hipErrorInvalidValue;
-    if (!launch_weight_stream<Atom, Elem, 0, 0, TM, false>(a, nullptr, 0, 0, b, nullptr, c, m, n, k * 2, num_sms, stream)) return hipErrorInvalidValue;
+    if (!launch_weight_stream<Atom, Elem, 0, 0, TM, kDense>(a, nullptr, 0, 0, b, nullptr, c, m, n, k * 2, num_sms, stream)) return hipErrorInvalidValue;
     return hipGetLastError();
 }
 

@@ -20,8 +20,21 @@ inline hipError_t launch_fp8_skinny(__hip_bfloat16* out, const void* lhs, const 
     if (m < 0 || m > 16 * TM || n < 0 || k <= 0 || (n % 4) != 0 || (k % 128) != 0) return hipErrorInvalidValue;
     if ((SHAPE_N && n != SHAPE_N) || (SHAPE_K && k != SHAPE_K)) return hipErrorInvalidValue;
     if (!out || !lhs || !lhs_scales || !rhs || !rhs_scales) return hipErrorInvalidValue;
-    if (!launch_weight_stream<MfmaFP8_16x16x128, __bf16, SHAPE_N, SHAPE_K, TM, true>(lhs, lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k, rhs,
+    if (!launch_weight_stream<MfmaFP8_16x16x128, __bf16, SHAPE_N, SHAPE_K, TM, kScaled>(lhs, lhs_scales, lhs_scales_stride_m, lhs_scales_stride_k, rhs,
                                                                                    rhs_scales, out, m, n, k, num_sms, stream)) return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+// bf16 activations, quantised as launch_per_token_cast does it in every workgroup: A_ROWS is cast_rows(m, k / 128).
+template <int SHAPE_N, int SHAPE_K, int A_ROWS>
+inline hipError_t launch_fp8_skinny_cast(__hip_bfloat16* out, const void* x, const void* rhs, const float* rhs_scales, int m, int n, int k,
+                                         hipStream_t stream, int num_sms = 0) {
+    if (m == 0 || n == 0) return hipSuccess;
+    if (m < 0 || n < 0 || k <= 0 || cast_rows(m, k / 128) != A_ROWS || (n % 4) != 0 || (k % 128) != 0) return hipErrorInvalidValue;
+    if ((SHAPE_N && n != SHAPE_N) || (SHAPE_K && k != SHAPE_K)) return hipErrorInvalidValue;
+    if (!out || !x || !rhs || !rhs_scales) return hipErrorInvalidValue;
+    if (!launch_weight_stream<MfmaFP8_16x16x128, __bf16, SHAPE_N, SHAPE_K, 1, kCast, A_ROWS>(x, nullptr, 0, 0, rhs, rhs_scales, out, m, n, k, num_sms,
+                                                                                           stream)) return hipErrorInvalidValue;
     return hipGetLastError();
 }
 

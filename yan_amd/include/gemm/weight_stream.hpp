@@ -19,17 +19,32 @@
 #include "utils.hpp"
 #include "mfma_utils.hpp"
 #include "tile_io.hpp"
+#include "fp8_cast.hpp"
 
 namespace yan {
 
 // ROWS weight rows and A_ROWS activation rows per workgroup; a slot holds one K block of both and, with SCALES, a float per row.
-template <int ROWS, int A_ROWS, bool SCALES>
+// OPERANDS: kDense (16-bit), kScaled (FP8 with scales), or kCast, FP8 weights with bf16 activations: a wave quantises the K blocks it owns
+// of all of them first, while its first weights are on the way (up to kCastSteps times 4 groups of 128 numbers, 1 KB of LDS each).
+// Every workgroup repeats that, bound by vector arithmetic of about 0.3 us a step, where a launch of the quantiser costs 2.5 to 3 us:
+// 1 x 2112 x 7168 7.9 -> 6.0 us call to call, 4 x 5120 x 8192 11.6 -> 10.9. Quantising a block right in front of its MFMA instead put 0.4 us
+// per block into the waves' chain (2112 x 7168 8.0).
+enum StreamOperands { kDense, kScaled, kCast };
+constexpr int kCastSteps = 8;
+// Activation rows a workgroup of kCast works with for m rows and that many K blocks, or 0 when a wave's share does not fit.
+__host__ __device__ constexpr int cast_rows(int m, int num_k_blocks) {
+    const int rows = m <= 1 ? 1 : m <= 2 ? 2 : m <= 4 ? 4 : 8;
+    return m >= 1 && m <= 8 && ceil_div(num_k_blocks, 8) * rows <= 4 * kCastSteps ? rows : 0;
+}
+template <int ROWS, int A_ROWS, StreamOperands OPERANDS>
 struct WeightStreamShape {
-    static_assert(ROWS % 8 == 0 && (A_ROWS == 8 || A_ROWS % 16 == 0) && A_ROWS <= kWaveSize);
+    static constexpr bool SCALES = OPERANDS != kDense, CAST = OPERANDS == kCast;
+    static_assert(ROWS % 8 == 0 && (A_ROWS == 8 || A_ROWS % 16 == 0 || CAST) && A_ROWS <= (CAST ? 8 : kWaveSize));
     static constexpr int NUM_WAVES = 8;
-    static constexpr int LOADS = ROWS / 8 + A_ROWS / 8 + (SCALES ? 1 : 0);
-    static constexpr int SLOT  = (ROWS + A_ROWS) * kRowBytes + (SCALES ? kWaveSize * 4 : 0);
-    static constexpr int FIT   = 152 * 1024 / (SLOT * NUM_WAVES);
+    static constexpr int LOADS = ROWS / 8 + (CAST ? 0 : A_ROWS / 8 + (SCALES ? 1 : 0));
+    static constexpr int SLOT  = ROWS * kRowBytes + (CAST ? 0 : A_ROWS * kRowBytes + (SCALES ? kWaveSize * 4 : 0));
+    static constexpr int CODES = CAST ? kCastSteps * 1024 : 0;         // of a wave
+    static constexpr int FIT   = (152 * 1024 / NUM_WAVES - CODES) / SLOT;
     static constexpr int DEPTH = FIT < 4 ? FIT : 4;         // 3 to 5 measure alike; 8 is slower on a row (more copies in front of the first sum)
     static constexpr int ATOMS = ceil_div(A_ROWS, 16), B_ATOMS = ceil_div(ROWS, 16);
     static constexpr bool TWO_SCALES = SCALES && 128 % ROWS != 0;       // a tile can lie in two blocks of 128 weight rows
@@ -48,30 +63,32 @@ __device__ __forceinline__ void wait_for_block(int later) {
 
 // SCALES: FP8 operands with a scale per row and K block of the activations and per 128 weight rows and K block; else 16-bit ones.
 // SHAPE_N, SHAPE_K_BYTES: the sizes when known at compile time, or 0.
-template <typename Atom, typename Out, int SHAPE_N, int SHAPE_K_BYTES, int ROWS, int A_ROWS, bool SCALES>
+template <typename Atom, typename Out, int SHAPE_N, int SHAPE_K_BYTES, int ROWS, int A_ROWS, StreamOperands OPERANDS>
 __global__ void __launch_bounds__(8 * kWaveSize)
 weight_stream_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ lhs_scales, const uint8_t* __restrict__ rhs,
                      const float* __restrict__ rhs_scales, Out* __restrict__ out, int m, int n_rt, int k_bytes_rt, int sa_stride_m, int sa_stride_k) {
-    using Shape = WeightStreamShape<ROWS, A_ROWS, SCALES>;
+    using Shape = WeightStreamShape<ROWS, A_ROWS, OPERANDS>;
+    constexpr bool SCALES = Shape::SCALES, CAST = Shape::CAST;
     constexpr int NUM_WAVES = Shape::NUM_WAVES, DEPTH = Shape::DEPTH, SLOT = Shape::SLOT, ATOMS = Shape::ATOMS, B_ATOMS = Shape::B_ATOMS;
     constexpr int A_AT = ROWS * kRowBytes, SCALES_AT = (ROWS + A_ROWS) * kRowBytes;         // within a slot
     const int n = SHAPE_N ? SHAPE_N : n_rt, k_bytes = SHAPE_K_BYTES ? SHAPE_K_BYTES : k_bytes_rt;
     const int num_k_blocks = k_bytes / kRowBytes;
 
-    __shared__ __attribute__((aligned(1024))) uint8_t slots[NUM_WAVES * DEPTH * SLOT];
+    __shared__ __attribute__((aligned(1024))) uint8_t slots[NUM_WAVES * (DEPTH * SLOT + Shape::CODES)];
 
     const int n0 = blockIdx.x * ROWS;
     const int lane = get_lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
     const int g = lane / 16, col = lane % 16, sub = lane / 8;
 
-    const __amdgpu_buffer_rsrc_t rsrc_a = make_rsrc(lhs, uint32_t(m) * k_bytes);
+    const int a_pitch = CAST ? 2 * k_bytes : k_bytes;
+    const __amdgpu_buffer_rsrc_t rsrc_a = make_rsrc(lhs, uint32_t(m) * a_pitch);
     const __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(rhs, uint32_t(n) * k_bytes);
     __amdgpu_buffer_rsrc_t rsrc_sa = rsrc_a;
     const float* sb_row = nullptr, *sb_next = nullptr;
     bool in_next[B_ATOMS];          // this lane's four sums of an atom are in the second block of 128 rows (it starts at a multiple of 8)
     if constexpr (SCALES) {
-        rsrc_sa = make_rsrc(lhs_scales, (uint32_t(m - 1) * sa_stride_m + uint32_t(num_k_blocks - 1) * sa_stride_k + 1) * 4);
+        if constexpr (!CAST) rsrc_sa = make_rsrc(lhs_scales, (uint32_t(m - 1) * sa_stride_m + uint32_t(num_k_blocks - 1) * sa_stride_k + 1) * 4);
         sb_row = rhs_scales + size_t(n0 / 128) * num_k_blocks;
         sb_next = rhs_scales + size_t(min(n0 / 128 + 1, ceil_div(n, 128) - 1)) * num_k_blocks;
 #pragma unroll
@@ -86,6 +103,7 @@ weight_stream_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ 
     auto rotated = [&](int kb) { const int r = kb + rot; return r >= num_k_blocks ? r - num_k_blocks : r; };
 
     uint8_t* const own = slots + wave * (DEPTH * SLOT);
+    [[maybe_unused]] uint8_t* const codes = slots + NUM_WAVES * (DEPTH * SLOT) + wave * Shape::CODES;
     auto issue = [&](int block, int slot) {
         const int kb = rotated(block);
         uint8_t* const to = own + slot * SLOT;
@@ -93,6 +111,7 @@ weight_stream_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ 
         for (int p = 0; p < ROWS / 8; ++p)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, YAN_LDS_PTR(to + p * 8 * kRowBytes), kChunk, voff_b + (chunk ^ (p & 1) * kChunk),
                                                      kb * kRowBytes + p * 8 * k_bytes, 0, 0);
+        if constexpr (CAST) return;
 #pragma unroll
         for (int p = 0; p < A_ROWS / 8; ++p)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, YAN_LDS_PTR(to + A_AT + p * 8 * kRowBytes), kChunk, voff_a + (chunk ^ (p & 1) * kChunk),
@@ -102,7 +121,7 @@ weight_stream_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ 
 
     // Lane (col, g) holds chunks 2g and 2g + 1 of row `col` of an atom. Half an atom of 8 rows is read twice, its second sums go nowhere.
     auto offset = [&](int row, int c) { return row * kRowBytes + ((c ^ swizzle_of_row(row)) * kChunk); };
-    const int row_a = A_ROWS == 8 ? col & 7 : col;
+    const int row_a = A_ROWS < 16 ? col & (A_ROWS - 1) : col;
     const int b_lo = offset(col, 2 * g), b_hi = offset(col, 2 * g + 1), a_lo = A_AT + offset(row_a, 2 * g), a_hi = A_AT + offset(row_a, 2 * g + 1);
     const int half_lo = offset(col & 7, 2 * g), half_hi = offset(col & 7, 2 * g + 1);
 
@@ -112,9 +131,35 @@ weight_stream_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ 
 #pragma unroll
         for (int j = 0; j < ATOMS; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+    // kCast: group q of a wave is row q % A_ROWS of its block q / A_ROWS; a step is four groups, 16 lanes and 256 bytes of bf16 each
+    [[maybe_unused]] const int own_blocks = wave < num_k_blocks ? (num_k_blocks - 1 - wave) / NUM_WAVES + 1 : 0;
+    [[maybe_unused]] const int steps = ceil_div(own_blocks * A_ROWS, 4);
+    if constexpr (CAST) {
+        for (int t = 0; t < steps; ++t) {
+            const int q = 4 * t + g, row = q % A_ROWS, kb = rotated(min(wave + q / A_ROWS * NUM_WAVES, num_k_blocks - 1));
+            const uint32_t from = row < m ? uint32_t(row) * a_pitch + uint32_t(kb) * (2 * kRowBytes) + col * kChunk : kOutOfRange;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, YAN_LDS_PTR(codes + t * 1024), kChunk, from, 0, 0, 0);
+        }
+    }
 #pragma unroll
     for (int s = 0; s < DEPTH; ++s)
         if (wave + s * NUM_WAVES < num_k_blocks) issue(wave + s * NUM_WAVES, s);
+    // The codes of a step and, behind them, its scales take the place of its bf16 numbers; arithmetic of per_token_cast_kernel.
+    auto code_at = [&](int q, int c) { return q / 4 * 1024 + q % 4 * kRowBytes + ((c ^ (q % 4)) * kChunk); };
+    auto scale_at = [&](int q) { return q / 4 * 1024 + 4 * kRowBytes + q % 4 * 4; };
+    if constexpr (CAST) {
+        wait_for_block<Shape::LOADS, DEPTH>(min(own_blocks, DEPTH));
+#pragma unroll 2
+        for (int t = 0; t < steps; ++t) {
+            Raw8<__hip_bfloat16> x;
+            x.w[0] = *reinterpret_cast<const i32x4*>(codes + t * 1024 + lane * kChunk);
+            const F32x8 f = to_f32(x);
+            const float amax = fmaxf(max_over_16_lanes(abs_max8(f)), 1e-4f);
+            const uint2 packed = quantise8(f, kFp8Max / amax);
+            *reinterpret_cast<uint2*>(codes + code_at(4 * t + g, col / 2) + col % 2 * 8) = packed;
+            if (col == 0) *reinterpret_cast<float*>(codes + scale_at(4 * t + g)) = amax / kFp8Max;
+        }
+    }
     for (int first = wave; first < num_k_blocks; first += DEPTH * NUM_WAVES) {
 #pragma unroll
         for (int s = 0; s < DEPTH; ++s) {
@@ -135,9 +180,16 @@ weight_stream_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ 
             }
 #pragma unroll
             for (int j = 0; j < ATOMS; ++j) {
-                a[j][0] = *reinterpret_cast<const i32x4*>(from + a_lo + j * 16 * kRowBytes);
-                a[j][1] = *reinterpret_cast<const i32x4*>(from + a_hi + j * 16 * kRowBytes);
-                if constexpr (SCALES) scale[j] = *reinterpret_cast<const float*>(from + SCALES_AT + (j * 16 + col) * 4);
+                if constexpr (CAST) {
+                    const int q = (block / NUM_WAVES) * A_ROWS + row_a;
+                    a[j][0] = *reinterpret_cast<const i32x4*>(codes + code_at(q, 2 * g));
+                    a[j][1] = *reinterpret_cast<const i32x4*>(codes + code_at(q, 2 * g + 1));
+                    scale[j] = *reinterpret_cast<const float*>(codes + scale_at(q));
+                } else {
+                    a[j][0] = *reinterpret_cast<const i32x4*>(from + a_lo + j * 16 * kRowBytes);
+                    a[j][1] = *reinterpret_cast<const i32x4*>(from + a_hi + j * 16 * kRowBytes);
+                    if constexpr (SCALES) scale[j] = *reinterpret_cast<const float*>(from + SCALES_AT + (j * 16 + col) * 4);
+                }
             }
             // the slot is read: its next block may come
             __builtin_amdgcn_s_waitcnt(waitcnt_imm(kNoWaitVm, 0));
@@ -184,13 +236,13 @@ weight_stream_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ 
 // 4096 x 7168 7.0 us (8: 7.4); 24 for 8 x 4100 x 16384 14.0 (32: 15.6); 32 for 32 x 7168 x 2048 in bf16 8.0 us (16, two rounds: 10.2). Beyond that
 // up to 32 activation rows (one sum per wave): 40 for 32 x 8200 x 8192 15.3 (48: 16.3; 64: 19.8; tiles: 25.7), 48 for 32 x 12288 x 2048 7.3
 // (64: 7.9; tiles: 10.0), then 64: with 56 HBM-bound shapes lose (13000 x 16384 bf16 70.5 -> 74.2). False when a 32-bit offset does not reach.
-template <typename Atom, typename Out, int SHAPE_N, int SHAPE_K_BYTES, int TM, bool SCALES>
+template <typename Atom, typename Out, int SHAPE_N, int SHAPE_K_BYTES, int TM, StreamOperands OPERANDS, int CAST_ROWS = 0>
 inline bool launch_weight_stream(const void* lhs, const float* lhs_scales, int sa_stride_m, int sa_stride_k, const void* rhs, const float* rhs_scales,
                                  void* out, int m, int n, int k_bytes, int num_sms, hipStream_t stream) {
-    if (uint64_t(16 * TM) * k_bytes >= kOutOfRange || (uint64_t(n) + 64) * k_bytes >= kOutOfRange) return false;
+    if (uint64_t(16 * TM) * k_bytes * (OPERANDS == kCast ? 2 : 1) >= kOutOfRange || (uint64_t(n) + 64) * k_bytes >= kOutOfRange) return false;
     const int cus = num_sms > 0 && num_sms < device_cu_count() ? num_sms : device_cu_count();
     auto launch = [&]<int ROWS, int A_ROWS>() {
-        hipLaunchKernelGGL((weight_stream_kernel<Atom, Out, SHAPE_N, SHAPE_K_BYTES, ROWS, A_ROWS, SCALES>), dim3(ceil_div(n, ROWS)), dim3(8 * kWaveSize), 0,
+        hipLaunchKernelGGL((weight_stream_kernel<Atom, Out, SHAPE_N, SHAPE_K_BYTES, ROWS, A_ROWS, OPERANDS>), dim3(ceil_div(n, ROWS)), dim3(8 * kWaveSize), 0,
                            stream, static_cast<const uint8_t*>(lhs), lhs_scales, static_cast<const uint8_t*>(rhs), rhs_scales,
                            static_cast<Out*>(out), m, n, k_bytes, sa_stride_m, sa_stride_k);
     };
@@ -205,7 +257,8 @@ inline bool launch_weight_stream(const void* lhs, const float* lhs_scales, int s
             else launch.template operator()<64, A_ROWS>();
         }
     };
-    if constexpr (TM == 1) {
+    if constexpr (OPERANDS == kCast) rows.template operator()<CAST_ROWS>();
+    else if constexpr (TM == 1) {
         if (m <= 8) rows.template operator()<8>();
         else rows.template operator()<16>();
     } else rows.template operator()<16 * TM>();

@@ -17,7 +17,7 @@ import torch
 
 from .fp8_cast import per_token_cast_to_fp8
 from .heuristics import (get_best_fp8_config, get_fp8_num_stages, get_fp8_tile_space, get_skinny_fp8_config,
-                         get_split_k_fp8_config, get_weight_stream_fp8_config, tuning_enabled)
+                         get_split_k_fp8_config, get_weight_stream_fp8_config, get_cast_stream_rows, tuning_enabled)
 from .host_calls import CAST_FP8, FP8, remember_call, repeat_call
 from .split_k import SPLIT_K_COUNTER_BYTES, SPLIT_K_WORKSPACE_BYTES, split_k_enabled, split_k_launch_failed, split_k_workspace
 from .tuner import FrozenKeys, jit_tuner
@@ -54,7 +54,7 @@ __return_code = static_cast<int>(GemmType::run(out, lhs, lhs_scales, lhs_scales_
                                                rhs, rhs_scales, m, stream, num_sms, smem_size, kTokenContiguous));
 """
 # Few activation rows: BLOCK_M / 16 activation atoms; BLOCK_N = 16 names the weight-streaming kernel, whose launch chooses the weight
-# rows of a workgroup by n, the m and the workgroups allowed (gemm/weight_stream.hpp).
+# rows of a workgroup by n and the workgroups allowed (gemm/weight_stream.hpp).
 _skinny_launch = """static_assert(BLOCK_N == 16 && BLOCK_M % 16 == 0);
 
 // Launch kernel
@@ -86,6 +86,19 @@ if (__return_code != 0) return;
 """
 _cast_arg_defs_head = (('x', torch.bfloat16), ('buffer', torch.uint8), ('scratch_bytes', int))
 cast_includes = includes + ('"gemm/fp8_cast.hpp"', )
+
+# A few rows of bf16 activations: the weight-streaming kernel quantises them itself, one launch and no scratch.
+_cast_stream_template = """
+using namespace yan;
+
+// Templated args from Python JIT call
+constexpr auto N = {N}, K = {K};
+
+// Launch kernel
+__return_code = static_cast<int>(launch_fp8_skinny_cast<N, K, {CAST_ROWS}>(out, x, rhs, rhs_scales, m, N, K, stream, num_sms));
+"""
+_cast_stream_arg_defs = (('x', torch.bfloat16), ('rhs', torch.float8_e4m3fn), ('rhs_scales', torch.float), ('out', torch.bfloat16), ('m', int),
+                         ('stream', torch.cuda.Stream), ('num_sms', int))
 
 # The reference's keys and run-time names, nothing else (yan/jit_kernels/gemm.py:9-30): code that formats this template
 # with `N, K, BLOCK_M, BLOCK_N, NUM_STAGES, NUM_TMA_MULTICAST` and builds it with `arg_defs` gets the kernel for
@@ -247,6 +260,16 @@ def fp8_cast_chain_plan(m: int, n: int, k: int, num_cus: int, split_k_allowed: b
     return 'gemm_bf16_fp8_bf16_nt', keys, _cast_arg_defs_head + inner, chained, smem_size
 
 
+@functools.lru_cache(maxsize=None)
+def fp8_cast_stream_plan(m: int, n: int, k: int, num_cus: int):
+    """(name, keys, arg_defs, template) of the kernel that quantises a few rows of bf16 activations and streams the weights in one launch, or
+    None when that is not what `gemm_bf16_fp8_bf16_nt` runs (`get_cast_stream_rows`); needs no GPU."""
+    rows = get_cast_stream_rows(m, n, k, num_cus)
+    if not rows:
+        return None
+    return 'gemm_bf16_fp8_bf16_nt_stream', FrozenKeys({'N': n, 'K': k, 'CAST_ROWS': rows}), _cast_stream_arg_defs, _cast_stream_template
+
+
 def gemm_bf16_fp8_bf16_nt(x: torch.Tensor, rhs: Tuple[torch.Tensor, torch.Tensor], out: torch.Tensor) -> None:
     """`gemm_fp8_fp8_bf16_nt(per_token_cast_to_fp8(x, col_major_scales=True), rhs, out)` for bf16 activations `x` `[m, k]`,
     bit for bit (the same two kernels), as ONE call: one trip through Python and one `launch`, which enqueues the quantiser and
@@ -257,7 +280,8 @@ def gemm_bf16_fp8_bf16_nt(x: torch.Tensor, rhs: Tuple[torch.Tensor, torch.Tensor
     out of the decode latency. Quantising inside the GEMM kernel itself was built and measured, and is slower than the two
     kernels: every one of the 64 workgroups that share a K range repeats the quantisation of its 64 x 1792 activations,
     9.6 us of vector arithmetic per workgroup against 2.5 us for the quantiser kernel spread over the chip (21.5 us in one
-    kernel against 3 + 9.7 us in two; same bits). Problems whose codes do not fit the scratch area (or with
+    kernel against 3 + 9.7 us in two; same bits); with up to 8 rows in front of the weight-streaming kernel it pays
+    (`fp8_cast_stream_plan`: one launch, no scratch). Problems whose codes do not fit the scratch area (or with
     `YAN_SPLIT_K=0`, which means no memory kept by the entries) run the two entries one after the other."""
     rhs_q, rhs_scales = rhs
     if repeat_call(CAST_FP8, x, rhs_q, rhs_scales, out):
@@ -271,7 +295,15 @@ def gemm_bf16_fp8_bf16_nt(x: torch.Tensor, rhs: Tuple[torch.Tensor, torch.Tensor
     if m == 0:
         return
     num_sms = get_num_sms()
-    plan = None
+    plan = None if tuning_enabled() else fp8_cast_stream_plan(m, n, k, num_sms)
+    if plan is not None:
+        name, keys, defs, code_template = plan
+        args = (x, rhs_q, rhs_scales, out, m, current_raw_stream(), num_sms)
+        runtime = jit_tuner.compile_and_tune(name=name, keys=keys, space=(), includes=includes, arg_defs=defs, template=code_template, args=args)
+        rc = runtime(*args)
+        assert rc == 0, f'{name} failed with HIP error {rc}'
+        remember_call((CAST_FP8, x, rhs_q, rhs_scales, out), runtime, args)
+        return
     if split_k_enabled() and not tuning_enabled():
         plan = fp8_cast_chain_plan(m, n, k, num_sms, split_k_allowed=not get_weight_stream_fp8_config(m, n, k, num_sms))
     if plan is None:

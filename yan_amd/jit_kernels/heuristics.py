@@ -251,6 +251,21 @@ def get_weight_stream_dense_config(m: int, n: int, k: int, num_cus: int) -> int:
     return ceil_div(m, 16) if pull <= limit or (m <= 16 and rows in (8, 16, 32)) else 0
 
 
+def get_cast_stream_rows(m: int, n: int, k: int, num_cus: int) -> int:
+    """Activation rows (1, 2, 4 or 8) the weight-streaming kernel quantises itself when it takes bf16 activations, else 0: problems it
+    takes with FP8 activations, up to 8 rows, whose quantising is shorter than the launch it saves. Every workgroup repeats it for
+    all rows, four groups of 128 numbers a step, the waves a share of K each while their first weights are on the way. Measured per call, weights
+    cycling, against quantiser and GEMM in two launches, same bits: 1 row: 2112 x 7168 7.9 -> 6.0 us, 1024 x 2048 6.0 -> 3.9, 5120 x 8192 11.6 -> 9.4,
+    9152 x 16000 29.3 -> 26.9; 4 rows: 7 steps, 2112 x 7168 8.2 -> 7.8, 16384 x 2048 9.8 -> 7.8; 2 rows x 1472 x 15104, 8 steps on 8 weight rows a
+    workgroup, 9.3 -> 9.5 (not taken); 8 rows: 4 steps, 7168 x 2048 7.6 -> 6.1, 8 steps, 3008 x 3328 6.3 -> 6.7 (not taken). `cast_rows` in
+    gemm/weight_stream.hpp names the rows."""
+    if not 0 < m <= 8 or not get_weight_stream_fp8_config(m, n, k, num_cus):
+        return 0
+    rows = 1 if m == 1 else 2 if m == 2 else 4 if m <= 4 else 8
+    steps = ceil_div(ceil_div(k // 128, 8) * rows, 4)
+    return rows if steps <= (4 if rows == 8 else 8 if n > 8 * num_cus else 7) else 0
+
+
 def get_dense_tile(m: int, n: int, k: int, num_cus: int) -> Tuple[int, int]:
     """(BLOCK_M, BLOCK_N) of the dense kernel that runs: (16 * atoms, 16) for the weight-streaming kernel."""
     atoms = get_weight_stream_dense_config(m, n, k, num_cus) or get_skinny_dense_config(m, n, k, num_cus)
