@@ -4,6 +4,7 @@ import ctypes
 import os
 import re
 import subprocess
+import sys
 
 import pytest
 
@@ -96,6 +97,23 @@ def test_weight_stream_choice_matches_python(lib):
                         assert atoms in (0, yan.ceil_div(m, 16))
                         assert not atoms or (m <= 64 and 16 <= n <= 64 * cus and n % 4 == 0 and row_bytes % 128 == 0 and (n + 64) * row_bytes < 1 << 31)
     assert taken > 500
+
+
+def test_weight_streaming_kernel_takes_operands_of_nearly_two_gib(repo_root):
+    """Up to 16 rows on at most 16 weight rows per compute unit the weight-streaming kernel runs whatever K is, up to where 16 rows behind the
+    matrix are out of reach. In a process that sees no device: a call whose sizes are accepted fails at the launch, not as invalid."""
+    code = """
+import ctypes
+from yan_amd import capi
+lib, p = capi.load(), ctypes.c_void_p(4096)
+for m, n, k in ((1, 4096, 259072), (16, 4096, 260096), (16, 4096, 261120), (1, 4096, 261184), (8, 2048, 520192), (9, 2048, 520256)):
+    print(lib.yan_gemm_bf16_tn(m, n, k, p, p, p, None), lib.yan_gemm_fp16_tn(m, n, k, p, p, p, None),
+          lib.yan_gemm_fp8_fp8_bf16_nt(p, p, 1, m, p, p, p, m, n, 2 * k, None, 0))
+"""
+    env = dict(os.environ, HIP_VISIBLE_DEVICES='-1', ROCR_VISIBLE_DEVICES='-1', PYTHONPATH=str(repo_root))
+    done = subprocess.run([sys.executable, '-c', code], stdout=subprocess.PIPE, universal_newlines=True, check=True, env=env)
+    refused = [[int(code) == 1 for code in line.split()] for line in done.stdout.splitlines()]
+    assert refused == [[False] * 3, [False] * 3, [False] * 3, [True] * 3, [False] * 3, [True] * 3]
 
 
 def test_compute_entry_points_validate_before_touching_a_device(lib):

@@ -239,30 +239,32 @@ weight_stream_kernel(const uint8_t* __restrict__ lhs, const float* __restrict__ 
 template <typename Atom, typename Out, int SHAPE_N, int SHAPE_K_BYTES, int TM, StreamOperands OPERANDS, int CAST_ROWS = 0>
 inline bool launch_weight_stream(const void* lhs, const float* lhs_scales, int sa_stride_m, int sa_stride_k, const void* rhs, const float* rhs_scales,
                                  void* out, int m, int n, int k_bytes, int num_sms, hipStream_t stream) {
-    if (uint64_t(16 * TM) * k_bytes * (OPERANDS == kCast ? 2 : 1) >= kOutOfRange || (uint64_t(n) + 64) * k_bytes >= kOutOfRange) return false;
+    if (uint64_t(16 * TM) * k_bytes * (OPERANDS == kCast ? 2 : 1) >= kOutOfRange) return false;
     const int cus = num_sms > 0 && num_sms < device_cu_count() ? num_sms : device_cu_count();
     auto launch = [&]<int ROWS, int A_ROWS>() {
+        // the last workgroup's rows lie up to ROWS - 1 behind the matrix
+        if ((uint64_t(n) + (ROWS < 16 ? 16 : ROWS)) * k_bytes >= kOutOfRange) return false;
         hipLaunchKernelGGL((weight_stream_kernel<Atom, Out, SHAPE_N, SHAPE_K_BYTES, ROWS, A_ROWS, OPERANDS>), dim3(ceil_div(n, ROWS)), dim3(8 * kWaveSize), 0,
                            stream, static_cast<const uint8_t*>(lhs), lhs_scales, static_cast<const uint8_t*>(rhs), rhs_scales,
                            static_cast<Out*>(out), m, n, k_bytes, sa_stride_m, sa_stride_k);
+        return true;
     };
     auto rows = [&]<int A_ROWS>() {
-        if (ceil_div(n, 8) <= cus) launch.template operator()<8, A_ROWS>();
-        else if (ceil_div(n, 16) <= cus) launch.template operator()<16, A_ROWS>();
-        else if (ceil_div(n, 24) <= cus) launch.template operator()<24, A_ROWS>();
-        else if (TM > 2 || ceil_div(n, 32) <= cus) launch.template operator()<32, A_ROWS>();
-        else if constexpr (TM <= 2) {
-            if (ceil_div(n, 40) <= cus) launch.template operator()<40, A_ROWS>();
-            else if (ceil_div(n, 48) <= cus) launch.template operator()<48, A_ROWS>();
-            else launch.template operator()<64, A_ROWS>();
+        if (ceil_div(n, 8) <= cus) return launch.template operator()<8, A_ROWS>();
+        if (ceil_div(n, 16) <= cus) return launch.template operator()<16, A_ROWS>();
+        if (ceil_div(n, 24) <= cus) return launch.template operator()<24, A_ROWS>();
+        if constexpr (TM <= 2) {
+            if (ceil_div(n, 32) > cus) {
+                if (ceil_div(n, 40) <= cus) return launch.template operator()<40, A_ROWS>();
+                if (ceil_div(n, 48) <= cus) return launch.template operator()<48, A_ROWS>();
+                return launch.template operator()<64, A_ROWS>();
+            }
         }
+        return launch.template operator()<32, A_ROWS>();
     };
-    if constexpr (OPERANDS == kCast) rows.template operator()<CAST_ROWS>();
-    else if constexpr (TM == 1) {
-        if (m <= 8) rows.template operator()<8>();
-        else rows.template operator()<16>();
-    } else rows.template operator()<16 * TM>();
-    return true;
+    if constexpr (OPERANDS == kCast) return rows.template operator()<CAST_ROWS>();
+    else if constexpr (TM == 1) return m <= 8 ? rows.template operator()<8>() : rows.template operator()<16>();
+    else return rows.template operator()<16 * TM>();
 }
 
 } // namespace yan
