@@ -1,0 +1,77 @@
+"""The native side of repeated calls (yan_amd/csrc/host_calls.cpp) without a GPU: the module is set up with a device, streams, workspaces and
+launches of the test's own, and gets calls whose arguments are plain numbers."""
+import ctypes
+import os
+
+import pytest
+import torch
+
+from yan_amd.jit_kernels import host_calls, split_k, utils
+
+TENSOR, CONSTANT, STREAM, WORKSPACE = range(4)
+ENTRY = 1 << 20         # no entry's number
+
+
+class Stage:
+    """What the native module looks at, and a launch that notes what it gets."""
+
+    def __init__(self):
+        self.device, self.stream, self.capturing, self.looks = 0, 111, False, 0
+        self.launched, self.code, self.failed = [], 0, []
+        self.make = lambda: torch.zeros(64, dtype=torch.uint8)
+        self.split_k = {'_last': (None, None), '_book': split_k.WorkspaceBook(make=self.make, clear=lambda w: None),
+                        'split_k_launch_failed': self.failed.append}
+
+        def launch(first, second, rc, *_):
+            self.launched.append((first, second))
+            rc[0] = self.code
+        self.function = ctypes.CFUNCTYPE(None, ctypes.c_uint64, ctypes.c_uint64, ctypes.POINTER(ctypes.c_int), ctypes.c_float, ctypes.c_float)(launch)
+
+    def look(self):
+        self.looks += 1
+        return self.device
+
+    def setup(self):
+        native = host_calls._host_calls
+        native.setup({'_num_sms': 256}, self.split_k, os.__dict__, os.environ, os.environ._data, self.look, lambda device: self.stream,
+                     lambda: self.capturing)
+        native.forget()
+
+    def remember(self, call, *spec):
+        return host_calls._host_calls.remember(call, 'a_kernel', ctypes.cast(self.function, ctypes.c_void_p).value, spec)
+
+    def call(self, *call):
+        return host_calls._host_calls.call(*call)
+
+    def take(self, stream):
+        """A workspace for `stream`, as an eager launch gets it by way of Python."""
+        workspace = self.split_k['_book'].get(self.device, stream)
+        self.split_k['_last'] = ((self.device, stream, None), workspace)
+        return workspace
+
+
+@pytest.fixture
+def stage(monkeypatch):
+    assert host_calls._host_calls is not None, 'yan_amd/csrc/build.py builds it'
+    for name in ('YAN_SPLIT_K', 'YAN_TUNE_TILES'):
+        monkeypatch.delenv(name, raising=False)
+    stage = Stage()
+    stage.setup()
+    yield stage
+    host_calls.setup_native()
+    host_calls._host_calls.forget()
+
+
+@pytest.mark.parametrize('workspace', [False, True])
+def test_a_launch_that_reports_an_error_is_not_made_twice(stage, workspace):
+    """The code may be an older error's, behind a launch that ran: the call raises what the Python way raises, and the workspace is marked."""
+    held = stage.take(111)
+    token = stage.split_k['_last'][0]
+    assert stage.remember((ENTRY, 1.0), (WORKSPACE if workspace else CONSTANT, 5), (STREAM, 0))
+    assert stage.call(ENTRY, 1.0) is True and stage.launched == [(held.data_ptr() if workspace else 5, 111)]
+    stage.code = 98
+    with pytest.raises(AssertionError, match='a_kernel failed with HIP error 98'):
+        stage.call(ENTRY, 1.0)
+    assert len(stage.launched) == 2 and stage.failed == ([token] if workspace else [])
+    stage.code = 0
+    assert stage.call(ENTRY, 1.0) is True and len(stage.launched) == 3

@@ -13,6 +13,7 @@
 #include <cstdint>
 #include <cstring>
 #include <memory>
+#include <string>
 #include <unordered_map>
 #include <utility>
 #include <vector>
@@ -26,6 +27,7 @@ enum Kind : int { kTensor = 0, kConstant = 1, kStream = 2, kWorkspace = 3 };
 
 struct Launch {
     std::vector<int64_t> key;
+    std::string name;                           // for the error message
     void* function;
     int count;
     bool workspace;
@@ -35,7 +37,7 @@ struct Launch {
 
 std::unordered_multimap<uint64_t, std::unique_ptr<Launch>> g_launches;
 PyObject *g_utils, *g_split_k, *g_os, *g_environ, *g_environ_bytes, *g_device, *g_stream, *g_capturing;
-PyObject *s_num_sms, *s_last, *s_environ, *b_split_k, *b_tune;
+PyObject *s_num_sms, *s_last, *s_failed, *s_environ, *b_split_k, *b_tune;
 
 struct Call {
     int64_t key[kMaxKey];
@@ -144,7 +146,19 @@ int launch_of(int count, void* f, const uint64_t* a, const float* fl) {
     return -1;
 }
 
-// call(entry, *arguments): True if the launch was made.
+// A launch that reported an error, as the Python way reports it. It is not made again: the code can be that of an older error of this
+// thread, asked for behind a launch that did run (c = alpha a b + beta c would be applied twice).
+PyObject* launch_failed(const std::string& name, PyObject* token, int rc) {
+    if (token) {
+        PyObject* mark = PyDict_GetItemWithError(g_split_k, s_failed);
+        PyObject* done = mark ? PyObject_CallOneArg(mark, token) : nullptr;
+        Py_XDECREF(done);
+        if (PyErr_Occurred()) return nullptr;
+    }
+    return PyErr_Format(PyExc_AssertionError, "%s failed with HIP error %d", name.c_str(), rc);
+}
+
+// call(entry, *arguments): True if the launch was made, AssertionError if it failed.
 PyObject* call(PyObject*, PyObject* const* objs, Py_ssize_t n) {
     if (!g_utils || g_launches.empty()) Py_RETURN_FALSE;
     try {
@@ -157,7 +171,7 @@ PyObject* call(PyObject*, PyObject* const* objs, Py_ssize_t n) {
         const bool have_stream = call_int(g_stream, device, &stream);
         Py_DECREF(device);
         if (!have_stream) Py_RETURN_FALSE;
-        PyObject* workspace = nullptr;
+        PyObject *workspace = nullptr, *token = nullptr;
         uint64_t workspace_address = 0;
         if (l->workspace) {
             // the latest eager launch's workspace, if it is this stream's; a capture has its own
@@ -170,7 +184,7 @@ PyObject* call(PyObject*, PyObject* const* objs, Py_ssize_t n) {
                 PyErr_Clear();
                 Py_RETURN_FALSE;
             }
-            PyObject* token = PyTuple_GET_ITEM(last, 0);
+            token = PyTuple_GET_ITEM(last, 0);
             workspace = PyTuple_GET_ITEM(last, 1);
             if (!PyTuple_CheckExact(token) || PyTuple_GET_SIZE(token) != 3 || PyTuple_GET_ITEM(token, 2) != Py_None ||
                 !plain_int(PyTuple_GET_ITEM(token, 0), &index) || index != c.device || !plain_int(PyTuple_GET_ITEM(token, 1), &owner) ||
@@ -189,14 +203,17 @@ PyObject* call(PyObject*, PyObject* const* objs, Py_ssize_t n) {
             }
         }
         // other threads may run meanwhile, and clear the table: nothing of it is looked at from here on
+        const std::string name = l->name;
         Py_XINCREF(workspace);
+        Py_XINCREF(token);
         int rc;
         Py_BEGIN_ALLOW_THREADS
         rc = launch_of<kMaxArgs>(count, function, args, c.floats);
         Py_END_ALLOW_THREADS
         Py_XDECREF(workspace);
-        // a launch that was refused started nothing: Python makes it again and reports the error
-        if (rc != 0) Py_RETURN_FALSE;
+        PyObject* const failed = rc != 0 ? launch_failed(name, token, rc) : nullptr;
+        Py_XDECREF(token);
+        if (rc != 0) return failed;
         Py_RETURN_TRUE;
     } catch (...) {         // a tensor without storage, say: the checks in Python will say so
         PyErr_Clear();
@@ -204,11 +221,12 @@ PyObject* call(PyObject*, PyObject* const* objs, Py_ssize_t n) {
     }
 }
 
-// remember((entry, *arguments), address, ((kind, value), ...)): the launch that served these arguments.
+// remember((entry, *arguments), name, address, ((kind, value), ...)): the launch that served these arguments.
 PyObject* remember(PyObject*, PyObject* args) {
     PyObject *objs, *spec;
+    const char* name;
     unsigned long long address;
-    if (!PyArg_ParseTuple(args, "O!KO!", &PyTuple_Type, &objs, &address, &PyTuple_Type, &spec)) return nullptr;
+    if (!PyArg_ParseTuple(args, "O!sKO!", &PyTuple_Type, &objs, &name, &address, &PyTuple_Type, &spec)) return nullptr;
     try {
         Call c;
         std::vector<PyObject*> items;
@@ -217,6 +235,7 @@ PyObject* remember(PyObject*, PyObject* args) {
         if (!g_utils || count < 1 || count > kMaxArgs || !describe(c, items.data(), Py_ssize_t(items.size()))) Py_RETURN_FALSE;
         auto l = std::make_unique<Launch>();
         l->key.assign(c.key, c.key + c.used);
+        l->name = name;
         l->function = reinterpret_cast<void*>(address);
         l->count = int(count);
         l->workspace = false;
@@ -268,6 +287,7 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_host_calls", nullptr, -1, met
 PyMODINIT_FUNC PyInit__host_calls() {
     s_num_sms = PyUnicode_InternFromString("_num_sms");
     s_last = PyUnicode_InternFromString("_last");
+    s_failed = PyUnicode_InternFromString("split_k_launch_failed");
     s_environ = PyUnicode_InternFromString("environ");
     b_split_k = PyBytes_FromString("YAN_SPLIT_K");
     b_tune = PyBytes_FromString("YAN_TUNE_TILES");

@@ -121,7 +121,7 @@ def _gemm_16bit_tn(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, dtype: tor
     if rc != 0 and workspace_token is not None:
         split_k_launch_failed(workspace_token)
     assert rc == 0, f'{name} failed with HIP error {rc}'
-    remember_call((entry, a, b, c), runtime, args, workspace)
+    remember_call((entry, a, b, c), name, runtime, args, workspace)
 
 
 def gemm_bf16_tn(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor) -> None:

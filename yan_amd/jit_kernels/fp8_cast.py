@@ -78,7 +78,7 @@ def per_token_cast_to_fp8(x: torch.Tensor, col_major_scales: bool = False) -> Tu
                                          template=template, args=args)
     rc = runtime(*args)
     assert rc == 0, f'{name} failed with HIP error {rc}'
-    remember_call((PER_TOKEN, x, q, scales), runtime, args)
+    remember_call((PER_TOKEN, x, q, scales), name, runtime, args)
     return q, scales
 
 
@@ -99,5 +99,5 @@ def per_block_cast_to_fp8(w: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
                                          template=template, args=args)
     rc = runtime(*args)
     assert rc == 0, f'{name} failed with HIP error {rc}'
-    remember_call((PER_BLOCK, w, q, scales), runtime, args)
+    remember_call((PER_BLOCK, w, q, scales), name, runtime, args)
     return q, scales

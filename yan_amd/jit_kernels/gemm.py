@@ -230,7 +230,7 @@ def gemm_fp8_fp8_bf16_nt(lhs: Tuple[torch.Tensor, torch.Tensor],
     assert rc == 0, f'{name} failed with HIP error {rc}'
     # (what `scales_for_kernel` does with a large problem's other layouts is decided by the addresses of each call)
     if flop < SCALE_RELAYOUT_MIN_FLOP or token_contiguous:
-        remember_call((FP8, lhs, lhs_scales, rhs, rhs_scales, out), runtime, args, workspace)
+        remember_call((FP8, lhs, lhs_scales, rhs, rhs_scales, out), name, runtime, args, workspace)
 
 
 # Scratch of the chained entry: behind the 16 MB of the split-K workspace, room for the codes and scales of up to
@@ -302,7 +302,7 @@ def gemm_bf16_fp8_bf16_nt(x: torch.Tensor, rhs: Tuple[torch.Tensor, torch.Tensor
         runtime = jit_tuner.compile_and_tune(name=name, keys=keys, space=(), includes=includes, arg_defs=defs, template=code_template, args=args)
         rc = runtime(*args)
         assert rc == 0, f'{name} failed with HIP error {rc}'
-        remember_call((CAST_FP8, x, rhs_q, rhs_scales, out), runtime, args)
+        remember_call((CAST_FP8, x, rhs_q, rhs_scales, out), name, runtime, args)
         return
     if split_k_enabled() and not tuning_enabled():
         plan = fp8_cast_chain_plan(m, n, k, num_sms, split_k_allowed=not get_weight_stream_fp8_config(m, n, k, num_sms))
@@ -321,4 +321,4 @@ def gemm_bf16_fp8_bf16_nt(x: torch.Tensor, rhs: Tuple[torch.Tensor, torch.Tensor
     if rc != 0:
         split_k_launch_failed(workspace_token)
     assert rc == 0, f'{name} failed with HIP error {rc}'
-    remember_call((CAST_FP8, x, rhs_q, rhs_scales, out), runtime, args, workspace)
+    remember_call((CAST_FP8, x, rhs_q, rhs_scales, out), name, runtime, args, workspace)

@@ -31,19 +31,24 @@ def _never(*_) -> bool:
     return False
 
 
+def setup_native() -> None:
+    """Hands the native module what it looks at on every call."""
+    _host_calls.setup(utils.__dict__, split_k.__dict__, os.__dict__, utils._environ, utils._environ_bytes, torch._C._cuda_getDevice,
+                      torch._C._cuda_getCurrentRawStream, split_k._is_capturing)
+
+
 repeat_call = _never
 if _host_calls is not None and utils._environ is not None:
     try:
-        _host_calls.setup(utils.__dict__, split_k.__dict__, os.__dict__, utils._environ, utils._environ_bytes, torch._C._cuda_getDevice,
-                          torch._C._cuda_getCurrentRawStream, split_k._is_capturing)
+        setup_native()
         repeat_call = _host_calls.call
     except (AttributeError, TypeError):          # a torch without the raw accessors
         pass
 
 
-def remember_call(call: tuple, runtime: Runtime, args: tuple, workspace=None) -> None:
-    """`call`: the entry and its arguments as `repeat_call` gets them, tensors and floats in the order of `args`, which `runtime` has just
-    been launched with. `workspace`: the split-K workspace among them, looked up anew by every call."""
+def remember_call(call: tuple, name: str, runtime: Runtime, args: tuple, workspace=None) -> None:
+    """`call`: the entry and its arguments as `repeat_call` gets them, tensors and floats in the order of `args`, which `runtime`, the kernel
+    `name`, has just been launched with. `workspace`: the split-K workspace among them, looked up anew by every call."""
     if repeat_call is _never or type(runtime) is not Runtime or runtime._launch is None or not split_k.split_k_enabled() or tuning_enabled():
         return
     spec, tensors = [], 0
@@ -58,4 +63,4 @@ def remember_call(call: tuple, runtime: Runtime, args: tuple, workspace=None) ->
         elif kind is not float:
             spec.append((_CONSTANT, int(arg)))
     if tensors == sum(isinstance(a, torch.Tensor) for a in call):
-        _host_calls.remember(call, ctypes.cast(runtime._launch, ctypes.c_void_p).value, tuple(spec))
+        _host_calls.remember(call, name, ctypes.cast(runtime._launch, ctypes.c_void_p).value, tuple(spec))

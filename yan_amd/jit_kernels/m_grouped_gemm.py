@@ -88,7 +88,7 @@ def _launch(gemm_type, num_groups, plan_m, m, n, k, lhs, lhs_scales, rhs, rhs_sc
     assert rc == 0, f'{name} failed with HIP error {rc}'
     # (what `scales_for_kernel` does with a large problem's other layouts is decided by the addresses of each call)
     if flop < SCALE_RELAYOUT_MIN_FLOP or (lhs_scales.stride(-2) == 1 and lhs_scales.stride(-1) == lhs_scales.size(-2)):
-        remember_call((call[0], lhs, lhs_scales, rhs, rhs_scales, out, layout, *call[1:]), runtime, args)
+        remember_call((call[0], lhs, lhs_scales, rhs, rhs_scales, out, layout, *call[1:]), name, runtime, args)
 
 
 def m_grouped_gemm_fp8_fp8_bf16_nt_contiguous(lhs: Tuple[torch.Tensor, torch.Tensor],

@@ -159,7 +159,7 @@ def gemm_float_nt(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor,
     if rc != 0 and workspace_token is not None:
         split_k_launch_failed(workspace_token)
     assert rc == 0, f'{name} failed with HIP error {rc}'
-    remember_call((FLOAT, float(alpha), a, b, float(beta), c), runtime, args, workspace)
+    remember_call((FLOAT, float(alpha), a, b, float(beta), c), name, runtime, args, workspace)
 
 
 def accuracy_test():
