@@ -75,3 +75,22 @@ def test_a_launch_that_reports_an_error_is_not_made_twice(stage, workspace):
     assert len(stage.launched) == 2 and stage.failed == ([token] if workspace else [])
     stage.code = 0
     assert stage.call(ENTRY, 1.0) is True and len(stage.launched) == 3
+
+
+@pytest.mark.parametrize('when', ['stream', 'capturing'])
+def test_a_launch_outlives_what_runs_while_it_is_prepared(stage, when):
+    """Python code that runs between the look into the table and the launch (a finaliser, another thread) may clear and refill the table."""
+    held = stage.take(111)
+    assert stage.remember((ENTRY, 1.0), (CONSTANT, 5), (WORKSPACE, 0))
+
+    def meddle(answer):
+        host_calls._host_calls.forget()
+        for i in range(64):
+            assert stage.remember((ENTRY, i), (CONSTANT, 1000 + i), (CONSTANT, 7))
+        return answer
+
+    look = {'stream': lambda device: 111, 'capturing': lambda: False}
+    look[when] = lambda *_, plain=look[when]: meddle(plain(*_))
+    host_calls._host_calls.setup({'_num_sms': 256}, stage.split_k, os.__dict__, os.environ, os.environ._data, stage.look, look['stream'],
+                                 look['capturing'])
+    assert stage.call(ENTRY, 1.0) is True and stage.launched == [(5, held.data_ptr())]

@@ -35,7 +35,7 @@ struct Launch {
     std::array<int64_t, kMaxArgs> value;        // a constant, or which tensor
 };
 
-std::unordered_multimap<uint64_t, std::unique_ptr<Launch>> g_launches;
+std::unordered_multimap<uint64_t, std::shared_ptr<Launch>> g_launches;
 PyObject *g_utils, *g_split_k, *g_os, *g_environ, *g_environ_bytes, *g_device, *g_stream, *g_capturing;
 PyObject *s_num_sms, *s_last, *s_failed, *s_environ, *b_split_k, *b_tune;
 
@@ -113,10 +113,10 @@ bool describe(Call& c, PyObject* const* objs, Py_ssize_t n) {
     return true;
 }
 
-Launch* find(const Call& c) {
+std::shared_ptr<Launch> find(const Call& c) {
     const auto range = g_launches.equal_range(c.hash());
     for (auto it = range.first; it != range.second; ++it)
-        if (int(it->second->key.size()) == c.used && std::memcmp(it->second->key.data(), c.key, size_t(c.used) * 8) == 0) return it->second.get();
+        if (int(it->second->key.size()) == c.used && std::memcmp(it->second->key.data(), c.key, size_t(c.used) * 8) == 0) return it->second;
     return nullptr;
 }
 
@@ -164,7 +164,8 @@ PyObject* call(PyObject*, PyObject* const* objs, Py_ssize_t n) {
     try {
         Call c;
         if (!describe(c, objs, n) || !usual_switches()) Py_RETURN_FALSE;
-        const Launch* l = find(c);
+        // held, not looked at in the table: what is called below can run other Python code, and other threads, that clear it
+        const std::shared_ptr<const Launch> l = find(c);
         if (!l) Py_RETURN_FALSE;
         PyObject* device = PyLong_FromLongLong(c.device);
         int64_t stream;
@@ -192,9 +193,7 @@ PyObject* call(PyObject*, PyObject* const* objs, Py_ssize_t n) {
             workspace_address = reinterpret_cast<uint64_t>(THPVariable_Unpack(workspace).data_ptr());
         }
         uint64_t args[kMaxArgs];
-        const int count = l->count;
-        void* const function = l->function;
-        for (int i = 0; i < count; ++i) {
+        for (int i = 0; i < l->count; ++i) {
             switch (l->kind[i]) {
                 case kTensor: args[i] = c.address[l->value[i]]; break;
                 case kConstant: args[i] = uint64_t(l->value[i]); break;
@@ -202,16 +201,14 @@ PyObject* call(PyObject*, PyObject* const* objs, Py_ssize_t n) {
                 default: args[i] = workspace_address;
             }
         }
-        // other threads may run meanwhile, and clear the table: nothing of it is looked at from here on
-        const std::string name = l->name;
         Py_XINCREF(workspace);
         Py_XINCREF(token);
         int rc;
         Py_BEGIN_ALLOW_THREADS
-        rc = launch_of<kMaxArgs>(count, function, args, c.floats);
+        rc = launch_of<kMaxArgs>(l->count, l->function, args, c.floats);
         Py_END_ALLOW_THREADS
         Py_XDECREF(workspace);
-        PyObject* const failed = rc != 0 ? launch_failed(name, token, rc) : nullptr;
+        PyObject* const failed = rc != 0 ? launch_failed(l->name, token, rc) : nullptr;
         Py_XDECREF(token);
         if (rc != 0) return failed;
         Py_RETURN_TRUE;
@@ -233,7 +230,7 @@ PyObject* remember(PyObject*, PyObject* args) {
         for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(objs); ++i) items.push_back(PyTuple_GET_ITEM(objs, i));
         const Py_ssize_t count = PyTuple_GET_SIZE(spec);
         if (!g_utils || count < 1 || count > kMaxArgs || !describe(c, items.data(), Py_ssize_t(items.size()))) Py_RETURN_FALSE;
-        auto l = std::make_unique<Launch>();
+        auto l = std::make_shared<Launch>();
         l->key.assign(c.key, c.key + c.used);
         l->name = name;
         l->function = reinterpret_cast<void*>(address);
@@ -248,7 +245,10 @@ PyObject* remember(PyObject*, PyObject* args) {
             l->workspace |= kind == kWorkspace;
         }
         if (g_launches.size() >= kMaxCalls) g_launches.clear();
-        if (Launch* old = find(c)) *old = *l;
+        const auto range = g_launches.equal_range(c.hash());
+        auto at = range.first;
+        while (at != range.second && at->second->key != l->key) ++at;
+        if (at != range.second) at->second = std::move(l);
         else g_launches.emplace(c.hash(), std::move(l));
         Py_RETURN_TRUE;
     } catch (...) {
