@@ -94,3 +94,38 @@ def test_a_launch_outlives_what_runs_while_it_is_prepared(stage, when):
     host_calls._host_calls.setup({'_num_sms': 256}, stage.split_k, os.__dict__, os.environ, os.environ._data, stage.look, look['stream'],
                                  look['capturing'])
     assert stage.call(ENTRY, 1.0) is True and stage.launched == [(5, held.data_ptr())]
+
+
+def test_streams_in_turn_are_served_from_their_workspaces(stage):
+    """Each stream gets the workspace the book holds for it, whichever stream was served last; a stream without one, one whose last launch
+    failed and a capture go back to Python."""
+    first, second = stage.take(111), stage.take(222)
+    assert stage.remember((ENTRY, 1.0), (WORKSPACE, 0), (STREAM, 0))
+    for stream in (111, 222, 111, 111, 222):
+        stage.stream = stream
+        assert stage.call(ENTRY, 1.0) is True
+        assert stage.launched[-1] == ((first if stream == 111 else second).data_ptr(), stream)
+    stage.stream = 333
+    assert stage.call(ENTRY, 1.0) is False
+    stage.device, stage.stream = 1, 111
+    assert stage.call(ENTRY, 1.0) is False
+    stage.device, stage.capturing = 0, True
+    assert stage.call(ENTRY, 1.0) is False
+    stage.capturing, stage.code = False, 98
+    with pytest.raises(AssertionError):
+        stage.call(ENTRY, 1.0)
+    assert stage.failed == [(0, 111, None)]
+    stage.split_k['_book'].launch_failed(*stage.failed[0])
+    assert stage.call(ENTRY, 1.0) is False and len(stage.launched) == 6
+    stage.stream, stage.code = 222, 0
+    assert stage.call(ENTRY, 1.0) is True
+
+
+@pytest.mark.parametrize('name,value', [('YAN_SPLIT_K', '0'), ('YAN_TUNE_TILES', '1')])
+def test_calls_under_a_switch_cost_no_description(stage, name, value, monkeypatch):
+    assert stage.remember((ENTRY, 1.0), (CONSTANT, 5), (STREAM, 0))
+    looks = stage.looks
+    monkeypatch.setenv(name, value)
+    assert stage.call(ENTRY, 1.0) is False and stage.looks == looks
+    monkeypatch.delenv(name)
+    assert stage.call(ENTRY, 1.0) is True and stage.looks > looks

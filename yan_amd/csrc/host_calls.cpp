@@ -37,7 +37,7 @@ struct Launch {
 
 std::unordered_multimap<uint64_t, std::shared_ptr<Launch>> g_launches;
 PyObject *g_utils, *g_split_k, *g_os, *g_environ, *g_environ_bytes, *g_device, *g_stream, *g_capturing;
-PyObject *s_num_sms, *s_last, *s_failed, *s_environ, *b_split_k, *b_tune;
+PyObject *s_num_sms, *s_last, *s_book, *s_eager, *s_suspect, *s_failed, *s_environ, *b_split_k, *b_tune;
 
 struct Call {
     int64_t key[kMaxKey];
@@ -146,6 +146,41 @@ int launch_of(int count, void* f, const uint64_t* a, const float* fl) {
     return -1;
 }
 
+// The workspace of eager launches on a stream and the token that goes with it, as new references: the latest launch's if it was on this
+// stream (split_k._last), else what the book holds for it, unless a launch there failed. False: for Python to make or clear.
+bool eager_workspace(int64_t device, int64_t stream, PyObject** token, PyObject** workspace) {
+    PyObject* last = PyDict_GetItemWithError(g_split_k, s_last);
+    int64_t index, owner;
+    if (last && PyTuple_CheckExact(last) && PyTuple_GET_SIZE(last) == 2) {
+        PyObject *t = PyTuple_GET_ITEM(last, 0), *w = PyTuple_GET_ITEM(last, 1);
+        if (PyTuple_CheckExact(t) && PyTuple_GET_SIZE(t) == 3 && PyTuple_GET_ITEM(t, 2) == Py_None && plain_int(PyTuple_GET_ITEM(t, 0), &index) &&
+            index == device && plain_int(PyTuple_GET_ITEM(t, 1), &owner) && owner == stream && THPVariable_CheckExact(w)) {
+            Py_INCREF(*token = t);
+            Py_INCREF(*workspace = w);
+            return true;
+        }
+    }
+    PyObject* book = PyDict_GetItemWithError(g_split_k, s_book);
+    PyObject* held = book ? PyObject_GetAttr(book, s_eager) : nullptr;
+    PyObject* suspect = held ? PyObject_GetAttr(book, s_suspect) : nullptr;
+    PyObject* key = suspect ? Py_BuildValue("(LL)", (long long)device, (long long)stream) : nullptr;
+    bool found = false;
+    if (key && PyDict_CheckExact(held) && PyAnySet_Check(suspect)) {
+        PyObject* w = PyDict_GetItemWithError(held, key);
+        if (w && THPVariable_CheckExact(w) && PySet_Contains(suspect, key) == 0) {
+            Py_INCREF(w);
+            if ((*token = Py_BuildValue("(LLO)", (long long)device, (long long)stream, Py_None))) {
+                *workspace = w;
+                found = true;
+            } else Py_DECREF(w);
+        }
+    }
+    Py_XDECREF(key);
+    Py_XDECREF(suspect);
+    Py_XDECREF(held);
+    return found;
+}
+
 // A launch that reported an error, as the Python way reports it. It is not made again: the code can be that of an older error of this
 // thread, asked for behind a launch that did run (c = alpha a b + beta c would be applied twice).
 PyObject* launch_failed(const std::string& name, PyObject* token, int rc) {
@@ -163,7 +198,7 @@ PyObject* call(PyObject*, PyObject* const* objs, Py_ssize_t n) {
     if (!g_utils || g_launches.empty()) Py_RETURN_FALSE;
     try {
         Call c;
-        if (!describe(c, objs, n) || !usual_switches()) Py_RETURN_FALSE;
+        if (!usual_switches() || !describe(c, objs, n)) Py_RETURN_FALSE;
         // held, not looked at in the table: what is called below can run other Python code, and other threads, that clear it
         const std::shared_ptr<const Launch> l = find(c);
         if (!l) Py_RETURN_FALSE;
@@ -175,21 +210,14 @@ PyObject* call(PyObject*, PyObject* const* objs, Py_ssize_t n) {
         PyObject *workspace = nullptr, *token = nullptr;
         uint64_t workspace_address = 0;
         if (l->workspace) {
-            // the latest eager launch's workspace, if it is this stream's; a capture has its own
+            // a capture has its own
             PyObject* capturing = PyObject_CallNoArgs(g_capturing);
             const bool eager = capturing == Py_False;
             Py_XDECREF(capturing);
-            PyObject* last = PyDict_GetItemWithError(g_split_k, s_last);
-            int64_t index, owner;
-            if (!eager || !last || !PyTuple_CheckExact(last) || PyTuple_GET_SIZE(last) != 2) {
+            if (!eager || !eager_workspace(c.device, stream, &token, &workspace)) {
                 PyErr_Clear();
                 Py_RETURN_FALSE;
             }
-            token = PyTuple_GET_ITEM(last, 0);
-            workspace = PyTuple_GET_ITEM(last, 1);
-            if (!PyTuple_CheckExact(token) || PyTuple_GET_SIZE(token) != 3 || PyTuple_GET_ITEM(token, 2) != Py_None ||
-                !plain_int(PyTuple_GET_ITEM(token, 0), &index) || index != c.device || !plain_int(PyTuple_GET_ITEM(token, 1), &owner) ||
-                owner != stream || !THPVariable_CheckExact(workspace)) Py_RETURN_FALSE;
             workspace_address = reinterpret_cast<uint64_t>(THPVariable_Unpack(workspace).data_ptr());
         }
         uint64_t args[kMaxArgs];
@@ -201,8 +229,6 @@ PyObject* call(PyObject*, PyObject* const* objs, Py_ssize_t n) {
                 default: args[i] = workspace_address;
             }
         }
-        Py_XINCREF(workspace);
-        Py_XINCREF(token);
         int rc;
         Py_BEGIN_ALLOW_THREADS
         rc = launch_of<kMaxArgs>(l->count, l->function, args, c.floats);
@@ -287,6 +313,9 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_host_calls", nullptr, -1, met
 PyMODINIT_FUNC PyInit__host_calls() {
     s_num_sms = PyUnicode_InternFromString("_num_sms");
     s_last = PyUnicode_InternFromString("_last");
+    s_book = PyUnicode_InternFromString("_book");
+    s_eager = PyUnicode_InternFromString("eager");
+    s_suspect = PyUnicode_InternFromString("suspect");
     s_failed = PyUnicode_InternFromString("split_k_launch_failed");
     s_environ = PyUnicode_InternFromString("environ");
     b_split_k = PyBytes_FromString("YAN_SPLIT_K");
