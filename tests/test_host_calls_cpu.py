@@ -2,6 +2,9 @@
 launches of the test's own, and gets calls whose arguments are plain numbers."""
 import ctypes
 import os
+import subprocess
+import sys
+import sysconfig
 
 import pytest
 import torch
@@ -129,3 +132,23 @@ def test_calls_under_a_switch_cost_no_description(stage, name, value, monkeypatc
     assert stage.call(ENTRY, 1.0) is False and stage.looks == looks
     monkeypatch.delenv(name)
     assert stage.call(ENTRY, 1.0) is True and stage.looks > looks
+
+
+def test_a_module_of_another_torch_is_not_used(repo_root):
+    """Neither loaded over nor kept by the build: the name of the torch is compiled in, that of the Python is in the file's name."""
+    code = """
+import torch
+torch.__version__ = {version}
+import yan_amd
+from yan_amd.jit_kernels import host_calls
+import importlib.util
+spec = importlib.util.spec_from_file_location('build', 'yan_amd/csrc/build.py')
+build = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(build)
+print(host_calls._host_calls is not None, host_calls.repeat_call is not host_calls._never, build.host_calls_up_to_date())
+"""
+    for version, used in (('torch.__version__', True), ('"2.0.1+other"', False)):
+        done = subprocess.run([sys.executable, '-c', code.format(version=version)], stdout=subprocess.PIPE, universal_newlines=True, check=True,
+                              cwd=repo_root)
+        assert done.stdout.split() == [str(used)] * 3
+    assert host_calls._host_calls.__file__.endswith('_host_calls' + sysconfig.get_config_var('EXT_SUFFIX'))

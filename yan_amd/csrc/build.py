@@ -1,11 +1,13 @@
 #!/usr/bin/env python3
 """Builds yan_amd/csrc/libyan_gemm.so, the ahead-of-time C-ABI library (declared in include/yan_gemm.h), with
-hipcc for gfx950, and yan_amd/_host_calls.so, the host side of repeated calls, with the host compiler against torch's headers.
-Needs no GPU. `--force` rebuilds even when the libraries are newer than their sources."""
+hipcc for gfx950, and yan_amd/_host_calls.<ABI of this Python>.so, the host side of repeated calls, with the host compiler against torch's
+headers. Needs no GPU. `--force` rebuilds even when the libraries are newer than their sources."""
 import glob
 import os
+import platform
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(os.path.dirname(HERE))
@@ -37,17 +39,32 @@ def build(force: bool = False) -> str:
 
 
 HOST_SRC = os.path.join(HERE, 'host_calls.cpp')
-HOST_OUT = os.path.join(ROOT, 'yan_amd', '_host_calls.so')
+# in the file's name as Python looks for it: another Python does not load it
+HOST_OUT = os.path.join(ROOT, 'yan_amd', '_host_calls' + sysconfig.get_config_var('EXT_SUFFIX'))
+
+
+def built_for() -> str:
+    """The torch whose object layouts are compiled in; jit_kernels/host_calls.py asks the module for it before anything else."""
+    import torch
+    return f'torch {torch.__version__} {torch.version.git_version}'
+
+
+def host_calls_up_to_date() -> bool:
+    if not os.path.exists(HOST_OUT) or os.path.getmtime(HOST_OUT) < os.path.getmtime(HOST_SRC):
+        return False
+    with open(HOST_OUT, 'rb') as f:
+        return built_for().encode() + b'\0' in f.read()
 
 
 def build_host_calls(force: bool = False) -> str:
-    if not force and os.path.exists(HOST_OUT) and os.path.getmtime(HOST_OUT) >= os.path.getmtime(HOST_SRC):
+    if platform.machine() != 'x86_64':          # it passes arguments as that ABI has it; without it every call goes through Python
+        return ''
+    if not force and host_calls_up_to_date():
         return HOST_OUT
-    import sysconfig
     import torch
     from torch.utils import cpp_extension
     lib = os.path.join(os.path.dirname(torch.__file__), 'lib')
-    cmd = [os.getenv('CXX') or 'g++', HOST_SRC, '-o', HOST_OUT + '.tmp', '-std=c++17', '-O2', '-shared', '-fPIC',
+    cmd = [os.getenv('CXX') or 'g++', HOST_SRC, '-o', HOST_OUT + '.tmp', '-std=c++17', '-O2', '-shared', '-fPIC', f'-DYAN_BUILT_FOR="{built_for()}"',
            f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}', *(f'-isystem{p}' for p in cpp_extension.include_paths()),
            f'-I{sysconfig.get_paths()["include"]}', f'-L{lib}', '-ltorch_python', '-ltorch_cpu', '-lc10']
     done = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, universal_newlines=True)

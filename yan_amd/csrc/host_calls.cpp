@@ -4,6 +4,7 @@
 // have changed the plan (the compute-unit cap, the environment switches, another stream's workspace, a capture), goes back to Python.
 //
 // What it is for: one 1 x 2112 x 7168 FP8 call costs the host 8.5 us from Python and 3.5 from here, of which 2.5 are the launch; the kernel takes 7.
+// What it compiles in of torch's objects holds for one torch: `built_for` names it, and host_calls.py uses no module built for another.
 // Nothing is kept by address or identity: addresses are read from the tensors of each call, the workspace from split_k.py's own record.
 #include <Python.h>
 
@@ -132,6 +133,9 @@ bool usual_switches() {
     return on(b_split_k, true) && !on(b_tune, false);
 }
 
+#if !defined(__x86_64__) || !defined(__linux__)
+#error "launch_with passes arguments as the System V ABI of x86-64 does"
+#endif
 // Integer arguments go where integers go and floating-point ones where those go, whatever their order among each other (x86-64).
 template <size_t... I>
 int launch_with(void* f, const uint64_t* a, const float* fl, std::index_sequence<I...>) {
@@ -320,5 +324,7 @@ PyMODINIT_FUNC PyInit__host_calls() {
     s_environ = PyUnicode_InternFromString("environ");
     b_split_k = PyBytes_FromString("YAN_SPLIT_K");
     b_tune = PyBytes_FromString("YAN_TUNE_TILES");
-    return PyModule_Create(&module_def);
+    PyObject* m = PyModule_Create(&module_def);
+    if (m && PyModule_AddStringConstant(m, "built_for", YAN_BUILT_FOR) != 0) Py_CLEAR(m);
+    return m;
 }

@@ -21,6 +21,9 @@ try:
     from .. import _host_calls
 except ImportError:
     _host_calls = None
+# (a module of another torch would read its tensors at wrong offsets; csrc/build.py compiles the name in)
+if getattr(_host_calls, 'built_for', None) != f'torch {torch.__version__} {torch.version.git_version}':
+    _host_calls = None
 
 # which entry a remembered call belongs to
 FP8, CAST_FP8, BF16, FP16, FLOAT, CONTIGUOUS, MASKED, PER_TOKEN, PER_BLOCK = range(1, 10)
