@@ -152,3 +152,33 @@ print(host_calls._host_calls is not None, host_calls.repeat_call is not host_cal
                               cwd=repo_root)
         assert done.stdout.split() == [str(used)] * 3
     assert host_calls._host_calls.__file__.endswith('_host_calls' + sysconfig.get_config_var('EXT_SUFFIX'))
+
+
+@pytest.mark.parametrize('entry', ['plain', 'contiguous', 'masked'])
+@pytest.mark.parametrize('layout,noted', [('token_contiguous', 1), ('row_major', 0)])
+def test_calls_on_a_copy_of_the_scales_are_not_noted(monkeypatch, entry, layout, noted):
+    """Large problems get a token-contiguous copy of row-major scales. What was launched then is no call that comes again, so noting it would
+    be work on every call."""
+    import yan_amd as yan
+    from yan_amd.jit_kernels import gemm, m_grouped_gemm
+    calls = []
+    for module in (gemm, m_grouped_gemm):
+        monkeypatch.setattr(module, 'remember_call', lambda call, *_: calls.append(call))
+        monkeypatch.setattr(module, 'current_raw_stream', lambda: 0)
+        monkeypatch.setattr(module, 'get_num_sms', lambda: 256)
+    monkeypatch.setattr(gemm.jit_tuner, 'compile_and_tune', lambda **_: lambda *args: 0)
+    m, n, k, groups = 4096, 7168, 7168, 4
+    meta = lambda *shape, dtype: torch.empty(*shape, dtype=dtype, device='meta')
+    code, scale, half = torch.float8_e4m3fn, torch.float32, torch.bfloat16
+    lead = (groups, m // groups) if entry == 'masked' else (m, )
+    scales = torch.ones(*lead, k // 128)
+    lhs = meta(*lead, k, dtype=code), yan.get_col_major_tensor(scales) if layout == 'token_contiguous' else scales
+    experts = () if entry == 'plain' else (groups, )
+    rhs, out = (meta(*experts, n, k, dtype=code), meta(*experts, n // 128, k // 128, dtype=scale)), meta(*lead, n, dtype=half)
+    if entry == 'plain':
+        yan.gemm_fp8_fp8_bf16_nt(lhs, rhs, out)
+    elif entry == 'contiguous':
+        yan.m_grouped_gemm_fp8_fp8_bf16_nt_contiguous(lhs, rhs, out, meta(m, dtype=torch.int32))
+    else:
+        yan.m_grouped_gemm_fp8_fp8_bf16_nt_masked(lhs, rhs, out, meta(groups, dtype=torch.int32), m // groups)
+    assert len(calls) == noted and all(call[2] is lhs[1] for call in calls)

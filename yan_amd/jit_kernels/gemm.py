@@ -200,7 +200,7 @@ def gemm_fp8_fp8_bf16_nt(lhs: Tuple[torch.Tensor, torch.Tensor],
         return
 
     num_sms = get_num_sms()
-    flop = 2.0 * m * n * k
+    flop, given_scales = 2.0 * m * n * k, lhs_scales
     if flop >= SCALE_RELAYOUT_MIN_FLOP:
         lhs_scales = scales_for_kernel(lhs_scales, flop, fp8_kernel_plan(m, n, k, num_sms)[1])
     stride_m, stride_k = lhs_scales.stride()
@@ -228,8 +228,8 @@ def gemm_fp8_fp8_bf16_nt(lhs: Tuple[torch.Tensor, torch.Tensor],
     if rc != 0 and workspace_token is not None:
         split_k_launch_failed(workspace_token)
     assert rc == 0, f'{name} failed with HIP error {rc}'
-    # (what `scales_for_kernel` does with a large problem's other layouts is decided by the addresses of each call)
-    if flop < SCALE_RELAYOUT_MIN_FLOP or token_contiguous:
+    # (what `scales_for_kernel` does with a large problem's other layouts is decided by the addresses of each call; a copy's call never comes back)
+    if lhs_scales is given_scales and (flop < SCALE_RELAYOUT_MIN_FLOP or token_contiguous):
         remember_call((FP8, lhs, lhs_scales, rhs, rhs_scales, out), name, runtime, args, workspace)
 
 

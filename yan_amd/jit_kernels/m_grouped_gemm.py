@@ -86,8 +86,9 @@ def _launch(gemm_type, num_groups, plan_m, m, n, k, lhs, lhs_scales, rhs, rhs_sc
                                          template=rows_on_device_template if 'ROWS' in keys else template, args=args)
     rc = runtime(*args)
     assert rc == 0, f'{name} failed with HIP error {rc}'
-    # (what `scales_for_kernel` does with a large problem's other layouts is decided by the addresses of each call)
-    if flop < SCALE_RELAYOUT_MIN_FLOP or (lhs_scales.stride(-2) == 1 and lhs_scales.stride(-1) == lhs_scales.size(-2)):
+    # (what `scales_for_kernel` does with a large problem's other layouts is decided by the addresses of each call; a copy's call, None here,
+    # never comes back)
+    if call is not None and (flop < SCALE_RELAYOUT_MIN_FLOP or (lhs_scales.stride(-2) == 1 and lhs_scales.stride(-1) == lhs_scales.size(-2))):
         remember_call((call[0], lhs, lhs_scales, rhs, rhs_scales, out, layout, *call[1:]), name, runtime, args)
 
 
@@ -126,11 +127,11 @@ def m_grouped_gemm_fp8_fp8_bf16_nt_contiguous(lhs: Tuple[torch.Tensor, torch.Ten
 
     if m == 0:
         return
-    flop = 2.0 * m * n * k
+    flop, given_scales = 2.0 * m * n * k, lhs_scales
     if flop >= SCALE_RELAYOUT_MIN_FLOP:
         lhs_scales = scales_for_kernel(lhs_scales, flop, grouped_kernel_plan('GroupedContiguous', num_groups, m, n, k, get_num_sms())[1])
     _launch('GroupedContiguous', num_groups, m, m, n, k, lhs, lhs_scales, rhs, rhs_scales, out, m_indices,
-            (lhs_scales.stride(0), lhs_scales.stride(1), 0, 0), flop, (CONTIGUOUS, ))
+            (lhs_scales.stride(0), lhs_scales.stride(1), 0, 0), flop, (CONTIGUOUS, ) if lhs_scales is given_scales else None)
 
 
 def m_grouped_gemm_fp8_fp8_bf16_nt_masked(lhs: Tuple[torch.Tensor, torch.Tensor],
@@ -168,8 +169,8 @@ def m_grouped_gemm_fp8_fp8_bf16_nt_masked(lhs: Tuple[torch.Tensor, torch.Tensor]
 
     if m == 0 or num_groups == 0:
         return
-    flop = 2.0 * num_groups * min(expected_m, m) * n * k
+    flop, given_scales = 2.0 * num_groups * min(expected_m, m) * n * k, lhs_scales
     if flop >= SCALE_RELAYOUT_MIN_FLOP:
         lhs_scales = scales_for_kernel(lhs_scales, flop, grouped_kernel_plan('GroupedMasked', num_groups, min(expected_m, m), n, k, get_num_sms())[1])
     _launch('GroupedMasked', num_groups, min(expected_m, m), m, n, k, lhs, lhs_scales, rhs, rhs_scales, out, masked_m,
-            (lhs_scales.stride(1), lhs_scales.stride(2), lhs_scales.stride(0), min(expected_m, m)), flop, (MASKED, expected_m))
+            (lhs_scales.stride(1), lhs_scales.stride(2), lhs_scales.stride(0), min(expected_m, m)), flop, (MASKED, expected_m) if lhs_scales is given_scales else None)
