@@ -454,6 +454,65 @@ def test_floats_that_do_not_come_apart_take_the_fp32_cores(tile, parts):
         assert bool(((c.double() - want).abs() <= bound)[~beyond].all())
 
 
+@pytest.mark.parametrize('tile,parts', [((256, 256), 1), ((128, 128), 5), ((128, 64), 7)])
+def test_k_tiles_that_do_not_come_apart_are_added_once(tile, parts):
+    """From the first such k-tile on the fp32 cores go on: in the first and the last, in neighbours, in one wave's step of a k-tile and in
+    several, in either operand. One row (column) holds nothing but numbers that do not come apart, so that each of them is seen in the sum; the
+    others see a k-tile that is left out or added twice."""
+    m, n, k = 256, 256, 700
+    for places in ([0], [k - 1], [15, 16], [300], [64, 150], [131, 132, 200], list(range(0, k, 97)), list(range(k))):
+        for swapped in (False, True):
+            _announce('k-tiles that do not come apart', tile, parts, places[:3], swapped)
+            a, b, c = testing.make_float_case(m, n, k, seed=29, device='cuda')
+            a[5] = 0.0
+            a[5, places] = 2.0 ** -125 * (1.0 + 2.0 ** -20 * torch.arange(1, len(places) + 1, device='cuda'))
+            b *= 2.0 ** 60
+            if swapped:
+                a, b = b, a
+            results = []
+            for _ in range(2):
+                c.fill_(float('nan'))
+                _run_float_bf16x3(tile, parts, a, b, c)
+                results.append(c.clone())
+            assert torch.equal(results[0], results[1])
+            ad, bd = a.double(), b.double()
+            bound = (k + 16) * 2.0 ** -24 * (ad.abs() @ bd.abs().t()) * 2
+            assert bool(((c.double() - ad @ bd.t()).abs() <= bound).all())
+
+
+def test_small_numbers_cost_no_second_run_of_their_tiles():
+    """A number that does not come apart in every row: the entry takes about the time of the fp32 cores (measured 1.05 of it, 1.7 when such tiles
+    were run on both), and about its own where it is the last k-tile's."""
+    from yan_amd.jit_kernels import simple_gemm
+    m, n, k = 4096, 4096, 1024
+    _announce('time of small numbers', m, n, k)
+    a, b, c = testing.make_float_case(m, n, k, seed=31, device='cuda')
+    name, keys, arg_defs = simple_gemm.float_kernel_plan(m, n, 256)
+    fp32 = jit.build(name, arg_defs, jit.generate(simple_gemm.includes, arg_defs, jit.cpp_format(simple_gemm.template, keys)))
+
+    def microseconds(run):
+        times = []
+        for _ in range(12):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            for _ in range(5):
+                run()
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end) * 200)
+        return sorted(times)[3]
+
+    entry = lambda: yan.gemm_float_nt(a, b, c)
+    cores = microseconds(lambda: fp32(m, n, k, 1.0, a, m, b, n, 0.0, c, n, torch.cuda.current_stream()))
+    usual = microseconds(entry)
+    a[:, -1] = 3e-36
+    late = microseconds(entry)
+    a[:, 0] = 3e-36
+    early = microseconds(entry)
+    print(f'fp32 cores {cores:.1f} us, entry {usual:.1f}, small numbers in the last k-tile {late:.1f}, in the first {early:.1f}', flush=True)
+    assert early < 1.3 * cores and late < 0.5 * (usual + cores)
+
+
 @pytest.mark.parametrize('m,n,k', [(1024, 1024, 1024), (128, 2112, 7168), (640, 5120, 331)])
 def test_float_on_the_bf16_cores_is_no_further_from_the_product(m, n, k):
     """Against 64 bits the error is no larger than on the fp32 matrix cores, with the same tile's parts of K or without."""
