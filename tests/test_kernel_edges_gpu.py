@@ -386,12 +386,12 @@ def test_activations_quantised_by_the_weight_streaming_kernel(m, n, k):
         assert torch.equal(one.isnan(), two.isnan()) and torch.equal(one.nan_to_num(), two.nan_to_num())
 
 
-def _run_float_bf16x3(tile, parts, a, b, c, alpha=1.0, beta=0.0):
+def _run_float_bf16x3(tile, parts, a, b, c, alpha=1.0, beta=0.0, lda=0, ldb=0):
     from yan_amd.jit_kernels import simple_gemm, split_k
     name, keys, arg_defs = testing.float_bf16x3_explicit_plan(tile, parts)
     kernel = jit.build(name, arg_defs, jit.generate(simple_gemm.bf16x3_includes, arg_defs, jit.cpp_format(simple_gemm.bf16x3_template, keys)))
     stream = torch.cuda.current_stream()
-    args = (a.size(0), b.size(0), a.size(1), alpha, a, a.size(0), b, b.size(0), beta, c, c.size(1), stream)
+    args = (a.size(0), b.size(0), a.size(1), alpha, a, lda or a.size(0), b, ldb or b.size(0), beta, c, c.size(1), stream)
     if parts > 1:
         workspace, _ = split_k.split_k_workspace(c.device, stream.cuda_stream)
         args += (workspace, split_k.SPLIT_K_WORKSPACE_BYTES)
@@ -417,6 +417,22 @@ def test_float_on_the_bf16_cores_matches_the_product(tile, parts, shape):
         assert torch.equal(results[0][:m], results[1][:m])
         assert bool(((results[0][:m].double() - want).abs() <= bound).all())
         assert torch.equal(results[0][m], start[m]) if beta else bool(results[0][m].isnan().all())
+
+
+@pytest.mark.parametrize('tile,parts,shape', testing.FLOAT_BF16X3_CASES)
+def test_what_lies_beside_the_operands_stays_out_of_the_bf16_cores(tile, parts, shape):
+    """Leading dimensions beyond m and n with NaN or numbers that do not come apart behind the rows: the bits of operands without padding. (A
+    tile that had gone to the fp32 cores for it would round otherwise.)"""
+    m, n, k = shape
+    _announce('fp32 on bf16 cores, padded', tile, parts, shape)
+    a, b, want = testing.make_float_case(m, n, k, seed=37, device='cuda')
+    _run_float_bf16x3(tile, parts, a, b, want)
+    for junk in (float('nan'), 3e-36):
+        wide_a, wide_b = (torch.full((k, rows + pad), junk, device='cuda') for rows, pad in ((m, 260), (n, 252)))
+        wide_a[:, :m], wide_b[:, :n] = a.t(), b.t()
+        got = torch.full((m + 1, n), 7.0, device='cuda')
+        _run_float_bf16x3(tile, parts, wide_a.t()[:m], wide_b.t()[:n], got[:m], lda=m + 260, ldb=n + 252)
+        assert torch.equal(got[:m], want) and bool((got[m:] == 7.0).all())
 
 
 @pytest.mark.parametrize('tile,parts', [((256, 256), 1), ((128, 128), 5), ((128, 64), 7)])

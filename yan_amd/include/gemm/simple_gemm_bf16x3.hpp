@@ -106,8 +106,10 @@ float_gemm_split_body(const float* __restrict__ A, const float* __restrict__ B, 
     const __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(B, k_end > 0 ? (uint32_t(k_end - 1) * uint32_t(ldB) + uint32_t(n)) * 4u : 0u);
     constexpr int A_LANES = BLOCK_M / 4, B_LANES = BLOCK_N / 4;
     constexpr int A_ROWS = kWaveSize / A_LANES, B_ROWS = kWaveSize / B_LANES;
-    const uint32_t voff_a = (uint32_t(lane / A_LANES) * uint32_t(ldA) + uint32_t(m0 + (lane % A_LANES) * 4)) * 4u;
-    const uint32_t voff_b = (uint32_t(lane / B_LANES) * uint32_t(ldB) + uint32_t(n0 + (lane % B_LANES) * 4)) * 4u;
+    // rows past m and n read as zero: what lies there (padding, another matrix) could be NaN and send the tile to the fp32 cores
+    const int row_a = m0 + (lane % A_LANES) * 4, row_b = n0 + (lane % B_LANES) * 4;
+    const uint32_t voff_a = row_a < m ? (uint32_t(lane / A_LANES) * uint32_t(ldA) + uint32_t(row_a)) * 4u : kOutOfRange;
+    const uint32_t voff_b = row_b < n ? (uint32_t(lane / B_LANES) * uint32_t(ldB) + uint32_t(row_b)) * 4u : kOutOfRange;
     auto copy_op = [&](int d, int kt, uint8_t* stage) {
         const int q = d * Cfg::NUM_WAVES + wave;
         if (d < Cfg::A_COPIES / Cfg::NUM_WAVES) {
