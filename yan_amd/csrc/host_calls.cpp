@@ -1,5 +1,5 @@
 // The host side of a repeated call, in native code: a GEMM entry point that has served a call once (yan_amd/jit_kernels) leaves here what
-// its launch takes, under the sizes, strides, types and devices of its tensors and its plain arguments. A later call that agrees in all of
+// its launch takes, under the sizes, strides, types, devices and alignment of its tensors and its plain arguments. A later call that agrees in all of
 // them would pass the same checks and make the same launch from other addresses; it is made from here. Everything else, and whatever could
 // have changed the plan (the compute-unit cap, the environment switches, another stream's workspace, a capture), goes back to Python.
 //
@@ -99,10 +99,12 @@ bool describe(Call& c, PyObject* const* objs, Py_ssize_t n) {
             const at::Tensor& t = THPVariable_Unpack(o);
             if (t.layout() != at::kStrided || !t.is_cuda() || t.device().index() != c.device) return false;
             const auto sizes = t.sizes(), strides = t.strides();
-            if (!c.put(int64_t(t.scalar_type()) * 64 + int64_t(sizes.size()))) return false;
+            const uint64_t address = reinterpret_cast<uint64_t>(t.data_ptr());
+            // (of an address Python looks at nothing but the alignment, scales_for_kernel)
+            if (!c.put((int64_t(t.scalar_type()) * 64 + int64_t(sizes.size())) * 16 + int64_t(address % 16))) return false;
             for (size_t d = 0; d < sizes.size(); ++d)
                 if (!c.put(sizes[d]) || !c.put(strides[d])) return false;
-            c.address[c.tensors++] = reinterpret_cast<uint64_t>(t.data_ptr());
+            c.address[c.tensors++] = address;
         } else if (PyFloat_CheckExact(o)) {
             if (c.num_floats == kMaxFloats || !c.put(-7)) return false;
             c.floats[c.num_floats++] = float(PyFloat_AS_DOUBLE(o));

@@ -228,8 +228,7 @@ def gemm_fp8_fp8_bf16_nt(lhs: Tuple[torch.Tensor, torch.Tensor],
     if rc != 0 and workspace_token is not None:
         split_k_launch_failed(workspace_token)
     assert rc == 0, f'{name} failed with HIP error {rc}'
-    # (what `scales_for_kernel` does with a large problem's other layouts is decided by the addresses of each call; a copy's call never comes back)
-    if lhs_scales is given_scales and (flop < SCALE_RELAYOUT_MIN_FLOP or token_contiguous):
+    if lhs_scales is given_scales:          # the call of a copy never comes back
         remember_call((FP8, lhs, lhs_scales, rhs, rhs_scales, out), name, runtime, args, workspace)
 
 

@@ -77,7 +77,7 @@ def grouped_kernel_plan(gemm_type: str, num_groups: int, m: int, n: int, k: int,
     return name, keys, arg_defs, keys['NUM_STAGES'] * (block_m + block_n) * 128
 
 
-def _launch(gemm_type, num_groups, plan_m, m, n, k, lhs, lhs_scales, rhs, rhs_scales, out, layout, strides, flop, call):
+def _launch(gemm_type, num_groups, plan_m, m, n, k, lhs, lhs_scales, rhs, rhs_scales, out, layout, strides, call):
     # `strides`: the three strides of the activation scales, then expected_m (masked layout; 0 otherwise)
     num_sms = get_num_sms()
     name, keys, defs, smem_size = grouped_kernel_plan(gemm_type, num_groups, plan_m, n, k, num_sms)
@@ -86,9 +86,7 @@ def _launch(gemm_type, num_groups, plan_m, m, n, k, lhs, lhs_scales, rhs, rhs_sc
                                          template=rows_on_device_template if 'ROWS' in keys else template, args=args)
     rc = runtime(*args)
     assert rc == 0, f'{name} failed with HIP error {rc}'
-    # (what `scales_for_kernel` does with a large problem's other layouts is decided by the addresses of each call; a copy's call, None here,
-    # never comes back)
-    if call is not None and (flop < SCALE_RELAYOUT_MIN_FLOP or (lhs_scales.stride(-2) == 1 and lhs_scales.stride(-1) == lhs_scales.size(-2))):
+    if call is not None:            # the call of a copy never comes back
         remember_call((call[0], lhs, lhs_scales, rhs, rhs_scales, out, layout, *call[1:]), name, runtime, args)
 
 
@@ -131,7 +129,7 @@ def m_grouped_gemm_fp8_fp8_bf16_nt_contiguous(lhs: Tuple[torch.Tensor, torch.Ten
     if flop >= SCALE_RELAYOUT_MIN_FLOP:
         lhs_scales = scales_for_kernel(lhs_scales, flop, grouped_kernel_plan('GroupedContiguous', num_groups, m, n, k, get_num_sms())[1])
     _launch('GroupedContiguous', num_groups, m, m, n, k, lhs, lhs_scales, rhs, rhs_scales, out, m_indices,
-            (lhs_scales.stride(0), lhs_scales.stride(1), 0, 0), flop, (CONTIGUOUS, ) if lhs_scales is given_scales else None)
+            (lhs_scales.stride(0), lhs_scales.stride(1), 0, 0), (CONTIGUOUS, ) if lhs_scales is given_scales else None)
 
 
 def m_grouped_gemm_fp8_fp8_bf16_nt_masked(lhs: Tuple[torch.Tensor, torch.Tensor],
@@ -173,4 +171,4 @@ def m_grouped_gemm_fp8_fp8_bf16_nt_masked(lhs: Tuple[torch.Tensor, torch.Tensor]
     if flop >= SCALE_RELAYOUT_MIN_FLOP:
         lhs_scales = scales_for_kernel(lhs_scales, flop, grouped_kernel_plan('GroupedMasked', num_groups, min(expected_m, m), n, k, get_num_sms())[1])
     _launch('GroupedMasked', num_groups, min(expected_m, m), m, n, k, lhs, lhs_scales, rhs, rhs_scales, out, masked_m,
-            (lhs_scales.stride(1), lhs_scales.stride(2), lhs_scales.stride(0), min(expected_m, m)), flop, (MASKED, expected_m) if lhs_scales is given_scales else None)
+            (lhs_scales.stride(1), lhs_scales.stride(2), lhs_scales.stride(0), min(expected_m, m)), (MASKED, expected_m) if lhs_scales is given_scales else None)
