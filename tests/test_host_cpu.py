@@ -26,6 +26,17 @@ def test_get_col_major_tensor():
         yan.get_col_major_tensor(torch.zeros(3))
 
 
+def test_col_major_copies_of_matrices_are_those_of_batches():
+    """A matrix is laid out as the only one of a batch is, whatever strides and sizes it comes with."""
+    for rows in (0, 1, 2, 7):
+        for cols in (0, 1, 3, 8):
+            x = torch.randn(rows, 2 * cols + 1)
+            for m in (x[:, :cols], x[:, ::2][:, :cols], torch.randn(cols, rows).t(), torch.randn(1, cols).expand(rows, cols), torch.randn(rows, cols)):
+                got, want = yan.get_col_major_tensor(m), yan.get_col_major_tensor(m.unsqueeze(0)).squeeze(0)
+                assert got.shape == want.shape and got.stride() == want.stride() and torch.equal(got, want)
+                assert (got is m) == (m.stride() == (1, rows))
+
+
 def test_tile_heuristics_fill_256_cus():
     # the headline FP8 shape: 256x256 tiles give 448 workgroups = 1.75 rounds
     assert heuristics.get_best_fp8_config(4096, 7168, 7168, 256) in ((256, 256), (256, 128), (128, 256))

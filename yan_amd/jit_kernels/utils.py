@@ -80,11 +80,9 @@ def get_col_major_tensor(x: torch.Tensor) -> torch.Tensor:
     contiguous; `x` itself when it already is (reference: utils.py:58-85). The FP8 kernel reads activation
     scales in this layout: one K-block's scales for consecutive tokens sit next to each other."""
     assert x.dim() in (2, 3)
-    batched = x if x.dim() == 3 else x.unsqueeze(0)
-    rows = batched.shape[1]
-    if not (batched.stride(1) == 1 and batched.stride(2) == rows):
-        batched = batched.transpose(1, 2).contiguous().transpose(1, 2)
-    return batched if x.dim() == 3 else batched.squeeze(0)
+    if x.stride(-2) == 1 and x.stride(-1) == x.size(-2):
+        return x
+    return x.transpose(-2, -1).contiguous().transpose(-2, -1)
 
 
 # From this much arithmetic on (about 40 us of kernel time) a GEMM whose activation scales are not token-contiguous gets a
