@@ -247,6 +247,10 @@ FLOAT_BF16X3_CASES = [((256, 256), 1, (300, 260, 1)), ((256, 256), 1, (256, 516,
                       ((128, 64), 1, (4, 4, 16)), ((128, 64), 1, (132, 68, 64)), ((128, 64), 7, (128, 2112, 1000)), ((128, 64), 15, (256, 64, 200))]
 
 
+# fp32 problems whose plan on the fp32 cores cuts K by four waves, by parts, or both, where the fastest tiles on the bf16 cores do not
+FLOAT_ERROR_SHAPES = [(1024, 4224, 300), (3456, 2496, 481), (2048, 2176, 3000), (512, 1216, 4741), (896, 4928, 3543), (128, 2112, 7168), (1024, 1024, 1024)]
+
+
 def float_bf16x3_explicit_plan(tile, parts):
     """(name, keys, arg_defs) of the fp32 kernel on the bf16 matrix cores with this tile and split."""
     from yan_amd.jit_kernels import simple_gemm
@@ -647,7 +651,13 @@ def jit_kernels_in_use(num_cus: int = 256):
         plan = simple_gemm.float_split_k_plan(m, n, k, num_cus)
         if plan is not None:
             add(plan[0], plan[2], simple_gemm.includes, simple_gemm.split_k_template, plan[1])
-    for m, n, k in list(FLOAT_SPLIT_K_SHAPES) + REFERENCE_FLOAT_TEST_SHAPES + FLOAT_TEST_SHAPES + [(5120, 2048, 4096), (4096, 4096, 1024), (8192, 8192, 8192)]:
+    for m, n, k in FLOAT_ERROR_SHAPES:
+        for plan, code_template in ((simple_gemm.float_split_k_plan(m, n, k, num_cus), simple_gemm.split_k_template),
+                                    (simple_gemm.float_kernel_plan(m, n, num_cus), simple_gemm.template)):
+            if plan is not None:
+                add(plan[0], plan[2], simple_gemm.includes, code_template, plan[1])
+    for m, n, k in (list(FLOAT_SPLIT_K_SHAPES) + REFERENCE_FLOAT_TEST_SHAPES + FLOAT_TEST_SHAPES + FLOAT_ERROR_SHAPES
+                    + [(5120, 2048, 4096), (4096, 4096, 1024), (8192, 8192, 8192)]):
         plan = simple_gemm.float_bf16x3_plan(m, n, k, num_cus)
         if plan is not None:
             add(plan[0], plan[2], simple_gemm.bf16x3_includes, simple_gemm.bf16x3_template, plan[1])

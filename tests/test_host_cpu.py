@@ -750,6 +750,24 @@ def test_fp32_plans_on_the_bf16_cores_fit_their_workspace():
                     assert simple_gemm.float_bf16x3_plan(m, n, k, 256)[2] is (simple_gemm.split_k_arg_defs if plan[2] > 1 else simple_gemm.arg_defs)
 
 
+def test_fp32_plans_on_the_bf16_cores_cut_k_as_the_fp32_cores_would():
+    """The rounding of a sum grows with what is added up in a row: K is cut (by waves that share it, by parts) no less often than by the plan on the
+    fp32 cores."""
+    waves = {(256, 256): 1, (256, 128): 2, (128, 256): 2, (128, 128): 4, (128, 64): 4}
+    checked = 0
+    for m in range(128, 4097, 384):
+        for n in range(256, 8193, 448):
+            for k in (257, 300, 690, 1255, 3543, 8191):
+                for may_split in (True, False):
+                    plan = heuristics.get_float_bf16x3_config(m, n, k, 256, may_split)
+                    if plan is None:
+                        continue
+                    on_fp32 = (may_split and heuristics.get_split_k_float_config(m, n, k, 256)) or (*heuristics.get_best_float_config(m, n, 256), 1)
+                    assert waves[plan[:2]] * plan[2] >= (4 if on_fp32[0] < 128 else 1) * on_fp32[2], (m, n, k, plan, on_fp32)
+                    checked += 1
+    assert checked > 1500
+
+
 @pytest.mark.parametrize('kind,streams_codes', [('per_token', False), ('per_block', True)])
 def test_codes_of_activations_are_stored_for_the_gemm_behind(tmp_path, kind, streams_codes):
     """The GEMM that follows a per-token cast reads its codes from the caches: no store of them carries the non-temporal hint.

@@ -552,6 +552,37 @@ def test_float_on_the_bf16_cores_is_no_further_from_the_product(m, n, k):
         assert after <= before
 
 
+@pytest.mark.parametrize('m,n,k', testing.FLOAT_ERROR_SHAPES)
+def test_float_entry_is_no_further_from_the_product_than_the_fp32_cores(m, n, k):
+    """The entry's own plan on the bf16 cores against the plan that the fp32 cores would run, split or not: the error against 64 bits is no larger."""
+    from yan_amd.jit_kernels import simple_gemm, split_k
+    _announce('fp32 error of the entry', m, n, k)
+    assert simple_gemm.float_bf16x3_plan(m, n, k, 256) is not None
+    split = simple_gemm.float_split_k_plan(m, n, k, 256)
+    name, keys, arg_defs = split or simple_gemm.float_kernel_plan(m, n, 256)
+    code_template = simple_gemm.split_k_template if split else simple_gemm.template
+    fp32 = jit.build(name, arg_defs, jit.generate(simple_gemm.includes, arg_defs, jit.cpp_format(code_template, keys)))
+    stream = torch.cuda.current_stream()
+    for kind in ('normal', 'positive', 'wide'):
+        a, b, c = testing.make_float_case(m, n, k, seed=41, device='cuda', gen_device='cuda')
+        if kind == 'positive':
+            a, b = a.abs(), b.abs()
+        elif kind == 'wide':
+            a = a * torch.exp(3.0 * torch.randn(k, m, generator=torch.Generator().manual_seed(42)).cuda().t())
+        want = a.double() @ b.double().t()
+        args = (m, n, k, 1.0, a, m, b, n, 0.0, c, n, stream)
+        if split:
+            workspace, _ = split_k.split_k_workspace(c.device, stream.cuda_stream)
+            args += (workspace, split_k.SPLIT_K_WORKSPACE_BYTES)
+        assert fp32(*args) == 0
+        before = ((c.double() - want).norm() / want.norm()).item()
+        c.fill_(float('nan'))
+        yan.gemm_float_nt(a, b, c)
+        after = ((c.double() - want).norm() / want.norm()).item()
+        print(f'{kind}: {before:.2e} -> {after:.2e}', flush=True)
+        assert after <= before
+
+
 def _odd_floats(shape, dtype, seed):
     """Every kind of bit pattern: subnormals, huge values, zeros of both signs, and infinities and NaN here and there."""
     g = torch.Generator().manual_seed(seed)

@@ -434,8 +434,8 @@ def get_split_k_float_config(m: int, n: int, k: int, num_cus: int) -> Optional[T
     return best_plan
 
 
-# The fp32 GEMM on the bf16 matrix cores (gemm/simple_gemm_bf16x3.hpp): depth of a k-tile, microseconds per k-tile while few compute
-# units work, microseconds a tile costs besides (first copies, sums of its waves, epilogue). Fitted, with the rest of the model below, to
+# The fp32 GEMM on the bf16 matrix cores (gemm/simple_gemm_bf16x3.hpp): depth of a k-tile (16 for each of the waves that share K), microseconds
+# per k-tile while few compute units work, microseconds a tile costs besides (first copies, sums of its waves, epilogue). Fitted, with the rest of the model below, to
 # 190 shapes with every tile and split forced in turn, operands cycling: its pick takes 1.015 of the fastest's time on average, 1.13 at
 # worst above the limit.
 _FLOAT_BF16X3_TILES = {(256, 256): (16, 1.16, 9.8), (256, 128): (32, 1.15, 7.0), (128, 256): (32, 1.17, 6.8), (128, 128): (64, 1.18, 6.9),
@@ -449,13 +449,23 @@ FLOAT_BF16X3_MIN_MNK = 1 << 30
 def get_float_bf16x3_config(m: int, n: int, k: int, num_cus: int, may_split: bool = True) -> Optional[Tuple[int, int, int]]:
     """(BLOCK_M, BLOCK_N, SPLIT_K) when the fp32 GEMM should run on the bf16 matrix cores, else None. Modelled time: rounds x (k-tiles of a
     part x the tile's time per k-tile, twice that where every compute unit works (the power limit) + the tile's other costs) + 1.5 us, and
-    for a split 1.8 us + 13 ns per KB of partial sums the last part reads."""
+    for a split 1.8 us + 13 ns per KB of partial sums the last part reads.
+
+    The rounding of a sum grows with the products added up in a row. Sixteen of them are six roundings here and eight on the fp32 cores, so K is
+    cut at least as often as the plan there cuts it, by waves that share it (tiles below 128 rows: four) and by parts: against 64 bits the
+    error is then 0.80 to 0.90 of that plan's (all positive operands 0.66 to 0.99), over 158 shapes where the fastest plan cuts it less often and
+    is 1.07 to 1.73 (1.02 to 2.90) times as far off. What that costs (fp32 cores, fastest plan, this one): 3200 x 4096 x 995 204.5, 132.3, 155.8 us,
+    2048 x 3200 x 866 93.5, 60.9, 66.4, 1920 x 2368 x 318 31.7, 24.3, 31.3; 0.60 to 1.03 of the fp32 cores' time, 0.77 on average."""
     if m * n * k < FLOAT_BF16X3_MIN_MNK:
         return None
+    on_fp32 = (may_split and get_split_k_float_config(m, n, k, num_cus)) or (*get_best_float_config(m, n, num_cus), 1)
+    fp32_ways = on_fp32[2] * (4 if on_fp32[0] < 128 else 1)
     best, plan = None, None
     for (bm, bn), (block_k, per_k_tile, per_tile) in _FLOAT_BF16X3_TILES.items():
         tiles, k_tiles = ceil_div(m, bm) * ceil_div(n, bn), ceil_div(k, block_k)
         for split in FLOAT_BF16X3_SPLIT_FACTORS if may_split else (1,):
+            if split * (block_k // 16) < fp32_ways:
+                continue
             # 16 MB of partial sums, eight counters per tile in 16 KB, two k-tiles per part
             if split > 1 and (tiles * split * bm * bn * 4 > 1 << 24 or tiles > 512 or ceil_div(k_tiles, split) < 2):
                 continue
