@@ -223,6 +223,10 @@ FLOAT_SPLIT_K_SHAPES = {(128, 64, 2050): (32, 32, 7), (256, 320, 3001): (32, 32,
 # shift from row to row (8 and 56 elements a row, 24, 40), K that ends right behind a window and one chunk into it, operands shifted alike and not
 DENSE_LINE_WINDOW_TILES = [((128, 256), 3), ((128, 192), 4), ((128, 128), 5), ((64, 192), 5), ((64, 128), 6)]
 DENSE_LINE_WINDOW_SHAPES = [(131, 260, 264, 0, 0), (70, 132, 312, 8, 40), (257, 388, 328, 56, 0), (64, 68, 424, 24, 24), (130, 516, 1016, 48, 8)]
+# The same with as many workgroups and k-tiles as it takes for a launch to copy lines: 11 x 13 tiles, their last ones ragged. (K, elements the
+# operands start behind a line): every shift from row to row, K that ends in a whole k-tile, operands that start off lines, alike and not
+DENSE_LINE_WINDOW_DEPTHS = [(1224, 0, 0), (1304, 8, 40), (1320, 0, 24), (1336, 56, 0), (1280, 8, 40), (1344, 24, 24)]
+DENSE_LINE_WINDOW_CAP = 136         # workgroups that walk the 143 tiles
 
 
 # The weight-streaming kernel through the entry points: every number of activation atoms on 8, 16, 24, 32, 40, 48 and 64 weight rows per
@@ -663,8 +667,9 @@ def jit_kernels_in_use(num_cus: int = 256):
             add(plan[0], plan[2], simple_gemm.bf16x3_includes, simple_gemm.bf16x3_template, plan[1])
     for tile, _ in DENSE_LINE_WINDOW_TILES + [((64, 64), 8)]:
         for dtype in (torch.bfloat16, torch.half):
-            name, keys, arg_defs, includes, code_template = dense_tile_plan(tile, dtype, 0)
-            add(name, arg_defs, includes, code_template, keys)
+            for cap in (0, DENSE_LINE_WINDOW_CAP):
+                name, keys, arg_defs, includes, code_template = dense_tile_plan(tile, dtype, cap)
+                add(name, arg_defs, includes, code_template, keys)
     for m, n, k in CAST_STREAM_SHAPES:
         name, keys, arg_defs, code_template = gemm.fp8_cast_stream_plan(m, n, k, num_cus)
         add(name, arg_defs, gemm.includes, code_template, keys)

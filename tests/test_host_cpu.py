@@ -314,6 +314,37 @@ def test_tile_scheduler_visits_every_tile_once_and_walks_cover_every_slot(tmp_pa
     assert int(done.stdout.split()[1]) > 400
 
 
+def test_launches_copy_lines_only_where_that_pays(tmp_path):
+    """copies_whole_lines: rows off lines, by K or by where both operands start; half of the chip at work; enough k-tiles for the tile."""
+    import subprocess
+    from yan_amd.jit.compiler import get_hipcc_compiler, get_jit_include_dir
+    source, exe = tmp_path / 'rule.cpp', tmp_path / 'rule'
+    source.write_text("""
+#include "gemm/bf16_gemm.hpp"
+#include <cstdio>
+int main() {
+    int block_m, block_n, parts, groups, k;
+    long a, b;
+    while (std::scanf("%d %d %d %d %d %ld %ld", &block_m, &block_n, &parts, &groups, &k, &a, &b) == 7)
+        std::printf("%d ", int(yan::copies_whole_lines(block_m, block_n, parts, groups, k, reinterpret_cast<void*>(a), reinterpret_cast<void*>(b))));
+}
+""")
+    subprocess.check_call([get_hipcc_compiler()[0], '-x', 'hip', '--cuda-host-only', '-std=c++20', '-O1', '-w', f'-I{get_jit_include_dir()}', str(source),
+                           '-o', str(exe)])
+    cases = {
+        # the tile, parts of K, workgroups, K, where the operands start
+        (64, 128, 1, 136, 600, 4096, 4096): 0, (64, 128, 1, 136, 1272, 4096, 4096): 1, (64, 128, 1, 250, 968, 4096, 4096): 1, (64, 128, 1, 250, 952, 4096, 4096): 0,
+        (64, 128, 1, 120, 4104, 4096, 4096): 0, (64, 192, 1, 190, 520, 4096, 4096): 1, (64, 192, 1, 190, 504, 4096, 4096): 0,
+        (128, 128, 1, 255, 600, 4096, 4096): 0, (128, 128, 1, 255, 712, 4096, 4096): 1, (128, 192, 1, 230, 600, 4096, 4096): 0,
+        (128, 192, 1, 200, 600, 4096, 4096): 1, (64, 128, 3, 216, 4104, 4096, 4096): 1, (64, 128, 4, 216, 4104, 4096, 4096): 1, (64, 128, 4, 216, 3960, 4096, 4096): 0,
+        (64, 128, 4, 216, 4040, 4096, 4096): 1,
+        (128, 192, 1, 200, 4096, 4096, 4096): 0, (128, 192, 1, 200, 4096, 4112, 4096): 0, (128, 192, 1, 200, 4096, 4096, 4112): 0,
+        (128, 192, 1, 200, 4096, 4112, 4128): 1, (128, 192, 1, 200, 4128, 4096, 4096): 0,
+    }
+    done = subprocess.run([str(exe)], input='\n'.join(' '.join(map(str, c)) for c in cases), stdout=subprocess.PIPE, universal_newlines=True, check=True)
+    assert dict(zip(cases, map(int, done.stdout.split()))) == cases
+
+
 @pytest.mark.parametrize('shape,dtype_name', [((8192, 8192, 8192), 'bfloat16'), ((4096, 5120, 5120), 'bfloat16'), ((8192, 8192, 8192), 'half')])
 def test_tied_accumulators_of_the_8_wave_kernel_stay_where_the_mfmas_left_them(tmp_path, shape, dtype_name):
     """The 8-wave dense kernel writes its MFMAs as asm statements whose destination is their own addend. The compiler does

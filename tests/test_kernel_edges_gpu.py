@@ -332,6 +332,28 @@ def test_rows_off_cache_lines_give_the_bits_of_the_smallest_tile(tile, stages, d
         assert bool(((got[:m].double() - ref).abs() <= bound).all())
 
 
+@pytest.mark.parametrize('cap', [0, testing.DENSE_LINE_WINDOW_CAP])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.half])
+@pytest.mark.parametrize('tile', [tile for tile, _ in testing.DENSE_LINE_WINDOW_TILES])
+def test_launches_that_copy_lines_give_the_bits_of_the_smallest_tile(tile, dtype, cap):
+    """Sizes from which ring tiles copy lines, a workgroup per tile and fewer of them that walk the tiles."""
+    def kernel(which, workgroups):
+        name, keys, arg_defs, includes, code_template = testing.dense_tile_plan(which, dtype, workgroups)
+        return jit.build(name, arg_defs, jit.generate(includes, arg_defs, jit.cpp_format(code_template, keys)))
+    lines, plain = kernel(tile, cap), kernel((64, 64), 0)
+    m, n = 11 * tile[0] - 5, 13 * tile[1] - 4
+    for k, off_a, off_b in testing.DENSE_LINE_WINDOW_DEPTHS:
+        _announce('launches that copy lines', tile, dtype, cap, k, off_a, off_b)
+        g = torch.Generator(device='cuda').manual_seed(29)
+        a_buf, b_buf = (torch.randn(rows * k + off + 64, generator=g, device='cuda').to(dtype) for rows, off in ((m, off_a), (n, off_b)))
+        a_buf[:off_a], a_buf[off_a + m * k:], b_buf[:off_b], b_buf[off_b + n * k:] = (float('nan'),) * 4
+        a, b = a_buf[off_a:off_a + m * k].view(m, k), b_buf[off_b:off_b + n * k].view(n, k)
+        got, want = (torch.full((m + 2, n), 7.0, dtype=dtype, device='cuda') for _ in range(2))
+        stream = torch.cuda.current_stream()
+        assert lines(m, n, k, a, b, got[:m], stream) == 0 and plain(m, n, k, a, b, want[:m], stream) == 0
+        assert torch.equal(got, want) and bool((got[m:] == 7.0).all())
+
+
 @pytest.mark.parametrize('m,n,k', testing.WEIGHT_STREAM_SHAPES)
 def test_weight_streaming_kernel_at_the_edges_of_its_tiles(m, n, k):
     """FP8 with both layouts of the activation scales, bf16 and fp16, through the entry points, against the product in float64; the

@@ -958,19 +958,27 @@ inline hipError_t check_dense_args(int m, int n, int k, const void* a, const voi
 // halves of lines it gains 0 to 10 % and loses as much (512 x 4096 x 4128 on 64 x 128 30.5 -> 27.5 us, 200 x 5000 x 2976 on 128 x 128 22.3 ->
 // 24.9), elsewhere it takes 0.79 to 1.0 of the time (1111 x 5004 x 2056 on 128 x 192 35.5 -> 32.0, on 64 x 192 45.6 -> 37.7, 512 x 4096 x 4104
 // on 64 x 128 31.1 -> 26.7, 2000^2 x 2008 on 128 x 128 24.7 -> 22.3); the 64 x 64 tile, whose k-tiles are too short for where its chunks lie
-// to be worked out beside them, takes up to 1.04 and keeps its copies, as do the 256-row rings.
-inline bool copies_whole_lines(int k, const void* a, const void* b) {
-    return k >= 256 && ((uintptr_t(k) * 2) | reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) % 64 != 0;
+// to be worked out beside them, takes up to 1.04 and keeps its copies, as do the 256-row rings (with_dense_copies).
+// What it gains are requests for lines, what it costs is a longer way from a barrier to the first fragment: it loses where few
+// workgroups leave the memory idle (48 of them, K = 600: 1.07 to 1.13 of the time) and where K is short. The least k-tiles are from 970 shapes,
+// time of the k-tile copies = 1: 64 x 128 tiles, up to 192 workgroups, 8 to 16 k-tiles 0.96 to 1.08 (worst 1.12), from 20 on 0.89; more workgroups 8 to
+// 14 0.98 to 1.05, from 16 on 0.90; 64 x 192 8 to 12 0.93 to 0.97; 128 x 128 8 to 12 0.95 to 1.03 (worst 1.27), 12 to 16 0.94; 128 x 192 up to 224
+// workgroups 0.94, more 8 to 16 0.99 to 1.03 (worst 1.12). Operands with one of them off its lines pay for both (K = 4096, 1.02 to 1.08), and 128 x 128
+// in four parts, without waves that only copy, takes 0.94 to 1.08.
+inline bool copies_whole_lines(int block_m, int block_n, int split_k, int workgroups, int k, const void* a, const void* b) {
+    const int k_tiles = ceil_div(k, 64) / split_k, area = block_m * block_n;
+    const int least = area == 64 * 128 ? (workgroups >= 192 ? 16 : 20) : area == 64 * 192 ? 9 : area == 128 * 128 ? 12 : workgroups >= 224 ? 16 : 5;
+    const bool off_lines = uintptr_t(k) * 2 % 64 != 0 || (reinterpret_cast<uintptr_t>(a) % 64 != 0 && reinterpret_cast<uintptr_t>(b) % 64 != 0);
+    return off_lines && workgroups >= 128 && k_tiles >= least;
 }
-
 
 // Calls `launch` with the copies (COPIES, a std::integral_constant) of a ring tile's launch. A kernel is compiled for each that a plan
 // can ask for: none for 256-row rings, and no streamed weights in six and eight parts, which have 96 MB of weights from
 // K = 24576 on only.
 template <int BLOCK_M, int BLOCK_N, int SPLIT_K, typename Launch>
-inline void with_dense_copies(int tiles_m, int m, int n, int k, const void* a, const void* b, Launch&& launch) {
-    if constexpr (BLOCK_M < 256 && BLOCK_M * BLOCK_N > 64 * 64 && SPLIT_K <= 4)
-        if (copies_whole_lines(k, a, b)) return launch(std::integral_constant<int, kLineWindows>{});
+inline void with_dense_copies(int tiles_m, int workgroups, int m, int n, int k, const void* a, const void* b, Launch&& launch) {
+    if constexpr (BLOCK_M < 256 && BLOCK_M * BLOCK_N > 64 * 64 && SPLIT_K <= 4 && dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) == 8)
+        if (copies_whole_lines(BLOCK_M, BLOCK_N, SPLIT_K, workgroups, k, a, b)) return launch(std::integral_constant<int, kLineWindows>{});
     const uint64_t weight_bytes = uint64_t(n) * k * 2;
     const bool streamed = streams_weights(tiles_m, weight_bytes, k * 2), spread = spreads_starts(tiles_m, m, weight_bytes, k, SPLIT_K);
     if constexpr (BLOCK_M < 256 && SPLIT_K <= 4) {
@@ -1032,7 +1040,7 @@ inline hipError_t launch_dense(int m, int n, int k, const void* a, const void* b
                                    dim3(dense_launch_waves(BLOCK_M, BLOCK_N) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
                                    static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, slots);
         };
-        with_dense_copies<BLOCK_M, BLOCK_N, 1>(sched.tiles_m, m, n, k, a, b, launch);
+        with_dense_copies<BLOCK_M, BLOCK_N, 1>(sched.tiles_m, grid, m, n, k, a, b, launch);
     }
     return hipGetLastError();
 }
@@ -1065,7 +1073,7 @@ inline hipError_t launch_dense_split_k(int m, int n, int k, const void* a, const
                                dim3(dense_launch_waves(BLOCK_M, BLOCK_N, SPLIT_K) * kWaveSize), 0, stream, static_cast<const uint8_t*>(a),
                                static_cast<const uint8_t*>(b), static_cast<Elem*>(c), m, n, k, partials, counters);
     };
-    with_dense_copies<BLOCK_M, BLOCK_N, SPLIT_K>(sched.tiles_m, m, n, k, a, b, launch);
+    with_dense_copies<BLOCK_M, BLOCK_N, SPLIT_K>(sched.tiles_m, int(slots) * SPLIT_K, m, n, k, a, b, launch);
     return hipGetLastError();
 }
 
