@@ -117,7 +117,8 @@ StreamPull weight_stream_pull(int m, int n, long long k_bytes, int num_cus) {
 int weight_stream_fp8_atoms(int m, int n, int k, int num_cus) {
     const auto [pull, rows, groups] = weight_stream_pull(m, n, k, num_cus);
     const bool full = rows >= 16 && groups * 8 >= num_cus * 7, wide = rows >= 24;
-    const bool takes = m <= 32   ? pull <= 400000 || full || n >= 16 * num_cus
+    const bool takes = m <= 16 && rows == 64 ? pull <= 800000
+                       : m <= 32 ? pull <= (rows == 8 && m > 16 ? 285000 : 400000) || full || n >= 16 * num_cus
                        : m <= 40 ? pull <= 400000 || full || wide
                        : m <= 48 ? pull <= (wide ? 400000 : 300000) || (rows == 32 && full)
                                  : pull <= (rows == 24 ? 365000 : 130000);
@@ -126,12 +127,12 @@ int weight_stream_fp8_atoms(int m, int n, int k, int num_cus) {
 int weight_stream_dense_atoms(int m, int n, int k, int num_cus) {
     const auto [pull, rows, groups] = weight_stream_pull(m, n, 2ll * k, num_cus);
     const bool full = groups * 8 >= num_cus * 7;
-    const long long share = 3000000ll * groups / num_cus - 1490000;
-    const long long limit = rows <= 16   ? (rows == 16 && full ? 580000 : 450000)
-                            : rows == 24 ? (m <= 16 ? 1400000 : share < 850000 ? share : 850000)
-                            : rows == 32 ? (full ? 780000 : 600000)
-                                         : (rows == 64 ? 600000 : 1400000);
-    return pull && (pull <= limit || (m <= 16 && (rows <= 16 || rows == 32))) ? (m + 15) / 16 : 0;
+    const long long limit = rows <= 16   ? (rows == 16 && full && m <= 32 ? 580000 : 450000)
+                            : rows == 24 ? (m <= 16 ? (full ? 850000 : 700000) : m <= 32 ? (full ? 850000 : 500000) : full ? 450000 : 350000)
+                            : rows == 32 ? (m <= 16 ? 750000 : m > 48 ? 450000 : full ? 780000 : 600000)
+                            : rows == 64 ? (m <= 16 ? 440000 : k >= 2048 ? 600000 : 0)
+                                         : (rows == 48 && m <= 16 ? 830000 : 1200000);
+    return pull && (pull <= limit || (m <= 16 && rows <= 16)) ? (m + 15) / 16 : 0;
 }
 
 // Whether a workspace holds what a split-K plan needs (launch_dense_split_k, Gemm::run_split_k): asked for also where the

@@ -204,8 +204,9 @@ def get_weight_stream_fp8_config(m: int, n: int, k: int, num_cus: int) -> int:
     more matrices than the caches hold, 60 shapes of n = 128 .. 16384, k = 512 .. 16384, up to ten m each (split-K plan or tiles -> this
     kernel): 1 x 2112 x 7168 8.7 -> 5.4 us, 1 x 4096 x 7168 9.8 -> 7.6, 16 x 1984 x 4608 6.7 -> 4.5, 32 x 2944 x 5632 10.3 -> 7.8,
     40 x 4096 x 16384 22.3 -> 19.8, 8 x 10240 x 7168 22.5 -> 15.0, 32 x 16384 x 16384 53.8 -> 47.5. It loses
-    up to 40 rows only where a workgroup of 8 or 16 weight rows pulls more than 400 KB and they do not fill the chip
-    (20 x 1472 x 15104 10.9 -> 11.3); with 48 rows it is level from 300 KB on (4096 x 7168 11.1 -> 11.3), 400 KB on more weight rows
+    up to 40 rows only where a workgroup of 8 or 16 weight rows pulls more than 400 KB (8 weight rows from 17 rows on: 285 KB, 25 x 1856 x 9728
+    8.1 -> 8.7) and they do not fill the chip (20 x 1472 x 15104 10.9 -> 11.3), and up to 16 rows on 64 weight rows beyond 800 KB (10 x 13184 x 11264
+    30.0 -> 30.9); with 48 rows it is level from 300 KB on (4096 x 7168 11.1 -> 11.3), 400 KB on more weight rows
     (4100 x 7168 12.2 at 516 KB both ways, but 8192 x 4096 11.1 -> 10.1); with 64 from 130 KB on (4096 x 2048 4.7 -> 4.8;
     3072 x 1536 4.5 -> 4.2; 2112 x 7168 10.3 -> 12.2; 7168 x 2048 7.1 both ways), on 24 weight rows 365 KB (4224 x 4096
     10.5 -> 9.5; 5120 x 8192 14.2 -> 16.2 at 721 KB). Same rule as `weight_stream_fp8_atoms` in yan_amd/csrc/yan_gemm_capi.hip."""
@@ -214,7 +215,9 @@ def get_weight_stream_fp8_config(m: int, n: int, k: int, num_cus: int) -> int:
     if not pull:
         return 0
     if m <= 32:
-        takes = pull <= 400_000 or full or n >= 16 * num_cus
+        takes = pull <= (285_000 if rows == 8 and m > 16 else 400_000) or full or n >= 16 * num_cus
+        if rows == 64 and m <= 16:
+            takes = pull <= 800_000
     elif m <= 40:
         takes = pull <= 400_000 or full or wide
     elif m <= 48:
@@ -227,28 +230,28 @@ def get_weight_stream_fp8_config(m: int, n: int, k: int, num_cus: int) -> int:
 @functools.lru_cache(maxsize=None)
 def get_weight_stream_dense_config(m: int, n: int, k: int, num_cus: int) -> int:
     """The same for the dense 16-bit GEMM, whose smallest tile holds 64 weight rows: while a workgroup pulls no more than a limit that
-    depends on its weight rows and on how much of the chip they fill. 8 and 16 weight rows: 450 KB (40 x 1984 x 4608 10.8 -> 10.3 us at
-    442 KB, 48 rows 11.1 -> 11.0 at 516 KB, 32 x 1024 x 7168 11.1 -> 11.7 at 573 KB), 580 KB where they fill the chip (24 x 4096 x 7168
-    15.9 -> 15.2 at 573 KB, 32 rows 16.2 -> 16.4 at 688 KB). 24: 510 KB for two thirds of the chip up to 850 KB (40 x 4224 x 4096 12.0 -> 12.1 at
-    524 KB, 24 x 4100 x 7168 16.7 -> 16.5 at 688 KB, 32 x 5120 x 8192 21.5 -> 19.5 at 918 KB, 40 rows 21.6 -> 21.4). 32: 600 KB, full
-    780 KB (64 x 8192 x 4096 19.7 -> 18.8 at 786 KB, 24 x 7168 x 7168 22.2 -> 22.1 at 860 KB, 32 x 8192 x 7168 24.0 -> 24.6 at 917 KB). 40, 48:
-    1.4 MB (32 x 10240 x 7168 33.3 -> 28.2, 32 x 12288 x 8192 36.5 -> 36.0, 1 x 8256 x 16384 49.2 -> 46.9; 24 rows there 48.4 both ways).
-    64: 600 KB (32 x 14336 x 2048 15.4 -> 13.0; 12 x 16384 x 4096 27.2 -> 28.1 at 623 KB). Up to 16 rows also beyond: 24 weight rows
-    1.4 MB (16 x 4100 x 16384 30.7 -> 28.3), 8, 16 and 32 on any K (1 x 1024 x 7168 12.7 -> 5.5, 16 x 1472 x 15104 31.1 -> 16.7,
-    16 x 2112 x 7168 11.5 -> 11.6, the closest). Same rule as `weight_stream_dense_atoms` in yan_amd/csrc/yan_gemm_capi.hip."""
+    depends on its weight rows, on m and on how much of the chip they fill. The limits are from 2000 shapes of n = 1024 .. 16384, k = 1024 ..
+    16384, weights cycling (time here : time of split-K plan or tiles): there and below it is 0.70 to 1.02 (0.81 on average over 700 other shapes in
+    the upper half of the limits, three above 1.03), beyond, on 24 weight rows, 0.97 to 1.11 (14 x 4428 x 15360 26.0 -> 28.9 us, 17 x 4736 x 8832 19.6 ->
+    21.8), on 32 1.0 to 1.12 (6 x 7992 x 15872 40.5 -> 45.6), on 48 0.86 to 1.10 (4 x 12288 x 8192 33.3 -> 36.5), on 64 1.04 to 1.10 (1 x 15116 x 4608
+    23.0 -> 25.3, and 30 x 13888 x 1408 9.9 -> 10.3), with 33 to 64 rows 1.03 to 1.09 (48 x 4096 x 4480 11.7 -> 12.8, 63 x 7872 x 2688 12.9 -> 13.6). Up to 16
+    rows 8 and 16 weight rows go on any K (1 x 1024 x 7168 12.7 -> 5.5, 16 x 1472 x 15104 31.1 -> 16.7, 16 x 2112 x 7168 11.5 -> 11.6, the
+    closest). Same rule as `weight_stream_dense_atoms` in yan_amd/csrc/yan_gemm_capi.hip."""
     pull, rows, groups = _weight_stream_pull(m, n, 2 * k, num_cus)
     full = groups * 8 >= num_cus * 7
     if not pull:
         return 0
     if rows <= 16:
-        limit = 580_000 if rows == 16 and full else 450_000
+        limit = 580_000 if rows == 16 and full and m <= 32 else 450_000
     elif rows == 24:
-        limit = 1_400_000 if m <= 16 else min(850_000, 3_000_000 * groups // num_cus - 1_490_000)
+        limit = (850_000 if full else 700_000) if m <= 16 else (850_000 if full else 500_000) if m <= 32 else 450_000 if full else 350_000
     elif rows == 32:
-        limit = 780_000 if full else 600_000
+        limit = 750_000 if m <= 16 else 450_000 if m > 48 else 780_000 if full else 600_000
+    elif rows == 64:
+        limit = 440_000 if m <= 16 else 600_000 if k >= 2048 else 0
     else:
-        limit = 600_000 if rows == 64 else 1_400_000
-    return ceil_div(m, 16) if pull <= limit or (m <= 16 and rows in (8, 16, 32)) else 0
+        limit = 830_000 if rows == 48 and m <= 16 else 1_200_000
+    return ceil_div(m, 16) if pull <= limit or (m <= 16 and rows <= 16) else 0
 
 
 def get_cast_stream_rows(m: int, n: int, k: int, num_cus: int) -> int:
