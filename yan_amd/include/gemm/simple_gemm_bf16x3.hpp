@@ -20,7 +20,7 @@
 //   cycles. Both kinds of work mixed in every wave were slower: 128 x 128 tiles 0.97 us a k-tile of 32, 0.74 in turns.
 // * What bounds it: with few workgroups 1.48 us for 16 k-rows of a 256 x 256 tile (1.28 are MFMAs at 2.4 GHz), with all 256 compute units at
 //   work 2.1 to 2.5, the power limit. 8192 x 8192 x 4096 3650 -> 2280 us (241 TFLOP/s; the fp32 cores peak at 157), 4096^2 x 2048
-//   522 -> 297, 2048 x 1664 x 7227 427 -> 235, 128 x 2112 x 7168 45 -> 32. Small problems stay on the fp32 cores: a tile here costs 5 to 10 us
+//   522 -> 297, 2048 x 1664 x 7227 427 -> 235, 128 x 2112 x 7168 with beta = 0 45 -> 32. Small problems stay on the fp32 cores: a tile here costs 5 to 10 us
 //   besides its k-tiles (get_float_bf16x3_config).
 #pragma once
 

@@ -6,7 +6,7 @@
 //     has no barrier, only the wave's own counts of copies in flight.
 //   * Whole 128-byte lines are what a compute unit copies fast. Read straight into fragments (16 rows at 16 or 64 bytes per lane
 //     group) operands that sit in L2 come in at 40 bytes/ns per compute unit, 8 rows x 128 bytes at a time at 125 - 190, into registers or
-//     into LDS alike. The kernel that loaded fragments, 1 row, FP8, call to call: 2112 x 7168 9.7 us, this one 5.3 (split K over 3
+//     into LDS alike. The kernel that loaded fragments, 1 row, FP8, weights cycling: 2112 x 7168 9.7 us, this one 5.3 (split K over 3
 //     workgroups per tile, their sums meeting in memory: 8.5); 1024 x 7168 9.3 / 4.5 (7.5); bf16 4096 x 2048 6.9 / 4.9,
 //     16 rows x 1984 x 4608 12.6 / 6.8 (split: 9.8).
 //   * What bounds it: weights at 6 - 7 TB/s where every compute unit has a tile, else the tile's rows + activation rows, pulled at

@@ -271,7 +271,7 @@ def fp8_cast_stream_plan(m: int, n: int, k: int, num_cus: int):
 
 def gemm_bf16_fp8_bf16_nt(x: torch.Tensor, rhs: Tuple[torch.Tensor, torch.Tensor], out: torch.Tensor) -> None:
     """`gemm_fp8_fp8_bf16_nt(per_token_cast_to_fp8(x, col_major_scales=True), rhs, out)` for bf16 activations `x` `[m, k]`,
-    bit for bit (the same two kernels), as ONE call: one trip through Python and one `launch`, which enqueues the quantiser and
+    bit for bit, as ONE call: one trip through Python and one `launch`, which enqueues the quantiser and
     the GEMM back to back; the codes and scales live in scratch memory the entry keeps per stream, so nothing is allocated
     per call. What a decode step saves is host time: two entry calls cost 18-22 us of Python, which is more than both
     kernels take on the device (64 x 4096 x 7168: 21.7 -> about 13 us call to call). The reference names only the GEMM's
@@ -280,8 +280,9 @@ def gemm_bf16_fp8_bf16_nt(x: torch.Tensor, rhs: Tuple[torch.Tensor, torch.Tensor
     kernels: every one of the 64 workgroups that share a K range repeats the quantisation of its 64 x 1792 activations,
     9.6 us of vector arithmetic per workgroup against 2.5 us for the quantiser kernel spread over the chip (21.5 us in one
     kernel against 3 + 9.7 us in two; same bits); with up to 8 rows in front of the weight-streaming kernel it pays
-    (`fp8_cast_stream_plan`: one launch, no scratch). Problems whose codes do not fit the scratch area (or with
-    `YAN_SPLIT_K=0`, which means no memory kept by the entries) run the two entries one after the other."""
+    (`fp8_cast_stream_plan`: one kernel with the quantiser's arithmetic, no scratch, whatever `YAN_SPLIT_K` says). Other problems whose codes
+    do not fit the scratch area (or with `YAN_SPLIT_K=0`, which means no memory kept by the entries) run the two entries one after
+    the other."""
     rhs_q, rhs_scales = rhs
     if repeat_call(CAST_FP8, x, rhs_q, rhs_scales, out):
         return

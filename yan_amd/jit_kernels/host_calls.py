@@ -6,7 +6,9 @@ The reference's entries do their checks, their plan lookup and one ctypes call i
 not, or a process without the built module, takes the Python way, whose checks and errors are unchanged.
 
 Host time of a call, Python -> native: FP8 1 x 2112 x 7168 8.5 -> 3.5 us, of which 2.5 are the launch; 16-bit 6.4 -> 3.1, from bf16 activations
-14.1 -> 5.9. 256 x 832 x 455 in fp32 takes 4.7 us a call instead of 7.3, four 2 x 1984 x 4608 from bf16 activations 29 instead of 41.
+14.1 -> 5.9. 256 x 832 x 455 in fp32 takes 4.7 us a call instead of 7.3, four 2 x 1984 x 4608 from bf16 activations 29 instead of 41. A call
+that cannot be native pays the look: 0.8 us where the scales of a large problem are copied first, 0.2 under `YAN_SPLIT_K=0` and
+`YAN_TUNE_TILES=1`, whose switches are asked before anything else.
 """
 import ctypes
 import os
