@@ -317,7 +317,7 @@ def test_tile_scheduler_visits_every_tile_once_and_walks_cover_every_slot(tmp_pa
 def test_weights_are_streamed_where_that_measured_faster():
     """Shapes that the split-K plan or the tiles measured faster on go there, neighbours that they did not stay with the weight-streaming kernel."""
     dense = {(14, 4428, 15360): 0, (16, 4428, 7168): 1, (17, 4736, 8832): 0, (18, 5888, 8832): 2, (6, 7992, 15872): 0, (3, 7936, 9984): 1,
-             (4, 12288, 8192): 0, (4, 12288, 6144): 1, (1, 15116, 4608): 0, (4, 14080, 3072): 1, (30, 13888, 1408): 0, (32, 14336, 2048): 2,
+             (4, 12288, 8192): 0, (4, 12288, 6144): 1, (1, 15116, 4608): 0, (4, 14080, 3072): 1, (30, 13888, 1408): 0, (32, 14336, 2048): 2, (32, 16384, 256): 2,
              (48, 4096, 4480): 0, (24, 4096, 7168): 2, (63, 7872, 2688): 0, (58, 7168, 1792): 4, (16, 1472, 15104): 1}
     fp8 = {(25, 1856, 9728): 0, (25, 1856, 7168): 2, (10, 13184, 11264): 0, (2, 13184, 11264): 1, (32, 16384, 16384): 2}
     for (m, n, k), atoms in dense.items():

@@ -130,7 +130,7 @@ int weight_stream_dense_atoms(int m, int n, int k, int num_cus) {
     const long long limit = rows <= 16   ? (rows == 16 && full && m <= 32 ? 580000 : 450000)
                             : rows == 24 ? (m <= 16 ? (full ? 850000 : 700000) : m <= 32 ? (full ? 850000 : 500000) : full ? 450000 : 350000)
                             : rows == 32 ? (m <= 16 ? 750000 : m > 48 ? 450000 : full ? 780000 : 600000)
-                            : rows == 64 ? (m <= 16 ? 440000 : k >= 2048 ? 600000 : 0)
+                            : rows == 64 ? (m <= 16 ? 440000 : k >= 2048 || k <= 1024 ? 600000 : 0)
                                          : (rows == 48 && m <= 16 ? 830000 : 1200000);
     return pull && (pull <= limit || (m <= 16 && rows <= 16)) ? (m + 15) / 16 : 0;
 }

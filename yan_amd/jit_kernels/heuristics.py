@@ -234,7 +234,7 @@ def get_weight_stream_dense_config(m: int, n: int, k: int, num_cus: int) -> int:
     16384, weights cycling (time here : time of split-K plan or tiles): there and below it is 0.70 to 1.02 (0.81 on average over 700 other shapes in
     the upper half of the limits, three above 1.03), beyond, on 24 weight rows, 0.97 to 1.11 (14 x 4428 x 15360 26.0 -> 28.9 us, 17 x 4736 x 8832 19.6 ->
     21.8), on 32 1.0 to 1.12 (6 x 7992 x 15872 40.5 -> 45.6), on 48 0.86 to 1.10 (4 x 12288 x 8192 33.3 -> 36.5), on 64 1.04 to 1.10 (1 x 15116 x 4608
-    23.0 -> 25.3, and 30 x 13888 x 1408 9.9 -> 10.3), with 33 to 64 rows 1.03 to 1.09 (48 x 4096 x 4480 11.7 -> 12.8, 63 x 7872 x 2688 12.9 -> 13.6). Up to 16
+    23.0 -> 25.3, and from 17 rows on between K = 1024 and 2048, 30 x 13888 x 1408 9.9 -> 10.3), with 33 to 64 rows 1.03 to 1.09 (48 x 4096 x 4480 11.7 -> 12.8, 63 x 7872 x 2688 12.9 -> 13.6). Up to 16
     rows 8 and 16 weight rows go on any K (1 x 1024 x 7168 12.7 -> 5.5, 16 x 1472 x 15104 31.1 -> 16.7, 16 x 2112 x 7168 11.5 -> 11.6, the
     closest). Same rule as `weight_stream_dense_atoms` in yan_amd/csrc/yan_gemm_capi.hip."""
     pull, rows, groups = _weight_stream_pull(m, n, 2 * k, num_cus)
@@ -248,7 +248,7 @@ def get_weight_stream_dense_config(m: int, n: int, k: int, num_cus: int) -> int:
     elif rows == 32:
         limit = 750_000 if m <= 16 else 450_000 if m > 48 else 780_000 if full else 600_000
     elif rows == 64:
-        limit = 440_000 if m <= 16 else 600_000 if k >= 2048 else 0
+        limit = 440_000 if m <= 16 else 600_000 if k >= 2048 or k <= 1024 else 0
     else:
         limit = 830_000 if rows == 48 and m <= 16 else 1_200_000
     return ceil_div(m, 16) if pull <= limit or (m <= 16 and rows <= 16) else 0
