@@ -182,3 +182,30 @@ def test_calls_on_a_copy_of_the_scales_are_not_noted(monkeypatch, entry, layout,
     else:
         yan.m_grouped_gemm_fp8_fp8_bf16_nt_masked(lhs, rhs, out, meta(groups, dtype=torch.int32), m // groups)
     assert len(calls) == noted and all(call[2] is lhs[1] for call in calls)
+
+
+def test_a_kernel_is_looked_at_once_for_all_sizes(monkeypatch):
+    """Programs with ever new sizes note each of their calls: what is the kernel's own, its address and its kinds of arguments, is kept with it."""
+    from yan_amd.jit.runtime import Runtime
+    noted, looks = [], []
+    cast = ctypes.cast
+    monkeypatch.setattr(host_calls, '_host_calls', type('Module', (), {'remember': staticmethod(lambda *call: noted.append(call))}))
+    monkeypatch.setattr(host_calls, 'repeat_call', lambda *_: False)
+    monkeypatch.setattr(host_calls.ctypes, 'cast', lambda *a: (looks.append(a), cast(*a))[1])
+    for name in ('YAN_SPLIT_K', 'YAN_TUNE_TILES'):
+        monkeypatch.delenv(name, raising=False)
+    monkeypatch.setattr(Runtime, 'is_path_valid', staticmethod(lambda path: True))
+    runtime = Runtime('a_kernel')
+    runtime._launch = ctypes.CFUNCTYPE(None)(lambda: None)
+    runtime.args = (('a', torch.float32), ('alpha', float), ('workspace', torch.uint8), ('m', int), ('streamed', bool), ('b', torch.float32),
+                    ('stream', torch.cuda.Stream))
+    b, workspace = torch.nn.Parameter(torch.zeros(2)), torch.zeros(4, dtype=torch.uint8)
+    for m in (1, 2, 3):
+        a = torch.zeros(m)
+        host_calls.remember_call((ENTRY, 1.0, a, b), 'a_kernel', runtime, (a, 1.0, workspace, m, True, b, 0), workspace)
+        call, name, address, spec = noted.pop()
+        assert call[2] is a and name == 'a_kernel' and address == cast(runtime._launch, ctypes.c_void_p).value
+        assert spec == ((TENSOR, 0), (WORKSPACE, 0), (CONSTANT, m), (CONSTANT, 1), (TENSOR, 1), (STREAM, 0))
+        host_calls.remember_call((ENTRY, 1.0, a), 'a_kernel', runtime, (a, 1.0, workspace, m, True, b, 0), workspace)
+        assert not noted            # not every tensor of the launch is one of the call's
+    assert len(looks) == 1

@@ -23,6 +23,7 @@ class Runtime:
         self.args = None
         self._launch = None
         self._call = None
+        self.native = None          # what the native repeat calls need of it
         assert self.is_path_valid(path), f'{path} is not a complete JIT kernel directory'
 
     @staticmethod
